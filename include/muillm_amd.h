@@ -101,8 +101,8 @@ int mui_linear(mui_stream_t stream, int dtype, const void* weights, long w_pitch
  * inside its calls, csrc/linear/linear.cu:178-189). With more than MUI_MAX_TOKENS tokens on a matrix of
  * few rows and a long K (the down projection up to about 256 tokens) one workgroup per output tile
  * would leave most of the chip idle: given a workspace, K is shared between several workgroups per
- * tile, which exchange fp32 partial tiles through it (4096 x 14336 at 64 tokens: 44 instead of
- * 59 us, at 256 tokens 57 instead of 109 us). workspace: mui_linear_workspace_bytes() bytes of device memory, 256-byte aligned,
+ * tile, which exchange fp32 partial tiles through it (4096 x 14336 at 64 tokens: 27 instead of
+ * 38 us, at 256 tokens 57 instead of 109 us). workspace: mui_linear_workspace_bytes() bytes of device memory, 256-byte aligned,
  * zero-filled ONCE by the caller before its first use (the kernels leave its counters at zero);
  * calls that may overlap on the device (different streams) need a workspace each. workspace may
  * be NULL (workspace_bytes 0): then, or when norm_weights is given, or for shapes that do not

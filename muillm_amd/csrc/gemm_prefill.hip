@@ -77,18 +77,6 @@ __device__ __forceinline__ f32x4 xs_load(const float* src) {
                __uint_as_float((uint32_t)(b >> 32))};
 }
 
-// SiLU(g) * u of the gate/up epilogues, the product rounded to fp32 before it is rounded to the 16-bit
-// type. Left alone the compiler merges the product and the conversion into one mixed-precision
-// instruction (v_fma_mixlo_f16) for some outputs and not for others, depending on the code around
-// them, and the instruction does not round like the pair it replaces: two kernels of the same tile
-// then differ in the last place of a few outputs in a hundred thousand. The empty asm keeps the
-// product a value of its own.
-__device__ __forceinline__ float gateup_f32(float g, float u) {
-  float r = silu_f32(g) * u;
-  asm volatile("" : "+v"(r));
-  return r;
-}
-
 // XS: K is also split over p.k_splits workgroups per tile (short prompts on matrices of few row
 // tiles, where one workgroup per tile would leave most CUs idle and a long K to each): every
 // workgroup delivers its partial tile in fp32 and counts itself in; whoever arrives last adds the
@@ -1235,16 +1223,22 @@ static int g_wide_max_tokens = kWideDefaultMaxTokens;  // longest prompt taken b
 // int8 codes; SkinnyParams as for the decode kernels (x, residual and y dense).
 int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const SkinnyParams& q) {
   if (q.tokens < 1 || q.n < 1 || q.k < 1) return MUI_ERR_INVALID_ARG;
-  // the shortest prompts are bound by the weight stream: 16 rows per workgroup, K split over the
-  // waves, no LDS tiling (gemm_wide.hip). It wins while its grid is a single round of workgroups
-  // and the token tiles are few: up to 40 tokens (o_proj at 33 tokens 16.0 vs 20.4 us for the
-  // smallest LDS tile, 19.6 vs 20.6 at 48, 23.1 vs 21.2 at 64)
+  // up to 128 tokens are bound by the weight stream. 16-bit weights: gemm_stream.hip, which takes rows of whole 256-value steps.
+  // What it declines and int8 codes: up to 40 tokens 16 rows per workgroup, K split over the waves, no LDS tiling
+  // (gemm_wide.hip), while its grid is a single round of workgroups (o_proj at 33 tokens 16.0 vs 20.4 us for the smallest LDS
+  // tile, 19.6 vs 20.6 at 48, 23.1 vs 21.2 at 64)
   PrefillGemmParams p = {};
   const long esz = (wf == WF_16BIT) ? 2 : 1;
   p.w0 = (const uint8_t*)q.w0; p.w1 = (const uint8_t*)q.w1; p.pitch = q.pitch * esz;
   p.s0 = q.s0; p.s1 = q.s1; p.s_pitch = q.s_pitch; p.group_shift = q.group_shift;
   p.x = q.x; p.gamma = q.gamma; p.mul_bias = q.mul_bias; p.add_bias = q.add_bias; p.residual = q.residual;
   p.y = q.y; p.y_pitch = q.n; p.n = q.n; p.k = q.k; p.tokens = q.tokens; p.eps = q.eps;
+  const bool scratch = q.workspace && ((uintptr_t)q.workspace & 255u) == 0 && q.workspace_bytes >= prefill_workspace_bytes();
+  if (wf == WF_16BIT && q.tokens <= 128 && g_prefill_tile == 0 && g_wide_max_tokens == kWideDefaultMaxTokens) {
+    const int st = launch_gemm_stream(s, dtype, epilogue, q, scratch ? (float*)((char*)q.workspace + kXsCounterBytes) : nullptr,
+                                      scratch ? q.workspace_bytes - kXsCounterBytes : 0);
+    if (st != MUI_ERR_UNSUPPORTED) return st;
+  }
   // a caller-provided workspace lets a long K be shared between workgroups when the tiles are few
   // (in front of the 16-rows-per-workgroup kernel only for K beyond 8192: down at 33 tokens 31 vs 50 us)
   const bool wide_default = q.tokens <= 40 && epilogue == SK_LINEAR && ceil_div(q.n, 16) <= device_cus();

@@ -1,0 +1,388 @@
+// Linear layers of 16-bit weights for 17..128 tokens (batched decoding beyond 16 rows, short prompts).
+//
+// Bound by the weight stream, and by the tokens: a matrix is read once, but every workgroup reads all token rows again from L2.
+// A CU's vector cache returns data in the order of the requests, whichever wave made them, and holds a few tens of KB of them:
+// weights arrive at 27.5 KB per microsecond and CU (7 TB/s in all), token rows at 105, and the two times ADD UP, however far ahead
+// either is requested and however the waves divide the loads (measured on 4096 x 14336 with one, the other and both; waves that
+// load only weights beside waves that load only tokens change nothing). So a unit of work is wide in rows -- what it reads of the
+// tokens, it reads for ROWS weight rows --, and where the matrix has too few rows to give every CU a wide unit, K is divided
+// between workgroups: their fp32 partial outputs go through a workspace and a second kernel adds them in order (about 3 us
+// and the bytes; down 4096 x 14336 at 32 tokens, 64 rows x a quarter of K instead of 16 rows x all of K).
+//
+// A step of 256 or 128 k-values of ROWS weight rows and all tokens is a stage of LDS (global_load_lds_dwordx4, rows of 512 or 256 bytes
+// contiguous); three to eight stages, all but one of them on their way. One barrier per step: the loads of a step go into the
+// stage that the barrier has freed. The waves divide a step by shares of 64 k-values, token tiles and (few tokens) row
+// tiles; the shares' partial tiles meet in LDS at the end of a unit and are added in order. A workgroup takes the units blockIdx,
+// blockIdx + grid, ...; the stages run on across units, so the next unit is on its way while the last one is added up.
+//
+// us at 32 tokens in bf16, tiled GEMM or 16-rows-per-workgroup kernel -> here: 6144 x 4096 20.7 -> 12.7, 4096 x 4096 15.0 -> 10.9,
+// gate/up 14336 x 4096 42.6 -> 37.4, 4096 x 14336 47 -> 24.2, 2048 x 8192 25.8 -> 11.7, 128256 x 4096 226 -> 167; at 101
+// tokens 24.3 -> 20.6, 19.6 -> 17.2, (gate/up stays on the tiled GEMM beyond 64 tokens), 49.3 -> 33.9, 33.2 -> 18.6.
+#include "skinny.cuh"
+
+namespace mui {
+
+constexpr int kStreamWaves = 8;
+constexpr int kStreamThreads = kStreamWaves * kWave;
+
+struct StreamParams {
+  const uint8_t* w0; const uint8_t* w1; long pitch;  // bytes
+  const uint16_t* x;
+  const uint16_t* mul_bias; const uint16_t* add_bias; const uint16_t* residual;
+  uint16_t* y;
+  float* part;     // [k_splits][tokens][n] where K is divided between workgroups
+  int n, k, tokens;
+  int n_units;     // bands of ROWS weight rows (gate/up: gate and up rows together)
+  int k_splits;    // more than one: every workgroup has one unit, a share of K of one band
+};
+
+// Geometry for ROWS weight rows x NT token tiles of 16 per unit
+template <int ROWS, int NT>
+struct StreamShape {
+  static constexpr int KS = ROWS + 16 * NT <= 96 ? 256 : 128;     // k-values per step: at least three stages fit
+  static constexpr int KSH = KS / 64;                              // shares of a step
+  static constexpr int RT = (ROWS + 15) / 16;
+  static constexpr int GROUPS = kStreamWaves / KSH;
+  static constexpr int GT = NT == 2 ? 2 : NT == 6 ? 3 : GROUPS;    // groups of token tiles (six tiles: two waves only load)
+  static constexpr int GR = GROUPS / GT;                           // groups of row tiles
+  static constexpr int TW = NT / GT, RW = (RT + GR - 1) / GR;      // token and row tiles per wave
+  static constexpr int RPI = 512 / KS;                             // rows per load instruction (1 KB)
+  static constexpr int W_INSTR = ROWS / RPI, INSTR = (ROWS + 16 * NT) / RPI;
+  static constexpr int Q = (INSTR + kStreamWaves - 1) / kStreamWaves;  // load instructions per wave and step (at most)
+  static constexpr int FULL = INSTR - (Q - 1) * kStreamWaves;      // waves that have Q of them, the others Q - 1
+  static constexpr int STAGE = (ROWS + 16 * NT) * KS * 2;
+  static constexpr int MEET = RT * NT < 16 / KSH ? RT * NT : 16 / KSH;  // tiles that meet at a time (KSH KB each)
+  static constexpr int PAD = ROWS % 16 ? 4096 : 0;                 // a half tile's other half, behind the last stage
+  static constexpr int FIT = (160 * 1024 - MEET * KSH * 1024 - PAD) / STAGE;
+  static constexpr int S = FIT < 8 ? FIT : 8;
+  static constexpr int LDS = S * STAGE + PAD + MEET * KSH * 1024;
+  static_assert(S >= 3 && (S - 2) * Q <= 63 && ROWS % 8 == 0 && TW * GT == NT && GR >= 1, "shape");
+};
+
+extern __shared__ __align__(16) unsigned char st_smem[];
+
+template <int AUX>
+__device__ __forceinline__ void stream_load16(const uint8_t* base, unsigned off, unsigned char* dst) {
+  asm volatile("" : "+v"(off));  // (kept a 32-bit lane offset from a scalar base)
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + off),
+                                   (__attribute__((address_space(3))) void*)dst, 16, 0, AUX);
+}
+
+// wait until at most `steps` steps' loads (Q each) are outstanding; steps beyond MOST count as MOST
+template <int MOST, int Q>
+__device__ __forceinline__ void stream_wait_steps(int steps) {
+  if constexpr (MOST > 0) {
+    if (steps >= MOST) wait_loads<MOST * Q>();
+    else stream_wait_steps<MOST - 1, Q>(steps);
+  } else {
+    wait_loads<0>();
+  }
+}
+
+template <typename T, int EPI, int ROWS, int NT>
+__global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const StreamParams p) {
+  using G = StreamShape<ROWS, NT>;
+  constexpr int KS = G::KS, KSH = G::KSH, RT = G::RT, TW = G::TW, RW = G::RW, RPI = G::RPI, S = G::S, MEET = G::MEET;
+  constexpr int CPR = KS / 8;  // 16-byte chunks per row of a stage
+  constexpr int ROW_BYTES = KS * 2;
+  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  f32x4* meet = (f32x4*)(st_smem + S * G::STAGE + G::PAD);
+
+  // this lane's place in a load instruction: row lr of RPI, chunk ls. Chunk c of row r lives in slot c ^ (r % 16) (16 rows
+  // read at one chunk fall into 16 different bank groups); the row's upper bits come with the instruction.
+  const int lr = lane / CPR, ls = (lane % CPR) ^ lr;
+
+  const int all_steps = p.k / KS;
+  const int share_k = p.k_splits > 1 ? (int)(blockIdx.x % (unsigned)p.k_splits) : 0;
+  const int first_unit = p.k_splits > 1 ? (int)(blockIdx.x / (unsigned)p.k_splits) : (int)blockIdx.x;
+  const int sb = (int)((long)all_steps * share_k / p.k_splits);
+  const int unit_steps = (int)((long)all_steps * (share_k + 1) / p.k_splits) - sb;
+  const int units = p.k_splits > 1 ? 1 : (p.n_units - first_unit + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int steps = unit_steps * units;
+  // workgroups start at different steps: their rows are whole multiples of the memory channels' interleave apart, so
+  // workgroups that walked K in step would all ask the same channels (reads of a matrix 6.0 -> 6.9 TB/s)
+  const int turn = (int)((blockIdx.x >> 3) % (unsigned)unit_steps);
+
+  // the step that is loaded next
+  int lu = first_unit, lc = 0, lslot = 0;
+  auto load_next = [&]() {
+    const int turned = lc + turn < unit_steps ? lc + turn : lc + turn - unit_steps;
+    const long kb = (long)(sb + turned) * ROW_BYTES;
+    const int row0 = lu * ROWS;
+    unsigned char* stage = st_smem + lslot * G::STAGE;
+#pragma unroll
+    for (int q = 0; q < G::Q; ++q) {
+      const int i = q * kStreamWaves + wave;
+      if (q == G::Q - 1 && G::FULL < kStreamWaves && wave >= G::FULL) continue;
+      const int r = i * RPI;  // rows r .. r + RPI of the stage
+      if (i < G::W_INSTR) {
+        const uint8_t* base;
+        if constexpr (EPI == SK_GATEUP) {  // a tile of 16 rows: eight gate rows, then the up rows of the same outputs
+          int o = (row0 >> 1) + (r >> 4) * 8 + (r & 7);
+          o = o < p.n - RPI ? o : p.n - RPI;  // (past the matrix: rows that are there, never stored)
+          base = ((r & 8) ? p.w1 : p.w0) + (long)o * p.pitch;
+        } else {
+          const int o = row0 + r < p.n - RPI ? row0 + r : p.n - RPI;
+          base = p.w0 + (long)o * p.pitch;
+        }
+        stream_load16<2>(base + kb, (unsigned)(lr * (unsigned)p.pitch) + (unsigned)((ls ^ (r & 15)) * 16), stage + r * ROW_BYTES);  // non-temporal
+      } else {
+        const int tr = r - ROWS;  // tokens past the end read the last one
+        const int rb = tr < p.tokens ? tr : p.tokens - 1, most = p.tokens - 1 - rb;
+        const int tk = lr < most ? lr : most;
+        stream_load16<0>((const uint8_t*)p.x + (long)rb * p.k * 2 + kb, (unsigned)(tk * p.k * 2) + (unsigned)((ls ^ (tr & 15)) * 16),
+                         stage + r * ROW_BYTES);
+      }
+    }
+    lslot = lslot + 1 == S ? 0 : lslot + 1;
+    if (++lc == unit_steps) { lc = 0; lu += (int)gridDim.x; }
+  };
+
+  // operand reads: lane l takes row l % 16 of a tile, chunk 8 share + l / 16 (+ 4)
+  const int share = wave % KSH, group = wave / KSH;
+  const int gt = group % G::GT, gr = group / G::GT;
+  const int rr = lane & 15, rc = share * 8 + (lane >> 4);
+  const int ro0 = rr * ROW_BYTES + ((rc ^ rr) * 16), ro1 = rr * ROW_BYTES + (((rc + 4) ^ rr) * 16);
+  const bool multiplies = gr < G::GR;
+
+  f32x4 acc[RW][TW];
+#pragma unroll
+  for (int i = 0; i < RW; ++i)
+#pragma unroll
+    for (int j = 0; j < TW; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  for (int s = 0; s < S - 1 && s < steps; ++s) load_next();
+  int slot = 0, c = 0, u = first_unit;
+  for (int s = 0; s < steps; ++s) {
+    const int left = steps - s;
+    // this wave's part of step s has landed: what is outstanding belongs to the steps behind it
+    if (G::FULL == kStreamWaves || wave < G::FULL) stream_wait_steps<S - 2, G::Q>(left - 1);
+    else stream_wait_steps<S - 2, G::Q - 1>(left - 1);
+    __builtin_amdgcn_s_barrier();  // ... and everybody's, and everybody has read step s - 1: its stage is free
+    asm volatile("" ::: "memory");
+    if (S - 1 < left) load_next();
+    if (multiplies) {
+      const unsigned char* ws = st_smem + slot * G::STAGE + gr * RW * 16 * ROW_BYTES;
+      const unsigned char* xs = st_smem + slot * G::STAGE + (ROWS + gt * TW * 16) * ROW_BYTES;
+      u32x4 b[TW][2];
+#pragma unroll
+      for (int j = 0; j < TW; ++j) {
+        b[j][0] = *(const u32x4*)(xs + j * 16 * ROW_BYTES + ro0);
+        b[j][1] = *(const u32x4*)(xs + j * 16 * ROW_BYTES + ro1);
+      }
+#pragma unroll
+      for (int i = 0; i < RW; ++i) {
+        const u32x4 a0 = *(const u32x4*)(ws + i * 16 * ROW_BYTES + ro0), a1 = *(const u32x4*)(ws + i * 16 * ROW_BYTES + ro1);
+#pragma unroll
+        for (int j = 0; j < TW; ++j) {
+          acc[i][j] = mfma16x16x32<T>(a0, b[j][0], acc[i][j]);
+          acc[i][j] = mfma16x16x32<T>(a1, b[j][1], acc[i][j]);
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    slot = slot + 1 == S ? 0 : slot + 1;
+    if (++c < unit_steps) continue;
+    // ---- end of a unit: the shares' partial tiles meet, MEET tiles at a time; wave w finishes tile w of a round
+    const int row0 = u * ROWS;
+    c = 0;
+    u += (int)gridDim.x;
+#pragma unroll
+    for (int r0 = 0; r0 < RT * NT; r0 += MEET) {
+      if (r0 > 0) __builtin_amdgcn_s_barrier();  // the round before has been read
+      if (multiplies) {
+#pragma unroll
+        for (int i = 0; i < RW; ++i)
+#pragma unroll
+          for (int j = 0; j < TW; ++j) {
+            const int id = (gr * RW + i) * NT + gt * TW + j;
+            if (id >= r0 && id < r0 + MEET && gr * RW + i < RT) meet[((id - r0) * KSH + share) * 64 + lane] = acc[i][j];
+          }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const int id = r0 + wave;
+      if (wave < MEET && id < RT * NT) {
+        const int i = id / NT, j = id % NT;
+        const f32x4* in = meet + wave * KSH * 64;
+        const int tok = 16 * j + (lane & 15), sub = lane >> 4;  // acc[e]: row 4 sub + e of the tile
+        if constexpr (EPI == SK_GATEUP) {
+          // rows 0-7 of a tile are gate rows, 8-15 the up rows of the same outputs
+          const int o = (row0 >> 1) + 8 * i + 4 * (sub & 1);
+          f32x4 g = in[lane & 31], h = in[(lane & 31) + 32];
+#pragma unroll
+          for (int w = 1; w < KSH; ++w) {
+            g += in[w * 64 + (lane & 31)];
+            h += in[w * 64 + (lane & 31) + 32];
+          }
+          if (lane < 32 && tok < p.tokens && o < p.n && 16 * i < ROWS) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              float gv = g[e], uv = h[e];
+              if (p.add_bias) {
+                gv += T::one(p.add_bias[o + e]);
+                uv += T::one(p.mul_bias[o + e]);
+              }
+              v[e] = gateup_f32(gv, uv);
+            }
+            u32x2 pk;
+            pk.x = (uint32_t)T::pack(v[0]) | ((uint32_t)T::pack(v[1]) << 16);
+            pk.y = (uint32_t)T::pack(v[2]) | ((uint32_t)T::pack(v[3]) << 16);
+            *(u32x2*)(p.y + (long)tok * p.n + o) = pk;
+          }
+        } else {
+          const int o = row0 + 16 * i + 4 * sub;
+          f32x4 a = in[lane];
+#pragma unroll
+          for (int w = 1; w < KSH; ++w) a += in[w * 64 + lane];
+          if (tok < p.tokens && o < p.n && 16 * i + 4 * sub < ROWS) {
+            if (p.k_splits > 1) {
+              *(f32x4*)(p.part + ((long)share_k * p.tokens + tok) * p.n + o) = a;
+            } else {
+            float res[4] = {0.f, 0.f, 0.f, 0.f};
+            if (p.residual) {
+              const u32x2 q = ld8(p.residual + (long)tok * p.n + o);
+              res[0] = T::one((uint16_t)(q.x & 0xffffu)); res[1] = T::one((uint16_t)(q.x >> 16));
+              res[2] = T::one((uint16_t)(q.y & 0xffffu)); res[3] = T::one((uint16_t)(q.y >> 16));
+            }
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v[e] = a[e];
+              if (p.mul_bias) v[e] *= T::one(p.mul_bias[o + e]);
+              if (p.add_bias) v[e] += T::one(p.add_bias[o + e]);
+              if (p.residual) v[e] += res[e];
+            }
+            u32x2 pk;
+            pk.x = (uint32_t)T::pack(v[0]) | ((uint32_t)T::pack(v[1]) << 16);
+            pk.y = (uint32_t)T::pack(v[2]) | ((uint32_t)T::pack(v[3]) << 16);
+            *(u32x2*)(p.y + (long)tok * p.n + o) = pk;
+            }
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < RW; ++i)
+#pragma unroll
+      for (int j = 0; j < TW; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+}
+
+// adds the partial outputs of the shares of K in order and applies what a linear's end applies; four outputs per thread
+template <typename T>
+__global__ void __launch_bounds__(256) gemm_stream_add_kernel(const StreamParams p) {
+  const long at = ((long)blockIdx.x * 256 + threadIdx.x) * 4, all = (long)p.tokens * p.n;
+  if (at >= all) return;
+  f32x4 a = *(const f32x4*)(p.part + at);
+  for (int s = 1; s < p.k_splits; ++s) a += *(const f32x4*)(p.part + s * all + at);
+  const int o = (int)(at % p.n);
+  float v[4] = {a.x, a.y, a.z, a.w};
+  u32x2 q = {0u, 0u};
+  if (p.residual) q = ld8(p.residual + at);
+  const uint32_t q0 = q.x, q1 = q.y;
+  const float res[4] = {T::lo(q0), T::hi(q0), T::lo(q1), T::hi(q1)};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (p.mul_bias) v[e] *= T::one(p.mul_bias[o + e]);
+    if (p.add_bias) v[e] += T::one(p.add_bias[o + e]);
+    if (p.residual) v[e] += res[e];
+  }
+  u32x2 pk;
+  pk.x = (uint32_t)T::pack(v[0]) | ((uint32_t)T::pack(v[1]) << 16);
+  pk.y = (uint32_t)T::pack(v[2]) | ((uint32_t)T::pack(v[3]) << 16);
+  *(u32x2*)(p.y + at) = pk;
+}
+
+template <typename T, int EPI, int ROWS, int NT>
+static int launch_stream_cfg(hipStream_t s, const StreamParams& p) {
+  using G = StreamShape<ROWS, NT>;
+  static_assert(G::LDS <= 160 * 1024, "LDS of a workgroup");
+  const int cus = device_cus(), wgs = p.n_units * p.k_splits;
+  const int st = launch_with_lds(gemm_stream_kernel<T, EPI, ROWS, NT>, dim3(wgs < cus ? wgs : cus), dim3(kStreamThreads), G::LDS, s, p);
+  if (st != MUI_OK || p.k_splits == 1) return st;
+  const long threads = (long)p.tokens * p.n / 4;
+  hipLaunchKernelGGL(gemm_stream_add_kernel<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p);
+  return launch_status();
+}
+
+// token tiles of 16 per unit
+static int stream_token_tiles(int tokens) { return tokens <= 32 ? 2 : tokens <= 64 ? 4 : tokens <= 96 ? 6 : 8; }
+constexpr int stream_widest(int nt) { return 192 - 16 * nt < 128 ? 192 - 16 * nt : 128; }  // rows with three stages of 128 k-values
+
+template <typename T, int EPI, int ROWS>
+static int launch_stream_rows(hipStream_t s, const StreamParams& p) {
+  switch (stream_token_tiles(p.tokens)) {
+    case 2: return launch_stream_cfg<T, EPI, ROWS, 2>(s, p);
+    case 4: return launch_stream_cfg<T, EPI, ROWS, 4>(s, p);
+    case 6: if constexpr (EPI == SK_LINEAR && ROWS <= stream_widest(6)) return launch_stream_cfg<T, EPI, ROWS, 6>(s, p); break;
+    default: if constexpr (EPI == SK_LINEAR && ROWS <= stream_widest(8)) return launch_stream_cfg<T, EPI, ROWS, 8>(s, p); break;
+  }
+  return MUI_ERR_UNSUPPORTED;
+}
+
+template <typename T, int EPI>
+static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
+  // Rows per unit and shares of K by the least time: what a CU takes in (27.5 KB of weights, 105 KB of token rows per microsecond, 82 in
+  // steps of 128 k-values), a barrier per step, a fixed part per round of workgroups; for shares of K the second launch and the
+  // partial outputs, written and read. Measured against every other pair at 17 to 128 tokens on matrices from 2048 x 2048 to 128256 x 4096 it
+  // is within 5 % of the best: 4096 x 4096 takes 16 rows x all of K (10.9 us at 32 tokens; 64 rows x a quarter 12.1), 4096 x 14336 64 x a
+  // quarter (24.2; 16 rows x all 32.3), 2048 x 8192 32 x a quarter (11.6; 8 x all 16.3).
+  constexpr int kLinear[] = {128, 96, 64, 56, 48, 40, 32, 24, 16, 8}, kGateup[] = {112, 96, 64, 48, 32, 16};
+  const int rows = EPI == SK_GATEUP ? 2 * p.n : p.n, cus = device_cus(), nt = stream_token_tiles(p.tokens);
+  const int tried = EPI == SK_GATEUP ? 6 : 10;
+  float best = 0.f;
+  int width = 0;
+  for (int c = 0; c < tried; ++c) {
+    const int r = EPI == SK_GATEUP ? kGateup[c] : kLinear[c];
+    if (r > stream_widest(nt)) continue;
+    const int units = ceil_div(rows, r);
+    for (int k = 1; k <= 8; ++k) {
+      if (k > 1 && ((long)units * k > cus || (size_t)k * p.tokens * p.n * 4 > part_bytes || p.k / 256 < 2 * k)) break;
+      const float one = (float)p.k / k * 2.f * ((float)r / 27.5e3f + 16.f * nt / (nt > 4 ? 82e3f : 105e3f));
+      const float barriers = (float)p.k / k / (r + 16 * nt <= 96 ? 256 : 128) * 0.08f;
+      const float cost = ceil_div(units, cus) * (one + barriers + 1.f) + (k > 1 ? 2.5f + 0.3f * k + (float)k * p.tokens * p.n * 8.f / 4e6f : 0.f);
+      if (width == 0 || cost < best) { best = cost; width = r; p.n_units = units; p.k_splits = k; }
+    }
+  }
+  switch (width) {
+    case 16: return launch_stream_rows<T, EPI, 16>(s, p);
+    case 32: return launch_stream_rows<T, EPI, 32>(s, p);
+    case 48: return launch_stream_rows<T, EPI, 48>(s, p);
+    case 64: return launch_stream_rows<T, EPI, 64>(s, p);
+    case 96: return launch_stream_rows<T, EPI, 96>(s, p);
+  }
+  if constexpr (EPI == SK_LINEAR) {
+    switch (width) {
+      case 8: return launch_stream_rows<T, EPI, 8>(s, p);
+      case 24: return launch_stream_rows<T, EPI, 24>(s, p);
+      case 40: return launch_stream_rows<T, EPI, 40>(s, p);
+      case 56: return launch_stream_rows<T, EPI, 56>(s, p);
+      case 128: return launch_stream_rows<T, EPI, 128>(s, p);
+    }
+  } else if (width == 112) {
+    return launch_stream_rows<T, EPI, 112>(s, p);
+  }
+  return MUI_ERR_UNSUPPORTED;
+}
+
+// 17..128 tokens, 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve
+int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
+  if (q.tokens < 1 || q.tokens > 128 || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;
+  if (q.k % 256 || q.n % 8 || q.n < 8 || q.pitch % 8 || q.pitch > (1L << 26)) return MUI_ERR_UNSUPPORTED;
+  if ((((uintptr_t)q.w0 | (uintptr_t)q.w1 | (uintptr_t)q.x) & 15) || (((uintptr_t)q.y | (uintptr_t)q.residual) & 7)) return MUI_ERR_UNSUPPORTED;
+  StreamParams p = {};
+  p.w0 = (const uint8_t*)q.w0; p.w1 = (const uint8_t*)q.w1; p.pitch = q.pitch * 2;
+  p.x = q.x; p.mul_bias = q.mul_bias; p.add_bias = q.add_bias; p.residual = q.residual; p.y = q.y;
+  p.n = q.n; p.k = q.k; p.tokens = q.tokens; p.part = part; p.k_splits = 1;
+  if (dtype == MUI_DTYPE_F16) return epilogue == SK_GATEUP ? launch_stream_t<F16, SK_GATEUP>(s, p, 0) : launch_stream_t<F16, SK_LINEAR>(s, p, part_bytes);
+  if (dtype == MUI_DTYPE_BF16) return epilogue == SK_GATEUP ? launch_stream_t<BF16, SK_GATEUP>(s, p, 0) : launch_stream_t<BF16, SK_LINEAR>(s, p, part_bytes);
+  return MUI_ERR_UNSUPPORTED;
+}
+
+}  // namespace mui
+

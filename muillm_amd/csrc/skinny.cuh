@@ -62,6 +62,18 @@ struct PrefillGemmParams {
   unsigned* part_count;   // [tiles], zero between launches
 };
 
+// SiLU(g) * u of the gate/up epilogues, the product rounded to fp32 before it is rounded to the 16-bit
+// type. Left alone the compiler merges the product and the conversion into one mixed-precision
+// instruction (v_fma_mixlo_f16) for some outputs and not for others, depending on the code around
+// them, and the instruction does not round like the pair it replaces: two kernels of the same tile
+// then differ in the last place of a few outputs in a hundred thousand. The empty asm keeps the
+// product a value of its own.
+__device__ __forceinline__ float gateup_f32(float g, float u) {
+  float r = silu_f32(g) * u;
+  asm volatile("" : "+v"(r));
+  return r;
+}
+
 // B operand of one k-chunk: gamma * x rounded to the 16-bit type, sum of squares on the side.
 // fp16: packed multiply (one rounding, same result as the fp32 product rounded once) and a
 // packed dot for the squares.
@@ -170,6 +182,8 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int weight_format, int epilogu
 size_t prefill_workspace_bytes();  // what SkinnyParams::workspace must hold for the prompt GEMM to use it
 // 17..128 tokens: 16 weight rows per workgroup, K split over its waves, token columns in up to 8 MFMA tiles (gemm_wide.hip)
 int launch_gemm_wide(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
+// 17..128 tokens, 16-bit weights: waves that stream weight and token chunks through LDS rings of their own (gemm_stream.hip)
+int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);
 // launches gemm_skinny_kernel<dtype, weight format, epilogue>; returns a MUI_* status
 int launch_skinny(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
 // experiments: 0 disables the B-stationary persistent variant

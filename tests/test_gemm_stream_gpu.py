@@ -1,0 +1,96 @@
+"""Linears of 16-bit weights at 17..128 tokens (csrc/gemm_stream.hip) at the sizes where its tiles, rounds and shares of K end,
+against the same product in 64 bits. Gate: the output's own rounding (half a unit of its type) and fp32 accumulation,
+k 2^-24 of the sum of the products' magnitudes."""
+
+import pytest
+import torch
+
+from muillm_amd import _lib
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+HALF_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+CODE = {torch.float16: _lib.MUI_DTYPE_F16, torch.bfloat16: _lib.MUI_DTYPE_BF16}
+
+
+def _rand(shape, dtype, gen, std=1.0):
+    return torch.empty(shape, dtype=dtype, device=DEV).normal_(0.0, std, generator=gen)
+
+
+def _gen(seed):
+    g = torch.Generator(device=DEV)
+    g.manual_seed(seed)
+    return g
+
+
+def _assert_within(y, ref, magnitude, k, dtype):
+    assert bool(torch.isfinite(y).all())
+    off = (y.double() - ref).abs()
+    bound = HALF_ULP[dtype] * ref.abs() + 2.0 * k * 2.0 ** -24 * magnitude + 2.0 ** -24
+    worst = float((off / bound).max())
+    assert worst <= 1.0, f"{worst:.2f} times the bound"
+
+
+def _linear(x, w, pitch, mul=None, add=None, res=None, ws=None):
+    tokens, k = x.shape
+    n = w.shape[0]
+    y = torch.full((tokens, n), float("nan"), dtype=x.dtype, device=DEV)
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    _lib.check(_lib.load().mui_linear_ws(torch.cuda.current_stream().cuda_stream, CODE[x.dtype], w.data_ptr(), pitch, x.data_ptr(), None, 0.0,
+                                         ptr(mul), ptr(add), ptr(res), y.data_ptr(), n, k, tokens, ptr(ws), 0 if ws is None else ws.numel()),
+               "mui_linear_ws")
+    return y
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [17, 32, 33, 64, 65, 96, 97, 127, 128])
+@pytest.mark.parametrize("n,k", [(8, 256), (24, 512), (2040, 768), (4096, 1024), (1000, 4096), (1024, 8192), (33000, 256), (17416, 512)])
+def test_linear_against_64_bits(n, k, tokens, dtype):
+    """With and without a workspace (shares of K on the long rows), pitched weights, every operand of the end."""
+    g = _gen(n + k + tokens)
+    pitch = k + 8
+    w = _rand((n, pitch), dtype, g, k ** -0.5)[:, :k]
+    x, res = _rand((tokens, k), dtype, g), _rand((tokens, n), dtype, g)
+    mul, add = _rand((n,), dtype, g, 0.5), _rand((n,), dtype, g)
+    ws = torch.zeros(_lib.load().mui_linear_workspace_bytes(), dtype=torch.uint8, device=DEV)
+    plain = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    for scratch in (None, ws):
+        _assert_within(_linear(x, w, pitch, ws=scratch), plain, size, k, dtype)
+        got = _linear(x, w, pitch, mul, add, res, scratch)
+        ref = plain * mul.double() + add.double() + res.double()
+        _assert_within(got, ref, size * mul.double().abs() + add.double().abs() + res.double().abs(), k, dtype)
+        assert torch.equal(got, _linear(x, w, pitch, mul, add, res, scratch)), "not the same twice"
+    assert int(ws[:4096].sum()) == 0, "the counters of the workspace"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [17, 32, 33, 48, 64])
+@pytest.mark.parametrize("n,k", [(8, 256), (56, 512), (1000, 1024), (16400, 256), (14336, 512)])
+@pytest.mark.parametrize("packed,bias", [(True, False), (False, True)])
+def test_gateup_against_64_bits(n, k, tokens, packed, bias, dtype):
+    g = _gen(n + k + tokens)
+    w = _rand((n, 2, k) if packed else (2, n, k), dtype, g, k ** -0.5)
+    gate, up, pitch = (w[:, 0], w[:, 1], 2 * k) if packed else (w[0], w[1], k)
+    x = _rand((tokens, k), dtype, g)
+    bg, bu = (_rand((n,), dtype, g) for _ in range(2)) if bias else (None, None)
+    h = torch.full((tokens, n), float("nan"), dtype=dtype, device=DEV)
+    _lib.check(_lib.load().mui_gateup_silu_bias(torch.cuda.current_stream().cuda_stream, CODE[dtype], gate.data_ptr(), up.data_ptr(), pitch,
+                                                x.data_ptr(), None, 0.0, bg.data_ptr() if bias else None, bu.data_ptr() if bias else None,
+                                                h.data_ptr(), n, k, tokens), "mui_gateup_silu_bias")
+    gv, uv = (x.double() @ m.double().T + (0.0 if b is None else b.double()) for m, b in ((gate, bg), (up, bu)))
+    sg, su = (x.double().abs() @ m.double().abs().T + (0.0 if b is None else b.double().abs()) for m, b in ((gate, bg), (up, bu)))
+    # |d silu| <= 1.1 |d g|; silu itself a few units of fp32 off
+    size = 1.1 * sg * uv.abs() + gv.abs() * su + gv.abs() * uv.abs()
+    _assert_within(h, gv * torch.sigmoid(gv) * uv, size, k, dtype)
+
+
+def test_tokens_do_not_mix():
+    """What one token holds, infinities and NaN among it, stays with it."""
+    g = _gen(3)
+    w, x = _rand((4096, 1024), torch.bfloat16, g, 0.03), _rand((33, 1024), torch.bfloat16, g)
+    clean = _linear(x, w, 1024)
+    x[32, 5], x[7, 9] = float("inf"), float("nan")
+    dirty = _linear(x, w, 1024)
+    rest = [t for t in range(33) if t not in (7, 32)]
+    assert torch.equal(dirty[rest], clean[rest]) and bool(dirty[7].isnan().all()) and not bool(dirty[32].isfinite().any())
