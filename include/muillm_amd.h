@@ -619,6 +619,12 @@ int mui_latent_prefill_attention(mui_stream_t stream, int dtype, const void* q, 
                                  long r_batch_stride, const int64_t* row_start, float scale, int window,
                                  int q_first, void* out, int batch_row, int t, int heads, int dim, int rot_dim,
                                  int vdim);
+/* ... and of the `batch` rows batch_row ... in one launch, their keys and values kv_batch_stride elements apart. */
+int mui_latent_prefill_attention_rows(mui_stream_t stream, int dtype, const void* q, const float* cos_sin,
+                                      const void* kv, long kv_batch_stride, int kv_first, int kv_rows,
+                                      const void* r_cache, long r_batch_stride, const int64_t* row_start, float scale,
+                                      int window, int q_first, void* out, int batch_row, int batch, int t, int heads,
+                                      int dim, int rot_dim, int vdim);
 
 /* Matrix-memory recurrence over t tokens per batch row, from and to the state S [batch, heads, dk, dv],
  * n [batch, heads, slices, dk], m [batch, heads, slices] (fp32; slices = mui_mlstm_slices(dv) equal copies; all

@@ -117,6 +117,8 @@ _SIGNATURES = {
                                      _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "mui_latent_prefill_attention": (c_int, [_P, c_int, _P, _P, _P, c_int, c_int, _P, c_long, _P, c_float, c_int,
                                              c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int]),
+    "mui_latent_prefill_attention_rows": (c_int, [_P, c_int, _P, _P, _P, c_long, c_int, c_int, _P, c_long, _P, c_float, c_int,
+                                                  c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "mui_mlstm_slices": (c_int, [c_int]),
     "mui_mlstm_workspace_bytes": (ctypes.c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "mui_mlstm": (c_int, [_P, c_int, _P, _P, _P, c_long, _P, c_float, c_float, _P, _P, _P, _P, _P, _P, _P, c_int,

@@ -372,7 +372,8 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
 
 // 17..128 tokens, 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
-  if (q.tokens < 1 || q.tokens > 128 || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;
+  // gate/up beyond 64 tokens: the tiled GEMM (52 against 64 us at 128 tokens and 14336 x 4096)
+  if (q.tokens < 1 || q.tokens > (epilogue == SK_GATEUP ? 64 : 128) || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;
   if (q.k % 256 || q.n % 8 || q.n < 8 || q.pitch % 8 || q.pitch > (1L << 26)) return MUI_ERR_UNSUPPORTED;
   if ((((uintptr_t)q.w0 | (uintptr_t)q.w1 | (uintptr_t)q.x) & 15) || (((uintptr_t)q.y | (uintptr_t)q.residual) & 7)) return MUI_ERR_UNSUPPORTED;
   StreamParams p = {};

@@ -47,7 +47,8 @@ struct LatentParams {
   int kp, splits, split_keys;
 
   const void* kv;    // prefill: [keys, heads * (dim + vdim)], key row 0 = slot kv_first
-  int kv_first, kv_rows, q_first, b0;
+  int kv_first, kv_rows, q_first, b0;  // (b0: first batch row; keys of the next rows kv_batch elements on)
+  long kv_batch;
 };
 
 // ---------------------------------------------------------------------------------------
@@ -505,8 +506,9 @@ __global__ void __launch_bounds__(256) latent_output_kernel(const LatentParams p
 }
 
 // ---------------------------------------------------------------------------------------
-// prefill: grid (heads, tiles of 32 NW queries, longest first) of one batch row; NW waves of 32 queries, two or more
-// workgroups per CU. LDS holds two stages of 64 keys and one of their values: while block s is multiplied with
+// prefill: grid (heads, tiles of 32 NW queries, longest first, batch rows); NW waves of 32 queries, two or more
+// workgroups per CU. Rows of a batch share a launch: a row of 150 tokens and 16 heads is 48 workgroups, and eight launches of
+// those took 24 us each where one takes 29 us (the keys and values of all rows come from one product likewise). LDS holds two stages of 64 keys and one of their values: while block s is multiplied with
 // the queries, its values and the keys of block s + 1 are on their way (LDS-direct loads, no registers).
 // ---------------------------------------------------------------------------------------
 template <int DKC, int DVT, int NW>
@@ -526,7 +528,8 @@ __global__ void __launch_bounds__(64 * NW, DKC > 6 ? 1 : 2) latent_prefill_kerne
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4, i16 = lane & 15;
   const int h = blockIdx.x, qt0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * QT;
   const int hd = p.dim + p.rot, dk = hd;
-  const long first_row = p.row_start ? p.row_start[p.b0] : 0;
+  const int b = p.b0 + (int)blockIdx.z;
+  const long first_row = p.row_start ? p.row_start[b] : 0;
   f32x4 acc[2][DVT];
   float m[2] = {-1e30f, -1e30f}, l[2] = {0.f, 0.f};
 #pragma unroll
@@ -541,9 +544,10 @@ __global__ void __launch_bounds__(64 * NW, DKC > 6 ? 1 : 2) latent_prefill_kerne
   lo = lo > p.kv_first ? lo : p.kv_first;
   const int kvp = p.heads * (p.dim + p.vdim);
   // key / value rows counted from lo
-  const uint16_t* kbase = (const uint16_t*)p.kv + (lo - p.kv_first) * kvp + (long)h * p.dim;
-  const uint16_t* vbase = (const uint16_t*)p.kv + (lo - p.kv_first) * kvp + (long)p.heads * p.dim + (long)h * p.vdim;
-  const uint16_t* rc = (const uint16_t*)p.r_cache + p.b0 * p.r_batch + lo * p.rot;
+  const uint16_t* kv = (const uint16_t*)p.kv + blockIdx.z * p.kv_batch + (lo - p.kv_first) * kvp;
+  const uint16_t* kbase = kv + (long)h * p.dim;
+  const uint16_t* vbase = kv + (long)p.heads * p.dim + (long)h * p.vdim;
+  const uint16_t* rc = (const uint16_t*)p.r_cache + b * p.r_batch + lo * p.rot;
   const int n_keys = hi >= lo ? (int)(hi - lo + 1) : 0;
   const bool vec = p.dim % 8 == 0 && p.rot % 8 == 0 && p.vdim % 8 == 0;  // 16-byte chunks stay aligned
   // Wave w delivers rows 8 w .., 8 (w + NW) .., ... of a block (their swizzles agree). Rows past the last key
@@ -593,7 +597,7 @@ __global__ void __launch_bounds__(64 * NW, DKC > 6 ? 1 : 2) latent_prefill_kerne
 #pragma unroll 4
   for (int c = t; c < QT * DKC * 4; c += 64 * NW) {
     const int r = c / (DKC * 4), e0 = (c - r * DKC * 4) * 8;
-    const long tok = (long)p.b0 * p.t + (qt0 + r < p.t ? qt0 + r : p.t - 1);
+    const long tok = (long)b * p.t + (qt0 + r < p.t ? qt0 + r : p.t - 1);
     *(u32x4*)&ql[tile_at<QT>(r, e0)] =
         rotated_q8<T>((const uint16_t*)p.q + (tok * p.heads + h) * hd, p.cos_sin + tok * p.rot, p.dim, p.rot, e0, qvec);
   }
@@ -705,7 +709,7 @@ __global__ void __launch_bounds__(64 * NW, DKC > 6 ? 1 : 2) latent_prefill_kerne
     const float inv = s > 0.f ? 1.f / s : 0.f;
     const int tq = qt0 + wave * 32 + qt * 16 + i16;
     if (tq >= p.t) continue;
-    uint16_t* dst = (uint16_t*)p.out + (((long)p.b0 * p.t + tq) * p.heads + h) * p.vdim;
+    uint16_t* dst = (uint16_t*)p.out + (((long)b * p.t + tq) * p.heads + h) * p.vdim;
 #pragma unroll
     for (int j = 0; j < DVT; ++j)
 #pragma unroll
@@ -750,15 +754,15 @@ static int launch_latent_decode(hipStream_t s, const LatentParams& p) {
 template <typename T, int DKC, int DVT, int NW>
 static int launch_latent_prefill_w(hipStream_t s, const LatentParams& p) {
   const int tiles = ceil_div(p.t, 32 * NW);
-  if (tiles > 65535) return MUI_ERR_UNSUPPORTED;
-  return launch_with_lds(latent_prefill_kernel<T, DKC, DVT, NW>, dim3(p.heads, tiles), dim3(64 * NW),
+  if (tiles > 65535 || p.batch > 65535) return MUI_ERR_UNSUPPORTED;
+  return launch_with_lds(latent_prefill_kernel<T, DKC, DVT, NW>, dim3(p.heads, tiles, p.batch), dim3(64 * NW),
                          latent_prefill_lds<DKC, DVT, NW>(), s, p);
 }
 
 template <typename T, int DKC, int DVT>
 static int launch_latent_prefill_t(hipStream_t s, const LatentParams& p) {
   // short prompts: half as many queries per workgroup, so that there are workgroups for every CU
-  if (p.heads * ceil_div(p.t, 128) <= device_cus()) return launch_latent_prefill_w<T, DKC, DVT, 2>(s, p);
+  if ((long)p.heads * ceil_div(p.t, 128) * p.batch <= device_cus()) return launch_latent_prefill_w<T, DKC, DVT, 2>(s, p);
   return launch_latent_prefill_w<T, DKC, DVT, 4>(s, p);
 }
 
@@ -864,20 +868,30 @@ extern "C" int mui_latent_attention(mui_stream_t stream, int dtype, int route, c
   return MUI_ERR_INVALID_ARG;
 }
 
+extern "C" int mui_latent_prefill_attention_rows(mui_stream_t stream, int dtype, const void* q, const float* cos_sin,
+                                                 const void* kv, long kv_batch_stride, int kv_first, int kv_rows, const void* r_cache,
+                                            long r_batch_stride, const int64_t* row_start, float scale, int window,
+                                            int q_first, void* out, int batch_row, int batch, int t, int heads, int dim, int rot_dim,
+                                            int vdim) {
+  MUI_CHECK_ARG(q && cos_sin && kv && r_cache && out && batch_row >= 0 && batch > 0 && t > 0 && heads > 0 && dim > 0 && rot_dim >= 0);
+  MUI_CHECK_ARG(vdim > 0 && kv_first >= 0 && kv_rows > 0 && q_first >= kv_first && q_first + t == kv_first + kv_rows);
+  MUI_CHECK_ARG(kv_first == 0 || (window > 0 && q_first - window + 1 >= kv_first));
+  if (!aligned16(kv) || !aligned16(r_cache) || (rot_dim % 8 == 0 && r_batch_stride % 8) || (batch > 1 && kv_batch_stride % 8 && dim % 8 == 0 && rot_dim % 8 == 0 && vdim % 8 == 0))
+    return MUI_ERR_ALIGNMENT;
+  LatentParams p = {};
+  p.q = q; p.cos_sin = (float*)cos_sin; p.kv = kv; p.kv_first = kv_first; p.kv_rows = kv_rows; p.r_cache = (void*)r_cache;
+  p.r_batch = r_batch_stride; p.row_start = row_start; p.scale = scale; p.window = window; p.q_first = q_first; p.out = out;
+  p.b0 = batch_row; p.batch = batch; p.kv_batch = kv_batch_stride; p.t = t; p.heads = heads; p.dim = dim; p.rot = rot_dim; p.vdim = vdim;
+  if (dtype == MUI_DTYPE_F16) return launch_latent_prefill<F16>((hipStream_t)stream, p);
+  if (dtype == MUI_DTYPE_BF16) return launch_latent_prefill<BF16>((hipStream_t)stream, p);
+  return MUI_ERR_INVALID_ARG;
+}
+
 extern "C" int mui_latent_prefill_attention(mui_stream_t stream, int dtype, const void* q, const float* cos_sin,
                                             const void* kv, int kv_first, int kv_rows, const void* r_cache,
                                             long r_batch_stride, const int64_t* row_start, float scale, int window,
                                             int q_first, void* out, int batch_row, int t, int heads, int dim, int rot_dim,
                                             int vdim) {
-  MUI_CHECK_ARG(q && cos_sin && kv && r_cache && out && batch_row >= 0 && t > 0 && heads > 0 && dim > 0 && rot_dim >= 0);
-  MUI_CHECK_ARG(vdim > 0 && kv_first >= 0 && kv_rows > 0 && q_first >= kv_first && q_first + t == kv_first + kv_rows);
-  MUI_CHECK_ARG(kv_first == 0 || (window > 0 && q_first - window + 1 >= kv_first));
-  if (!aligned16(kv) || !aligned16(r_cache) || (rot_dim % 8 == 0 && r_batch_stride % 8)) return MUI_ERR_ALIGNMENT;
-  LatentParams p = {};
-  p.q = q; p.cos_sin = (float*)cos_sin; p.kv = kv; p.kv_first = kv_first; p.kv_rows = kv_rows; p.r_cache = (void*)r_cache;
-  p.r_batch = r_batch_stride; p.row_start = row_start; p.scale = scale; p.window = window; p.q_first = q_first; p.out = out;
-  p.b0 = batch_row; p.t = t; p.heads = heads; p.dim = dim; p.rot = rot_dim; p.vdim = vdim;
-  if (dtype == MUI_DTYPE_F16) return launch_latent_prefill<F16>((hipStream_t)stream, p);
-  if (dtype == MUI_DTYPE_BF16) return launch_latent_prefill<BF16>((hipStream_t)stream, p);
-  return MUI_ERR_INVALID_ARG;
+  return mui_latent_prefill_attention_rows(stream, dtype, q, cos_sin, kv, 0, kv_first, kv_rows, r_cache, r_batch_stride, row_start,
+                                           scale, window, q_first, out, batch_row, 1, t, heads, dim, rot_dim, vdim);
 }

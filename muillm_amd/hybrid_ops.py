@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
-from typing import List, Optional, Tuple
+from typing import List, Optional, Tuple, Union
 
 import torch
 
@@ -244,11 +244,11 @@ def latent_attention(q: torch.Tensor, cos_sin: torch.Tensor, w_uk: torch.Tensor,
     return out
 
 
-def latent_prefill_attention(q: torch.Tensor, cos_sin: torch.Tensor, kv: List[torch.Tensor], kv_first: int,
+def latent_prefill_attention(q: torch.Tensor, cos_sin: torch.Tensor, kv: Union[torch.Tensor, List[torch.Tensor]], kv_first: int,
                              r_cache: torch.Tensor, row_start: Optional[torch.Tensor], q_first: int, heads: int, dim: int,
                              vdim: int, scale: float, window: int) -> torch.Tensor:
     """The same for a prompt (or a portion of one) with the keys and values of slots kv_first .. made
-    beforehand: kv[b] = [rows, heads * (dim | vdim)] per batch row."""
+    beforehand: kv[b] = [rows, heads * (dim | vdim)] per batch row; a tensor [B, rows, .] takes one launch."""
     rot = r_cache.shape[-1]
     b, t = _check_latent(q, cos_sin, heads, dim, rot)
     _operand(r_cache, "r_cache", q)
@@ -258,6 +258,13 @@ def latent_prefill_attention(q: torch.Tensor, cos_sin: torch.Tensor, kv: List[to
         raise RuntimeError("the tokens lie outside the cache")
     lib = _lib.load()
     out = torch.empty((b, t, heads * vdim), dtype=q.dtype, device=q.device)
+    if torch.is_tensor(kv):
+        _operand(kv, "kv", q, (b, rows, heads * (dim + vdim)))
+        check(lib.mui_latent_prefill_attention_rows(_stream(q), dtype_code(q.dtype), q.data_ptr(), cos_sin.data_ptr(), kv.data_ptr(),
+                                                    kv.stride(0), kv_first, rows, r_cache.data_ptr(), r_cache.stride(0), _ptr(row_start),
+                                                    float(scale), int(window), q_first, out.data_ptr(), 0, b, t, heads, dim, rot, vdim),
+              "mui_latent_prefill_attention_rows")
+        return out
     for i in range(b):
         _operand(kv[i], "kv", q, (rows, heads * (dim + vdim)))
         check(lib.mui_latent_prefill_attention(_stream(q), dtype_code(q.dtype), q.data_ptr(), cos_sin.data_ptr(),

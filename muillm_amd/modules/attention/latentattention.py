@@ -74,7 +74,7 @@ class MuiLatentAttention(MuiModule):
             # keys and values of everything the tokens can see, once per call
             q_first = cache.get_seq_length()
             kv_first = max(0, q_first - c.window + 1) if c.window else 0
-            kv = [self.up_kv(state.c[i, kv_first:q_first + t]) for i in range(b)]
+            kv = self.up_kv(state.c[:b, kv_first:q_first + t].contiguous())
             o = hybrid_ops.latent_prefill_attention(q, cos_sin, kv, kv_first, state.r, cache.row_start, q_first, c.heads, c.dim,
                                                     c.vdim, c.scale, c.window)
         else:

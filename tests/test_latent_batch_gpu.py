@@ -1,0 +1,30 @@
+"""Prompt attention over latent rows: the rows of a batch in one launch are the rows one at a time, bit for bit."""
+
+import pytest
+import torch
+
+from muillm_amd import hybrid_ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads,dim,rot,vdim", [(3, 24, 8, 40), (1, 6, 2, 10), (16, 128, 64, 128), (5, 20, 6, 12)])
+@pytest.mark.parametrize("batch,t,q_first,window", [(2, 17, 0, 0), (3, 130, 21, 40), (8, 150, 0, 64), (32, 33, 5, 0)])
+def test_one_launch_is_the_rows_one_at_a_time(batch, t, q_first, window, heads, dim, rot, vdim, dtype):
+    g = torch.Generator(device=DEV).manual_seed(batch + t)
+    first = max(0, q_first - window + 1) if window else 0
+    rows, cap = q_first + t - first, q_first + t + 3
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV).to(dtype)  # noqa: E731
+    q, kv, r = rand(batch, t, heads * (dim + rot)), rand(batch, rows, heads * (dim + vdim)), rand(batch, cap, rot)
+    cos_sin = torch.randn(batch * t, rot, generator=g, device=DEV)
+    for starts in (None, torch.arange(batch, device=DEV) % (q_first + t)):
+        # per row: batches of one cannot tell their place, so every row's buffers are its own
+        apart = torch.cat([ops.latent_prefill_attention(q[i:i + 1], cos_sin[i * t:(i + 1) * t].contiguous(), [kv[i].clone()], first,
+                                                        r[i:i + 1].clone(), None if starts is None else starts[i:i + 1].contiguous(), q_first,
+                                                        heads, dim, vdim, (dim + rot) ** -0.5, window) for i in range(batch)])
+        listed = ops.latent_prefill_attention(q, cos_sin, [k.clone() for k in kv], first, r, starts, q_first, heads, dim, vdim,
+                                              (dim + rot) ** -0.5, window)
+        got = ops.latent_prefill_attention(q, cos_sin, kv, first, r, starts, q_first, heads, dim, vdim, (dim + rot) ** -0.5, window)
+        assert torch.equal(got, listed) and torch.equal(got, apart)
