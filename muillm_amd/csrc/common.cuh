@@ -140,6 +140,26 @@ __device__ __forceinline__ void load8(const typename T::storage* p, float (&f)[8
     unpack8<T>(ld16(p), f);
   }
 }
+// the same in two steps, for operands that are requested early and unpacked where they are used
+template <typename T>
+struct Raw8 { u32x4 v[T::kDtype == MUI_DTYPE_F32 ? 2 : 1]; };
+template <typename T>
+__device__ __forceinline__ Raw8<T> load_raw8(const typename T::storage* p) {
+  Raw8<T> r;
+  r.v[0] = ld16(p);
+  if constexpr (T::kDtype == MUI_DTYPE_F32) r.v[1] = ld16(p + 4);
+  return r;
+}
+template <typename T>
+__device__ __forceinline__ void unpack_raw8(const Raw8<T>& r, float (&f)[8]) {
+  if constexpr (T::kDtype == MUI_DTYPE_F32) {
+    const uint32_t w[8] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w, r.v[1].x, r.v[1].y, r.v[1].z, r.v[1].w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = __builtin_bit_cast(float, w[i]);
+  } else {
+    unpack8<T>(r.v[0], f);
+  }
+}
 template <typename T>
 __device__ __forceinline__ void store8(typename T::storage* p, const float (&f)[8]) {
   if constexpr (T::kDtype == MUI_DTYPE_F32) {
@@ -155,6 +175,11 @@ __device__ __forceinline__ void store8(typename T::storage* p, const float (&f)[
 __device__ __forceinline__ void load_lds16(const uint16_t* src, uint16_t* dst) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                    (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+// the same for bytes that are read once (weights of few tokens): non-temporal
+__device__ __forceinline__ void load_lds16_stream(const uint16_t* src, uint16_t* dst) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)dst, 16, 0, 2);
 }
 // until at most N vector memory loads of this wave are outstanding (they return in order); no memory
 // access moves across it

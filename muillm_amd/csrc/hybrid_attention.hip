@@ -59,6 +59,17 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
   const S* row = (const S*)p.proj + (long)tok * p.pitch;
   const S *qr = row, *kr = row + p.k_off, *vr = row + p.v_off;
   const int nq = p.heads * p.dim, nk = p.kv_heads * p.dim, nv = p.kv_heads * p.vdim;
+  // a thread's first chunk of every part and of its gain is requested before the sums over the workgroup (1 token, 4096 + 1024 +
+  // 1024 columns: 5.4 -> 4.6 us); further chunks are read where they are used
+  Raw8<T> eq, ek, ev, egq, egk;
+  if constexpr (VEC) {
+    const int cq = t * 8 < nq ? t * 8 : 0, ck = t * 8 < nk ? t * 8 : 0, cv = t * 8 < nv ? t * 8 : 0;
+    eq = load_raw8<T>(qr + cq);
+    ek = load_raw8<T>(kr + ck);
+    if (p.q_gain) egq = load_raw8<T>((const S*)p.q_gain + cq);
+    if (p.k_gain) egk = load_raw8<T>((const S*)p.k_gain + ck);
+    ev = load_raw8<T>(vr + cv);
+  }
   const long slot = p.cache_position[tok - b * p.t];
   const long pos = slot - (p.row_start ? p.row_start[b] : 0);
   for (int i = t; i < (p.dim + 1) / 2; i += nt) {
@@ -67,13 +78,14 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
     cs[i] = CosSin{c, s};
   }
   float sq = 0.f, sk = 0.f;
-  auto squares = [&](const S* x, int n) {
+  auto squares = [&](const S* x, int n, const Raw8<T>& first) {
     float a = 0.f;
     if constexpr (VEC) {
 #pragma unroll 2
       for (int c = t * 8; c < n; c += nt * 8) {
         float f[8];
-        load8<T>(x + c, f);
+        if (c == t * 8) unpack_raw8<T>(first, f);
+        else load8<T>(x + c, f);
 #pragma unroll
         for (int i = 0; i < 8; ++i) a = fmaf(f[i], f[i], a);
       }
@@ -85,8 +97,8 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
     }
     return wave_sum(a);
   };
-  if (p.q_gain) sq = squares(qr, nq);
-  if (p.k_gain) sk = squares(kr, nk);
+  if (p.q_gain) sq = squares(qr, nq, eq);
+  if (p.k_gain) sk = squares(kr, nk, ek);
   if ((t & 63) == 0) {
     red[0][t >> 6] = sq;
     red[1][t >> 6] = sk;
@@ -98,14 +110,16 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
     sk += red[1][w];
   }
   const float rq = p.q_gain ? rsqrtf(sq / (float)nq + p.eps) : 1.f, rk = p.k_gain ? rsqrtf(sk / (float)nk + p.eps) : 1.f;
-  auto emit = [&](const S* x, const S* gain, float rs, int n, S* dst) {
+  auto emit = [&](const S* x, const S* gain, float rs, int n, S* dst, const Raw8<T>& first, const Raw8<T>& first_gain) {
     if constexpr (VEC) {
 #pragma unroll 2
       for (int c = t * 8; c < n; c += nt * 8) {
         float f[8], g[8];
-        load8<T>(x + c, f);
+        if (c == t * 8) unpack_raw8<T>(first, f);
+        else load8<T>(x + c, f);
         if (gain) {
-          load8<T>(gain + c, g);
+          if (c == t * 8) unpack_raw8<T>(first_gain, g);
+          else load8<T>(gain + c, g);
 #pragma unroll
           for (int i = 0; i < 8; ++i) f[i] = g[i] * (f[i] * rs);
         }
@@ -132,14 +146,15 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
       }
     }
   };
-  emit(qr, (const S*)p.q_gain, rq, nq, (S*)p.q_out + (long)tok * nq);
+  emit(qr, (const S*)p.q_gain, rq, nq, (S*)p.q_out + (long)tok * nq, eq, egq);
   if (slot < 0 || slot >= p.max_cache_len) return;
-  emit(kr, (const S*)p.k_gain, rk, nk, (S*)p.k_cache + b * p.k_batch + slot * nk);
+  emit(kr, (const S*)p.k_gain, rk, nk, (S*)p.k_cache + b * p.k_batch + slot * nk, ek, egk);
   S* vd = (S*)p.v_cache + b * p.v_batch + slot * nv;
   if constexpr (VEC) {
     for (int c = t * 8; c < nv; c += nt * 8) {
       float f[8];
-      load8<T>(vr + c, f);
+      if (c == t * 8) unpack_raw8<T>(ev, f);
+      else load8<T>(vr + c, f);
       store8<T>(vd + c, f);
     }
   } else {

@@ -54,11 +54,61 @@ struct LatentParams {
 // ---------------------------------------------------------------------------------------
 // prepare: one workgroup per token
 // ---------------------------------------------------------------------------------------
-template <typename T>
+// VEC: a thread per chunk of eight values, the query latent's in front of the latent row's; row, gains, position and
+// frequencies are all requested before the sums over the workgroup (1 token, ranks 1536 and 512: 8.1 -> 2.9 us).
+template <typename T, bool VEC>
 __global__ void __launch_bounds__(256) latent_prepare_kernel(const LatentParams p) {
   typedef typename T::storage S;
   __shared__ float red[2][4];
   const int tok = blockIdx.x, b = tok / p.t, t = threadIdx.x;
+  if constexpr (VEC) {
+    const S* row = (const S*)p.down + (long)tok * p.down_pitch;
+    const bool kv_here = p.kv_gain != nullptr;
+    const int qc = p.q_rank >> 3, all = qc + (kv_here ? p.kv_rank >> 3 : 0), half = p.rot >> 1;
+    const int c = t < all ? t : 0;
+    const bool of_q = c < qc;
+    const Raw8<T> rx = load_raw8<T>(row + 8 * c), rg = load_raw8<T>(of_q ? (const S*)p.q_gain + 8 * c : (const S*)p.kv_gain + 8 * (c - qc));
+    // the rotation belongs to the last threads: the first ones have the longer chain
+    const int i = 255 - t;
+    const bool turns = i < half;
+    const S* kr = row + p.q_rank + p.kv_rank;
+    const double f = turns ? p.inv_freq[i] : 0.0;
+    const float ku = turns && kv_here ? T::one(kr[i]) : 0.f, kw = turns && kv_here ? T::one(kr[half + i]) : 0.f;
+    const long slot = p.cache_position[tok - b * p.t];
+    const long pos = slot - (p.row_start ? p.row_start[b] : 0);
+    float x[8], g[8], sq = 0.f;
+    unpack_raw8<T>(rx, x);
+    unpack_raw8<T>(rg, g);
+    if (t < all) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sq = fmaf(x[e], x[e], sq);
+    }
+    const float aq = wave_sum(of_q && t < all ? sq : 0.f), ak = wave_sum(of_q ? 0.f : sq);
+    if ((t & 63) == 0) {
+      red[0][t >> 6] = aq;
+      red[1][t >> 6] = ak;
+    }
+    const bool kv = kv_here && slot >= 0 && slot < p.max_cache_len;
+    if (turns) {
+      float co, si;
+      rope_angle((double)(pos > 0 ? pos : 0), f, co, si);
+      p.cos_sin[(long)tok * p.rot + i] = co;
+      p.cos_sin[(long)tok * p.rot + half + i] = si;
+      if (kv) {
+        S* dst = (S*)p.r_cache + b * p.r_batch + slot * p.rot;
+        dst[i] = T::pack(ku * co - kw * si);
+        dst[half + i] = T::pack(kw * co + ku * si);
+      }
+    }
+    __syncthreads();
+    const float* r = red[of_q ? 0 : 1];
+    const float rs = rsqrtf(((r[0] + r[1]) + (r[2] + r[3])) / (float)(of_q ? p.q_rank : p.kv_rank) + p.eps);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] *= x[e] * rs;
+    if (t < qc) store8<T>((S*)p.q_latent + (long)tok * p.q_rank + 8 * t, g);
+    else if (t < all && kv) store8<T>((S*)p.c_cache + b * p.c_batch + slot * p.kv_rank + 8 * (t - qc), g);
+    return;
+  }
   const S* row = (const S*)p.down + (long)tok * p.down_pitch;
   const S* cr = row + p.q_rank;
   const bool kv_here = p.kv_gain != nullptr;
@@ -465,6 +515,18 @@ __global__ void __launch_bounds__(256) latent_output_kernel(const LatentParams p
   const int h = blockIdx.x, tok = blockIdx.z, t = threadIdx.x;
   const long at = ((long)tok * p.heads + h) * p.splits;
   const float* part = p.part + at * p.kv_rank;
+  // the value map's row is requested before the splits are merged: its way from memory is the longer one (1 token, 512
+  // columns: 5.6 -> 5.3 us)
+  const int v = blockIdx.y * 32 + (t >> 3);
+  const int vc = v < p.vdim ? v : p.vdim - 1;
+  const uint16_t* w = (const uint16_t*)p.w_uv + ((long)h * p.vdim + vc) * p.kv_rank;
+  constexpr int kEarly = 8;
+  u32x4 early[kEarly];
+#pragma unroll
+  for (int u = 0; u < kEarly; ++u) {
+    const int c = (t & 7) * 8 + 64 * u;
+    early[u] = ld16_stream(w + (c < p.kv_rank ? c : 0));
+  }
   long lo, hi;
   visible(p, tok, tok / p.t, lo, hi);
   const int live = live_splits(p, lo, hi);
@@ -488,12 +550,18 @@ __global__ void __launch_bounds__(256) latent_output_kernel(const LatentParams p
     o[r] = a;
   }
   __syncthreads();
-  const int v = blockIdx.y * 32 + (t >> 3);
-  const int vc = v < p.vdim ? v : p.vdim - 1;
-  const uint16_t* w = (const uint16_t*)p.w_uv + ((long)h * p.vdim + vc) * p.kv_rank;
   float a = 0.f;
-#pragma unroll 8
-  for (int c = (t & 7) * 8; c < p.kv_rank; c += 64) {
+#pragma unroll
+  for (int u = 0; u < kEarly; ++u) {
+    const int c = (t & 7) * 8 + 64 * u;
+    if (c >= p.kv_rank) break;
+    float f[8];
+    unpack8<T>(early[u], f);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a = fmaf(f[i], o[c + i], a);
+  }
+#pragma unroll 4
+  for (int c = (t & 7) * 8 + 64 * kEarly; c < p.kv_rank; c += 64) {
     float f[8];
     unpack8<T>(ld16_stream(w + c), f);
 #pragma unroll
@@ -799,10 +867,16 @@ extern "C" int mui_latent_prepare(mui_stream_t stream, int dtype, const void* do
   p.batch = batch; p.t = t; p.q_rank = q_rank; p.kv_rank = kv_rank; p.rot = rot_dim; p.max_cache_len = max_cache_len;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(batch * t), block(256);
-  if (dtype == MUI_DTYPE_F16) hipLaunchKernelGGL((latent_prepare_kernel<F16>), grid, block, 0, s, p);
-  else if (dtype == MUI_DTYPE_BF16) hipLaunchKernelGGL((latent_prepare_kernel<BF16>), grid, block, 0, s, p);
-  else if (dtype == MUI_DTYPE_F32) hipLaunchKernelGGL((latent_prepare_kernel<F32>), grid, block, 0, s, p);
+  bool vec = q_rank % 8 == 0 && q_rank + (kv_gain ? kv_rank : 0) <= 8 * 256 && rot_dim <= 2 * 256 && down_pitch % 8 == 0 && aligned16(down) &&
+             aligned16(q_gain) && aligned16(q_latent);
+  if (kv_gain) vec = vec && kv_rank % 8 == 0 && c_batch_stride % 8 == 0 && aligned16(kv_gain) && aligned16(c_cache);
+#define MUI_LAUNCH_PREPARE(T) \
+  hipLaunchKernelGGL((vec ? latent_prepare_kernel<T, true> : latent_prepare_kernel<T, false>), grid, block, 0, s, p)
+  if (dtype == MUI_DTYPE_F16) MUI_LAUNCH_PREPARE(F16);
+  else if (dtype == MUI_DTYPE_BF16) MUI_LAUNCH_PREPARE(BF16);
+  else if (dtype == MUI_DTYPE_F32) MUI_LAUNCH_PREPARE(F32);
   else return MUI_ERR_INVALID_ARG;
+#undef MUI_LAUNCH_PREPARE
   return launch_status();
 }
 

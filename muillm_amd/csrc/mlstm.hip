@@ -403,7 +403,7 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
 // ---------------------------------------------------------------------------------------
 // output: one wave per (token, head)
 // ---------------------------------------------------------------------------------------
-template <typename T>
+template <typename T, bool VEC>  // VEC: dv a multiple of 8, at most 512, 16-byte aligned rows
 __global__ void __launch_bounds__(256) mlstm_output_kernel(const float* o, const typename T::storage* gain,
                                                            const typename T::storage* gate, long gate_pitch, float eps,
                                                            typename T::storage* y, long units, int heads, int dv) {
@@ -414,6 +414,26 @@ __global__ void __launch_bounds__(256) mlstm_output_kernel(const float* o, const
   const int h = (int)(u - tok * heads);
   const float* src = o + u * dv;
   float ss = 0.f;
+  if constexpr (VEC) {
+    // eight values per lane, everything requested before the sum over the head (1 row of 8 heads 6.5 -> 2.5 us)
+    const int c = lane * 8, cc = c < dv ? c : 0;
+    const Raw8<F32> ro = load_raw8<F32>(src + cc);
+    const Raw8<T> rg = load_raw8<T>(gate + tok * gate_pitch + (long)h * dv + cc), rw = load_raw8<T>(gain + (long)h * dv + cc);
+    float f[8], g[8], w[8];
+    unpack_raw8<F32>(ro, f);
+    if (c < dv) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss = fmaf(f[i], f[i], ss);
+    }
+    const float rs = rsqrtf(wave_sum(ss) / (float)dv + eps);
+    if (c >= dv) return;
+    unpack_raw8<T>(rg, g);
+    unpack_raw8<T>(rw, w);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = f[i] * rs * w[i] / (1.f + expf(-g[i]));
+    store8<T>(y + u * dv + c, f);
+    return;
+  }
   for (int i = lane; i < dv; i += 64) ss = fmaf(src[i], src[i], ss);
   const float rs = rsqrtf(wave_sum(ss) / (float)dv + eps);
   for (int i = lane; i < dv; i += 64) {
@@ -484,9 +504,10 @@ extern "C" int mui_mlstm_output(mui_stream_t stream, int dtype, const float* o, 
   const long units = (long)tokens * heads;
   const dim3 grid((unsigned)((units + 3) / 4)), block(256);
   hipStream_t s = (hipStream_t)stream;
+  const bool vec = dv % 8 == 0 && dv <= 512 && gate_pitch % 8 == 0 && aligned16(o) && aligned16(gain) && aligned16(gate) && aligned16(y);
 #define MUI_LAUNCH_OUT(T)                                                                                              \
-  hipLaunchKernelGGL((mlstm_output_kernel<T>), grid, block, 0, s, o, (const T::storage*)gain, (const T::storage*)gate, \
-                     gate_pitch, epsilon, (T::storage*)y, units, heads, dv)
+  hipLaunchKernelGGL((vec ? mlstm_output_kernel<T, true> : mlstm_output_kernel<T, false>), grid, block, 0, s, o,       \
+                     (const T::storage*)gain, (const T::storage*)gate, gate_pitch, epsilon, (T::storage*)y, units, heads, dv)
   if (dtype == MUI_DTYPE_F16) MUI_LAUNCH_OUT(F16);
   else if (dtype == MUI_DTYPE_BF16) MUI_LAUNCH_OUT(BF16);
   else if (dtype == MUI_DTYPE_F32) MUI_LAUNCH_OUT(F32);

@@ -41,16 +41,83 @@ __device__ __forceinline__ float rn_block_sum(float v, float* red) {
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// k % 8 == 0, 16-byte aligned rows, k <= 8 * 256 * CH: the row stays in registers
-template <typename T, int CH, bool MOE>
-__global__ void __launch_bounds__(kRnThreads) residual_norm_vec_kernel(const ResidualNormParams p) {
+// k % 8 == 0, 16-byte aligned rows, k <= 8 * 256 * CH: the row stays in registers. One row is a chain of two sums over the
+// workgroup; with few rows nothing hides a load inside it, and the gains are cold (a step streams gigabytes between two uses),
+// so both gains are requested with the row where registers allow (CH <= 4): 1 row of 4096 5.5 -> 3.9 us. FEW (experts, up to
+// eight per token): so are all chosen experts' rows, before it is known which of them are identity experts -- their rows are
+// read and not used --: 7.8 -> 5.2 us.
+constexpr int kRnFewRows = 256, kRnFewTop = 8;
+// The arguments are scalars, the ones of the first loads first: the first sixteen dwords are in registers when a wave starts, a
+// struct is fetched from memory before anything else can be.
+template <typename T, int CH, bool MOE, bool FEW = false>
+__global__ void __launch_bounds__(kRnThreads)
+    residual_norm_vec_kernel(const float* residual_in, const void* y_or_pairs, const void* post_gain, const void* next_gain, int k_arg, int top,
+                             const void* identity, const int* expert, const float* weight, int n_experts, float* residual_out, void* h,
+                             float y_scale, float branch_scale, float next_scale, float eps) {
+  const ResidualNormParams p = {residual_in, y_or_pairs, y_scale, post_gain, branch_scale, next_gain, next_scale, eps, residual_out, h, k_arg,
+                                y_or_pairs, identity, expert, weight, n_experts, top};
   typedef typename T::storage S;
   __shared__ float red[kRnThreads / kWave];
+  constexpr bool EARLY = CH <= 4;
   const int t = threadIdx.x;
   const long row = blockIdx.x, base = row * p.k;
   const int kc = p.k >> 3;
   float x[CH][8], y[CH][8];
+  Raw8<T> gp[EARLY ? CH : 1], gn[EARLY ? CH : 1];
   float ss = 0.f;
+  auto request_gains = [&]() {
+    if constexpr (EARLY) {
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        const int c = t + kRnThreads * j < kc ? t + kRnThreads * j : 0;
+        if (p.post_gain) gp[j] = load_raw8<T>((const S*)p.post_gain + (c << 3));
+        if (p.next_gain) gn[j] = load_raw8<T>((const S*)p.next_gain + (c << 3));
+      }
+    }
+  };
+  auto gain = [&](const void* from, const Raw8<T>* early, int j, int c, float (&g)[8]) {
+    if constexpr (EARLY) unpack_raw8<T>(early[j], g);
+    else load8<T>((const S*)from + (c << 3), g);
+  };
+  if constexpr (MOE && FEW) {
+    Raw8<T> rows[kRnFewTop][CH], own[CH];
+    int e[kRnFewTop];
+    float w[kRnFewTop];
+#pragma unroll
+    for (int u = 0; u < kRnFewTop; ++u) {
+      const int s = u < p.top ? u : p.top - 1;
+      e[u] = p.expert[row * p.top + s];
+      w[u] = p.weight[row * p.top + s];
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        const int c = t + kRnThreads * j < kc ? t + kRnThreads * j : 0;
+        rows[u][j] = load_raw8<T>((const S*)p.pairs + (row * p.top + s) * p.k + (c << 3));
+        if (u == 0) own[j] = load_raw8<T>((const S*)p.identity + base + (c << 3));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int c = t + kRnThreads * j < kc ? t + kRnThreads * j : 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[j][i] = 0.f;
+      if (p.residual_in) load8<F32>(p.residual_in + base + (c << 3), x[j]);
+    }
+    request_gains();
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      float mine[8], f[8];
+      unpack_raw8<T>(own[j], mine);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[j][i] = 0.f;
+#pragma unroll
+      for (int u = 0; u < kRnFewTop; ++u) {
+        if (u >= p.top) break;
+        unpack_raw8<T>(rows[u][j], f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[j][i] = fmaf(w[u], e[u] < p.n_experts ? f[i] : mine[i], y[j][i]);
+      }
+    }
+  } else {
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
     const int c = t + kRnThreads * j;
@@ -68,6 +135,7 @@ __global__ void __launch_bounds__(kRnThreads) residual_norm_vec_kernel(const Res
       }
     }
   }
+  request_gains();
   if constexpr (MOE) {
     // four experts' rows requested together
     for (int s0 = 0; s0 < p.top; s0 += 4) {
@@ -95,6 +163,7 @@ __global__ void __launch_bounds__(kRnThreads) residual_norm_vec_kernel(const Res
       }
     }
   }
+  }
   if (p.post_gain) {
 #pragma unroll
     for (int j = 0; j < CH; ++j)
@@ -107,7 +176,7 @@ __global__ void __launch_bounds__(kRnThreads) residual_norm_vec_kernel(const Res
       const int c = t + kRnThreads * j;
       if (c < kc) {
         float g[8];
-        load8<T>((const S*)p.post_gain + (c << 3), g);
+        gain(p.post_gain, gp, j, c, g);
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[j][i] = fmaf(g[i] * p.branch_scale, y[j][i] * rs, x[j][i]);
       }
@@ -136,7 +205,7 @@ __global__ void __launch_bounds__(kRnThreads) residual_norm_vec_kernel(const Res
     if (c < kc) {
       float g[8], o[8];
       if (p.next_gain) {
-        load8<T>((const S*)p.next_gain + (c << 3), g);
+        gain(p.next_gain, gn, j, c, g);
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) g[i] = 1.f;
@@ -202,10 +271,20 @@ static int launch_residual_norm(hipStream_t s, const ResidualNormParams& p, int 
     hipLaunchKernelGGL((residual_norm_any_kernel<T, MOE>), grid, block, 0, s, p);
   } else {
     const int ch = ceil_div(p.k >> 3, kRnThreads);
-    if (ch <= 1) hipLaunchKernelGGL((residual_norm_vec_kernel<T, 1, MOE>), grid, block, 0, s, p);
-    else if (ch <= 2) hipLaunchKernelGGL((residual_norm_vec_kernel<T, 2, MOE>), grid, block, 0, s, p);
-    else if (ch <= 4) hipLaunchKernelGGL((residual_norm_vec_kernel<T, 4, MOE>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((residual_norm_vec_kernel<T, 8, MOE>), grid, block, 0, s, p);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, 0, s, p.residual_in, MOE ? p.pairs : p.y, p.post_gain, p.next_gain, p.k, p.top, p.identity,
+                         p.expert, p.weight, p.n_experts, p.residual_out, p.h, p.y_scale, p.branch_scale, p.next_scale, p.eps);
+      return launch_status();
+    };
+    if constexpr (MOE) {
+      // a row per CU at most: nothing but the chain of one row's loads; more rows read only what they need
+      if (rows <= kRnFewRows && p.top <= kRnFewTop && ch <= 2)
+        return ch <= 1 ? launch(residual_norm_vec_kernel<T, 1, true, true>) : launch(residual_norm_vec_kernel<T, 2, true, true>);
+    }
+    if (ch <= 1) return launch(residual_norm_vec_kernel<T, 1, MOE>);
+    if (ch <= 2) return launch(residual_norm_vec_kernel<T, 2, MOE>);
+    if (ch <= 4) return launch(residual_norm_vec_kernel<T, 4, MOE>);
+    return launch(residual_norm_vec_kernel<T, 8, MOE>);
   }
   return launch_status();
 }
