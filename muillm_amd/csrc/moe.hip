@@ -534,17 +534,23 @@ __global__ void __launch_bounds__(64 * NWR * NWT, NWR * NWT == 4 ? 2 : 1) moe_ti
   }
 }
 
-// 256 rows x 256 pairs on eight waves of 128 x 64 (a quarter less LDS traffic per product than waves of 64 x 64,
+// 256 rows x up to 256 pairs on eight waves of 128 x up to 64 (a quarter less LDS traffic per product than waves of 64 x 64,
 // which is what bounds those), k a multiple of 64. A wave holds two sets of operands: the LDS reads of one
 // half of a k-step are in flight while the other half is multiplied, and the one barrier per step has a
-// half's multiplications behind it.
+// half's multiplications behind it. An expert's weights come from HBM, mostly once: they have three stages and are
+// requested two and a half steps ahead, the tokens (L2) two stages; 160 KB in all, so pairs are read again from memory where
+// they are needed. The pairs that there are, in strips of 32, are split evenly over the SIMDs. Gate and up, us, 64 experts,
+// with two stages and pairs in strips of 64 -> now: width 4096 x 1792, 2000 tokens of 8 experts 508 -> 470, 1200 tokens 452 -> 397;
+// 2048 x 1408, 2000 tokens of 6 experts 206 -> 180. Down 300 -> 286, 243 -> 225, 110 -> 104. The weights at 4 to 5 TB/s and
+// the matrix instructions at 0.9 PFLOP/s share the bound; a last round of workgroups that is half empty takes the rest.
+// Waiting for all the first loads before the first step looks idle, but it keeps the workgroups that share rows in step:
+// without it they miss in L2 (470 -> 500).
 template <typename T, int EPI>
 __global__ void __launch_bounds__(512) moe_pipe_kernel(const MoeGemmParams p) {
-  constexpr int NW = 8, TILE = 256, OUT = EPI == MOE_GATEUP ? TILE / 2 : TILE, WR = 8, WT = 4;
+  constexpr int NW = 8, TILE = 256, OUT = EPI == MOE_GATEUP ? TILE / 2 : TILE, WR = 8;
   typedef uint16_t Stage[TILE * kMgK];
   Stage* w_lds = (Stage*)moe_smem;
-  Stage* x_lds = (Stage*)(moe_smem + 2 * sizeof(Stage));
-  __shared__ int prow[TILE];
+  Stage* x_lds = (Stage*)(moe_smem + 3 * sizeof(Stage));
   constexpr int SUP = 2;
   const int n_tiles = p.tiles[0].count;
   const int r_tiles = (p.n + OUT - 1) / OUT;
@@ -559,14 +565,19 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(const MoeGemmParams p) {
   const int o0 = (in_sup / SUP) * OUT;
 
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  // SIMD i runs waves i and i + 4, which are 128 pairs apart: a tile of few pairs leaves every SIMD its share
-  const int wr = wave & 1, wt = wave >> 1;
-  if (t < TILE) prow[t] = p.pairs[tile.first + (t < tile.count ? t : 0)];
-  __syncthreads();
+  // SIMD i runs waves i and i + 4: the pairs are dealt out in strips of 32, the odd one to waves 0 .. 3
+  const int wr = wave & 1, wt = wave >> 1, strips = (tile.count + 31) >> 5;
+  const int cols = 16 * (wt < 2 ? (strips + 1) >> 1 : strips >> 1);  // pairs of this wave, 0 .. 64
+  const int col0 = wt < 2 ? wt * cols : 32 * ((strips + 1) >> 1) + (wt - 2) * cols;
+  auto pair_at = [&](int c) { return p.pairs[tile.first + (c < tile.count ? c : 0)]; };
   // wave instruction q covers tile rows (q NW + wave) * 8 ..: 32-bit offsets from bases that are the same for
   // the wave (gate and up rows change at multiples of 64)
   const int sr = lane >> 3, sc = lane & 7;
   const int chunk = (sc ^ (((wave * 8 + sr) >> 1) & 7)) * 8;
+  const int steps = p.k / kMgK;
+  int pr[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) pr[q] = pair_at((q * NW + wave) * 8 + sr);
   const uint16_t* wbase[4];
   unsigned woff[4], xoff[4];
   const long eb = (long)tile.expert * p.expert_stride;
@@ -583,88 +594,36 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(const MoeGemmParams p) {
     }
     o = o < p.n ? o : p.n - 1;
     woff[q] = (unsigned)o * (unsigned)p.k + chunk;
-    const int pr = prow[r];
-    xoff[q] = (unsigned)(EPI == MOE_GATEUP ? pr / p.top : pr) * (unsigned)p.k + chunk;
   }
-  auto dma = [&](int s, int buf) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      unsigned off = woff[q];
-      asm volatile("" : "+v"(off));  // (kept as a 32-bit offset from a scalar base)
-      load_lds16(wbase[q] + s * kMgK + off, &w_lds[buf][(q * NW + wave) * 8 * kMgK]);
-    }
+  auto load_x = [&](int s) {
+    const uint16_t* base = p.x + (s < steps ? s : steps - 1) * kMgK;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       unsigned off = xoff[q];
+      asm volatile("" : "+v"(off));  // (kept as a 32-bit offset from a scalar base)
+      load_lds16(base + off, &x_lds[s & 1][(q * NW + wave) * 8 * kMgK]);
+    }
+  };
+  auto load_w = [&](int s, int stage) {
+    s = s < steps ? s : steps - 1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      unsigned off = woff[q];
       asm volatile("" : "+v"(off));
-      load_lds16(p.x + s * kMgK + off, &x_lds[buf][(q * NW + wave) * 8 * kMgK]);
+      load_lds16(wbase[q] + s * kMgK + off, &w_lds[stage][(q * NW + wave) * 8 * kMgK]);
     }
   };
-  f32x4 acc[WR][WT];
-#pragma unroll
-  for (int i = 0; i < WR; ++i)
-#pragma unroll
-    for (int j = 0; j < WT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int r16 = lane & 15, lg = lane >> 4, lsw = (r16 >> 1) & 7;
-  const int a_base = (wr * 128 + r16) * kMgK, b_base = (wt * 64 + r16) * kMgK;
-  u32x4 a[2][WR], b[2][WT];
-  auto read = [&](int buf, int kk, int set) {
-    const int c = ((kk * 4 + lg) ^ lsw) * 8;
+  const int a_base = (wr * 128 + r16) * kMgK, b_base = (col0 + r16) * kMgK;
+  load_w(0, 0);
 #pragma unroll
-    for (int j = 0; j < WT; ++j) b[set][j] = *(const u32x4*)&x_lds[buf][b_base + j * 16 * kMgK + c];
-#pragma unroll
-    for (int i = 0; i < WR; ++i) a[set][i] = *(const u32x4*)&w_lds[buf][a_base + i * 16 * kMgK + c];
-  };
-  auto multiply = [&](int set) {
-#pragma unroll
-    for (int i = 0; i < WR; ++i)
-#pragma unroll
-      for (int j = 0; j < WT; ++j) acc[i][j] = mfma16x16x32<T>(a[set][i], b[set][j], acc[i][j]);
-  };
-  const int steps = p.k / kMgK;
-  dma(0, 0);
-  wait_loads<0>();
+  for (int q = 0; q < 4; ++q) xoff[q] = (unsigned)(EPI == MOE_GATEUP ? pr[q] / p.top : pr[q]) * (unsigned)p.k + chunk;
+  load_x(0);
+  load_x(1);
+  load_w(1, 1);
+  load_w(2, 2);
+  wait_loads<12>();
   __syncthreads();
-  dma(steps > 1 ? 1 : 0, 1);
-  // Loads past the last step repeat it, into a stage nobody reads any more: no branches in the loop.
-  if (wt * 64 < tile.count) {
-    read(0, 0, 0);
-    for (int s = 0; s < steps; ++s) {
-      const int buf = s & 1;
-      read(buf, 1, 1);
-      multiply(0);
-      // issue order of the half: two matrix instructions, an LDS read, ...
-#pragma unroll
-      for (int i = 0; i < WR + WT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, WR * WT - 2 * (WR + WT), 0);
-      wait_loads<0>();  // step s + 1 has landed
-      __syncthreads();  // ... for everybody, and everybody has read step s
-      dma(s + 2 < steps ? s + 2 : steps - 1, buf);
-      read(buf ^ 1, 0, 0);
-      multiply(1);
-      // ... a matrix instruction and a load, eight times, then two matrix instructions and a read
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < WR + WT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
-    }
-  } else {  // none of this wave's pairs exist: it only keeps the loads going
-    for (int s = 0; s < steps; ++s) {
-      wait_loads<0>();
-      __syncthreads();
-      dma(s + 2 < steps ? s + 2 : steps - 1, s & 1);
-    }
-  }
-  wait_loads<0>();  // no load is still on its way into LDS when the workgroup ends
   const bool n4 = (p.n & 3) == 0;
   auto store4 = [&](uint16_t* yr, int o, const float (&v)[4]) {
     if (n4 && o + 4 <= p.n) {
@@ -675,27 +634,101 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(const MoeGemmParams p) {
         if (o + r < p.n) yr[o + r] = T::pack(v[r]);
     }
   };
+  // Loads past the last step repeat it, into a stage nobody reads any more: no branches in the loop. Every wave
+  // meets the same barriers, whatever its width.
+  auto run = [&](auto width) {
+    constexpr int WT = decltype(width)::value;
+    constexpr int MF = WT > 2 ? 2 : 1;  // matrix instructions between two LDS reads
+    f32x4 acc[WR][WT];
 #pragma unroll
-  for (int j = 0; j < WT; ++j) {
-    const int c = wt * 64 + j * 16 + r16;
-    if (c >= tile.count) continue;
-    uint16_t* yr = (uint16_t*)p.y + (long)prow[c] * p.n;
-    float v[4];
-    if constexpr (EPI == MOE_GATEUP) {
+    for (int i = 0; i < WR; ++i)
 #pragma unroll
-      for (int i = 0; i < WR / 2; ++i) {
+      for (int j = 0; j < WT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 a[2][WR], b[2][WT];
+    auto read = [&](int buf, int stage, int kk, int set) {
+      const int c = ((kk * 4 + lg) ^ lsw) * 8;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = moe_act(acc[i][j][r], acc[i + WR / 2][j][r], p.limit);
-        store4(yr, o0 + wr * 64 + i * 16 + 4 * lg, v);
+      for (int j = 0; j < WT; ++j) b[set][j] = *(const u32x4*)&x_lds[buf][b_base + j * 16 * kMgK + c];
+#pragma unroll
+      for (int i = 0; i < WR; ++i) a[set][i] = *(const u32x4*)&w_lds[stage][a_base + i * 16 * kMgK + c];
+    };
+    auto multiply = [&](int set) {
+#pragma unroll
+      for (int i = 0; i < WR; ++i)
+#pragma unroll
+        for (int j = 0; j < WT; ++j) acc[i][j] = mfma16x16x32<T>(a[set][i], b[set][j], acc[i][j]);
+    };
+    read(0, 0, 0, 0);
+    for (int s = 0, stage = 0; s < steps; ++s) {
+      const int buf = s & 1, next = stage < 2 ? stage + 1 : 0;
+      read(buf, stage, 1, 1);
+      multiply(0);
+      // issue order of the half: matrix instructions, an LDS read, ...
+#pragma unroll
+      for (int i = 0; i < WR + WT; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, MF, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
-    } else {
+      if constexpr (WR * WT > MF * (WR + WT)) __builtin_amdgcn_sched_group_barrier(0x008, WR * WT - MF * (WR + WT), 0);
+      wait_loads<4>();  // step s + 1 has landed, the weights of step s + 2 may be on their way
+      __syncthreads();  // ... for everybody, and everybody has read step s
+      load_x(s + 2);
+      load_w(s + 3, stage);
+      read(buf ^ 1, next, 0, 0);
+      multiply(1);
+      stage = next;
+      // ... a matrix instruction and a load, eight times, then matrix instructions and a read
 #pragma unroll
-      for (int i = 0; i < WR; ++i) {
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+      }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r];
-        store4(yr, o0 + wr * 128 + i * 16 + 4 * lg, v);
+      for (int i = 0; i < WR + WT; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, WT > 3 ? 2 : 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
     }
+    wait_loads<0>();  // no load is still on its way into LDS when the workgroup ends
+    int out[WT];
+#pragma unroll
+    for (int j = 0; j < WT; ++j) out[j] = pair_at(col0 + j * 16 + r16);
+#pragma unroll
+    for (int j = 0; j < WT; ++j) {
+      const int c = col0 + j * 16 + r16;
+      if (c >= tile.count) continue;
+      uint16_t* yr = (uint16_t*)p.y + (long)out[j] * p.n;
+      float v[4];
+      if constexpr (EPI == MOE_GATEUP) {
+#pragma unroll
+        for (int i = 0; i < WR / 2; ++i) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = moe_act(acc[i][j][r], acc[i + WR / 2][j][r], p.limit);
+          store4(yr, o0 + wr * 64 + i * 16 + 4 * lg, v);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < WR; ++i) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r];
+          store4(yr, o0 + wr * 128 + i * 16 + 4 * lg, v);
+        }
+      }
+    }
+  };
+  if (cols == 64) run(std::integral_constant<int, 4>());
+  else if (cols == 48) run(std::integral_constant<int, 3>());
+  else if (cols == 32) run(std::integral_constant<int, 2>());
+  else if (cols == 16) run(std::integral_constant<int, 1>());
+  else {  // no pairs for this wave: it only keeps the loads going
+    for (int s = 0, stage = 0; s < steps; ++s) {
+      wait_loads<4>();
+      __syncthreads();
+      load_x(s + 2);
+      load_w(s + 3, stage);
+      stage = stage < 2 ? stage + 1 : 0;
+    }
+    wait_loads<0>();
   }
 }
 
@@ -772,7 +805,7 @@ static int launch_moe_product(hipStream_t s, const MoeGemmParams& p, const int32
         const long total = (long)ceil_div(p.max_tiles, 2) * 2 * ceil_div(p.n, EPI == MOE_GATEUP ? 128 : 256);
         if (total > (1L << 30)) return MUI_ERR_UNSUPPORTED;
         return launch_with_lds(moe_pipe_kernel<T, EPI>, dim3((unsigned)((total + 7) / 8 * 8)), dim3(512),
-                               (size_t)4 * 256 * kMgK * 2, s, p);
+                               (size_t)5 * 256 * kMgK * 2, s, p);
       }
       return launch_moe_tile<T, EPI, 4, 4>(s, p);
     }
@@ -848,10 +881,12 @@ extern "C" int mui_linear_f32(mui_stream_t stream, int dtype, const void* weight
 extern "C" int mui_moe_tile_pairs(int dtype, int tokens, int top, int n_experts, int width, int ff) {
   if (dtype == MUI_DTYPE_F32 || width % 8 || ff % 8 || n_experts < 1) return 0;
   // 16-pair tiles stream an expert's weights once per tile; from about a dozen pairs per expert on a wide tile
-  // is cheaper even half empty. Of the two widths the one whose tiles cost less (a 256-pair tile, rarely full,
-  // about 1.3 times as much as a 128-pair one).
+  // is cheaper even half empty. 256-pair tiles of the pipelined kernel cost what their pairs cost (us of both products, 128 / 256
+  // pairs: width 4096, 66 pairs per expert 552 / 551, 111: 628 / 601; width 2048, 75: 232 / 233, 112: 252 / 247); those of the other
+  // kernel (k no multiple of 64), rarely full, about 1.3 times as much as a 128-pair one.
   const long per = (long)tokens * top / n_experts;
   if (per < 12) return 16;
+  if (width % kMgK == 0 && ff % kMgK == 0) return per < 96 ? 128 : 256;
   return 13 * ((per + 255) / 256) < 10 * ((per + 127) / 128) ? 256 : 128;
 }
 

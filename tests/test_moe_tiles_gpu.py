@@ -1,0 +1,40 @@
+"""Experts' products on 256-pair tiles at the edges of their 32-pair strips, their row tiles and their k-steps, against float64."""
+
+import pytest
+import torch
+
+from muillm_amd import hybrid_ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+COUNTS = [1, 31, 32, 33, 64, 65, 96, 97, 129, 160, 193, 0, 224, 225, 255, 256, 257, 300]
+# the output's rounding (half a unit: 2^-9, 2^-12 of the value) and as much again for values of the activation that round the
+# other way, against the largest output
+REL = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("width,ff", [(64, 64), (128, 192), (192, 128), (320, 576)])
+def test_products_of_uneven_experts(width, ff, dtype):
+    g = torch.Generator().manual_seed(width)
+    n, tokens = len(COUNTS), sum(COUNTS)
+    chosen = torch.repeat_interleave(torch.arange(n), torch.tensor(COUNTS))[torch.randperm(tokens, generator=g)]
+    logits = torch.full((tokens, n), -4.0).scatter_(1, chosen[:, None], 4.0)
+    x = torch.randn(tokens, width, generator=g).to(dtype).to(DEV)
+    gate, up = (torch.randn(n, ff, width, generator=g).mul_(width ** -0.5).to(dtype).to(DEV) for _ in range(2))
+    down = torch.randn(n, width, ff, generator=g).mul_(ff ** -0.5).to(dtype).to(DEV)
+    expert, _, pairs, tiles = ops.moe_route(logits.to(DEV), None, n, 1, 256)
+    assert torch.equal(expert[:, 0].cpu().long(), chosen)
+    for _ in range(2):
+        out = ops.moe_experts(x, gate, up, down, 7.0, expert, pairs, tiles, 256)
+        for e in range(n):
+            rows = (chosen == e).nonzero()[:, 0].to(DEV)
+            if not len(rows):
+                continue
+            xe = x[rows].double()
+            a = (xe @ gate[e].double().T).clamp(max=7.0)
+            u = (xe @ up[e].double().T).clamp(-7.0, 7.0)
+            act = (a * torch.sigmoid(1.702 * a) * (u + 1.0)).to(dtype).double()
+            ref = act @ down[e].double().T
+            err = float((out[rows].double() - ref).abs().max() / ref.abs().max())
+            assert err <= REL[dtype], f"expert {e}, {COUNTS[e]} pairs: {err:.2e}"

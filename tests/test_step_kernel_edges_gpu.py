@@ -1,5 +1,5 @@
 """Small kernels of a decode step where their fast forms begin and end, against float64: experts' sums of up to 256 rows and eight
-experts, grouping of up to 64 pairs by one wave, chunks of eight values per thread."""
+experts, chunks of eight values per thread; and the grouping of few pairs by expert."""
 
 import pytest
 import torch
