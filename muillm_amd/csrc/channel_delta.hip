@@ -15,7 +15,8 @@
 //           1. prepare: convolutions, norms, decays, A, and W, U0 from U = U0 - W S_in, all chunks at once
 //           2. scan: one workgroup per head and 16 value columns walks the chunks, S in accumulators
 //           3. output: norm, gain, gate; the last inputs of the convolutions for the next call
-//           All products with S or U are v_mfma_f32_16x16x4_f32.
+//           All products with S or U are v_mfma_f32_16x16x4_f32. What 1. hands to 2. (qe, w, kd, aqk, u0) lies in 16 x 16 tiles of
+//           64 lanes x 4 values, as the lanes of 2. hold them: row (u0: column) lane % 16, columns (u0: rows) 4 (lane / 16) ..
 // The last taps - 1 inputs of the convolutions are kept in a ring of rows by slot. Tokens in front of a row's
 // first slot (left padding) leave the state alone and are zeros to the convolutions.
 #include "hybrid.cuh"
@@ -43,6 +44,7 @@ struct DeltaParams {
   void* y;           // [tokens, heads * dv]
   int batch, t, heads, kv_heads, dk, dv, ra, rg, taps, ring_rows, channels;
   bool vec;  // the low-rank operands may be read 16 bytes at a time (where their rank is a multiple of 8)
+  bool yvec;  // four elements of y may be written at a time (where dv is a multiple of 4)
   // chunks
   float *qe, *w, *kd, *gc, *aqk, *u0, *o;  // per (batch, head, chunk); o [tokens, heads, dv]
   int chunks, dkp, dvp;
@@ -426,8 +428,8 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
 // chunks
 // ---------------------------------------------------------------------------------------
 // N 16 x 16 tiles of X W^T over r: lane's row of X and of each tile's W (row lane % 16 each); D: column W row lane % 16,
-// rows X 4 (lane / 16) + r
-template <typename T, int N>
+// rows X 4 (lane / 16) + r; SWAP: column X row lane % 16, rows W 4 (lane / 16) + r
+template <typename T, int N, bool SWAP = false>
 __device__ __forceinline__ void low_rank_tiles(const typename T::storage* x, const typename T::storage* const (&w)[N], int r, bool vec, f32x4 (&acc)[N]) {
   const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
@@ -437,7 +439,7 @@ __device__ __forceinline__ void low_rank_tiles(const typename T::storage* x, con
       const int e = k + g < r ? k + g : 0;
       const float a = k + g < r ? x[e] : 0.f;
 #pragma unroll
-      for (int n = 0; n < N; ++n) acc[n] = mfma_f32(a, w[n][e], acc[n]);
+      for (int n = 0; n < N; ++n) acc[n] = SWAP ? mfma_f32(w[n][e], a, acc[n]) : mfma_f32(a, w[n][e], acc[n]);
     }
   } else if (vec) {
     for (int k = 0; k < r; k += 128) {
@@ -453,7 +455,7 @@ __device__ __forceinline__ void low_rank_tiles(const typename T::storage* x, con
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int n = 0; n < N; ++n) acc[n] = mfma16x16x32<T>(a[u], b[u][n], acc[n]);
+        for (int n = 0; n < N; ++n) acc[n] = SWAP ? mfma16x16x32<T>(b[u][n], a[u], acc[n]) : mfma16x16x32<T>(a[u], b[u][n], acc[n]);
     }
   } else {
 #pragma unroll 1
@@ -470,8 +472,45 @@ __device__ __forceinline__ void low_rank_tiles(const typename T::storage* x, con
       };
       const u32x4 a = words(x);
 #pragma unroll
-      for (int n = 0; n < N; ++n) acc[n] = mfma16x16x32<T>(a, words(w[n]), acc[n]);
+      for (int n = 0; n < N; ++n) acc[n] = SWAP ? mfma16x16x32<T>(words(w[n]), a, acc[n]) : mfma16x16x32<T>(a, words(w[n]), acc[n]);
     }
+  }
+}
+
+// The same for the whole workgroup of four waves, vec: 64 neighbouring rows of W (`rows` are left, the last one stands in for those behind it) for the rows of
+// X of every wave. Per wave the rows would come four times, 64 bytes of each at a time; they go through LDS (16 KB: rows
+// of 128 values, 16-byte chunk c of row n at chunk c ^ (n % 16)).
+template <typename T, bool SWAP>
+__device__ __forceinline__ void low_rank_block(const typename T::storage* x, const typename T::storage* w, int rows, int r, uint16_t* lds, f32x4 (&acc)[4]) {
+  const int t = threadIdx.x, g = (t & 63) >> 4, i16 = t & 15;
+#pragma unroll
+  for (int n = 0; n < 4; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int k = 0; k < r; k += 128) {
+    u32x4 v[4], a[4];
+    const int ck = k + 8 * i16 < r ? k + 8 * i16 : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (t >> 4) + 16 * i;
+      v[i] = ld16(w + (long)(row < rows ? row : rows - 1) * r + ck);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = k + 32 * u + 8 * g;
+      a[u] = ld16(x + (e < r ? e : 0));
+      if (e >= r) a[u] = u32x4{0u, 0u, 0u, 0u};
+    }
+    __syncthreads();  // the rows before have been read
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *(u32x4*)&lds[((t >> 4) + 16 * i) * 128 + (i16 ^ (t >> 4)) * 8] = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const u32x4 b = *(const u32x4*)&lds[(16 * n + i16) * 128 + ((4 * u + g) ^ i16) * 8];
+        acc[n] = SWAP ? mfma16x16x32<T>(b, a[u], acc[n]) : mfma16x16x32<T>(a[u], b, acc[n]);
+      }
   }
 }
 
@@ -526,6 +565,8 @@ __device__ __forceinline__ int delta_lead(const DeltaParams& p, const DeltaRow<T
 }
 
 // 1. grid (chunks, heads, batch); wave w owns sub-chunk w, lane = channel of a block of 64 (NB blocks: dk <= 64 NB)
+// Bound by vector instructions: some six thousand per wave at 128 channels, two waves per SIMD. 201 us at 4000 tokens, 32 heads, 128 x 128
+// (246 with the roots of the unit vectors taken by every lane, W by way of memory, A2 read by every wave).
 constexpr int kDPitch = 68;  // 16 rows x 4 consecutive k in 64 different banks
 constexpr int kDInvPitch = 20;
 template <typename T, int NB, int TAPS>
@@ -586,7 +627,12 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
         wr[ct] = (const S*)p.a2 + (long)dc * p.ra;
         bias[ct] = T::one(((const S*)p.dt_bias)[dc]);
       }
-      low_rank_tiles<T, 4>(x, wr, p.ra, vec, v);
+      if (T::kDtype != MUI_DTYPE_F32 && vec) {
+        if constexpr (T::kDtype != MUI_DTYPE_F32)
+          low_rank_block<T, false>(x, (const S*)p.a2 + (long)(h * p.dk + nb * 64) * p.ra, p.dk - nb * 64, p.ra, (uint16_t*)kh, v);
+      } else {
+        low_rank_tiles<T, 4>(x, wr, p.ra, vec, v);
+      }
 #pragma unroll
       for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
@@ -605,20 +651,33 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
     const int tk = chunk * kDChunk + t;
     bt[t] = tk < p.t && row.live(tk) ? sigm(T::one(row.proj[(long)tk * p.pitch + p.b_off + h])) : 0.f;
   }
-  // unit vectors
+  // unit vectors: lane i of a row of 16 lanes sums up and takes the root for token i
+  {
+    float sq[16], sk[16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    float sq = 0.f, sk = 0.f;
+    for (int i = 0; i < 16; ++i) {
+      sq[i] = sk[i] = 0.f;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      sq = fmaf(q[nb][i], q[nb][i], sq);
-      sk = fmaf(k[nb][i], k[nb][i], sk);
+      for (int nb = 0; nb < NB; ++nb) {
+        sq[i] = fmaf(q[nb][i], q[nb][i], sq[i]);
+        sk[i] = fmaf(k[nb][i], k[nb][i], sk[i]);
+      }
     }
-    const float rq = p.q_scale / sqrtf(wave_sum(sq) + kUnitEps), rk = 1.f / sqrtf(wave_sum(sk) + kUnitEps);
+    row16_reduce_scatter<16>(sq, lane);
+    row16_reduce_scatter<16>(sk, lane);
+    sq[0] += __shfl_xor(sq[0], 16);
+    sk[0] += __shfl_xor(sk[0], 16);
+    sq[0] += __shfl_xor(sq[0], 32);
+    sk[0] += __shfl_xor(sk[0], 32);
+    const float rq = p.q_scale / sqrtf(sq[0] + kUnitEps), rk = 1.f / sqrtf(sk[0] + kUnitEps);
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      q[nb][i] *= rq;
-      k[nb][i] *= rk;
+    for (int i = 0; i < 16; ++i) {
+      const float fq = readlane_f32(rq, i), fk = readlane_f32(rk, i);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        q[nb][i] *= fq;
+        k[nb][i] *= fk;
+      }
     }
   }
 #pragma unroll
@@ -630,6 +689,7 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
   }
   __syncthreads();  // bt, gm
   // pairs inside this wave's sub-chunk: k_s times a running product of decays, against k_t and q_t
+  f32x4 near;  // A^qk, row lane % 16, columns 4 g ..
 #pragma unroll
   for (int s = 0; s < 16; ++s) {
     float w[NB], vk[16], vq[16];
@@ -656,15 +716,13 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
     c += __shfl_xor(c, 16);
     a += __shfl_xor(a, 32);
     c += __shfl_xor(c, 32);
-    if (g4 == 0) {
-      const int tr = wave * kDSub + i16, sc = wave * kDSub + s;
-      lm[tr * kDPitch + sc] = -a * bt[tr];  // zero on and above the diagonal
-      aqk_out[tr * kDChunk + sc] = c;      // zero above it
-    }
+    if (g4 == (s >> 2)) near[s & 3] = c;  // zero above the diagonal
+    if (g4 == 0) lm[(wave * kDSub + i16) * kDPitch + wave * kDSub + s] = -a * bt[wave * kDSub + i16];  // zero on and above it
   }
+  *(f32x4*)&aqk_out[((wave * 4 + wave) * 64 + lane) * 4] = near;
   // pairs of different sub-chunks (row I, column J < I): (3,0) (3,1) | (3,2) (2,0) | (2,1) | (1,0)
   const int pi[2] = {wave < 2 ? 3 : (wave == 2 ? 2 : 1), wave == 0 ? 3 : 2}, pj[2] = {wave == 1 ? 2 : (wave == 2 ? 1 : 0), wave == 0 ? 1 : 0};
-  f32x4 akk[2], aqk[2];
+  f32x4 akk[2], aqk[2], x[NB][4];  // x: the decayed keys, columns 64 n + 16 wave + lane % 16, rows 4 g ..
 #pragma unroll
   for (int u = 0; u < 2; ++u) akk[u] = aqk[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -688,18 +746,32 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       a *= g[nb][i];
-      const float x = q[nb][i] * a, y = k[nb][i] * a;
+      const float xq = q[nb][i] * a, xk = k[nb][i] * a;
       const int tr = wave * kDSub + i;
-      qh[tr * kDPitch + lane] = x;
-      kh[tr * kDPitch + lane] = y;
-      qe_out[tr * DKP + d] = x * before;
-      w_out[tr * DKP + d] = y * before;  // (solved in place below)
+      qh[tr * kDPitch + lane] = xq;
+      kh[tr * kDPitch + lane] = xk;
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      *(f32x4*)&kd_out[(long)d * kDChunk + wave * kDSub + 4 * i] = f32x4{kd[4 * i], kd[4 * i + 1], kd[4 * i + 2], kd[4 * i + 3]};
+      *(f32x4*)&kd_out[(((nb * 4 + g4) * 4 + wave) * 64 + 16 * i + i16) * 4] = f32x4{kd[4 * i], kd[4 * i + 1], kd[4 * i + 2], kd[4 * i + 3]};
     if (wave == 3) p.gc[bhc * DKP + d] = before * gm[3][d];
     __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) {  // this wave's rows of q
+      f32x4 e = *(const f32x4*)&qh[(wave * kDSub + i16) * kDPitch + ct * 16 + 4 * g4], m = {1.f, 1.f, 1.f, 1.f};
+      for (int j = 0; j < wave; ++j) m *= *(const f32x4*)&gm[j][nb * 64 + ct * 16 + 4 * g4];
+      *(f32x4*)&qe_out[(((nb * 4 + ct) * 4 + wave) * 64 + lane) * 4] = e * m;
+    }
+    {
+      const int dx = nb * 64 + wave * 16 + i16;
+      float m = 1.f;
+#pragma unroll
+      for (int I = 0; I < 4; ++I) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[nb][I][r] = kh[(I * kDSub + 4 * g4 + r) * kDPitch + wave * 16 + i16] * m;
+        m *= gm[I][dx];
+      }
+    }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       if (u == 1 && wave > 1) continue;
@@ -709,7 +781,7 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
         float e = ke[(J * kDSub + i16) * kDPitch + k0 + g4];
         for (int m = J + 1; m < I; ++m) e *= gm[m][nb * 64 + k0 + g4];
         akk[u] = mfma_f32(kh[(I * kDSub + i16) * kDPitch + k0 + g4], e, akk[u]);
-        aqk[u] = mfma_f32(qh[(I * kDSub + i16) * kDPitch + k0 + g4], e, aqk[u]);
+        aqk[u] = mfma_f32(e, qh[(I * kDSub + i16) * kDPitch + k0 + g4], aqk[u]);  // (transposed)
       }
     }
     __syncthreads();
@@ -721,8 +793,8 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
     for (int r = 0; r < 4; ++r) {
       const int tr = pi[u] * kDSub + 4 * g4 + r, sc = pj[u] * kDSub + i16;
       lm[tr * kDPitch + sc] = -akk[u][r] * bt[tr];
-      aqk_out[tr * kDChunk + sc] = aqk[u][r];
     }
+    *(f32x4*)&aqk_out[((pi[u] * 4 + pj[u]) * 64 + lane) * 4] = aqk[u];
   }
   // the values' inputs in front of their convolution (columns v0 + i16 and v0 + 64 + i16, rows 4 g .. of every sub-chunk)
   S vw[2][TAPS], vx[2][4][TAPS + 3];
@@ -747,7 +819,7 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
     }
   };
   if (wave * 16 < p.dvp) load_v(wave * 16);
-  __syncthreads();  // lm, and w_out as seen by this workgroup
+  __syncthreads();  // lm
   // X = (1 + L)^-1 diag(beta) R by blocks of 16 rows, X_I = D_I^-1 (beta_I R_I - sum_{J < I} L_IJ X_J): W from the decayed
   // keys, U0 from the values. First the inverses of the diagonal blocks, one per wave, one column per lane.
   float* dinv = qh;  // [64][kDInvPitch]
@@ -775,7 +847,7 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
   }
   // columns in the layout of accumulators: an accumulator is the next product's right operand with the contraction
   // dealt out as 4 g + r
-  auto solve = [&](auto& x) {
+  auto solve = [&](auto& x, auto each) {  // each(I, c): with block I of the right-hand side before its last product
     constexpr int N = sizeof(x) / sizeof(x[0]);
 #pragma unroll
     for (int I = 0; I < 4; ++I) {
@@ -794,25 +866,19 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int n = 0; n < N; ++n) x[n][I] = mfma_f32(di[I][r], c[n][r], x[n][I]);
+      each(I, c);
     }
   };
-  {
-    f32x4 x[NB][4];
-    float* wp = w_out + (4 * g4) * DKP + wave * 16 + i16;
+  // (the scan takes W by rows: the last product once more with its operands exchanged gives the transposed tile)
+  solve(x, [&](int I, const f32x4 (&c)[NB]) {
 #pragma unroll
-    for (int n = 0; n < NB; ++n)
+    for (int n = 0; n < NB; ++n) {
+      f32x4 w = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int I = 0; I < 4; ++I)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x[n][I][r] = wp[(I * kDSub + r) * DKP + n * 64];
-    solve(x);
-#pragma unroll
-    for (int n = 0; n < NB; ++n)
-#pragma unroll
-      for (int I = 0; I < 4; ++I)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) wp[(I * kDSub + r) * DKP + n * 64] = x[n][I][r];
-  }
+      for (int r = 0; r < 4; ++r) w = mfma_f32(c[n][r], di[I][r], w);
+      *(f32x4*)&w_out[(((n * 4 + wave) * 4 + I) * 64 + lane) * 4] = w;
+    }
+  });
 #pragma unroll 1
   for (int v0 = wave * 16; v0 < p.dvp; v0 += 128) {  // columns v0 .. and v0 + 64 ..
     f32x4 x[2][4];
@@ -836,31 +902,35 @@ __global__ void __launch_bounds__(256, NB > 2 || TAPS > 4 ? 1 : 2) delta_prepare
         }
       }
     }
-    solve(x);
+    solve(x, [](int, const f32x4 (&)[2]) {});
 #pragma unroll
     for (int n = 0; n < 2; ++n)
       if (v0 + 64 * n < p.dvp)
 #pragma unroll
-        for (int I = 0; I < 4; ++I) *(f32x4*)(p.u0 + (bhc * p.dvp + v0 + 64 * n + i16) * kDChunk + I * kDSub + 4 * g4) = x[n][I];
+        for (int I = 0; I < 4; ++I) *(f32x4*)(p.u0 + bhc * p.dvp * kDChunk + (((v0 / 16 + 4 * n) * 4 + I) * 64 + lane) * 4) = x[n][I];
   }
 }
 
-// 2. grid (heads * slices of 16 value columns, batch); wave w owns key rows 16 NT w .. of S (dkp = 64 NT). The slices
+// 2. grid (heads * slices of 16 value columns, batch). Wave w owns key rows 16 NT w .. of S (dkp = 64 NT) and tokens 16 w ..
+// of every chunk: it needs all of S for those and all of U for the rows, which go round through LDS. The slices
 // of a head are `heads` workgroups apart: one XCD's L2 serves them all where the heads are a multiple of 8.
 // An accumulator tile (rows 4 g + r, column lane % 16) is the B operand of the next product as it stands, with
-// the contraction dealt out as 4 g + r.
+// the contraction dealt out as 4 g + r; the A operands arrive as this kernel's lanes hold them, 1 KB per instruction.
+// Bound by the matrix instructions of the longest wave, 56 NT of them 32 cycles each per chunk: with all operands in cache 173 us
+// at 4000 tokens, 32 heads, 128 x 128, else 181 (267 when a wave multiplied its key rows by all tokens, and partial sums of U went
+// round instead of U and S; 202 of that with today's layouts).
 template <int NT>
 __global__ void __launch_bounds__(256, 1) delta_scan_kernel(const DeltaParams p) {
-  __shared__ __align__(16) f32x4 xu[2][4][4][64], xo[2][4][4][64];  // [buffer][wave][row tile][lane]
+  __shared__ __align__(16) f32x4 us[4][64], ss[4 * NT][64];  // tiles of U and of S by lane
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4, i16 = lane & 15;
   const int h = blockIdx.x % p.heads, c0 = (blockIdx.x / p.heads) * 16, b = blockIdx.y;
   const long bh = (long)b * p.heads + h;
   const int d0 = wave * NT * 16;
   float* st = p.s + bh * p.dk * p.dv;
   const bool col = c0 + i16 < p.dv;
-  f32x4 s[NT];
+  f32x4 s[NT], all[4 * NT];
 #pragma unroll
-  for (int i = 0; i < NT; ++i)
+  for (int i = 0; i < NT; ++i) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int d = d0 + 16 * i + 4 * g + r;
@@ -868,100 +938,115 @@ __global__ void __launch_bounds__(256, 1) delta_scan_kernel(const DeltaParams p)
       const float x = st[in ? (long)d * p.dv + c0 + i16 : 0];
       s[i][r] = in ? x : 0.f;
     }
-  f32x4 w[4][NT], q[4][NT], kd[4][NT], gc[NT], aq[4], u0[4];
-  auto load_wq = [&](int c) {
-    const float* wp = p.w + (bh * p.chunks + c) * kDChunk * p.dkp + (long)i16 * p.dkp + d0 + 4 * g;
-    const float* qp = p.qe + (bh * p.chunks + c) * kDChunk * p.dkp + (long)i16 * p.dkp + d0 + 4 * g;
+    ss[wave * NT + i][lane] = s[i];
+  }
+  f32x4 w[4 * NT], q[4 * NT], kd[NT][4], gc[NT], aq[4], u0;
+  auto rows_at = [&](int c) { return (bh * p.chunks + c) * kDChunk * p.dkp + (wave * 64 + lane) * 4; };
+  auto load_w = [&](int c) {
+    const float* wp = p.w + rows_at(c);
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        w[rt][i] = *(const f32x4*)(wp + (long)16 * rt * p.dkp + 16 * i);
-        q[rt][i] = *(const f32x4*)(qp + (long)16 * rt * p.dkp + 16 * i);
-      }
+    for (int i = 0; i < 4 * NT; ++i) w[i] = *(const f32x4*)(wp + i * 1024);
+    u0 = *(const f32x4*)(p.u0 + ((bh * p.chunks + c) * p.dvp + c0) * kDChunk + (wave * 64 + lane) * 4);
   };
-  auto load_u = [&](int c) {
-    const float* up = p.u0 + ((bh * p.chunks + c) * p.dvp + c0 + i16) * kDChunk + 4 * g;
+  auto load_q = [&](int c) {
+    const float* qp = p.qe + rows_at(c);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) u0[j] = *(const f32x4*)(up + 16 * j);
+    for (int i = 0; i < 4 * NT; ++i) q[i] = *(const f32x4*)(qp + i * 1024);
   };
   auto load_a = [&](int c) {
-    const float* ap = p.aqk + (bh * p.chunks + c) * kDChunk * kDChunk + (long)(16 * wave + i16) * kDChunk + 4 * g;
+    const float* ap = p.aqk + (bh * p.chunks + c) * kDChunk * kDChunk + (wave * 4 * 64 + lane) * 4;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) aq[j] = *(const f32x4*)(ap + 16 * (j <= wave ? j : wave));
+    for (int j = 0; j < 4; ++j) aq[j] = *(const f32x4*)(ap + (j <= wave ? j : wave) * 256);
   };
   auto load_k = [&](int c) {
-    const float* kp = p.kd + ((bh * p.chunks + c) * p.dkp + d0 + i16) * kDChunk + 4 * g;
+    const float* kp = p.kd + (bh * p.chunks + c) * kDChunk * p.dkp + ((long)wave * NT * 4 * 64 + lane) * 4;
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) kd[j][i] = *(const f32x4*)(kp + (long)16 * i * kDChunk + 16 * j);
+      for (int j = 0; j < 4; ++j) kd[i][j] = *(const f32x4*)(kp + (i * 4 + j) * 256);
       gc[i] = *(const f32x4*)(p.gc + (bh * p.chunks + c) * p.dkp + d0 + 16 * i + 4 * g);
     }
   };
-  // (what the next chunk needs is requested as soon as its registers are free, and stays there)
-  auto stay = [] { asm volatile("" ::: "memory"); };
-  load_wq(0);
-  load_u(0);
-  load_a(0);
+  // (what the next chunk needs is requested as soon as its registers are free, and stays there; so do the products between
+  // a tile's way into LDS and its way out, which they cover)
+  auto stay = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  load_w(0);
+  load_q(0);
   load_k(0);
+  load_a(0);
   stay();
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4 * NT; ++i) all[i] = ss[i][lane];
   for (int c = 0; c < p.chunks; ++c) {
-    const int buf = c & 1, next = c + 1 < p.chunks ? c + 1 : c;
-    // this wave's key rows of W S and Q S
+    const int next = c + 1 < p.chunks ? c + 1 : c;
+    f32x4 a[2], o[2], u[4];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      f32x4 a = {0.f, 0.f, 0.f, 0.f}, o = a;
+    for (int i = 0; i < 2; ++i) a[i] = o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // this wave's tokens of U0 - W S
 #pragma unroll
-      for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          a = mfma_f32(w[rt][i][r], s[i][r], a);
-          o = mfma_f32(q[rt][i][r], s[i][r], o);
-        }
-      xu[buf][wave][rt][lane] = a;
-      xo[buf][wave][rt][lane] = o;
-    }
-    load_wq(next);
-    stay();
-    __syncthreads();
-    f32x4 u[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const f32x4 a = xu[buf][0][j][lane], b4 = xu[buf][1][j][lane], c4 = xu[buf][2][j][lane], d4 = xu[buf][3][j][lane];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) u[j][r] = u0[j][r] - ((a[r] + b4[r]) + (c4[r] + d4[r]));
-    }
-    load_u(next);
-    stay();
-    {
-      const f32x4 a = xo[buf][0][wave][lane], b4 = xo[buf][1][wave][lane], c4 = xo[buf][2][wave][lane], d4 = xo[buf][3][wave][lane];
-      f32x4 o;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = (a[r] + b4[r]) + (c4[r] + d4[r]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (j <= wave)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o = mfma_f32(aq[j][r], u[j][r], o);
-      const int tk = c * kDChunk + 16 * wave + 4 * g;
-      float* dst = p.o + (((long)b * p.t + tk) * p.heads + h) * p.dv + c0 + i16;
+    for (int i = 0; i < 4 * NT; i += 2)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (tk + r < p.t && col) dst[(long)r * p.heads * p.dv] = o[r];
-    }
-    load_a(next);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) a[e] = mfma_f32(w[i + e][r], all[i + e][r], a[e]);
+    us[wave][lane] = u0 - (a[0] + a[1]);
+    load_w(next);
+    stay();
+    // and of Q S
+    auto q_s = [&](int from) {
+#pragma unroll
+      for (int i = from; i < from + 2 * NT; i += 2)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) o[e] = mfma_f32(q[i + e][r], all[i + e][r], o[e]);
+    };
+    q_s(0);
+    stay();
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) u[j] = us[j][lane];
+    stay();
+    q_s(2 * NT);
+    load_q(next);
+    stay();
+    // its rows of S
+#pragma unroll
+    for (int i = 0; i < NT; ++i) s[i] *= gc[i];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) s[i] = mfma_f32(kd[i][j][r], u[j][r], s[i]);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) ss[wave * NT + i][lane] = s[i];
+    load_k(next);
+    stay();
+    auto a_u = [&](int j) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r & 1] = mfma_f32(aq[j][r], u[j][r], o[r & 1]);
+    };
+    a_u(0);
+    stay();
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4 * NT; ++i) all[i] = ss[i][lane];
     stay();
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
+    for (int j = 1; j < 4; ++j)
+      if (j <= wave) a_u(j);
+    o[0] += o[1];
+    const int tk = c * kDChunk + 16 * wave + 4 * g;
+    float* dst = p.o + (((long)b * p.t + tk) * p.heads + h) * p.dv + c0 + i16;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s[i][r] *= gc[i][r];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[i] = mfma_f32(kd[j][i][r], u[j][r], s[i]);
-    }
-    load_k(next);
+    for (int r = 0; r < 4; ++r)
+      if (tk + r < p.t && col) dst[(long)r * p.heads * p.dv] = o[0][r];
+    load_a(next);
     stay();
   }
 #pragma unroll
@@ -973,7 +1058,9 @@ __global__ void __launch_bounds__(256, 1) delta_scan_kernel(const DeltaParams p)
     }
 }
 
-// 3. grid (chunks, heads, batch); wave w takes tokens 16 w .. of the chunk
+// 3. grid (chunks, heads, batch); wave w takes tokens 16 w .. of the chunk. A lane holds four neighbouring columns of one token
+// (the gate's tiles come transposed out of the matrix instructions): 16-byte loads and 8-byte stores. Bound by the way of G2 to the
+// CUs, 32 KB per chunk and head: 44 us at 4000 tokens, 32 heads of 128, rank 128 (71 with G2 read by every wave).
 template <typename T>
 __global__ void __launch_bounds__(256) delta_output_kernel(const DeltaParams p) {
   typedef typename T::storage S;
@@ -981,48 +1068,73 @@ __global__ void __launch_bounds__(256) delta_output_kernel(const DeltaParams p) 
   const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int tok0 = chunk * kDChunk + wave * kDSub;
   if (chunk == p.chunks - 1) keep_inputs<T>(p, b, h, t, 256);
-  if (tok0 >= p.t) return;
-  const bool vec = p.rg % 8 == 0 && p.vec;
-  const int tk = tok0 + i16 < p.t ? tok0 + i16 : p.t - 1;
+  __shared__ __align__(16) uint16_t lds[T::kDtype == MUI_DTYPE_F32 ? 8 : 64 * 128];
+  const bool vec = p.rg % 8 == 0 && p.vec, whole = p.dv % 4 == 0;
+  const bool live = tok0 + i16 < p.t;
+  const int tk = live ? tok0 + i16 : p.t - 1;
   const S* x = (const S*)p.proj + ((long)b * p.t + tk) * p.pitch + p.g_off;
-  long at[4];  // rows of this lane
-  float ss[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int tr = tok0 + 4 * g + r < p.t ? tok0 + 4 * g + r : p.t - 1;
-    at[r] = (((long)b * p.t + tr) * p.heads + h) * p.dv;
-  }
-  for (int c0 = 0; c0 < p.dv; c0 += 64)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      const int c = c0 + 16 * n + i16;
+  const long at = (((long)b * p.t + tk) * p.heads + h) * p.dv;
+  auto row = [&](int c) {  // four columns; zero past the last
+    f32x4 o;
+    if (whole) {
+      o = *(const f32x4*)(p.o + at + (c < p.dv ? c : 0));
+      if (c >= p.dv) o = f32x4{0.f, 0.f, 0.f, 0.f};
+    } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float o = p.o[at[r] + (c < p.dv ? c : 0)];
-        ss[r] = c < p.dv ? fmaf(o, o, ss[r]) : ss[r];
+        o[r] = p.o[at + (c + r < p.dv ? c + r : 0)];
+        if (c + r >= p.dv) o[r] = 0.f;
       }
     }
+    return o;
+  };
+  float ss = 0.f;
+  for (int c0 = 0; c0 < p.dv; c0 += 64) {
+    f32x4 o[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) ss[r] = 1.f / sqrtf(row16_sum(ss[r]) / (float)p.dv + p.eps);
+    for (int n = 0; n < 4; ++n) o[n] = row(c0 + 16 * n + 4 * g);
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ss = fmaf(o[n][r], o[n][r], ss);
+  }
+  ss += __shfl_xor(ss, 16);
+  ss += __shfl_xor(ss, 32);
+  const float scale = 1.f / sqrtf(ss / (float)p.dv + p.eps);
   for (int c0 = 0; c0 < p.dv; c0 += 64) {
     const S* wr[4];
-    float gain[4], o[4][4];
-    f32x4 z[4];
+    float gain[4][4];
+    f32x4 o[4], z[4];
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      const int c = c0 + 16 * n + i16, cc = c < p.dv ? c : p.dv - 1;
-      wr[n] = (const S*)p.g2 + ((long)h * p.dv + cc) * p.rg;
-      gain[n] = T::one(((const S*)p.gain)[cc]);
+      const int cw = c0 + 16 * n + i16, c = c0 + 16 * n + 4 * g;
+      wr[n] = (const S*)p.g2 + ((long)h * p.dv + (cw < p.dv ? cw : p.dv - 1)) * p.rg;
+      o[n] = row(c);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[n][r] = p.o[at[r] + cc];
+      for (int r = 0; r < 4; ++r) gain[n][r] = T::one(((const S*)p.gain)[c + r < p.dv ? c + r : p.dv - 1]);
     }
-    low_rank_tiles<T, 4>(x, wr, p.rg, vec, z);
+    if (T::kDtype != MUI_DTYPE_F32 && vec) {
+      if constexpr (T::kDtype != MUI_DTYPE_F32) low_rank_block<T, true>(x, (const S*)p.g2 + ((long)h * p.dv + c0) * p.rg, p.dv - c0, p.rg, lds, z);
+    } else {
+      low_rank_tiles<T, 4, true>(x, wr, p.rg, vec, z);
+    }
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      const int c = c0 + 16 * n + i16;
+      const int c = c0 + 16 * n + 4 * g;
+      S* y = (S*)p.y + at + c;
+      float v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (c < p.dv && tok0 + 4 * g + r < p.t) ((S*)p.y)[at[r] + c] = T::pack(o[n][r] * ss[r] * gain[n] * sigm(z[n][r]));
+      for (int r = 0; r < 4; ++r) v[r] = o[n][r] * scale * gain[n][r] * sigm(z[n][r]);
+      if (!live) continue;
+      if (whole && p.yvec) {
+        if (c >= p.dv) continue;
+        if constexpr (T::kDtype == MUI_DTYPE_F32) *(f32x4*)y = f32x4{v[0], v[1], v[2], v[3]};
+        else *(u32x2*)y = u32x2{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (c + r < p.dv) y[r] = T::pack(v[r]);
+      }
     }
   }
 }
@@ -1124,6 +1236,7 @@ extern "C" int mui_channel_delta(mui_stream_t stream, int dtype, const mui_chann
   p.cache_position = cache_position; p.row_start = row_start; p.y = y; p.batch = batch; p.t = t; p.heads = d->heads;
   p.kv_heads = d->kv_heads; p.dk = d->dk; p.dv = d->dv; p.ra = d->ra; p.rg = d->rg; p.taps = d->taps;
   p.vec = aligned16(proj) && aligned16(d->a2) && aligned16(d->g2) && pitch % 8 == 0 && d->a_offset % 8 == 0 && d->g_offset % 8 == 0;
+  p.yvec = ((uintptr_t)y & 15) == 0;
   p.ring_rows = mui_channel_delta_ring_rows(d->taps); p.channels = (int)(2 * nq + nv);
   if (t > MUI_MAX_TOKENS) {
     if (!delta_chunked(d->dk, d->taps)) return MUI_ERR_UNSUPPORTED;
