@@ -40,6 +40,7 @@ struct MlstmParams {
   float* cn;   // [batch, heads, chunks, dk]
   float* cg;   // [batch, heads, chunks, 4]: sum of f, m of the contribution, m at the start
   int chunks;
+  int group;   // value tiles per workgroup of the contributions
 };
 
 __device__ __forceinline__ bool mlstm_live(const MlstmParams& p, int b, int t) {
@@ -205,17 +206,20 @@ __device__ __forceinline__ void load_tile(float* dst, int pitch, const typename 
   for (int i = 0; i < 4; ++i) *(f32x4*)&dst[(r0 + 16 * i) * pitch + k] = v[i];
 }
 
-// 1. contribution of a chunk: grid (chunks, heads * dk tiles * dv tiles, batch)
+// 1. contribution of a chunk: grid (chunks, heads * dk tiles * groups of p.group dv tiles, batch): the gates' sums and the keys are
+// worth several tiles of values where there are workgroups enough. Its products and its output (134 MB at 2000 tokens, 8 heads, 256 x 512)
+// take about 30 us each there: 71 us (82 with one tile per workgroup and single floats stored).
 template <typename T>
 __global__ void __launch_bounds__(256) mlstm_chunk_state_kernel(const MlstmParams p) {
   typedef typename T::storage S;
   __shared__ __align__(16) float kt[kChunk * kPitchCol], vt[kChunk * kPitchCol];
   __shared__ float w[kChunk];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, g = lane >> 4, i16 = lane & 15;
-  const int kts = (p.dk + 63) / 64, vts = (p.dv + 63) / 64;
+  const int kts = (p.dk + 63) / 64, groups = (p.dv + 64 * p.group - 1) / (64 * p.group);
   const int chunk = blockIdx.x, b = blockIdx.z;
-  const int h = blockIdx.y / (kts * vts), tile = blockIdx.y - h * kts * vts;
-  const int k0 = (tile / vts) * 64, v0 = (tile % vts) * 64;
+  const int h = blockIdx.y / (kts * groups), tile = blockIdx.y - h * kts * groups;
+  const int k0 = (tile / groups) * 64, first = (tile % groups) * 64 * p.group;
+  const int end = first + 64 * p.group < p.dv ? first + 64 * p.group : p.dv;
   const long bh = (long)b * p.heads + h, bhc = bh * p.chunks + chunk;
   const int rows = p.t - chunk * kChunk < kChunk ? p.t - chunk * kChunk : kChunk;
   if (wave == 0) {
@@ -230,26 +234,37 @@ __global__ void __launch_bounds__(256) mlstm_chunk_state_kernel(const MlstmParam
   }
   const long base = ((long)b * p.t + chunk * kChunk) * p.pitch;
   load_tile<T>(kt, kPitchCol, (const S*)p.k + base + (long)h * p.dk + k0, p.pitch, rows, p.dk - k0, 1.f);
-  load_tile<T>(vt, kPitchCol, (const S*)p.v + base + (long)h * p.dv + v0, p.pitch, rows, p.dv - v0, 1.f);
-  __syncthreads();
-  f32x4 acc[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int s = 0; s < kChunk; s += 4) {
-    const float a = kt[(s + g) * kPitchCol + wave * 16 + i16] * w[s + g];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] = mfma_f32(a, vt[(s + g) * kPitchCol + 16 * j + i16], acc[j]);
-  }
   float* dst = p.cs + bhc * p.dk * p.dv;
+  const int d = k0 + wave * 16 + i16;
+#pragma unroll 1
+  for (int v0 = first; v0 < end; v0 += 64) {
+    if (v0 != first) __syncthreads();
+    load_tile<T>(vt, kPitchCol, (const S*)p.v + base + (long)h * p.dv + v0, p.pitch, rows, p.dv - v0, 1.f);
+    __syncthreads();
+    f32x4 acc[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // (values times keys: a lane gets four neighbouring columns of a row)
+#pragma unroll 4
+    for (int s = 0; s < kChunk; s += 4) {
+      const float a = kt[(s + g) * kPitchCol + wave * 16 + i16] * w[s + g];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = k0 + wave * 16 + 4 * g + r, c = v0 + 16 * j + i16;
-      if (d < p.dk && c < p.dv) dst[(long)d * p.dv + c] = acc[j][r];
+      for (int j = 0; j < 4; ++j) acc[j] = mfma_f32(vt[(s + g) * kPitchCol + 16 * j + i16], a, acc[j]);
     }
-  if (v0 == 0 && t < 64 && k0 + t < p.dk) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = v0 + 16 * j + 4 * g;
+      if (d >= p.dk) continue;
+      if ((p.dv & 3) == 0 && ((uintptr_t)dst & 15) == 0) {
+        if (c < p.dv) *(f32x4*)&dst[(long)d * p.dv + c] = acc[j];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (c + r < p.dv) dst[(long)d * p.dv + c + r] = acc[j][r];
+      }
+    }
+  }
+  if (first == 0 && t < 64 && k0 + t < p.dk) {
     float a = 0.f;
     for (int s = 0; s < kChunk; ++s) a = fmaf(kt[s * kPitchCol + t], w[s], a);
     p.cn[bhc * p.dk + k0 + t] = a;
@@ -306,18 +321,20 @@ __global__ void __launch_bounds__(64) mlstm_max_kernel(const MlstmParams p) {
   for (int i = threadIdx.x; i < p.slices; i += 64) p.m[bh * p.slices + i] = m;
 }
 
-// 3. outputs of a chunk: grid (chunks, heads * dv tiles, batch); wave w owns tokens 16 w .. of the chunk
-template <typename T>
+// 3. outputs of a chunk: grid (chunks, heads * dv tiles of 64 NV columns, batch); wave w owns tokens 16 w .. of the chunk. Bound by the matrix
+// instructions, half of which are the scores where NV is 1: at 2000 tokens, 8 heads, 256 x 512 153 us, 122 with NV = 2.
+template <typename T, int NV>
 __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams p) {
   typedef typename T::storage S;
   float* qt = (float*)ml_smem;                 // [64][kPitchRow] q block; later the weighted scores
   float* kt = qt + kChunk * kPitchRow;         // [64][kPitchRow] k block
-  float* st = kt + kChunk * kPitchRow;         // [64][kPitchCol] state block; later v
+  float* st = kt + kChunk * kPitchRow;         // NV x [64][kPitchCol] state block; later v
+  constexpr int kBlock = 64 * kPitchCol;
   __shared__ double fm[kChunk], as[kChunk];  // F - m, a
   __shared__ float ms[kChunk], inter[kChunk], nq[kChunk], nb[64];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, g = lane >> 4, i16 = lane & 15;
-  const int vts = (p.dv + 63) / 64;
-  const int chunk = blockIdx.x, b = blockIdx.z, h = blockIdx.y / vts, v0 = (blockIdx.y % vts) * 64;
+  const int vts = (p.dv + 64 * NV - 1) / (64 * NV);
+  const int chunk = blockIdx.x, b = blockIdx.z, h = blockIdx.y / vts, v0 = (blockIdx.y % vts) * 64 * NV;
   const long bh = (long)b * p.heads + h, bhc = bh * p.chunks + chunk;
   const int rows = p.t - chunk * kChunk < kChunk ? p.t - chunk * kChunk : kChunk;
   const float m_in = p.cg[bhc * 4 + 2];
@@ -332,14 +349,18 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
     nq[lane] = 0.f;
   }
   const long base = ((long)b * p.t + chunk * kChunk) * p.pitch;
-  f32x4 sc[4], acc[4];
+  f32x4 sc[4], acc[4 * NV];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) sc[j] = acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < 4; ++j) sc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4 * NV; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int k0 = 0; k0 < p.dk; k0 += 64) {
     __syncthreads();
     load_tile<T>(qt, kPitchRow, (const S*)p.q + base + (long)h * p.dk + k0, p.pitch, rows, p.dk - k0, p.q_scale);
     load_tile<T>(kt, kPitchRow, (const S*)p.k + base + (long)h * p.dk + k0, p.pitch, rows, p.dk - k0, 1.f);
-    load_tile<F32>(st, kPitchCol, p.cs + bhc * p.dk * p.dv + (long)k0 * p.dv + v0, p.dv, p.dk - k0, p.dv - v0, 1.f);
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      load_tile<F32>(st + n * kBlock, kPitchCol, p.cs + bhc * p.dk * p.dv + (long)k0 * p.dv + v0 + 64 * n, p.dv, p.dk - k0, p.dv - v0 - 64 * n, 1.f);
     if (t < 64) nb[t] = k0 + t < p.dk ? p.cn[bhc * p.dk + k0 + t] : 0.f;
     __syncthreads();
     // (the state product is scaled by the tokens' decay after the loop over k)
@@ -349,7 +370,8 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         sc[j] = mfma_f32(a, kt[(16 * j + i16) * kPitchRow + k + g], sc[j]);
-        acc[j] = mfma_f32(a, st[(k + g) * kPitchCol + 16 * j + i16], acc[j]);
+#pragma unroll
+        for (int n = 0; n < NV; ++n) acc[4 * n + j] = mfma_f32(a, st[n * kBlock + (k + g) * kPitchCol + 16 * j + i16], acc[4 * n + j]);
       }
     }
     {
@@ -362,7 +384,9 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
     }
   }
   __syncthreads();  // the q block turns into the weighted scores, the state block into v
-  load_tile<T>(st, kPitchCol, (const S*)p.v + base + (long)h * p.dv + v0, p.pitch, rows, p.dv - v0, 1.f);
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+    load_tile<T>(st + n * kBlock, kPitchCol, (const S*)p.v + base + (long)h * p.dv + v0 + 64 * n, p.pitch, rows, p.dv - v0 - 64 * n, 1.f);
   float den[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -375,8 +399,9 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
       const float v = s <= tr ? sc[j][r] * expf((float)(fmr + as[s])) : 0.f;
       qt[tr * kPitchRow + s] = v;
       sum += v;
-      acc[j][r] *= inter[tr];
     }
+#pragma unroll
+    for (int j = 0; j < 4 * NV; ++j) acc[j][r] *= inter[tr];
     sum = row16_sum(sum);
     den[r] = fmaxf(fabsf(sum + inter[tr] * nq[tr]), expf(-ms[tr])) + kLstmEps;
   }
@@ -385,7 +410,7 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
   for (int s = 0; s < kChunk; s += 4) {
     const float a = qt[(wave * 16 + i16) * kPitchRow + s + g];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] = mfma_f32(a, st[(s + g) * kPitchCol + 16 * j + i16], acc[j]);
+    for (int j = 0; j < 4 * NV; ++j) acc[j] = mfma_f32(a, st[(j / 4) * kBlock + (s + g) * kPitchCol + 16 * (j % 4) + i16], acc[j]);
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -393,7 +418,7 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
     if (tr >= rows) continue;
     float* orow = p.o + (((long)b * p.t + chunk * kChunk + tr) * p.heads + h) * p.dv;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < 4 * NV; ++j) {
       const int c = v0 + 16 * j + i16;
       if (c < p.dv) orow[c] = acc[j][r] / den[r];
     }
@@ -452,12 +477,16 @@ static int launch_mlstm(hipStream_t s, const MlstmParams& p, bool chunked) {
   }
   const int kts = ceil_div(p.dk, 64), vts = ceil_div(p.dv, 64);
   if ((long)p.heads * kts * vts > 65535 || p.batch > 65535) return MUI_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL((mlstm_chunk_state_kernel<T>), dim3(p.chunks, p.heads * kts * vts, p.batch), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((mlstm_chunk_state_kernel<T>), dim3(p.chunks, p.heads * kts * ceil_div(vts, p.group), p.batch), dim3(256), 0, s, p);
   const long elements = (long)p.dk * p.dv + p.dk;
   hipLaunchKernelGGL(mlstm_scan_kernel, dim3((unsigned)((elements + 255) / 256), p.batch * p.heads), dim3(256), 0, s, p);
   hipLaunchKernelGGL(mlstm_max_kernel, dim3(p.batch * p.heads), dim3(64), 0, s, p);
-  const size_t lds = (size_t)kChunk * (2 * kPitchRow + kPitchCol) * 4;
-  return launch_with_lds(mlstm_chunk_out_kernel<T>, dim3(p.chunks, p.heads * vts, p.batch), dim3(256), lds, s, p);
+  const size_t rows = (size_t)kChunk * 2 * kPitchRow * 4, block = (size_t)kChunk * kPitchCol * 4;
+  // Two neighbouring blocks of value columns share the scores, a third fewer matrix instructions per output, where the grid is more than
+  // a round of workgroups without (three per CU) and no block is empty
+  if (vts % 2 == 0 && (long)p.chunks * p.heads * vts * p.batch > 3L * device_cus())
+    return launch_with_lds(mlstm_chunk_out_kernel<T, 2>, dim3(p.chunks, p.heads * ceil_div(vts, 2), p.batch), dim3(256), rows + 2 * block, s, p);
+  return launch_with_lds(mlstm_chunk_out_kernel<T, 1>, dim3(p.chunks, p.heads * vts, p.batch), dim3(256), rows + block, s, p);
 }
 
 }  // namespace mui
@@ -490,6 +519,9 @@ extern "C" int mui_mlstm(mui_stream_t stream, int dtype, const void* q, const vo
     p.cs = (float*)workspace;
     p.cn = p.cs + units * dk * dv;
     p.cg = p.cn + units * dk;
+    // (at least four workgroups per CU, of which three fit at a time; eight measure the same)
+    const long vts = ceil_div(dv, 64), most = (long)units * ceil_div(dk, 64) * vts / (4L * device_cus());
+    p.group = (int)(most < 1 ? 1 : (most < vts ? most : vts));
   }
   hipStream_t s = (hipStream_t)stream;
   if (dtype == MUI_DTYPE_F16) return launch_mlstm<F16>(s, p, chunked);
