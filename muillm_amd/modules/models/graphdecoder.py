@@ -16,6 +16,7 @@ from typing import Optional
 import torch
 
 from ... import muillm_ext
+from ..._lib import MUI_MAX_TOKENS
 from ..kvcache.cache_utils import MuiCache, _next_pow2
 
 
@@ -56,6 +57,7 @@ class MuiGraphDecoder:
         self.graph = None
         self.graph_multi = None  # STEPS_PER_REPLAY steps in one graph, captured on first use
         self._graph_key = None  # what the captured graph has baked in (see _capture_key)
+        self._linear_ws = None  # scratch of the captured steps' linears: no other decoder, no eager call uses it
         self.cache: Optional[MuiCache] = None
         self.owns_cache = False  # True when prefill() created self.cache itself
         self._window = 0  # sliding window kept in mask4d by every step (0: none)
@@ -159,15 +161,18 @@ class MuiGraphDecoder:
         # warm up on a side stream (allocator, lazy module state), then restore the cache counters and
         # whatever else the step moved on (recurrent state)
         saved = [t.clone() for t in self._step_state()]
+        if self._batch > MUI_MAX_TOKENS and self._linear_ws is None:
+            # (32 rows: down 4096 x 14336 25 us with scratch, which lets it share its K, 33 us without)
+            self._linear_ws = muillm_ext.new_linear_workspace(self.ids.device)
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
+        with torch.cuda.stream(side), muillm_ext.linear_workspace(self._linear_ws):
             self._step()
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         self._restore(saved, seen)
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with torch.cuda.graph(self.graph), muillm_ext.linear_workspace(self._linear_ws):
             self._graph_logits = self._step()  # where every replay leaves its logits
         self.logits = self._graph_logits
         self.graph_multi = None
@@ -181,7 +186,7 @@ class MuiGraphDecoder:
         self.cache.device_length_mode = True  # (prefill switches it off) lengths are read on the device
         seen = self.cache._seen_tokens
         g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
+        with torch.cuda.graph(g), muillm_ext.linear_workspace(self._linear_ws):
             for _ in range(self.STEPS_PER_REPLAY):
                 self._multi_logits = self._step()  # the last step's
         self.graph_multi = g

@@ -18,6 +18,8 @@ CPU fallback for CUDA inputs and no silent one for a missing library.
 
 from __future__ import annotations
 
+import contextlib
+import threading
 from typing import List, Optional, Tuple
 
 import torch
@@ -120,18 +122,39 @@ def _norm_first(x: torch.Tensor, norm_weights: Optional[torch.Tensor], epsilon: 
     return x, norm_weights
 
 
-# Scratch of the prompt GEMM (mui_linear_ws), one per device and stream: calls on one stream follow
-# each other and can share it, calls on different streams may overlap. Zero-filled once.
+# Scratch of the linears beyond MUI_MAX_TOKENS tokens (mui_linear_ws), one per device and stream: calls on one
+# stream follow each other and can share it, calls on different streams may overlap. Zero-filled once.
 _PROMPT_WORKSPACES: dict = {}
+_own_workspace = threading.local()  # .tensor: what linear_workspace() has set for this thread
+
+
+def new_linear_workspace(device) -> torch.Tensor:
+    return torch.zeros(_lib.load().mui_linear_workspace_bytes(), dtype=torch.uint8, device=device)
+
+
+@contextlib.contextmanager
+def linear_workspace(workspace: Optional[torch.Tensor]):
+    """Linears that this thread issues inside use `workspace` (new_linear_workspace; None: the stream's) instead of
+    the scratch of the stream they run on. For calls that are captured into a HIP graph: a graph
+    keeps the address and may be replayed on any stream, so its scratch must be its owner's alone and live as long."""
+    before = getattr(_own_workspace, "tensor", None)
+    _own_workspace.tensor = workspace
+    try:
+        yield
+    finally:
+        _own_workspace.tensor = before
 
 
 def _prompt_workspace(x: torch.Tensor) -> Optional[torch.Tensor]:
+    own = getattr(_own_workspace, "tensor", None)
+    if own is not None and own.device == x.device:
+        return own
     key = (x.device.index, torch.cuda.current_stream(x.device).cuda_stream)
     ws = _PROMPT_WORKSPACES.get(key)
     if ws is None:
         if torch.cuda.is_current_stream_capturing():
             return None  # no allocation inside a capture: the call runs without the workspace
-        ws = torch.zeros(_lib.load().mui_linear_workspace_bytes(), dtype=torch.uint8, device=x.device)
+        ws = new_linear_workspace(x.device)
         _PROMPT_WORKSPACES[key] = ws
     return ws
 
