@@ -149,11 +149,13 @@ def _prompt_workspace(x: torch.Tensor) -> Optional[torch.Tensor]:
     own = getattr(_own_workspace, "tensor", None)
     if own is not None and own.device == x.device:
         return own
+    if torch.cuda.is_current_stream_capturing():
+        # the graph may be replayed on any stream, beside eager calls on this one. Whether the stream has run a linear before
+        # is no rule either: streams come round from a pool, and results would hang on the process's history
+        return None
     key = (x.device.index, torch.cuda.current_stream(x.device).cuda_stream)
     ws = _PROMPT_WORKSPACES.get(key)
     if ws is None:
-        if torch.cuda.is_current_stream_capturing():
-            return None  # no allocation inside a capture: the call runs without the workspace
         ws = new_linear_workspace(x.device)
         _PROMPT_WORKSPACES[key] = ws
     return ws
