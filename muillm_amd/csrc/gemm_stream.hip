@@ -190,7 +190,10 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
     u += (int)gridDim.x;
 #pragma unroll
     for (int r0 = 0; r0 < RT * NT; r0 += MEET) {
-      if (r0 > 0) __builtin_amdgcn_s_barrier();  // the round before has been read
+      if (r0 > 0) {
+        __builtin_amdgcn_s_barrier();  // the round before has been read
+        asm volatile("" ::: "memory");
+      }
       if (multiplies) {
 #pragma unroll
         for (int i = 0; i < RW; ++i)
@@ -263,8 +266,8 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
             }
           }
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
 #pragma unroll
     for (int i = 0; i < RW; ++i)

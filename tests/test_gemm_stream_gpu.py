@@ -65,6 +65,21 @@ def test_linear_against_64_bits(n, k, tokens, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [17, 32, 33, 64, 65, 96])
+@pytest.mark.parametrize("n", [32776, 65000])
+def test_units_that_follow_each_other(n, tokens, dtype):
+    """A workgroup takes several bands of up to 128 rows, each longer than the ring of stages and with more tiles than meet at a
+    time (up to eight rounds): what one round or band leaves in LDS must not reach the next."""
+    k = 2048
+    g = _gen(n + tokens)
+    w, x = _rand((n, k), dtype, g, k ** -0.5), _rand((tokens, k), dtype, g)
+    y = _linear(x, w, k)
+    _assert_within(y, x.double() @ w.double().T, x.double().abs() @ w.double().abs().T, k, dtype)
+    for _ in range(3):
+        assert torch.equal(y, _linear(x, w, k)), "not the same twice"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("tokens", [17, 32, 33, 48, 64])
 @pytest.mark.parametrize("n,k", [(8, 256), (56, 512), (1000, 1024), (16400, 256), (14336, 512)])
 @pytest.mark.parametrize("packed,bias", [(True, False), (False, True)])
