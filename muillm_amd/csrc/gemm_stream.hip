@@ -328,6 +328,26 @@ static int launch_stream_rows(hipStream_t s, const StreamParams& p) {
   return MUI_ERR_UNSUPPORTED;
 }
 
+// Whether the tiled GEMM of longer prompts is faster than linear units of `width` rows x all of K: from 65 tokens on a narrow unit takes longer for its
+// token rows than for its weights, and the tiles read tokens less often. The tiles' time over this kernel's on 250 matrices, 17 to 128 tokens:
+// up to 64 tokens 1.04 to 2, one round of units of 40 rows or more 1.02 to 1.4, and else, by K:
+//   8, 16 rows      65 tokens 1.17 at 1024, 1.0 at 14336; 96 tokens 1.10 at 1024, 1.0 at 4096, 0.93 at 14336; 97 .. 128 tokens 1.03 at 2048, 0.95 at 3072, 0.85 at 28672
+//   24, 32 rows     up to 104 tokens 1.0 to 1.4; 128 tokens 1.2 at 1024, 1.0 at 4096, 0.91 at 28672
+//   several rounds  65 .. 96 tokens 0.86 to 1.05 (28672, 32000 rows), 97 .. 128 tokens 0.81 to 1.05 (28672 to 50304 rows)
+// Of several rounds those stay whose rows are whole multiples of 4 KB apart, which slows the tiles, with a last round that is nearly full: 1.0 to 1.25 where the units
+// are as wide as they can be (40960 to 151936 rows) or the rows a multiple of 8192.
+static bool tiles_are_faster(int tokens, int rows, int k, int width, int rounds) {
+  if (tokens <= 64) return false;
+  const bool most = tokens > 96;
+  if (rounds > 1) {
+    const long full = (long)rounds * device_cus() * width;
+    if (k % 2048 || k > 8192 || width < 64) return true;
+    return most ? rows % 8192 || rounds > 4 || rows * 20L < full * 19 : (width < 96 && rows % 8192) || rows * 5L < full * 4;
+  }
+  if (width <= 16) return most ? k > 2560 : (long)(tokens - 56) * k > 130000;
+  return width <= 32 && tokens > 104 && (long)(tokens - 80) * k > 240000;
+}
+
 template <typename T, int EPI>
 static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
   // Rows per unit and shares of K by the least time: what a CU takes in (27.5 KB of weights, 105 KB of token rows per microsecond, 82 in
@@ -352,6 +372,7 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
       if (width == 0 || cost < best) { best = cost; width = r; p.n_units = units; p.k_splits = k; }
     }
   }
+  if (EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
   switch (width) {
     case 16: return launch_stream_rows<T, EPI, 16>(s, p);
     case 32: return launch_stream_rows<T, EPI, 32>(s, p);
@@ -373,7 +394,8 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
   return MUI_ERR_UNSUPPORTED;
 }
 
-// 17..128 tokens, 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve
+// 17..128 tokens (gate/up ..64), 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve and for
+// what the tiled GEMM does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
   // gate/up beyond 64 tokens: the tiled GEMM (52 against 64 us at 128 tokens and 14336 x 4096)
   if (q.tokens < 1 || q.tokens > (epilogue == SK_GATEUP ? 64 : 128) || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;

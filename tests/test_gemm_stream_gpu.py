@@ -109,3 +109,23 @@ def test_tokens_do_not_mix():
     dirty = _linear(x, w, 1024)
     rest = [t for t in range(33) if t not in (7, 32)]
     assert torch.equal(dirty[rest], clean[rest]) and bool(dirty[7].isnan().all()) and not bool(dirty[32].isfinite().any())
+
+
+@pytest.mark.parametrize("n,k,tokens", [(4096, 14336, 128), (4096, 4096, 97), (2560, 8192, 96), (5120, 10240, 112), (28672, 512, 65), (128256, 256, 128)])
+def test_calls_that_the_tiles_serve(n, k, tokens):
+    """No workspace, or more rows than it can help with: where units of all of K take longer than the tiled GEMM, that
+    runs (bit for bit what it gives by itself)."""
+    g = _gen(n + k + tokens)
+    w, x = _rand((n, k), torch.bfloat16, g, k ** -0.5), _rand((tokens, k), torch.bfloat16, g)
+    got = _linear(x, w, k)
+    lib = _lib.load()
+    _lib.check(lib.mui_tune_prefill(0, -1), "mui_tune_prefill")
+    try:
+        tiles = _linear(x, w, k)
+    finally:
+        _lib.check(lib.mui_tune_prefill(0, 0), "mui_tune_prefill")
+    assert torch.equal(got, tiles)
+    if n == 4096:
+        ws = torch.zeros(lib.mui_linear_workspace_bytes(), dtype=torch.uint8, device=DEV)
+        _assert_within(_linear(x, w, k, ws=ws), x.double() @ w.double().T, x.double().abs() @ w.double().abs().T, k, torch.bfloat16)
+        assert int(ws.count_nonzero()) > 0, "K is shared where there is a workspace"
