@@ -83,6 +83,12 @@ int mui_tune_skinny(int min_tokens, int stream_b, int multi_max_tokens);
  * instead of the LDS-tiled one (0 restores the built-in choice; at most 128; negative: never) */
 int mui_tune_prefill(int tile, int wide_max_tokens);
 
+/* The kernel that streams 16-bit weights for 17..128 tokens: weight rows per unit (8, 16, 24, 32, 40, 48, 56, 64, 96 or 128; gate and up
+ * rows together 16, 32, 48, 64, 96 or 112) and shares of K (1..8; more than one needs a workspace). 0 restores the built-in
+ * choice. A pair that does not exist for a call (too wide for its tokens, more units than CUs, less than 512 k-values a
+ * share) makes the call return MUI_ERR_INVALID_ARG. */
+int mui_tune_stream(int rows_per_unit, int shares);
+
 /* Prompt attention (mui_prefill_attention): fewest query tokens that take the kernel sharing each
  * K/V block between all query heads of a KV head (0 = built-in choice, negative = never);
  * 1000000 + n: the same as n, and that kernel stages its K/V rows through registers instead of

@@ -144,6 +144,7 @@ _SIGNATURES = {
     "mui_tune_int8_quad": (c_int, [c_int, c_int, c_int, c_int]),
     "mui_tune_skinny": (c_int, [c_int, c_int, c_int]),
     "mui_tune_prefill": (c_int, [c_int, c_int]),
+    "mui_tune_stream": (c_int, [c_int, c_int]),
     "mui_tune_prefill_attention": (c_int, [c_int]),
     "mui_tune_warm": (c_int, [c_int, c_int, c_int]),
     "mui_probe_chain_flag_bytes": (ctypes.c_size_t, [c_int]),

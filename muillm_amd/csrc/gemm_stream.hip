@@ -348,6 +348,8 @@ static bool tiles_are_faster(int tokens, int rows, int k, int width, int rounds)
   return width <= 32 && tokens > 104 && (long)(tokens - 80) * k > 240000;
 }
 
+static int g_stream_rows = 0, g_stream_shares = 0;  // mui_tune_stream
+
 template <typename T, int EPI>
 static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
   // Rows per unit and shares of K by the least time: what a CU takes in (27.5 KB of weights, 105 KB of token rows per microsecond, 82 in
@@ -362,17 +364,20 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
   int width = 0;
   for (int c = 0; c < tried; ++c) {
     const int r = EPI == SK_GATEUP ? kGateup[c] : kLinear[c];
-    if (r > stream_widest(nt)) continue;
+    if (r > stream_widest(nt) || (g_stream_rows && r != g_stream_rows)) continue;
     const int units = ceil_div(rows, r);
     for (int k = 1; k <= 8; ++k) {
       if (k > 1 && ((long)units * k > cus || (size_t)k * p.tokens * p.n * 4 > part_bytes || p.k / 256 < 2 * k)) break;
+      if (g_stream_shares && k != g_stream_shares) continue;
       const float one = (float)p.k / k * 2.f * ((float)r / 27.5e3f + 16.f * nt / (nt > 4 ? 82e3f : 105e3f));
       const float barriers = (float)p.k / k / (r + 16 * nt <= 96 ? 256 : 128) * 0.08f;
       const float cost = ceil_div(units, cus) * (one + barriers + 1.f) + (k > 1 ? 2.5f + 0.3f * k + (float)k * p.tokens * p.n * 8.f / 4e6f : 0.f);
       if (width == 0 || cost < best) { best = cost; width = r; p.n_units = units; p.k_splits = k; }
     }
   }
-  if (EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
+  const bool forced = g_stream_rows || g_stream_shares;
+  if (forced && !width) return MUI_ERR_INVALID_ARG;
+  if (!forced && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
   switch (width) {
     case 16: return launch_stream_rows<T, EPI, 16>(s, p);
     case 32: return launch_stream_rows<T, EPI, 32>(s, p);
@@ -412,3 +417,10 @@ int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParam
 
 }  // namespace mui
 
+extern "C" int mui_tune_stream(int rows_per_unit, int shares) {
+  MUI_TUNE_GUARD();
+  if (rows_per_unit < 0 || rows_per_unit > 128 || shares < 0 || shares > 8) return MUI_ERR_INVALID_ARG;
+  mui::g_stream_rows = rows_per_unit;
+  mui::g_stream_shares = shares;
+  return MUI_OK;
+}

@@ -100,6 +100,54 @@ def test_gateup_against_64_bits(n, k, tokens, packed, bias, dtype):
     _assert_within(h, gv * torch.sigmoid(gv) * uv, size, k, dtype)
 
 
+LINEAR_ROWS = [8, 16, 24, 32, 40, 48, 56, 64, 96, 128]
+GATEUP_ROWS = [16, 32, 48, 64, 96, 112]
+TOKENS = [17, 32, 33, 64, 65, 96, 97, 128]  # the first and last of every number of token tiles
+
+
+def _widest(tokens):
+    tiles = 2 if tokens <= 32 else 4 if tokens <= 64 else 6 if tokens <= 96 else 8
+    return min(128, 192 - 16 * tiles)
+
+
+@pytest.fixture
+def forced():
+    lib = _lib.load()
+    yield lambda rows, shares: _lib.check(lib.mui_tune_stream(rows, shares), "mui_tune_stream")
+    _lib.check(lib.mui_tune_stream(0, 0), "mui_tune_stream")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,tokens", [(r, t) for r in LINEAR_ROWS for t in TOKENS if r <= _widest(t)])
+def test_every_linear_unit(rows, tokens, dtype, forced):
+    """Every width with every number of token tiles: one step, a ring of stages that goes round several times, a last unit of eight rows;
+    several units per workgroup; shares of K of different lengths."""
+    g = _gen(rows + tokens)
+    ws = torch.zeros(_lib.load().mui_linear_workspace_bytes(), dtype=torch.uint8, device=DEV)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for n, k, shares in [(rows + 8, 256, 1), (3 * rows + 8, 3328, 1), ((cus + 1) * rows + 8, 512, 1), (2 * rows + 8, 1792, 3), (5 * rows, 4352, 8)]:
+        w, x, res = _rand((n, k), dtype, g, k ** -0.5), _rand((tokens, k), dtype, g), _rand((tokens, n), dtype, g)
+        forced(rows, shares)
+        got = _linear(x, w, k, res=res, ws=ws)
+        _assert_within(got, x.double() @ w.double().T + res.double(), x.double().abs() @ w.double().abs().T + res.double().abs(), k, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,tokens", [(r, t) for r in GATEUP_ROWS for t in TOKENS if t <= 64])
+def test_every_gateup_unit(rows, tokens, dtype, forced):
+    g = _gen(rows + tokens)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for n, k in [(rows // 2 + 8, 256), (rows + 8, 3328), ((cus + 1) * rows // 2 + 8, 512)]:
+        w, x = _rand((2, n, k), dtype, g, k ** -0.5), _rand((tokens, k), dtype, g)
+        h = torch.full((tokens, n), float("nan"), dtype=dtype, device=DEV)
+        forced(rows, 1)
+        _lib.check(_lib.load().mui_gateup_silu(torch.cuda.current_stream().cuda_stream, CODE[dtype], w[0].data_ptr(), w[1].data_ptr(), k,
+                                               x.data_ptr(), None, 0.0, h.data_ptr(), n, k, tokens), "mui_gateup_silu")
+        gv, uv = (x.double() @ m.double().T for m in w)
+        sg, su = (x.double().abs() @ m.double().abs().T for m in w)
+        _assert_within(h, gv * torch.sigmoid(gv) * uv, 1.1 * sg * uv.abs() + gv.abs() * su + gv.abs() * uv.abs(), k, dtype)
+
+
 def test_tokens_do_not_mix():
     """What one token holds, infinities and NaN among it, stays with it."""
     g = _gen(3)
