@@ -52,10 +52,11 @@ struct StreamShape {
   static constexpr int FULL = INSTR - (Q - 1) * kStreamWaves;      // waves that have Q of them, the others Q - 1
   static constexpr int STAGE = (ROWS + 16 * NT) * KS * 2;
   static constexpr int MEET = RT * NT < 16 / KSH ? RT * NT : 16 / KSH;  // tiles that meet at a time (KSH KB each)
-  static constexpr int PAD = ROWS % 16 ? 4096 : 0;                 // a half tile's other half, behind the last stage
-  static constexpr int FIT = (160 * 1024 - MEET * KSH * 1024 - PAD) / STAGE;
+  static constexpr int FIT = (160 * 1024 - MEET * KSH * 1024) / STAGE;
   static constexpr int S = FIT < 8 ? FIT : 8;
-  static constexpr int LDS = S * STAGE + PAD + MEET * KSH * 1024;
+  static constexpr int LDS = S * STAGE + MEET * KSH * 1024;
+  // row tiles read past the weights' rows (a half tile's other half, a last row group's spare tile) read token rows of the stage
+  static_assert(GR * RW * 16 <= ROWS + 16 * NT, "a wave's rows lie in its stage");
   static_assert(S >= 3 && (S - 2) * Q <= 63 && ROWS % 8 == 0 && TW * GT == NT && GR >= 1, "shape");
 };
 
@@ -87,7 +88,7 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
   constexpr int ROW_BYTES = KS * 2;
   const int t = threadIdx.x, lane = t & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  f32x4* meet = (f32x4*)(st_smem + S * G::STAGE + G::PAD);
+  f32x4* meet = (f32x4*)(st_smem + S * G::STAGE);
 
   // this lane's place in a load instruction: row lr of RPI, chunk ls. Chunk c of row r lives in slot c ^ (r % 16) (16 rows
   // read at one chunk fall into 16 different bank groups); the row's upper bits come with the instruction.
