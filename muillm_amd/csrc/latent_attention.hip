@@ -819,12 +819,20 @@ static int launch_latent_decode(hipStream_t s, const LatentParams& p) {
                          (size_t)p.kv_rank * 4, s, p);
 }
 
+constexpr int kMaxGridRows = 65535;
+
 template <typename T, int DKC, int DVT, int NW>
-static int launch_latent_prefill_w(hipStream_t s, const LatentParams& p) {
+static int launch_latent_prefill_w(hipStream_t s, LatentParams p) {
   const int tiles = ceil_div(p.t, 32 * NW);
-  if (tiles > 65535 || p.batch > 65535) return MUI_ERR_UNSUPPORTED;
-  return launch_with_lds(latent_prefill_kernel<T, DKC, DVT, NW>, dim3(p.heads, tiles, p.batch), dim3(64 * NW),
-                         latent_prefill_lds<DKC, DVT, NW>(), s, p);
+  if (tiles > 65535) return MUI_ERR_UNSUPPORTED;
+  for (int left = p.batch; left > 0; left -= kMaxGridRows) {  // a launch holds so many rows
+    const int st = launch_with_lds(latent_prefill_kernel<T, DKC, DVT, NW>, dim3(p.heads, tiles, left < kMaxGridRows ? left : kMaxGridRows),
+                                   dim3(64 * NW), latent_prefill_lds<DKC, DVT, NW>(), s, p);
+    if (st != MUI_OK) return st;
+    p.b0 += kMaxGridRows;
+    p.kv = (const uint16_t*)p.kv + kMaxGridRows * p.kv_batch;
+  }
+  return MUI_OK;
 }
 
 template <typename T, int DKC, int DVT>

@@ -28,3 +28,15 @@ def test_one_launch_is_the_rows_one_at_a_time(batch, t, q_first, window, heads, 
                                               (dim + rot) ** -0.5, window)
         got = ops.latent_prefill_attention(q, cos_sin, kv, first, r, starts, q_first, heads, dim, vdim, (dim + rot) ** -0.5, window)
         assert torch.equal(got, listed) and torch.equal(got, apart)
+
+
+def test_more_rows_than_a_launch_holds():
+    """The grid's third dimension ends at 65535."""
+    batch, t, heads, dim, rot, vdim, cut = 65535 + 3, 17, 1, 6, 2, 10, 65535
+    g = torch.Generator(device=DEV).manual_seed(1)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.float16)  # noqa: E731
+    q, kv, r = rand(batch, t, heads * (dim + rot)), rand(batch, t, heads * (dim + vdim)), rand(batch, t, rot)
+    cos_sin, starts = torch.randn(batch * t, rot, generator=g, device=DEV), torch.arange(batch, device=DEV) % t
+    call = lambda a, b: ops.latent_prefill_attention(q[a:b], cos_sin[a * t:b * t], kv[a:b], 0, r[a:b].clone(), starts[a:b], 0,  # noqa: E731
+                                                     heads, dim, vdim, (dim + rot) ** -0.5, 0)
+    assert torch.equal(call(0, batch), torch.cat([call(0, 40000), call(40000, cut - 1), call(cut - 1, batch - 1), call(batch - 1, batch)]))
