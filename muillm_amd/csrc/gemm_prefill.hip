@@ -995,8 +995,9 @@ size_t prefill_workspace_bytes() { return kXsCounterBytes + kXsMaxWorkgroups * k
 // shares of K per 128 x 128 tile worth taking, or 0: the grid of whole tiles leaves at least three
 // quarters of the CUs idle and every share keeps at least twelve k-steps of 128 -- the exchange
 // (write-through of the partial tile, the counter, the last workgroup's reads) costs 10-15 us, so
-// it pays on long rows only. Measured on MI355X: down 4096 x 14336 at 64 tokens 59 -> 44 us, at 256
-// tokens 109 -> 57 us (8 and 4 shares); o_proj 4096 x 4096 at 64 tokens would go 20 -> 31 us.
+// it pays on long rows only. gemm_stream.hip has the 17 to 128 tokens of rows whose K is a multiple of 256; what comes here
+// is longer, or a K like 14344. Measured on MI355X: 4096 x 14336 at 192 and 256 tokens 68 -> 61 us, 4096 x 14344 at 64 tokens
+// 62 -> 51 us, at 128 61 -> 55 us (8 shares, 4 beyond 128 tokens); 1000 x 6152 is below the line's gain (29 -> 31 us at 64 tokens).
 static int xs_shares(const PrefillGemmParams& p) {
   const long tiles = (long)ceil_div(p.n, 128) * ceil_div(p.tokens, 128);
   const long cus = device_cus();
@@ -1240,7 +1241,7 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
     if (st != MUI_ERR_UNSUPPORTED) return st;
   }
   // a caller-provided workspace lets a long K be shared between workgroups when the tiles are few
-  // (in front of the 16-rows-per-workgroup kernel only for K beyond 8192: down at 33 tokens 31 vs 50 us)
+  // (in front of the 16-rows-per-workgroup kernel only for K beyond 8192: 4096 x 14344 at 33 tokens 49 vs 57 us, at 17 tokens 49 vs 40)
   const bool wide_default = q.tokens <= 40 && epilogue == SK_LINEAR && ceil_div(q.n, 16) <= device_cus();
   const bool wide = g_wide_max_tokens == kWideDefaultMaxTokens ? wide_default : q.tokens <= g_wide_max_tokens;
   if (q.workspace && g_prefill_tile == 0 && g_wide_max_tokens == kWideDefaultMaxTokens && wf == WF_16BIT &&

@@ -60,3 +60,27 @@ def test_linear_workspace_entry_shares_k_between_workgroups(tokens, n, k, dtype)
     assert torch.equal(small, plain)
     assert lib.mui_linear_ws(s, code, wd.data_ptr(), k, xd.data_ptr(), None, 0.0, None, bd.data_ptr(), rd.data_ptr(),
                              small.data_ptr(), n, k, tokens, None, 4096) == -1
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens,n,k", [(17, 4096, 14344), (33, 1000, 10248), (41, 1000, 6152), (64, 4096, 14344), (96, 1000, 6152),
+                                        (128, 4096, 14344), (128, 1000, 6152), (256, 4096, 14336)])
+def test_tile_exchange_at_a_k_that_steps_do_not_divide(tokens, n, k, dtype):
+    """K no multiple of 256 (or more than 128 tokens): 128 x 128 tiles whose workgroups exchange partial tiles and count themselves in.
+    The scratch behind the counters has been written, the counters are back at zero, and call after call gives the same bits."""
+    lib = _lib.load()
+    g = _gen(tokens + k)
+    w, x, r = _mk((n, k), g, 0.02, dtype=dtype), _mk((tokens, k), g, dtype=dtype), _mk((tokens, n), g, dtype=dtype)
+    ref = oracle.linear(x, w, None, 0.0, None, r)
+    wd, xd, rd = w.to(DEV), x.to(DEV), r.to(DEV)
+    ws = torch.zeros(lib.mui_linear_workspace_bytes(), dtype=torch.uint8, device=DEV)
+    outs = []
+    for _ in range(4):
+        y = torch.zeros(tokens, n, dtype=dtype, device=DEV)
+        _lib.check(lib.mui_linear_ws(torch.cuda.current_stream().cuda_stream, 0 if dtype == torch.float16 else 1, wd.data_ptr(), k, xd.data_ptr(),
+                                     None, 0.0, None, None, rd.data_ptr(), y.data_ptr(), n, k, tokens, ws.data_ptr(), ws.numel()), "mui_linear_ws")
+        assert int(ws[:4096].count_nonzero()) == 0
+        outs.append(y)
+    assert int(ws[4096:].count_nonzero()) > 0, "K was not shared"
+    assert_parity(outs[0], ref, 1e-2, f"tile exchange {tokens}x{n}x{k}")
+    assert all(torch.equal(outs[0], y) for y in outs[1:])
