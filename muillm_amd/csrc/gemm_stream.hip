@@ -246,24 +246,24 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
             if (p.k_splits > 1) {
               *(f32x4*)(p.part + ((long)share_k * p.tokens + tok) * p.n + o) = a;
             } else {
-            float res[4] = {0.f, 0.f, 0.f, 0.f};
-            if (p.residual) {
-              const u32x2 q = ld8(p.residual + (long)tok * p.n + o);
-              res[0] = T::one((uint16_t)(q.x & 0xffffu)); res[1] = T::one((uint16_t)(q.x >> 16));
-              res[2] = T::one((uint16_t)(q.y & 0xffffu)); res[3] = T::one((uint16_t)(q.y >> 16));
-            }
-            float v[4];
+              float res[4] = {0.f, 0.f, 0.f, 0.f};
+              if (p.residual) {
+                const u32x2 q = ld8(p.residual + (long)tok * p.n + o);
+                res[0] = T::one((uint16_t)(q.x & 0xffffu)); res[1] = T::one((uint16_t)(q.x >> 16));
+                res[2] = T::one((uint16_t)(q.y & 0xffffu)); res[3] = T::one((uint16_t)(q.y >> 16));
+              }
+              float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              v[e] = a[e];
-              if (p.mul_bias) v[e] *= T::one(p.mul_bias[o + e]);
-              if (p.add_bias) v[e] += T::one(p.add_bias[o + e]);
-              if (p.residual) v[e] += res[e];
-            }
-            u32x2 pk;
-            pk.x = (uint32_t)T::pack(v[0]) | ((uint32_t)T::pack(v[1]) << 16);
-            pk.y = (uint32_t)T::pack(v[2]) | ((uint32_t)T::pack(v[3]) << 16);
-            *(u32x2*)(p.y + (long)tok * p.n + o) = pk;
+              for (int e = 0; e < 4; ++e) {
+                v[e] = a[e];
+                if (p.mul_bias) v[e] *= T::one(p.mul_bias[o + e]);
+                if (p.add_bias) v[e] += T::one(p.add_bias[o + e]);
+                if (p.residual) v[e] += res[e];
+              }
+              u32x2 pk;
+              pk.x = (uint32_t)T::pack(v[0]) | ((uint32_t)T::pack(v[1]) << 16);
+              pk.y = (uint32_t)T::pack(v[2]) | ((uint32_t)T::pack(v[3]) << 16);
+              *(u32x2*)(p.y + (long)tok * p.n + o) = pk;
             }
           }
         }

@@ -952,9 +952,9 @@ extern "C" int mui_latent_attention(mui_stream_t stream, int dtype, int route, c
 
 extern "C" int mui_latent_prefill_attention_rows(mui_stream_t stream, int dtype, const void* q, const float* cos_sin,
                                                  const void* kv, long kv_batch_stride, int kv_first, int kv_rows, const void* r_cache,
-                                            long r_batch_stride, const int64_t* row_start, float scale, int window,
-                                            int q_first, void* out, int batch_row, int batch, int t, int heads, int dim, int rot_dim,
-                                            int vdim) {
+                                                 long r_batch_stride, const int64_t* row_start, float scale, int window,
+                                                 int q_first, void* out, int batch_row, int batch, int t, int heads, int dim,
+                                                 int rot_dim, int vdim) {
   MUI_CHECK_ARG(q && cos_sin && kv && r_cache && out && batch_row >= 0 && batch > 0 && t > 0 && heads > 0 && dim > 0 && rot_dim >= 0);
   MUI_CHECK_ARG(vdim > 0 && kv_first >= 0 && kv_rows > 0 && q_first >= kv_first && q_first + t == kv_first + kv_rows);
   MUI_CHECK_ARG(kv_first == 0 || (window > 0 && q_first - window + 1 >= kv_first));
