@@ -883,11 +883,17 @@ extern "C" int mui_moe_tile_pairs(int dtype, int tokens, int top, int n_experts,
   if (dtype == MUI_DTYPE_F32 || width % 8 || ff % 8 || n_experts < 1) return 0;
   // 16-pair tiles stream an expert's weights once per tile; from about a dozen pairs per expert on a wide tile
   // is cheaper even half empty. 256-pair tiles of the pipelined kernel cost what their pairs cost (us of both products, 128 / 256
-  // pairs: width 4096, 66 pairs per expert 552 / 551, 111: 628 / 601; width 2048, 75: 232 / 233, 112: 252 / 247); those of the other
-  // kernel (k no multiple of 64), rarely full, about 1.3 times as much as a 128-pair one.
+  // pairs: width 4096, 66 pairs per expert 552 / 551, 111: 628 / 601; width 2048, 75: 232 / 233, 112: 252 / 247), where there are
+  // enough of them for the chip: one tile per expert, gate and up in tiles of 128 rows, on three quarters of the CUs (100 and 110 pairs per
+  // expert: 8 experts of 1408 x 2048, 88 tiles, 53 / 65 and 56 / 66; 8 of 1792 x 4096, 112, 96 / 109 and 100 / 111; 16 of 768 x 2048, 96, 52 / 62 both; 32 of
+  // 512 x 1024, 128, 32 / 37 and 34 / 37; 32 of 768 x 2048, 192, 80 / 81 and 85 / 80; 16 of 1792 x 4096, 224, 150 / 147 and 177 / 150). Those of the other
+  // kernel (k no multiple of 64), rarely full, cost about 1.3 times as much as a 128-pair one.
   const long per = (long)tokens * top / n_experts;
   if (per < 12) return 16;
-  if (width % kMgK == 0 && ff % kMgK == 0) return per < 96 ? 128 : 256;
+  if (width % kMgK == 0 && ff % kMgK == 0) {
+    const bool fill = (long)n_experts * ceil_div(ff, 128) * 4 >= 3L * device_cus();
+    return per < (fill ? 96 : 129) ? 128 : 256;
+  }
   return 13 * ((per + 255) / 256) < 10 * ((per + 127) / 128) ? 256 : 128;
 }
 
