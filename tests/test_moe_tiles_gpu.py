@@ -38,3 +38,31 @@ def test_products_of_uneven_experts(width, ff, dtype):
             ref = act @ down[e].double().T
             err = float((out[rows].double() - ref).abs().max() / ref.abs().max())
             assert err <= REL[dtype], f"expert {e}, {COUNTS[e]} pairs: {err:.2e}"
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("width,ff,experts", [(64, 48, 11), (2048, 520, 20)])  # (gate and up below and above 32 MB: ordinary and non-temporal loads)
+def test_neighbouring_tiles_of_one_expert(width, ff, experts, dtype):
+    """16-pair tiles: experts with one tile and with several, side by side, at the first and the last place."""
+    counts = ([17, 16, 1, 0, 33, 48, 15, 32, 2, 0, 20] + [0] * experts)[:experts]
+    counts[-1] = max(counts[-1], 31)
+    g = torch.Generator().manual_seed(width)
+    tokens = sum(counts)
+    chosen = torch.repeat_interleave(torch.arange(experts), torch.tensor(counts))[torch.randperm(tokens, generator=g)]
+    logits = torch.full((tokens, experts), -4.0).scatter_(1, chosen[:, None], 4.0)
+    x = torch.randn(tokens, width, generator=g).to(dtype).to(DEV)
+    gate, up = (torch.randn(experts, ff, width, generator=g).mul_(width ** -0.5).to(dtype).to(DEV) for _ in range(2))
+    down = torch.randn(experts, width, ff, generator=g).mul_(ff ** -0.5).to(dtype).to(DEV)
+    expert, _, pairs, tiles = ops.moe_route(logits.to(DEV), None, experts, 1, 16)
+    assert torch.equal(expert[:, 0].cpu().long(), chosen)
+    out = ops.moe_experts(x, gate, up, down, 7.0, expert, pairs, tiles, 16)
+    for e in range(experts):
+        rows = (chosen == e).nonzero()[:, 0].to(DEV)
+        if not len(rows):
+            continue
+        xe = x[rows].double()
+        a = (xe @ gate[e].double().T).clamp(max=7.0)
+        u = (xe @ up[e].double().T).clamp(-7.0, 7.0)
+        ref = (a * torch.sigmoid(1.702 * a) * (u + 1.0)).to(dtype).double() @ down[e].double().T
+        err = float((out[rows].double() - ref).abs().max() / ref.abs().max())
+        assert err <= REL[dtype], f"expert {e}, {counts[e]} pairs: {err:.2e}"
