@@ -428,7 +428,7 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
 // ---------------------------------------------------------------------------------------
 // output: one wave per (token, head)
 // ---------------------------------------------------------------------------------------
-template <typename T, bool VEC>  // VEC: dv a multiple of 8, at most 512, 16-byte aligned rows
+template <typename T, bool VEC>  // VEC: dv a multiple of 8, 192 .. 512, 16-byte aligned rows
 __global__ void __launch_bounds__(256) mlstm_output_kernel(const float* o, const typename T::storage* gain,
                                                            const typename T::storage* gate, long gate_pitch, float eps,
                                                            typename T::storage* y, long units, int heads, int dv) {
@@ -536,7 +536,9 @@ extern "C" int mui_mlstm_output(mui_stream_t stream, int dtype, const float* o, 
   const long units = (long)tokens * heads;
   const dim3 grid((unsigned)((units + 3) / 4)), block(256);
   hipStream_t s = (hipStream_t)stream;
-  const bool vec = dv % 8 == 0 && dv <= 512 && gate_pitch % 8 == 0 && aligned16(o) && aligned16(gain) && aligned16(gate) && aligned16(y);
+  // (narrower heads leave the vector form too few lanes: us at 20 and at 8000 tokens of 8 heads, single values / vectors: 64 columns 2.3 / 3.9 and 18 / 36,
+  // 128 2.5 / 2.4 and 28 / 36, 192 2.8 / 2.4 and 39 / 39, 256 3.1 / 2.4 and 48 / 40)
+  const bool vec = dv % 8 == 0 && dv >= 192 && dv <= 512 && gate_pitch % 8 == 0 && aligned16(o) && aligned16(gain) && aligned16(gate) && aligned16(y);
 #define MUI_LAUNCH_OUT(T)                                                                                              \
   hipLaunchKernelGGL((vec ? mlstm_output_kernel<T, true> : mlstm_output_kernel<T, false>), grid, block, 0, s, o,       \
                      (const T::storage*)gain, (const T::storage*)gate, gate_pitch, epsilon, (T::storage*)y, units, heads, dv)

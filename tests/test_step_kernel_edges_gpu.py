@@ -91,3 +91,14 @@ def test_mlstm_output_edges(heads, dv, dtype):
     gate = torch.randn(1, 7, heads * dv + 8, generator=g, device=DEV).to(dtype)[..., 8:]
     ref = _rms(o.double(), 0.02).reshape(1, 7, -1) * gain.double() * torch.sigmoid(gate.double())
     _close(ops.mlstm_output(o, gain, gate, 0.02), ref, REL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,dv", [(8, 24), (8, 64), (3, 128), (5, 184), (5, 192), (2, 200)])
+def test_mlstm_output_of_narrow_heads(heads, dv, dtype):
+    """Both sides of the width from which a lane holds eight values."""
+    g = _gen(dv)
+    o, gain = torch.randn(2, 300, heads, dv, generator=g, device=DEV), (1 + 0.2 * torch.randn(heads * dv, generator=g, device=DEV)).to(dtype)
+    gate = torch.randn(2, 300, heads * dv, generator=g, device=DEV).to(dtype)
+    ref = _rms(o.double(), 0.02).reshape(2, 300, -1) * gain.double() * torch.sigmoid(gate.double())
+    _close(ops.mlstm_output(o, gain, gate, 0.02), ref, REL[dtype])
