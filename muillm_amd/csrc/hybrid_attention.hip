@@ -59,8 +59,9 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
   const S* row = (const S*)p.proj + (long)tok * p.pitch;
   const S *qr = row, *kr = row + p.k_off, *vr = row + p.v_off;
   const int nq = p.heads * p.dim, nk = p.kv_heads * p.dim, nv = p.kv_heads * p.vdim;
-  // a thread's first chunk of every part and of its gain is requested before the sums over the workgroup (1 token, 4096 + 1024 +
-  // 1024 columns: 5.4 -> 4.6 us); further chunks are read where they are used
+  // a thread's first chunk of every part and of its gain is requested before the sums over the workgroup; further chunks are read where they
+  // are used, two at a time, in loops of their own (1 token, 4096 + 1024 + 1024 columns 4.0 -> 3.3 us, 20 tokens of 8192 + 1024 + 1024
+  // 6.0 -> 5.4, 6.3 with loops that ask for the first chunk)
   Raw8<T> eq, ek, ev, egq, egk;
   if constexpr (VEC) {
     const int cq = t * 8 < nq ? t * 8 : 0, ck = t * 8 < nk ? t * 8 : 0, cv = t * 8 < nv ? t * 8 : 0;
@@ -81,11 +82,15 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
   auto squares = [&](const S* x, int n, const Raw8<T>& first) {
     float a = 0.f;
     if constexpr (VEC) {
+      float f[8];
+      unpack_raw8<T>(first, f);
+      if (t * 8 < n) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a = fmaf(f[i], f[i], a);
+      }
 #pragma unroll 2
-      for (int c = t * 8; c < n; c += nt * 8) {
-        float f[8];
-        if (c == t * 8) unpack_raw8<T>(first, f);
-        else load8<T>(x + c, f);
+      for (int c = (t + nt) * 8; c < n; c += nt * 8) {
+        load8<T>(x + c, f);
 #pragma unroll
         for (int i = 0; i < 8; ++i) a = fmaf(f[i], f[i], a);
       }
@@ -112,14 +117,8 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
   const float rq = p.q_gain ? rsqrtf(sq / (float)nq + p.eps) : 1.f, rk = p.k_gain ? rsqrtf(sk / (float)nk + p.eps) : 1.f;
   auto emit = [&](const S* x, const S* gain, float rs, int n, S* dst, const Raw8<T>& first, const Raw8<T>& first_gain) {
     if constexpr (VEC) {
-#pragma unroll 2
-      for (int c = t * 8; c < n; c += nt * 8) {
-        float f[8], g[8];
-        if (c == t * 8) unpack_raw8<T>(first, f);
-        else load8<T>(x + c, f);
+      auto turn = [&](int c, float (&f)[8], float (&g)[8]) {
         if (gain) {
-          if (c == t * 8) unpack_raw8<T>(first_gain, g);
-          else load8<T>(gain + c, g);
 #pragma unroll
           for (int i = 0; i < 8; ++i) f[i] = g[i] * (f[i] * rs);
         }
@@ -131,6 +130,18 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
           g[2 * i + 1] = v * co + u * si;
         }
         store8<T>(dst + c, g);
+      };
+      float f[8], g[8];
+      if (t * 8 < n) {
+        unpack_raw8<T>(first, f);
+        if (gain) unpack_raw8<T>(first_gain, g);
+        turn(t * 8, f, g);
+      }
+#pragma unroll 2
+      for (int c = (t + nt) * 8; c < n; c += nt * 8) {
+        load8<T>(x + c, f);
+        if (gain) load8<T>(gain + c, g);
+        turn(c, f, g);
       }
     } else {
       for (int c = t; c < n; c += nt) {
@@ -151,10 +162,13 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
   emit(kr, (const S*)p.k_gain, rk, nk, (S*)p.k_cache + b * p.k_batch + slot * nk, ek, egk);
   S* vd = (S*)p.v_cache + b * p.v_batch + slot * nv;
   if constexpr (VEC) {
-    for (int c = t * 8; c < nv; c += nt * 8) {
-      float f[8];
-      if (c == t * 8) unpack_raw8<T>(ev, f);
-      else load8<T>(vr + c, f);
+    float f[8];
+    if (t * 8 < nv) {
+      unpack_raw8<T>(ev, f);
+      store8<T>(vd + t * 8, f);
+    }
+    for (int c = (t + nt) * 8; c < nv; c += nt * 8) {
+      load8<T>(vr + c, f);
       store8<T>(vd + c, f);
     }
   } else {

@@ -102,3 +102,27 @@ def test_mlstm_output_of_narrow_heads(heads, dv, dtype):
     gate = torch.randn(2, 300, heads * dv, generator=g, device=DEV).to(dtype)
     ref = _rms(o.double(), 0.02).reshape(2, 300, -1) * gain.double() * torch.sigmoid(gate.double())
     _close(ops.mlstm_output(o, gain, gate, 0.02), ref, REL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,kv_heads", [(4, 1), (32, 8), (33, 3), (66, 33), (97, 97)])
+def test_hybrid_prepare_wide_rows(heads, kv_heads, dtype):
+    """Rows of less than a round of 512 chunks, of exactly one, and of up to three, with a ragged last one."""
+    g, dim, rot, t = _gen(heads), 128, 32, 3
+    nq, nk = heads * dim, kv_heads * dim
+    proj = torch.randn(1, t, nq + 2 * nk, generator=g, device=DEV).to(dtype)
+    qg, kg = ((1 + 0.2 * torch.randn(n, generator=g, device=DEV)).to(dtype) for n in (nq, nk))
+    freq = 100.0 ** (-torch.arange(rot // 2, dtype=torch.float64, device=DEV) * 2 / rot)
+    kc, vc = (torch.zeros(1, t + 6, nk, dtype=dtype, device=DEV) for _ in range(2))
+    q = ops.hybrid_prepare(proj, heads, kv_heads, dim, dim, qg, kg, 0.1, freq, torch.arange(5, 5 + t, device=DEV), None, kc, vc)
+
+    def turned(x, gain, n):
+        x = (_rms(x.double(), 0.1) * gain.double()).reshape(t, n, dim // 2, 2)
+        angle = torch.zeros(t, dim // 2, dtype=torch.float64, device=DEV)
+        angle[:, :rot // 2] = torch.arange(5, 5 + t, device=DEV).double()[:, None] * freq
+        c, s = angle.cos()[:, None], angle.sin()[:, None]
+        return torch.stack([x[..., 0] * c - x[..., 1] * s, x[..., 1] * c + x[..., 0] * s], -1).reshape(t, -1)
+
+    _close(q[0], turned(proj[0, :, :nq], qg, heads), REL[dtype])
+    _close(kc[0, 5:5 + t], turned(proj[0, :, nq:nq + nk], kg, kv_heads), REL[dtype])
+    assert torch.equal(vc[0, 5:5 + t], proj[0, :, nq + nk:]) and float(kc[0, :5].abs().max()) == 0
