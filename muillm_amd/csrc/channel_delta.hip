@@ -1070,6 +1070,7 @@ __global__ void __launch_bounds__(256) delta_output_kernel(const DeltaParams p) 
   if (chunk == p.chunks - 1) keep_inputs<T>(p, b, h, t, 256);
   __shared__ __align__(16) uint16_t lds[T::kDtype == MUI_DTYPE_F32 ? 8 : 64 * 128];
   const bool vec = p.rg % 8 == 0 && p.vec, whole = p.dv % 4 == 0;
+  if (tok0 >= p.t && (T::kDtype == MUI_DTYPE_F32 || !vec)) return;  // (otherwise the workgroup loads G2 together)
   const bool live = tok0 + i16 < p.t;
   const int tk = live ? tok0 + i16 : p.t - 1;
   const S* x = (const S*)p.proj + ((long)b * p.t + tk) * p.pitch + p.g_off;
