@@ -506,24 +506,22 @@ __global__ void __launch_bounds__(kDecThreads) latent_decode_kernel(const Latent
 }
 
 // Grid (heads, blocks of 32 value rows, tokens): merges the splits of a head, then Wuv_h times the result;
-// eight lanes per value row
+// eight lanes per value row. The first 64 EARLY columns of a row are requested before the splits are merged: their way from memory is the longer
+// one (us of the whole decode step's attention, 8 heads of rank 128 and 256 at 1 token 12.3 -> 11.2, 14.0 -> 12.2; 128 heads of rank 512 in bf16 at 20 87.0 -> 82.9).
 constexpr int kMaxSplits = 64;
-template <typename T>
+template <typename T, int EARLY>
 __global__ void __launch_bounds__(256) latent_output_kernel(const LatentParams p) {
   __shared__ float ws[kMaxSplits];
   float* o = (float*)la_smem;  // kv_rank
   const int h = blockIdx.x, tok = blockIdx.z, t = threadIdx.x;
   const long at = ((long)tok * p.heads + h) * p.splits;
   const float* part = p.part + at * p.kv_rank;
-  // the value map's row is requested before the splits are merged: its way from memory is the longer one (1 token, 512
-  // columns: 5.6 -> 5.3 us)
   const int v = blockIdx.y * 32 + (t >> 3);
   const int vc = v < p.vdim ? v : p.vdim - 1;
   const uint16_t* w = (const uint16_t*)p.w_uv + ((long)h * p.vdim + vc) * p.kv_rank;
-  constexpr int kEarly = 8;
-  u32x4 early[kEarly];
+  u32x4 early[EARLY ? EARLY : 1];
 #pragma unroll
-  for (int u = 0; u < kEarly; ++u) {
+  for (int u = 0; u < EARLY; ++u) {
     const int c = (t & 7) * 8 + 64 * u;
     early[u] = ld16_stream(w + (c < p.kv_rank ? c : 0));
   }
@@ -552,7 +550,7 @@ __global__ void __launch_bounds__(256) latent_output_kernel(const LatentParams p
   __syncthreads();
   float a = 0.f;
 #pragma unroll
-  for (int u = 0; u < kEarly; ++u) {
+  for (int u = 0; u < EARLY; ++u) {
     const int c = (t & 7) * 8 + 64 * u;
     if (c >= p.kv_rank) break;
     float f[8];
@@ -560,8 +558,9 @@ __global__ void __launch_bounds__(256) latent_output_kernel(const LatentParams p
 #pragma unroll
     for (int i = 0; i < 8; ++i) a = fmaf(f[i], o[c + i], a);
   }
-#pragma unroll 4
-  for (int c = (t & 7) * 8 + 64 * kEarly; c < p.kv_rank; c += 64) {
+  constexpr int kAtOnce = EARLY ? 4 : 8;
+#pragma unroll kAtOnce
+  for (int c = (t & 7) * 8 + 64 * EARLY; c < p.kv_rank; c += 64) {
     float f[8];
     unpack8<T>(ld16_stream(w + c), f);
 #pragma unroll
@@ -815,8 +814,14 @@ static int launch_latent_decode(hipStream_t s, const LatentParams& p) {
                      dim3(256), 0, s, p);
   const int st = p.heads > 16 ? launch_latent_decode_h<T, 2>(s, p) : launch_latent_decode_h<T, 1>(s, p);
   if (st != MUI_OK) return st;
-  return launch_with_lds(latent_output_kernel<T>, dim3(p.heads, ceil_div(p.vdim, 32), tokens), dim3(256),
-                         (size_t)p.kv_rank * 4, s, p);
+  const dim3 grid(p.heads, ceil_div(p.vdim, 32), tokens);
+  const size_t lds = (size_t)p.kv_rank * 4;
+  // in fp16 nothing is gained once several workgroups per CU hide each other's loads (16 heads of rank 512, 64 tokens: 40.5 us early, 38.5 late);
+  // requests behind a row's end are not free either (8 heads of rank 128, 64 tokens, fp16 18.0 -> 19.7 with eight of them)
+  if (T::kDtype == MUI_DTYPE_F16 && (long)grid.x * grid.y * grid.z > 6L * device_cus()) return launch_with_lds(latent_output_kernel<T, 0>, grid, dim3(256), lds, s, p);
+  if (p.kv_rank <= 128) return launch_with_lds(latent_output_kernel<T, 2>, grid, dim3(256), lds, s, p);
+  if (p.kv_rank <= 256) return launch_with_lds(latent_output_kernel<T, 4>, grid, dim3(256), lds, s, p);
+  return launch_with_lds(latent_output_kernel<T, 8>, grid, dim3(256), lds, s, p);
 }
 
 constexpr int kMaxGridRows = 65535;

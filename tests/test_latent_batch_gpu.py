@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+from muillm_amd import _lib
 from muillm_amd import hybrid_ops as ops
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +41,23 @@ def test_more_rows_than_a_launch_holds():
     call = lambda a, b: ops.latent_prefill_attention(q[a:b], cos_sin[a * t:b * t], kv[a:b], 0, r[a:b].clone(), starts[a:b], 0,  # noqa: E731
                                                      heads, dim, vdim, (dim + rot) ** -0.5, 0)
     assert torch.equal(call(0, batch), torch.cat([call(0, 40000), call(40000, cut - 1), call(cut - 1, batch - 1), call(batch - 1, batch)]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kv_rank", [8, 64, 120, 128, 136, 256, 264, 512])
+@pytest.mark.parametrize("tokens", [1, 400])
+def test_value_map_of_decode_steps(kv_rank, tokens, dtype):
+    """Columns of the value map that are requested early, and those behind them, with few and with many workgroups: against the
+    plain kernel on the same values in fp32."""
+    heads, dim, rot, vdim, keys = 5, 16, 8, 40, 9
+    g = torch.Generator(device=DEV).manual_seed(kv_rank + tokens)
+    rand = lambda *s, std=1.0: torch.randn(*s, generator=g, device=DEV).mul_(std).to(dtype)  # noqa: E731
+    q, c, r = rand(tokens, 1, heads * (dim + rot)), rand(tokens, keys, kv_rank), rand(tokens, keys, rot)
+    uk, uv = rand(heads * dim, kv_rank, std=kv_rank ** -0.5), rand(heads * vdim, kv_rank, std=kv_rank ** -0.5)
+    cos_sin, pos = torch.randn(tokens, rot, generator=g, device=DEV), torch.tensor([keys - 1], device=DEV)
+    args = (pos, None, heads, dim, vdim, (dim + rot) ** -0.5, 0)
+    got = ops.latent_attention(q, cos_sin, uk, uv, c, r, *args, _lib.MUI_LATENT_DECODE)
+    ref = ops.latent_attention(q.float(), cos_sin, uk.float(), uv.float(), c.float(), r.float(), *args, _lib.MUI_LATENT_PLAIN)
+    err = float((got.double() - ref.double()).abs().max() / ref.double().abs().max())
+    # rounded to 16 bits: the absorbed query, the probabilities and the output
+    assert err <= {torch.float16: 3.0 * 2.0 ** -10, torch.bfloat16: 3.0 * 2.0 ** -7}[dtype], f"{err:.1e}"
