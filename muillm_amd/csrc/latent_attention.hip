@@ -350,6 +350,7 @@ __device__ __forceinline__ int live_splits(const LatentParams& p, long lo, long 
 //           16 + 4 g + r of 32
 constexpr int kDecKeys = 64, kDecThreads = 512;
 constexpr int kMaxDecodeWidth = 576;  // kv_rank + rot, rounded up to 64
+constexpr int kMaxDecodeRank = 512;   // kv_rank
 template <typename T, int NT, int HT>  // kv_rank <= 128 NT
 __global__ void __launch_bounds__(kDecThreads) latent_decode_kernel(const LatentParams p) {
   constexpr int KG = 2 * NT + 1, HEADS = 16 * HT;  // blocks of 64 columns (kv_rank + rot <= 128 NT + 64)
@@ -558,13 +559,14 @@ __global__ void __launch_bounds__(256) latent_output_kernel(const LatentParams p
 #pragma unroll
     for (int i = 0; i < 8; ++i) a = fmaf(f[i], o[c + i], a);
   }
-  constexpr int kAtOnce = EARLY ? 4 : 8;
-#pragma unroll kAtOnce
-  for (int c = (t & 7) * 8 + 64 * EARLY; c < p.kv_rank; c += 64) {
-    float f[8];
-    unpack8<T>(ld16_stream(w + c), f);
+  if constexpr (EARLY == 0) {
+#pragma unroll 8
+    for (int c = (t & 7) * 8; c < p.kv_rank; c += 64) {
+      float f[8];
+      unpack8<T>(ld16_stream(w + c), f);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) a = fmaf(f[i], o[c + i], a);
+      for (int i = 0; i < 8; ++i) a = fmaf(f[i], o[c + i], a);
+    }
   }
   a += dpp_f32<kDppXor1>(a);
   a += dpp_f32<kDppXor2>(a);
@@ -909,7 +911,7 @@ static void latent_split(int batch, int t, int heads, int span, int* splits, int
 extern "C" int mui_latent_attention_route(int dtype, int tokens, int heads, int dim, int rot_dim, int vdim, int kv_rank) {
   if (dtype == MUI_DTYPE_F32 || kv_rank % 8) return MUI_LATENT_PLAIN;
   if (tokens > MUI_MAX_TOKENS && prefill_covers(dim + rot_dim, vdim)) return MUI_LATENT_PREFILL;
-  return latent_kp(kv_rank, rot_dim) <= kMaxDecodeWidth ? MUI_LATENT_DECODE : MUI_LATENT_PLAIN;
+  return kv_rank <= kMaxDecodeRank && latent_kp(kv_rank, rot_dim) <= kMaxDecodeWidth ? MUI_LATENT_DECODE : MUI_LATENT_PLAIN;
 }
 
 extern "C" size_t mui_latent_decode_scratch_bytes(int batch, int t, int heads, int kv_rank, int rot_dim, int span) {
@@ -941,7 +943,7 @@ extern "C" int mui_latent_attention(mui_stream_t stream, int dtype, int route, c
     return MUI_ERR_INVALID_ARG;
   }
   MUI_CHECK_ARG(route == MUI_LATENT_DECODE && scratch && span > 0);
-  if (kv_rank % 8 || latent_kp(kv_rank, rot_dim) > kMaxDecodeWidth) return MUI_ERR_UNSUPPORTED;
+  if (kv_rank % 8 || kv_rank > kMaxDecodeRank || latent_kp(kv_rank, rot_dim) > kMaxDecodeWidth) return MUI_ERR_UNSUPPORTED;
   if (!aligned16(w_uk) || !aligned16(w_uv) || !aligned16(c_cache) || !aligned16(r_cache) || c_batch_stride % 8 ||
       (rot_dim % 8 == 0 && r_batch_stride % 8) || ((uintptr_t)scratch & 255))
     return MUI_ERR_ALIGNMENT;

@@ -61,3 +61,20 @@ def test_value_map_of_decode_steps(kv_rank, tokens, dtype):
     err = float((got.double() - ref.double()).abs().max() / ref.double().abs().max())
     # rounded to 16 bits: the absorbed query, the probabilities and the output
     assert err <= {torch.float16: 3.0 * 2.0 ** -10, torch.bfloat16: 3.0 * 2.0 ** -7}[dtype], f"{err:.1e}"
+
+
+@pytest.mark.parametrize("kv_rank,rot", [(520, 8), (568, 8), (512, 72)])
+def test_ranks_beyond_the_decode_kernel(kv_rank, rot):
+    heads, dim, vdim, keys, tokens = 3, 16, 40, 9, 4
+    g = torch.Generator(device=DEV).manual_seed(kv_rank)
+    rand = lambda *s, std=1.0: torch.randn(*s, generator=g, device=DEV).mul_(std).to(torch.bfloat16)  # noqa: E731
+    q, c, r = rand(tokens, 1, heads * (dim + rot)), rand(tokens, keys, kv_rank), rand(tokens, keys, rot)
+    uk, uv = rand(heads * dim, kv_rank, std=kv_rank ** -0.5), rand(heads * vdim, kv_rank, std=kv_rank ** -0.5)
+    cos_sin, pos = torch.randn(tokens, rot, generator=g, device=DEV), torch.tensor([keys - 1], device=DEV)
+    args = (pos, None, heads, dim, vdim, (dim + rot) ** -0.5, 0)
+    route = ops.latent_route(torch.bfloat16, 1, heads, dim, rot, vdim, kv_rank)
+    got = ops.latent_attention(q, cos_sin, uk, uv, c, r, *args, route)
+    ref = ops.latent_attention(q.float(), cos_sin, uk.float(), uv.float(), c.float(), r.float(), *args, _lib.MUI_LATENT_PLAIN)
+    assert float((got.double() - ref.double()).abs().max() / ref.double().abs().max()) <= 3.0 * 2.0 ** -7
+    with pytest.raises(_lib.MuiLibraryError):
+        ops.latent_attention(q, cos_sin, uk, uv, c, r, *args, _lib.MUI_LATENT_DECODE)
