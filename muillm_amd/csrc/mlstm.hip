@@ -426,20 +426,22 @@ __global__ void __launch_bounds__(256) mlstm_chunk_out_kernel(const MlstmParams 
 }
 
 // ---------------------------------------------------------------------------------------
-// output: one wave per (token, head)
+// output: one wave per (token, head), or two of them per wave
 // ---------------------------------------------------------------------------------------
-template <typename T, bool VEC>  // VEC: dv a multiple of 8, 192 .. 512, 16-byte aligned rows
+// LANES: lanes per (token, head) where dv is a multiple of 8, 192 .. 8 LANES, and rows are 16-byte aligned; 0: any dv, a value per lane of a wave
+template <typename T, int LANES>
 __global__ void __launch_bounds__(256) mlstm_output_kernel(const float* o, const typename T::storage* gain,
                                                            const typename T::storage* gate, long gate_pitch, float eps,
                                                            typename T::storage* y, long units, int heads, int dv) {
-  const int lane = threadIdx.x & 63;
-  const long u = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  constexpr int PER = LANES ? LANES : 64;
+  const int lane = threadIdx.x % PER;
+  const long u = (long)blockIdx.x * (256 / PER) + threadIdx.x / PER;
   if (u >= units) return;
   const long tok = u / heads;
   const int h = (int)(u - tok * heads);
   const float* src = o + u * dv;
   float ss = 0.f;
-  if constexpr (VEC) {
+  if constexpr (LANES > 0) {
     // eight values per lane, everything requested before the sum over the head (1 row of 8 heads 6.5 -> 2.5 us)
     const int c = lane * 8, cc = c < dv ? c : 0;
     const Raw8<F32> ro = load_raw8<F32>(src + cc);
@@ -450,7 +452,13 @@ __global__ void __launch_bounds__(256) mlstm_output_kernel(const float* o, const
 #pragma unroll
       for (int i = 0; i < 8; ++i) ss = fmaf(f[i], f[i], ss);
     }
-    const float rs = rsqrtf(wave_sum(ss) / (float)dv + eps);
+    if constexpr (LANES == 32) {
+      ss = row16_sum(ss);
+      ss += __shfl_xor(ss, 16);
+    } else {
+      ss = wave_sum(ss);
+    }
+    const float rs = rsqrtf(ss / (float)dv + eps);
     if (c >= dv) return;
     unpack_raw8<T>(rg, g);
     unpack_raw8<T>(rw, w);
@@ -534,14 +542,16 @@ extern "C" int mui_mlstm_output(mui_stream_t stream, int dtype, const float* o, 
                                 long gate_pitch, float epsilon, void* y, int tokens, int heads, int dv) {
   MUI_CHECK_ARG(o && gain && gate && y && tokens > 0 && heads > 0 && dv > 0);
   const long units = (long)tokens * heads;
-  const dim3 grid((unsigned)((units + 3) / 4)), block(256);
   hipStream_t s = (hipStream_t)stream;
   // (narrower heads leave the vector form too few lanes: us at 20 and at 8000 tokens of 8 heads, single values / vectors: 64 columns 2.3 / 3.9 and 18 / 36,
   // 128 2.5 / 2.4 and 28 / 36, 192 2.8 / 2.4 and 39 / 39, 256 3.1 / 2.4 and 48 / 40)
   const bool vec = dv % 8 == 0 && dv >= 192 && dv <= 512 && gate_pitch % 8 == 0 && aligned16(o) && aligned16(gain) && aligned16(gate) && aligned16(y);
+  // (a wave for one head of up to 256 columns leaves half its lanes idle: 2000 tokens of 8 heads of 256 single values 9.5 us, 64 lanes a head 11.1, 32 lanes 7.4)
+  const int lanes = !vec ? 0 : (dv <= 256 ? 32 : 64), per = lanes == 32 ? 8 : 4;
+  const dim3 grid((unsigned)((units + per - 1) / per)), block(256);
 #define MUI_LAUNCH_OUT(T)                                                                                              \
-  hipLaunchKernelGGL((vec ? mlstm_output_kernel<T, true> : mlstm_output_kernel<T, false>), grid, block, 0, s, o,       \
-                     (const T::storage*)gain, (const T::storage*)gate, gate_pitch, epsilon, (T::storage*)y, units, heads, dv)
+  hipLaunchKernelGGL((lanes == 0 ? mlstm_output_kernel<T, 0> : lanes == 32 ? mlstm_output_kernel<T, 32> : mlstm_output_kernel<T, 64>), grid, block, \
+                     0, s, o, (const T::storage*)gain, (const T::storage*)gate, gate_pitch, epsilon, (T::storage*)y, units, heads, dv)
   if (dtype == MUI_DTYPE_F16) MUI_LAUNCH_OUT(F16);
   else if (dtype == MUI_DTYPE_BF16) MUI_LAUNCH_OUT(BF16);
   else if (dtype == MUI_DTYPE_F32) MUI_LAUNCH_OUT(F32);
