@@ -50,7 +50,7 @@ struct HybridAttnParams {
 extern __shared__ __align__(16) unsigned char ha_smem[];
 struct CosSin { float c, s; };
 
-template <typename T, bool VEC>
+template <typename T, bool VEC, bool EARLY>
 __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnParams p) {
   typedef typename T::storage S;
   __shared__ float red[2][8];
@@ -61,9 +61,9 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
   const int nq = p.heads * p.dim, nk = p.kv_heads * p.dim, nv = p.kv_heads * p.vdim;
   // a thread's first chunk of every part and of its gain is requested before the sums over the workgroup; further chunks are read where they
   // are used, two at a time, in loops of their own (1 token, 4096 + 1024 + 1024 columns 4.0 -> 3.3 us, 20 tokens of 8192 + 1024 + 1024
-  // 6.0 -> 5.4, 6.3 with loops that ask for the first chunk)
+  // 6.0 -> 5.4, 6.3 with loops that ask for the first chunk). Not EARLY: no gains, so no sums, and workgroups enough to hide a load
   Raw8<T> eq, ek, ev, egq, egk;
-  if constexpr (VEC) {
+  if constexpr (VEC && EARLY) {
     const int cq = t * 8 < nq ? t * 8 : 0, ck = t * 8 < nk ? t * 8 : 0, cv = t * 8 < nv ? t * 8 : 0;
     eq = load_raw8<T>(qr + cq);
     ek = load_raw8<T>(kr + ck);
@@ -132,13 +132,13 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
         store8<T>(dst + c, g);
       };
       float f[8], g[8];
-      if (t * 8 < n) {
+      if (EARLY && t * 8 < n) {
         unpack_raw8<T>(first, f);
         if (gain) unpack_raw8<T>(first_gain, g);
         turn(t * 8, f, g);
       }
 #pragma unroll 2
-      for (int c = (t + nt) * 8; c < n; c += nt * 8) {
+      for (int c = (EARLY ? t + nt : t) * 8; c < n; c += nt * 8) {
         load8<T>(x + c, f);
         if (gain) load8<T>(gain + c, g);
         turn(c, f, g);
@@ -163,11 +163,11 @@ __global__ void __launch_bounds__(512) hybrid_prepare_kernel(const HybridAttnPar
   S* vd = (S*)p.v_cache + b * p.v_batch + slot * nv;
   if constexpr (VEC) {
     float f[8];
-    if (t * 8 < nv) {
+    if (EARLY && t * 8 < nv) {
       unpack_raw8<T>(ev, f);
       store8<T>(vd + t * 8, f);
     }
-    for (int c = (t + nt) * 8; c < nv; c += nt * 8) {
+    for (int c = (EARLY ? t + nt : t) * 8; c < nv; c += nt * 8) {
       load8<T>(vr + c, f);
       store8<T>(vd + c, f);
     }
@@ -639,8 +639,9 @@ static int launch_hybrid_prepare(hipStream_t s, const HybridAttnParams& p) {
   const int tokens = p.batch * p.t;
   const dim3 grid(tokens), block(tokens <= MUI_MAX_TOKENS ? 512 : 256);
   const size_t lds = (size_t)(p.dim + 1) / 2 * 8;
-  if (vec) return launch_with_lds(hybrid_prepare_kernel<T, true>, grid, block, lds, s, p);
-  return launch_with_lds(hybrid_prepare_kernel<T, false>, grid, block, lds, s, p);
+  if (!vec) return launch_with_lds(hybrid_prepare_kernel<T, false, false>, grid, block, lds, s, p);
+  if (p.q_gain || p.k_gain || tokens <= 4 * device_cus()) return launch_with_lds(hybrid_prepare_kernel<T, true, true>, grid, block, lds, s, p);
+  return launch_with_lds(hybrid_prepare_kernel<T, true, false>, grid, block, lds, s, p);
 }
 
 template <typename T>

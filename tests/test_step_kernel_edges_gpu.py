@@ -104,6 +104,15 @@ def test_mlstm_output_of_narrow_heads(heads, dv, dtype):
     _close(ops.mlstm_output(o, gain, gate, 0.02), ref, REL[dtype])
 
 
+def _turned(x, n, freq):
+    """x [t, n * dim] in slots 5 .., pairs of neighbours turned by their slot's angles"""
+    x = x.reshape(x.shape[0], n, -1, 2)
+    angle = torch.zeros(x.shape[0], x.shape[2], dtype=torch.float64, device=DEV)
+    angle[:, :len(freq)] = torch.arange(5, 5 + x.shape[0], device=DEV).double()[:, None] * freq
+    c, s = angle.cos()[:, None], angle.sin()[:, None]
+    return torch.stack([x[..., 0] * c - x[..., 1] * s, x[..., 1] * c + x[..., 0] * s], -1).reshape(x.shape[0], -1)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("heads,kv_heads", [(4, 1), (32, 8), (33, 3), (66, 33), (97, 97)])
 def test_hybrid_prepare_wide_rows(heads, kv_heads, dtype):
@@ -116,13 +125,22 @@ def test_hybrid_prepare_wide_rows(heads, kv_heads, dtype):
     kc, vc = (torch.zeros(1, t + 6, nk, dtype=dtype, device=DEV) for _ in range(2))
     q = ops.hybrid_prepare(proj, heads, kv_heads, dim, dim, qg, kg, 0.1, freq, torch.arange(5, 5 + t, device=DEV), None, kc, vc)
 
-    def turned(x, gain, n):
-        x = (_rms(x.double(), 0.1) * gain.double()).reshape(t, n, dim // 2, 2)
-        angle = torch.zeros(t, dim // 2, dtype=torch.float64, device=DEV)
-        angle[:, :rot // 2] = torch.arange(5, 5 + t, device=DEV).double()[:, None] * freq
-        c, s = angle.cos()[:, None], angle.sin()[:, None]
-        return torch.stack([x[..., 0] * c - x[..., 1] * s, x[..., 1] * c + x[..., 0] * s], -1).reshape(t, -1)
+    _close(q[0], _turned(_rms(proj[0, :, :nq].double(), 0.1) * qg.double(), heads, freq), REL[dtype])
+    _close(kc[0, 5:5 + t], _turned(_rms(proj[0, :, nq:nq + nk].double(), 0.1) * kg.double(), kv_heads, freq), REL[dtype])
+    assert torch.equal(vc[0, 5:5 + t], proj[0, :, nq + nk:]) and float(kc[0, :5].abs().max()) == 0
 
-    _close(q[0], turned(proj[0, :, :nq], qg, heads), REL[dtype])
-    _close(kc[0, 5:5 + t], turned(proj[0, :, nq:nq + nk], kg, kv_heads), REL[dtype])
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,kv_heads", [(8, 2), (33, 3)])
+@pytest.mark.parametrize("t", [1024, 1025])
+def test_hybrid_prepare_without_gains(t, heads, kv_heads, dtype):
+    """Both sides of the number of tokens from which nothing is requested early (256 CUs), with and without a second round of chunks."""
+    g, dim, rot = _gen(heads), 128, 32
+    nq, nk = heads * dim, kv_heads * dim
+    proj = torch.randn(1, t, nq + 2 * nk, generator=g, device=DEV).to(dtype)
+    freq = 100.0 ** (-torch.arange(rot // 2, dtype=torch.float64, device=DEV) * 2 / rot)
+    kc, vc = (torch.zeros(1, t + 6, nk, dtype=dtype, device=DEV) for _ in range(2))
+    q = ops.hybrid_prepare(proj, heads, kv_heads, dim, dim, None, None, 0.1, freq, torch.arange(5, 5 + t, device=DEV), None, kc, vc)
+    _close(q[0], _turned(proj[0, :, :nq].double(), heads, freq), REL[dtype])
+    _close(kc[0, 5:5 + t], _turned(proj[0, :, nq:nq + nk].double(), kv_heads, freq), REL[dtype])
     assert torch.equal(vc[0, 5:5 + t], proj[0, :, nq + nk:]) and float(kc[0, :5].abs().max()) == 0
