@@ -44,6 +44,19 @@ def test_moe_residual_norm_edges(rows, top, k, dtype):
     _close(h, _rms(ref, 1e-3) * gn.double(), REL[dtype])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("following", [True, False])
+@pytest.mark.parametrize("k", [2048, 2056, 4104, 8192, 8200])
+def test_residual_norm_without_a_first_norm(k, following, dtype):
+    g = _gen(k)
+    x, y = torch.randn(3, k, generator=g, device=DEV), torch.randn(3, k, generator=g, device=DEV).to(dtype)
+    gain = (1 + 0.2 * torch.randn(k, generator=g, device=DEV)).to(dtype) if following else None
+    ref = x.double() + 0.5 * y.double()
+    out, h = ops.residual_norm(x, y, None, gain, 1e-3, y_scale=0.5, emit=True)
+    _close(out, ref, 3e-6)
+    _close(h, _rms(ref, 1e-3) * gain.double() if following else ref, REL[dtype])
+
+
 @pytest.mark.parametrize("tokens,top,experts,identity", [(1, 8, 64, 8), (8, 8, 64, 8), (13, 5, 64, 8), (64, 1, 3, 1), (32, 2, 2, 0), (65, 1, 7, 1)])
 @pytest.mark.parametrize("skew", [0.0, 30.0])
 def test_grouping_of_few_pairs(tokens, top, experts, identity, skew):
