@@ -46,7 +46,7 @@ __device__ __forceinline__ float rn_block_sum(float v, float* red) {
 // so both gains are requested with the row where registers allow (CH <= 4): 1 row of 4096 5.5 -> 3.9 us. FEW (experts, up to
 // eight per token): so are all chosen experts' rows, before it is known which of them are identity experts -- their rows are
 // read and not used --: 7.8 -> 5.2 us.
-constexpr int kRnFewRows = 256, kRnFewTop = 8;
+constexpr int kRnFewRows = 256, kRnFewLeast = 5, kRnFewTop = 8;
 // The arguments are scalars, the ones of the first loads first: the first sixteen dwords are in registers when a wave starts, a
 // struct is fetched from memory before anything else can be.
 template <typename T, int CH, bool MOE, bool EARLY, bool FEW = false>
@@ -276,8 +276,10 @@ static int launch_residual_norm(hipStream_t s, const ResidualNormParams& p, int 
       return launch_status();
     };
     if constexpr (MOE) {
-      // a row per CU at most: nothing but the chain of one row's loads; more rows read only what they need
-      if (rows <= kRnFewRows && p.top <= kRnFewTop && ch <= 2)
+      // A row per CU at most: nothing but the chain of one row's loads; more rows read only what they need. Up to four experts' rows are requested together anyway (256
+      // rows of 4096, 4 experts, bf16 5.45 us so, 5.64 with FEW). In fp32, twice the bytes, short rows gain nothing (64 of 1024, 8 experts 3.9 / 4.1) and
+      // many long ones lose (256 of 4096 9.2 / 9.9, 200 7.3 / 7.1).
+      if (rows <= kRnFewRows && p.top >= kRnFewLeast && p.top <= kRnFewTop && ch <= 2 && (T::kDtype != MUI_DTYPE_F32 || (p.k > 1024 && (long)rows * p.k <= 200L * 4096)))
         return ch <= 1 ? launch(residual_norm_vec_kernel<T, 1, true, true, true>) : launch(residual_norm_vec_kernel<T, 2, true, true, true>);
     }
     // without a first norm the gain of the second one is all there is to request, behind one sum instead of two, and the wait for the row becomes one for both

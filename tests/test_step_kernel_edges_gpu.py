@@ -26,7 +26,8 @@ def _gen(seed):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("rows,top,k", [(1, 8, 4096), (256, 8, 2048), (257, 8, 2048), (3, 9, 2056), (2, 1, 8), (5, 7, 4104), (2, 8, 4088)])
+@pytest.mark.parametrize("rows,top,k", [(1, 8, 4096), (256, 8, 2048), (257, 8, 2048), (3, 9, 2056), (2, 1, 8), (5, 7, 4104), (2, 8, 4088),
+                                        (3, 4, 4096), (3, 5, 2056), (200, 8, 4096), (201, 8, 4096), (3, 8, 1024), (3, 8, 1032)])
 def test_moe_residual_norm_edges(rows, top, k, dtype):
     g = _gen(rows + top + k)
     n_exp = 5
