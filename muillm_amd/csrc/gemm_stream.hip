@@ -349,6 +349,14 @@ static bool tiles_are_faster(int tokens, int rows, int k, int width, int rounds)
   return width <= 32 && tokens > 104 && (long)(tokens - 80) * k > 240000;
 }
 
+// Whether the 16-rows-per-workgroup kernel (gemm_wide.hip, one round of workgroups, up to 40 tokens) is faster than linear units: a ring of stages pays from a few
+// steps on. Its time over this kernel's, up to 4096 rows: K 256 0.79 to 1.01; K 512 17 to 24 tokens 0.82 to 0.98 up to 2048 rows and 0.94 to 1.05 at 4096, 25 to 32
+// tokens 0.95 to 1.02 and 1.02 to 1.08, 33 tokens 0.99 to 1.10; K 768 and more 0.98 to 1.4.
+static bool wide_is_faster(int tokens, int rows, int k) {
+  if (tokens > 40 || ceil_div(rows, 16) > device_cus()) return false;
+  return k <= 256 || (k <= 512 && tokens <= 32 && rows <= 8 * device_cus());
+}
+
 static int g_stream_rows = 0, g_stream_shares = 0;  // mui_tune_stream
 
 template <typename T, int EPI>
@@ -377,6 +385,7 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
     }
   }
   const bool forced = g_stream_rows || g_stream_shares;
+  if (!forced && EPI == SK_LINEAR && wide_is_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
   if (forced && !width) return MUI_ERR_INVALID_ARG;
   if (!forced && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
   switch (width) {
@@ -401,7 +410,7 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
 }
 
 // 17..128 tokens (gate/up ..64), 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve and for
-// what the tiled GEMM does faster
+// what another kernel does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
   // gate/up beyond 64 tokens: the tiled GEMM (52 against 64 us at 128 tokens and 14336 x 4096)
   if (q.tokens < 1 || q.tokens > (epilogue == SK_GATEUP ? 64 : 128) || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;

@@ -177,3 +177,23 @@ def test_calls_that_the_tiles_serve(n, k, tokens):
         ws = torch.zeros(lib.mui_linear_workspace_bytes(), dtype=torch.uint8, device=DEV)
         _assert_within(_linear(x, w, k, ws=ws), x.double() @ w.double().T, x.double().abs() @ w.double().abs().T, k, torch.bfloat16)
         assert int(ws.count_nonzero()) > 0, "K is shared where there is a workspace"
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("n,k,tokens,wide", [(296, 256, 17, True), (4096, 256, 40, True), (2048, 512, 32, True), (24, 512, 24, True),
+                                             (4104, 256, 17, False), (512, 256, 41, False), (2056, 512, 32, False), (512, 512, 33, False), (512, 768, 17, False)])
+def test_calls_of_one_or_two_steps(n, k, tokens, wide, dtype):
+    """A K of one or two steps, few rows and tokens: 16 rows per workgroup without a ring of stages, bit for bit what that kernel gives by itself
+    (it adds K in another order); on the other side of each line, units."""
+    g = _gen(n + k + tokens)
+    w, x, res = _rand((n, k), dtype, g, k ** -0.5), _rand((tokens, k), dtype, g), _rand((tokens, n), dtype, g)
+    got = _linear(x, w, k, res=res)
+    _assert_within(got, x.double() @ w.double().T + res.double(), x.double().abs() @ w.double().abs().T + res.double().abs(), k, dtype)
+    if wide:
+        lib = _lib.load()
+        _lib.check(lib.mui_tune_prefill(0, 40), "mui_tune_prefill")
+        try:
+            by_itself = _linear(x, w, k, res=res)
+        finally:
+            _lib.check(lib.mui_tune_prefill(0, 0), "mui_tune_prefill")
+        assert torch.equal(got, by_itself)
