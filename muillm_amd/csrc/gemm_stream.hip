@@ -357,6 +357,14 @@ static bool wide_is_faster(int tokens, int rows, int k) {
   return k <= 256 || (k <= 512 && tokens <= 32 && rows <= 8 * device_cus());
 }
 
+// And the tiled GEMM against units of gate and up rows. Both take matrices in rounds, units 112 rows per CU at most, tiles 128: where units need a round more they
+// are slower beyond 32 tokens (their us over the tiles', 33 to 64 tokens: 14400 to 15632 outputs 1.02 to 1.06 at K 1024, 0.90 to 1.11 at 4096, 1.10 to 1.15
+// at 5120 and 8192; 30000 outputs 0.90 to 1.15), else faster (0.63 to 1.02).
+static bool gateup_tiles_are_faster(int tokens, int rows) {
+  const int cus = device_cus();
+  return tokens > 32 && ceil_div(rows, 112 * cus) > ceil_div(rows, 128 * cus);
+}
+
 static int g_stream_rows = 0, g_stream_shares = 0;  // mui_tune_stream
 
 template <typename T, int EPI>
@@ -388,6 +396,7 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
   if (!forced && EPI == SK_LINEAR && wide_is_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
   if (forced && !width) return MUI_ERR_INVALID_ARG;
   if (!forced && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
+  if (!forced && EPI == SK_GATEUP && gateup_tiles_are_faster(p.tokens, rows)) return MUI_ERR_UNSUPPORTED;
   switch (width) {
     case 16: return launch_stream_rows<T, EPI, 16>(s, p);
     case 32: return launch_stream_rows<T, EPI, 32>(s, p);

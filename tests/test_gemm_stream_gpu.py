@@ -197,3 +197,29 @@ def test_calls_of_one_or_two_steps(n, k, tokens, wide, dtype):
         finally:
             _lib.check(lib.mui_tune_prefill(0, 0), "mui_tune_prefill")
         assert torch.equal(got, by_itself)
+
+
+@pytest.mark.parametrize("n,k,tokens,tiles", [(14400, 512, 33, True), (16384, 512, 64, True), (28680, 256, 48, True), (14336, 512, 64, False), (16392, 512, 33, False),
+                                              (14400, 512, 32, False)])
+def test_gateup_calls_that_the_tiles_serve(n, k, tokens, tiles):
+    """Units that need a round more than the tiled GEMM leave the call to it (256 CUs), bit for bit."""
+    g = _gen(n + k + tokens)
+    gate, up = _rand((n, k), torch.bfloat16, g, k ** -0.5), _rand((n, k), torch.bfloat16, g, k ** -0.5)
+    x, lib = _rand((tokens, k), torch.bfloat16, g), _lib.load()
+
+    def run():
+        h = torch.full((tokens, n), float("nan"), dtype=x.dtype, device=DEV)
+        _lib.check(lib.mui_gateup_silu(torch.cuda.current_stream().cuda_stream, CODE[x.dtype], gate.data_ptr(), up.data_ptr(), k,
+                                       x.data_ptr(), None, 0.0, h.data_ptr(), n, k, tokens), "mui_gateup_silu")
+        return h
+
+    got = run()
+    a, b = x.double() @ gate.double().T, x.double() @ up.double().T
+    ref = a * torch.sigmoid(a) * b
+    assert float((got.double() - ref).abs().max() / ref.abs().max()) <= 2.0 ** -8
+    if tiles:
+        _lib.check(lib.mui_tune_prefill(0, -1), "mui_tune_prefill")
+        try:
+            assert torch.equal(got, run())
+        finally:
+            _lib.check(lib.mui_tune_prefill(0, 0), "mui_tune_prefill")
