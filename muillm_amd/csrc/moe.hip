@@ -942,7 +942,9 @@ extern "C" int mui_moe_gateup(mui_stream_t stream, int dtype, const void* gate, 
   p.limit = limit; p.max_tiles = mui_moe_max_tiles(tokens, top, n_experts, tile_pairs);
   // that cache holds 256 MB: the experts of eight layers and more of 32 MB don't stay there. Below (8 experts of 512 x 1024, 17 MB) a model may stay:
   // 4 tokens 4.7 us ordinary, 5.1 non-temporal while it does, 5.5 either way when it does not
-  p.once = (long)n_experts * n_inter * k_in * 4 > (32L << 20);
+  // Rows that are no whole cache lines share one at their ends and where two runs meet: non-temporal it came twice (64 experts of 1000 x 2000, 1 token each
+  // for 32 of them 16.1 us ordinary, 17.8 non-temporal, 100 tokens of 2 137 and 148).
+  p.once = (long)n_experts * n_inter * k_in * 4 > (32L << 20) && k_in % 64 == 0 && (((uintptr_t)gate | (uintptr_t)up) & 127) == 0;
   MUI_BY_DTYPE((launch_moe_product<TT, MOE_GATEUP>((hipStream_t)stream, p, expert, n_experts, tokens * top, tile_pairs)));
 }
 

@@ -41,7 +41,7 @@ def test_products_of_uneven_experts(width, ff, dtype):
 
 
 @pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
-@pytest.mark.parametrize("width,ff,experts", [(64, 48, 11), (2048, 520, 20)])  # (gate and up below and above 32 MB: ordinary and non-temporal loads)
+@pytest.mark.parametrize("width,ff,experts", [(64, 48, 11), (2048, 520, 20), (2008, 520, 20)])  # (gate and up below and above 32 MB, rows of no whole cache lines)
 def test_neighbouring_tiles_of_one_expert(width, ff, experts, dtype):
     """16-pair tiles: experts with one tile and with several, side by side, at the first and the last place."""
     counts = ([17, 16, 1, 0, 33, 48, 15, 32, 2, 0, 20] + [0] * experts)[:experts]
