@@ -895,17 +895,21 @@ extern "C" int mui_linear_f32(mui_stream_t stream, int dtype, const void* weight
 extern "C" int mui_moe_tile_pairs(int dtype, int tokens, int top, int n_experts, int width, int ff) {
   if (dtype == MUI_DTYPE_F32 || width % 8 || ff % 8 || n_experts < 1) return 0;
   // 16-pair tiles stream an expert's weights once per tile; from about a dozen pairs per expert on a wide tile
-  // is cheaper even half empty. 256-pair tiles of the pipelined kernel cost what their pairs cost (us of both products, 128 / 256
-  // pairs: width 4096, 66 pairs per expert 552 / 551, 111: 628 / 601; width 2048, 75: 232 / 233, 112: 252 / 247), where there are
-  // enough of them for the chip: one tile per expert, gate and up in tiles of 128 rows, on three quarters of the CUs (100 and 110 pairs per
-  // expert: 8 experts of 1408 x 2048, 88 tiles, 53 / 65 and 56 / 66; 8 of 1792 x 4096, 112, 96 / 109 and 100 / 111; 16 of 768 x 2048, 96, 52 / 62 both; 32 of
-  // 512 x 1024, 128, 32 / 37 and 34 / 37; 32 of 768 x 2048, 192, 80 / 81 and 85 / 80; 16 of 1792 x 4096, 224, 150 / 147 and 177 / 150). Those of the other
-  // kernel (k no multiple of 64), rarely full, cost about 1.3 times as much as a 128-pair one.
+  // is cheaper even half empty. 256-pair tiles of the pipelined kernel cost what their pairs cost, where there are
+  // enough of them for the chip: one tile per expert, gate and up in tiles of 128 rows and down of 256, on three quarters of the CUs. Below (97, 104, 112 and 120 pairs per
+  // expert, tokens spread evenly, us of both products, 128 / 256 pairs): 8 experts of 1792 x 4096 97 / 109, 112 tiles of down; 16 of 2048 x 1024, 64 tiles,
+  // 51 / 58, 52 / 59, 60 / 60, 53 / 59; 16 of 2048 x 2048, 128, 99 / 104, 101 / 105, 101 / 105, 139 / 106; 32 of 1024 x 1024, 128, 45 / 49, 44 / 49, 45 / 49, 58 / 50.
+  // Above, 128-pair tiles take what an expert has beyond 128 pairs in a tile of its own, which the mean foretells the better the more experts there are:
+  // 64 of 1408 x 2048 279 / 276, 294 / 280, 304 / 282, 320 / 279; 128 of 768 x 2048 274 / 286, 304 / 293, 316 / 297, 328 / 299; 32 of 1024 x 2048 108 / 110, 138 / 112,
+  // 139 / 112, 135 / 113; 24 of 1408 x 2048 123 / 129, 122 / 130, 126 / 132, 128 / 133; and a long K makes up for more: 64 of 1792 x 4096 603 / 593, 614 / 599, 636 / 602,
+  // 687 / 611; 16 of it 165 / 164, 161 / 159, 216 / 157, 236 / 163. Those of the other kernel (k no multiple of 64), rarely full, cost about 1.3 times as much as a
+  // 128-pair one.
   const long per = (long)tokens * top / n_experts;
   if (per < 12) return 16;
   if (width % kMgK == 0 && ff % kMgK == 0) {
-    const bool fill = (long)n_experts * ceil_div(ff, 128) * 4 >= 3L * device_cus();
-    return per < (fill ? 96 : 129) ? 128 : 256;
+    const int gateup = ceil_div(ff, 128), down = ceil_div(width, 256);
+    const bool fill = (long)n_experts * (gateup < down ? gateup : down) * 4 >= 3L * device_cus();
+    return per < (!fill ? 129 : width >= 4096 ? 96 : n_experts >= 32 ? 104 : 120) ? 128 : 256;
   }
   return 13 * ((per + 255) / 256) < 10 * ((per + 127) / 128) ? 256 : 128;
 }
