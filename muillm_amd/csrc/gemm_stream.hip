@@ -357,12 +357,13 @@ static bool wide_is_faster(int tokens, int rows, int k) {
   return k <= 256 || (k <= 512 && tokens <= 32 && rows <= 8 * device_cus());
 }
 
-// And the tiled GEMM against units of gate and up rows. Both take matrices in rounds, units 112 rows per CU at most, tiles 128: where units need a round more they
-// are slower beyond 32 tokens (their us over the tiles', 33 to 64 tokens: 14400 to 15632 outputs 1.02 to 1.06 at K 1024, 0.90 to 1.11 at 4096, 1.10 to 1.15
-// at 5120 and 8192; 30000 outputs 0.90 to 1.15), else faster (0.63 to 1.02).
-static bool gateup_tiles_are_faster(int tokens, int rows) {
+// And the tiled GEMM against units of gate and up rows. Both take matrices in rounds, units 112 rows per CU at most, tiles 128. Where units need a round more they
+// are slower beyond 32 tokens, but for rows that are whole multiples of 4 KB apart, which slows the tiles (us at 33 to 64 tokens, tiles / units: 14400 to 15600 outputs, K 512 12.5 to 14.1 / 12.6 to 14.2, 1024
+// 17.5 to 18.9 / 18.0 to 20.0, 2048 28.8 to 35 / 29 to 31, 4096 48 to 59 / 48 to 55, 5120 57 to 60 / 63 to 69, 8192 87 to 117 / 98 to 106; 30000 outputs, K 512 23 to 24 / 22 to 23, 4096
+// 93 to 114 / 96 to 105, 5120 111 to 125 / 124 to 144, 8192 183 to 222 / 182 to 189); elsewhere units take 0.63 to 1.02 of the tiles' time.
+static bool gateup_tiles_are_faster(int tokens, int rows, int k) {
   const int cus = device_cus();
-  return tokens > 32 && ceil_div(rows, 112 * cus) > ceil_div(rows, 128 * cus);
+  return tokens > 32 && k > 512 && k % 2048 && ceil_div(rows, 112 * cus) > ceil_div(rows, 128 * cus);
 }
 
 static int g_stream_rows = 0, g_stream_shares = 0;  // mui_tune_stream
@@ -396,7 +397,7 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
   if (!forced && EPI == SK_LINEAR && wide_is_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
   if (forced && !width) return MUI_ERR_INVALID_ARG;
   if (!forced && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
-  if (!forced && EPI == SK_GATEUP && gateup_tiles_are_faster(p.tokens, rows)) return MUI_ERR_UNSUPPORTED;
+  if (!forced && EPI == SK_GATEUP && gateup_tiles_are_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
   switch (width) {
     case 16: return launch_stream_rows<T, EPI, 16>(s, p);
     case 32: return launch_stream_rows<T, EPI, 32>(s, p);
@@ -421,7 +422,8 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
 // 17..128 tokens (gate/up ..64), 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve and for
 // what another kernel does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
-  // gate/up beyond 64 tokens: the tiled GEMM (52 against 64 us at 128 tokens and 14336 x 4096)
+  // gate/up beyond 64 tokens: the tiled GEMM. Units of six and eight token tiles are built for linears only; for gate/up they were measured at 128 tokens and
+  // 14336 x 4096 alone (64 us, tiles 52), between 65 and 127 not at all
   if (q.tokens < 1 || q.tokens > (epilogue == SK_GATEUP ? 64 : 128) || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;
   if (q.k % 256 || q.n % 8 || q.n < 8 || q.pitch % 8 || q.pitch > (1L << 26)) return MUI_ERR_UNSUPPORTED;
   if ((((uintptr_t)q.w0 | (uintptr_t)q.w1 | (uintptr_t)q.x) & 15) || (((uintptr_t)q.y | (uintptr_t)q.residual) & 7)) return MUI_ERR_UNSUPPORTED;
