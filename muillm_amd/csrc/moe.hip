@@ -896,20 +896,24 @@ extern "C" int mui_moe_tile_pairs(int dtype, int tokens, int top, int n_experts,
   if (dtype == MUI_DTYPE_F32 || width % 8 || ff % 8 || n_experts < 1) return 0;
   // 16-pair tiles stream an expert's weights once per tile; from about a dozen pairs per expert on a wide tile
   // is cheaper even half empty. 256-pair tiles of the pipelined kernel cost what their pairs cost, where there are
-  // enough of them for the chip: one tile per expert, gate and up in tiles of 128 rows and down of 256, on three quarters of the CUs. Below (97, 104, 112 and 120 pairs per
-  // expert, tokens spread evenly, us of both products, 128 / 256 pairs): 8 experts of 1792 x 4096 97 / 109, 112 tiles of down; 16 of 2048 x 1024, 64 tiles,
-  // 51 / 58, 52 / 59, 60 / 60, 53 / 59; 16 of 2048 x 2048, 128, 99 / 104, 101 / 105, 101 / 105, 139 / 106; 32 of 1024 x 1024, 128, 45 / 49, 44 / 49, 45 / 49, 58 / 50.
-  // Above, 128-pair tiles take what an expert has beyond 128 pairs in a tile of its own, which the mean foretells the better the more experts there are:
-  // 64 of 1408 x 2048 279 / 276, 294 / 280, 304 / 282, 320 / 279; 128 of 768 x 2048 274 / 286, 304 / 293, 316 / 297, 328 / 299; 32 of 1024 x 2048 108 / 110, 138 / 112,
-  // 139 / 112, 135 / 113; 24 of 1408 x 2048 123 / 129, 122 / 130, 126 / 132, 128 / 133; and a long K makes up for more: 64 of 1792 x 4096 603 / 593, 614 / 599, 636 / 602,
-  // 687 / 611; 16 of it 165 / 164, 161 / 159, 216 / 157, 236 / 163. Those of the other kernel (k no multiple of 64), rarely full, cost about 1.3 times as much as a
-  // 128-pair one.
+  // enough of them for the chip (one tile per expert, gate and up in tiles of 128 rows and down of 256). 128-pair tiles take what an expert has beyond 128 pairs in a tile
+  // of its own, which the mean foretells the better the more experts there are. us of both products, 128 / 256 pairs, at 97, 104, 112 and 120 pairs per expert,
+  // tokens spread evenly (two figures: with and without experts beyond 128):
+  //   gate and up on less than three quarters of the CUs: 8 of 1792 x 4096 97 / 109, 16 of 768 x 2048 52 / 62
+  //   down on less than half: 16 of 2048 x 1024 51 / 58, 52 / 59, 60 / 60, 52 and 62 / 60; 16 of 4096 x 1024 123 / 139 to 152, 124 / 139 to 153, 125 / 140 to 154, 141 / 142 to 155
+  //   down on half: 32 of 1024 x 1024 44 / 49, 44 / 49, 44 and 57 / 50, 57 / 51; 32 of 2048 x 1024 108 / 114, 111 and 124 / 116, 112 and 124 / 116, 130 / 117; 16 of
+  //   2048 x 2048 98 / 104, 100 / 105, 101 and 136 / 106, 136 / 107; 64 of 512 x 512 29 / 34, 37 / 35, 38 / 35, 37 / 36; 8 of 4096 x 4096, 125 pairs, 232 to 261 / 194 to 206
+  //   down on three quarters: 24 of 1408 x 2048 123 / 129, 122 / 130, 126 / 132, 128 / 133; 32 of 1024 x 2048 92 to 108 / 99 to 110, 92 to 138 / 100 to 112,
+  //   126 to 139 / 95 to 112, 128 to 135 / 95 to 113; 64 of 1408 x 2048 260 / 261, 265 to 294 / 265 to 280, 291 to 306 / 264 to 282, 303 to 320 / 261 to 279; 128 of 768 x 2048
+  //   274 / 286, 304 / 293, 316 / 297, 328 / 299; and a long K makes up for more: 64 of 1792 x 4096 597 / 591, 609 / 598, 635 / 603, 690 / 611; 16 of it 163 / 164,
+  //   162 / 160, 179 and 216 / 157, 217 / 160.
+  // Those of the other kernel (k no multiple of 64), rarely full, cost about 1.3 times as much as a 128-pair one.
   const long per = (long)tokens * top / n_experts;
   if (per < 12) return 16;
   if (width % kMgK == 0 && ff % kMgK == 0) {
-    const int gateup = ceil_div(ff, 128), down = ceil_div(width, 256);
-    const bool fill = (long)n_experts * (gateup < down ? gateup : down) * 4 >= 3L * device_cus();
-    return per < (!fill ? 129 : width >= 4096 ? 96 : n_experts >= 32 ? 104 : 120) ? 128 : 256;
+    const long cus = device_cus(), gateup = (long)n_experts * ceil_div(ff, 128), down = (long)n_experts * ceil_div(width, 256);
+    const int line = gateup * 4 < cus * 3 || down * 2 < cus ? 129 : down * 4 < cus * 3 ? 108 : width >= 4096 ? 96 : n_experts >= 32 ? 104 : 120;
+    return per < line ? 128 : 256;
   }
   return 13 * ((per + 255) / 256) < 10 * ((per + 127) / 128) ? 256 : 128;
 }
