@@ -217,8 +217,11 @@ struct LowRankHeld {
 };
 
 // NR > 0: NR rows of S per thread in registers, for the sizes that delta_step_held names. 0: every size, S stays in memory.
-template <typename T, int NR>
-__global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaParams p, int cgp) {
+// TWO, for more workgroups than CUs: at most 128 registers, so that a CU runs two workgroups and one's chain of barriers lies under the other's. The low-rank matrices
+// are then read where they are used (batch rows share them in L2), and addresses are formed again instead of kept. us in bf16, one per CU / two, heads of
+// 128 x 128: 320 workgroups (16 heads, 20 rows) 24.4 / 18.9, 512 27.0 / 21.7, 288 (32 heads, 9 rows) 23.9 / 18.1, 544 36.0 / 32.5, 1024 51.2 / 39.5; heads of 64 x 64, 512 17.8 / 13.0.
+template <typename T, int NR, bool TWO = false>
+__global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 1, 8))) delta_step_kernel(const DeltaParams p, int cgp) {
   typedef typename T::storage S;
   __shared__ float red[8][4];
   int t = threadIdx.x;
@@ -245,7 +248,7 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
     f32x4 x = {0.f, 0.f, 0.f, 0.f};
     const bool in = d < p.dk && c0 < p.dv;
     if constexpr (NR > 0) {  // dv is a multiple of 4
-      const f32x4 y = *(const f32x4*)(st + (in ? d * p.dv + c0 : 0));
+      const f32x4 y = *(const f32x4*)((const char*)st + (in ? (unsigned)(d * p.dv + c0) * 4u : 0u));
 #pragma unroll
       for (int j = 0; j < 4; ++j) x[j] = in ? y[j] : 0.f;
     } else {
@@ -258,7 +261,7 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
   auto store_s = [&](int d, f32x4 x) {
     if (d >= p.dk || c0 >= p.dv) return;
     if constexpr (NR > 0) {
-      *(f32x4*)(st + d * p.dv + c0) = x;
+      *(f32x4*)((char*)st + (unsigned)(d * p.dv + c0) * 4u) = x;
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -267,9 +270,11 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
   };
   const S *a2 = (const S*)p.a2 + (long)h * p.dk * p.ra, *g2 = (const S*)p.g2 + (long)h * p.dv * p.rg;
   LowRankHeld<T> held_a, held_g;
-  if constexpr (NR > 0) {
+  if constexpr (NR > 0 && !TWO) {
     held_a.load(t, a2, p.dk, p.ra);
     held_g.load(t, g2, p.dv, p.rg);
+  }
+  if constexpr (NR > 0) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) sreg[i] = load_s(rg + RG * i);
   }
@@ -281,6 +286,8 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
   for (int i = p.dv + t; i < cols; i += kStepThreads) vs[i] = 0.f;
   for (int tok = 0; tok < p.t; ++tok) {
     asm volatile("" : "+v"(t));  // (one token is the rule: addresses kept from token to token would only cost registers)
+    int r0 = rg;
+    if constexpr (TWO) asm volatile("" : "+v"(r0));
     S* yrow = (S*)p.y + (((long)b * p.t + tok) * p.heads + h) * p.dv;
     if (!row.live(tok)) {  // uniform for the workgroup
       for (int i = t; i < p.dv; i += kStepThreads) yrow[i] = T::pack(0.f);
@@ -318,12 +325,12 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
     __syncthreads();
     auto decay = [&](int d, float z) { gs[d] += z; };
     auto open = [&](int e, float z) { gz[e] = z; };
-    if constexpr (NR > 0) {
+    if constexpr (NR > 0 && !TWO) {
       held_a.run(t, av, p.ra, decay);
       held_g.run(t, gv, p.rg, open);
     } else {
-      low_rank_rows<T>(a2, av, p.dk, p.ra, p.ra % 8 == 0 && p.vec, decay);
-      low_rank_rows<T>(g2, gv, p.dv, p.rg, p.rg % 8 == 0 && p.vec, open);
+      low_rank_rows<T>(a2, av, p.dk, p.ra, TWO || (p.ra % 8 == 0 && p.vec), decay);
+      low_rank_rows<T>(g2, gv, p.dv, p.rg, TWO || (p.rg % 8 == 0 && p.vec), open);
     }
     qq = kk = qk = 0.f;
 #pragma unroll
@@ -351,7 +358,7 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
     if constexpr (NR > 0) {
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
-        sweep(sreg[i], rg + RG * i);
+        sweep(sreg[i], r0 + RG * i);
         if (i % 4 == 3) asm volatile("" ::: "memory");  // (LDS reads of four rows ahead are enough)
       }
     } else {
@@ -398,7 +405,7 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
     if constexpr (NR > 0) {
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
-        write(sreg[i], rg + RG * i);
+        write(sreg[i], r0 + RG * i);
         if (i % 4 == 3) asm volatile("" ::: "memory");
       }
     } else {
@@ -418,8 +425,10 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const DeltaPar
     __syncthreads();  // everything in LDS is free
   }
   if constexpr (NR > 0) {
+    int r0 = rg;
+    asm volatile("" : "+v"(r0));  // (addresses kept from the loads on would cost registers)
 #pragma unroll
-    for (int i = 0; i < NR; ++i) store_s(rg + RG * i, sreg[i]);
+    for (int i = 0; i < NR; ++i) store_s(r0 + RG * i, sreg[i]);
   }
   keep_inputs<T>(p, b, h, t, kStepThreads);
 }
@@ -1172,8 +1181,9 @@ static int launch_delta_step(hipStream_t s, const DeltaParams& p) {
   };
   if constexpr (T::kDtype != MUI_DTYPE_F32) {
     if (delta_step_held(p)) {
-      if (rows <= 4) return launch(delta_step_kernel<T, 4>, 4);
-      if (rows <= 8) return launch(delta_step_kernel<T, 8>, 8);
+      const bool two = (long)p.heads * p.batch > device_cus();  // (up to there a workgroup has its CU to itself: 256 of 128 x 128 14.6 us)
+      if (rows <= 4) return two ? launch(delta_step_kernel<T, 4, true>, 4) : launch(delta_step_kernel<T, 4>, 4);
+      if (rows <= 8) return two ? launch(delta_step_kernel<T, 8, true>, 8) : launch(delta_step_kernel<T, 8>, 8);
       if (rows <= 16) return launch(delta_step_kernel<T, 16>, 16);
     }
   }
