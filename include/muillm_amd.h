@@ -115,6 +115,13 @@ int mui_linear_ws(mui_stream_t stream, int dtype, const void* weights, long w_pi
                   const void* mul_bias, const void* add_bias, const void* residual,
                   void* y, int n_out, int k_in, int tokens, void* workspace, size_t workspace_bytes);
 
+/* A linear with a residual and the norm that follows it, in one call: y = W x (+ add_bias) + residual, h = next_gain * y * rsqrt(mean(y^2) + epsilon)
+ * over each row of y -- mui_linear_ws and mui_rmsnorm, whose contracts hold here. Where K is divided between workgroups (17 to 128 tokens, a
+ * workspace given, at most 8192 outputs) the launch that adds the partial outputs up takes the norm as well. */
+int mui_linear_norm(mui_stream_t stream, int dtype, const void* weights, long w_pitch, const void* x, const void* add_bias,
+                    const void* residual, const void* next_gain, float epsilon, void* y, void* h, int n_out, int k_in, int tokens,
+                    void* workspace, size_t workspace_bytes);
+
 /* muillm_rmsnorm_forward (csrc/module.cpp:251; csrc/norm/rmsnorm.cu:31-85; kernel
  * csrc/norm/rmsnorm_fp16_kernels.cu:35-126).
  *   y[r, :] = weights * x[r, :] * rsqrt(mean(x[r, :]^2) + epsilon), rows r < rows.
@@ -545,6 +552,13 @@ int mui_moe_residual_norm(mui_stream_t stream, int dtype, const float* residual_
                           const void* identity_in, const int32_t* expert, const float* weight, int n_experts,
                           int top, const void* post_gain, float branch_scale, const void* next_gain,
                           float next_scale, float epsilon, float* residual_out, void* h, int rows, int k);
+
+/* y = W x (+ add_bias) and mui_residual_norm of it (y_scale 1), in one call; 16-bit types. workspace as for mui_linear_ws. Where K is divided
+ * between workgroups (17 to 128 tokens, a workspace given, at most 8192 outputs, h given) the launch that adds the partial outputs up joins them, too. */
+int mui_linear_residual_norm(mui_stream_t stream, int dtype, const void* weights, long w_pitch, const void* x, const void* add_bias,
+                             const float* residual_in, const void* post_gain, float branch_scale, const void* next_gain, float next_scale,
+                             float epsilon, void* y, float* residual_out, void* h, int n_out, int k_in, int tokens, void* workspace,
+                             size_t workspace_bytes);
 
 /* y[t, n] = W[n, :] . x[t, :] + bias[n] with fp32 outputs: router logits, recurrence gates. W [n_out, k_in],
  * x [tokens, k_in] and bias [n_out] (may be NULL) in the activations' type. Any sizes. */

@@ -55,6 +55,7 @@ _SIGNATURES = {
     "mui_linear_ws": (c_int, [_P, c_int, _P, c_long, _P, _P, c_float, _P, _P, _P, _P, c_int, c_int, c_int, _P,
                               ctypes.c_size_t]),
     "mui_linear_workspace_bytes": (ctypes.c_size_t, []),
+    "mui_linear_norm": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_float, _P, _P, c_int, c_int, c_int, _P, ctypes.c_size_t]),
     "mui_rmsnorm": (c_int, [_P, c_int, _P, _P, c_float, _P, c_int, c_int]),
     "mui_gateup_silu": (c_int, [_P, c_int, _P, _P, c_long, _P, _P, c_float, _P, c_int, c_int, c_int]),
     "mui_gateup_silu_bias": (c_int, [_P, c_int, _P, _P, c_long, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int]),
@@ -100,6 +101,8 @@ _SIGNATURES = {
     "mui_decoder_stack_workspace_bytes": (ctypes.c_size_t, [_P, c_int, c_int]),
     "mui_decoder_stack_step": (c_int, [_P, _P, c_int, _P, _P, _P, c_long, _P, c_int, _P, c_long, c_int, _P]),
     "mui_residual_norm": (c_int, [_P, c_int, _P, _P, c_float, _P, c_float, _P, c_float, c_float, _P, _P, c_int, c_int]),
+    "mui_linear_residual_norm": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_float, _P, c_float, c_float, _P, _P, _P, c_int, c_int,
+                                         c_int, _P, ctypes.c_size_t]),
     "mui_moe_residual_norm": (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int, c_int, _P, c_float, _P, c_float, c_float, _P, _P,
                                       c_int, c_int]),
     "mui_linear_f32": (c_int, [_P, c_int, _P, _P, _P, _P, c_int, c_int, c_int]),

@@ -990,6 +990,7 @@ constexpr int kXsMaxTiles = 1024;                              // counters
 constexpr int kXsMaxWorkgroups = 512;                          // partial tiles
 constexpr size_t kXsSlotBytes = 128 * 128 * sizeof(float);     // one 128 x 128 partial tile
 constexpr size_t kXsCounterBytes = kXsMaxTiles * sizeof(unsigned);
+size_t prefill_counter_bytes() { return kXsCounterBytes; }
 size_t prefill_workspace_bytes() { return kXsCounterBytes + kXsMaxWorkgroups * kXsSlotBytes; }
 
 // shares of K per 128 x 128 tile worth taking, or 0: the grid of whole tiles leaves at least three

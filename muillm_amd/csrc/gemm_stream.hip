@@ -31,6 +31,8 @@ struct StreamParams {
   const uint16_t* mul_bias; const uint16_t* add_bias; const uint16_t* residual;
   uint16_t* y;
   float* part;     // [k_splits][tokens][n] where K is divided between workgroups
+  bool add;        // a launch behind this one adds the partial outputs up (else the caller's does)
+  bool free_add;   // ... and would run anyway
   int n, k, tokens;
   int n_units;     // bands of ROWS weight rows (gate/up: gate and up rows together)
   int k_splits;    // more than one: every workgroup has one unit, a share of K of one band
@@ -308,7 +310,7 @@ static int launch_stream_cfg(hipStream_t s, const StreamParams& p) {
   static_assert(G::LDS <= 160 * 1024, "LDS of a workgroup");
   const int cus = device_cus(), wgs = p.n_units * p.k_splits;
   const int st = launch_with_lds(gemm_stream_kernel<T, EPI, ROWS, NT>, dim3(wgs < cus ? wgs : cus), dim3(kStreamThreads), G::LDS, s, p);
-  if (st != MUI_OK || p.k_splits == 1) return st;
+  if (st != MUI_OK || p.k_splits == 1 || !p.add) return st;
   const long threads = (long)p.tokens * p.n / 4;
   hipLaunchKernelGGL(gemm_stream_add_kernel<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p);
   return launch_status();
@@ -369,7 +371,7 @@ static bool gateup_tiles_are_faster(int tokens, int rows, int k) {
 static int g_stream_rows = 0, g_stream_shares = 0;  // mui_tune_stream
 
 template <typename T, int EPI>
-static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
+static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int* splits = nullptr) {
   // Rows per unit and shares of K by the least time: what a CU takes in (27.5 KB of weights, 105 KB of token rows per microsecond, 82 in
   // steps of 128 k-values), a barrier per step, a fixed part per round of workgroups; for shares of K the second launch and the
   // partial outputs, written and read. Measured against every other pair at 17 to 128 tokens on matrices from 2048 x 2048 to 128256 x 4096 it
@@ -389,11 +391,14 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
       if (g_stream_shares && k != g_stream_shares) continue;
       const float one = (float)p.k / k * 2.f * ((float)r / 27.5e3f + 16.f * nt / (nt > 4 ? 82e3f : 105e3f));
       const float barriers = (float)p.k / k / (r + 16 * nt <= 96 ? 256 : 128) * 0.08f;
-      const float cost = ceil_div(units, cus) * (one + barriers + 1.f) + (k > 1 ? 2.5f + 0.3f * k + (float)k * p.tokens * p.n * 8.f / 4e6f : 0.f);
+      const float shares = k > 1 ? (p.free_add ? 0.f : 2.5f) + 0.3f * k + (float)k * p.tokens * p.n * 8.f / 4e6f : p.free_add ? 2.5f : 0.f;
+      const float cost = ceil_div(units, cus) * (one + barriers + 1.f) + shares;
       if (width == 0 || cost < best) { best = cost; width = r; p.n_units = units; p.k_splits = k; }
     }
   }
   const bool forced = g_stream_rows || g_stream_shares;
+  if (!p.add && p.k_splits == 1) return MUI_ERR_UNSUPPORTED;
+  if (splits) *splits = p.k_splits;
   if (!forced && EPI == SK_LINEAR && wide_is_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
   if (forced && !width) return MUI_ERR_INVALID_ARG;
   if (!forced && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
@@ -419,20 +424,41 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes) {
   return MUI_ERR_UNSUPPORTED;
 }
 
+// what the loads cannot serve
+static bool stream_serves(const SkinnyParams& q, int most) {
+  if (q.tokens < 1 || q.tokens > most || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return false;
+  if (q.k % 256 || q.n % 8 || q.n < 8 || q.pitch % 8 || q.pitch > (1L << 26)) return false;
+  return !((((uintptr_t)q.w0 | (uintptr_t)q.w1 | (uintptr_t)q.x) & 15) || (((uintptr_t)q.y | (uintptr_t)q.residual) & 7));
+}
+
+static StreamParams stream_params(const SkinnyParams& q, float* part, bool add) {
+  StreamParams p = {};
+  p.w0 = (const uint8_t*)q.w0; p.w1 = (const uint8_t*)q.w1; p.pitch = q.pitch * 2;
+  p.x = q.x; p.mul_bias = q.mul_bias; p.add_bias = q.add_bias; p.residual = q.residual; p.y = q.y;
+  p.n = q.n; p.k = q.k; p.tokens = q.tokens; p.part = part; p.k_splits = 1; p.add = add;
+  return p;
+}
+
 // 17..128 tokens (gate/up ..64), 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve and for
 // what another kernel does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
   // gate/up beyond 64 tokens: the tiled GEMM. Units of six and eight token tiles are built for linears only; for gate/up they were measured at 128 tokens and
   // 14336 x 4096 alone (64 us, tiles 52), between 65 and 127 not at all
-  if (q.tokens < 1 || q.tokens > (epilogue == SK_GATEUP ? 64 : 128) || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;
-  if (q.k % 256 || q.n % 8 || q.n < 8 || q.pitch % 8 || q.pitch > (1L << 26)) return MUI_ERR_UNSUPPORTED;
-  if ((((uintptr_t)q.w0 | (uintptr_t)q.w1 | (uintptr_t)q.x) & 15) || (((uintptr_t)q.y | (uintptr_t)q.residual) & 7)) return MUI_ERR_UNSUPPORTED;
-  StreamParams p = {};
-  p.w0 = (const uint8_t*)q.w0; p.w1 = (const uint8_t*)q.w1; p.pitch = q.pitch * 2;
-  p.x = q.x; p.mul_bias = q.mul_bias; p.add_bias = q.add_bias; p.residual = q.residual; p.y = q.y;
-  p.n = q.n; p.k = q.k; p.tokens = q.tokens; p.part = part; p.k_splits = 1;
+  if (!stream_serves(q, epilogue == SK_GATEUP ? 64 : 128)) return MUI_ERR_UNSUPPORTED;
+  const StreamParams p = stream_params(q, part, true);
   if (dtype == MUI_DTYPE_F16) return epilogue == SK_GATEUP ? launch_stream_t<F16, SK_GATEUP>(s, p, 0) : launch_stream_t<F16, SK_LINEAR>(s, p, part_bytes);
   if (dtype == MUI_DTYPE_BF16) return epilogue == SK_GATEUP ? launch_stream_t<BF16, SK_GATEUP>(s, p, 0) : launch_stream_t<BF16, SK_LINEAR>(s, p, part_bytes);
+  return MUI_ERR_UNSUPPORTED;
+}
+
+// The same for a caller whose next launch adds the partial outputs up itself: part [*splits][tokens][n] gets the products, nothing else is applied.
+// free_add: that launch runs whether K is divided or not (without: K is divided as by launch_gemm_stream). MUI_ERR_UNSUPPORTED also where K is better left undivided.
+int launch_gemm_stream_parts(hipStream_t s, int dtype, const SkinnyParams& q, float* part, size_t part_bytes, bool free_add, int* splits) {
+  if (!part || !stream_serves(q, 128)) return MUI_ERR_UNSUPPORTED;
+  StreamParams p = stream_params(q, part, false);
+  p.free_add = free_add;
+  if (dtype == MUI_DTYPE_F16) return launch_stream_t<F16, SK_LINEAR>(s, p, part_bytes, splits);
+  if (dtype == MUI_DTYPE_BF16) return launch_stream_t<BF16, SK_LINEAR>(s, p, part_bytes, splits);
   return MUI_ERR_UNSUPPORTED;
 }
 

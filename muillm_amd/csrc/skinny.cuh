@@ -180,12 +180,14 @@ __device__ __forceinline__ u32x4 convert_a_pair(uint32_t w0, uint32_t w1, uint32
 // tiled matrix-core GEMM for prompts (gemm_prefill.hip): any token count, 16-bit weights or int8 codes of either format
 int launch_prefill_gemm(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
 size_t prefill_workspace_bytes();  // what SkinnyParams::workspace must hold for the prompt GEMM to use it
+size_t prefill_counter_bytes();    // of that, at its start: counters that stay zero
 // 17..128 tokens: 16 weight rows per workgroup, K split over its waves, token columns in up to 8 MFMA tiles (gemm_wide.hip)
 int launch_gemm_wide(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
 // 17..128 tokens (gate/up ..64), 16-bit weights, k % 256 == 0, n % 8 == 0, no fused norm: bands of weight rows streamed through LDS stages that
 // the workgroup shares; part (part_bytes, may be none): fp32 partial outputs where shares of K are worth it (gemm_stream.hip). MUI_ERR_UNSUPPORTED
 // for everything else and for what the tiled GEMM does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);
+int launch_gemm_stream_parts(hipStream_t s, int dtype, const SkinnyParams& p, float* part, size_t part_bytes, bool free_add, int* splits);
 // launches gemm_skinny_kernel<dtype, weight format, epilogue>; returns a MUI_* status
 int launch_skinny(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
 // experiments: 0 disables the B-stationary persistent variant

@@ -42,6 +42,9 @@ class MuiHybridAttentionConfig:
 
 
 class MuiHybridAttention(MuiModule):
+    def takes_behind(self) -> bool:
+        return type(self.out_proj) is MuiLinear
+
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiHybridAttentionConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):
         super().__init__(engine_config=engine_config)
@@ -63,12 +66,13 @@ class MuiHybridAttention(MuiModule):
     def new_state(self, batch: int, capacity: int, device, dtype) -> MuiKeyValueState:
         return MuiKeyValueState(batch, capacity, self.config.kv_heads, self.config.dim, self.config.vdim, device, dtype)
 
-    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
         """h [B, T, hidden] -> [B, T, hidden]; the tokens' rows go to slots cache_position."""
         c, state = self.config, cache.layers[self.layer_idx]
         proj = self.proj.linear(h)
         q = hybrid_ops.hybrid_prepare(proj, c.heads, c.kv_heads, c.dim, c.vdim, self.q_norm, self.k_norm, self.eps, self.inv_freq,
                                       cache_position, cache.row_start, state.k, state.v)
         gate = proj[..., self.proj.slice_starts[3]:] if c.gated else None
-        return self.out_proj(hybrid_ops.hybrid_attention(q, state.k, state.v, gate, cache_position, cache.row_start, c.heads,
-                                                         c.kv_heads, c.scale, c.softcap, c.window, c.keep_first))
+        o = hybrid_ops.hybrid_attention(q, state.k, state.v, gate, cache_position, cache.row_start, c.heads, c.kv_heads, c.scale,
+                                        c.softcap, c.window, c.keep_first)
+        return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

@@ -37,6 +37,9 @@ class MuiLatentAttentionConfig:
 
 
 class MuiLatentAttention(MuiModule):
+    def takes_behind(self) -> bool:
+        return type(self.out_proj) is MuiLinear
+
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiLatentAttentionConfig, layer_idx: int,
                  eps: float, device=None, dtype=None):
         super().__init__(engine_config=engine_config)
@@ -60,7 +63,7 @@ class MuiLatentAttention(MuiModule):
             return None
         return MuiLatentState(batch, capacity, self.config.kv_rank, self.config.rot_dim, device, dtype)
 
-    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
         """h [B, T, hidden] (normed) -> [B, T, hidden]; the tokens' rows go to slots cache_position."""
         c = self.config
         b, t = h.shape[0], h.shape[1]
@@ -80,4 +83,4 @@ class MuiLatentAttention(MuiModule):
         else:
             o = hybrid_ops.latent_attention(q, cos_sin, w[:c.heads * c.dim], w[c.heads * c.dim:], state.c, state.r,
                                             cache_position, cache.row_start, c.heads, c.dim, c.vdim, c.scale, c.window, route)
-        return self.out_proj(o)
+        return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

@@ -12,13 +12,15 @@ import torch.nn as nn
 
 from ... import hybrid_ops
 from ...engineconfig import MuiEngineConfig
+from ...muillm_ext import ResidualBehind
 from ..module import MuiModule
 from ..norm.rmsnorm import MuiRMSNorm
 
 
 class MuiSandwichDecoderLayer(MuiModule):
     """mixer: a module with forward(h, cache, cache_position) and new_state(...); mlp: a module with
-    forward(h), or None for a layer without feed-forward. branch_scale: m."""
+    forward(h), or None for a layer without feed-forward. Where the class of either has a takes_behind() that is true, its forward takes a
+    `behind` for its last linear. branch_scale: m."""
 
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, mixer: MuiModule, mlp: Optional[MuiModule], eps: float,
                  device=None, dtype=None, pre_norms: bool = True, branch_scale: float = 1.0):
@@ -42,14 +44,25 @@ def run_layers(layers: List[MuiSandwichDecoderLayer], x: torch.Tensor, h: torch.
         return hybrid_ops.residual_norm(x, y, post.weight, None if following is None else following.weight, eps,
                                         branch_scale=m, next_scale=scale, emit=True)
 
+    # where it saves a launch the sublayer's last linear takes the join along
+    along = ResidualBehind.worth_it(h.numel() // h.shape[-1])
+
+    def sublayer(module, args, x, post: MuiRMSNorm, m: float, following: Optional[MuiRMSNorm], scale: float = 1.0):
+        if not (along and "takes_behind" in type(module).__dict__ and module.takes_behind()):
+            return join(x, module(*args), post, m, following, scale)
+        behind = ResidualBehind(x, post.weight, m, None if following is None else following.weight, scale, eps)
+        y = module(*args, behind=behind)
+        return behind.take(y) or join(x, y, post, m, following, scale)
+
     for i, layer in enumerate(layers):
         last, m = i + 1 == len(layers), layer.branch_scale
         following = (final_norm, final_scale) if last else (layers[i + 1].pre_mixer_norm,)
-        y, post = layer.mixer(h, cache, cache_position), layer.post_mixer_norm
-        if layer.mlp is not None:
-            x, h = join(x, y, post, m, layer.pre_mlp_norm)
-            y, post = layer.mlp(h), layer.post_mlp_norm
-        x, h = join(x, y, post, m, *following)
+        mixer = (layer.mixer, (h, cache, cache_position))
+        if layer.mlp is None:
+            x, h = sublayer(*mixer, x, layer.post_mixer_norm, m, *following)
+        else:
+            x, h = sublayer(*mixer, x, layer.post_mixer_norm, m, layer.pre_mlp_norm)
+            x, h = sublayer(layer.mlp, (h,), x, layer.post_mlp_norm, m, *following)
         h = h.reshape(shape)
         if collect is not None:
             collect.append(x.clone())

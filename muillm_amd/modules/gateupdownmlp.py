@@ -36,9 +36,9 @@ class _MuiGateUpSiLUMethod(Enum):
 class _MuiGateUpSiLU(torch.autograd.Function):
     @staticmethod
     def forward(ctx, engine, inputs, norm_weights, variance_epsilon, gate_weights, up_weights,
-                down_weights, residual, biases):
+                down_weights, residual, biases, behind=None):
         return muillm_ext.muillm_gateupsilu_forward(
-            engine, norm_weights, variance_epsilon, gate_weights, up_weights, down_weights, residual, inputs, biases)
+            engine, norm_weights, variance_epsilon, gate_weights, up_weights, down_weights, residual, inputs, biases, behind)
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -48,9 +48,9 @@ class _MuiGateUpSiLU(torch.autograd.Function):
 class _MuiGateUpSiLUSplit(torch.autograd.Function):
     @staticmethod
     def forward(ctx, engine, inputs, norm_weights, variance_epsilon, gate_weights, up_weights,
-                down_weights, residual, biases):
+                down_weights, residual, biases, behind=None):
         return muillm_ext.muillm_gateupsilu_split_forward(
-            engine, norm_weights, variance_epsilon, gate_weights, up_weights, down_weights, residual, inputs, biases)
+            engine, norm_weights, variance_epsilon, gate_weights, up_weights, down_weights, residual, inputs, biases, behind)
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -207,23 +207,26 @@ class MuiGateUpDownMLP(MuiModule):
         return (self.dispatchable and muillm_ext.kernel_dispatchable(input)
                 and isinstance(self.gate_proj, MuiLinear) and isinstance(self.up_proj, MuiLinear))
 
-    def _forward_fused(self, input: Tensor, residual: Optional[Tensor] = None) -> Tensor:
+    def _forward_fused(self, input: Tensor, residual: Optional[Tensor] = None, behind=None) -> Tensor:
         if self._kernel_ok(input):
             return _MuiGateUpSiLU.apply(self.cpp_engine, input, self.norm_weights, self.variance_epsilon,
-                                        self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases())
+                                        self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind)
         return self._forward_unfused(input=input, residual=residual)
 
-    def _forward_split(self, input: Tensor, residual: Optional[Tensor] = None) -> Tensor:
+    def _forward_split(self, input: Tensor, residual: Optional[Tensor] = None, behind=None) -> Tensor:
         if self._kernel_ok(input):
             return _MuiGateUpSiLUSplit.apply(self.cpp_engine, input, self.norm_weights, self.variance_epsilon,
-                                             self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases())
+                                             self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind)
         return self._forward_unfused(input=input, residual=residual)
 
-    def forward(self, input: Tensor, residual: Optional[Tensor] = None) -> Tensor:
+    def takes_behind(self) -> bool:
+        return type(self.down_proj) is MuiLinear and self.method != _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED
+
+    def forward(self, input: Tensor, residual: Optional[Tensor] = None, behind: Optional[muillm_ext.ResidualBehind] = None) -> Tensor:
         if self.method == _MuiGateUpSiLUMethod.GATEUPSILU_FUSED:
-            return self._forward_fused(input=input, residual=residual)
+            return self._forward_fused(input=input, residual=residual, behind=behind)
         elif self.method == _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED:
             return self._forward_unfused(input=input, residual=residual)
         elif self.method == _MuiGateUpSiLUMethod.GATEUPSILU_SPLIT:
-            return self._forward_split(input=input, residual=residual)
+            return self._forward_split(input=input, residual=residual, behind=behind)
         raise ValueError("Unsupported Gate/Up Silu method")

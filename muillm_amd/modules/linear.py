@@ -27,8 +27,8 @@ class _MuiLinear(torch.autograd.Function):
     """The library call as an autograd node without a backward (inference only)."""
 
     @staticmethod
-    def forward(ctx, module, x, residual):
-        return muillm_ext.muillm_linear_module_forward(module, x, residual=residual)
+    def forward(ctx, module, x, residual, behind=None):
+        return muillm_ext.muillm_linear_module_forward(module, x, residual=residual, behind=behind)
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -128,9 +128,9 @@ class MuiLinear(MuiModule, nn.Linear):
         self.dispatchable = is_kernel_dtype(self.weight)
 
     # ---- forward -----------------------------------------------------------------------------
-    def forward(self, input: Tensor, residual: Optional[Tensor] = None) -> Tensor:
+    def forward(self, input: Tensor, residual: Optional[Tensor] = None, behind: Optional[muillm_ext.ResidualBehind] = None) -> Tensor:
         if self.cpp_module is not None:
-            return _MuiLinear.apply(self.cpp_module, input, residual)
+            return _MuiLinear.apply(self.cpp_module, input, residual, behind)
         # before finalize_init: plain torch, with the library's norm kernel where it applies
         x = input
         if self.normalize:

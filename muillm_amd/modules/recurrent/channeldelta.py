@@ -38,6 +38,9 @@ class MuiChannelDelta(MuiModule):
     """Everything that reads h is one projection q | k | v | a1 | g1 | b. The low-rank parts and b are padded with zero
     rows (and a2, g2 with zero columns) to multiples of eight, so that every part starts on a 16-byte boundary."""
 
+    def takes_behind(self) -> bool:
+        return type(self.out_proj) is MuiLinear
+
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiChannelDeltaConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):
         super().__init__(engine_config=engine_config)
@@ -71,7 +74,7 @@ class MuiChannelDelta(MuiModule):
         return MuiRecurrentState(torch.zeros((batch, c.heads, c.dim, c.vdim), dtype=torch.float32, device=device),
                                  torch.zeros((batch, layer.ring_rows, layer.channels), dtype=dtype, device=device))
 
-    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
         memory, ring = cache.layers[self.layer_idx].values
-        return self.out_proj(hybrid_ops.channel_delta(self.layer(), self.proj.linear(h), memory, ring, cache_position,
-                                                      cache.row_start))
+        o = hybrid_ops.channel_delta(self.layer(), self.proj.linear(h), memory, ring, cache_position, cache.row_start)
+        return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

@@ -22,6 +22,9 @@ class MuiMLstmConfig:
 
 
 class MuiMLstm(MuiModule):
+    def takes_behind(self) -> bool:
+        return type(self.out_proj) is MuiLinear
+
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiMLstmConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):
         super().__init__(engine_config=engine_config)
@@ -42,11 +45,12 @@ class MuiMLstm(MuiModule):
                                  torch.zeros((batch, c.heads, slices, c.dim), dtype=torch.float32, device=device),
                                  torch.zeros((batch, c.heads, slices), dtype=torch.float32, device=device))
 
-    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
         c = self.config
         b, t = h.shape[0], h.shape[1]
         q, k, v, gate = self.proj(h)
         gates = hybrid_ops.linear_f32(h, self.gate_weight, self.gate_bias).view(b, t, 2 * c.heads)
         o = hybrid_ops.mlstm(q, k, v, gates, cache.layers[self.layer_idx].values, c.dim ** -0.5, c.gate_cap, cache_position,
                              cache.row_start, c.heads)
-        return self.out_proj(hybrid_ops.mlstm_output(o, self.head_norm, gate, self.eps))
+        o = hybrid_ops.mlstm_output(o, self.head_norm, gate, self.eps)
+        return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

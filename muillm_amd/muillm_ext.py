@@ -162,6 +162,44 @@ def _prompt_workspace(x: torch.Tensor, stream: int) -> Optional[torch.Tensor]:
     return ws
 
 
+class ResidualBehind:
+    """The boundary between two sublayers with an fp32 residual stream (hybrid_ops.residual_norm) that follows a linear and is taken along by its
+    library call: the stream and the next sublayer's input. An object lives for one boundary of one forward pass: whoever makes it hands it to
+    the linear, which fills it in where it can, and asks with the very tensor that the sublayer has returned whether it was. A tensor that somebody (a module
+    hook) has put in its place, or has written to since, finds nothing here and is joined the ordinary way: the stream is not updated in place."""
+    MAX_TOKENS = 128  # beyond, K is not divided and nothing is saved
+
+    def __init__(self, stream: torch.Tensor, post_gain: torch.Tensor, branch_scale: float, next_gain: Optional[torch.Tensor], next_scale: float,
+                 eps: float):
+        self.stream, self.post_gain, self.next_gain = stream, post_gain, next_gain
+        self.branch_scale, self.next_scale, self.eps = float(branch_scale), float(next_scale), float(eps)
+        self.of = None  # the linear's output
+
+    @classmethod
+    def worth_it(cls, tokens: int) -> bool:
+        return not torch.is_grad_enabled() and MUI_MAX_TOKENS < tokens <= cls.MAX_TOKENS
+
+    def linear(self, y: torch.Tensor, call) -> bool:
+        """call(name, arguments between the linear's operands and its sizes)"""
+        x = self.stream
+        if torch.is_grad_enabled() or y.is_inference():  # (versions cannot be asked for in inference mode)
+            return False
+        if x.dtype != torch.float32 or x.device != y.device or x.numel() != y.numel() or not x.is_contiguous():
+            return False
+        for gain in (self.post_gain, self.next_gain):
+            if gain is not None and (gain.dtype != y.dtype or gain.device != y.device or gain.numel() != y.shape[-1] or not gain.is_contiguous()):
+                return False
+        out, h = torch.empty_like(x), torch.empty_like(y)
+        call("mui_linear_residual_norm", (x.data_ptr(), _ptr(self.post_gain), self.branch_scale, _ptr(self.next_gain), self.next_scale, self.eps,
+                                          y.data_ptr(), out.data_ptr(), h.data_ptr()))
+        self.result, self.of, self._version = (out, h), y, y._version
+        return True
+
+    def take(self, y) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+        """(the stream, the next sublayer's input)"""
+        return self.result if self.of is not None and y is self.of and y._version == self._version else None
+
+
 def _token_calls(tokens: int, chunk_max: int):
     """(first token, count) of the library calls that cover `tokens` rows: chunks of MUI_MAX_TOKENS
     for the decode kernels up to chunk_max tokens, one call (the tiled GEMM) beyond."""
@@ -255,8 +293,10 @@ def muillm_linear_forward(
     mul_bias: Optional[torch.Tensor] = None,
     add_bias: Optional[torch.Tensor] = None,
     residual: Optional[torch.Tensor] = None,
+    behind: Optional[ResidualBehind] = None,
 ) -> torch.Tensor:
-    """y = (W . rmsnorm?(x)) * mul_bias + add_bias + residual, output shape x.shape[:-1] + [N]."""
+    """y = (W . rmsnorm?(x)) * mul_bias + add_bias + residual, output shape x.shape[:-1] + [N]. behind: filled in where the call can
+    take it along."""
     if weights.dim() != 2:
         raise RuntimeError("weights must be 2-D [out_features, in_features]")
     n, k = weights.shape
@@ -292,14 +332,21 @@ def muillm_linear_forward(
     y = torch.empty(out_shape, dtype=x.dtype, device=x.device)
     lib, stream, code, esz = _lib.load(), _stream(x), _dtype_code(x), x.element_size()
     ws = _prompt_workspace(x, stream) if tokens > FUSED_CHUNK_MAX_TOKENS else None
+    ws_args = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
+    if behind is not None and tokens > FUSED_CHUNK_MAX_TOKENS and norm_weights is None and mul_bias is None and residual is None:
+
+        def call(name, args):
+            check(getattr(lib, name)(stream, code, weights.data_ptr(), pitch, x.data_ptr(), _ptr(add_bias), *args, n, k, tokens, *ws_args), name)
+
+        if behind.linear(y, call):
+            return y
     for off, cnt in _token_calls(tokens, FUSED_CHUNK_MAX_TOKENS):
         check(
             lib.mui_linear_ws(
                 stream, code, weights.data_ptr(), pitch, x.data_ptr() + off * k * esz,
                 _ptr(norm_weights), float(epsilon), _ptr(mul_bias), _ptr(add_bias),
                 None if residual is None else residual.data_ptr() + off * n * esz,
-                y.data_ptr() + off * n * esz, n, k, cnt,
-                None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+                y.data_ptr() + off * n * esz, n, k, cnt, *ws_args,
             ),
             "mui_linear",
         )
@@ -327,10 +374,10 @@ def muillm_linear_module_deinit(module: MuiLinearModuleHandle) -> None:
     module.weights = module.norm_weights = module.mul_bias = module.add_bias = None
 
 
-def muillm_linear_module_forward(module: MuiLinearModuleHandle, inputs: torch.Tensor, residual=None):
+def muillm_linear_module_forward(module: MuiLinearModuleHandle, inputs: torch.Tensor, residual=None, behind=None):
     return muillm_linear_forward(
         module.engine, inputs, module.weights, module.norm_weights, module.epsilon,
-        module.mul_bias, module.add_bias, residual,
+        module.mul_bias, module.add_bias, residual, behind,
     )
 
 
@@ -385,23 +432,23 @@ def mui_silu_mul_interleaved(gate_up: torch.Tensor) -> torch.Tensor:
 
 
 def muillm_gateupsilu_forward(engine, norm_weights, epsilon, gate_weights, up_weights, down_weights,
-                              residual, x, biases=None) -> torch.Tensor:
+                              residual, x, biases=None, behind: Optional[ResidualBehind] = None) -> torch.Tensor:
     """out = Wd (silu(Wg xn) * (Wu xn)) + residual, argument order of csrc/module.cpp:182. biases: (gate, up, down)
-    vectors added to the three products, or None."""
+    vectors added to the three products, or None; behind: as muillm_linear_forward's."""
     if not (kernel_dispatchable(x) and gate_weights.dtype == x.dtype):
         raise RuntimeError("muillm_gateupsilu_forward needs fp16 / bf16 CUDA tensors with k % 8 == 0")
     gate_bias, up_bias, down_bias = biases or (None, None, None)
     h = mui_gateup_silu(norm_weights, epsilon, gate_weights, up_weights, x, gate_bias, up_bias)
-    return muillm_linear_forward(engine, h, down_weights, add_bias=down_bias, residual=residual)
+    return muillm_linear_forward(engine, h, down_weights, add_bias=down_bias, residual=residual, behind=behind)
 
 
 def muillm_gateupsilu_split_forward(engine, norm_weights, epsilon, gate_weights, up_weights,
-                                    down_weights, residual, x, biases=None) -> torch.Tensor:
+                                    down_weights, residual, x, biases=None, behind=None) -> torch.Tensor:
     """The reference's split-K variant (csrc/module.cpp:215) exists to create more blocks on
     MI300; the gfx950 kernel already sizes its grid to the CU count, so both names run the
     same path."""
     return muillm_gateupsilu_forward(engine, norm_weights, epsilon, gate_weights, up_weights,
-                                     down_weights, residual, x, biases)
+                                     down_weights, residual, x, biases, behind)
 
 
 # --------------------------------------------------------------------------------------
