@@ -522,6 +522,18 @@ int mui_decoder_stack_step(mui_stream_t stream, const mui_decoder_stack_t* model
                            long position_batch_stride, const int64_t* cache_position, int seq_len,
                            const void* mask, long mask_batch_stride, int n_splits, void* workspace);
 
+/* The same layers for any number of rows: prompts (tokens > 1: RoPE and cache write, then causal attention over the cache) and steps of more batch
+ * rows than MUI_MAX_TOKENS (tokens 1). hidden_in, hidden_out: [batch, tokens, hidden]; position_ids: [batch or 1, tokens], rows position_batch_stride
+ * apart (0: one row for all); cache_position: [tokens] slots. seq_len: tokens in the cache, these included (tokens 1 also -1: read from cache_position on the device).
+ * mask: NULL; with tokens > 1 the key mask of mui_prefill_attention_masked, with tokens 1 the additive rows of mui_decoder_stack_step.
+ * workspace: mui_decoder_stack_prompt_bytes bytes, 256-byte aligned; linear_workspace: as mui_linear_ws's, or NULL. int8 projections convert on the way
+ * whatever the number of rows. On an error part of the layers may have been enqueued. */
+size_t mui_decoder_stack_prompt_bytes(const mui_decoder_stack_t* m, int batch, int tokens, int n_splits);
+int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_stack_t* m, int batch, int tokens, const void* hidden_in, void* hidden_out,
+                             const int64_t* position_ids, long position_batch_stride, const int64_t* cache_position, int seq_len,
+                             const void* mask, long mask_batch_stride, int n_splits, void* workspace, void* linear_workspace,
+                             size_t linear_workspace_bytes);
+
 /* muillm_embedding_module_forward (csrc/module.cpp:320; csrc/embedding/embedding.cu:31-100; kernels
  * csrc/embedding/embedding_xx16_kernels.cu:26-112): out[t, :] = table[ids[t], :] for a 16-bit
  * [vocab, dim] table with row pitch row_pitch elements; ids int64, or int32 when ids_are_int32.

@@ -99,6 +99,8 @@ _SIGNATURES = {
                                    c_long, c_int, _P, _P, c_int, c_long]),
     "mui_embedding": (c_int, [_P, c_int, _P, c_long, _P, c_int, _P, c_int, c_int, c_int]),
     "mui_decoder_stack_workspace_bytes": (ctypes.c_size_t, [_P, c_int, c_int]),
+    "mui_decoder_stack_prompt_bytes": (ctypes.c_size_t, [_P, c_int, c_int, c_int]),
+    "mui_decoder_stack_prompt": (c_int, [_P, _P, c_int, c_int, _P, _P, _P, c_long, _P, c_int, _P, c_long, c_int, _P, _P, ctypes.c_size_t]),
     "mui_decoder_stack_step": (c_int, [_P, _P, c_int, _P, _P, _P, c_long, _P, c_int, _P, c_long, c_int, _P]),
     "mui_residual_norm": (c_int, [_P, c_int, _P, _P, c_float, _P, c_float, _P, c_float, c_float, _P, _P, c_int, c_int]),
     "mui_linear_residual_norm": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_float, _P, c_float, c_float, _P, _P, _P, c_int, c_int,

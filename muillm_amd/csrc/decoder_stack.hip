@@ -125,3 +125,124 @@ extern "C" int mui_decoder_stack_step(mui_stream_t stream, const mui_decoder_sta
   }
   return MUI_OK;
 }
+
+// ---------------------------------------------------------------------------------------
+// Any number of rows: prompts, and steps of more batch rows than the decode kernels take
+// ---------------------------------------------------------------------------------------
+namespace {
+
+struct PromptWorkspace {
+  char *h_a, *h_b;  // [rows, hidden]  residual stream
+  char* normed;     // [rows, hidden]  the next linear's input
+  char *qkv, *q_rot, *attn, *scratch;  // up to the output projection
+  char* mid;                           // [rows, intermediate], in the same place
+  size_t total;
+};
+
+PromptWorkspace carve_rows(const mui_decoder_stack_t* m, int batch, int tokens, int n_splits, char* base) {
+  PromptWorkspace w;
+  const size_t rows = (size_t)batch * tokens, e = 2;
+  const size_t hid = align256(rows * m->hidden * e), att = align256(rows * m->n_q_heads * m->head_dim * e);
+  const size_t qkv = align256(rows * (m->n_q_heads + 2 * m->n_kv_heads) * m->head_dim * e), mid = align256(rows * m->intermediate * e);
+  const size_t scr = tokens == 1 ? align256(mui_flash_decode_scratch_bytes(batch, m->n_q_heads, m->head_dim, n_splits)) : 0;
+  w.h_a = base;
+  w.h_b = w.h_a + hid;
+  w.normed = w.h_b + hid;
+  w.qkv = w.normed + hid;
+  w.q_rot = w.qkv + qkv;
+  w.attn = w.q_rot + (tokens == 1 ? 0 : att);
+  w.scratch = w.attn + att;
+  w.mid = w.qkv;  // (the output projection has read the rest when the gate and up products start)
+  const size_t before = (size_t)(w.scratch - w.qkv) + scr;
+  w.total = 3 * hid + (before > mid ? before : mid);
+  return w;
+}
+
+}  // namespace
+
+extern "C" size_t mui_decoder_stack_prompt_bytes(const mui_decoder_stack_t* m, int batch, int tokens, int n_splits) {
+  if (!m || batch < 1 || tokens < 1 || n_splits < 1) return 0;
+  return carve_rows(m, batch, tokens, n_splits, nullptr).total;
+}
+
+extern "C" int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_stack_t* m, int batch, int tokens, const void* hidden_in,
+                                        void* hidden_out, const int64_t* position_ids, long position_batch_stride,
+                                        const int64_t* cache_position, int seq_len, const void* mask, long mask_batch_stride, int n_splits,
+                                        void* workspace, void* linear_workspace, size_t linear_workspace_bytes) {
+  MUI_CHECK_ARG(m && m->layers && m->n_layers > 0 && hidden_in && hidden_out && workspace);
+  MUI_CHECK_ARG(batch >= 1 && tokens >= 1 && n_splits >= 1 && position_ids && cache_position);
+  MUI_CHECK_ARG(((uintptr_t)workspace & 255u) == 0 && (long)batch * tokens <= (1L << 30));
+  MUI_CHECK_ARG(tokens == 1 || seq_len >= tokens);
+  const int rows = batch * tokens;
+  const PromptWorkspace w = carve_rows(m, batch, tokens, n_splits, (char*)workspace);
+  const int hid = m->hidden, qd = m->n_q_heads * m->head_dim, kvd = m->n_kv_heads * m->head_dim, qkv_n = qd + 2 * kvd;
+  const bool fused = rows <= MUI_MAX_TOKENS;  // the decode kernels take the norm in front of a linear; beyond, it is a launch of its own or rides behind the linear in front
+  for (int l = 0; l < m->n_layers; ++l) {
+    const mui_decoder_layer_t& L = m->layers[l];
+    if (L.int8_group_size_shift < 0 || (L.gate_scales == nullptr) != (L.up_scales == nullptr)) return MUI_ERR_INVALID_ARG;
+  }
+  // y = W x (+ residual); next: the gain of the norm behind it, into w.normed
+  auto linear = [&](const void* weight, long pitch, const void* scales, int shift, const void* x, const void* gain, const void* residual, void* y, int n,
+                    int k, const void* next) -> int {
+    int st;
+    if (scales) {
+      st = shift ? mui_int8_group_linear(stream, m->dtype, weight, pitch, scales, shift, x, gain, m->norm_eps, nullptr, residual, y, n, k, rows)
+                 : mui_int8_linear(stream, m->dtype, weight, pitch, scales, x, gain, m->norm_eps, nullptr, residual, y, n, k, rows);
+    } else if (next) {
+      return mui_linear_norm(stream, m->dtype, weight, pitch, x, nullptr, residual, next, m->norm_eps, y, w.normed, n, k, rows, linear_workspace,
+                             linear_workspace_bytes);
+    } else {
+      st = mui_linear_ws(stream, m->dtype, weight, pitch, x, gain, m->norm_eps, nullptr, nullptr, residual, y, n, k, rows, linear_workspace,
+                         linear_workspace_bytes);
+    }
+    if (st != MUI_OK || !next) return st;
+    return mui_rmsnorm(stream, m->dtype, next, y, m->norm_eps, w.normed, rows, n);
+  };
+  const char* h = (const char*)hidden_in;  // residual stream entering the layer
+  if (!fused) {
+    const int st = mui_rmsnorm(stream, m->dtype, m->layers[0].input_norm, h, m->norm_eps, w.normed, rows, hid);
+    if (st != MUI_OK) return st;
+  }
+  for (int l = 0; l < m->n_layers; ++l) {
+    const mui_decoder_layer_t& L = m->layers[l];
+    const bool last = l + 1 == m->n_layers;
+    const int gs = L.int8_group_size_shift;
+    char* out = last ? (char*)hidden_out : w.h_b;
+    int st = linear(L.qkv_weight, L.qkv_pitch, L.qkv_scales, gs, fused ? h : w.normed, fused ? L.input_norm : nullptr, nullptr, w.qkv, qkv_n, hid, nullptr);
+    if (st != MUI_OK) return st;
+    const char *q = w.qkv, *k = q + (size_t)qd * 2, *v = k + (size_t)kvd * 2;
+    if (tokens == 1) {
+      st = mui_attn_decode_fused_warm(stream, m->dtype, q, qkv_n, k, qkv_n, v, qkv_n, m->cos_table, m->sin_table, (int)m->rope_row_stride,
+                                      (int)m->rope_rows, position_ids, position_batch_stride, cache_position, seq_len, L.k_cache, L.v_cache,
+                                      m->cache_batch_stride, m->cache_head_stride, m->cache_token_stride, mask, mask_batch_stride, nullptr,
+                                      w.scratch, n_splits, w.attn, batch, m->n_q_heads, m->n_kv_heads, m->head_dim, m->max_cache_len, nullptr, 0, 0);
+    } else {
+      const long tb = (long)tokens * qkv_n;
+      st = mui_rope_kv_write(stream, m->dtype, q, tb, qkv_n, m->head_dim, k, tb, qkv_n, m->head_dim, v, tb, qkv_n, m->head_dim, m->cos_table,
+                             m->sin_table, (int)m->rope_row_stride, (int)m->rope_rows, position_ids, position_batch_stride, cache_position, w.q_rot,
+                             L.k_cache, L.v_cache, m->cache_batch_stride, m->cache_head_stride, m->cache_token_stride, batch, tokens, m->n_q_heads,
+                             m->n_kv_heads, m->head_dim, m->max_cache_len);
+      if (st != MUI_OK) return st;
+      st = mask ? mui_prefill_attention_masked(stream, m->dtype, w.q_rot, L.k_cache, L.v_cache, m->cache_batch_stride, m->cache_head_stride,
+                                               m->cache_token_stride, seq_len, seq_len - tokens, mask, mask_batch_stride, w.attn, batch, m->n_q_heads,
+                                               m->n_kv_heads, tokens, m->head_dim)
+                : mui_prefill_attention(stream, m->dtype, w.q_rot, L.k_cache, L.v_cache, m->cache_batch_stride, m->cache_head_stride,
+                                        m->cache_token_stride, seq_len, seq_len - tokens, w.attn, batch, m->n_q_heads, m->n_kv_heads, tokens, m->head_dim);
+    }
+    if (st != MUI_OK) return st;
+    st = linear(L.o_weight, L.o_pitch, L.o_scales, gs, w.attn, nullptr, h, w.h_a, hid, qd, fused ? nullptr : L.post_norm);
+    if (st != MUI_OK) return st;
+    const void *mx = fused ? w.h_a : w.normed, *gain = fused ? L.post_norm : nullptr;
+    st = !L.gate_scales ? mui_gateup_silu(stream, m->dtype, L.gate_weight, L.up_weight, L.gateup_pitch, mx, gain, m->norm_eps, w.mid, m->intermediate, hid, rows)
+         : gs ? mui_int8_group_gateup_silu(stream, m->dtype, L.gate_weight, L.up_weight, L.gateup_pitch, L.gate_scales, L.up_scales,
+                                           L.gateup_scale_stride, gs, mx, gain, m->norm_eps, w.mid, m->intermediate, hid, rows)
+              : mui_int8_gateup_silu(stream, m->dtype, L.gate_weight, L.up_weight, L.gateup_pitch, L.gate_scales, L.up_scales, L.gateup_scale_stride, mx,
+                                     gain, m->norm_eps, w.mid, m->intermediate, hid, rows);
+    if (st != MUI_OK) return st;
+    st = linear(L.down_weight, L.down_pitch, L.down_scales, gs, w.mid, nullptr, w.h_a, out, hid, m->intermediate,
+                fused || last ? nullptr : m->layers[l + 1].input_norm);
+    if (st != MUI_OK) return st;
+    h = out;
+  }
+  return MUI_OK;
+}

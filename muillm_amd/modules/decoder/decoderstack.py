@@ -5,8 +5,12 @@ The reference walks its layers from C++ only under tensor parallelism
 one GPU it calls its Python layer modules one by one (muillm/modules/decoder/decoder.py:130-165).
 Here `mui_decoder_stack_step` enqueues the same per-layer sequence for every layer, so a step
 that is not replayed from a HIP graph pays the host cost of one call instead of ~160.
+`mui_decoder_stack_prompt` does the same for prompts and for steps of more batch rows than
+the decode kernels take (~180 us of host time per layer otherwise, more than a prompt of 100 tokens keeps the GPU busy).
 """
+import copy
 import ctypes
+import weakref
 from typing import Optional
 
 import torch
@@ -14,12 +18,14 @@ import torch.nn as nn
 
 from ... import _lib, muillm_ext
 from ..attention.baseattention import MuiBaseAttention
-from ..gateupdownmlp import MuiGateUpDownMLP
+from ..attention.sdpaattention import MuiSdpaAttention
+from ..gateupdownmlp import MuiGateUpDownMLP, _MuiGateUpSiLUMethod
 from ..kvcache.cache_utils import MuiStaticCache
 from ..linear import MuiLinear
 from ..multilinear import MuiMultiLinear
 from ..quantized.int8gateupdownmlp import MuiInt8GateUpDownMLP
 from ..quantized.int8linear import MuiInt8Linear
+from .decoder import MuiDecoderLayer
 
 
 def _group_shift(m) -> int:
@@ -225,4 +231,183 @@ class MuiDecoderStack:
                                        pos.data_ptr(), 1 if pos.numel() > 1 else 0, cache_position.data_ptr(),
                                        -1 if seq_len is None else int(seq_len), mask_ptr, mask_bs, n_splits, ws_ptr),
             "mui_decoder_stack_step")
+        return out
+
+
+class MuiPromptStack(MuiDecoderStack):
+    """The same for `mui_decoder_stack_prompt`: prompts, and steps of more batch rows than the decode kernels take. Layers called one by one run the same
+    kernels; here nobody can listen in between, so a model with hooks stays with its modules.
+
+    What the descriptor was built from is watched by object and by address (current(), asked before every call, takes a few us per layer, where examining the
+    layers anew takes ~35 with an idle GPU waiting), through weak references: nothing is kept alive beyond a call."""
+
+    _ATTRIBUTES = ("training", "method", "cpp_module", "variance_epsilon", "normalize", "layer_idx", "prefill_kernel_max_tokens", "dispatchable", "num_heads",
+                   "num_key_value_heads", "head_dim", "in_features", "out_features", "intermediate_size", "per_channel", "group_size_shift", "quantizer")
+
+    def __init__(self, layers, rotary_emb, cache: MuiStaticCache):
+        super().__init__(layers, rotary_emb, cache, 1)
+        self._keep, self._owners, self._layer_list = [], [], None
+        self._watched, self._layer_refs = None, [weakref.ref(layer) for layer in layers]
+        self._cache_layers = [layer.self_attn.layer_idx for layer in layers]
+        self._bound(cache)
+        self._tables = rotary_emb
+        int8 = any(type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP)
+                   for layer in layers for m in (layer.qkv_proj.linear, layer.self_attn.o_proj, layer.mlp, layer.mlp.down_proj))
+        self._most_rows = min(muillm_ext.INT8_DEQUANT_MIN_TOKENS, muillm_ext.INT8_GROUP_DEQUANT_MIN_TOKENS) - 1 if int8 else 1 << 30
+        self._most_tokens = min([65535] + [x.self_attn.prefill_kernel_max_tokens for x in layers if x.self_attn.prefill_kernel_max_tokens is not None])
+
+    def _watch(self) -> None:
+        """(Made behind the first call, while the GPU is at work.)"""
+        def weak(v) -> bool:
+            return isinstance(v, (torch.Tensor, nn.Module)) or hasattr(v, "__weakref__")
+
+        def ref(v):
+            return weakref.ref(v) if weak(v) else (lambda: v)
+
+        self._watched = []  # per module: itself, its children, its tensors with their addresses, what else was read from it
+        for layer in [r() for r in self._layer_refs]:
+            qkv, attn, mlp = layer.qkv_proj, layer.self_attn, layer.mlp
+            inside = [getattr(mlp, n) for n in ("gate_proj", "up_proj", "down_proj") if isinstance(getattr(mlp, n, None), nn.Module)]
+            for m in [layer, qkv, qkv.linear, attn, attn.o_proj, mlp] + inside:
+                self._watched.append((weakref.ref(m), [(k, ref(v)) for k, v in m._modules.items()],
+                                      [(k, ref(v), _ptr(v)) for k, v in m._parameters.items()],
+                                      [(k, m.__dict__[k]) for k in self._ATTRIBUTES if k in m.__dict__ and not weak(m.__dict__[k])],
+                                      [(k, weakref.ref(m.__dict__[k])) for k in self._ATTRIBUTES if k in m.__dict__ and weak(m.__dict__[k])]))
+
+    @staticmethod
+    def eligible(layers, rotary_emb, cache) -> bool:
+        """Whether the layers, called one by one, would run the kernels that mui_decoder_stack_prompt runs."""
+        if not MuiDecoderStack.eligible(layers, rotary_emb, cache, 1):
+            return False
+        if not MuiPromptStack._cache_serves(cache):
+            return False
+        for layer in layers:
+            qkv, attn, mlp = layer.qkv_proj.linear, layer.self_attn, layer.mlp
+            if type(layer) is not MuiDecoderLayer or type(attn) is not MuiSdpaAttention or attn.training:
+                return False
+            if type(mlp) is MuiGateUpDownMLP and (not mlp.dispatchable or mlp.method == _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED):
+                return False
+            for m in (qkv, attn.o_proj) + ((mlp.down_proj,) if type(mlp) is MuiInt8GateUpDownMLP else ()):
+                if type(m) is MuiLinear and (m.cpp_module is None or m.cpp_module.weights is not m.weight):
+                    return False
+            hidden, inter = qkv.in_features, mlp.intermediate_size
+            if hidden % 8 or inter % 8 or hidden > 16384:
+                return False
+            int8 = any(type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP) for m in (qkv, attn.o_proj, mlp, mlp.down_proj))
+            if int8 and (hidden % 16 or inter % 16 or (inter > 16384 and qkv.norm_weights.dtype != torch.float16)):
+                return False
+        return True
+
+    @staticmethod
+    def _cache_serves(cache: MuiStaticCache) -> bool:
+        kc = cache.key_cache[0]
+        return (kc.stride(3) == 1 and not any(x % 8 for x in kc.stride()[:3])
+                and all(x.stride() == kc.stride() and x.dtype == kc.dtype and x.device == kc.device and x.data_ptr() % 16 == 0 for x in cache.tensors()))
+
+    def _bound(self, cache: MuiStaticCache) -> None:
+        self._cache = weakref.ref(cache)
+        self._cache_tensors = [(weakref.ref(t), t.data_ptr()) for t in cache.tensors()]
+
+    def bound_to(self, cache: MuiStaticCache) -> Optional["MuiPromptStack"]:
+        """The same for another cache (a request brings its own), or None. A descriptor of its own: another thread may be in a call with this one."""
+        kc = cache.key_cache[0]
+        if (len(cache.key_cache) <= max(self._cache_layers) or kc.dtype != self.dtype or kc.device != self.device or kc.shape[1] != self.hkv
+                or kc.shape[3] != self.d or not self._cache_serves(cache)):
+            return None
+        new = copy.copy(self)
+        new._layers = type(self._layers).from_buffer_copy(self._layers)
+        for i, at in enumerate(self._cache_layers):
+            new._layers[i].k_cache, new._layers[i].v_cache = cache.key_cache[at].data_ptr(), cache.value_cache[at].data_ptr()
+        new.desc = type(self.desc).from_buffer_copy(self.desc)
+        new.desc.layers = ctypes.cast(new._layers, ctypes.POINTER(_lib.MuiDecoderLayerDesc))
+        new.desc.cache_batch_stride, new.desc.cache_head_stride, new.desc.cache_token_stride = kc.stride()[:3]
+        new.desc.max_cache_len = new.max_cache_len = kc.shape[2]
+        new._bound(cache)
+        return new
+
+    def current(self, layers) -> bool:
+        """Whether everything is as it was when the descriptor was built."""
+        if len(layers) != len(self._layer_refs) or self._tables.cos32 is not self.cos32 or self._tables.sin32 is not self.sin32:
+            return False
+        for layer, r in zip(layers, self._layer_refs):
+            if layer is not r():
+                return False
+        if self._watched is None:
+            return False  # the first call did not come about
+        for r, children, tensors, values, objects in self._watched:
+            m = r()
+            if m is None:
+                return False
+            d = m.__dict__
+            mods, params = d["_modules"], d["_parameters"]
+            if len(mods) != len(children) or len(params) != len(tensors):
+                return False
+            for k, v in children:
+                if mods.get(k) is not v():
+                    return False
+            for k, v, p in tensors:
+                t = params.get(k)
+                if t is not v() or (p is not None and t.data_ptr() != p):
+                    return False
+            for k, v in values:
+                if d.get(k) is not v:
+                    return False
+            for k, v in objects:
+                if d.get(k) is not v():
+                    return False
+        return True
+
+    def holds(self, cache: MuiStaticCache) -> bool:
+        tensors = cache.tensors()
+        return (cache is self._cache() and len(tensors) == len(self._cache_tensors)
+                and all(t is r() and t.data_ptr() == p for t, (r, p) in zip(tensors, self._cache_tensors)))
+
+    def takes(self, hidden_states: torch.Tensor, position_ids: torch.Tensor, cache_position: torch.Tensor, key_mask: Optional[torch.Tensor]) -> bool:
+        """Whether this call can be made: its sizes, and nobody who listens to the modules."""
+        b, t = hidden_states.shape[0], hidden_states.shape[1]
+        if hidden_states.dtype != self.dtype or hidden_states.device != self.device or hidden_states.shape[2] != self.hidden:
+            return False
+        cache = self._cache()
+        if b > cache.max_batch_size or b > 65535 or t > self._most_tokens or not 1 <= b * t <= self._most_rows:
+            return False
+        if position_ids.dtype != torch.int64 or cache_position.dtype != torch.int64 or not (position_ids.is_cuda and cache_position.is_cuda):
+            return False
+        if tuple(position_ids.shape) not in ((1, t), (b, t)) or tuple(cache_position.shape) != (t,) or not cache_position.is_contiguous():
+            return False
+        if key_mask is not None and (key_mask.dtype != self.dtype or key_mask.dim() != 2 or key_mask.shape[0] != b or key_mask.stride(1) != 1
+                                     or key_mask.shape[1] < (cache.get_seq_length() + t + 3) // 4 * 4 or not key_mask.is_cuda):
+            return False
+        g = nn.modules.module
+        if g._global_forward_hooks or g._global_forward_pre_hooks:
+            return False
+        modules = [r() for r, *_ in self._watched] if self._watched else [m for r in self._layer_refs for m in r().modules()]
+        for m in modules:
+            d = m.__dict__
+            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
+                return False
+        return True
+
+    def run(self, hidden_in: torch.Tensor, position_ids: torch.Tensor, cache_position: torch.Tensor, seq_len: Optional[int],
+            mask: Optional[torch.Tensor]) -> torch.Tensor:
+        """hidden_in [B, T, hidden] -> output of the last layer [B, T, hidden]. mask: T > 1 a key mask (see mui_prefill_attention), T 1 additive."""
+        lib = self.lib
+        x = hidden_in.contiguous()
+        b, t = x.shape[0], x.shape[1]
+        stream = muillm_ext._stream(x)
+        n_splits = 1
+        if t == 1:
+            n_splits = lib.mui_flash_decode_splits(b, self.hq, self.hkv, int(seq_len if seq_len is not None else self.max_cache_len))
+            mask = None if mask is None else muillm_ext._mask_rows(mask, b, x.dtype)
+        ws = torch.empty(lib.mui_decoder_stack_prompt_bytes(ctypes.byref(self.desc), b, t, n_splits) + 256, dtype=torch.uint8, device=x.device)
+        linear_ws = muillm_ext._prompt_workspace(x, stream) if b * t > _lib.MUI_MAX_TOKENS else None
+        pos = position_ids.contiguous()
+        out = torch.empty_like(x)
+        muillm_ext.check(
+            lib.mui_decoder_stack_prompt(stream, ctypes.byref(self.desc), b, t, x.data_ptr(), out.data_ptr(), pos.data_ptr(),
+                                         t if pos.shape[0] > 1 else 0, cache_position.data_ptr(), -1 if seq_len is None else int(seq_len),
+                                         _ptr(mask), 0 if mask is None else mask.stride(0), n_splits, (ws.data_ptr() + 255) & ~255,
+                                         _ptr(linear_ws), 0 if linear_ws is None else linear_ws.numel()),
+            "mui_decoder_stack_prompt")
+        if self._watched is None:
+            self._watch()
         return out

@@ -22,13 +22,14 @@ import torch.nn as nn
 
 from .... import muillm_ext
 from ...._hf import (LlamaForCausalLM, LlamaModel, MistralForCausalLM, MistralModel, head_dim_of)
+from ...._lib import MUI_MAX_TOKENS
 from ....engineconfig import MuiEngineConfig
 from ....memorymanagement.gc import trigger_gc
 from ....replacement.replacementcontext import MuiReplacementContext
 from ...attention.rotaryembedding import MuiRotaryEmbedding, is_hf_static_cache
 from ...attention.sdpaattention import MuiSdpaAttention, _ignore_causal_mask_sdpa
 from ...decoder.decoder import MuiDecoderLayer
-from ...decoder.decoderstack import MuiDecoderStack
+from ...decoder.decoderstack import MuiDecoderStack, MuiPromptStack
 from ...embedding import MuiEmbedding
 from ...gateupdownmlp import MuiGateUpDownMLP
 from ...kvcache.cache_utils import (MuiCache, MuiStaticCache, create_static_cache,
@@ -106,6 +107,7 @@ class MuiLlamaModel(MuiModule):
         self.use_decoder_stack = True  # False: always walk the layer modules from Python
         self._stack: Optional[MuiDecoderStack] = None
         self._stack_rejected = None
+        self._prompt_layers = None  # what _prompt_stack has built
 
     def finalize_init(self):
         self.mdevice = self.embed_tokens.weight.device
@@ -157,6 +159,19 @@ class MuiLlamaModel(MuiModule):
         else:
             self._stack_rejected = key
         return self._stack
+
+    def _prompt_stack(self, cache, hidden_states, position_ids, cache_position, key_mask) -> Optional[MuiPromptStack]:
+        """The single-call layer stack for a prompt, or for a step of more batch rows than the decode kernels take; None: layer by layer."""
+        if (not self.use_decoder_stack or torch.is_grad_enabled() or not muillm_ext.PROMPT_NORM_FIRST or not hidden_states.is_cuda
+                or not isinstance(cache, MuiStaticCache)):
+            return None
+        st = self._prompt_layers
+        if st is not None and st.current(self.layers):
+            st = st if st.holds(cache) else st.bound_to(cache)
+        else:
+            st = MuiPromptStack(self.layers, self.rotary_emb, cache) if MuiPromptStack.eligible(self.layers, self.rotary_emb, cache) else None
+        self._prompt_layers = st
+        return st if st is not None and st.takes(hidden_states, position_ids, cache_position, key_mask) else None
 
     def _update_causal_mask(self, attention_mask, inputs_shape, cache_position, past_key_values,
                             output_attentions, all_ones_mask, past_seen_tokens: int,
@@ -265,16 +280,27 @@ class MuiLlamaModel(MuiModule):
             inputs_embeds = self.embed_tokens(input_ids)
         hidden_states = inputs_embeds
 
-        # shared position embeddings for the layers that take the unfused route
-        position_embeddings = None
-        if not (q_len == 1 and isinstance(past_key_values, MuiStaticCache) and hidden_states.is_cuda):
-            position_embeddings = self.rotary_emb(hidden_states, position_ids)
-
         all_hidden_states = () if output_hidden_states else None
         all_self_attns = () if output_attentions else None
         stack = None
         if q_len == 1 and use_cache and not output_hidden_states and not output_attentions:
             stack = self._decode_stack(past_key_values, batch_size, hidden_states)
+        prompt_stack = None
+        if stack is None and use_cache and not output_hidden_states and not output_attentions and (
+                batch_size > MUI_MAX_TOKENS if q_len == 1 else all_ones_mask or causal_mask is None or key_padding_mask is not None):
+            key_mask = None if all_ones_mask or q_len == 1 else key_padding_mask
+            prompt_stack = self._prompt_stack(past_key_values, hidden_states, position_ids, cache_position, key_mask)
+        # shared position embeddings for the layers that take the unfused route
+        position_embeddings = None
+        if prompt_stack is None and not (q_len == 1 and isinstance(past_key_values, MuiStaticCache) and hidden_states.is_cuda):
+            position_embeddings = self.rotary_emb(hidden_states, position_ids)
+        if prompt_stack is not None:
+            past_key_values._seen_tokens += q_len
+            if past_key_values.cpp_module is not None:
+                past_key_values.cpp_module.seen_tokens = past_key_values._seen_tokens
+            seen = None if q_len == 1 and past_key_values.device_length_mode else past_key_values._seen_tokens
+            mask = key_mask if q_len > 1 or all_ones_mask else causal_mask
+            hidden_states = prompt_stack.run(hidden_states, position_ids, cache_position, seen, mask)
         if stack is not None:
             # every layer through one library call (what the loop below does, layer by layer)
             past_key_values._seen_tokens += 1
@@ -283,7 +309,7 @@ class MuiLlamaModel(MuiModule):
             seq_len = None if past_key_values.device_length_mode else past_key_values._seen_tokens
             hidden_states = stack.step(hidden_states, position_ids, cache_position, seq_len,
                                        None if all_ones_mask else causal_mask)
-        for decoder_layer in (self.layers if stack is None else ()):
+        for decoder_layer in (self.layers if stack is None and prompt_stack is None else ()):
             if output_hidden_states:
                 all_hidden_states += (hidden_states,)
             layer_outputs = decoder_layer(

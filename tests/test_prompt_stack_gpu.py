@@ -1,0 +1,140 @@
+"""Prompts, and steps of more rows than the decode kernels take, through one library call against the same layers called one by one: plain and int8 weights, several
+turns, padding, captured steps; and what has to stay with the single layers. The two run the same products and sums: the same bits."""
+
+import pytest
+import torch
+
+from muillm_amd.engine import init_engine
+from muillm_amd.engineconfig import MuiEngineConfig
+from muillm_amd.modules.decoder.decoderstack import MuiPromptStack
+from muillm_amd.modules.models.graphdecoder import MuiGraphDecoder
+from muillm_amd.modules.models.llama.model import MuiDecoderConfig, MuiLlamaForCausalLM
+from muillm_amd.quantization.quantizationmethod import Int8WeightOnlyQuantizationMethod
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _lm(dtype=torch.bfloat16, group=None, **kw):
+    cfg = MuiDecoderConfig(**{**dict(hidden_size=512, intermediate_size=1280, num_hidden_layers=3, num_attention_heads=4, num_key_value_heads=2, vocab_size=512,
+                                     max_position_embeddings=2048), **kw})
+    lm = MuiLlamaForCausalLM.from_config(MuiEngineConfig(), cfg, dtype=dtype, device=DEV, seed=0, init_std=0.05, finalize=group is None)
+    if group is None:
+        return lm
+    method = Int8WeightOnlyQuantizationMethod(group_size=group, modules=["qkv_proj", "o_proj", "mlp"])
+    return init_engine(lm, device=DEV, engine_config=MuiEngineConfig(method))
+
+
+def _ids(b, t, seed=3):
+    return torch.randint(0, 512, (b, t), generator=torch.Generator().manual_seed(seed)).to(DEV)
+
+
+def _run(lm, one_call, turns, capacity, batch, mask=None):
+    """Logits of every turn and the cache, and whether the stack has run."""
+    calls = []
+    plain = MuiPromptStack.run
+
+    def counted(self, *a):
+        calls.append(a[0].shape)
+        return plain(self, *a)
+
+    lm.model.use_decoder_stack = one_call
+    MuiPromptStack.run = counted
+    try:
+        cache = lm.create_cache(batch, capacity)
+        out = [lm(input_ids=ids, past_key_values=cache, attention_mask=mask if i == 0 else None, all_ones_mask=mask is None).logits.float()
+               for i, ids in enumerate(turns)]
+        seen = cache.get_seq_length()
+        return torch.cat(out, 1), torch.stack(cache.tensors())[..., :seen, :].float(), len(calls), seen
+    finally:
+        MuiPromptStack.run = plain
+        lm.model.use_decoder_stack = True
+
+
+def _off(a, b):
+    return float((a - b).norm() / b.norm())
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "int8", "int8_group"])
+@pytest.mark.parametrize("batch,lengths", [(1, [5]), (1, [16]), (1, [17]), (3, [6]), (1, [101, 2, 40]), (2, [64, 65]), (1, [300]), (20, [1, 1]), (17, [3, 1])])
+def test_same_as_layer_by_layer(kind, batch, lengths):
+    lm = _lm(torch.bfloat16 if kind == "bf16" else torch.float16, {"int8": 0, "int8_group": 128}.get(kind))
+    turns = [_ids(batch, t, seed=t + i) for i, t in enumerate(lengths)]
+    got, cache, calls, seen = _run(lm, True, turns, 512, batch)
+    want, cache_want, none, seen_want = _run(lm, False, turns, 512, batch)
+    assert calls == len(turns) and none == 0 and seen == seen_want == sum(lengths)
+    assert torch.equal(got, want) and torch.equal(cache, cache_want)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("t", [40, 150])
+def test_padded_prompts(t):
+    lm, batch = _lm(), 4
+    ids = _ids(batch, t)
+    mask = torch.ones(batch, t, dtype=torch.int64, device=DEV)
+    mask[0, :t // 2] = 0
+    mask[2, :3] = 0
+    got, _, calls, _ = _run(lm, True, [ids * mask], 512, batch, mask)
+    want, _, _, _ = _run(lm, False, [ids * mask], 512, batch, mask)
+    assert calls == 1
+    live = mask.bool()
+    assert torch.equal(got[live], want[live])
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("padded", [False, True])
+def test_captured_steps_of_many_rows(padded):
+    lm, batch, t = _lm(), 20, 7
+    ids = _ids(batch, t)
+    mask = None
+    if padded:
+        mask = torch.ones(batch, t, dtype=torch.int64, device=DEV)
+        mask[::2, :3] = 0
+        ids = ids * mask
+    tokens = []
+    for graph in (True, False):
+        decoder = MuiGraphDecoder(lm, use_graph=graph)
+        for _ in range(2):
+            cache = lm.create_cache(batch, 64)
+            decoder.prefill(ids, 12, cache, attention_mask=mask)
+            decoder.decode(11)
+            tokens.append(decoder.out_tokens.clone())
+    assert all(torch.equal(tokens[0], x) for x in tokens[1:])
+
+
+@torch.no_grad()
+def test_what_stays_layer_by_layer():
+    lm = _lm()
+    ids = _ids(1, 30)
+    want = _run(lm, True, [ids], 64, 1)[0]
+    heard = []
+    for m in (lm.model.layers[1], lm.model.layers[0].self_attn.o_proj, lm.model.layers[2].qkv_proj.linear, lm.model.layers[2].mlp):
+        handle = m.register_forward_hook(lambda mod, args, out: heard.append(mod))
+        got, _, calls, _ = _run(lm, True, [ids], 64, 1)
+        handle.remove()
+        assert calls == 0 and heard.pop() is m and torch.equal(got, want)
+    lm.model.layers[0].mlp.forward = lm.model.layers[0].mlp.forward
+    assert _run(lm, True, [ids], 64, 1)[2] == 0
+    del lm.model.layers[0].mlp.forward
+    assert _run(lm, True, [ids], 64, 1)[2] == 1
+    # another cache, a larger one: bound to it without a look at the layers
+    stack = lm.model._prompt_layers
+    for capacity, batch in ((64, 1), (512, 3)):
+        got, cache, calls, _ = _run(lm, True, [_ids(batch, 30)], capacity, batch)
+        other = _run(lm, False, [_ids(batch, 30)], capacity, batch)
+        assert calls == 1 and lm.model._prompt_layers._watched is stack._watched and torch.equal(got, other[0]) and torch.equal(cache, other[1])
+    # hidden states are asked for, no cache, gradients are on
+    assert len(lm(input_ids=ids, output_hidden_states=True).hidden_states) == 4
+    with torch.enable_grad():
+        assert _run(lm, True, [ids], 64, 1)[2] == 0
+    # weights replaced behind the stack's back: the parameter, its storage
+    lm.model.layers[0].mlp.down_proj.weight.data = lm.model.layers[0].mlp.down_proj.weight.data * 1.5
+    got, _, calls, _ = _run(lm, True, [ids], 64, 1)
+    assert calls == 1 and torch.equal(got, _run(lm, False, [ids], 64, 1)[0]) and _off(got, want) > 0.02
+    want = got
+    layer = lm.model.layers[1].self_attn.o_proj
+    layer.weight = torch.nn.Parameter(layer.weight * 2, requires_grad=False)
+    layer.finalize_init()
+    got, _, calls, _ = _run(lm, True, [ids], 64, 1)
+    assert calls == 1 and torch.equal(got, _run(lm, False, [ids], 64, 1)[0]) and _off(got, want) > 0.02
