@@ -15,8 +15,8 @@
 // the routing does.
 //
 // Products, wave64 v_mfma_f32_16x16x32 (weights = A rows, pairs = B columns):
-//   tile 16   up to 16 pairs of an expert: 16 gate + 16 up rows (or 32 rows) per workgroup, K dealt out to
-//             its four waves, operands straight from global memory in matrix order. Decode and short
+//   tile 16   up to 16 pairs of an expert: 16 gate + 16 up rows (or 32 rows) at a time by a workgroup, K dealt out to
+//             its four waves, rows in runs of 256 bytes through LDS. Decode and short
 //             prompts: every chosen expert's weights are streamed once.
 //   tile 128 / 256   as many pairs x as many rows, both operands through swizzled LDS stages filled by
 //             LDS-direct loads; waves of 64 x 64, or of 128 x 64 with operands read a half step ahead.
@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(256) moe_route_kernel(const float* logits, con
 }
 
 // One workgroup: (ROUTE: the routing of all tokens, then) count per expert, cut into tiles, scatter.
-// tiles[0].count = number of tiles, tiles[1 + i] the i-th tile; unused entries up to max_tiles get count 0.
+// tiles[0].count = number of tiles, tiles[0].pad: some expert has several; tiles[1 + i] the i-th tile, unused entries up to max_tiles get count 0.
 constexpr int kChosen = 1024;
 template <typename T, bool ROUTE>
 __global__ void __launch_bounds__(kRouteThreads) moe_group_kernel(const float* logits, const typename T::storage* corr,
@@ -221,7 +221,10 @@ __global__ void __launch_bounds__(kRouteThreads) moe_group_kernel(const float* l
     }
     if (t == 0) n_tiles_s = tile_base < max_tiles ? tile_base : max_tiles;
   }
-  __syncthreads();
+  // whether an expert has several tiles
+  int several = 0;
+  for (int e = t; e < n_experts; e += nt_threads) several |= count[e] > tile_pairs;
+  several = __syncthreads_or(several);
   const int n_tiles = n_tiles_s;
   for (int e = t; e < n_experts; e += nt_threads) {
     const int c = count[e], base = cursor[e], ft = first_tile[e];
@@ -231,7 +234,7 @@ __global__ void __launch_bounds__(kRouteThreads) moe_group_kernel(const float* l
     }
   }
   for (int i = n_tiles + t; i < max_tiles; i += nt_threads) tiles[1 + i] = MoeTile{0, 0, 0, 0};
-  if (t == 0) tiles[0] = MoeTile{0, 0, n_tiles, 0};
+  if (t == 0) tiles[0] = MoeTile{0, 0, n_tiles, several != 0};
   __syncthreads();  // cursors are read above before they move
   for (int i = t; i < n_pairs; i += nt_threads) {
     const int e = expert_of(i);
@@ -269,22 +272,27 @@ __device__ __forceinline__ MoeTile moe_tile_at(const MoeGemmParams& p, int i, in
 // bytes arrive at about two thirds of the rate.
 constexpr int kT16Seg = 128;
 template <typename T, int EPI>
-__global__ void __launch_bounds__(256, 2) moe_tile16_kernel(const MoeGemmParams p) {
+__global__ void __launch_bounds__(256, 2) moe_tile16_kernel(const MoeTile* tiles, const uint16_t* w0, const uint16_t* w1, long expert_stride, int n, int k, int max_tiles,
+                                                            int once, const int32_t* pairs, const uint16_t* x, MoeGemmParams p) {
+  p.tiles = tiles; p.w0 = w0; p.w1 = w1; p.expert_stride = expert_stride; p.n = n; p.k = k; p.max_tiles = max_tiles; p.once = once; p.pairs = pairs; p.x = x;
   constexpr int ROWS = EPI == MOE_GATEUP ? 16 : 32;  // outputs per workgroup
   // [wave][tile]; the stages are arrays of their own, so that the compiler can tell which loads a read waits for
   __shared__ __align__(16) uint16_t wl0[4][2][16 * kT16Seg], wl1[4][2][16 * kT16Seg];
   __shared__ int prow[16];
-  const MoeTile tile = moe_tile_at(p, blockIdx.y, 16);
-  if (tile.count <= 0) return;
+  MoeTile tile;
   // Gate and up rows that only this tile reads, in this call and the next, are requested non-temporally: 38.6 -> 36.8 us for 1 token, 8 of 64 experts of
-  // 1792 x 4096 (the down product gained nothing). An expert's further tiles find the rows in L2 only if they are requested
+  // 1792 x 4096 (the down product gained nothing here). An expert's further tiles find the rows in L2 only if they are requested
   // ordinarily: 95 tokens that favour 20 of the experts 180 us, 225 with all rows non-temporal.
   bool alone = false;
   if constexpr (EPI == MOE_GATEUP) {
     // (entries requested together: tile i is entry i + 1, entry 0 holds their count)
     const int i = (int)blockIdx.y, count = p.tiles[0].count, before = p.tiles[i].expert, behind = p.tiles[i + 1 < p.max_tiles ? i + 2 : i + 1].expert;
+    tile = p.tiles[1 + i];
     alone = p.once & ((i == 0) | (before != tile.expert)) & ((i + 1 >= count) | (behind != tile.expert));
+  } else {
+    tile = moe_tile_at(p, blockIdx.y, 16);
   }
+  if (tile.count <= 0) return;
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int r16 = lane & 15, g = lane >> 4;
   const int o0 = blockIdx.x * ROWS;
@@ -382,6 +390,164 @@ __global__ void __launch_bounds__(256, 2) moe_tile16_kernel(const MoeGemmParams 
     if (n0 < p.n) ((float*)p.y)[out + n0] = v0 + (p.bias ? T::one(p.bias[n0]) : 0.f);
     if (n1 < p.n) ((float*)p.y)[out + n1] = v1 + (p.bias ? T::one(p.bias[n1]) : 0.f);
   }
+}
+
+// The same tiles for K in whole segments (four at least), by a round of workgroups, two per CU, that take the units (tile, block of rows) blockIdx, blockIdx + grid, ..
+// The segments run on across units: while a unit's partial tiles meet in LDS, the next one's first segment is on its way, and tiles that are not there cost nothing.
+// A wave takes every fourth segment of its workgroup's units, counted through (so it has some of every unit). Rows go through registers to LDS: of a
+// wave that has loads into LDS and loads into registers (the pairs' operands) under way the compiler waits for ALL where it needs one of the latter, and
+// every second segment drained the wave.
+// Bound by the weight stream (7.1 TB/s at best). Rows that only one unit reads, in this call and the next, are requested non-temporally, of down too: ordinarily
+// 4096 x 1792, 8 / 50 tokens of 8 experts, 96 / 158 us, non-temporally 85 / 143. An expert's further tiles find the rows in L2 only if they are requested ordinarily; where
+// there are any it is decided by unit (the branch costs 1 to 2 % of gate and up). us of gate and up / down, a workgroup per tile and block before -> now, 64
+// experts: 4096 x 1792, 8 of them per token, 1 token 41.2 / 23.9 -> 39.2 / 20.6, 8 tokens 176.7 / 94.1 -> 169.8 / 85.4, 50 tokens 287 / 156 -> 273 / 143;
+// 2048 x 1408, 6 per token, 1 token 17.1 / 10.3 -> 15.4 / 9.7, 8 tokens 67.8 / 36.7 -> 62.0 / 31.4, 50 tokens 125.9 / 66.5 -> 120 / 57.6. Three workgroups per CU: the same to 5 % more.
+template <typename T, int EPI>
+__global__ void __launch_bounds__(256, 2) moe_units_kernel(const MoeTile* tiles, const uint16_t* w0, const uint16_t* w1, long expert_stride, const int32_t* pairs, int n, int k,
+                                                           const uint16_t* x, int top, int blocks, int max_tiles, int once, float limit, uint16_t* y) {
+  constexpr int ROWS = EPI == MOE_GATEUP ? 16 : 32;  // outputs per unit
+  __shared__ __align__(16) uint16_t wl[4][2][16 * kT16Seg];
+  __shared__ float red[4][2][16][17];
+  typedef const __attribute__((address_space(4))) MoeTile ConstTile;
+  ConstTile* list = (ConstTile*)(uintptr_t)tiles;
+  const int grid = gridDim.x, units = list[0].count * blocks;
+  if ((int)blockIdx.x >= units) return;
+  const int t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int segs = k / kT16Seg;
+  // how rows are requested: 0 ordinarily, 1 non-temporally, 2 by unit
+  auto run = [&](auto how) {
+    constexpr int HOW = decltype(how)::value;
+
+    // a unit as the loads need it
+    struct Unit { int id, o0, count, first; bool alone; const uint8_t *b0, *b1; };
+    auto unit_at = [&](int id) {
+      Unit u;
+      u.id = id < units ? id : units - 1;  // (past the last: one that is there; what comes of it is not used)
+      const int ti = u.id / blocks;
+      u.o0 = (u.id - ti * blocks) * ROWS;
+      const int expert = list[1 + ti].expert;
+      u.first = list[1 + ti].first;
+      u.count = list[1 + ti].count;
+      if constexpr (HOW == 2) {
+        const int before = list[ti].expert, behind = list[ti + 1 < max_tiles ? ti + 2 : ti + 1].expert;
+        u.alone = (ti == 0 || before != expert) && (u.id + blocks >= units || behind != expert);
+      } else {
+        u.alone = HOW == 1;
+      }
+      const long at = (long)expert * expert_stride + (long)u.o0 * k;
+      u.b0 = (const uint8_t*)(w0 + at);
+      u.b1 = EPI == MOE_GATEUP ? (const uint8_t*)(w1 + at) : u.b0;
+      return u;
+    };
+    auto pair_of = [&](const Unit& u) { return pairs + u.first + (r16 < u.count ? r16 : 0); };
+    Unit lu = unit_at(blockIdx.x), nu = unit_at(blockIdx.x + grid);  // the unit that is loaded, and the one after it
+    int lpair = *pair_of(lu), npair = *pair_of(nu);
+    int ls = wave;
+    unsigned woff[2][4], xoff;
+    auto place = [&]() {  // this lane's rows of the unit: load instruction q of a tile takes rows 4 q + lane / 16, 256 bytes each
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = 4 * q + g, last = n - 1 - lu.o0, chunk = (r16 ^ r) * 8;
+        woff[0][q] = (unsigned)((r < last ? r : last) * k + chunk) * 2u;
+        if constexpr (EPI != MOE_GATEUP) woff[1][q] = (unsigned)((16 + r < last ? 16 + r : last) * k + chunk) * 2u;
+        else woff[1][q] = woff[0][q];
+      }
+      xoff = (unsigned)((EPI == MOE_GATEUP ? lpair / top : lpair) * k + 8 * g) * 2u;
+    };
+    place();
+    struct Segment { u32x4 w[2][4], x[4]; } s0, s1;
+    // the next segment of this wave
+    auto issue = [&](Segment& sg) {
+      if (ls >= segs) {
+        ls -= segs;
+        lu = nu;
+        lpair = npair;
+        nu = unit_at(lu.id + grid);
+        place();
+      }
+      npair = *pair_of(nu);  // (again with every segment: a value that is loaded only sometimes has to be waited for where the ways meet)
+      const int kb = ls * (kT16Seg * 2);
+      auto rows = [&](auto stream) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            unsigned off = woff[j][q];
+            asm volatile("" : "+v"(off));  // (kept a 32-bit lane offset from a scalar base)
+            sg.w[j][q] = ld16_sel<decltype(stream)::value>((j ? lu.b1 : lu.b0) + kb + off);
+          }
+      };
+      if constexpr (HOW == 2) {
+        if (lu.alone) rows(std::true_type());
+        else rows(std::false_type());
+      } else {
+        rows(std::integral_constant<bool, HOW == 1>());
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sg.x[u] = ld16((const uint16_t*)((const uint8_t*)x + kb + 64 * u + xoff));
+      ls += 4;
+      asm volatile("" ::: "memory");  // the loads stay in front of what follows
+    };
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    int cid = lu.id, cs = wave, ccount = lu.count, co0 = lu.o0, cpair = lpair;  // the unit that is multiplied
+    // true at the end of the last unit
+    auto step = [&](const Segment& sg) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *(u32x4*)&wl[wave][j][q * 4 * kT16Seg + lane * 8] = sg.w[j][q];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = mfma16x16x32<T>(*(const u32x4*)&wl[wave][j][r16 * kT16Seg + ((4 * u + g) ^ r16) * 8], sg.x[u], acc[j]);
+      cs += 4;
+      if (cs < segs) return false;
+      cs -= segs;
+      // ---- end of a unit; these barriers do not wait for the loads on their way
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();  // the unit before has been read
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        red[wave][0][4 * g + r][r16] = acc[0][r];
+        red[wave][1][4 * g + r][r16] = acc[1][r];
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const int row = t & 15, col = t >> 4;
+      float v0 = 0.f, v1 = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) { v0 += red[w][0][row][col]; v1 += red[w][1][row][col]; }
+      const long out = (long)__shfl(cpair, col) * n;
+      if (col < ccount) {
+        if constexpr (EPI == MOE_GATEUP) {
+          if (co0 + row < n) y[out + co0 + row] = T::pack(moe_act(v0, v1, limit));
+        } else {
+          if (co0 + row < n) y[out + co0 + row] = T::pack(v0);
+          if (co0 + 16 + row < n) y[out + co0 + 16 + row] = T::pack(v1);
+        }
+      }
+      acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      // (the segment requested last is this wave's first of the next unit)
+      cid += grid;
+      ccount = lu.count;
+      co0 = lu.o0;
+      cpair = lpair;
+      return cid >= units;
+    };
+    issue(s0);
+    while (true) {
+      issue(s1);
+      if (step(s0)) break;
+      issue(s0);
+      if (step(s1)) break;
+    }
+  };
+  if (!once) run(std::integral_constant<int, 0>());
+  else if (!list[0].pad) run(std::integral_constant<int, 1>());
+  else run(std::integral_constant<int, 2>());
 }
 
 // NWR x NWT waves of 64 rows x 64 pairs each (gate/up: a wave's rows are 32 gate rows and the 32 up rows of the
@@ -774,6 +940,11 @@ __global__ void __launch_bounds__(256) moe_rows_kernel(const typename T::storage
   if (lane == 0) y[pair * n + row] = T::pack(s0);
 }
 
+template <typename T, int EPI>
+static void launch_moe_tile16(hipStream_t s, dim3 grid, const MoeGemmParams& p) {
+  hipLaunchKernelGGL((moe_tile16_kernel<T, EPI>), grid, dim3(256), 0, s, p.tiles, p.w0, p.w1, p.expert_stride, p.n, p.k, p.max_tiles, (int)p.once, p.pairs, p.x, p);
+}
+
 template <typename T, int EPI, int NWR, int NWT>
 static int launch_moe_tile(hipStream_t s, const MoeGemmParams& p) {
   constexpr int OUT = (EPI == MOE_GATEUP ? 32 : 64) * NWR, SUP = NWT == 2 ? 4 : 2;
@@ -807,8 +978,15 @@ static int launch_moe_product(hipStream_t s, const MoeGemmParams& p, const int32
   if constexpr (T::kDtype != MUI_DTYPE_F32) {
     if (tile_pairs == 16) {
       if (p.max_tiles > 65535) return MUI_ERR_UNSUPPORTED;
-      hipLaunchKernelGGL((moe_tile16_kernel<T, EPI>), dim3(ceil_div(p.n, EPI == MOE_GATEUP ? 16 : 32), p.max_tiles),
-                         dim3(256), 0, s, p);
+      const int blocks = ceil_div(p.n, EPI == MOE_GATEUP ? 16 : 32);
+      const long units = (long)blocks * p.max_tiles, xrows = EPI == MOE_GATEUP ? p.tokens : (long)p.tokens * p.top;
+      if (p.tiles && p.k % kT16Seg == 0 && p.k >= 4 * kT16Seg && (long)p.n * p.k < (1L << 30) && xrows * p.k < (1L << 30) && units < (1L << 30)) {
+        const long round = 2L * device_cus();
+        hipLaunchKernelGGL((moe_units_kernel<T, EPI>), dim3((unsigned)(units < round ? units : round)), dim3(256), 0, s, p.tiles, p.w0, p.w1, p.expert_stride,
+                           p.pairs, p.n, p.k, p.x, p.top, blocks, p.max_tiles, (int)p.once, p.limit, (uint16_t*)p.y);
+        return launch_status();
+      }
+      launch_moe_tile16<T, EPI>(s, dim3(blocks, p.max_tiles), p);
       return launch_status();
     }
     if (((uintptr_t)p.y & 7) != 0) return MUI_ERR_ALIGNMENT;
@@ -840,7 +1018,7 @@ static int launch_linear_f32(hipStream_t s, const void* w, const void* x, const 
       p.top = 1; p.tokens = tokens;
       const int tiles = ceil_div(tokens, 16);
       if (tiles > 65535) return MUI_ERR_UNSUPPORTED;
-      hipLaunchKernelGGL((moe_tile16_kernel<T, MOE_F32>), dim3(ceil_div(n, 32), tiles), dim3(256), 0, s, p);
+      launch_moe_tile16<T, MOE_F32>(s, dim3(ceil_div(n, 32), tiles), p);
       return launch_status();
     }
   }
@@ -938,6 +1116,15 @@ extern "C" int mui_moe_route(mui_stream_t stream, int dtype, const float* logits
                                  expert, weight, pairs, (MoeTile*)tiles)));
 }
 
+// Whether a layer's experts (n x k each) are too large to be found in the memory-side cache at the next call:
+// that cache holds 256 MB: the experts of eight layers and more of 32 MB don't stay there. Below (8 experts of 512 x 1024, 17 MB) a model may stay:
+// 4 tokens 4.7 us ordinary, 5.1 non-temporal while it does, 5.5 either way when it does not
+// Rows that are no whole cache lines share one at their ends and where two runs meet: non-temporal it came twice (64 experts of 1000 x 2000, 1 token each
+// for 32 of them 16.1 us ordinary, 17.8 non-temporal, 100 tokens of 2 137 and 148).
+static bool read_once(int n_experts, int n, int k, const void* a, const void* b) {
+  return (long)n_experts * n * k * 4 > (32L << 20) && k % 64 == 0 && (((uintptr_t)a | (uintptr_t)b) & 127) == 0;
+}
+
 extern "C" int mui_moe_gateup(mui_stream_t stream, int dtype, const void* gate, const void* up, long expert_stride,
                               const void* x, float limit, const int32_t* expert, const int32_t* pairs,
                               const void* tiles, int tile_pairs, void* act, int n_experts, int n_inter, int k_in,
@@ -948,11 +1135,7 @@ extern "C" int mui_moe_gateup(mui_stream_t stream, int dtype, const void* gate, 
   p.w0 = (const uint16_t*)gate; p.w1 = (const uint16_t*)up; p.expert_stride = expert_stride; p.x = (const uint16_t*)x;
   p.y = act; p.pairs = pairs; p.tiles = (const MoeTile*)tiles; p.n = n_inter; p.k = k_in; p.top = top; p.tokens = tokens;
   p.limit = limit; p.max_tiles = mui_moe_max_tiles(tokens, top, n_experts, tile_pairs);
-  // that cache holds 256 MB: the experts of eight layers and more of 32 MB don't stay there. Below (8 experts of 512 x 1024, 17 MB) a model may stay:
-  // 4 tokens 4.7 us ordinary, 5.1 non-temporal while it does, 5.5 either way when it does not
-  // Rows that are no whole cache lines share one at their ends and where two runs meet: non-temporal it came twice (64 experts of 1000 x 2000, 1 token each
-  // for 32 of them 16.1 us ordinary, 17.8 non-temporal, 100 tokens of 2 137 and 148).
-  p.once = (long)n_experts * n_inter * k_in * 4 > (32L << 20) && k_in % 64 == 0 && (((uintptr_t)gate | (uintptr_t)up) & 127) == 0;
+  p.once = read_once(n_experts, n_inter, k_in, gate, up);
   MUI_BY_DTYPE((launch_moe_product<TT, MOE_GATEUP>((hipStream_t)stream, p, expert, n_experts, tokens * top, tile_pairs)));
 }
 
@@ -965,5 +1148,6 @@ extern "C" int mui_moe_down(mui_stream_t stream, int dtype, const void* down, lo
   p.w0 = (const uint16_t*)down; p.expert_stride = expert_stride; p.x = (const uint16_t*)act; p.y = out; p.pairs = pairs;
   p.tiles = (const MoeTile*)tiles; p.n = n_out; p.k = k_in; p.top = top; p.tokens = tokens;
   p.max_tiles = mui_moe_max_tiles(tokens, top, n_experts, tile_pairs);
+  p.once = read_once(n_experts, n_out, k_in, down, down);
   MUI_BY_DTYPE((launch_moe_product<TT, MOE_DOWN>((hipStream_t)stream, p, expert, n_experts, tokens * top, tile_pairs)));
 }

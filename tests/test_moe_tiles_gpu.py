@@ -66,3 +66,46 @@ def test_neighbouring_tiles_of_one_expert(width, ff, experts, dtype):
         ref = (a * torch.sigmoid(1.702 * a) * (u + 1.0)).to(dtype).double() @ down[e].double().T
         err = float((out[rows].double() - ref).abs().max() / ref.abs().max())
         assert err <= REL[dtype], f"expert {e}, {counts[e]} pairs: {err:.2e}"
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("width,ff,experts,counts", [
+    (512, 640, 5, [3, 0, 16, 1, 2]),               # four and five segments: every wave has one of every unit; fewer units than workgroups
+    (768, 520, 7, [0, 0, 0, 0, 0, 0, 1]),          # one tile; k of down in no whole segments (a workgroup per block)
+    (2048, 1152, 24, [1] * 24),                    # more units than workgroups, gate and up beyond 32 MB: all rows non-temporal
+    (2048, 1152, 24, [2, 17, 0, 40] + [1] * 20),   # ... and by unit: experts with one tile and with several
+    (1032, 2056, 12, [5, 1, 33] + [0] * 9)])       # blocks that end inside the matrix; no whole segments
+def test_units_of_a_round_of_workgroups(width, ff, experts, counts, dtype):
+    g = torch.Generator().manual_seed(width + ff)
+    tokens = sum(counts)
+    chosen = torch.repeat_interleave(torch.arange(experts), torch.tensor(counts))[torch.randperm(tokens, generator=g)]
+    logits = torch.full((tokens, experts), -4.0).scatter_(1, chosen[:, None], 4.0)
+    x = torch.randn(tokens, width, generator=g).to(dtype).to(DEV)
+    gate, up = (torch.randn(experts, ff, width, generator=g).mul_(width ** -0.5).to(dtype).to(DEV) for _ in range(2))
+    down = torch.randn(experts, width, ff, generator=g).mul_(ff ** -0.5).to(dtype).to(DEV)
+    expert, _, pairs, tiles = ops.moe_route(logits.to(DEV), None, experts, 1, 16)
+    assert int(tiles[0, 3]) == (max(counts) > 16)
+    for _ in range(2):
+        out = ops.moe_experts(x, gate, up, down, 7.0, expert, pairs, tiles, 16)
+        for e in range(experts):
+            rows = (chosen == e).nonzero()[:, 0].to(DEV)
+            if not len(rows):
+                continue
+            xe = x[rows].double()
+            a = (xe @ gate[e].double().T).clamp(max=7.0)
+            u = (xe @ up[e].double().T).clamp(-7.0, 7.0)
+            ref = (a * torch.sigmoid(1.702 * a) * (u + 1.0)).to(dtype).double() @ down[e].double().T
+            err = float((out[rows].double() - ref).abs().max() / ref.abs().max())
+            assert err <= REL[dtype], f"expert {e}, {counts[e]} pairs: {err:.2e}"
+
+
+def test_units_without_a_tile():
+    """All tokens choose identity experts: nothing is written."""
+    experts, width, ff, tokens = 4, 512, 512, 3
+    logits = torch.full((tokens, experts + 1), -4.0)
+    logits[:, experts] = 4.0
+    expert, _, pairs, tiles = ops.moe_route(logits.to(DEV), None, experts, 1, 16)
+    assert int(tiles[0, 2]) == 0
+    w = torch.ones(experts, ff, width, dtype=torch.bfloat16, device=DEV)
+    ops.moe_experts(torch.ones(tokens, width, dtype=torch.bfloat16, device=DEV), w, w, w, 7.0, expert, pairs, tiles, 16)
+    torch.cuda.synchronize()
