@@ -256,23 +256,27 @@ class MuiPromptStack(MuiDecoderStack):
         self._most_rows = min(muillm_ext.INT8_DEQUANT_MIN_TOKENS, muillm_ext.INT8_GROUP_DEQUANT_MIN_TOKENS) - 1 if int8 else 1 << 30
         self._most_tokens = min([65535] + [x.self_attn.prefill_kernel_max_tokens for x in layers if x.self_attn.prefill_kernel_max_tokens is not None])
 
-    def _watch(self) -> None:
-        """(Made behind the first call, while the GPU is at work.)"""
+    def remember(self) -> None:
+        """What current() compares with. (Made behind the first call, while the GPU is at work.)"""
+        if self._watched is not None:
+            return
+
         def weak(v) -> bool:
             return isinstance(v, (torch.Tensor, nn.Module)) or hasattr(v, "__weakref__")
 
         def ref(v):
             return weakref.ref(v) if weak(v) else (lambda: v)
 
-        self._watched = []  # per module: itself, its children, its tensors with their addresses, what else was read from it
+        watched = []  # per module: itself, its children, its tensors with their addresses, what else was read from it
         for layer in [r() for r in self._layer_refs]:
             qkv, attn, mlp = layer.qkv_proj, layer.self_attn, layer.mlp
             inside = [getattr(mlp, n) for n in ("gate_proj", "up_proj", "down_proj") if isinstance(getattr(mlp, n, None), nn.Module)]
             for m in [layer, qkv, qkv.linear, attn, attn.o_proj, mlp] + inside:
-                self._watched.append((weakref.ref(m), [(k, ref(v)) for k, v in m._modules.items()],
-                                      [(k, ref(v), _ptr(v)) for k, v in m._parameters.items()],
-                                      [(k, m.__dict__[k]) for k in self._ATTRIBUTES if k in m.__dict__ and not weak(m.__dict__[k])],
-                                      [(k, weakref.ref(m.__dict__[k])) for k in self._ATTRIBUTES if k in m.__dict__ and weak(m.__dict__[k])]))
+                watched.append((weakref.ref(m), [(k, ref(v)) for k, v in m._modules.items()],
+                                [(k, ref(v), _ptr(v)) for k, v in m._parameters.items()],
+                                [(k, m.__dict__[k]) for k in self._ATTRIBUTES if k in m.__dict__ and not weak(m.__dict__[k])],
+                                [(k, weakref.ref(m.__dict__[k])) for k in self._ATTRIBUTES if k in m.__dict__ and weak(m.__dict__[k])]))
+        self._watched = watched  # whole: another thread may ask meanwhile
 
     @staticmethod
     def eligible(layers, rotary_emb, cache) -> bool:
@@ -408,6 +412,5 @@ class MuiPromptStack(MuiDecoderStack):
                                          _ptr(mask), 0 if mask is None else mask.stride(0), n_splits, (ws.data_ptr() + 255) & ~255,
                                          _ptr(linear_ws), 0 if linear_ws is None else linear_ws.numel()),
             "mui_decoder_stack_prompt")
-        if self._watched is None:
-            self._watch()
+        self.remember()
         return out

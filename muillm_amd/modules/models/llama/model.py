@@ -171,7 +171,10 @@ class MuiLlamaModel(MuiModule):
         else:
             st = MuiPromptStack(self.layers, self.rotary_emb, cache) if MuiPromptStack.eligible(self.layers, self.rotary_emb, cache) else None
         self._prompt_layers = st
-        return st if st is not None and st.takes(hidden_states, position_ids, cache_position, key_mask) else None
+        if st is None or st.takes(hidden_states, position_ids, cache_position, key_mask):
+            return st
+        st.remember()  # the next call need not examine the layers either
+        return None
 
     def _update_causal_mask(self, attention_mask, inputs_shape, cache_position, past_key_values,
                             output_attentions, all_ones_mask, past_seen_tokens: int,

@@ -138,3 +138,17 @@ def test_what_stays_layer_by_layer():
     layer.finalize_init()
     got, _, calls, _ = _run(lm, True, [ids], 64, 1)
     assert calls == 1 and torch.equal(got, _run(lm, False, [ids], 64, 1)[0]) and _off(got, want) > 0.02
+
+
+@torch.no_grad()
+def test_layers_are_examined_once_where_calls_are_refused():
+    lm, built = _lm(), []
+    handle = lm.model.layers[1].register_forward_hook(lambda *a: None)
+    examine = MuiPromptStack.eligible
+    MuiPromptStack.eligible = staticmethod(lambda *a: built.append(1) or examine(*a))
+    try:
+        assert [_run(lm, True, [_ids(1, 30)], 64, 1)[2] for _ in range(3)] == [0, 0, 0] and len(built) == 1
+        handle.remove()
+        assert _run(lm, True, [_ids(1, 30)], 64, 1)[2] == 1 and len(built) == 1
+    finally:
+        MuiPromptStack.eligible = staticmethod(examine)
