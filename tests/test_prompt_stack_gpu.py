@@ -141,6 +141,19 @@ def test_what_stays_layer_by_layer():
 
 
 @torch.no_grad()
+def test_forward_mode_is_refused_as_by_the_modules():
+    """The linears have no forward-mode rule: a tangent on the way in is an error, never lost."""
+    lm = _lm()
+    embeds = lm.model.embed_tokens(_ids(1, 30))
+    for one_call in (True, False):
+        lm.model.use_decoder_stack = one_call
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(embeds, torch.ones_like(embeds))
+            with pytest.raises(NotImplementedError):
+                lm.model(inputs_embeds=dual, past_key_values=lm.create_cache(1, 64), use_cache=True, all_ones_mask=True)
+
+
+@torch.no_grad()
 def test_layers_are_examined_once_where_calls_are_refused():
     lm, built = _lm(), []
     handle = lm.model.layers[1].register_forward_hook(lambda *a: None)
