@@ -90,6 +90,11 @@ class MuiCausalLMOutput:
     loss: Optional[torch.Tensor] = None
 
 
+# Products of a layer and a first prompt (rows x weights) from which the GPU is longer at work on a layer (~200 us) than the host on its modules: such a
+# prompt runs on the modules, and the layers are examined for the single call behind it (~35 us per layer) instead of in front of it, with an idle GPU.
+_BUSY_PRODUCTS = 10 ** 11
+
+
 class MuiLlamaModel(MuiModule):
     def __init__(self, engine_config: MuiEngineConfig, config, embed_tokens: nn.Embedding, layers,
                  norm: MuiRMSNorm, rotary_emb: MuiRotaryEmbedding):
@@ -161,7 +166,8 @@ class MuiLlamaModel(MuiModule):
         return self._stack
 
     def _prompt_stack(self, cache, hidden_states, position_ids, cache_position, key_mask) -> Optional[MuiPromptStack]:
-        """The single-call layer stack for a prompt, or for a step of more batch rows than the decode kernels take; None: layer by layer."""
+        """The single-call layer stack for a prompt, or for a step of more batch rows than the decode kernels take; None: layer by layer;
+        False: layer by layer, and _examine_layers() behind it."""
         if (not self.use_decoder_stack or torch.is_grad_enabled() or not muillm_ext.PROMPT_NORM_FIRST or not hidden_states.is_cuda
                 or not isinstance(cache, MuiStaticCache)):
             return None
@@ -169,12 +175,18 @@ class MuiLlamaModel(MuiModule):
         if st is not None and st.current(self.layers):
             st = st if st.holds(cache) else st.bound_to(cache)
         else:
-            st = MuiPromptStack(self.layers, self.rotary_emb, cache) if MuiPromptStack.eligible(self.layers, self.rotary_emb, cache) else None
+            hidden, inner = hidden_states.shape[-1], getattr(self.config, "intermediate_size", 0)
+            if hidden_states.shape[0] * hidden_states.shape[1] * hidden * (3 * inner + 2 * hidden) > _BUSY_PRODUCTS:
+                return False
+            st = self._examine_layers(cache)
         self._prompt_layers = st
         if st is None or st.takes(hidden_states, position_ids, cache_position, key_mask):
             return st
         st.remember()  # the next call need not examine the layers either
         return None
+
+    def _examine_layers(self, cache) -> Optional[MuiPromptStack]:
+        return MuiPromptStack(self.layers, self.rotary_emb, cache) if MuiPromptStack.eligible(self.layers, self.rotary_emb, cache) else None
 
     def _update_causal_mask(self, attention_mask, inputs_shape, cache_position, past_key_values,
                             output_attentions, all_ones_mask, past_seen_tokens: int,
@@ -288,11 +300,12 @@ class MuiLlamaModel(MuiModule):
         stack = None
         if q_len == 1 and use_cache and not output_hidden_states and not output_attentions:
             stack = self._decode_stack(past_key_values, batch_size, hidden_states)
-        prompt_stack = None
+        prompt_stack, examine_behind = None, False
         if stack is None and use_cache and not output_hidden_states and not output_attentions and (
                 batch_size > MUI_MAX_TOKENS if q_len == 1 else all_ones_mask or causal_mask is None or key_padding_mask is not None):
             key_mask = None if all_ones_mask or q_len == 1 else key_padding_mask
             prompt_stack = self._prompt_stack(past_key_values, hidden_states, position_ids, cache_position, key_mask)
+        examine_behind, prompt_stack = prompt_stack is False, prompt_stack or None
         # shared position embeddings for the layers that take the unfused route
         position_embeddings = None
         if prompt_stack is None and not (q_len == 1 and isinstance(past_key_values, MuiStaticCache) and hidden_states.is_cuda):
@@ -328,6 +341,11 @@ class MuiLlamaModel(MuiModule):
             hidden_states = self.norm(hidden_states)
         if output_hidden_states:
             all_hidden_states += (hidden_states,)
+        if examine_behind:
+            st = self._examine_layers(past_key_values)
+            if st is not None:
+                st.remember()
+            self._prompt_layers = st
         if use_cache and isinstance(past_key_values, MuiCache):
             past_key_values.sync_back()
         return MuiModelOutput(last_hidden_state=hidden_states,

@@ -165,3 +165,17 @@ def test_layers_are_examined_once_where_calls_are_refused():
         assert _run(lm, True, [_ids(1, 30)], 64, 1)[2] == 1 and len(built) == 1
     finally:
         MuiPromptStack.eligible = staticmethod(examine)
+
+
+@torch.no_grad()
+def test_first_long_prompt_runs_on_the_modules(monkeypatch):
+    """... and has the layers examined behind it: the second one goes by the single call, with the same bits."""
+    from muillm_amd.modules.models.llama import model as llama
+
+    rows, per_row = 150, 512 * (3 * 1280 + 2 * 512)
+    for most, calls_first in ((rows * per_row, 1), (rows * per_row - 1, 0)):
+        monkeypatch.setattr(llama, "_BUSY_PRODUCTS", most)
+        lm, ids = _lm(), _ids(1, rows)
+        first, second = _run(lm, True, [ids], 256, 1), _run(lm, True, [ids], 256, 1)
+        assert first[2] == calls_first and second[2] == 1
+        assert torch.equal(first[0], second[0]) and torch.equal(first[1], second[1])
