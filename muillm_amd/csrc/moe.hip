@@ -394,7 +394,8 @@ __global__ void __launch_bounds__(256, 2) moe_tile16_kernel(const MoeTile* tiles
 
 // The same tiles for K in whole segments (four at least), by a round of workgroups, two per CU, that take the units (tile, block of rows) blockIdx, blockIdx + grid, ..
 // The segments run on across units: while a unit's partial tiles meet in LDS, the next one's first segment is on its way, and tiles that are not there cost nothing.
-// A wave takes every fourth segment of its workgroup's units, counted through (so it has some of every unit). Rows go through registers to LDS: of a
+// A wave takes every fourth segment of its workgroup's units, counted through (so it has some of every unit): which of a unit's four runs of segments that is moves on from unit to
+// unit where their number is no multiple of four. Partial tiles are kept by run and added in the order of the runs: a row's sums don't depend on where its tile stands. Rows go through registers to LDS: of a
 // wave that has loads into LDS and loads into registers (the pairs' operands) under way the compiler waits for ALL where it needs one of the latter, and
 // every second segment drained the wave.
 // Bound by the weight stream (7.1 TB/s at best). Rows that only one unit reads, in this call and the next, are requested non-temporally, of down too: ordinarily
@@ -407,7 +408,7 @@ __global__ void __launch_bounds__(256, 2) moe_units_kernel(const MoeTile* tiles,
                                                            const uint16_t* x, int top, int blocks, int max_tiles, int once, float limit, uint16_t* y) {
   constexpr int ROWS = EPI == MOE_GATEUP ? 16 : 32;  // outputs per unit
   __shared__ __align__(16) uint16_t wl[4][2][16 * kT16Seg];
-  __shared__ float red[4][2][16][17];
+  __shared__ float red[4][2][16][17];  // by run of segments
   typedef const __attribute__((address_space(4))) MoeTile ConstTile;
   ConstTile* list = (ConstTile*)(uintptr_t)tiles;
   const int grid = gridDim.x, units = list[0].count * blocks;
@@ -490,7 +491,7 @@ __global__ void __launch_bounds__(256, 2) moe_units_kernel(const MoeTile* tiles,
       asm volatile("" ::: "memory");  // the loads stay in front of what follows
     };
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    int cid = lu.id, cs = wave, ccount = lu.count, co0 = lu.o0, cpair = lpair;  // the unit that is multiplied
+    int cid = lu.id, cs = wave, run_of = wave, ccount = lu.count, co0 = lu.o0, cpair = lpair;  // the unit that is multiplied
     // true at the end of the last unit
     auto step = [&](const Segment& sg) {
 #pragma unroll
@@ -510,9 +511,10 @@ __global__ void __launch_bounds__(256, 2) moe_units_kernel(const MoeTile* tiles,
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        red[wave][0][4 * g + r][r16] = acc[0][r];
-        red[wave][1][4 * g + r][r16] = acc[1][r];
+        red[run_of][0][4 * g + r][r16] = acc[0][r];
+        red[run_of][1][4 * g + r][r16] = acc[1][r];
       }
+      run_of = cs;
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");

@@ -109,3 +109,24 @@ def test_units_without_a_tile():
     w = torch.ones(experts, ff, width, dtype=torch.bfloat16, device=DEV)
     ops.moe_experts(torch.ones(tokens, width, dtype=torch.bfloat16, device=DEV), w, w, w, 7.0, expert, pairs, tiles, 16)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("width,ff", [(2176, 1152), (2048, 1408), (2304, 1280)])  # gate/up, down: 17 and 9 segments, 16 and 11, 18 and 10
+def test_a_rows_bits_beside_other_rows(width, ff, dtype):
+    """Alone a token's units are a workgroup's first; among others they come later, where the waves hold other segments of them."""
+    experts = 24
+    g = torch.Generator().manual_seed(width + ff)
+    x = torch.randn(experts, width, generator=g).to(dtype).to(DEV)
+    gate, up = (torch.randn(experts, ff, width, generator=g).mul_(width ** -0.5).to(dtype).to(DEV) for _ in range(2))
+    down = torch.randn(experts, width, ff, generator=g).mul_(ff ** -0.5).to(dtype).to(DEV)
+    logits = torch.full((experts, experts), -4.0).fill_diagonal_(4.0).to(DEV)
+
+    def run(rows):
+        expert, _, pairs, tiles = ops.moe_route(logits[rows].contiguous(), None, experts, 1, 16)
+        return ops.moe_experts(x[rows].contiguous(), gate, up, down, 7.0, expert, pairs, tiles, 16)
+
+    together = run(list(range(experts)))
+    for e in (3, 11, 19, 23):
+        assert torch.equal(run([e])[0], together[e]), f"expert {e}"
+        assert torch.equal(run(list(range(e, experts)))[0], together[e]), f"expert {e} first"
