@@ -32,7 +32,6 @@ struct StreamParams {
   uint16_t* y;
   float* part;     // [k_splits][tokens][n] where K is divided between workgroups
   bool add;        // a launch behind this one adds the partial outputs up (else the caller's does)
-  bool free_add;   // ... and would run anyway
   int n, k, tokens;
   int n_units;     // bands of ROWS weight rows (gate/up: gate and up rows together)
   int k_splits;    // more than one: every workgroup has one unit, a share of K of one band
@@ -391,8 +390,7 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int
       if (g_stream_shares && k != g_stream_shares) continue;
       const float one = (float)p.k / k * 2.f * ((float)r / 27.5e3f + 16.f * nt / (nt > 4 ? 82e3f : 105e3f));
       const float barriers = (float)p.k / k / (r + 16 * nt <= 96 ? 256 : 128) * 0.08f;
-      const float shares = k > 1 ? (p.free_add ? 0.f : 2.5f) + 0.3f * k + (float)k * p.tokens * p.n * 8.f / 4e6f : p.free_add ? 2.5f : 0.f;
-      const float cost = ceil_div(units, cus) * (one + barriers + 1.f) + shares;
+      const float cost = ceil_div(units, cus) * (one + barriers + 1.f) + (k > 1 ? 2.5f + 0.3f * k + (float)k * p.tokens * p.n * 8.f / 4e6f : 0.f);
       if (width == 0 || cost < best) { best = cost; width = r; p.n_units = units; p.k_splits = k; }
     }
   }
@@ -452,11 +450,10 @@ int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParam
 }
 
 // The same for a caller whose next launch adds the partial outputs up itself: part [*splits][tokens][n] gets the products, nothing else is applied.
-// free_add: that launch runs whether K is divided or not (without: K is divided as by launch_gemm_stream). MUI_ERR_UNSUPPORTED also where K is better left undivided.
-int launch_gemm_stream_parts(hipStream_t s, int dtype, const SkinnyParams& q, float* part, size_t part_bytes, bool free_add, int* splits) {
+// K is divided as by launch_gemm_stream; MUI_ERR_UNSUPPORTED also where it is left undivided.
+int launch_gemm_stream_parts(hipStream_t s, int dtype, const SkinnyParams& q, float* part, size_t part_bytes, int* splits) {
   if (!part || !stream_serves(q, 128)) return MUI_ERR_UNSUPPORTED;
-  StreamParams p = stream_params(q, part, false);
-  p.free_add = free_add;
+  const StreamParams p = stream_params(q, part, false);
   if (dtype == MUI_DTYPE_F16) return launch_stream_t<F16, SK_LINEAR>(s, p, part_bytes, splits);
   if (dtype == MUI_DTYPE_BF16) return launch_stream_t<BF16, SK_LINEAR>(s, p, part_bytes, splits);
   return MUI_ERR_UNSUPPORTED;

@@ -6,10 +6,11 @@
 // With 17 to 128 tokens the linear divides its K between workgroups wherever that is worth a launch that adds the fp32 partial
 // outputs up (gemm_stream.hip). That launch and the norm's are one here: one workgroup per token adds the token's row up and has it in registers for
 // the norms. Neither is bound by its bytes (a few hundred KB per row at most); each is a launch, a chain of cold loads and one or two sums over the
-// workgroup, so one of them is what is saved. With an fp32 stream K is now also divided where it was not because of the adding launch. Everything
-// else runs as the two calls it stands for. us in bf16 as captured, two calls -> one, at 32 / 128 tokens: with an fp32 stream 4096 x 4096 14.5 -> 12.5 / 22.1 -> 19.8,
-// 4096 x 14336 27.4 -> 25.0 / 39.3 -> 36.8, 2048 x 2048 9.7 -> 8.5 / 14.4 -> 11.4, 2048 x 8192 14.2 -> 11.9 / 22.1 -> 19.7; with a 16-bit one 4096 x 4096 (K not
-// divided / divided) 13.6 -> 13.6 / 21.0 -> 19.1, 4096 x 14336 26.4 -> 24.5 / 38.3 -> 36.3, 2048 x 8192 13.9 -> 11.7 / 21.5 -> 19.1.
+// workgroup, so one of them is what is saved. Everything else runs as the two calls it stands for, and K is divided as without the norm: the bits are those of the two
+// calls. (Dividing it also where only the adding launch spoke against it gave 14.8 -> 12.5 us for 4096 x 4096 at 32 tokens, and other sums than a model whose boundaries are not
+// taken along.) us in bf16 as captured, two calls -> one, at 32 / 128 tokens: with an fp32 stream 4096 x 4096 (K undivided / divided) 14.8 -> 14.6 / 22.6 -> 19.9,
+// 4096 x 14336 28.5 -> 25.1 / 39.4 -> 36.8, 2048 x 2048 (undivided) 9.7 -> 9.7 / 14.4 -> 14.4, 2048 x 8192 14.4 -> 12.1 / 22.2 -> 19.7; with a 16-bit one 4096 x 4096
+// 13.7 -> 13.5 / 21.5 -> 19.4, 4096 x 14336 27.5 -> 25.4 / 38.6 -> 36.4, 2048 x 8192 13.8 -> 11.8 / 22.1 -> 19.3.
 #include "skinny.cuh"
 
 namespace mui {
@@ -194,8 +195,8 @@ static int linear_join(hipStream_t s, int dtype, const void* weights, long w_pit
   SkinnyParams q = {};
   q.w0 = weights; q.pitch = w_pitch; q.x = (const uint16_t*)x; q.y = p.y; q.n = p.n; q.k = k; q.tokens = p.tokens;
   float* part = (float*)((char*)workspace + prefill_counter_bytes());
-  // (with a 16-bit stream K is divided only where it is without the norm, too: layers called one by one and all in one call give the same bits)
-  const int st = launch_gemm_stream_parts(s, dtype, q, part, workspace_bytes - prefill_counter_bytes(), f32, &p.splits);
+  // (K is divided only where it is without the norm, too: whether the boundary was taken along, a hook was listening or all layers came in one call does not show in the bits)
+  const int st = launch_gemm_stream_parts(s, dtype, q, part, workspace_bytes - prefill_counter_bytes(), &p.splits);
   if (st != MUI_OK) return st;
   p.part = part;
   if (dtype == MUI_DTYPE_F16) return f32 ? launch_join<F16, true>(s, p) : launch_join<F16, false>(s, p);

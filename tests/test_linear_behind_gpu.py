@@ -68,6 +68,34 @@ def test_against_64_bits(n, k, tokens, dtype):
     assert not bool(ws[:4096].any())  # the counters
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [17, 20, 32, 48, 64, 65, 97, 128])
+@pytest.mark.parametrize("n,k", [(1024, 14336), (2048, 2048), (2048, 8192), (4096, 4096), (4096, 14336), (8192, 1024)])
+def test_same_bits_as_the_two_calls(n, k, tokens, dtype):
+    """K divided (long K, few outputs) and undivided: what is taken along is what two calls give, bit for bit."""
+    g = _gen(n + k + tokens)
+    w, x, res = _rand((n, k), dtype, g, k ** -0.5), _rand((tokens, k), dtype, g), _rand((tokens, n), dtype, g)
+    post, after = 1 + _rand((n,), dtype, g, 0.2), 1 + _rand((n,), dtype, g, 0.2)
+    stream = torch.empty(tokens, n, device=DEV).normal_(0.0, 1.0, generator=g)
+    ws = torch.zeros(_lib.load().mui_linear_workspace_bytes(), dtype=torch.uint8, device=DEV)
+    lib, s, code = _lib.load(), torch.cuda.current_stream().cuda_stream, CODE[dtype]
+
+    def linear(residual):
+        y = torch.empty_like(res)
+        _lib.check(lib.mui_linear_ws(s, code, w.data_ptr(), k, x.data_ptr(), None, 0.0, None, None, _ptr(residual), y.data_ptr(), n, k, tokens, ws.data_ptr(), ws.numel()), "linear")
+        return y
+
+    y, h, out = torch.empty_like(res), torch.empty_like(res), torch.empty_like(stream)
+    y2, h2, out2 = linear(res), torch.empty_like(res), torch.empty_like(stream)
+    _lib.check(lib.mui_rmsnorm(s, code, after.data_ptr(), y2.data_ptr(), EPS, h2.data_ptr(), tokens, n), "norm")
+    _call("mui_linear_norm", x, w, k, None, (res.data_ptr(), after.data_ptr(), EPS, y.data_ptr(), h.data_ptr()), y, ws)
+    assert torch.equal(y, y2) and torch.equal(h, h2)
+    y2 = linear(None)
+    _lib.check(lib.mui_residual_norm(s, code, stream.data_ptr(), y2.data_ptr(), 1.0, post.data_ptr(), 0.5, after.data_ptr(), 2.0, EPS, out2.data_ptr(), h2.data_ptr(), tokens, n), "norm")
+    _call("mui_linear_residual_norm", x, w, k, None, (stream.data_ptr(), post.data_ptr(), 0.5, after.data_ptr(), 2.0, EPS, y.data_ptr(), out.data_ptr(), h.data_ptr()), y, ws)
+    assert torch.equal(y, y2) and torch.equal(out, out2) and torch.equal(h, h2)
+
+
 def test_in_place_and_empty_rows():
     """The stream may be updated in place; a row of zeros stays one."""
     g = _gen(1)
