@@ -524,7 +524,8 @@ int mui_decoder_stack_step(mui_stream_t stream, const mui_decoder_stack_t* model
 
 /* The same layers for any number of rows: prompts (tokens > 1: RoPE and cache write, then causal attention over the cache) and steps of more batch
  * rows than MUI_MAX_TOKENS (tokens 1). hidden_in, hidden_out: [batch, tokens, hidden]; position_ids: [batch or 1, tokens], rows position_batch_stride
- * apart (0: one row for all); cache_position: [tokens] slots. seq_len: tokens in the cache, these included (tokens 1 also -1: read from cache_position on the device).
+ * apart (0: one row for all); cache_position: [tokens] slots. seq_len: tokens in the cache, these included (tokens 1 also -1: read from cache_position on the device), at most model's
+ * max_cache_len.
  * mask: NULL; with tokens > 1 the key mask of mui_prefill_attention_masked, with tokens 1 the additive rows of mui_decoder_stack_step.
  * workspace: mui_decoder_stack_prompt_bytes bytes, 256-byte aligned; linear_workspace: as mui_linear_ws's, or NULL. int8 projections convert on the way
  * whatever the number of rows. On an error part of the layers may have been enqueued. */

@@ -173,6 +173,7 @@ extern "C" int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_s
   MUI_CHECK_ARG(batch >= 1 && tokens >= 1 && n_splits >= 1 && position_ids && cache_position);
   MUI_CHECK_ARG(((uintptr_t)workspace & 255u) == 0 && (long)batch * tokens <= (1L << 30));
   MUI_CHECK_ARG(tokens == 1 || seq_len >= tokens);
+  MUI_CHECK_ARG(seq_len <= m->max_cache_len);  // (the prompt's attention takes no capacity: it reads seq_len rows of every head)
   const int rows = batch * tokens;
   const PromptWorkspace w = carve_rows(m, batch, tokens, n_splits, (char*)workspace);
   const int hid = m->hidden, qd = m->n_q_heads * m->head_dim, kvd = m->n_kv_heads * m->head_dim, qkv_n = qd + 2 * kvd;

@@ -377,6 +377,8 @@ class MuiPromptStack(MuiDecoderStack):
         cache = self._cache()
         if b > cache.max_batch_size or b > 65535 or t > self._most_tokens or not 1 <= b * t <= self._most_rows:
             return False
+        if cache.get_seq_length() + t > self.max_cache_len:
+            return False  # the modules refuse to read a cache beyond its rows
         if position_ids.dtype != torch.int64 or cache_position.dtype != torch.int64 or not (position_ids.is_cuda and cache_position.is_cuda):
             return False
         if tuple(position_ids.shape) not in ((1, t), (b, t)) or tuple(cache_position.shape) != (t,) or not cache_position.is_contiguous():

@@ -1,0 +1,48 @@
+"""What the descriptors of the single-call layer stacks are made from, and when they no longer hold. Examined on the CPU with tensors that say they are on a GPU: nothing is launched."""
+import ctypes
+
+import pytest
+import torch
+
+from muillm_amd import _lib
+from muillm_amd.engineconfig import MuiEngineConfig
+from muillm_amd.modules.decoder.decoderstack import MuiDecoderStack, MuiPromptStack
+from muillm_amd.modules.models.llama.model import MuiDecoderConfig, MuiLlamaForCausalLM
+
+
+def _lm(**kw):
+    cfg = MuiDecoderConfig(**{**dict(hidden_size=512, intermediate_size=1280, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2, vocab_size=32,
+                                     max_position_embeddings=128), **kw})
+    return MuiLlamaForCausalLM.from_config(MuiEngineConfig(), cfg, dtype=torch.bfloat16, device="cpu", seed=0, init_std=0.05).eval()
+
+
+@pytest.fixture
+def lm(monkeypatch):
+    lm = _lm()
+    lm.cache = lm.create_cache(2, 64)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
+    for rotary in [lm.model.rotary_emb] + [layer.self_attn.rotary_emb for layer in lm.model.layers]:
+        rotary.dispatchable = True
+    for layer in lm.model.layers:
+        layer.mlp.dispatchable = True
+    return lm
+
+
+def _prompt_stack(lm):
+    assert MuiPromptStack.eligible(lm.model.layers, lm.model.rotary_emb, lm.cache)
+    return MuiPromptStack(lm.model.layers, lm.model.rotary_emb, lm.cache)
+
+
+def _takes(stack, t=20, b=1):
+    ids = torch.arange(t)
+    with torch.no_grad():
+        return stack.takes(torch.zeros(b, t, 512, dtype=torch.bfloat16), ids[None], ids, None)
+
+
+def test_no_row_beyond_the_cache_is_read(lm):
+    stack, at = _prompt_stack(lm), ctypes.c_void_p(256)
+    for tokens, seq_len in ((20, 65), (64, 1 << 20), (1, 65)):
+        status = _lib.load().mui_decoder_stack_prompt(None, ctypes.byref(stack.desc), 1, tokens, at, at, at, 0, at, seq_len, None, 0, 1, at, None, 0)
+        assert status == -1  # MUI_ERR_INVALID_ARG, and nothing enqueued
+    lm.cache.set_seen_tokens(44)
+    assert _takes(stack, 20) and not _takes(stack, 21)
