@@ -64,6 +64,33 @@ def _linear_fields(m):
     return m.weight, m.weight.stride(0), None, [(m, "weight", m.weight)]
 
 
+def _layer_sizes(layer) -> Optional[tuple]:
+    """(hidden, query heads, key / value heads, intermediate) of a layer, or None where its tensors are of other sizes: kernels go by the sizes that a descriptor states."""
+    qkv, attn, mlp = layer.qkv_proj.linear, layer.self_attn, layer.mlp
+    hidden, inter = qkv.in_features, mlp.intermediate_size
+    q, kv = attn.num_heads * attn.head_dim, attn.num_key_value_heads * attn.head_dim
+
+    def fits(m, n: int, k: int) -> bool:
+        if type(m) is not MuiInt8Linear:
+            return m.weight.shape == (n, k)
+        if m.per_channel:
+            return m.weights_int8.shape == (n, k) and m.scales.shape == (n,)
+        return m.weights_uint8.shape == (n, k) and m.scales_min_vals.numel() == 2 * n * (k >> m.quantizer.group_size_shift)
+
+    if not (fits(qkv, q + 2 * kv, hidden) and fits(attn.o_proj, hidden, q) and fits(mlp.down_proj, hidden, inter)):
+        return None
+    if layer.qkv_proj.slice_starts != [0, q, q + kv] or qkv.norm_weights.shape != (hidden,) or mlp.norm_weights.shape != (hidden,):
+        return None
+    if type(mlp) is MuiGateUpDownMLP:
+        if not (fits(mlp.gate_proj, inter, hidden) and fits(mlp.up_proj, inter, hidden)):
+            return None
+    elif mlp.gate_up_weights.shape != (inter, 2, hidden) or (
+            mlp.gate_up_scales.shape != (inter, 2) if mlp.per_channel
+            else mlp.gate_up_scales_min_vals.numel() != 4 * inter * (hidden >> mlp.group_size_shift)):
+        return None
+    return hidden, attn.num_heads, attn.num_key_value_heads, inter
+
+
 def _ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
@@ -136,13 +163,13 @@ class MuiDecoderStack:
 
     @staticmethod
     def eligible(layers, rotary_emb, cache, batch: int) -> bool:
-        """fp16 / bf16 Llama-shaped layers without biases on a static cache, head_dim 128; every
-        projection 16-bit or int8 (per-channel, or the reference's group format)."""
+        """fp16 / bf16 Llama-shaped layers of one size without biases on a static cache, head_dim 128;
+        every projection 16-bit or int8 (per-channel, or the reference's group format)."""
         if not isinstance(cache, MuiStaticCache) or len(layers) == 0 or batch > _lib.MUI_MAX_TOKENS:
             return False
         if not getattr(rotary_emb, "dispatchable", False):
             return False
-        eps, dtype = None, None
+        eps, dtype, sizes = None, None, None
         for layer in layers:
             qkv, attn, mlp = getattr(layer, "qkv_proj", None), getattr(layer, "self_attn", None), getattr(layer, "mlp", None)
             if type(qkv) is not MuiMultiLinear or not _plain_linear(qkv.linear, True):
@@ -174,6 +201,10 @@ class MuiDecoderStack:
             if cache.key_cache[attn.layer_idx].dtype != w.dtype or (dtype is not None and w.dtype != dtype):
                 return False
             dtype = w.dtype
+            of = _layer_sizes(layer)
+            if of is None or (sizes is not None and of != sizes):
+                return False
+            sizes = of
             for m in (qkv.linear, attn.o_proj, mlp.down_proj):
                 if type(m) is MuiInt8Linear:
                     wd = m.scales.dtype if m.per_channel else m.scales_min_vals.dtype

@@ -46,3 +46,34 @@ def test_no_row_beyond_the_cache_is_read(lm):
         assert status == -1  # MUI_ERR_INVALID_ARG, and nothing enqueued
     lm.cache.set_seen_tokens(44)
     assert _takes(stack, 20) and not _takes(stack, 21)
+
+
+def _eligible(lm):
+    found = [MuiDecoderStack.eligible(lm.model.layers, lm.model.rotary_emb, lm.cache, 1), MuiPromptStack.eligible(lm.model.layers, lm.model.rotary_emb, lm.cache)]
+    assert found[0] == found[1]
+    return found[0]
+
+
+def test_layers_of_other_sizes(lm, monkeypatch):
+    """One descriptor states the sizes of all layers: a narrower one would be read beyond its ends."""
+    assert _eligible(lm)
+    layer = lm.model.layers[1]
+    with monkeypatch.context() as m:
+        m.undo()
+        narrow, more_heads = _lm(intermediate_size=640).model.layers[1], _lm(num_key_value_heads=4).model.layers[1]
+    narrow.mlp.dispatchable = more_heads.self_attn.rotary_emb.dispatchable = True
+    mlp, layer.mlp = layer.mlp, narrow.mlp
+    assert not _eligible(lm)
+    layer.mlp = mlp
+    qkv, attn = layer.qkv_proj, layer.self_attn
+    layer.qkv_proj, layer.self_attn = more_heads.qkv_proj, more_heads.self_attn
+    assert not _eligible(lm)
+    layer.qkv_proj, layer.self_attn = qkv, attn
+    assert _eligible(lm)
+    # tensors that are not of their modules' sizes
+    for m, name in ((mlp.gate_proj, "weight"), (mlp.down_proj, "weight"), (attn.o_proj, "weight"), (qkv.linear, "weight"), (mlp, "norm_weights"), (qkv.linear, "norm_weights")):
+        plain = getattr(m, name)
+        setattr(m, name, torch.nn.Parameter(plain.detach()[:8], requires_grad=False))
+        assert not _eligible(lm), (type(m), name)
+        setattr(m, name, plain)
+    assert _eligible(lm)

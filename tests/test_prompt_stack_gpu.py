@@ -141,6 +141,15 @@ def test_what_stays_layer_by_layer():
 
 
 @torch.no_grad()
+def test_layers_that_differ():
+    lm, other = _lm(), _lm(intermediate_size=640)
+    lm.model.layers[1].mlp = other.model.layers[1].mlp
+    got, cache, calls, _ = _run(lm, True, [_ids(1, 30)], 64, 1)
+    want, cache_want, _, _ = _run(lm, False, [_ids(1, 30)], 64, 1)
+    assert calls == 0 and torch.equal(got, want) and torch.equal(cache, cache_want)
+
+
+@torch.no_grad()
 def test_forward_mode_is_refused_as_by_the_modules():
     """The linears have no forward-mode rule: a tangent on the way in is an error, never lost."""
     lm = _lm()
