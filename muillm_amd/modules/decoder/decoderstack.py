@@ -91,6 +91,18 @@ def _layer_sizes(layer) -> Optional[tuple]:
     return hidden, attn.num_heads, attn.num_key_value_heads, inter
 
 
+def _rotate_with(attentions, cos, sin) -> bool:
+    """Whether all of them still rotate with these tables (looked up past nn.Module's slow attribute access: asked before every call)."""
+    for attn in attentions:
+        rotary = attn.__dict__["_modules"].get("rotary_emb")
+        if rotary is None:
+            return False
+        d = rotary.__dict__
+        if d.get("cos32") is not cos or d.get("sin32") is not sin:
+            return False
+    return True
+
+
 def _ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
@@ -108,7 +120,8 @@ class MuiDecoderStack:
         self.batch = batch
         self.hidden = first.qkv_proj.linear.in_features
         self.hq, self.hkv, self.d = attn0.num_heads, attn0.num_key_value_heads, attn0.head_dim
-        self.cos32, self.sin32 = rotary_emb.cos32, rotary_emb.sin32
+        self.cos32, self.sin32 = attn0.rotary_emb.cos32, attn0.rotary_emb.sin32
+        self._attentions = [layer.self_attn for layer in layers]
         kc0 = cache.key_cache[0]
         cb, chs, cts = kc0.stride(0), kc0.stride(1), kc0.stride(2)
         self.max_cache_len = kc0.shape[2]
@@ -169,7 +182,7 @@ class MuiDecoderStack:
             return False
         if not getattr(rotary_emb, "dispatchable", False):
             return False
-        eps, dtype, sizes = None, None, None
+        eps, dtype, sizes, tables = None, None, None, None
         for layer in layers:
             qkv, attn, mlp = getattr(layer, "qkv_proj", None), getattr(layer, "self_attn", None), getattr(layer, "mlp", None)
             if type(qkv) is not MuiMultiLinear or not _plain_linear(qkv.linear, True):
@@ -178,6 +191,11 @@ class MuiDecoderStack:
                 return False
             if attn.head_dim != 128:
                 return False
+            # a layer rotates with its own module's tables: they have to be the same for all
+            rotary = attn.rotary_emb
+            if not rotary.dispatchable or (tables is not None and (rotary.cos32 is not tables[0] or rotary.sin32 is not tables[1])):
+                return False
+            tables = (rotary.cos32, rotary.sin32)
             if type(mlp) is MuiGateUpDownMLP:
                 if not all(_plain_linear(m, False) and type(m) is MuiLinear for m in (mlp.gate_proj, mlp.up_proj)):
                     return False
@@ -233,6 +251,8 @@ class MuiDecoderStack:
         for owner, name, obj in self._owners:
             if getattr(owner, name, None) is not obj:
                 return False
+        if not _rotate_with(self._attentions, self.cos32, self.sin32):
+            return False
         ptrs = tuple(t.data_ptr() for t in cache.key_cache) + tuple(t.data_ptr() for t in cache.value_cache)
         return ptrs == self._cache_ptrs
 
@@ -282,7 +302,7 @@ class MuiPromptStack(MuiDecoderStack):
         self._watched, self._layer_refs = None, [weakref.ref(layer) for layer in layers]
         self._cache_layers = [layer.self_attn.layer_idx for layer in layers]
         self._bound(cache)
-        self._tables = rotary_emb
+        self._attentions = None  # (layers are held weakly here)
         int8 = any(type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP)
                    for layer in layers for m in (layer.qkv_proj.linear, layer.self_attn.o_proj, layer.mlp, layer.mlp.down_proj))
         self._most_rows = min(muillm_ext.INT8_DEQUANT_MIN_TOKENS, muillm_ext.INT8_GROUP_DEQUANT_MIN_TOKENS) - 1 if int8 else 1 << 30
@@ -320,6 +340,9 @@ class MuiPromptStack(MuiDecoderStack):
         for layer in layers:
             qkv, attn, mlp = layer.qkv_proj.linear, layer.self_attn, layer.mlp
             if type(layer) is not MuiDecoderLayer or type(attn) is not MuiSdpaAttention or attn.training:
+                return False
+            rotary, handle = attn.rotary_emb, attn.rotary_emb.cpp_module  # (prompts rotate by what the handle names)
+            if handle is None or handle.cos32 is not rotary.cos32 or handle.sin32 is not rotary.sin32 or handle.layer_idx != attn.layer_idx:
                 return False
             if type(mlp) is MuiGateUpDownMLP and (not mlp.dispatchable or mlp.method == _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED):
                 return False
@@ -363,13 +386,21 @@ class MuiPromptStack(MuiDecoderStack):
 
     def current(self, layers) -> bool:
         """Whether everything is as it was when the descriptor was built."""
-        if len(layers) != len(self._layer_refs) or self._tables.cos32 is not self.cos32 or self._tables.sin32 is not self.sin32:
+        if len(layers) != len(self._layer_refs):
             return False
         for layer, r in zip(layers, self._layer_refs):
             if layer is not r():
                 return False
         if self._watched is None:
             return False  # the first call did not come about
+        attentions = [layer.__dict__["_modules"].get("self_attn") for layer in layers]
+        if None in attentions or not _rotate_with(attentions, self.cos32, self.sin32):
+            return False
+        for attn in attentions:
+            rotary = attn.__dict__["_modules"]["rotary_emb"].__dict__
+            handle = rotary["cpp_module"]
+            if handle is None or handle.cos32 is not self.cos32 or handle.sin32 is not self.sin32 or handle.layer_idx != attn.layer_idx or not rotary["dispatchable"]:
+                return False
         for r, children, tensors, values, objects in self._watched:
             m = r()
             if m is None:

@@ -77,3 +77,30 @@ def test_layers_of_other_sizes(lm, monkeypatch):
         assert not _eligible(lm), (type(m), name)
         setattr(m, name, plain)
     assert _eligible(lm)
+
+
+def test_layers_of_other_tables(lm, monkeypatch):
+    """A layer rotates with its own module's tables, whatever the model's module holds."""
+    steps, prompts = MuiDecoderStack(lm.model.layers, lm.model.rotary_emb, lm.cache, 1), _prompt_stack(lm)
+    prompts.remember()
+    asked = (lambda: steps.matches(lm.model.layers, lm.cache, 1), lambda: prompts.current(lm.model.layers))
+    assert _eligible(lm) and all(a() for a in asked)
+    with monkeypatch.context() as m:
+        m.undo()
+        other = _lm(rope_theta=1e4).model.rotary_emb
+    other.dispatchable = True
+    rotary = lm.model.layers[1].self_attn.rotary_emb
+    assert other.cos32 is not rotary.cos32 and lm.model.rotary_emb.cos32 is rotary.cos32
+    # a table built anew in place, in the module and (for prompts) in its handle; another module
+    for owner, name in ((rotary, "cos32"), (rotary, "sin32"), (lm.model.layers[1].self_attn, "rotary_emb")):
+        plain = getattr(owner, name)
+        setattr(owner, name, getattr(other, name, other))
+        assert not _eligible(lm) and not any(a() for a in asked), name
+        setattr(owner, name, plain)
+        assert _eligible(lm) and all(a() for a in asked)
+    rotary.cpp_module.sin32 = other.sin32
+    assert not asked[1]() and not MuiPromptStack.eligible(lm.model.layers, lm.model.rotary_emb, lm.cache)
+    rotary.cpp_module.sin32 = rotary.sin32
+    # the model's own module rotates no layer
+    lm.model.rotary_emb = other
+    assert MuiDecoderStack(lm.model.layers, other, lm.cache, 1).cos32 is rotary.cos32 and _prompt_stack(lm).cos32 is rotary.cos32

@@ -150,6 +150,20 @@ def test_layers_that_differ():
 
 
 @torch.no_grad()
+def test_layers_rotate_with_their_own_tables():
+    """... also where they were given others after a first prompt: all, one, the model's own module."""
+    lm, other = _lm(), _lm(rope_theta=1e4)
+    first = _run(lm, True, [_ids(1, 30), _ids(1, 1)], 64, 1)[0]
+    for change in (lambda: [setattr(x.self_attn, "rotary_emb", y.self_attn.rotary_emb) for x, y in zip(lm.model.layers, other.model.layers)],
+                   lambda: setattr(lm.model, "rotary_emb", other.model.rotary_emb),
+                   lambda: setattr(lm.model.layers[1].self_attn, "rotary_emb", _lm().model.layers[1].self_attn.rotary_emb)):
+        change()
+        got = _run(lm, True, [_ids(1, 30), _ids(1, 1)], 64, 1)
+        want = _run(lm, False, [_ids(1, 30), _ids(1, 1)], 64, 1)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and _off(got[0], first) > 0.01
+
+
+@torch.no_grad()
 def test_forward_mode_is_refused_as_by_the_modules():
     """The linears have no forward-mode rule: a tangent on the way in is an error, never lost."""
     lm = _lm()
