@@ -103,6 +103,12 @@ def _rotate_with(attentions, cos, sin) -> bool:
     return True
 
 
+def _held(t) -> Optional[tuple]:
+    """What a descriptor takes from a tensor. As long as the module's tensor gives the same, the memory is the module's and the descriptor holds: the tensor itself is neither
+    kept alive nor referred to (torch.utils.swap_tensors refuses tensors with weak references)."""
+    return None if t is None else (t.data_ptr(), t.dtype, t.shape, t.stride())
+
+
 def _ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
@@ -290,8 +296,8 @@ class MuiPromptStack(MuiDecoderStack):
     """The same for `mui_decoder_stack_prompt`: prompts, and steps of more batch rows than the decode kernels take. Layers called one by one run the same
     kernels; here nobody can listen in between, so a model with hooks stays with its modules.
 
-    What the descriptor was built from is watched by object and by address (current(), asked before every call, takes a few us per layer, where examining the
-    layers anew takes ~35 with an idle GPU waiting), through weak references: nothing is kept alive beyond a call."""
+    What the descriptor was built from is watched, modules by weak references and tensors by what they hold (current(), asked before every call, takes a few us per
+    layer, where examining the layers anew takes ~35 with an idle GPU waiting): nothing is kept alive beyond a call."""
 
     _ATTRIBUTES = ("training", "method", "cpp_module", "variance_epsilon", "normalize", "layer_idx", "prefill_kernel_max_tokens", "dispatchable", "num_heads",
                    "num_key_value_heads", "head_dim", "in_features", "out_features", "intermediate_size", "per_channel", "group_size_shift", "quantizer")
@@ -314,18 +320,18 @@ class MuiPromptStack(MuiDecoderStack):
             return
 
         def weak(v) -> bool:
-            return isinstance(v, (torch.Tensor, nn.Module)) or hasattr(v, "__weakref__")
+            return isinstance(v, nn.Module) or hasattr(v, "__weakref__")
 
         def ref(v):
             return weakref.ref(v) if weak(v) else (lambda: v)
 
-        watched = []  # per module: itself, its children, its tensors with their addresses, what else was read from it
+        watched = []  # per module: itself, its children, what its tensors hold, what else was read from it
         for layer in [r() for r in self._layer_refs]:
             qkv, attn, mlp = layer.qkv_proj, layer.self_attn, layer.mlp
             inside = [getattr(mlp, n) for n in ("gate_proj", "up_proj", "down_proj") if isinstance(getattr(mlp, n, None), nn.Module)]
             for m in [layer, qkv, qkv.linear, attn, attn.o_proj, mlp] + inside:
                 watched.append((weakref.ref(m), [(k, ref(v)) for k, v in m._modules.items()],
-                                [(k, ref(v), _ptr(v)) for k, v in m._parameters.items()],
+                                [(k, _held(v)) for k, v in m._parameters.items()],
                                 [(k, m.__dict__[k]) for k in self._ATTRIBUTES if k in m.__dict__ and not weak(m.__dict__[k])],
                                 [(k, weakref.ref(m.__dict__[k])) for k in self._ATTRIBUTES if k in m.__dict__ and weak(m.__dict__[k])]))
         self._watched = watched  # whole: another thread may ask meanwhile
@@ -365,7 +371,7 @@ class MuiPromptStack(MuiDecoderStack):
 
     def _bound(self, cache: MuiStaticCache) -> None:
         self._cache = weakref.ref(cache)
-        self._cache_tensors = [(weakref.ref(t), t.data_ptr()) for t in cache.tensors()]
+        self._cache_tensors = [_held(t) for t in cache.tensors()]
 
     def bound_to(self, cache: MuiStaticCache) -> Optional["MuiPromptStack"]:
         """The same for another cache (a request brings its own), or None. A descriptor of its own: another thread may be in a call with this one."""
@@ -412,9 +418,8 @@ class MuiPromptStack(MuiDecoderStack):
             for k, v in children:
                 if mods.get(k) is not v():
                     return False
-            for k, v, p in tensors:
-                t = params.get(k)
-                if t is not v() or (p is not None and t.data_ptr() != p):
+            for k, v in tensors:
+                if _held(params.get(k)) != v:
                     return False
             for k, v in values:
                 if d.get(k) is not v:
@@ -425,9 +430,7 @@ class MuiPromptStack(MuiDecoderStack):
         return True
 
     def holds(self, cache: MuiStaticCache) -> bool:
-        tensors = cache.tensors()
-        return (cache is self._cache() and len(tensors) == len(self._cache_tensors)
-                and all(t is r() and t.data_ptr() == p for t, (r, p) in zip(tensors, self._cache_tensors)))
+        return cache is self._cache() and [_held(t) for t in cache.tensors()] == self._cache_tensors
 
     def takes(self, hidden_states: torch.Tensor, position_ids: torch.Tensor, cache_position: torch.Tensor, key_mask: Optional[torch.Tensor]) -> bool:
         """Whether this call can be made: its sizes, and nobody who listens to the modules."""

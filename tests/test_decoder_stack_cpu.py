@@ -104,3 +104,34 @@ def test_layers_of_other_tables(lm, monkeypatch):
     # the model's own module rotates no layer
     lm.model.rotary_emb = other
     assert MuiDecoderStack(lm.model.layers, other, lm.cache, 1).cos32 is rotary.cos32 and _prompt_stack(lm).cos32 is rotary.cos32
+
+
+def _watching(lm):
+    stack = _prompt_stack(lm)
+    stack.remember()
+    assert stack.current(lm.model.layers) and stack.holds(lm.cache)
+    return stack
+
+
+def test_tensors_may_be_swapped(lm):
+    """... as module.to() and load_state_dict() do it where they are told to, and it is noticed."""
+    for m in (lm.model.layers[0].mlp.down_proj, lm.model.layers[1].qkv_proj.linear):
+        stack = _watching(lm)
+        torch.utils.swap_tensors(m.weight, torch.nn.Parameter(m.weight.detach().clone(), requires_grad=False))
+        assert not stack.current(lm.model.layers)
+    stack = _watching(lm)
+    torch.utils.swap_tensors(lm.cache.key_cache[1], lm.cache.key_cache[1].clone())
+    assert not stack.holds(lm.cache)
+
+
+def test_the_same_address_read_otherwise(lm):
+    layer = lm.model.layers[0]
+    for m, name in ((layer.self_attn.o_proj, "weight"), (layer.mlp.down_proj, "weight"), (layer.qkv_proj.linear, "norm_weights")):
+        t = getattr(m, name)
+        plain = t.data
+        for other in (plain.view(torch.float16), plain[:256], plain.reshape(-1, 256).T):
+            stack = _watching(lm)
+            t.data = other
+            assert other.data_ptr() == plain.data_ptr() and not stack.current(lm.model.layers), (name, other.shape, other.dtype)
+            t.data = plain
+            assert stack.current(lm.model.layers)
