@@ -109,6 +109,22 @@ def _held(t) -> Optional[tuple]:
     return None if t is None else (t.data_ptr(), t.dtype, t.shape, t.stride())
 
 
+_TENSORS = {MuiLinear: ("weight", "bias", "norm_weights"),
+            MuiInt8Linear: ("weights_int8", "scales", "weights_uint8", "scales_min_vals", "bias", "norm_weights"),
+            MuiGateUpDownMLP: ("norm_weights",),
+            MuiInt8GateUpDownMLP: ("norm_weights", "gate_up_weights", "gate_up_scales", "gate_up_scales_min_vals")}
+
+
+def _tensor(d: dict, name: str):
+    """A module's tensor, from its __dict__: an attribute (a parameter that was deleted and set again is a plain one), a parameter, a buffer."""
+    t = d.get(name)
+    if t is None:
+        t = d["_parameters"].get(name)
+        if t is None:
+            t = d["_buffers"].get(name)
+    return t
+
+
 def _ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
@@ -331,7 +347,7 @@ class MuiPromptStack(MuiDecoderStack):
             inside = [getattr(mlp, n) for n in ("gate_proj", "up_proj", "down_proj") if isinstance(getattr(mlp, n, None), nn.Module)]
             for m in [layer, qkv, qkv.linear, attn, attn.o_proj, mlp] + inside:
                 watched.append((weakref.ref(m), [(k, ref(v)) for k, v in m._modules.items()],
-                                [(k, _held(v)) for k, v in m._parameters.items()],
+                                [(k, _held(_tensor(m.__dict__, k))) for k in _TENSORS.get(type(m), ())],
                                 [(k, m.__dict__[k]) for k in self._ATTRIBUTES if k in m.__dict__ and not weak(m.__dict__[k])],
                                 [(k, weakref.ref(m.__dict__[k])) for k in self._ATTRIBUTES if k in m.__dict__ and weak(m.__dict__[k])]))
         self._watched = watched  # whole: another thread may ask meanwhile
@@ -412,14 +428,14 @@ class MuiPromptStack(MuiDecoderStack):
             if m is None:
                 return False
             d = m.__dict__
-            mods, params = d["_modules"], d["_parameters"]
-            if len(mods) != len(children) or len(params) != len(tensors):
+            mods = d["_modules"]
+            if len(mods) != len(children):
                 return False
             for k, v in children:
                 if mods.get(k) is not v():
                     return False
             for k, v in tensors:
-                if _held(params.get(k)) != v:
+                if _held(_tensor(d, k)) != v:
                     return False
             for k, v in values:
                 if d.get(k) is not v:

@@ -135,3 +135,29 @@ def test_the_same_address_read_otherwise(lm):
             assert other.data_ptr() == plain.data_ptr() and not stack.current(lm.model.layers), (name, other.shape, other.dtype)
             t.data = plain
             assert stack.current(lm.model.layers)
+
+
+def test_weights_that_are_plain_tensors(lm):
+    """A parameter that was deleted and set again as a tensor, or as a buffer, is what the modules read."""
+    mlp = lm.model.layers[0].mlp
+    for m in (mlp.gate_proj, mlp.up_proj, mlp.down_proj):
+        def another():
+            return torch.empty(m.out_features, m.in_features, dtype=torch.bfloat16)
+
+        del m.weight
+        m.weight = another()
+        if m is mlp.up_proj:
+            mlp.gate_proj.weight = another()  # (the two have one pitch)
+        if m is mlp.gate_proj:
+            del mlp.up_proj.weight
+            mlp.up_proj.weight = torch.nn.Parameter(another(), requires_grad=False)
+        kept, stack = m.weight, _watching(lm)
+        m.weight = another()
+        assert not stack.current(lm.model.layers)
+        m.weight = kept
+        assert stack.current(lm.model.layers)
+        del m.weight
+        m.register_buffer("weight", another())
+        stack = _watching(lm)
+        m.weight = another()
+        assert not stack.current(lm.model.layers)
