@@ -150,7 +150,7 @@ class MuiDecoderStack:
         self._cache_ptrs = tuple(t.data_ptr() for t in cache.key_cache) + tuple(t.data_ptr() for t in cache.value_cache)
         self._keep = []  # tensors the descriptor points into
         self._layer_list = layers
-        self._owners = []  # (module, attribute name, object) the descriptor was built from
+        self._owners = []  # (module, attribute name, object) the descriptor was built from, tensors with what they hold
         arr = (_lib.MuiDecoderLayerDesc * len(layers))()
         for i, layer in enumerate(layers):
             qkv, attn, mlp = layer.qkv_proj.linear, layer.self_attn, layer.mlp
@@ -177,16 +177,17 @@ class MuiDecoderStack:
                 g_ptr, u_ptr, g_pitch = g.data_ptr(), u.data_ptr(), g.stride(0)
                 gs_ptr, us_ptr, gs_stride = None, None, 0
                 gu_keep = [g, u]
-                gu_own = [(mlp.gate_proj, "weight", g), (mlp.up_proj, "weight", u)]
+                gu_own = [(mlp, "gate_proj", mlp.gate_proj), (mlp, "up_proj", mlp.up_proj), (mlp.gate_proj, "weight", g), (mlp.up_proj, "weight", u)]
             arr[i] = _lib.MuiDecoderLayerDesc(
                 qkv.norm_weights.data_ptr(), qw.data_ptr(), qp, ow.data_ptr(), op,
                 mlp.norm_weights.data_ptr(), g_ptr, u_ptr, g_pitch, dw.data_ptr(), dp, kc.data_ptr(), vc.data_ptr(),
                 _ptr(qs), _ptr(osc), gs_ptr, us_ptr, gs_stride, _ptr(ds), shift)
             self._keep += [qkv.norm_weights, qw, qs, ow, osc, mlp.norm_weights, dw, ds, kc, vc] + gu_keep
-            self._owners += [(layer, "qkv_proj", layer.qkv_proj), (layer, "self_attn", attn), (layer, "mlp", mlp),
-                             (layer.qkv_proj, "linear", qkv), (qkv, "norm_weights", qkv.norm_weights),
-                             (attn, "o_proj", attn.o_proj), (mlp, "norm_weights", mlp.norm_weights),
-                             (mlp, "down_proj", mlp.down_proj)] + q_own + o_own + d_own + gu_own
+            owners = [(layer, "qkv_proj", layer.qkv_proj), (layer, "self_attn", attn), (layer, "mlp", mlp),
+                      (layer.qkv_proj, "linear", qkv), (qkv, "norm_weights", qkv.norm_weights),
+                      (attn, "o_proj", attn.o_proj), (mlp, "norm_weights", mlp.norm_weights),
+                      (mlp, "down_proj", mlp.down_proj)] + q_own + o_own + d_own + gu_own
+            self._owners += [(m, name, v, _held(v) if isinstance(v, torch.Tensor) else None) for m, name, v in owners]
         self._layers = arr
         self.desc = _lib.MuiDecoderStackDesc(
             muillm_ext._dtype_code(first.qkv_proj.linear.norm_weights), len(layers), self.hidden, self.hq, self.hkv,
@@ -266,12 +267,16 @@ class MuiDecoderStack:
 
     def matches(self, layers, cache: MuiStaticCache, batch: int) -> bool:
         """Still valid for this step? The cache tensors are where they were, and every module and
-        parameter the descriptor was built from is still the object in place (a later
-        quantize_layers / .to() / weight swap replaces them)."""
+        tensor the descriptor was built from is still the object in place, with the memory it had (a
+        later quantize_layers / .to() / weight swap replaces them, `.data = ` its memory)."""
         if batch != self.batch or layers is not self._layer_list:
             return False
-        for owner, name, obj in self._owners:
-            if getattr(owner, name, None) is not obj:
+        for owner, name, obj, held in self._owners:
+            d = owner.__dict__
+            if held is None:
+                if d["_modules"].get(name) is not obj:
+                    return False
+            elif _tensor(d, name) is not obj or _held(obj) != held:
                 return False
         if not _rotate_with(self._attentions, self.cos32, self.sin32):
             return False

@@ -161,3 +161,21 @@ def test_weights_that_are_plain_tensors(lm):
         stack = _watching(lm)
         m.weight = another()
         assert not stack.current(lm.model.layers)
+
+
+def test_steps_notice_other_memory_and_modules(lm):
+    layers, model = lm.model.layers, lm.model
+    steps = MuiDecoderStack(layers, model.rotary_emb, lm.cache, 1)
+    assert steps.matches(layers, lm.cache, 1)
+    for m in (layers[1].mlp.gate_proj, layers[0].mlp.down_proj, layers[1].qkv_proj.linear, layers[0].self_attn.o_proj):
+        plain = m.weight.data
+        m.weight.data = plain.clone()
+        assert not steps.matches(layers, lm.cache, 1)
+        m.weight.data = plain
+        assert steps.matches(layers, lm.cache, 1)
+    for name in ("gate_proj", "up_proj", "down_proj"):
+        plain = getattr(layers[1].mlp, name)
+        setattr(layers[1].mlp, name, getattr(layers[0].mlp, name))
+        assert not steps.matches(layers, lm.cache, 1)
+        setattr(layers[1].mlp, name, plain)
+    assert steps.matches(layers, lm.cache, 1)
