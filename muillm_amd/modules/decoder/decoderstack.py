@@ -115,6 +115,23 @@ _TENSORS = {MuiLinear: ("weight", "bias", "norm_weights"),
             MuiInt8GateUpDownMLP: ("norm_weights", "gate_up_weights", "gate_up_scales", "gate_up_scales_min_vals")}
 
 
+# what else a descriptor, or the choice to use one, goes by (a name may be missing: its default stands in the class then)
+_LINEAR = ("variance_epsilon", "normalize", "in_features", "out_features", "dispatchable", "per_channel", "quantizer")
+_MLP = ("variance_epsilon", "normalize", "intermediate_size", "dispatchable", "method", "per_channel", "group_size_shift")
+_VALUES = {MuiLinear: _LINEAR, MuiInt8Linear: _LINEAR, MuiGateUpDownMLP: _MLP, MuiInt8GateUpDownMLP: _MLP, MuiMultiLinear: ("slice_starts", "slice_ends"),
+           MuiSdpaAttention: ("training", "layer_idx", "num_heads", "num_key_value_heads", "head_dim")}
+_ABSENT = object()
+
+
+def _nothing():  # in the place of a weak reference
+    return None
+
+
+def _same(v, ref) -> bool:
+    """Whether v is what ref was made of. (What has gone is nobody's.)"""
+    return v is ref() and (v is not None or ref is _nothing)
+
+
 def _tensor(d: dict, name: str):
     """A module's tensor, from its __dict__: an attribute (a parameter that was deleted and set again is a plain one), a parameter, a buffer."""
     t = d.get(name)
@@ -320,9 +337,6 @@ class MuiPromptStack(MuiDecoderStack):
     What the descriptor was built from is watched, modules by weak references and tensors by what they hold (current(), asked before every call, takes a few us per
     layer, where examining the layers anew takes ~35 with an idle GPU waiting): nothing is kept alive beyond a call."""
 
-    _ATTRIBUTES = ("training", "method", "cpp_module", "variance_epsilon", "normalize", "layer_idx", "prefill_kernel_max_tokens", "dispatchable", "num_heads",
-                   "num_key_value_heads", "head_dim", "in_features", "out_features", "intermediate_size", "per_channel", "group_size_shift", "quantizer")
-
     def __init__(self, layers, rotary_emb, cache: MuiStaticCache):
         super().__init__(layers, rotary_emb, cache, 1)
         self._keep, self._owners, self._layer_list = [], [], None
@@ -333,28 +347,25 @@ class MuiPromptStack(MuiDecoderStack):
         int8 = any(type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP)
                    for layer in layers for m in (layer.qkv_proj.linear, layer.self_attn.o_proj, layer.mlp, layer.mlp.down_proj))
         self._most_rows = min(muillm_ext.INT8_DEQUANT_MIN_TOKENS, muillm_ext.INT8_GROUP_DEQUANT_MIN_TOKENS) - 1 if int8 else 1 << 30
-        self._most_tokens = min([65535] + [x.self_attn.prefill_kernel_max_tokens for x in layers if x.self_attn.prefill_kernel_max_tokens is not None])
+        self._attention_refs = [weakref.ref(layer.self_attn) for layer in layers]
 
     def remember(self) -> None:
         """What current() compares with. (Made behind the first call, while the GPU is at work.)"""
         if self._watched is not None:
             return
 
-        def weak(v) -> bool:
-            return isinstance(v, nn.Module) or hasattr(v, "__weakref__")
-
         def ref(v):
-            return weakref.ref(v) if weak(v) else (lambda: v)
+            return _nothing if v is None else weakref.ref(v)
 
-        watched = []  # per module: itself, its children, what its tensors hold, what else was read from it
+        watched = []  # per module: itself, its children, what its tensors hold, what else was read from it, its handle
         for layer in [r() for r in self._layer_refs]:
             qkv, attn, mlp = layer.qkv_proj, layer.self_attn, layer.mlp
             inside = [getattr(mlp, n) for n in ("gate_proj", "up_proj", "down_proj") if isinstance(getattr(mlp, n, None), nn.Module)]
             for m in [layer, qkv, qkv.linear, attn, attn.o_proj, mlp] + inside:
+                d, kind = m.__dict__, type(m)
                 watched.append((weakref.ref(m), [(k, ref(v)) for k, v in m._modules.items()],
-                                [(k, _held(_tensor(m.__dict__, k))) for k in _TENSORS.get(type(m), ())],
-                                [(k, m.__dict__[k]) for k in self._ATTRIBUTES if k in m.__dict__ and not weak(m.__dict__[k])],
-                                [(k, weakref.ref(m.__dict__[k])) for k in self._ATTRIBUTES if k in m.__dict__ and weak(m.__dict__[k])]))
+                                [(k, _held(_tensor(d, k))) for k in _TENSORS.get(kind, ())],
+                                [(k, d.get(k, _ABSENT)) for k in _VALUES.get(kind, ())], ref(d.get("cpp_module"))))
         self._watched = watched  # whole: another thread may ask meanwhile
 
     @staticmethod
@@ -428,7 +439,7 @@ class MuiPromptStack(MuiDecoderStack):
             handle = rotary["cpp_module"]
             if handle is None or handle.cos32 is not self.cos32 or handle.sin32 is not self.sin32 or handle.layer_idx != attn.layer_idx or not rotary["dispatchable"]:
                 return False
-        for r, children, tensors, values, objects in self._watched:
+        for r, children, tensors, values, handle in self._watched:
             m = r()
             if m is None:
                 return False
@@ -437,17 +448,16 @@ class MuiPromptStack(MuiDecoderStack):
             if len(mods) != len(children):
                 return False
             for k, v in children:
-                if mods.get(k) is not v():
+                if not _same(mods.get(k), v):
                     return False
             for k, v in tensors:
                 if _held(_tensor(d, k)) != v:
                     return False
             for k, v in values:
-                if d.get(k) is not v:
+                if d.get(k, _ABSENT) is not v:
                     return False
-            for k, v in objects:
-                if d.get(k) is not v():
-                    return False
+            if not _same(d.get("cpp_module"), handle):
+                return False
         return True
 
     def holds(self, cache: MuiStaticCache) -> bool:
@@ -461,8 +471,12 @@ class MuiPromptStack(MuiDecoderStack):
         if unpack_dual(hidden_states).tangent is not None:
             return False  # forward mode: the linears' modules refuse it, here a tangent would be lost
         cache = self._cache()
-        if b > cache.max_batch_size or b > 65535 or t > self._most_tokens or not 1 <= b * t <= self._most_rows:
+        if b > cache.max_batch_size or b > 65535 or t > 65535 or not 1 <= b * t <= self._most_rows:
             return False
+        for r in self._attention_refs:  # (set at any time, on a module or for all of them)
+            most = r().prefill_kernel_max_tokens
+            if most is not None and t > most:
+                return False
         if cache.get_seq_length() + t > self.max_cache_len:
             return False  # the modules refuse to read a cache beyond its rows
         if position_ids.dtype != torch.int64 or cache_position.dtype != torch.int64 or not (position_ids.is_cuda and cache_position.is_cuda):

@@ -179,3 +179,31 @@ def test_steps_notice_other_memory_and_modules(lm):
         assert not steps.matches(layers, lm.cache, 1)
         setattr(layers[1].mlp, name, plain)
     assert steps.matches(layers, lm.cache, 1)
+
+
+def test_what_may_be_set_after_a_prompt(lm, monkeypatch):
+    """The number of tokens from which prompts use torch's attention, on a module or on the class; attributes that appear where there were none, or go."""
+    stack, layers = _watching(lm), lm.model.layers
+    assert _takes(stack)
+    attn = layers[1].self_attn
+    attn.prefill_kernel_max_tokens = 19
+    assert not _takes(stack) and _takes(stack, 19)
+    del attn.prefill_kernel_max_tokens
+    with monkeypatch.context() as m:
+        m.setattr(type(attn), "prefill_kernel_max_tokens", 19)
+        assert not _takes(stack)
+    assert _takes(stack) and stack.current(layers)
+    for m, name, value in ((layers[0].mlp.down_proj, "per_channel", True), (layers[0].mlp, "method", None), (layers[0].mlp, "intermediate_size", 640), (attn, "training", True),
+                           (layers[1].qkv_proj.linear, "variance_epsilon", 1e-3), (layers[1].qkv_proj, "slice_starts", [0, 512, 640]), (attn.o_proj, "cpp_module", None)):
+        before = m.__dict__.get(name, m)
+        setattr(m, name, value)
+        assert not stack.current(layers), name
+        delattr(m, name) if before is m else setattr(m, name, before)
+        assert stack.current(layers), name
+    # what has gone does not pass for what never was
+    attn.o_proj.cpp_module = None
+    assert not stack.current(layers)
+    attn.o_proj.finalize_init()
+    stack = _watching(lm)
+    layers[0].mlp = None
+    assert not stack.current(layers)
