@@ -15,7 +15,7 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-from torch.autograd.forward_ad import unpack_dual
+from torch.autograd import forward_ad
 
 from ... import _lib, muillm_ext
 from ..attention.baseattention import MuiBaseAttention
@@ -468,8 +468,8 @@ class MuiPromptStack(MuiDecoderStack):
         b, t = hidden_states.shape[0], hidden_states.shape[1]
         if hidden_states.dtype != self.dtype or hidden_states.device != self.device or hidden_states.shape[2] != self.hidden:
             return False
-        if unpack_dual(hidden_states).tangent is not None:
-            return False  # forward mode: the linears' modules refuse it, here a tangent would be lost
+        if forward_ad._current_level >= 0:
+            return False  # forward mode: the linears' modules refuse tangents, of inputs and of weights; here they would be lost
         cache = self._cache()
         if b > cache.max_batch_size or b > 65535 or t > 65535 or not 1 <= b * t <= self._most_rows:
             return False

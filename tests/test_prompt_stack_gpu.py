@@ -177,6 +177,26 @@ def test_forward_mode_is_refused_as_by_the_modules():
 
 
 @torch.no_grad()
+def test_forward_mode_of_a_weight_is_refused_as_by_the_modules():
+    """... of gate, up and down, which the MLP's node takes as arguments. A call without a tangent is an ordinary one."""
+    lm, ids = _lm(), _ids(1, 30)
+    want = lm(input_ids=ids).logits
+    mlp = lm.model.layers[1].mlp
+    for m in (mlp.gate_proj, mlp.up_proj, mlp.down_proj):
+        plain = m.weight
+        for one_call in (True, False):
+            lm.model.use_decoder_stack = one_call
+            with torch.autograd.forward_ad.dual_level():
+                assert torch.equal(lm(input_ids=ids).logits, want)
+                del m.weight
+                m.weight = torch.autograd.forward_ad.make_dual(plain.detach(), torch.ones_like(plain))
+                with pytest.raises(NotImplementedError):
+                    lm(input_ids=ids)
+                del m.weight
+                m.weight = plain
+
+
+@torch.no_grad()
 def test_layers_are_examined_once_where_calls_are_refused():
     lm, built = _lm(), []
     handle = lm.model.layers[1].register_forward_hook(lambda *a: None)
