@@ -11,7 +11,7 @@ from ... import hybrid_ops
 from ...engineconfig import MuiEngineConfig
 from ..kvcache.hybridcache import MuiHybridCache, MuiKeyValueState
 from ..linear import MuiLinear
-from ..module import MuiModule
+from ..module import MuiModule, heard
 from ..multilinear import MuiMultiLinear
 from .rotaryembedding import compute_rope_inv_freq
 
@@ -43,7 +43,7 @@ class MuiHybridAttentionConfig:
 
 class MuiHybridAttention(MuiModule):
     def takes_behind(self) -> bool:
-        return type(self.out_proj) is MuiLinear
+        return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiHybridAttentionConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):

@@ -14,7 +14,7 @@ from ... import _lib, hybrid_ops
 from ...engineconfig import MuiEngineConfig
 from ..kvcache.hybridcache import MuiHybridCache, MuiLatentState
 from ..linear import MuiLinear
-from ..module import MuiModule
+from ..module import MuiModule, heard
 from ..multilinear import MuiMultiLinear
 
 
@@ -38,7 +38,7 @@ class MuiLatentAttentionConfig:
 
 class MuiLatentAttention(MuiModule):
     def takes_behind(self) -> bool:
-        return type(self.out_proj) is MuiLinear
+        return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiLatentAttentionConfig, layer_idx: int,
                  eps: float, device=None, dtype=None):

@@ -19,7 +19,7 @@ from ..engineconfig import MuiEngineConfig
 from ..memorymanagement.gc import trigger_gc
 from ..replacement.replacementcontext import MuiReplacementContext
 from .linear import MuiLinear
-from .module import MuiModule
+from .module import MuiModule, heard
 from ._fusion import AbsorbedNorm
 from .norm.rmsnorm import MuiRMSNorm, _MuiRMSNorm
 
@@ -220,7 +220,7 @@ class MuiGateUpDownMLP(MuiModule):
         return self._forward_unfused(input=input, residual=residual)
 
     def takes_behind(self) -> bool:
-        return type(self.down_proj) is MuiLinear and self.method != _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED
+        return type(self.down_proj) is MuiLinear and self.method != _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED and not heard(self)
 
     def forward(self, input: Tensor, residual: Optional[Tensor] = None, behind: Optional[muillm_ext.ResidualBehind] = None) -> Tensor:
         if self.method == _MuiGateUpSiLUMethod.GATEUPSILU_FUSED:

@@ -5,6 +5,14 @@ import torch.nn as nn
 from ..engineconfig import MuiEngineConfig
 
 
+def heard(*modules: nn.Module) -> bool:
+    """Whether a hook listens to calls of one of them: it may change what comes out in ways that cannot be seen from outside (through .data, or by a kernel of its own)."""
+    every = nn.modules.module
+    if every._global_forward_hooks or every._global_forward_pre_hooks:
+        return True
+    return any(m.__dict__["_forward_hooks"] or m.__dict__["_forward_pre_hooks"] for m in modules)
+
+
 class MuiModule(nn.Module):
     def __init__(self, engine_config: MuiEngineConfig = None, **kargs) -> None:
         if engine_config is None:

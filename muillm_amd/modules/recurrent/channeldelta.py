@@ -9,7 +9,7 @@ from ... import hybrid_ops
 from ...engineconfig import MuiEngineConfig
 from ..kvcache.hybridcache import MuiHybridCache, MuiRecurrentState
 from ..linear import MuiLinear
-from ..module import MuiModule
+from ..module import MuiModule, heard
 from ..multilinear import MuiMultiLinear
 
 
@@ -39,7 +39,7 @@ class MuiChannelDelta(MuiModule):
     rows (and a2, g2 with zero columns) to multiples of eight, so that every part starts on a 16-byte boundary."""
 
     def takes_behind(self) -> bool:
-        return type(self.out_proj) is MuiLinear
+        return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiChannelDeltaConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):

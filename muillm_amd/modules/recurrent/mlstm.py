@@ -9,7 +9,7 @@ from ... import hybrid_ops
 from ...engineconfig import MuiEngineConfig
 from ..kvcache.hybridcache import MuiHybridCache, MuiRecurrentState
 from ..linear import MuiLinear
-from ..module import MuiModule
+from ..module import MuiModule, heard
 from ..multilinear import MuiMultiLinear
 
 
@@ -23,7 +23,7 @@ class MuiMLstmConfig:
 
 class MuiMLstm(MuiModule):
     def takes_behind(self) -> bool:
-        return type(self.out_proj) is MuiLinear
+        return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiMLstmConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):

@@ -165,8 +165,9 @@ def _prompt_workspace(x: torch.Tensor, stream: int) -> Optional[torch.Tensor]:
 class ResidualBehind:
     """The boundary between two sublayers with an fp32 residual stream (hybrid_ops.residual_norm) that follows a linear and is taken along by its
     library call: the stream and the next sublayer's input. An object lives for one boundary of one forward pass: whoever makes it hands it to
-    the linear, which fills it in where it can, and asks with the very tensor that the sublayer has returned whether it was. A tensor that somebody (a module
-    hook) has put in its place, or has written to since, finds nothing here and is joined the ordinary way: the stream is not updated in place."""
+    the linear, which fills it in where it can, and asks with the very tensor that the sublayer has returned whether it was. A tensor that somebody has put
+    in its place, or has written to since, finds nothing here and is joined the ordinary way: the stream is not updated in place. (A write that raises no version cannot be
+    seen: where a hook listens nothing is taken along to begin with.)"""
     MAX_TOKENS = 128  # beyond, K is not divided and nothing is saved
 
     def __init__(self, stream: torch.Tensor, post_gain: torch.Tensor, branch_scale: float, next_gain: Optional[torch.Tensor], next_scale: float,

@@ -3,6 +3,11 @@
 import pytest
 import torch
 
+from muillm_amd import hybrid_ops
+from muillm_amd.engineconfig import MuiEngineConfig
+from muillm_amd.modules.decoder import sandwichdecoder
+from muillm_amd.modules.linear import MuiLinear
+from muillm_amd.modules.recurrent.mlstm import MuiMLstm
 from muillm_amd.muillm_ext import ResidualBehind
 
 
@@ -49,3 +54,57 @@ def test_number_of_tokens(tokens, worth):
     with torch.no_grad():
         assert ResidualBehind.worth_it(tokens) == worth
     assert not ResidualBehind.worth_it(tokens)
+
+
+class _Mixer(MuiMLstm):
+    """y = out_proj(h), with the boundary filled in as the library's call does it."""
+    takes_behind = MuiMLstm.takes_behind
+
+    def __init__(self):
+        super(MuiMLstm, self).__init__(engine_config=MuiEngineConfig())
+        self.out_proj = MuiLinear(MuiEngineConfig(), 8, 8, bias=False)
+        self.got = []
+
+    def forward(self, h, cache, cache_position, behind=None):
+        self.got.append(behind)
+        y = self.out_proj(h)
+        if behind is not None:
+            assert behind.linear(y, lambda name, args: None)
+            behind.result = (behind.stream + y, y.clone())
+        return y
+
+
+@pytest.fixture
+def layer(monkeypatch):
+    monkeypatch.setattr(hybrid_ops, "residual_norm", lambda x, y, *a, **kw: (x + y, y.clone()))
+    return sandwichdecoder.MuiSandwichDecoderLayer(MuiEngineConfig(), 8, _Mixer(), None, 1e-5, pre_norms=False)
+
+
+def _through(layer):
+    """The residual stream behind the layer, and whether its mixer was given the boundary."""
+    out = []
+    with torch.no_grad():
+        h = torch.ones(1, 17, 8)
+        sandwichdecoder.run_layers([layer], torch.zeros_like(h), h, layer.post_mixer_norm, 1e-5, None, None, collect=out)
+    return out[0], layer.mixer.got.pop() is not None
+
+
+def _write_unseen(mod, args, out):
+    out.data.mul_(2.0)
+
+
+def test_a_hooks_write_is_heard(layer):
+    plain, given = _through(layer)
+    assert given
+    for m in (layer.mixer, layer.mixer.out_proj):
+        handle = m.register_forward_hook(_write_unseen)
+        assert torch.equal(_through(layer)[0], 2 * plain)
+        handle.remove()
+        handle = m.register_forward_pre_hook(lambda mod, args: (args[0] * 2,) + args[1:])
+        assert torch.equal(_through(layer)[0], 2 * plain) and torch.equal(_through(layer)[0], 2 * plain)
+        handle.remove()
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda mod, args, out: _write_unseen(mod, args, out) if mod is layer.mixer else None)
+    assert torch.equal(_through(layer)[0], 2 * plain)
+    handle.remove()
+    got, given = _through(layer)
+    assert given and torch.equal(got, plain)
