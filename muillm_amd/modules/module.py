@@ -6,11 +6,12 @@ from ..engineconfig import MuiEngineConfig
 
 
 def heard(*modules: nn.Module) -> bool:
-    """Whether a hook listens to calls of one of them: it may change what comes out in ways that cannot be seen from outside (through .data, or by a kernel of its own)."""
+    """Whether a hook listens to calls of one of them, or a forward of its own stands in for its class's: a hook may change what comes out in ways that cannot be seen from
+    outside (through .data, or by a kernel of its own), and another forward knows the documented arguments only."""
     every = nn.modules.module
     if every._global_forward_hooks or every._global_forward_pre_hooks:
         return True
-    return any(m.__dict__["_forward_hooks"] or m.__dict__["_forward_pre_hooks"] for m in modules)
+    return any(m.__dict__["_forward_hooks"] or m.__dict__["_forward_pre_hooks"] or "forward" in m.__dict__ for m in modules)
 
 
 class MuiModule(nn.Module):

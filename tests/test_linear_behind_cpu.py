@@ -108,3 +108,16 @@ def test_a_hooks_write_is_heard(layer):
     handle.remove()
     got, given = _through(layer)
     assert given and torch.equal(got, plain)
+
+
+def test_a_forward_of_an_instance_is_called_as_documented(layer):
+    plain, _ = _through(layer)
+    mixer, linear = layer.mixer, layer.mixer.out_proj
+    linear.forward = lambda x: 2 * torch.nn.functional.linear(x, linear.weight)
+    assert torch.equal(_through(layer)[0], 2 * plain)
+    del linear.forward
+    mixer.forward = lambda h, cache, cache_position: mixer.got.append(None) or 2 * linear(h)
+    assert torch.equal(_through(layer)[0], 2 * plain)
+    del mixer.forward
+    got, given = _through(layer)
+    assert given and torch.equal(got, plain)

@@ -136,3 +136,43 @@ def test_hybrid_layers_use_it_and_hooks_are_heard(monkeypatch):
     for h in handles:
         h.remove()
     assert float((got - want).norm() / want.norm()) < 0.03 and float((got - fused).norm() / fused.norm()) > 0.1
+
+
+def test_hybrid_layers_give_the_same_bits_whoever_listens():
+    """... and whether or not versions can be asked for (inference mode): the boundary is then joined behind the call. Writes without a version and forwards of an instance count."""
+    cfg = zufadra_util.default_config()
+    lm = zufadra_util.build(cfg, zufadra_util.random_weights(cfg, seed=1), torch.bfloat16, DEV)
+    ids = torch.randint(0, cfg["vocab"], (1, 60), generator=torch.Generator().manual_seed(2)).to(DEV)
+    outs = [m.mixer.out_proj for m in lm.model.layers]
+
+    @torch.no_grad()
+    def run():
+        return lm(input_ids=ids).logits.float()
+
+    plain = run()
+    with torch.inference_mode():
+        assert torch.equal(lm(input_ids=ids).logits.float(), plain)
+
+    def hooked(hook):
+        handles = [m.register_forward_hook(hook) for m in outs]
+        try:
+            return run()
+        finally:
+            for h in handles:
+                h.remove()
+
+    assert torch.equal(hooked(lambda mod, args, out: None), plain)
+    shifted = hooked(lambda mod, args, out: out + 1.0)
+    assert not torch.equal(shifted, plain)
+
+    def unseen(mod, args, out):
+        out.data.add_(1.0)
+
+    assert torch.equal(hooked(unseen), shifted)
+    for m in lm.model.layers:
+        m.mixer.forward = lambda h, cache, cache_position, f=m.mixer.forward: f(h, cache, cache_position)
+    assert torch.equal(run(), plain)
+    for m in lm.model.layers:
+        del m.mixer.forward
+        m.mixer.out_proj.forward = lambda x, f=m.mixer.out_proj.forward: f(x)
+    assert torch.equal(run(), plain)
