@@ -263,13 +263,12 @@ class MuiDecoderStack:
             if of is None or (sizes is not None and of != sizes):
                 return False
             sizes = of
-            for m in (qkv.linear, attn.o_proj, mlp.down_proj):
-                if type(m) is MuiInt8Linear:
-                    wd = m.scales.dtype if m.per_channel else m.scales_min_vals.dtype
-                else:
-                    wd = m.weight.dtype
-                if wd != dtype:
-                    return False
+            # one type throughout, as the kernels read it (the modules refuse others)
+            held = [m.weight if type(m) is MuiLinear else m.scales if m.per_channel else m.scales_min_vals for m in (qkv.linear, attn.o_proj, mlp.down_proj)]
+            held += [mlp.norm_weights] + ([mlp.gate_proj.weight, mlp.up_proj.weight] if type(mlp) is MuiGateUpDownMLP
+                                          else [mlp.gate_up_scales if mlp.per_channel else mlp.gate_up_scales_min_vals])
+            if any(t.dtype != dtype for t in held):
+                return False
             # the int8 projections of a layer share one format: all per-channel, or all in the group
             # format with one group size (the layer descriptor carries a single shift)
             int8_mods = [m for m in (qkv.linear, attn.o_proj, mlp, mlp.down_proj)

@@ -207,3 +207,16 @@ def test_what_may_be_set_after_a_prompt(lm, monkeypatch):
     stack = _watching(lm)
     layers[0].mlp = None
     assert not stack.current(layers)
+
+
+def test_tensors_of_another_type(lm):
+    """The modules refuse them; one descriptor has one type."""
+    mlp, qkv, o = lm.model.layers[1].mlp, lm.model.layers[1].qkv_proj.linear, lm.model.layers[1].self_attn.o_proj
+    for m, name in ((mlp.gate_proj, "weight"), (mlp.up_proj, "weight"), (mlp.down_proj, "weight"), (mlp, "norm_weights"), (qkv, "weight"), (qkv, "norm_weights"), (o, "weight")):
+        for dtype in (torch.float32, torch.float16):
+            t = getattr(m, name)
+            plain = t.data
+            t.data = plain.to(dtype).as_strided(plain.shape, plain.stride()) if plain.is_contiguous() else torch.empty_strided(plain.shape, plain.stride(), dtype=dtype)
+            assert not _eligible(lm), (type(m), name)
+            t.data = plain
+    assert _eligible(lm)
