@@ -29,6 +29,19 @@ from ..quantized.int8linear import MuiInt8Linear
 from .decoder import MuiDecoderLayer
 
 
+def _at(m, name: str):
+    """m.name, from where nn.Module keeps it; None where it has none. (A layer has some sixty to read, in front of an idle GPU; nn.Module's own lookup takes several times as long.)"""
+    d = m.__dict__
+    v = d.get(name)
+    if v is None:
+        v = d["_parameters"].get(name)
+        if v is None:
+            v = d["_modules"].get(name)
+            if v is None:
+                v = d["_buffers"].get(name)
+    return v
+
+
 def _group_shift(m) -> int:
     """0 for a 16-bit or per-channel int8 module, the group size's log2 for the group format."""
     if type(m) is MuiInt8Linear and not m.per_channel:
@@ -42,52 +55,60 @@ def _plain_linear(m, normalize: Optional[bool] = None) -> bool:
     """A bias-free MuiLinear, or a bias-free MuiInt8Linear (per-channel, or the group format with
     groups of at least 16 that divide the rows)."""
     if type(m) is MuiInt8Linear:
-        if m.bias is not None or not m.dispatchable or (normalize is not None and bool(m.normalize) != normalize):
+        if _at(m, "bias") is not None or not m.dispatchable or (normalize is not None and bool(m.normalize) != normalize):
             return False
         if m.per_channel:
-            return m.weights_int8.is_contiguous() and m.scales.is_contiguous()
-        return (m.quantizer.group_size_shift >= 4 and m.in_features % 16 == 0 and m.weights_uint8.is_contiguous()
-                and m.scales_min_vals.is_contiguous())
-    return (type(m) is MuiLinear and m.bias is None and m.weight.is_cuda and m.weight.stride(1) == 1
-            and (normalize is None or bool(m.normalize) == normalize))
+            return _at(m, "weights_int8").is_contiguous() and _at(m, "scales").is_contiguous()
+        return (m.quantizer.group_size_shift >= 4 and m.in_features % 16 == 0 and _at(m, "weights_uint8").is_contiguous()
+                and _at(m, "scales_min_vals").is_contiguous())
+    if type(m) is not MuiLinear or _at(m, "bias") is not None:
+        return False
+    w = _at(m, "weight")
+    return w.is_cuda and w.stride(1) == 1 and (normalize is None or bool(m.normalize) == normalize)
 
 
 def _linear_fields(m):
     """(weight tensor, row pitch, scales tensor or None, [(owner, attribute, object)]) of a projection;
     "scales" are per-channel scales or, in the group format, the (scale, min) pairs."""
     if type(m) is MuiInt8Linear:
-        if m.per_channel:
-            return m.weights_int8, m.weights_int8.stride(0), m.scales, [(m, "weights_int8", m.weights_int8),
-                                                                         (m, "scales", m.scales)]
-        return m.weights_uint8, m.weights_uint8.stride(0), m.scales_min_vals, [
-            (m, "weights_uint8", m.weights_uint8), (m, "scales_min_vals", m.scales_min_vals)]
-    return m.weight, m.weight.stride(0), None, [(m, "weight", m.weight)]
+        names = ("weights_int8", "scales") if m.per_channel else ("weights_uint8", "scales_min_vals")
+        w, sc = _at(m, names[0]), _at(m, names[1])
+        return w, w.stride(0), sc, [(m, names[0], w), (m, names[1], sc)]
+    w = _at(m, "weight")
+    return w, w.stride(0), None, [(m, "weight", w)]
+
+
+def _scales_of(mlp) -> str:
+    """What an int8 MLP calls its gate and up scales: [inter, 2], or [inter, 2, G, 2] (scale, min) pairs."""
+    return "gate_up_scales" if mlp.per_channel else "gate_up_scales_min_vals"
 
 
 def _layer_sizes(layer) -> Optional[tuple]:
     """(hidden, query heads, key / value heads, intermediate) of a layer, or None where its tensors are of other sizes: kernels go by the sizes that a descriptor states."""
-    qkv, attn, mlp = layer.qkv_proj.linear, layer.self_attn, layer.mlp
+    multi, attn, mlp = _at(layer, "qkv_proj"), _at(layer, "self_attn"), _at(layer, "mlp")
+    qkv = _at(multi, "linear")
     hidden, inter = qkv.in_features, mlp.intermediate_size
     q, kv = attn.num_heads * attn.head_dim, attn.num_key_value_heads * attn.head_dim
 
     def fits(m, n: int, k: int) -> bool:
         if type(m) is not MuiInt8Linear:
-            return m.weight.shape == (n, k)
+            return _at(m, "weight").shape == (n, k)
         if m.per_channel:
-            return m.weights_int8.shape == (n, k) and m.scales.shape == (n,)
-        return m.weights_uint8.shape == (n, k) and m.scales_min_vals.numel() == 2 * n * (k >> m.quantizer.group_size_shift)
+            return _at(m, "weights_int8").shape == (n, k) and _at(m, "scales").shape == (n,)
+        return _at(m, "weights_uint8").shape == (n, k) and _at(m, "scales_min_vals").numel() == 2 * n * (k >> m.quantizer.group_size_shift)
 
-    if not (fits(qkv, q + 2 * kv, hidden) and fits(attn.o_proj, hidden, q) and fits(mlp.down_proj, hidden, inter)):
+    if not (fits(qkv, q + 2 * kv, hidden) and fits(_at(attn, "o_proj"), hidden, q) and fits(_at(mlp, "down_proj"), hidden, inter)):
         return None
-    if layer.qkv_proj.slice_starts != [0, q, q + kv] or qkv.norm_weights.shape != (hidden,) or mlp.norm_weights.shape != (hidden,):
+    if multi.slice_starts != [0, q, q + kv] or _at(qkv, "norm_weights").shape != (hidden,) or _at(mlp, "norm_weights").shape != (hidden,):
         return None
     if type(mlp) is MuiGateUpDownMLP:
-        if not (fits(mlp.gate_proj, inter, hidden) and fits(mlp.up_proj, inter, hidden)):
+        if not (fits(_at(mlp, "gate_proj"), inter, hidden) and fits(_at(mlp, "up_proj"), inter, hidden)):
             return None
-    elif mlp.gate_up_weights.shape != (inter, 2, hidden) or (
-            mlp.gate_up_scales.shape != (inter, 2) if mlp.per_channel
-            else mlp.gate_up_scales_min_vals.numel() != 4 * inter * (hidden >> mlp.group_size_shift)):
-        return None
+    else:
+        sc = _at(mlp, _scales_of(mlp))
+        if _at(mlp, "gate_up_weights").shape != (inter, 2, hidden) or (
+                sc.shape != (inter, 2) if mlp.per_channel else sc.numel() != 4 * inter * (hidden >> mlp.group_size_shift)):
+            return None
     return hidden, attn.num_heads, attn.num_key_value_heads, inter
 
 
@@ -109,29 +130,6 @@ def _held(t) -> Optional[tuple]:
     return None if t is None else (t.data_ptr(), t.dtype, t.shape, t.stride())
 
 
-_TENSORS = {MuiLinear: ("weight", "bias", "norm_weights"),
-            MuiInt8Linear: ("weights_int8", "scales", "weights_uint8", "scales_min_vals", "bias", "norm_weights"),
-            MuiGateUpDownMLP: ("norm_weights",),
-            MuiInt8GateUpDownMLP: ("norm_weights", "gate_up_weights", "gate_up_scales", "gate_up_scales_min_vals")}
-
-
-# what else a descriptor, or the choice to use one, goes by (a name may be missing: its default stands in the class then)
-_LINEAR = ("variance_epsilon", "normalize", "in_features", "out_features", "dispatchable", "per_channel", "quantizer")
-_MLP = ("variance_epsilon", "normalize", "intermediate_size", "dispatchable", "method", "per_channel", "group_size_shift")
-_VALUES = {MuiLinear: _LINEAR, MuiInt8Linear: _LINEAR, MuiGateUpDownMLP: _MLP, MuiInt8GateUpDownMLP: _MLP, MuiMultiLinear: ("slice_starts", "slice_ends"),
-           MuiSdpaAttention: ("training", "layer_idx", "num_heads", "num_key_value_heads", "head_dim")}
-_ABSENT = object()
-
-
-def _nothing():  # in the place of a weak reference
-    return None
-
-
-def _same(v, ref) -> bool:
-    """Whether v is what ref was made of. (What has gone is nobody's.)"""
-    return v is ref() and (v is not None or ref is _nothing)
-
-
 def _tensor(d: dict, name: str):
     """A module's tensor, from its __dict__: an attribute (a parameter that was deleted and set again is a plain one), a parameter, a buffer."""
     t = d.get(name)
@@ -140,6 +138,40 @@ def _tensor(d: dict, name: str):
         if t is None:
             t = d["_buffers"].get(name)
     return t
+
+
+def _linear_reads(m) -> tuple:
+    """What a descriptor, or the choice to use one, goes by in a projection."""
+    d, kind = m.__dict__, type(m)
+    gain = _tensor(d, "norm_weights")
+    gain = None if gain is None else (gain.data_ptr(), gain.dtype, gain.shape, gain.stride())
+    if kind is MuiLinear:
+        w, handle = _tensor(d, "weight"), d["cpp_module"]
+        return (kind, w.data_ptr(), w.dtype, w.shape, w.stride(), gain, _tensor(d, "bias") is None, d["normalize"], d["variance_epsilon"], d["in_features"],
+                handle is not None and handle.weights is w)
+    codes, scales = ("weights_int8", "scales") if d["per_channel"] else ("weights_uint8", "scales_min_vals")
+    return (kind, _held(_tensor(d, codes)), _held(_tensor(d, scales)), gain, _tensor(d, "bias") is None, d["normalize"], d["variance_epsilon"], d["in_features"],
+            d["per_channel"], d["dispatchable"], None if d["per_channel"] else d["quantizer"].group_size_shift)
+
+
+def _layer_reads(layer) -> Optional[tuple]:
+    """The same of a whole layer. Modules are gone through by what they hold and not by which they are; None where they are not as expected."""
+    try:
+        parts = layer.__dict__["_modules"]
+        multi, attn, mlp = parts["qkv_proj"], parts["self_attn"], parts["mlp"]
+        attn_parts, mlp_parts = attn.__dict__["_modules"], mlp.__dict__["_modules"]
+        a, f, rotary = attn.__dict__, mlp.__dict__, attn_parts["rotary_emb"].__dict__
+        cos, sin, handle = rotary["cos32"], rotary["sin32"], rotary["cpp_module"]
+        reads = (type(layer), type(multi), tuple(multi.__dict__["slice_starts"]), _linear_reads(multi.__dict__["_modules"]["linear"]),
+                 type(attn), a["training"], a["layer_idx"], a["num_heads"], a["num_key_value_heads"], a["head_dim"], _linear_reads(attn_parts["o_proj"]),
+                 id(cos), id(sin), rotary["dispatchable"], handle is not None and handle.cos32 is cos and handle.sin32 is sin and handle.layer_idx,
+                 type(mlp), _held(_tensor(f, "norm_weights")), f["normalize"], f["variance_epsilon"], f["intermediate_size"], f["dispatchable"],
+                 type(mlp_parts["activation_function"]), _linear_reads(mlp_parts["down_proj"]))
+        if type(mlp) is MuiGateUpDownMLP:
+            return reads + (f["method"], _linear_reads(mlp_parts["gate_proj"]), _linear_reads(mlp_parts["up_proj"]))
+        return reads + (f["per_channel"], f.get("group_size_shift"), _held(_tensor(f, "gate_up_weights")), _held(_tensor(f, _scales_of(mlp))))
+    except (AttributeError, KeyError):
+        return None
 
 
 def _ptr(t) -> Optional[int]:
@@ -160,51 +192,45 @@ class MuiDecoderStack:
         self.hidden = first.qkv_proj.linear.in_features
         self.hq, self.hkv, self.d = attn0.num_heads, attn0.num_key_value_heads, attn0.head_dim
         self.cos32, self.sin32 = attn0.rotary_emb.cos32, attn0.rotary_emb.sin32
-        self._attentions = [layer.self_attn for layer in layers]
         kc0 = cache.key_cache[0]
         cb, chs, cts = kc0.stride(0), kc0.stride(1), kc0.stride(2)
         self.max_cache_len = kc0.shape[2]
+        self._layer_list, self._attentions = layers, [layer.self_attn for layer in layers]
         self._cache_ptrs = tuple(t.data_ptr() for t in cache.key_cache) + tuple(t.data_ptr() for t in cache.value_cache)
-        self._keep = []  # tensors the descriptor points into
-        self._layer_list = layers
-        self._owners = []  # (module, attribute name, object) the descriptor was built from, tensors with what they hold
+        self._keep, self._owners = [], []  # tensors the descriptor points into; what matches() compares
         arr = (_lib.MuiDecoderLayerDesc * len(layers))()
         for i, layer in enumerate(layers):
-            qkv, attn, mlp = layer.qkv_proj.linear, layer.self_attn, layer.mlp
+            multi, attn, mlp = _at(layer, "qkv_proj"), _at(layer, "self_attn"), _at(layer, "mlp")
+            qkv, o, down = _at(multi, "linear"), _at(attn, "o_proj"), _at(mlp, "down_proj")
             kc, vc = cache.key_cache[attn.layer_idx], cache.value_cache[attn.layer_idx]
             if (kc.stride(), vc.stride()) != (kc0.stride(), kc0.stride()):
                 raise ValueError("cache layers must share one layout")
             qw, qp, qs, q_own = _linear_fields(qkv)
-            ow, op, osc, o_own = _linear_fields(attn.o_proj)
-            dw, dp, ds, d_own = _linear_fields(mlp.down_proj)
-            shift = max(_group_shift(m) for m in (qkv, attn.o_proj, mlp, mlp.down_proj))
+            ow, op, osc, o_own = _linear_fields(o)
+            dw, dp, ds, d_own = _linear_fields(down)
+            shift = max(_group_shift(m) for m in (qkv, o, mlp, down))
             if type(mlp) is MuiInt8GateUpDownMLP:
-                gu = mlp.gate_up_weights  # [inter, 2, hidden] codes
+                gu = _at(mlp, "gate_up_weights")  # [inter, 2, hidden] codes
                 g_ptr, u_ptr, g_pitch = gu.data_ptr(), gu.data_ptr() + gu.stride(1), gu.stride(0)
-                if mlp.per_channel:
-                    gs, gs_name = mlp.gate_up_scales, "gate_up_scales"  # [inter, 2] scales
-                else:
-                    gs, gs_name = mlp.gate_up_scales_min_vals, "gate_up_scales_min_vals"  # [inter, 2, G, 2] pairs
+                gs_name = _scales_of(mlp)
+                gs = _at(mlp, gs_name)
                 gs_ptr, us_ptr = gs.data_ptr(), gs.data_ptr() + gs.stride(1) * gs.element_size()
                 gs_stride = gs.stride(0)
-                gu_keep = [gu, gs]
                 gu_own = [(mlp, "gate_up_weights", gu), (mlp, gs_name, gs)]
             else:
-                g, u = mlp.gate_proj.weight, mlp.up_proj.weight
+                gate, up = _at(mlp, "gate_proj"), _at(mlp, "up_proj")
+                g, u = _at(gate, "weight"), _at(up, "weight")
                 g_ptr, u_ptr, g_pitch = g.data_ptr(), u.data_ptr(), g.stride(0)
                 gs_ptr, us_ptr, gs_stride = None, None, 0
-                gu_keep = [g, u]
-                gu_own = [(mlp, "gate_proj", mlp.gate_proj), (mlp, "up_proj", mlp.up_proj), (mlp.gate_proj, "weight", g), (mlp.up_proj, "weight", u)]
+                gu_own = [(mlp, "gate_proj", gate), (mlp, "up_proj", up), (gate, "weight", g), (up, "weight", u)]
+            qn, mn = _at(qkv, "norm_weights"), _at(mlp, "norm_weights")
             arr[i] = _lib.MuiDecoderLayerDesc(
-                qkv.norm_weights.data_ptr(), qw.data_ptr(), qp, ow.data_ptr(), op,
-                mlp.norm_weights.data_ptr(), g_ptr, u_ptr, g_pitch, dw.data_ptr(), dp, kc.data_ptr(), vc.data_ptr(),
+                qn.data_ptr(), qw.data_ptr(), qp, ow.data_ptr(), op,
+                mn.data_ptr(), g_ptr, u_ptr, g_pitch, dw.data_ptr(), dp, kc.data_ptr(), vc.data_ptr(),
                 _ptr(qs), _ptr(osc), gs_ptr, us_ptr, gs_stride, _ptr(ds), shift)
-            self._keep += [qkv.norm_weights, qw, qs, ow, osc, mlp.norm_weights, dw, ds, kc, vc] + gu_keep
-            owners = [(layer, "qkv_proj", layer.qkv_proj), (layer, "self_attn", attn), (layer, "mlp", mlp),
-                      (layer.qkv_proj, "linear", qkv), (qkv, "norm_weights", qkv.norm_weights),
-                      (attn, "o_proj", attn.o_proj), (mlp, "norm_weights", mlp.norm_weights),
-                      (mlp, "down_proj", mlp.down_proj)] + q_own + o_own + d_own + gu_own
-            self._owners += [(m, name, v, _held(v) if isinstance(v, torch.Tensor) else None) for m, name, v in owners]
+            self._built_from([(layer, "qkv_proj", multi), (layer, "self_attn", attn), (layer, "mlp", mlp), (multi, "linear", qkv),
+                              (qkv, "norm_weights", qn), (attn, "o_proj", o), (mlp, "norm_weights", mn), (mlp, "down_proj", down)]
+                             + q_own + o_own + d_own + gu_own, (kc, vc))
         self._layers = arr
         self.desc = _lib.MuiDecoderStackDesc(
             muillm_ext._dtype_code(first.qkv_proj.linear.norm_weights), len(layers), self.hidden, self.hq, self.hkv,
@@ -213,6 +239,11 @@ class MuiDecoderStack:
             self.cos32.stride(0), self.cos32.shape[0], cb, chs, cts, self.max_cache_len)
         self._ws = None
         self._ws_splits = 0
+
+    def _built_from(self, owners, cache_tensors) -> None:
+        """owners: [(module, attribute name, object)] of a layer. The objects are kept, tensors with what they hold."""
+        self._keep += [v for _, _, v in owners if isinstance(v, torch.Tensor)] + list(cache_tensors)
+        self._owners += [(m, name, v, _held(v) if isinstance(v, torch.Tensor) else None) for m, name, v in owners]
 
     @staticmethod
     def eligible(layers, rotary_emb, cache, batch: int) -> bool:
@@ -224,37 +255,38 @@ class MuiDecoderStack:
             return False
         eps, dtype, sizes, tables = None, None, None, None
         for layer in layers:
-            qkv, attn, mlp = getattr(layer, "qkv_proj", None), getattr(layer, "self_attn", None), getattr(layer, "mlp", None)
-            if type(qkv) is not MuiMultiLinear or not _plain_linear(qkv.linear, True):
+            multi, attn, mlp = _at(layer, "qkv_proj"), _at(layer, "self_attn"), _at(layer, "mlp")
+            if type(multi) is not MuiMultiLinear or not isinstance(attn, MuiBaseAttention) or type(mlp) not in (MuiGateUpDownMLP, MuiInt8GateUpDownMLP):
                 return False
-            if not isinstance(attn, MuiBaseAttention) or not _plain_linear(attn.o_proj, False):
+            qkv, o, down = _at(multi, "linear"), _at(attn, "o_proj"), _at(mlp, "down_proj")
+            if not (_plain_linear(qkv, True) and _plain_linear(o, False) and _plain_linear(down, False)):
                 return False
             if attn.head_dim != 128:
                 return False
             # a layer rotates with its own module's tables: they have to be the same for all
-            rotary = attn.rotary_emb
+            rotary = _at(attn, "rotary_emb")
             if not rotary.dispatchable or (tables is not None and (rotary.cos32 is not tables[0] or rotary.sin32 is not tables[1])):
                 return False
             tables = (rotary.cos32, rotary.sin32)
             if type(mlp) is MuiGateUpDownMLP:
-                if not all(_plain_linear(m, False) and type(m) is MuiLinear for m in (mlp.gate_proj, mlp.up_proj)):
+                gate, up = _at(mlp, "gate_proj"), _at(mlp, "up_proj")
+                if type(gate) is not MuiLinear or type(up) is not MuiLinear or not (_plain_linear(gate, False) and _plain_linear(up, False)):
                     return False
-                if mlp.gate_proj.weight.stride(0) != mlp.up_proj.weight.stride(0):
+                gate, up = _at(gate, "weight"), _at(up, "weight")
+                if gate.stride(0) != up.stride(0):
                     return False
-            elif type(mlp) is MuiInt8GateUpDownMLP:
-                if not (mlp.dispatchable and mlp.gate_up_weights.is_contiguous()):
+                held = [gate, up]
+            else:
+                if not (mlp.dispatchable and _at(mlp, "gate_up_weights").is_contiguous()):
                     return False
-                sc = mlp.gate_up_scales if mlp.per_channel else mlp.gate_up_scales_min_vals
+                sc = _at(mlp, _scales_of(mlp))
                 if not sc.is_contiguous() or (not mlp.per_channel and mlp.group_size_shift < 4):
                     return False
-            else:
+                held = [sc]
+            if not mlp.normalize or not isinstance(_at(mlp, "activation_function"), nn.SiLU):
                 return False
-            if not mlp.normalize or not isinstance(mlp.activation_function, nn.SiLU):
-                return False
-            if not _plain_linear(mlp.down_proj, False):
-                return False
-            w = qkv.linear.norm_weights
-            if w is None or mlp.norm_weights is None or w.dtype not in (torch.float16, torch.bfloat16):
+            w, mw = _at(qkv, "norm_weights"), _at(mlp, "norm_weights")
+            if w is None or mw is None or w.dtype not in (torch.float16, torch.bfloat16):
                 return False
             if cache.key_cache[attn.layer_idx].dtype != w.dtype or (dtype is not None and w.dtype != dtype):
                 return False
@@ -264,18 +296,14 @@ class MuiDecoderStack:
                 return False
             sizes = of
             # one type throughout, as the kernels read it (the modules refuse others)
-            held = [m.weight if type(m) is MuiLinear else m.scales if m.per_channel else m.scales_min_vals for m in (qkv.linear, attn.o_proj, mlp.down_proj)]
-            held += [mlp.norm_weights] + ([mlp.gate_proj.weight, mlp.up_proj.weight] if type(mlp) is MuiGateUpDownMLP
-                                          else [mlp.gate_up_scales if mlp.per_channel else mlp.gate_up_scales_min_vals])
+            held += [_at(m, "weight") if type(m) is MuiLinear else _at(m, "scales") if m.per_channel else _at(m, "scales_min_vals") for m in (qkv, o, down)] + [mw]
             if any(t.dtype != dtype for t in held):
                 return False
             # the int8 projections of a layer share one format: all per-channel, or all in the group
             # format with one group size (the layer descriptor carries a single shift)
-            int8_mods = [m for m in (qkv.linear, attn.o_proj, mlp, mlp.down_proj)
-                         if type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP)]
-            if len({_group_shift(m) for m in int8_mods}) > 1:
+            if len({_group_shift(m) for m in (qkv, o, mlp, down) if type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP)}) > 1:
                 return False
-            e = (float(qkv.linear.variance_epsilon), float(mlp.variance_epsilon))
+            e = (float(qkv.variance_epsilon), float(mlp.variance_epsilon))
             if e[0] != e[1] or (eps is not None and e != eps):
                 return False
             eps = e
@@ -333,39 +361,25 @@ class MuiPromptStack(MuiDecoderStack):
     """The same for `mui_decoder_stack_prompt`: prompts, and steps of more batch rows than the decode kernels take. Layers called one by one run the same
     kernels; here nobody can listen in between, so a model with hooks stays with its modules.
 
-    What the descriptor was built from is watched, modules by weak references and tensors by what they hold (current(), asked before every call, takes a few us per
-    layer, where examining the layers anew takes ~35 with an idle GPU waiting): nothing is kept alive beyond a call."""
+    Before every call the layers are read again and compared with what they were (current(), a few us per layer, where examining them and building the descriptor takes
+    ~20 with an idle GPU waiting). Tensors are compared by what they hold: nothing is kept alive beyond a call."""
 
     def __init__(self, layers, rotary_emb, cache: MuiStaticCache):
         super().__init__(layers, rotary_emb, cache, 1)
-        self._keep, self._owners, self._layer_list = [], [], None
         self._watched, self._layer_refs = None, [weakref.ref(layer) for layer in layers]
-        self._cache_layers = [layer.self_attn.layer_idx for layer in layers]
+        self._cache_layers = [attn.layer_idx for attn in self._attentions]
+        self._layer_list = self._attentions = self._cache_ptrs = None  # (nothing is held but weakly)
         self._bound(cache)
-        self._attentions = None  # (layers are held weakly here)
-        int8 = any(type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP)
-                   for layer in layers for m in (layer.qkv_proj.linear, layer.self_attn.o_proj, layer.mlp, layer.mlp.down_proj))
+        int8 = any(x.qkv_scales or x.o_scales or x.gate_scales or x.down_scales for x in self._layers)
         self._most_rows = min(muillm_ext.INT8_DEQUANT_MIN_TOKENS, muillm_ext.INT8_GROUP_DEQUANT_MIN_TOKENS) - 1 if int8 else 1 << 30
-        self._attention_refs = [weakref.ref(layer.self_attn) for layer in layers]
+
+    def _built_from(self, owners, cache_tensors) -> None:
+        pass  # see remember()
 
     def remember(self) -> None:
         """What current() compares with. (Made behind the first call, while the GPU is at work.)"""
-        if self._watched is not None:
-            return
-
-        def ref(v):
-            return _nothing if v is None else weakref.ref(v)
-
-        watched = []  # per module: itself, its children, what its tensors hold, what else was read from it, its handle
-        for layer in [r() for r in self._layer_refs]:
-            qkv, attn, mlp = layer.qkv_proj, layer.self_attn, layer.mlp
-            inside = [getattr(mlp, n) for n in ("gate_proj", "up_proj", "down_proj") if isinstance(getattr(mlp, n, None), nn.Module)]
-            for m in [layer, qkv, qkv.linear, attn, attn.o_proj, mlp] + inside:
-                d, kind = m.__dict__, type(m)
-                watched.append((weakref.ref(m), [(k, ref(v)) for k, v in m._modules.items()],
-                                [(k, _held(_tensor(d, k))) for k in _TENSORS.get(kind, ())],
-                                [(k, d.get(k, _ABSENT)) for k in _VALUES.get(kind, ())], ref(d.get("cpp_module"))))
-        self._watched = watched  # whole: another thread may ask meanwhile
+        if self._watched is None:
+            self._watched = [_layer_reads(r()) for r in self._layer_refs]
 
     @staticmethod
     def eligible(layers, rotary_emb, cache) -> bool:
@@ -375,22 +389,24 @@ class MuiPromptStack(MuiDecoderStack):
         if not MuiPromptStack._cache_serves(cache):
             return False
         for layer in layers:
-            qkv, attn, mlp = layer.qkv_proj.linear, layer.self_attn, layer.mlp
+            attn, mlp = _at(layer, "self_attn"), _at(layer, "mlp")
+            qkv, o, down = _at(_at(layer, "qkv_proj"), "linear"), _at(attn, "o_proj"), _at(mlp, "down_proj")
             if type(layer) is not MuiDecoderLayer or type(attn) is not MuiSdpaAttention or attn.training:
                 return False
-            rotary, handle = attn.rotary_emb, attn.rotary_emb.cpp_module  # (prompts rotate by what the handle names)
+            rotary = _at(attn, "rotary_emb")
+            handle = rotary.cpp_module  # (prompts rotate by what the handle names)
             if handle is None or handle.cos32 is not rotary.cos32 or handle.sin32 is not rotary.sin32 or handle.layer_idx != attn.layer_idx:
                 return False
             if type(mlp) is MuiGateUpDownMLP and (not mlp.dispatchable or mlp.method == _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED):
                 return False
-            for m in (qkv, attn.o_proj) + ((mlp.down_proj,) if type(mlp) is MuiInt8GateUpDownMLP else ()):
-                if type(m) is MuiLinear and (m.cpp_module is None or m.cpp_module.weights is not m.weight):
+            for m in (qkv, o) + ((down,) if type(mlp) is MuiInt8GateUpDownMLP else ()):
+                if type(m) is MuiLinear and (m.cpp_module is None or m.cpp_module.weights is not _at(m, "weight")):
                     return False
             hidden, inter = qkv.in_features, mlp.intermediate_size
             if hidden % 8 or inter % 8 or hidden > 16384:
                 return False
-            int8 = any(type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP) for m in (qkv, attn.o_proj, mlp, mlp.down_proj))
-            if int8 and (hidden % 16 or inter % 16 or (inter > 16384 and qkv.norm_weights.dtype != torch.float16)):
+            int8 = any(type(m) in (MuiInt8Linear, MuiInt8GateUpDownMLP) for m in (qkv, o, mlp, down))
+            if int8 and (hidden % 16 or inter % 16 or (inter > 16384 and _at(qkv, "norm_weights").dtype != torch.float16)):
                 return False
         return True
 
@@ -430,32 +446,8 @@ class MuiPromptStack(MuiDecoderStack):
                 return False
         if self._watched is None:
             return False  # the first call did not come about
-        attentions = [layer.__dict__["_modules"].get("self_attn") for layer in layers]
-        if None in attentions or not _rotate_with(attentions, self.cos32, self.sin32):
-            return False
-        for attn in attentions:
-            rotary = attn.__dict__["_modules"]["rotary_emb"].__dict__
-            handle = rotary["cpp_module"]
-            if handle is None or handle.cos32 is not self.cos32 or handle.sin32 is not self.sin32 or handle.layer_idx != attn.layer_idx or not rotary["dispatchable"]:
-                return False
-        for r, children, tensors, values, handle in self._watched:
-            m = r()
-            if m is None:
-                return False
-            d = m.__dict__
-            mods = d["_modules"]
-            if len(mods) != len(children):
-                return False
-            for k, v in children:
-                if not _same(mods.get(k), v):
-                    return False
-            for k, v in tensors:
-                if _held(_tensor(d, k)) != v:
-                    return False
-            for k, v in values:
-                if d.get(k, _ABSENT) is not v:
-                    return False
-            if not _same(d.get("cpp_module"), handle):
+        for layer, reads in zip(layers, self._watched):
+            if _layer_reads(layer) != reads:
                 return False
         return True
 
@@ -472,10 +464,6 @@ class MuiPromptStack(MuiDecoderStack):
         cache = self._cache()
         if b > cache.max_batch_size or b > 65535 or t > 65535 or not 1 <= b * t <= self._most_rows:
             return False
-        for r in self._attention_refs:  # (set at any time, on a module or for all of them)
-            most = r().prefill_kernel_max_tokens
-            if most is not None and t > most:
-                return False
         if cache.get_seq_length() + t > self.max_cache_len:
             return False  # the modules refuse to read a cache beyond its rows
         if position_ids.dtype != torch.int64 or cache_position.dtype != torch.int64 or not (position_ids.is_cuda and cache_position.is_cuda):
@@ -488,10 +476,18 @@ class MuiPromptStack(MuiDecoderStack):
         g = nn.modules.module
         if g._global_forward_hooks or g._global_forward_pre_hooks:
             return False
-        modules = [r() for r, *_ in self._watched] if self._watched else [m for r in self._layer_refs for m in r().modules()]
-        for m in modules:
-            d = m.__dict__
-            if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
+        for r in self._layer_refs:
+            layer = r()
+            parts = layer.__dict__["_modules"]
+            multi, attn, mlp = parts["qkv_proj"], parts["self_attn"], parts["mlp"]
+            inside = mlp.__dict__["_modules"]
+            for m in (layer, multi, multi.__dict__["_modules"]["linear"], attn, attn.__dict__["_modules"]["o_proj"], mlp, inside["down_proj"], inside.get("gate_proj", mlp),
+                      inside.get("up_proj", mlp)):
+                d = m.__dict__
+                if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
+                    return False
+            most = attn.prefill_kernel_max_tokens  # (set at any time, on a module or for all of them)
+            if most is not None and t > most:
                 return False
         return True
 

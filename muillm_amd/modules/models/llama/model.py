@@ -91,7 +91,7 @@ class MuiCausalLMOutput:
 
 
 # Products of a layer and a first prompt (rows x weights) from which the GPU is longer at work on a layer (~200 us) than the host on its modules: such a
-# prompt runs on the modules, and the layers are examined for the single call behind it (~35 us per layer) instead of in front of it, with an idle GPU.
+# prompt runs on the modules, and the layers are examined for the single call behind it (~20 us per layer) instead of in front of it, with an idle GPU.
 _BUSY_PRODUCTS = 10 ** 11
 
 

@@ -193,7 +193,7 @@ def test_what_may_be_set_after_a_prompt(lm, monkeypatch):
         m.setattr(type(attn), "prefill_kernel_max_tokens", 19)
         assert not _takes(stack)
     assert _takes(stack) and stack.current(layers)
-    for m, name, value in ((layers[0].mlp.down_proj, "per_channel", True), (layers[0].mlp, "method", None), (layers[0].mlp, "intermediate_size", 640), (attn, "training", True),
+    for m, name, value in ((layers[0].mlp.down_proj, "normalize", True), (layers[0].mlp, "method", None), (layers[0].mlp, "intermediate_size", 640), (attn, "training", True),
                            (layers[1].qkv_proj.linear, "variance_epsilon", 1e-3), (layers[1].qkv_proj, "slice_starts", [0, 512, 640]), (attn.o_proj, "cpp_module", None)):
         before = m.__dict__.get(name, m)
         setattr(m, name, value)
