@@ -140,15 +140,22 @@ def _tensor(d: dict, name: str):
     return t
 
 
+def _handle_agrees(m, weight, gain) -> bool:
+    """Whether a MuiLinear's handle, by which its module computes, names what the module names (a tensor that was replaced is the module's alone until finalize_init())."""
+    handle = m.__dict__["cpp_module"]
+    return (handle is not None and handle.weights is weight and handle.norm_weights is gain and handle.epsilon == m.__dict__["variance_epsilon"]
+            and handle.mul_bias is None and handle.add_bias is None)
+
+
 def _linear_reads(m) -> tuple:
     """What a descriptor, or the choice to use one, goes by in a projection."""
     d, kind = m.__dict__, type(m)
-    gain = _tensor(d, "norm_weights")
-    gain = None if gain is None else (gain.data_ptr(), gain.dtype, gain.shape, gain.stride())
+    norm = _tensor(d, "norm_weights")
+    gain = None if norm is None else (norm.data_ptr(), norm.dtype, norm.shape, norm.stride())
     if kind is MuiLinear:
-        w, handle = _tensor(d, "weight"), d["cpp_module"]
+        w = _tensor(d, "weight")
         return (kind, w.data_ptr(), w.dtype, w.shape, w.stride(), gain, _tensor(d, "bias") is None, d["normalize"], d["variance_epsilon"], d["in_features"],
-                handle is not None and handle.weights is w)
+                _handle_agrees(m, w, norm))
     codes, scales = ("weights_int8", "scales") if d["per_channel"] else ("weights_uint8", "scales_min_vals")
     return (kind, _held(_tensor(d, codes)), _held(_tensor(d, scales)), gain, _tensor(d, "bias") is None, d["normalize"], d["variance_epsilon"], d["in_features"],
             d["per_channel"], d["dispatchable"], None if d["per_channel"] else d["quantizer"].group_size_shift)
@@ -400,7 +407,7 @@ class MuiPromptStack(MuiDecoderStack):
             if type(mlp) is MuiGateUpDownMLP and (not mlp.dispatchable or mlp.method == _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED):
                 return False
             for m in (qkv, o) + ((down,) if type(mlp) is MuiInt8GateUpDownMLP else ()):
-                if type(m) is MuiLinear and (m.cpp_module is None or m.cpp_module.weights is not _at(m, "weight")):
+                if type(m) is MuiLinear and not _handle_agrees(m, _at(m, "weight"), _at(m, "norm_weights")):
                     return False
             hidden, inter = qkv.in_features, mlp.intermediate_size
             if hidden % 8 or inter % 8 or hidden > 16384:

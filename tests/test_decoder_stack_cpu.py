@@ -220,3 +220,23 @@ def test_tensors_of_another_type(lm):
             assert not _eligible(lm), (type(m), name)
             t.data = plain
     assert _eligible(lm)
+
+
+def test_handles_that_name_other_tensors(lm):
+    """A projection's module computes by its handle, which names the tensors of the last finalize_init()."""
+    qkv, o = lm.model.layers[1].qkv_proj.linear, lm.model.layers[0].self_attn.o_proj
+    for m, name, value in ((qkv, "norm_weights", torch.nn.Parameter(2 * qkv.norm_weights.detach(), requires_grad=False)), (qkv, "variance_epsilon", 1e-5),
+                           (o, "weight", torch.nn.Parameter(2 * o.weight.detach(), requires_grad=False))):
+        stack, before = _watching(lm), getattr(m, name)
+        lm_eps = [(x.qkv_proj.linear, x.mlp) for x in lm.model.layers]
+        if name == "variance_epsilon":  # (of all layers: one descriptor has one)
+            value = 2 * before
+            for x, y in lm_eps:
+                x.variance_epsilon = y.variance_epsilon = value
+        else:
+            setattr(m, name, value)
+        assert not stack.current(lm.model.layers) and not MuiPromptStack.eligible(lm.model.layers, lm.model.rotary_emb, lm.cache), name
+        for x, _ in lm_eps:
+            x.finalize_init()
+        o.finalize_init()
+        assert MuiPromptStack.eligible(lm.model.layers, lm.model.rotary_emb, lm.cache), name
