@@ -35,7 +35,7 @@ from ...gateupdownmlp import MuiGateUpDownMLP
 from ...kvcache.cache_utils import (MuiCache, MuiStaticCache, create_static_cache,
                                     grow_static_cache_if_needed)
 from ...linear import MuiLinear
-from ...module import MuiModule
+from ...module import MuiModule, heard
 from ...multilinear import MuiMultiLinear
 from ...norm.rmsnorm import MuiRMSNorm
 from ..generation import MuiGenerationMixin
@@ -169,7 +169,7 @@ class MuiLlamaModel(MuiModule):
         """The single-call layer stack for a prompt, or for a step of more batch rows than the decode kernels take; None: layer by layer;
         False: layer by layer, and _examine_layers() behind it."""
         if (not self.use_decoder_stack or torch.is_grad_enabled() or not muillm_ext.PROMPT_NORM_FIRST or not hidden_states.is_cuda
-                or not isinstance(cache, MuiStaticCache)):
+                or not isinstance(cache, MuiStaticCache) or heard(self.rotary_emb)):  # (that module is called for layers one by one)
             return None
         st = self._prompt_layers
         if st is not None and st.current(self.layers):

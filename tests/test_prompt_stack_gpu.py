@@ -141,6 +141,17 @@ def test_what_stays_layer_by_layer():
 
 
 @torch.no_grad()
+def test_hook_on_the_models_positions():
+    lm, ids, heard = _lm(), _ids(1, 30), []
+    want = _run(lm, True, [ids], 64, 1)[0]
+    handle = lm.model.rotary_emb.register_forward_hook(lambda mod, args, out: heard.append(out[0].shape))
+    got, _, calls, _ = _run(lm, True, [ids], 64, 1)
+    handle.remove()
+    assert heard == [(1, 30, 128)] and calls == 0 and torch.equal(got, want)
+    assert _run(lm, True, [ids], 64, 1)[2] == 1
+
+
+@torch.no_grad()
 def test_layers_that_differ():
     lm, other = _lm(), _lm(intermediate_size=640)
     lm.model.layers[1].mlp = other.model.layers[1].mlp
