@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+from muillm_amd import _lib
 from muillm_amd import hybrid_ops as ops
 
 pytestmark = pytest.mark.gpu
@@ -107,8 +108,14 @@ def test_units_without_a_tile():
     expert, _, pairs, tiles = ops.moe_route(logits.to(DEV), None, experts, 1, 16)
     assert int(tiles[0, 2]) == 0
     w = torch.ones(experts, ff, width, dtype=torch.bfloat16, device=DEV)
-    ops.moe_experts(torch.ones(tokens, width, dtype=torch.bfloat16, device=DEV), w, w, w, 7.0, expert, pairs, tiles, 16)
-    torch.cuda.synchronize()
+    x, act = torch.ones(tokens, width, dtype=torch.bfloat16, device=DEV), torch.full((tokens, ff), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = torch.full((tokens, width), 7.0, dtype=torch.bfloat16, device=DEV)
+    lib, s, code = _lib.load(), torch.cuda.current_stream().cuda_stream, _lib.MUI_DTYPE_BF16
+    _lib.check(lib.mui_moe_gateup(s, code, w.data_ptr(), w.data_ptr(), ff * width, x.data_ptr(), 7.0, expert.data_ptr(), pairs.data_ptr(), tiles.data_ptr(), 16, act.data_ptr(),
+                                  experts, ff, width, 1, tokens), "gateup")
+    _lib.check(lib.mui_moe_down(s, code, w.data_ptr(), ff * width, act.data_ptr(), expert.data_ptr(), pairs.data_ptr(), tiles.data_ptr(), 16, out.data_ptr(),
+                                experts, width, ff, 1, tokens), "down")
+    assert bool((act == 7.0).all()) and bool((out == 7.0).all())
 
 
 @pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))

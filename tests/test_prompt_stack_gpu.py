@@ -92,15 +92,42 @@ def test_captured_steps_of_many_rows(padded):
         mask = torch.ones(batch, t, dtype=torch.int64, device=DEV)
         mask[::2, :3] = 0
         ids = ids * mask
-    tokens = []
-    for graph in (True, False):
-        decoder = MuiGraphDecoder(lm, use_graph=graph)
-        for _ in range(2):
-            cache = lm.create_cache(batch, 64)
-            decoder.prefill(ids, 12, cache, attention_mask=mask)
-            decoder.decode(11)
-            tokens.append(decoder.out_tokens.clone())
-    assert all(torch.equal(tokens[0], x) for x in tokens[1:])
+    shapes, plain = [], MuiPromptStack.run
+
+    def counted(self, *a):
+        shapes.append(tuple(a[0].shape[:2]))
+        return plain(self, *a)
+
+    MuiPromptStack.run = counted
+    found = []
+    try:
+        for one_call in (True, False):
+            lm.model.use_decoder_stack = one_call
+            for graph in (True, False):
+                decoder = MuiGraphDecoder(lm, use_graph=graph)
+                for _ in range(2):
+                    del shapes[:]
+                    cache = lm.create_cache(batch, 64)
+                    decoder.prefill(ids, 12, cache, attention_mask=mask)
+                    decoder.decode(11)
+                    found.append((decoder.out_tokens.clone(), decoder.logits.clone()))
+                    # the prompt, and every step that is not a replay, by the call that is asked for
+                    assert (shapes.count((batch, t)), (batch, 1) in shapes or graph) == (1, True) if one_call else not shapes
+    finally:
+        MuiPromptStack.run = plain
+        lm.model.use_decoder_stack = True
+    assert all(torch.equal(found[0][0], x) and torch.equal(found[0][1], y) for x, y in found[1:])
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("batch,t", [(1, 20), (1, 101), (2, 64), (20, 1)])
+def test_same_bits_where_k_is_divided(batch, t):
+    """Long rows, few outputs: the linears share K between workgroups, and the launch that adds the shares takes the norm along."""
+    lm = _lm(hidden_size=2048, intermediate_size=8192, num_hidden_layers=2, num_attention_heads=16, num_key_value_heads=4)
+    turns = [_ids(batch, t), _ids(batch, t, seed=4)]
+    got, cache, calls, _ = _run(lm, True, turns, 256, batch)
+    want, cache_want, none, _ = _run(lm, False, turns, 256, batch)
+    assert calls == 2 and none == 0 and torch.equal(got, want) and torch.equal(cache, cache_want)
 
 
 @torch.no_grad()
