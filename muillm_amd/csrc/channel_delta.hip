@@ -219,7 +219,8 @@ struct LowRankHeld {
 // NR > 0: NR rows of S per thread in registers, for the sizes that delta_step_held names. 0: every size, S stays in memory.
 // TWO, for more workgroups than CUs: at most 128 registers, so that a CU runs two workgroups and one's chain of barriers lies under the other's. The low-rank matrices
 // are then read where they are used (batch rows share them in L2), and addresses are formed again instead of kept. us in bf16, one per CU / two, heads of
-// 128 x 128: 320 workgroups (16 heads, 20 rows) 24.4 / 18.9, 512 27.0 / 21.7, 288 (32 heads, 9 rows) 23.9 / 18.1, 544 36.0 / 32.5, 1024 51.2 / 39.5; heads of 64 x 64, 512 17.8 / 13.0.
+// 128 x 128: 320 workgroups (16 heads, 20 rows) 24.4 / 18.9, 512 27.0 / 21.7, 288 (32 heads, 9 rows) 23.9 / 18.1, 544 36.0 / 32.5, 1024 51.2 / 39.5; heads of 64 x 64, 512 17.8 / 13.0. Calls of several tokens
+// read the low-rank matrices for each of them and are faster all the same: 320 workgroups of 128 x 128, 2 / 4 / 16 tokens 36.7 / 28.1, 61.3 / 45.2, 211 / 151; 64 x 64, 272, 16 tokens 163 / 97.
 template <typename T, int NR, bool TWO = false>
 __global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 1, 8))) delta_step_kernel(const DeltaParams p, int cgp) {
   typedef typename T::storage S;

@@ -441,7 +441,7 @@ static StreamParams stream_params(const SkinnyParams& q, float* part, bool add) 
 // what another kernel does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
   // gate/up beyond 64 tokens: the tiled GEMM. Units of six and eight token tiles are built for linears only; for gate/up they were measured at 128 tokens and
-  // 14336 x 4096 alone (64 us, tiles 52), between 65 and 127 not at all
+  // 14336 x 4096 alone (64 us, tiles 55), between 65 and 127 not at all (tiles: 51 us at 65 tokens, 54 at 101)
   if (!stream_serves(q, epilogue == SK_GATEUP ? 64 : 128)) return MUI_ERR_UNSUPPORTED;
   const StreamParams p = stream_params(q, part, true);
   if (dtype == MUI_DTYPE_F16) return epilogue == SK_GATEUP ? launch_stream_t<F16, SK_GATEUP>(s, p, 0) : launch_stream_t<F16, SK_LINEAR>(s, p, part_bytes);

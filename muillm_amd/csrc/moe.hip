@@ -270,6 +270,8 @@ __device__ __forceinline__ MoeTile moe_tile_at(const MoeGemmParams& p, int i, in
 // read back as operands: 16 rows x 128 k-values per tile and stage, rows of 256 bytes whose 16-byte chunk c
 // lives at chunk c ^ row. Loaded straight in operand order (64 bytes of 16 rows per instruction) the same
 // bytes arrive at about two thirds of the rate.
+// What a workgroup needs first stands in front of p as scalars: the first 16 dwords of a kernel's scalar arguments are in registers when a wave starts (the compiler's
+// kernarg preload, which a struct does not get), the rest comes with a load of its own.
 constexpr int kT16Seg = 128;
 template <typename T, int EPI>
 __global__ void __launch_bounds__(256, 2) moe_tile16_kernel(const MoeTile* tiles, const uint16_t* w0, const uint16_t* w1, long expert_stride, int n, int k, int max_tiles,
