@@ -272,7 +272,7 @@ class MuiDecoderStack:
                 return False
             # a layer rotates with its own module's tables: they have to be the same for all
             rotary = _at(attn, "rotary_emb")
-            if not rotary.dispatchable or (tables is not None and (rotary.cos32 is not tables[0] or rotary.sin32 is not tables[1])):
+            if not getattr(rotary, "dispatchable", False) or (tables is not None and (rotary.cos32 is not tables[0] or rotary.sin32 is not tables[1])):
                 return False
             tables = (rotary.cos32, rotary.sin32)
             if type(mlp) is MuiGateUpDownMLP:

@@ -98,6 +98,9 @@ def test_layers_of_other_tables(lm, monkeypatch):
         assert not _eligible(lm) and not any(a() for a in asked), name
         setattr(owner, name, plain)
         assert _eligible(lm) and all(a() for a in asked)
+    lm.model.layers[1].self_attn.rotary_emb = None
+    assert not _eligible(lm) and not any(a() for a in asked)
+    lm.model.layers[1].self_attn.rotary_emb = rotary
     rotary.cpp_module.sin32 = other.sin32
     assert not asked[1]() and not MuiPromptStack.eligible(lm.model.layers, lm.model.rotary_emb, lm.cache)
     rotary.cpp_module.sin32 = rotary.sin32
