@@ -127,7 +127,7 @@ def test_hybrid_layers_use_it_and_hooks_are_heard(monkeypatch):
     taken.clear()
     apart = lm(input_ids=ids).logits.float()
     assert taken and all(r is None for r in taken)
-    assert float((fused - apart).norm() / apart.norm()) < 0.03  # (K may be divided otherwise)
+    assert torch.equal(fused, apart)
     hook = lambda mod, args, out: out + 1.0  # noqa: E731
     handles = [layer.mixer.out_proj.register_forward_hook(hook) for layer in lm.model.layers]
     want = lm(input_ids=ids).logits.float()
