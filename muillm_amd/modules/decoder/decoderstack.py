@@ -454,7 +454,7 @@ class MuiPromptStack(MuiDecoderStack):
         if self._watched is None:
             return False  # the first call did not come about
         for layer, reads in zip(layers, self._watched):
-            if _layer_reads(layer) != reads:
+            if reads is None or _layer_reads(layer) != reads:
                 return False
         return True
 

@@ -210,6 +210,10 @@ def test_what_may_be_set_after_a_prompt(lm, monkeypatch):
     stack = _watching(lm)
     layers[0].mlp = None
     assert not stack.current(layers)
+    unread = MuiPromptStack.__new__(MuiPromptStack)  # what could not be read is not the same as before
+    unread.__dict__.update(stack.__dict__, _watched=None)
+    unread.remember()
+    assert unread._watched[0] is None and not unread.current(layers)
 
 
 def test_tensors_of_another_type(lm):
