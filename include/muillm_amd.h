@@ -435,6 +435,13 @@ int mui_greedy_advance_ws(mui_stream_t stream, int dtype, const void* logits, lo
                           size_t workspace_bytes, const void* embed_table, long embed_row_stride,
                           void* embed_out, int embed_dim);
 
+/* Sets `count` buffers, each to a 64-bit value of its own: buffers[i] (device memory) receives bytes[i] / 8 copies of
+ * values[i], in one launch per 64 buffers; buffers and sizes are multiples of 8 bytes (else MUI_ERR_ALIGNMENT, nothing
+ * is written), a size of 0 is skipped. The three arrays are host memory and read before the call returns. The beginning of a request:
+ * caches cleared, a decode loop's counters put back (the reference clears its caches layer by layer,
+ * muillm/modules/kvcache/cache_utils.py). */
+int mui_fill_buffers(mui_stream_t stream, int count, void* const* buffers, const size_t* bytes, const int64_t* values);
+
 /* Sampling twin of mui_greedy_advance: tok = argmax_v(logits[b, v] / temperature - log q_v) with
  * q_v ~ Exp(1), which is the draw of the reference's sync-free multinomial
  * argmax(softmax(logits / temperature) / q) (muillm/sampling/multinomial.py:4-6) without

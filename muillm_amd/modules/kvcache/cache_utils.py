@@ -138,9 +138,7 @@ class MuiStaticCache(MuiCache):
         return self.max_cache_len
 
     def reset(self):
-        for k, v in zip(self.key_cache, self.value_cache):
-            k.zero_()
-            v.zero_()
+        muillm_ext.fill_buffers(list(self.key_cache) + list(self.value_cache))
         self._seen_tokens = 0
         if self.cpp_module is not None:
             self.cpp_module.seen_tokens = 0

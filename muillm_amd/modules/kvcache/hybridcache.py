@@ -9,6 +9,7 @@ from typing import List, Optional, Sequence
 
 import torch
 
+from ... import muillm_ext
 from .cache_utils import MuiCache, _next_pow2
 
 
@@ -80,8 +81,7 @@ class MuiRecurrentState:
         pass
 
     def reset(self) -> None:
-        for t in self.values:
-            t.zero_()
+        muillm_ext.fill_buffers(self.values)
 
 
 class MuiHybridCache(MuiCache):
@@ -139,8 +139,11 @@ class MuiHybridCache(MuiCache):
         self.max_cache_len = capacity
 
     def reset(self) -> None:
+        plain = [s for s in self._states() if type(s) is MuiRecurrentState]  # all of them in one launch
+        muillm_ext.fill_buffers([t for s in plain for t in s.values])
         for s in self._states():
-            s.reset()
+            if type(s) is not MuiRecurrentState:
+                s.reset()
         self._seen_tokens = 0
         self.row_start = None
 

@@ -265,15 +265,14 @@ class MuiGraphDecoder:
             self.graph = None
         # the first new token goes through the same kernel as all later ones: the counters start
         # one step back and the launch advances them to (prompt_len, prompt_len, 1)
+        at = past + prompt_len - 1
+        begin = [(self.cpos, at), (self.step, 0), (self.unfinished, 1),
+                 (self.out_tokens, self.pad_token_id if self.eos is not None else 0)]  # columns never reached (early stop) read as padding
         if padded:
             self.pos.copy_(am.sum(-1, keepdim=True) - 1)
         else:
-            self.pos.fill_(past + prompt_len - 1)
-        self.cpos.fill_(past + prompt_len - 1)
-        self.step.zero_()
-        # columns never reached (early stop) read as padding
-        self.out_tokens.fill_(self.pad_token_id if self.eos is not None else 0)
-        self.unfinished.fill_(1)
+            begin.append((self.pos, at))
+        muillm_ext.fill_buffers(*zip(*begin))
         self._advance(out.logits[:, -1, :])
         return out.logits[:, -1, :]
 

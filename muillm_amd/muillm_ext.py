@@ -19,8 +19,9 @@ CPU fallback for CUDA inputs and no silent one for a missing library.
 from __future__ import annotations
 
 import contextlib
+import ctypes
 import threading
-from typing import List, Optional, Tuple
+from typing import List, Optional, Sequence, Tuple
 
 import torch
 import torch.nn.functional as F
@@ -1191,6 +1192,26 @@ def greedy_workspace(rows: int, device) -> torch.Tensor:
     """Zero-filled workspace for mui_greedy_advance on `rows` logits rows: one per decode loop (calls
     that share it must not overlap); every call leaves it zero-filled again."""
     return torch.zeros(_lib.load().mui_greedy_workspace_bytes(int(rows)), dtype=torch.uint8, device=device)
+
+
+def fill_buffers(tensors: Sequence[torch.Tensor], values: Optional[Sequence[int]] = None) -> None:
+    """Sets every tensor: int64 ones to values[i], any type to zero without values. Contiguous plain tensors of one GPU go in one
+    launch; whatever else there is takes torch's own fill."""
+    plain, here = [], torch.cuda.current_device() if any(t.is_cuda for t in tensors) else None
+    for i, t in enumerate(tensors):
+        value = 0 if values is None else int(values[i])
+        if (t.is_cuda and t.device.index == here and type(t) in (torch.Tensor, torch.nn.Parameter) and not t.requires_grad and t.is_contiguous()
+                and (value == 0 or t.dtype == torch.int64) and (t.numel() * t.element_size()) % 8 == 0 and t.data_ptr() % 8 == 0):
+            if t.numel():
+                plain.append((t, value))
+        else:
+            t.fill_(value)
+    n = len(plain)
+    if n:
+        check(_lib.load().mui_fill_buffers(
+            _stream(plain[0][0]), n, (ctypes.c_void_p * n)(*[t.data_ptr() for t, _ in plain]),
+            (ctypes.c_size_t * n)(*[t.numel() * t.element_size() for t, _ in plain]), (ctypes.c_int64 * n)(*[v for _, v in plain])),
+            "mui_fill_buffers")
 
 
 def mui_sample_advance(logits: torch.Tensor, next_ids: torch.Tensor, step: torch.Tensor, tokens_out: torch.Tensor,
