@@ -723,6 +723,18 @@ int mui_hybrid_attention(mui_stream_t stream, int dtype, int route, const void* 
                          float softcap, int window, int keep_first, void* scratch, int span, void* out, int batch,
                          int t, int heads, int kv_heads, int dim, int vdim, int max_cache_len);
 
+/* One step (one new token per row) in one launch: what mui_hybrid_prepare and mui_hybrid_attention give, up to the order of
+ * sums. mui_hybrid_step_serves: 1 for 16-bit models whose visible keys -- window + keep_first, or the capacity -- are few enough, else 0
+ * (a function of its arguments and the device's number of compute units); where it is 0 the call returns MUI_ERR_UNSUPPORTED. Alignments: 16 bytes for proj, gains,
+ * caches, out and their pitches and offsets, 8 for the gate. */
+int mui_hybrid_step_serves(int dtype, int batch, int heads, int kv_heads, int dim, int vdim, int window, int keep_first, int max_cache_len);
+int mui_hybrid_step(mui_stream_t stream, int dtype, const void* proj, long pitch, long k_offset, long v_offset,
+                    const void* q_gain, const void* k_gain, float epsilon, const double* inv_freq, int rot_dims,
+                    const void* gate, long gate_pitch, const int64_t* cache_position, const int64_t* row_start,
+                    void* k_cache, long k_batch_stride, void* v_cache, long v_batch_stride, float scale, float softcap,
+                    int window, int keep_first, void* out, int batch, int heads, int kv_heads, int dim, int vdim,
+                    int max_cache_len);
+
 /* Gated delta rule with one decay per head and key channel, over t tokens per batch row, from and to the state
  * S [batch, heads, dk, dv] (fp32; zero: a fresh sequence); value head h uses query / key head
  * h / (heads / kv_heads):

@@ -138,6 +138,9 @@ _SIGNATURES = {
     "mui_hybrid_decode_scratch_bytes": (ctypes.c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "mui_hybrid_attention": (c_int, [_P, c_int, c_int, _P, _P, c_long, _P, c_long, _P, c_long, _P, _P, c_float, c_float, c_int,
                                      c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
+    "mui_hybrid_step_serves": (c_int, [c_int] * 9),
+    "mui_hybrid_step": (c_int, [_P, c_int, _P, c_long, c_long, c_long, _P, _P, c_float, _P, c_int, _P, c_long, _P, _P, _P, c_long, _P, c_long,
+                                c_float, c_float, c_int, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int]),
     "mui_channel_delta_ring_rows": (c_int, [c_int]),
     "mui_channel_delta_max_tokens": (c_int, [c_int, c_int]),
     "mui_channel_delta_workspace_bytes": (ctypes.c_size_t, [c_int, c_int, c_int, c_int, c_int]),

@@ -15,6 +15,8 @@
 // Visible keys are counted compactly: n = 0 .. kf - 1 are the kept first tokens in front of the window, n >= kf
 // continue at the window's start, so kept tokens cost a walk over the window no special case but a shift.
 // Positions: a token's slot in the cache minus its row's first slot (left-padded batches).
+#include <type_traits>
+
 #include "hybrid.cuh"
 
 namespace mui {
@@ -275,6 +277,7 @@ constexpr float kLog2eF = 1.4426950408889634f;
 // ---------------------------------------------------------------------------------------
 constexpr int kHdKeys = 64;
 constexpr int kHdMaxSplits = 64;
+constexpr int kHsStripes = 2;  // of the one-launch step
 
 __device__ __forceinline__ int hybrid_live_splits(const HybridAttnParams& p, const KeyRange& kr) {
   return (kr.n + p.split_keys - 1) / p.split_keys;
@@ -400,6 +403,292 @@ __global__ void __launch_bounds__(256) hybrid_decode_kernel(const HybridAttnPara
   if (wave == 0 && g == 0) {
     p.part_ml[at * 2] = m;
     p.part_ml[at * 2 + 1] = l;
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// step: prepare, decode and merge in one launch for one new token per row and short caches. Grid (kv_heads * groups of 16
+// query heads, rows), two stripes of four waves; stripe s takes key blocks s and s + 2 as a workgroup of the decode kernel does (all of them
+// requested at the start), and the stripes are merged in LDS. Every workgroup takes the sums of squares over the whole of q and k (a few KB that its
+// neighbours have just read), turns its own heads' queries straight into operands and its key and value head's new rows into LDS,
+// from where they replace what the cache held in their slot; it writes them to the cache for later steps.
+// A step is a chain of cold loads here: three launches of 4.5 to 5 us each had one such chain apiece, and the bytes of a few
+// hundred keys are nothing. Where the line lies: launch_hybrid_step.
+// ---------------------------------------------------------------------------------------
+template <typename T, int DKC, int DVT, int ST, bool CAP>
+__global__ void __launch_bounds__(256 * kHsStripes) hybrid_step_kernel(const HybridAttnParams p) {
+  constexpr int NS = kHsStripes, KG = DKC / 2, VG = DVT / 4, NV = DVT / 4, NT = 256 * NS, QP = DKC * 32 + 8;
+  constexpr int KTILE = KG * kHdKeys * 64, VTILE = VG * kHdKeys * 64;
+  __shared__ float mred[NS][4][16], lred[NS][4][16], sums[2][4 * NS];
+  __shared__ __align__(16) uint16_t pl[NS][16][kHdKeys + 8], ql[16][QP], nk[DKC * 32], nv[DVT * 16];
+  __shared__ CosSin cs[DKC * 16];
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4, i16 = lane & 15;
+  const int stripe = wave >> 2, w4 = wave & 3;
+  auto k_tile = [&](int r) { return (uint16_t*)ha_smem + (r * NS + stripe) * (KTILE + VTILE); };  // [KG][64][64]
+  auto v_tile = [&](int r) { return k_tile(r) + KTILE; };                                      // [VG][64][64]
+  const int share = p.heads / p.kv_heads, groups = (share + 15) / 16;
+  const int kvh = blockIdx.x / groups, hg = (blockIdx.x - kvh * groups) * 16, b = blockIdx.y;
+  const int nq = p.heads * p.dim, nkd = p.kv_heads * p.dim, nvd = p.kv_heads * p.vdim;
+  const uint16_t *row = (const uint16_t*)p.proj + (long)b * p.pitch, *kr0 = row + p.k_off, *vr0 = row + p.v_off;
+  const uint16_t *qg = (const uint16_t*)p.q_gain, *kg = (const uint16_t*)p.k_gain;
+  const long slot = p.cache_position[0];
+  const long start = p.row_start ? p.row_start[b] : 0;
+  // requested together: this thread's part of the sums, its head's queries, the new key and value
+  const int c0 = t * 8;
+  const u32x4 sq0 = ld16(row + (c0 < nq ? c0 : 0)), sk0 = ld16(kr0 + (c0 < nkd ? c0 : 0));
+  const int hh = kvh * share + (hg + i16 < share ? hg + i16 : share - 1);  // this lane's head (columns past the share repeat one)
+  // queries: thread t turns chunk t % (dim / 8) of head t / (dim / 8) into LDS (two of them where heads are longer than 128)
+  constexpr int QN = (16 * DKC * 4 + NT - 1) / NT;
+  const int cph = p.dim >> 3;
+  u32x4 qraw[QN], qgain[QN];
+  int qhead[QN], qe[QN];
+#pragma unroll
+  for (int i = 0; i < QN; ++i) {
+    const int c = t + NT * i;
+    qhead[i] = c / cph;
+    qe[i] = (c - qhead[i] * cph) * 8;
+    const int h = kvh * share + (hg + qhead[i] < share ? hg + qhead[i] : share - 1);
+    qraw[i] = ld16(row + (long)h * p.dim + qe[i]);
+    qgain[i] = qg ? ld16(qg + (long)h * p.dim + qe[i]) : qraw[i];
+  }
+  const int ck = t * 8 < p.dim ? t * 8 : 0, cv = (t & 127) * 8 < p.vdim ? (t & 127) * 8 : 0;
+  const u32x4 nkraw = ld16(kr0 + kvh * p.dim + ck), nkgain = kg ? ld16(kg + kvh * p.dim + ck) : nkraw, nvraw = ld16(vr0 + kvh * p.vdim + cv);
+
+  const KeyRange kr = key_range(p, b, slot, slot);
+  const bool stored = slot >= 0 && slot < p.max_cache_len;
+  const int fresh = stored && kr.n > 0 ? kr.n - 1 : 0x7fffffff;  // keys from here on (the last one and its repetitions) are the new one
+  const long kp = nkd, vp = nvd;
+  const uint16_t* kc = (const uint16_t*)p.k_cache + b * p.k_batch + (long)kvh * p.dim;
+  const uint16_t* vc = (const uint16_t*)p.v_cache + b * p.v_batch + (long)kvh * p.vdim;
+  const int lrow = w4 * 8 + (lane >> 3), lc = ((lane & 7) ^ tile_swz(lrow)) * 8;
+  // rows past the last key repeat it (masked), columns past a row's end repeat its start (the queries hold zeros there; such values are never stored)
+  auto request = [&](int r) {
+    const int s0 = (r * NS + stripe) * kHdKeys;
+    uint16_t *kl = k_tile(r), *vl = v_tile(r);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int n = s0 + lrow + 32 * u;
+      const long s = kr.slot(n < kr.n ? n : kr.n - 1);
+#pragma unroll
+      for (int cg = 0; cg < KG; ++cg)
+        load_lds16(kc + s * kp + (cg * 64 + lc < p.dim ? cg * 64 + lc : 0), &kl[(cg * 64 + w4 * 8 + 32 * u) * 64]);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int n = s0 + lrow + 32 * u;
+      const long s = kr.slot(n < kr.n ? n : kr.n - 1);
+#pragma unroll
+      for (int cg = 0; cg < VG; ++cg)
+        load_lds16(vc + s * vp + (cg * 64 + lc < p.vdim ? cg * 64 + lc : 0), &vl[(cg * 64 + w4 * 8 + 32 * u) * 64]);
+    }
+  };
+  const int rounds = (kr.n + NS * kHdKeys - 1) / (NS * kHdKeys);  // uniform for the workgroup
+  if (rounds > 0) {
+#pragma unroll
+    for (int r = 0; r < ST; ++r) request(r);
+  }
+
+  // ---- the new token: sums, angles, queries as operands, key and value rows (the arithmetic of hybrid_prepare_kernel)
+  {
+    const long pos = slot - start;
+    if (t < (p.dim + 1) / 2) {
+      float c = 1.f, s = 0.f;
+      if (2 * t < p.rot) rope_angle((double)(pos > 0 ? pos : 0), p.inv_freq[t], c, s);
+      cs[t] = CosSin{c, s};
+    }
+    auto squares = [&](const uint16_t* x, int n, u32x4 first) {
+      float a = 0.f, f[8];
+      unpack8<T>(first, f);
+      if (c0 < n) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a = fmaf(f[i], f[i], a);
+      }
+      for (int c = c0 + NT * 8; c < n; c += NT * 8) {
+        unpack8<T>(ld16(x + c), f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a = fmaf(f[i], f[i], a);
+      }
+      return wave_sum(a);
+    };
+    const float sq = qg ? squares(row, nq, sq0) : 0.f, sk = kg ? squares(kr0, nkd, sk0) : 0.f;
+    if (lane == 0) {
+      sums[0][wave] = sq;
+      sums[1][wave] = sk;
+    }
+  }
+  __syncthreads();
+  float rq = 1.f, rk = 1.f;
+  if (qg) {
+    float a = 0.f;
+    for (int w = 0; w < 4 * NS; ++w) a += sums[0][w];
+    rq = rsqrtf(a / (float)nq + p.eps);
+  }
+  if (kg) {
+    float a = 0.f;
+    for (int w = 0; w < 4 * NS; ++w) a += sums[1][w];
+    rk = rsqrtf(a / (float)nkd + p.eps);
+  }
+  auto turned = [&](u32x4 x, u32x4 gain, bool gained, float rs, int e0) -> u32x4 {  // eight elements from e0 on of a head, normed, rotated, rounded
+    float f[8], h[8];
+    unpack8<T>(x, f);
+    if (gained) {
+      unpack8<T>(gain, h);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) f[i] = h[i] * (f[i] * rs);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float co = cs[(e0 >> 1) + i].c, si = cs[(e0 >> 1) + i].s, u = f[2 * i], v = f[2 * i + 1];
+      h[2 * i] = u * co - v * si;
+      h[2 * i + 1] = v * co + u * si;
+    }
+    return pack8<T>(h);
+  };
+#pragma unroll
+  for (int i = 0; i < QN; ++i)
+    if (qhead[i] < 16) *(u32x4*)&ql[qhead[i]][qe[i]] = turned(qraw[i], qgain[i], qg != nullptr, rq, qe[i]);
+  if (t * 8 < p.dim) {
+    const u32x4 v = turned(nkraw, nkgain, kg != nullptr, rk, t * 8);
+    *(u32x4*)&nk[t * 8] = v;
+    if (stored && hg == 0) *(u32x4*)((uint16_t*)p.k_cache + b * p.k_batch + slot * kp + (long)kvh * p.dim + t * 8) = v;
+  }
+  if (t >= 128 && (t - 128) * 8 < p.vdim) {
+    *(u32x4*)&nv[(t - 128) * 8] = nvraw;
+    if (stored && hg == 0) *(u32x4*)((uint16_t*)p.v_cache + b * p.v_batch + slot * vp + (long)kvh * p.vdim + (t - 128) * 8) = nvraw;
+  }
+  __syncthreads();
+  u32x4 q[DKC];
+#pragma unroll
+  for (int c = 0; c < DKC; ++c) {
+    const int e = c * 32 + 8 * g;
+    const u32x4 v = *(const u32x4*)&ql[i16][e < p.dim ? e : 0];
+    q[c] = e < p.dim ? v : u32x4{0u, 0u, 0u, 0u};
+  }
+
+  // ---- attention
+  f32x4 acc[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -1e30f, l = 0.f;
+  const float c1 = CAP ? 2.f * p.scale / p.softcap * kLog2eF : p.scale * kLog2eF, c2 = p.softcap * kLog2eF;
+  // what this wave's own loads of the new token's slot brought is replaced once they have landed
+  auto replace = [&](int s0, uint16_t* tile, const uint16_t* fresh_row, int width, auto groups_c) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (s0 + lrow + 32 * u >= fresh) {
+#pragma unroll
+        for (int cg = 0; cg < decltype(groups_c)::value; ++cg)
+          *(u32x4*)&tile[(cg * 64 + w4 * 8 + 32 * u) * 64 + lane * 8] = *(const u32x4*)&fresh_row[cg * 64 + lc < width ? cg * 64 + lc : 0];
+      }
+  };
+  auto round = [&](auto rc) {
+    constexpr int r = decltype(rc)::value;
+    const int s0 = (r * NS + stripe) * kHdKeys;
+    uint16_t *kl = k_tile(r), *vl = v_tile(r);
+    wait_loads<(ST - 1 - r) * 2 * (KG + VG) + 2 * VG>();  // the keys
+    replace(s0, kl, nk, p.dim, std::integral_constant<int, KG>{});
+    __syncthreads();
+    f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < DKC; ++c) s4 = mfma16x16x32<T>(*(const u32x4*)&kl[tile_at<kHdKeys>(16 * w4 + i16, c * 32 + 8 * g)], q[c], s4);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      s4[r4] = s0 + 16 * w4 + 4 * g + r4 < kr.n ? score_log2<CAP>(s4[r4], c1, c2) : -INFINITY;
+      mx = fmaxf(mx, s4[r4]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    if (g == 0) mred[stripe][w4][i16] = mx;
+    __syncthreads();
+    const float mn = fmaxf(m, fmaxf(fmaxf(mred[stripe][0][i16], mred[stripe][1][i16]), fmaxf(mred[stripe][2][i16], mred[stripe][3][i16])));
+    const float keep = exp2f(m - mn);
+    m = mn;
+    float e[4], sum = 0.f;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) { e[r4] = exp2f(s4[r4] - mn); sum += e[r4]; }
+    *(u32x2*)&pl[stripe][i16][16 * w4 + 4 * g] = u32x2{T::pack2(e[0], e[1]), T::pack2(e[2], e[3])};
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (g == 0) lred[stripe][w4][i16] = sum;
+    wait_loads<(ST - 1 - r) * 2 * (KG + VG)>();  // the values
+    replace(s0, vl, nv, p.vdim, std::integral_constant<int, VG>{});
+    __syncthreads();
+    l = l * keep + ((lred[stripe][0][i16] + lred[stripe][1][i16]) + (lred[stripe][2][i16] + lred[stripe][3][i16]));
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) acc[j][r4] *= keep;
+#pragma unroll
+    for (int kk = 0; kk < kHdKeys / 32; ++kk) {
+      const u32x2 plo = *(const u32x2*)&pl[stripe][i16][32 * kk + 4 * g], phi = *(const u32x2*)&pl[stripe][i16][32 * kk + 16 + 4 * g];
+      const u32x4 pb = {plo.x, plo.y, phi.x, phi.y};
+      const int vrow = 32 * kk + 4 * g + (i16 >> 2);
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        const int col = 16 * (w4 + 4 * j) + 4 * (i16 & 3);
+        const u32x2 a0 = lds_read_tr16(&vl[tile_at<kHdKeys>(vrow, col)]), a1 = lds_read_tr16(&vl[tile_at<kHdKeys>(vrow + 16, col)]);
+        acc[j] = mfma16x16x32<T>(u32x4{a0.x, a0.y, a1.x, a1.y}, pb, acc[j]);
+      }
+    }
+  };
+  if (rounds > 0) round(std::integral_constant<int, 0>{});
+  if constexpr (ST > 1) {
+    if (rounds > 1) round(std::integral_constant<int, 1>{});
+  }
+
+  // ---- the stripes' shares, through the tiles
+  f32x4* part = (f32x4*)ha_smem;  // [NS - 1][4 waves][NV][64 lanes]
+  static_assert((size_t)(NS - 1) * 4 * NV * 64 * 16 <= (size_t)NS * (KTILE + VTILE) * 2, "partial sums fit the tiles");
+  __syncthreads();
+  if (stripe > 0) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) part[(((stripe - 1) * 4 + w4) * NV + j) * 64 + lane] = acc[j];
+  }
+  if (w4 == 0 && g == 0) {
+    mred[stripe][0][i16] = m;
+    lred[stripe][0][i16] = l;
+  }
+  __syncthreads();
+  if (stripe > 0 || hg + i16 >= share) return;
+  float all = m;
+#pragma unroll
+  for (int s = 1; s < NS; ++s) all = fmaxf(all, mred[s][0][i16]);
+  const float mine = exp2f(m - all);
+  l *= mine;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) acc[j][r4] *= mine;
+#pragma unroll
+  for (int s = 1; s < NS; ++s) {
+    const float theirs = exp2f(mred[s][0][i16] - all);
+    l = fmaf(theirs, lred[s][0][i16], l);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const f32x4 v = part[(((s - 1) * 4 + w4) * NV + j) * 64 + lane];
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) acc[j][r4] = fmaf(theirs, v[r4], acc[j][r4]);
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const uint16_t* gr = (const uint16_t*)p.gate + b * p.gate_pitch + (long)hh * p.vdim;
+  uint16_t* dst = (uint16_t*)p.out + ((long)b * p.heads + hh) * p.vdim;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int v = 16 * (w4 + 4 * j) + 4 * g;  // (vdim is a multiple of 8)
+    if (v >= p.vdim) continue;
+    float o[4];
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) o[r4] = acc[j][r4] * inv;
+    if (p.gate) {
+      const u32x2 w = ld8(gr + v);
+      o[0] *= sigmoid_f32(T::lo(w.x));
+      o[1] *= sigmoid_f32(T::hi(w.x));
+      o[2] *= sigmoid_f32(T::lo(w.y));
+      o[3] *= sigmoid_f32(T::hi(w.y));
+    }
+    *(u32x2*)(dst + v) = u32x2{T::pack2(o[0], o[1]), T::pack2(o[2], o[3])};
   }
 }
 
@@ -662,6 +951,38 @@ static int launch_hybrid_decode_t(hipStream_t s, const HybridAttnParams& p) {
   return launch_status();
 }
 
+// key blocks per stripe of the one-launch step for caches of which up to `span` rows can be visible, or 0: not for it. Every block has its own LDS tile
+// (32 KB, 64 for heads beyond 128) and is requested at the start: a second round of requests costs a trip to memory, 3 us, which the separate
+// launches' key splits do not have (four stripes of two such rounds: 32 / 8 heads of 128, 512 keys, 1 row 10.2 -> 14.4 us). Two blocks per stripe leave one workgroup per CU,
+// so beyond a workgroup per CU they lose (64 rows of 8 key heads, 256 keys: 25.4 -> 27.3). us for prepare + decode + merge -> here, captured, cold caches,
+// 32 / 8 heads of 128: 1 row of 64 / 128 / 256 keys 10.1 / 9.9 / 9.7 -> 7.2 / 7.1 / 8.5, 16 rows 10.4 / 12.1 / 14.4 -> 7.4 / 7.4 / 9.9, 32 rows 11.6 / 15.4 / 19.0 -> 8.0 / 8.6 /
+// 14.6, 64 rows of 128 keys 17.9 -> 13.2.
+static int hybrid_step_rounds(int batch, int heads, int kv_heads, int dim, int vdim, int span) {
+  const int blocks = ceil_div(span, kHdKeys);
+  const bool small = dim <= 128 && vdim <= 128;
+  const int rounds = ceil_div(blocks, kHsStripes);
+  if (rounds <= 1) return 1;
+  return rounds == 2 && small && (long)batch * kv_heads * ceil_div(heads / kv_heads, 16) <= device_cus() ? 2 : 0;
+}
+
+template <typename T>
+static int launch_hybrid_step(hipStream_t s, const HybridAttnParams& p, int rounds) {
+  const int share = p.heads / p.kv_heads;
+  const dim3 grid(p.kv_heads * ceil_div(share, 16), p.batch), block(256 * kHsStripes);
+  auto launch = [&](auto dkc, auto dvt, auto st) {
+    constexpr int DKC = decltype(dkc)::value, DVT = decltype(dvt)::value, ST = decltype(st)::value;
+    const size_t lds = (size_t)kHsStripes * ST * kHdKeys * (DKC * 32 + DVT * 16) * 2;
+    return p.softcap > 0.f ? launch_with_lds(hybrid_step_kernel<T, DKC, DVT, ST, true>, grid, block, lds, s, p)
+                           : launch_with_lds(hybrid_step_kernel<T, DKC, DVT, ST, false>, grid, block, lds, s, p);
+  };
+  const bool d64 = p.dim <= 64 && p.vdim <= 64, d128 = p.dim <= 128 && p.vdim <= 128;
+  const std::integral_constant<int, 1> c1; const std::integral_constant<int, 2> c2; const std::integral_constant<int, 4> c4;
+  const std::integral_constant<int, 8> c8; const std::integral_constant<int, 16> c16;
+  if (d64) return rounds == 1 ? launch(c2, c4, c1) : launch(c2, c4, c2);
+  if (d128) return rounds == 1 ? launch(c4, c8, c1) : launch(c4, c8, c2);
+  return launch(c8, c16, c1);
+}
+
 template <typename T, int DKC, int DVT>
 static int launch_hybrid_prefill_t(hipStream_t s, const HybridAttnParams& p0) {
   HybridAttnParams p = p0;
@@ -773,4 +1094,41 @@ extern "C" int mui_hybrid_attention(mui_stream_t stream, int dtype, int route, c
   }
   if (dtype == MUI_DTYPE_F16) return launch_hybrid_attention<F16>(s, route, p);
   return launch_hybrid_attention<BF16>(s, route, p);
+}
+
+static int hybrid_span(int window, int keep_first, int max_cache_len) {
+  return window > 0 && window < max_cache_len - keep_first ? window + keep_first : max_cache_len;
+}
+
+extern "C" int mui_hybrid_step_serves(int dtype, int batch, int heads, int kv_heads, int dim, int vdim, int window, int keep_first, int max_cache_len) {
+  if (batch < 1 || batch > 65535 || heads < 1 || kv_heads < 1 || heads % kv_heads || dim < 1 || vdim < 1 || max_cache_len < 1 || window < 0 || keep_first < 0) return 0;
+  if (mui_hybrid_attention_route(dtype, 1, dim, vdim) != MUI_HYBRID_DECODE) return 0;
+  return hybrid_step_rounds(batch, heads, kv_heads, dim, vdim, hybrid_span(window, keep_first, max_cache_len)) > 0;
+}
+
+extern "C" int mui_hybrid_step(mui_stream_t stream, int dtype, const void* proj, long pitch, long k_offset, long v_offset, const void* q_gain,
+                               const void* k_gain, float epsilon, const double* inv_freq, int rot_dims, const void* gate, long gate_pitch,
+                               const int64_t* cache_position, const int64_t* row_start, void* k_cache, long k_batch_stride, void* v_cache,
+                               long v_batch_stride, float scale, float softcap, int window, int keep_first, void* out, int batch, int heads,
+                               int kv_heads, int dim, int vdim, int max_cache_len) {
+  MUI_CHECK_ARG(proj && cache_position && k_cache && v_cache && out && batch > 0 && heads > 0 && kv_heads > 0);
+  MUI_CHECK_ARG(heads % kv_heads == 0 && dim > 0 && vdim > 0 && rot_dims >= 0 && rot_dims <= dim && rot_dims % 2 == 0);
+  MUI_CHECK_ARG((rot_dims == 0 || inv_freq) && max_cache_len > 0 && keep_first >= 0 && window >= 0);
+  MUI_CHECK_ARG(k_offset >= 0 && v_offset >= 0 && pitch >= (long)heads * dim && pitch >= k_offset + (long)kv_heads * dim &&
+                pitch >= v_offset + (long)kv_heads * vdim);
+  MUI_CHECK_ARG(!gate || gate_pitch >= (long)heads * vdim);
+  if (!mui_hybrid_step_serves(dtype, batch, heads, kv_heads, dim, vdim, window, keep_first, max_cache_len)) return MUI_ERR_UNSUPPORTED;
+  const void* ptrs[] = {proj, q_gain, k_gain, k_cache, v_cache, out};
+  for (const void* q : ptrs)
+    if (!aligned16(q)) return MUI_ERR_ALIGNMENT;
+  if (pitch % 8 || k_offset % 8 || v_offset % 8 || k_batch_stride % 8 || v_batch_stride % 8 || (gate && (((uintptr_t)gate & 7) || gate_pitch % 4)))
+    return MUI_ERR_ALIGNMENT;
+  HybridAttnParams p = {};
+  p.proj = proj; p.pitch = pitch; p.k_off = k_offset; p.v_off = v_offset; p.q_gain = q_gain; p.k_gain = k_gain; p.eps = epsilon;
+  p.inv_freq = inv_freq; p.rot = rot_dims; p.cache_position = cache_position; p.row_start = row_start;
+  p.k_cache = k_cache; p.k_batch = k_batch_stride; p.v_cache = v_cache; p.v_batch = v_batch_stride; p.gate = gate; p.gate_pitch = gate_pitch;
+  p.scale = scale; p.softcap = softcap; p.window = window; p.keep = keep_first; p.out = out; p.batch = batch; p.t = 1;
+  p.heads = heads; p.kv_heads = kv_heads; p.dim = dim; p.vdim = vdim; p.max_cache_len = max_cache_len;
+  const int rounds = hybrid_step_rounds(batch, heads, kv_heads, dim, vdim, hybrid_span(window, keep_first, max_cache_len));
+  return dtype == MUI_DTYPE_F16 ? launch_hybrid_step<F16>((hipStream_t)stream, p, rounds) : launch_hybrid_step<BF16>((hipStream_t)stream, p, rounds);
 }

@@ -430,6 +430,39 @@ def hybrid_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     return out
 
 
+def hybrid_step(proj: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int, q_gain: Optional[torch.Tensor],
+                k_gain: Optional[torch.Tensor], eps: float, inv_freq: torch.Tensor, cache_position: torch.Tensor,
+                row_start: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: torch.Tensor, gated: bool, scale: float,
+                softcap: float = 0.0, window: int = 0, keep_first: int = 0) -> Optional[torch.Tensor]:
+    """hybrid_prepare and hybrid_attention of one new token per row in one launch, or None where that is not to be had (then
+    nothing has been done). proj [B, 1, .] starts with q | k | v; gated: the gate follows them."""
+    b, t, pitch = proj.shape
+    lib, nq, nk, nv = _lib.load(), heads * dim, kv_heads * dim, kv_heads * vdim
+    gate_at = nq + nk + nv
+    if t != 1 or not proj.is_cuda or proj.dtype not in _CODES or not proj.is_contiguous() or pitch < gate_at + (heads * vdim if gated else 0):
+        return None
+    if not lib.mui_hybrid_step_serves(_CODES[proj.dtype], b, heads, kv_heads, dim, vdim, window, keep_first, k_cache.shape[1]):
+        return None
+    if pitch % 8 or nq % 8 or (nq + nk) % 8 or gate_at % 4 or k_cache.stride(0) % 8 or v_cache.stride(0) % 8 or \
+            any(x is not None and x.data_ptr() % 16 for x in (proj, q_gain, k_gain, k_cache, v_cache)):
+        return None
+    _operand(q_gain, "q_gain", proj, (nq,))
+    _operand(k_gain, "k_gain", proj, (nk,))
+    _operand(inv_freq, "inv_freq", proj, None, torch.float64)
+    _operand(k_cache, "k_cache", proj, (k_cache.shape[0], k_cache.shape[1], nk))
+    _operand(v_cache, "v_cache", proj, (k_cache.shape[0], k_cache.shape[1], nv))
+    _positions(cache_position, row_start, proj, b, t)
+    if b > k_cache.shape[0]:
+        raise RuntimeError("more batch rows than the cache has")
+    out = torch.empty((b, t, heads * vdim), dtype=proj.dtype, device=proj.device)
+    check(lib.mui_hybrid_step(_stream(proj), _CODES[proj.dtype], proj.data_ptr(), pitch, nq, nq + nk, _ptr(q_gain), _ptr(k_gain), float(eps),
+                              inv_freq.data_ptr(), 2 * inv_freq.numel(), proj.data_ptr() + gate_at * proj.element_size() if gated else None, pitch,
+                              cache_position.data_ptr(), _ptr(row_start), k_cache.data_ptr(), k_cache.stride(0), v_cache.data_ptr(),
+                              v_cache.stride(0), float(scale), float(softcap), window, keep_first, out.data_ptr(), b, heads, kv_heads, dim, vdim,
+                              k_cache.shape[1]), "mui_hybrid_step")
+    return out
+
+
 # --------------------------------------------------------------------------------------
 # gated delta rule
 # --------------------------------------------------------------------------------------

@@ -70,9 +70,12 @@ class MuiHybridAttention(MuiModule):
         """h [B, T, hidden] -> [B, T, hidden]; the tokens' rows go to slots cache_position."""
         c, state = self.config, cache.layers[self.layer_idx]
         proj = self.proj.linear(h)
-        q = hybrid_ops.hybrid_prepare(proj, c.heads, c.kv_heads, c.dim, c.vdim, self.q_norm, self.k_norm, self.eps, self.inv_freq,
-                                      cache_position, cache.row_start, state.k, state.v)
-        gate = proj[..., self.proj.slice_starts[3]:] if c.gated else None
-        o = hybrid_ops.hybrid_attention(q, state.k, state.v, gate, cache_position, cache.row_start, c.heads, c.kv_heads, c.scale,
-                                        c.softcap, c.window, c.keep_first)
+        o = hybrid_ops.hybrid_step(proj, c.heads, c.kv_heads, c.dim, c.vdim, self.q_norm, self.k_norm, self.eps, self.inv_freq, cache_position,
+                                   cache.row_start, state.k, state.v, c.gated, c.scale, c.softcap, c.window, c.keep_first)
+        if o is None:
+            q = hybrid_ops.hybrid_prepare(proj, c.heads, c.kv_heads, c.dim, c.vdim, self.q_norm, self.k_norm, self.eps, self.inv_freq,
+                                          cache_position, cache.row_start, state.k, state.v)
+            gate = proj[..., self.proj.slice_starts[3]:] if c.gated else None
+            o = hybrid_ops.hybrid_attention(q, state.k, state.v, gate, cache_position, cache.row_start, c.heads, c.kv_heads, c.scale,
+                                            c.softcap, c.window, c.keep_first)
         return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)
