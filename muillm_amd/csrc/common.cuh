@@ -91,10 +91,10 @@ __device__ __forceinline__ void unpack8(const u32x4 w, float (&f)[8]) {
 template <typename T>
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
   u32x4 w;
-  w.x = (uint32_t)T::pack(f[0]) | ((uint32_t)T::pack(f[1]) << 16);
-  w.y = (uint32_t)T::pack(f[2]) | ((uint32_t)T::pack(f[3]) << 16);
-  w.z = (uint32_t)T::pack(f[4]) | ((uint32_t)T::pack(f[5]) << 16);
-  w.w = (uint32_t)T::pack(f[6]) | ((uint32_t)T::pack(f[7]) << 16);
+  w.x = T::pack2(f[0], f[1]);
+  w.y = T::pack2(f[2], f[3]);
+  w.z = T::pack2(f[4], f[5]);
+  w.w = T::pack2(f[6], f[7]);
   return w;
 }
 

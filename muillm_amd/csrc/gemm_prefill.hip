@@ -61,6 +61,11 @@ template <int ROWS, int TOKS, int KS, int NBUF>
 constexpr size_t pipe_lds_bytes() {  // (no fused norm in this loop: no per-token sums behind the stages)
   return (size_t)(NBUF * ROWS + pipe_x_stages<ROWS, TOKS, KS, NBUF>() * TOKS) * KS * 2;
 }
+// with 8-bit weights: stages of codes, of token rows and, in the group format, of the rows' (scale, min) pairs
+template <int WF, int ROWS, int TOKS, int KS, int NBUF>
+constexpr size_t pipe8_lds_bytes() {
+  return (size_t)NBUF * (ROWS * KS + TOKS * KS * 2 + (WF == WF_U8_GROUP ? ROWS * 4 : 0));
+}
 
 // partial tiles between workgroups: agent-scope relaxed atomics (write-through stores, loads that
 // bypass the non-coherent caches; the XCDs do not share an L2)
@@ -101,6 +106,10 @@ __device__ __forceinline__ f32x4 xs_load(const float* src) {
 // which is what a microsecond figure on this part reflects: the board's power limit sets the clock
 // under this load, and operand bytes read from LDS per matrix instruction are what the eight waves
 // save over sixteen (192 instead of 256 KB per k-step).
+// PIPE with 8-bit weights: the same loop over stages of codes. A wave reads a row's eight codes of a half step in place of
+// sixteen bytes and turns them into the operand while the matrix pipes work on the row before (packed
+// arithmetic for fp16: ten vector instructions per eight matrix instructions; the products and their order are those of the
+// kernels that convert on the way to LDS). Half the weight bytes leave room for three stages of everything.
 template <typename T, int WF, bool NORM, int EPI, int WR, int WT, int NWR, int NWT, int NWK, int KS, int NBUF,
           bool XS = false, bool DMA = false, bool PIPE = false>
 // one tile: the work of workgroup id `vb` of a grid of one workgroup per tile
@@ -134,12 +143,15 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   static_assert((XEXACT || XCHUNKS % 64 == 0) && (WEXACT || WCHUNKS % 64 == 0), "whole waves stage the last round of chunks");
   // NBUF == 2: step s + 1 is written to the other LDS stage while step s is multiplied, one
   // barrier per step instead of two
-  typedef uint16_t WStage[ROWS * PITCH];
+  constexpr bool W8 = PIPE && WF != WF_16BIT;  // codes in the stages
+  constexpr int WPITCH = W8 ? PITCH / 2 : PITCH;
+  typedef uint16_t WStage[ROWS * WPITCH];
   typedef uint16_t XStage[TOKS * PITCH];
   WStage* w_lds = (WStage*)pf_smem;
-  constexpr int XB = PIPE ? pipe_x_stages<ROWS, TOKS, KS, NBUF>() : NBUF;  // stages of the token tile
+  constexpr int XB = PIPE && !W8 ? pipe_x_stages<ROWS, TOKS, KS, NBUF>() : NBUF;  // stages of the token tile
   XStage* x_lds = (XStage*)(pf_smem + (size_t)NBUF * sizeof(WStage));
   float* rs_lds = (float*)(pf_smem + (size_t)NBUF * sizeof(WStage) + (size_t)XB * sizeof(XStage));  // (NORM only)
+  uint32_t* pr_lds = (uint32_t*)rs_lds;  // [NBUF][ROWS] (scale, min) pairs (pipelined loop over codes of the group format only)
 
   const int t = threadIdx.x;
   const int lane = t & (kWave - 1);
@@ -229,23 +241,27 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   // DMA: per wave instruction q the source of this lane's slot (fixed but for the k-step's offset)
   constexpr int kNWaves = kPfThreads / 64;
   constexpr int DRI = 64 / CPR;  // tile rows per load instruction (8 with k-steps of 64, 4 with 128, 2 with 256)
-  constexpr int WQ = DMA ? ROWS / (DRI * kNWaves) : 1, XQ = DMA ? TOKS / (DRI * kNWaves) : 1;
+  constexpr int DRW = W8 ? 1024 / KS : DRI;  // weight rows per load instruction
+  // (codes: where the waves do not divide the blocks, the last ones load their first block once more)
+  constexpr int WBLOCKS = ROWS / DRW;
+  constexpr int WQ = DMA ? (WBLOCKS + (W8 ? kNWaves - 1 : 0)) / kNWaves : 1, XQ = DMA ? TOKS / (DRI * kNWaves) : 1;
   // per wave instruction q: a base address that is the same for the wave's lanes (the matrix, or the
   // up matrix for the instructions that cover up rows: eight consecutive tile rows never straddle
   // the two) and this lane's 32-bit byte offset from it; only the base moves with the k-step
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   unsigned dma_wo[WQ], dma_xo[XQ];
+  auto w_block = [&](int q, int w) { return !W8 || q * kNWaves + w < WBLOCKS ? q * kNWaves + w : w; };
   if constexpr (DMA) {
-    static_assert(!DMA || (WF == WF_16BIT && !NORM && NBUF >= 2 && !XS && CPR >= 8 && CPR <= 64), "what the DMA path covers");
-    static_assert(!DMA || (WQ >= 1 && XQ >= 1 && WQ * DRI * kNWaves == ROWS && XQ * DRI * kNWaves == TOKS), "whole 1 KB blocks per wave");
-    static_assert(!DMA || EPI != SK_GATEUP || (8 * WR) % DRI == 0, "gate and up rows change at multiples of a block's rows");
+    static_assert(!DMA || ((WF == WF_16BIT || W8) && !NORM && NBUF >= 2 && !XS && CPR >= 8 && CPR <= 64), "what the DMA path covers");
+    static_assert(!DMA || (WQ >= 1 && XQ >= 1 && (W8 || WQ * DRW * kNWaves == ROWS) && XQ * DRI * kNWaves == TOKS), "whole 1 KB blocks per wave");
+    static_assert(!DMA || EPI != SK_GATEUP || (8 * WR) % DRW == 0, "gate and up rows change at multiples of a block's rows");
     const int sr = lane / CPR, sc = lane % CPR;
 #pragma unroll
     for (int q = 0; q < WQ; ++q) {
-      const int r = (q * kNWaves + wave) * DRI + sr;
+      const int r = w_block(q, wave) * DRW + (W8 ? lane >> 2 : sr);
       bool up;
       const int o = weight_row(r, up);
-      dma_wo[q] = (unsigned)((long)o * p.pitch + ((sc ^ swz(r)) * 16));
+      dma_wo[q] = (unsigned)((long)o * p.pitch + (W8 ? (lane & 3) ^ ((r >> 2) & 3) : sc ^ swz(r)) * 16);
     }
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
@@ -257,18 +273,18 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   }
   // load instruction i of a k-step: the weight blocks first, then the token blocks
   auto dma_one = [&](int step, int buf, int i) {
-    const long kb = (long)step * KS * 2;
+    const long kb = (long)step * KS * 2, kbw = W8 ? kb / 2 : kb;
     // (the lane offset is made opaque to the optimiser: widened to 64 bits outside the loop it would
     // cost a register pair and a 64-bit add per load instead of the scalar-base addressing mode)
     if (i < WQ) {
       const int q = i;
       bool up;
-      weight_row((q * kNWaves + wave_u) * DRI, up);
-      const uint8_t* base = ((EPI == SK_GATEUP && up) ? p.w1 : p.w0) + kb;
+      weight_row(w_block(q, wave_u) * DRW, up);
+      const uint8_t* base = ((EPI == SK_GATEUP && up) ? p.w1 : p.w0) + kbw;
       unsigned off = dma_wo[q];
       asm volatile("" : "+v"(off));
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + off),
-                                       (__attribute__((address_space(3))) void*)&w_lds[buf][(q * kNWaves + wave_u) * DRI * PITCH],
+                                       (__attribute__((address_space(3))) void*)&w_lds[buf][w_block(q, wave_u) * DRW * WPITCH],
                                        16, 0, 0);
     } else {
       const int q = i - WQ;
@@ -388,7 +404,116 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   const int sb = XS ? (int)((long)n_steps * xs_share / p.k_splits) : 0;
   const int se = XS ? (int)((long)n_steps * (xs_share + 1) / p.k_splits) : n_steps;
   Stage r0;
-  if constexpr (DMA && PIPE) {
+  if constexpr (DMA && W8) {
+    static_assert(!W8 || (KS == 64 && NWK == 1 && NBUF == 3), "two halves per k-step, three stages of everything");
+    constexpr bool PAIRS = WF == WF_U8_GROUP;
+    constexpr int PQ = PAIRS ? 1 : 0, NL = WQ + XQ + PQ;
+    static_assert(!W8 || 2 * NL <= 63, "the waits' load counts");
+    static_assert(!PAIRS || (ROWS % 64 == 0 && ROWS <= 64 * kNWaves), "a wave loads the pairs of 64 rows");
+    // pairs of a k-step: wave w has rows 64 (w % (ROWS / 64)) .. + 63 (where there are more waves than that, the same ones again)
+    const uint16_t* pair_at = nullptr;
+    const int pair_row = (wave_u % (ROWS / 64)) * 64;
+    if constexpr (PAIRS) {
+      bool up;
+      const int o = weight_row(pair_row + lane, up);
+      pair_at = (up ? p.s1 : p.s0) + (long)o * p.s_pitch;
+    }
+    auto load_one = [&](int step, int buf, int i) {
+      if (i < WQ + XQ) {
+        dma_one(step, buf, i);
+      } else {
+        const uint16_t* src = pair_at + 2 * ((step * KS) >> p.group_shift);
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)&pr_lds[buf * ROWS + pair_row], 4, 0, 0);
+      }
+    };
+    u32x2 a[2][WR];
+    u32x4 b[2][WT], cv[2];
+    uint32_t pr[PAIRS ? WR : 1], pr_next[PAIRS ? WR : 1];
+    // (a row's stage is four 16-byte chunks, chunk c in slot c ^ ((row >> 2) & 3): the sixteen rows of an operand fall into different banks)
+    const int ac = (lane & 12) >> 2, a8 = (wr * 16 * WR + (lane & 15)) * WPITCH + (lg & 1) * 4;
+    // reads of a half step: the codes first, they are converted ahead of use; then the token operands, then the pairs (of both halves)
+    auto read_one = [&](int buf, int kk, int i) {
+      if (i < WR) a[kk][i] = *(const u32x2*)&w_lds[buf][a8 + i * 16 * WPITCH + (((kk * 2 + (lg >> 1)) ^ ac) * 8)];
+      else if (i < WR + WT) b[kk][i - WR] = *(const u32x4*)&x_lds[buf][b_base + (i - WR) * 16 * PITCH + (((kk * 4 + lg) ^ lsw) * 8)];
+      else pr_next[i - WR - WT] = pr_lds[buf * ROWS + wr * 16 * WR + 16 * (i - WR - WT) + (lane & 15)];
+    };
+    auto operand = [&](int kk, int i, uint32_t pair) -> u32x4 {
+      if constexpr (PAIRS) return convert_a_pair_f16(a[kk][i].x, a[kk][i].y, pair);
+      else return convert_a<T, WF_I8_CHANNEL>(a[kk][i].x, a[kk][i].y, nullptr, 0, 0);
+    };
+    constexpr auto vm = [](int n) { return (n & 15) | ((n >> 4) << 14); };
+#pragma unroll
+    for (int st = 0; st < NBUF; ++st)
+#pragma unroll
+      for (int i = 0; i < NL; ++i) load_one(sb + st < se ? sb + st : se - 1, st, i);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | vm((NBUF - 1) * NL));  // the first step's loads
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < WR + WT + (PAIRS ? WR : 0); ++i) read_one(0, 0, i);
+    cv[0] = operand(0, 0, pr_next[0]);
+    int buf = 0;
+    for (int s = sb; s < se; ++s) {
+      if constexpr (PAIRS) {
+#pragma unroll
+        for (int i = 0; i < WR; ++i) pr[i] = pr_next[i];
+      }
+      const int nbuf = buf + 1 == NBUF ? 0 : buf + 1;
+      const int nxt = s + NBUF < se ? s + NBUF : se - 1;
+      // row i of half kk: its matrix instructions, its share of the next half's reads (and, in the second half, of a later step's loads),
+      // the conversion of the row behind it
+      auto region = [&](auto kc, auto ic) {
+        constexpr int kk = decltype(kc)::value, i = decltype(ic)::value;
+        constexpr int NR = WR + WT + (PAIRS && kk == 1 ? WR : 0), nloads = kk == 1 ? NL : 0;
+        // everything in all but the last row: the half behind it starts with them
+        constexpr int RD = (NR + WR - 2) / (WR - 1), LD = (nloads + WR - 2) / (WR - 1);
+        constexpr int r0_ = i * RD < NR ? i * RD : NR, r1_ = (i + 1) * RD < NR ? (i + 1) * RD : NR;
+        constexpr int l0_ = i * LD < nloads ? i * LD : nloads, l1_ = (i + 1) * LD < nloads ? (i + 1) * LD : nloads;
+        constexpr int nr = r1_ - r0_, nl = l1_ - l0_;
+#pragma unroll
+        for (int l = l0_; l < l1_; ++l) load_one(nxt, buf, l);
+#pragma unroll
+        for (int r = r0_; r < r1_; ++r) read_one(kk == 0 ? buf : nbuf, 1 - kk, r);
+#pragma unroll
+        for (int j = 0; j < WT; ++j) acc[i][j] = mfma16x16x32<T>(cv[(kk * WR + i) & 1], b[kk][j], acc[i][j]);
+        if constexpr (i + 1 < WR) cv[(kk * WR + i + 1) & 1] = operand(kk, i + 1, pr[PAIRS ? i + 1 : 0]);
+        else cv[(kk * WR + i + 1) & 1] = operand(1 - kk, 0, kk == 0 ? pr[0] : pr_next[0]);
+        // a matrix instruction, its share of the loads and reads, its share of the conversion
+        constexpr int kConvert = PAIRS ? 14 : (T::kDtype == MUI_DTYPE_F16 ? 10 : 12);
+        auto slot = [&](auto jc) {
+          constexpr int j = decltype(jc)::value;
+          if constexpr (j < WT) {
+            constexpr int loads = nl * (j + 1) / WT - nl * j / WT, reads = nr * (j + 1) / WT - nr * j / WT;
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if constexpr (loads > 0) __builtin_amdgcn_sched_group_barrier(0x010, loads, 0);
+            if constexpr (reads > 0) __builtin_amdgcn_sched_group_barrier(0x100, reads, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, (kConvert + WT - 1) / WT, 0);
+          }
+        };
+        slot(std::integral_constant<int, 0>{});
+        slot(std::integral_constant<int, 1>{});
+        slot(std::integral_constant<int, 2>{});
+        slot(std::integral_constant<int, 3>{});
+        slot(std::integral_constant<int, 4>{});
+        slot(std::integral_constant<int, 5>{});
+        slot(std::integral_constant<int, 6>{});
+        slot(std::integral_constant<int, 7>{});
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto half = [&](auto kc) {
+        region(kc, std::integral_constant<int, 0>{});
+        region(kc, std::integral_constant<int, 1>{});
+        if constexpr (WR > 2) region(kc, std::integral_constant<int, 2>{});
+        if constexpr (WR > 3) region(kc, std::integral_constant<int, 3>{});
+      };
+      half(std::integral_constant<int, 0>{});
+      // this wave's reads of the stage have returned, its share of the next one has landed (all loads but those of the step after it)
+      __builtin_amdgcn_s_waitcnt(0x0070 | vm((NBUF - 2) * NL));
+      __syncthreads();
+      half(std::integral_constant<int, 1>{});
+      buf = nbuf;
+    }
+  } else if constexpr (DMA && PIPE) {
     // Two operand register sets per wave: the LDS reads of one half of a k-step are issued while the
     // other half is multiplied, one read per two matrix instructions, so a wave always has sixteen
     // or more matrix instructions to issue that wait for nothing; the barrier sits between the two
@@ -764,6 +889,10 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
               const int oe = ow0 + 16 * i + 4 * ag + e;
               if constexpr (EPI == SK_GATEUP) {
                 float g = acc[i][j][e], u = acc[i + OT][j][e];
+                if constexpr (WF == WF_I8_CHANNEL) {
+                  g *= T::one(p.s0[(long)oe * p.s_pitch]);
+                  u *= T::one(p.s1[(long)oe * p.s_pitch]);
+                }
                 if (p.add_bias) {
                   g += T::one(p.add_bias[oe]);
                   u += T::one(p.mul_bias[oe]);
@@ -771,6 +900,7 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
                 v[e] = gateup_f32(g, u);
               } else {
                 float r = acc[i][j][e];
+                if constexpr (WF == WF_I8_CHANNEL) r *= T::one(p.s0[(long)oe * p.s_pitch]);
                 if (p.mul_bias) r *= T::one(p.mul_bias[oe]);
                 if (p.add_bias) r += T::one(p.add_bias[oe]);
                 if (p.residual) r += res4[e];
@@ -913,13 +1043,19 @@ static int g_prefill_persistent = 1;  // experiments: 0 launches one workgroup p
 static int g_prefill_stages3_big = 1;  // experiments: 0 keeps the pipelined 192 x 256 and 256 x 256 tiles on two stages of both tiles
 static int g_prefill_stages3 = 1;     // experiments: 0 keeps the pipelined 128 x 256 tile on two LDS stages
 
+// Weights that the software-pipelined loop takes. bf16 in the group format needs a float multiply-add and two conversions per code: more vector than
+// matrix time (gate/up at 800 tokens 264 us, 240 with the conversion on the way to LDS), so it keeps the older kernels.
+template <typename T, int WF>
+constexpr bool kPipelined = WF != WF_U8_GROUP || T::kDtype == MUI_DTYPE_F16;
+
 // what the LDS-direct loads need: whole k-steps, 16-byte aligned rows, 32-bit byte offsets from
 // the operands' bases
-static bool lds_direct_loads_serve(const PrefillGemmParams& p, int k_step = 64) {
-  return g_prefill_dma && p.k % k_step == 0 && p.pitch % 16 == 0 && (long)p.n * p.pitch < (1L << 32) &&
-         (long)p.tokens * p.k * 2 < (1L << 32);
+// (codes of the group format: a k-step of 64 lies in one group)
+static bool lds_direct_loads_serve(const PrefillGemmParams& p, int wf) {
+  return g_prefill_dma && p.k % 64 == 0 && p.pitch % 16 == 0 && (long)p.n * p.pitch < (1L << 32) &&
+         (long)p.tokens * p.k * 2 < (1L << 32) && (wf != WF_U8_GROUP || p.group_shift >= 6);
 }
-static bool pipelined_loop_serves(const PrefillGemmParams& p) { return lds_direct_loads_serve(p); }
+static bool pipelined_loop_serves(const PrefillGemmParams& p, int wf) { return lds_direct_loads_serve(p, wf); }
 
 template <typename T, int WF, int EPI, int WR, int WT, int NWR, int NWT, int NWK, int KS, int NBUF, bool PIPE = false>
 static int launch_prefill_cfg(hipStream_t s, PrefillGemmParams p) {
@@ -943,7 +1079,8 @@ static int launch_prefill_cfg(hipStream_t s, PrefillGemmParams p) {
   // every XCD gets the same number of slots: its share rounded up, the surplus exits
   const long grid = (long)ceil_div(p.n_tiles, p.row_split) * ceil_div(p.t_tiles, 8 / p.row_split) * 8;
   if (grid > 0x7fffffffL) return MUI_ERR_UNSUPPORTED;
-  constexpr size_t lds = PIPE ? pipe_lds_bytes<ROWS, TOKS, KS, NBUF>() : prefill_lds_bytes<ROWS, TOKS, KS, NBUF>();
+  constexpr size_t lds = PIPE && WF != WF_16BIT ? pipe8_lds_bytes<WF, ROWS, TOKS, KS, NBUF>()
+                         : PIPE ? pipe_lds_bytes<ROWS, TOKS, KS, NBUF>() : prefill_lds_bytes<ROWS, TOKS, KS, NBUF>();
   static_assert(lds <= kLdsPerWorkgroup, "LDS of a workgroup");
   auto launch = [&](auto kernel) {
     if constexpr (lds > 65536) {
@@ -971,14 +1108,14 @@ static int launch_prefill_cfg(hipStream_t s, PrefillGemmParams p) {
     if (p.gamma) return launch(prefill_gemm_kernel<T, WF, true, EPI, WR, WT, NWR, NWT, NWK, KS, NBUF>);
   }
   constexpr int kWaves8 = 8 * NWR * NWT * NWK;
-  if constexpr (WF == WF_16BIT && (NBUF == 2 || (PIPE && NBUF == 3)) && NWK == 1 && KS == 64 && ROWS % kWaves8 == 0 &&
+  if constexpr ((WF == WF_16BIT || (PIPE && kPipelined<T, WF>)) && (NBUF == 2 || (PIPE && NBUF == 3)) && NWK == 1 && KS == 64 && ROWS % kWaves8 == 0 &&
                 TOKS % kWaves8 == 0 && (PIPE || ROWS * TOKS >= 256 * 256)) {
     // LDS-direct operand loads: always with the software-pipelined loop; with the sixteen-wave loop
     // on the 256 x 256 tile only, where a k-step (2048 matrix-pipe cycles per SIMD) covers an L2
     // round trip (gate/up at 4096 tokens 834 -> 800 us, down 410 -> 390 us, o_proj 136 -> 123 us);
     // with that loop on 128 x 256, half of that, they lose (down at 2048 tokens 264 -> 293 us,
     // o_proj 77 -> 88 us, gate/up at 256 88 -> 99 us).
-    if (lds_direct_loads_serve(p))
+    if (lds_direct_loads_serve(p, WF))
       return launch(prefill_gemm_kernel<T, WF, false, EPI, WR, WT, NWR, NWT, NWK, KS, NBUF, false, true, PIPE>);
   }
   if constexpr (PIPE) return MUI_ERR_UNSUPPORTED;  // the caller falls back to the sixteen-wave tile
@@ -1089,20 +1226,23 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
         return (float)full * twin + last;
       };
       // (the three big tiles cost less per round where the software-pipelined loop serves them)
-      const bool pipe = WF == WF_16BIT && !p.gamma && pipelined_loop_serves(p);
-      float best = whole(tiles(256, 256), pipe ? 96.f : 100.f, pipe ? 100.f : 111.f);
+      const bool pipe = kPipelined<T, WF> && !p.gamma && pipelined_loop_serves(p, WF);
+      const bool pipe8 = pipe && WF != WF_16BIT;  // (the conversion costs the loop a tenth)
+      float best = whole(tiles(256, 256), pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f);
       which = 4;
       // (gate/up in two launches, see below: whole rounds of 256 x 256 and one round of 128 x 256)
-      if constexpr (WF == WF_16BIT && EPI == SK_GATEUP) {
-        if (pipe && gateup_bands(p) > 0) best = (float)((tiles(256, 256) + cus - 1) / cus - 1) * 100.f + 53.f;
+      if constexpr (EPI == SK_GATEUP) {
+        if (pipe && gateup_bands(p) > 0) best = (float)((tiles(256, 256) + cus - 1) / cus - 1) * (pipe8 ? 109.f : 100.f) + (pipe8 ? 60.f : 53.f);
       }
       auto offer = [&](int id, float cost) {
         if (cost < best * 0.97f) { best = cost; which = id; }  // bigger tiles win ties
       };
-      if (pipe && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 74.f, 80.f));
+      if (pipe8 && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 81.f, 87.f));
+      else if (pipe && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 74.f, 80.f));
       else if (pipe) offer(8, whole(tiles(192, 256), 92.f, 98.f));  // gate/up: twelve waves beside pipelined 256 x 256 and 128 x 256
       else offer(8, whole(tiles(192, 256), 85.f, 92.f));
-      if (pipe) offer(7, whole(tiles(128, 256), 53.f, 58.f));  // (three LDS stages; 63 / 66 with two)
+      if (pipe8) offer(7, whole(tiles(128, 256), 60.f, 64.f));
+      else if (pipe) offer(7, whole(tiles(128, 256), 53.f, 58.f));  // (three LDS stages; 63 / 66 with two)
       else offer(7, whole(tiles(128, 256), WF == WF_16BIT ? 67.f : 73.f, WF == WF_16BIT ? 70.f : 76.f));
       offer(1, pairs(tiles(128, 128), 68.f, 92.f));
       if (EPI == SK_LINEAR && WF == WF_16BIT) offer(10, pairs(tiles(96, 128), 60.f, 76.f));
@@ -1128,12 +1268,24 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
   // 4096 881 -> 854 us; 128 x 256: 75 -> 68 us per round; 128 x 128 splitting K: 46 -> 42 us).
   // int8 rows hold a quarter of the 16-byte chunks per k-step: where sixteen waves would leave
   // threads without a chunk to stage, the int8 kernels keep eight.
-  if constexpr (WF == WF_16BIT && EPI == SK_GATEUP) {
+  auto pipe_256 = [&](const PrefillGemmParams& q) {
+    if constexpr (WF == WF_16BIT) {
+      if (!g_prefill_stages3_big) return launch_prefill_cfg<T, WF, EPI, 4, 8, 4, 2, 1, 64, 2, true>(s, q);
+    }
+    return launch_prefill_cfg<T, WF, EPI, 4, 8, 4, 2, 1, 64, 3, true>(s, q);
+  };
+  auto pipe_128 = [&](const PrefillGemmParams& q) {
+    if constexpr (WF == WF_16BIT) {
+      if (!g_prefill_stages3) return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 2, true>(s, q);
+    }
+    return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 3, true>(s, q);
+  };
+  if constexpr (EPI == SK_GATEUP) {
     // Gate/up whose 256 x 256 tiles end in a round that is at most half full (2048 tokens: 896 tiles
     // = 3.5 rounds of 256 CUs): the outputs of the whole rounds in one launch, the rest as one round
     // of 128 x 256 tiles in a second one (a half-empty round of the big tile costs as much as a full
     // one, a round of the small tile two thirds of it).
-    if (g_prefill_tile == 0 && which == 4 && !p.gamma && pipelined_loop_serves(p)) {
+    if (g_prefill_tile == 0 && which == 4 && !p.gamma && pipelined_loop_serves(p, WF)) {
       {
         const long whole_rows = gateup_bands(p);
         if (whole_rows > 0) {
@@ -1147,37 +1299,41 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
             b.add_bias += a.n;
             b.mul_bias += a.n;
           }
-          int st = g_prefill_stages3_big ? launch_prefill_cfg<T, WF, EPI, 4, 8, 4, 2, 1, 64, 3, true>(s, a)
-                                         : launch_prefill_cfg<T, WF, EPI, 4, 8, 4, 2, 1, 64, 2, true>(s, a);
-          if (st == MUI_OK) st = g_prefill_stages3 ? launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 3, true>(s, b)
-                                                  : launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 2, true>(s, b);
+          if (WF != WF_16BIT) {
+            b.s0 += (long)a.n * p.s_pitch;
+            b.s1 += (long)a.n * p.s_pitch;
+          }
+          int st = pipe_256(a);
+          if (st == MUI_OK) st = pipe_128(b);
           if (st != MUI_ERR_UNSUPPORTED) return st;
         }
       }
     }
   }
-  if constexpr (WF == WF_16BIT) {
+  {
     // 256 x 256 on 4 x 2 waves of 64 x 128 with two operand register sets (the software-pipelined
     // loop): where its loads can go straight into LDS it is 5-8 % ahead of the sixteen waves below
     // (gate/up at 4096 tokens 775 -> 736 us, down 386 -> 356 us, QKV 224 -> 209 us, down at 2048
     // tokens 345 -> 315 us; bit-equal results: the same products in the same order)
     if (which == 4 && !p.gamma) {
-      const int st = g_prefill_stages3_big ? launch_prefill_cfg<T, WF, EPI, 4, 8, 4, 2, 1, 64, 3, true>(s, p)
-                                           : launch_prefill_cfg<T, WF, EPI, 4, 8, 4, 2, 1, 64, 2, true>(s, p);
+      const int st = pipe_256(p);
       if (st != MUI_ERR_UNSUPPORTED) return st;
     }
   }
   if (which == 13) which = 4;  // the sixteen-wave kernel on request
-  if constexpr (WF == WF_16BIT) {
+  {
     if (g_prefill_pipe_small && !p.gamma) {
       int st = MUI_ERR_UNSUPPORTED;
       // 128 x 256, 2 x 4 waves of 64 x 64, three LDS stages
-      if (which == 7) st = g_prefill_stages3 ? launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 3, true>(s, p)
-                                             : launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 2, true>(s, p);
+      if (which == 7) st = pipe_128(p);
       if constexpr (EPI == SK_LINEAR) {
         // 192 x 256, 4 x 2 waves of 48 x 128
-        if (which == 8) st = g_prefill_stages3_big ? launch_prefill_cfg<T, WF, EPI, 3, 8, 4, 2, 1, 64, 3, true>(s, p)
-                                                   : launch_prefill_cfg<T, WF, EPI, 3, 8, 4, 2, 1, 64, 2, true>(s, p);
+        if (which == 8) {
+          if constexpr (WF == WF_16BIT) {
+            if (!g_prefill_stages3_big) return launch_prefill_cfg<T, WF, EPI, 3, 8, 4, 2, 1, 64, 2, true>(s, p);
+          }
+          st = launch_prefill_cfg<T, WF, EPI, 3, 8, 4, 2, 1, 64, 3, true>(s, p);
+        }
       }
       if (st != MUI_ERR_UNSUPPORTED) return st;
     }

@@ -177,6 +177,23 @@ __device__ __forceinline__ u32x4 convert_a_pair(uint32_t w0, uint32_t w1, uint32
   return pack8<T>(f);
 }
 
+// the same for fp16 in packed arithmetic: 1024 + u8 by byte permutes, 1024 off again (exact), one fused multiply-add whose
+// single rounding is the one to fp16
+__device__ __forceinline__ u32x4 convert_a_pair_f16(uint32_t w0, uint32_t w1, uint32_t pair) {
+  const uint32_t v[2] = {w0, w1};
+  const f16x2 pr = __builtin_bit_cast(f16x2, pair), sc = {pr.x, pr.x}, mn = {pr.y, pr.y};
+  const f16x2 off = {(_Float16)1024.f, (_Float16)1024.f};
+  uint32_t o[4];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, v[m], 0x04010400u);
+    const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, v[m], 0x04030402u);
+    o[2 * m + 0] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, lo) - off, sc, mn));
+    o[2 * m + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, hi) - off, sc, mn));
+  }
+  return u32x4{o[0], o[1], o[2], o[3]};
+}
+
 // tiled matrix-core GEMM for prompts (gemm_prefill.hip): any token count, 16-bit weights or int8 codes of either format
 int launch_prefill_gemm(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
 size_t prefill_workspace_bytes();  // what SkinnyParams::workspace must hold for the prompt GEMM to use it

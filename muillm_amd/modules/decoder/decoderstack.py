@@ -377,8 +377,10 @@ class MuiPromptStack(MuiDecoderStack):
         self._cache_layers = [attn.layer_idx for attn in self._attentions]
         self._layer_list = self._attentions = self._cache_ptrs = None  # (nothing is held but weakly)
         self._bound(cache)
-        int8 = any(x.qkv_scales or x.o_scales or x.gate_scales or x.down_scales for x in self._layers)
-        self._most_rows = min(muillm_ext.INT8_DEQUANT_MIN_TOKENS, muillm_ext.INT8_GROUP_DEQUANT_MIN_TOKENS) - 1 if int8 else 1 << 30
+        # (the library's call converts codes, the modules dequantise long prompts' matrices)
+        ks = (self.hidden, self.hq * self.d, layers[0].mlp.intermediate_size)
+        shifts = {x.int8_group_size_shift for x in self._layers if x.qkv_scales or x.o_scales or x.gate_scales or x.down_scales}
+        self._most_rows = min([muillm_ext.int8_dequantised_from(self.dtype, k, shift) - 1 for k in ks for shift in shifts], default=1 << 30)
 
     def _built_from(self, owners, cache_tensors) -> None:
         pass  # see remember()

@@ -463,22 +463,30 @@ def _byte_pitch(w: torch.Tensor, name: str) -> int:
 
 
 # int8 weights: the decode kernels take chunks of MUI_MAX_TOKENS up to this many tokens; beyond, the
-# tiled matrix-core GEMM converts the codes on their way to LDS (per-channel format: no chunking,
+# tiled matrix-core GEMM converts the codes itself (per-channel format: no chunking,
 # 64 tokens of an 8B-shaped prefill take 5.6 ms on the GEMM against 8.9 ms in four chunks; group
-# format: 17..32 tokens 6.4 ms on the GEMM against 7.1 ms in two chunks); long prompts run on the
-# matrix dequantised by the library's kernel (about 4 ms per 8B-shaped pass).
+# format: 17..32 tokens 6.4 ms on the GEMM against 7.1 ms in two chunks).
 INT8_CHUNK_MAX_TOKENS = MUI_MAX_TOKENS
 INT8_GROUP_CHUNK_MAX_TOKENS = MUI_MAX_TOKENS
-# Per-channel format from this many tokens: the matrix is dequantised once per call (12–32 µs per
-# Llama-3-8B matrix) and the GEMM runs its software-pipelined loop on 16-bit weights, which the
-# converting loop cannot use (at 4096 tokens QKV 227 -> 182 µs, o_proj 128 -> 118, down 389 -> 381,
-# gate/up 817 -> 762; an 8B-shaped prefill 27.5 -> 25.8 ms at 1536 tokens, while at 1024 tokens the
-# conversion on the way to LDS is still ahead, 17.7 against 19.5 ms).
-INT8_DEQUANT_MIN_TOKENS = 1280
-# The group format likewise, from 1024 tokens; 33 .. 1023 tokens go to the GEMM that applies (scale, min)
-# on the way to LDS (an 8B-shaped prefill of 64 tokens 9.4 -> 6.1 ms, 512 tokens 14.3 -> 12.1 ms, level at
-# 1024, 35.0 against 29.9 ms at 2048).
-INT8_GROUP_DEQUANT_MIN_TOKENS = 1024
+# From this many tokens the matrix is dequantised once per call (12-32 us per Llama-3-8B matrix) and the GEMM runs on 16-bit weights. The
+# software-pipelined loop takes codes itself, a tenth slower per tile for the conversion, so only very long prompts gain: QKV + o_proj + gate/up + down of an
+# 8B-shaped layer, codes / dequantised: per-channel fp16 at 1536 / 4096 / 8192 tokens 606 / 1357 / 2672 us against 704 / 1440 / 2726, bf16 613 / 1328 / 2622 against
+# 684 / 1378 / 2606; groups of 128 in fp16 at 1024 / 1536 / 2048 tokens 480 / 695 / 864 against 542 / 687 / 853.
+INT8_DEQUANT_MIN_TOKENS = 8192
+INT8_GROUP_DEQUANT_MIN_TOKENS = 1536
+# What the pipelined loop does not take (rows that are no multiple of 64 codes, groups of fewer, the group format in bf16) is converted on the way to LDS:
+# at 4096 tokens QKV 227 against 182 us dequantised, gate/up 817 against 762; an 8B-shaped prefill 17.7 against 19.5 ms at 1024 tokens, 27.5 against 25.8 at 1536
+# (group format: level at 1024 tokens, 35.0 against 29.9 ms at 2048).
+INT8_STAGED_DEQUANT_MIN_TOKENS = 1280
+INT8_GROUP_STAGED_DEQUANT_MIN_TOKENS = 1024
+
+
+def int8_dequantised_from(dtype: torch.dtype, k: int, group_size_shift: int = 0) -> int:
+    """Tokens from which a matrix of rows of k codes is dequantised (group_size_shift 0: per-channel format)."""
+    if group_size_shift:
+        staged = k % 64 or group_size_shift < 6 or dtype != torch.float16
+        return min(INT8_GROUP_DEQUANT_MIN_TOKENS, INT8_GROUP_STAGED_DEQUANT_MIN_TOKENS) if staged else INT8_GROUP_DEQUANT_MIN_TOKENS
+    return min(INT8_DEQUANT_MIN_TOKENS, INT8_STAGED_DEQUANT_MIN_TOKENS) if k % 64 else INT8_DEQUANT_MIN_TOKENS
 
 
 def int8_kernel_dispatchable(x: torch.Tensor) -> bool:
@@ -527,7 +535,7 @@ def mui_int8_channel_linear_forward(x, weights_i8, scales, norm_weights=None, ep
     x = x.contiguous()
     x, norm_weights = _norm_first(x, norm_weights, epsilon, INT8_CHUNK_MAX_TOKENS)
     tokens = _num_tokens(x)
-    if tokens >= INT8_DEQUANT_MIN_TOKENS and k % 16 == 0:
+    if tokens >= int8_dequantised_from(x.dtype, k) and k % 16 == 0:
         w = mui_int8_channel_dequantize_forward(weights_i8, scales)
         return muillm_linear_forward(None, x, w, norm_weights, epsilon, None, add_bias, residual)
     if residual is not None:
@@ -571,7 +579,7 @@ def mui_int8_channel_gateupsilu_forward(norm_weights, epsilon, gate_i8, up_i8, g
     x = x.contiguous()
     x, norm_weights = _norm_first(x, norm_weights, epsilon, INT8_CHUNK_MAX_TOKENS)
     tokens = _num_tokens(x)
-    if tokens >= INT8_DEQUANT_MIN_TOKENS:
+    if tokens >= int8_dequantised_from(x.dtype, k):
         return mui_gateup_silu(norm_weights, epsilon, mui_int8_channel_dequantize_forward(gate_i8, gate_scales),
                                mui_int8_channel_dequantize_forward(up_i8, up_scales), x)
     h = torch.empty(list(x.shape[:-1]) + [n], dtype=x.dtype, device=x.device)
@@ -620,7 +628,7 @@ def muillm_int8_linear_forward(x, weights, scales_min_vals, group_size_shift, no
     _check_contiguous(scales_min_vals, "scales_min_vals")
     _check_activations(x, k, "muillm_int8_linear_forward", _MAX_CALL_TOKENS, weights,
                        scales_min_vals, norm_weights, add_bias, residual)
-    if _num_tokens(x) >= INT8_GROUP_DEQUANT_MIN_TOKENS:
+    if _num_tokens(x) >= int8_dequantised_from(x.dtype, k, group_size_shift):
         # a long prompt: the reference's route (dequantise the matrix, then a GEMM,
         # muillm/modules/quantized/int8linear.py:279-293) on this library's kernels; shorter ones go
         # to the GEMM that dequantises the codes on their way to LDS (one call below)
@@ -746,7 +754,7 @@ def muillm_int8_gateupsilu_forward(norm_weights, epsilon, gate_up_weights, gate_
         raise RuntimeError("gate_up_scales_min_vals must hold N * 2 * K / group (scale, min) pairs in the activation dtype")
     if norm_weights is not None and (norm_weights.dtype != x.dtype or norm_weights.numel() != k):
         raise RuntimeError("norm weights must be one value per input feature in the activation dtype")
-    if _num_tokens(x) >= INT8_GROUP_DEQUANT_MIN_TOKENS:
+    if _num_tokens(x) >= int8_dequantised_from(x.dtype, k, group_size_shift):
         # a long prompt: dequantise gate and up once, then the tiled GEMM with the SiLU * mul epilogue
         gd, ud = muillm_int8_gateupsilu_dequantize_forward(gate_up_weights, gate_up_scales_min_vals, group_size_shift)
         return mui_gateup_silu(norm_weights, epsilon, gd, ud, x)
