@@ -533,12 +533,15 @@ static int launch_lt_t(hipStream_t s, const SkinnyParams& p) {
                      dim3(kLtThreads), 0, s, p.w0, p.w1, p.pitch, p.x, p.n, p.k, p.tokens, n_tiles, SPW, p.gamma, p.y, \
                      p.eps, p.residual, p.mul_bias, p.add_bias, p.s0, p.s1, p.s_pitch, p.group_shift)
   // group format: groups of 128 codes carry two (scale, min) pairs with every 256-value pass, larger
-  // groups one; smaller groups load the pair of each MFMA step where it is used
+  // groups one; smaller groups load the pair of each MFMA step where it is used, and so do rows whose division between the
+  // waves cuts a stretch of `len` values, all of one pair then, out of two groups (B-stationary: K / 8 values per wave; 1280 values are 160 per wave)
+  const int range = p.k <= kLtWaves * 2 * kLtSub && p.k % 256 == 0 ? p.k / kLtWaves : 0;  // 0: whole passes
+  auto in_one_group = [&](int len) { return range % len == 0 || (range < len && (1 << p.group_shift) % range == 0); };
 #define MUI_LT(NORMV, BSTATV, FULLV, HBV, SPW)                                \
   do {                                                                        \
     if constexpr (WF == WF_U8_GROUP) {                                        \
-      if (p.group_shift == 7) MUI_LT_G(NORMV, BSTATV, FULLV, HBV, 2, SPW);    \
-      else if (p.group_shift >= 8) MUI_LT_G(NORMV, BSTATV, FULLV, HBV, 1, SPW); \
+      if (p.group_shift == 7 && in_one_group(128)) MUI_LT_G(NORMV, BSTATV, FULLV, HBV, 2, SPW);    \
+      else if (p.group_shift >= 8 && in_one_group(256)) MUI_LT_G(NORMV, BSTATV, FULLV, HBV, 1, SPW); \
       else MUI_LT_G(NORMV, BSTATV, FULLV, HBV, 0, SPW);                       \
     } else {                                                                  \
       MUI_LT_G(NORMV, BSTATV, FULLV, HBV, 0, SPW);                            \
