@@ -442,6 +442,10 @@ int mui_greedy_advance_ws(mui_stream_t stream, int dtype, const void* logits, lo
  * muillm/modules/kvcache/cache_utils.py). */
 int mui_fill_buffers(mui_stream_t stream, int count, void* const* buffers, const size_t* bytes, const int64_t* values);
 
+/* out[r, :] = in[index[r], :] for r < rows, zeros where index[r] is outside 0 .. in_rows - 1 (a batch's padding). Rows of row_bytes, a multiple
+ * of 16, one after the other in both; in and out 16-byte aligned and apart (else MUI_ERR_ALIGNMENT). */
+int mui_take_rows(mui_stream_t stream, const void* in, long in_rows, size_t row_bytes, const int64_t* index, void* out, long rows);
+
 /* Sampling twin of mui_greedy_advance: tok = argmax_v(logits[b, v] / temperature - log q_v) with
  * q_v ~ Exp(1), which is the draw of the reference's sync-free multinomial
  * argmax(softmax(logits / temperature) / q) (muillm/sampling/multinomial.py:4-6) without
@@ -541,6 +545,17 @@ int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_stack_t* m, 
                              const int64_t* position_ids, long position_batch_stride, const int64_t* cache_position, int seq_len,
                              const void* mask, long mask_batch_stride, int n_splits, void* workspace, void* linear_workspace,
                              size_t linear_workspace_bytes);
+
+/* The same for a padded batch of prompts, padding left out of everything that works on one token at a time: hidden_in and hidden_out
+ * hold real_rows rows (fewer than batch * tokens), number r of them token rows[r] of [batch, tokens] flattened; slots [batch * tokens] has
+ * every token's number among them, or -1 for padding (both int64, on the device). Attention sees [batch, tokens] with zeros for
+ * the padding, whose cache slots become zeros; mask has to hide them. Workspace: mui_decoder_stack_prompt_rows_bytes. */
+size_t mui_decoder_stack_prompt_rows_bytes(const mui_decoder_stack_t* m, int batch, int tokens, int real_rows);
+int mui_decoder_stack_prompt_rows(mui_stream_t stream, const mui_decoder_stack_t* m, int batch, int tokens, int real_rows,
+                                  const int64_t* rows, const int64_t* slots, const void* hidden_in, void* hidden_out,
+                                  const int64_t* position_ids, long position_batch_stride, const int64_t* cache_position, int seq_len,
+                                  const void* mask, long mask_batch_stride, void* workspace, void* linear_workspace,
+                                  size_t linear_workspace_bytes);
 
 /* muillm_embedding_module_forward (csrc/module.cpp:320; csrc/embedding/embedding.cu:31-100; kernels
  * csrc/embedding/embedding_xx16_kernels.cu:26-112): out[t, :] = table[ids[t], :] for a 16-bit

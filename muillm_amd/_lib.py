@@ -95,6 +95,7 @@ _SIGNATURES = {
     "mui_greedy_workspace_bytes": (ctypes.c_size_t, [c_int]),
     "mui_greedy_advance_ws": (c_int, [_P, c_int, _P, c_long, c_int, c_int, _P, _P, _P, _P, _P, c_long, c_int, _P, _P,
                                       c_int, c_long, _P, ctypes.c_size_t, _P, c_long, _P, c_int]),
+    "mui_take_rows": (c_int, [_P, _P, c_long, ctypes.c_size_t, _P, _P, c_long]),
     "mui_fill_buffers": (c_int, [_P, c_int, _P, _P, _P]),
     "mui_sample_advance": (c_int, [_P, c_int, _P, c_long, c_int, c_int, c_float, ctypes.c_uint64, _P, _P, _P, _P, _P,
                                    c_long, c_int, _P, _P, c_int, c_long]),
@@ -102,6 +103,8 @@ _SIGNATURES = {
     "mui_decoder_stack_workspace_bytes": (ctypes.c_size_t, [_P, c_int, c_int]),
     "mui_decoder_stack_prompt_bytes": (ctypes.c_size_t, [_P, c_int, c_int, c_int]),
     "mui_decoder_stack_prompt": (c_int, [_P, _P, c_int, c_int, _P, _P, _P, c_long, _P, c_int, _P, c_long, c_int, _P, _P, ctypes.c_size_t]),
+    "mui_decoder_stack_prompt_rows_bytes": (ctypes.c_size_t, [_P, c_int, c_int, c_int]),
+    "mui_decoder_stack_prompt_rows": (c_int, [_P, _P, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_long, _P, c_int, _P, c_long, _P, _P, ctypes.c_size_t]),
     "mui_decoder_stack_step": (c_int, [_P, _P, c_int, _P, _P, _P, c_long, _P, c_int, _P, c_long, c_int, _P]),
     "mui_residual_norm": (c_int, [_P, c_int, _P, _P, c_float, _P, c_float, _P, c_float, c_float, _P, _P, c_int, c_int]),
     "mui_linear_residual_norm": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_float, _P, c_float, c_float, _P, _P, _P, c_int, c_int,

@@ -135,21 +135,24 @@ struct PromptWorkspace {
   char *h_a, *h_b;  // [rows, hidden]  residual stream
   char* normed;     // [rows, hidden]  the next linear's input
   char *qkv, *q_rot, *attn, *scratch;  // up to the output projection
+  char* spread;  // [batch * tokens, .] qkv with the padding, where the rows leave it out
   char* mid;                           // [rows, intermediate], in the same place
   size_t total;
 };
 
-PromptWorkspace carve_rows(const mui_decoder_stack_t* m, int batch, int tokens, int n_splits, char* base) {
+// real: rows that are no padding (batch * tokens: all of them)
+PromptWorkspace carve_rows(const mui_decoder_stack_t* m, int batch, int tokens, int n_splits, char* base, int real) {
   PromptWorkspace w;
-  const size_t rows = (size_t)batch * tokens, e = 2;
-  const size_t hid = align256(rows * m->hidden * e), att = align256(rows * m->n_q_heads * m->head_dim * e);
+  const size_t all = (size_t)batch * tokens, rows = real, e = 2;
+  const size_t hid = align256(rows * m->hidden * e), att = align256(all * m->n_q_heads * m->head_dim * e);
   const size_t qkv = align256(rows * (m->n_q_heads + 2 * m->n_kv_heads) * m->head_dim * e), mid = align256(rows * m->intermediate * e);
   const size_t scr = tokens == 1 ? align256(mui_flash_decode_scratch_bytes(batch, m->n_q_heads, m->head_dim, n_splits)) : 0;
   w.h_a = base;
   w.h_b = w.h_a + hid;
   w.normed = w.h_b + hid;
   w.qkv = w.normed + hid;
-  w.q_rot = w.qkv + qkv;
+  w.spread = w.qkv + qkv;
+  w.q_rot = w.spread + (rows < all ? align256(all * (m->n_q_heads + 2 * m->n_kv_heads) * m->head_dim * e) : 0);
   w.attn = w.q_rot + (tokens == 1 ? 0 : att);
   w.scratch = w.attn + att;
   w.mid = w.qkv;  // (the output projection has read the rest when the gate and up products start)
@@ -162,20 +165,22 @@ PromptWorkspace carve_rows(const mui_decoder_stack_t* m, int batch, int tokens, 
 
 extern "C" size_t mui_decoder_stack_prompt_bytes(const mui_decoder_stack_t* m, int batch, int tokens, int n_splits) {
   if (!m || batch < 1 || tokens < 1 || n_splits < 1) return 0;
-  return carve_rows(m, batch, tokens, n_splits, nullptr).total;
+  return carve_rows(m, batch, tokens, n_splits, nullptr, batch * tokens).total;
 }
 
-extern "C" int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_stack_t* m, int batch, int tokens, const void* hidden_in,
-                                        void* hidden_out, const int64_t* position_ids, long position_batch_stride,
-                                        const int64_t* cache_position, int seq_len, const void* mask, long mask_batch_stride, int n_splits,
-                                        void* workspace, void* linear_workspace, size_t linear_workspace_bytes) {
+// rows, slots (both or neither): the rows that are no padding -- hidden_in and hidden_out have `real` rows, number r of them token rows[r] of [batch, tokens] --,
+// and every token's number among them, or -1
+static int prompt_layers(mui_stream_t stream, const mui_decoder_stack_t* m, int batch, int tokens, int real, const int64_t* real_rows, const int64_t* slots,
+                         const void* hidden_in, void* hidden_out, const int64_t* position_ids, long position_batch_stride, const int64_t* cache_position,
+                         int seq_len, const void* mask, long mask_batch_stride, int n_splits, void* workspace, void* linear_workspace,
+                         size_t linear_workspace_bytes) {
   MUI_CHECK_ARG(m && m->layers && m->n_layers > 0 && hidden_in && hidden_out && workspace);
   MUI_CHECK_ARG(batch >= 1 && tokens >= 1 && n_splits >= 1 && position_ids && cache_position);
   MUI_CHECK_ARG(((uintptr_t)workspace & 255u) == 0 && (long)batch * tokens <= (1L << 30));
   MUI_CHECK_ARG(tokens == 1 || seq_len >= tokens);
   MUI_CHECK_ARG(seq_len <= m->max_cache_len);  // (the prompt's attention takes no capacity: it reads seq_len rows of every head)
-  const int rows = batch * tokens;
-  const PromptWorkspace w = carve_rows(m, batch, tokens, n_splits, (char*)workspace);
+  const int rows = real;
+  const PromptWorkspace w = carve_rows(m, batch, tokens, n_splits, (char*)workspace, real);
   const int hid = m->hidden, qd = m->n_q_heads * m->head_dim, kvd = m->n_kv_heads * m->head_dim, qkv_n = qd + 2 * kvd;
   const bool fused = rows <= MUI_MAX_TOKENS;  // the decode kernels take the norm in front of a linear; beyond, it is a launch of its own or rides behind the linear in front
   for (int l = 0; l < m->n_layers; ++l) {
@@ -211,7 +216,11 @@ extern "C" int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_s
     char* out = last ? (char*)hidden_out : w.h_b;
     int st = linear(L.qkv_weight, L.qkv_pitch, L.qkv_scales, gs, fused ? h : w.normed, fused ? L.input_norm : nullptr, nullptr, w.qkv, qkv_n, hid, nullptr);
     if (st != MUI_OK) return st;
-    const char *q = w.qkv, *k = q + (size_t)qd * 2, *v = k + (size_t)kvd * 2;
+    if (slots) {
+      st = mui_take_rows(stream, w.qkv, real, (size_t)qkv_n * 2, slots, w.spread, (long)batch * tokens);
+      if (st != MUI_OK) return st;
+    }
+    const char *q = slots ? w.spread : w.qkv, *k = q + (size_t)qd * 2, *v = k + (size_t)kvd * 2;
     if (tokens == 1) {
       st = mui_attn_decode_fused_warm(stream, m->dtype, q, qkv_n, k, qkv_n, v, qkv_n, m->cos_table, m->sin_table, (int)m->rope_row_stride,
                                       (int)m->rope_rows, position_ids, position_batch_stride, cache_position, seq_len, L.k_cache, L.v_cache,
@@ -231,7 +240,13 @@ extern "C" int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_s
                                         m->cache_token_stride, seq_len, seq_len - tokens, w.attn, batch, m->n_q_heads, m->n_kv_heads, tokens, m->head_dim);
     }
     if (st != MUI_OK) return st;
-    st = linear(L.o_weight, L.o_pitch, L.o_scales, gs, w.attn, nullptr, h, w.h_a, hid, qd, fused ? nullptr : L.post_norm);
+    const char* attended = w.attn;
+    if (slots) {  // (the queries have been read)
+      st = mui_take_rows(stream, w.attn, (long)batch * tokens, (size_t)qd * 2, real_rows, w.q_rot, real);
+      if (st != MUI_OK) return st;
+      attended = w.q_rot;
+    }
+    st = linear(L.o_weight, L.o_pitch, L.o_scales, gs, attended, nullptr, h, w.h_a, hid, qd, fused ? nullptr : L.post_norm);
     if (st != MUI_OK) return st;
     const void *mx = fused ? w.h_a : w.normed, *gain = fused ? L.post_norm : nullptr;
     st = !L.gate_scales ? mui_gateup_silu(stream, m->dtype, L.gate_weight, L.up_weight, L.gateup_pitch, mx, gain, m->norm_eps, w.mid, m->intermediate, hid, rows)
@@ -246,4 +261,27 @@ extern "C" int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_s
     h = out;
   }
   return MUI_OK;
+}
+
+extern "C" int mui_decoder_stack_prompt(mui_stream_t stream, const mui_decoder_stack_t* m, int batch, int tokens, const void* hidden_in,
+                                        void* hidden_out, const int64_t* position_ids, long position_batch_stride,
+                                        const int64_t* cache_position, int seq_len, const void* mask, long mask_batch_stride, int n_splits,
+                                        void* workspace, void* linear_workspace, size_t linear_workspace_bytes) {
+  return prompt_layers(stream, m, batch, tokens, (int)((long)batch * tokens), nullptr, nullptr, hidden_in, hidden_out, position_ids,
+                       position_batch_stride, cache_position, seq_len, mask, mask_batch_stride, n_splits, workspace, linear_workspace,
+                       linear_workspace_bytes);
+}
+
+extern "C" size_t mui_decoder_stack_prompt_rows_bytes(const mui_decoder_stack_t* m, int batch, int tokens, int real_rows) {
+  if (!m || batch < 1 || tokens < 1 || real_rows < 1 || real_rows > (long)batch * tokens) return 0;
+  return carve_rows(m, batch, tokens, 1, nullptr, real_rows).total;
+}
+
+extern "C" int mui_decoder_stack_prompt_rows(mui_stream_t stream, const mui_decoder_stack_t* m, int batch, int tokens, int real_rows, const int64_t* rows,
+                                             const int64_t* slots, const void* hidden_in, void* hidden_out, const int64_t* position_ids,
+                                             long position_batch_stride, const int64_t* cache_position, int seq_len, const void* mask,
+                                             long mask_batch_stride, void* workspace, void* linear_workspace, size_t linear_workspace_bytes) {
+  MUI_CHECK_ARG(rows && slots && batch >= 1 && tokens > 1 && real_rows >= 1 && real_rows < (long)batch * tokens);
+  return prompt_layers(stream, m, batch, tokens, real_rows, rows, slots, hidden_in, hidden_out, position_ids, position_batch_stride, cache_position, seq_len,
+                       mask, mask_batch_stride, 1, workspace, linear_workspace, linear_workspace_bytes);
 }

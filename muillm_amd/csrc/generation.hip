@@ -63,6 +63,16 @@ __global__ void __launch_bounds__(kFillThreads) fill_buffers_kernel(const FillLi
 }
 
 // ---------------------------------------------------------------------------------------
+// rows by number: out[r] = in[index[r]], zeros for numbers outside 0 .. in_rows - 1; rows of whole 16-byte chunks. A copy, bound by its bytes
+// ---------------------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) take_rows_kernel(const u32x4* in, const int64_t* index, u32x4* out, unsigned chunks, long in_rows, long all) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= all) return;
+  const long r = i / chunks, c = i - r * chunks, from = index[r];
+  out[i] = from >= 0 && from < in_rows ? in[from * chunks + c] : u32x4{0u, 0u, 0u, 0u};
+}
+
+// ---------------------------------------------------------------------------------------
 // token embedding plus bigram embedding: x = scale * table[id] + bigram[(prev * mul_prev + id * mul_cur) mod buckets],
 // the last row (number `buckets`) for the first token of a sequence; x in fp32 and, rounded, as the first
 // sublayer's input. One workgroup per token; the one of a row's first token reads and replaces prev[row].
@@ -257,6 +267,18 @@ extern "C" int mui_bigram_embedding(mui_stream_t stream, int dtype, const int64_
   else if (dtype == MUI_DTYPE_BF16) hipLaunchKernelGGL((bigram_embedding_kernel<BF16>), grid, block, 0, s, p);
   else if (dtype == MUI_DTYPE_F32) hipLaunchKernelGGL((bigram_embedding_kernel<F32>), grid, block, 0, s, p);
   else return MUI_ERR_INVALID_ARG;
+  return launch_status();
+}
+
+extern "C" int mui_take_rows(mui_stream_t stream, const void* in, long in_rows, size_t row_bytes, const int64_t* index, void* out, long rows) {
+  MUI_CHECK_ARG(rows >= 0 && in_rows >= 0 && row_bytes > 0 && (rows == 0 || (index && out && (in || in_rows == 0))));
+  if (row_bytes % 16 || !aligned16(in) || !aligned16(out)) return MUI_ERR_ALIGNMENT;
+  if (rows == 0) return MUI_OK;
+  const size_t chunks = row_bytes / 16;
+  if (chunks > 0x7fffffffu || (size_t)rows > ((size_t)1 << 39) / chunks) return MUI_ERR_UNSUPPORTED;
+  const long all = rows * (long)chunks;
+  hipLaunchKernelGGL(take_rows_kernel, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (const u32x4*)in, index, (u32x4*)out,
+                     (unsigned)chunks, in_rows, all);
   return launch_status();
 }
 

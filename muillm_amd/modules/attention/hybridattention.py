@@ -42,6 +42,8 @@ class MuiHybridAttentionConfig:
 
 
 class MuiHybridAttention(MuiModule):
+    takes_real_rows = True
+
     def takes_behind(self) -> bool:
         return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
@@ -69,7 +71,7 @@ class MuiHybridAttention(MuiModule):
     def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
         """h [B, T, hidden] -> [B, T, hidden]; the tokens' rows go to slots cache_position."""
         c, state = self.config, cache.layers[self.layer_idx]
-        proj = self.proj.linear(h)
+        proj = cache.spread(self.proj.linear(h))
         o = hybrid_ops.hybrid_step(proj, c.heads, c.kv_heads, c.dim, c.vdim, self.q_norm, self.k_norm, self.eps, self.inv_freq, cache_position,
                                    cache.row_start, state.k, state.v, c.gated, c.scale, c.softcap, c.window, c.keep_first)
         if o is None:
@@ -78,4 +80,5 @@ class MuiHybridAttention(MuiModule):
             gate = proj[..., self.proj.slice_starts[3]:] if c.gated else None
             o = hybrid_ops.hybrid_attention(q, state.k, state.v, gate, cache_position, cache.row_start, c.heads, c.kv_heads, c.scale,
                                             c.softcap, c.window, c.keep_first)
+        o = cache.take(o)
         return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

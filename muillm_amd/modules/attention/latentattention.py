@@ -37,6 +37,8 @@ class MuiLatentAttentionConfig:
 
 
 class MuiLatentAttention(MuiModule):
+    takes_real_rows = True
+
     def takes_behind(self) -> bool:
         return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
@@ -66,9 +68,10 @@ class MuiLatentAttention(MuiModule):
     def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
         """h [B, T, hidden] (normed) -> [B, T, hidden]; the tokens' rows go to slots cache_position."""
         c = self.config
-        b, t = h.shape[0], h.shape[1]
+        down = cache.spread(self.down.linear(h))
+        b, t = down.shape[0], down.shape[1]
         state: MuiLatentState = cache.layers[self.layer_idx if self.own_rows else c.kv_source]
-        q_latent, cos_sin = hybrid_ops.latent_prepare(self.down.linear(h), self.q_norm, self.kv_norm, self.eps, self.inv_freq,
+        q_latent, cos_sin = hybrid_ops.latent_prepare(down, self.q_norm, self.kv_norm, self.eps, self.inv_freq,
                                                       cache_position, cache.row_start, state.c, state.r)
         q = self.up_q(q_latent)
         route = hybrid_ops.latent_route(h.dtype, t, c.heads, c.dim, c.rot_dim, c.vdim, c.kv_rank)
@@ -83,4 +86,5 @@ class MuiLatentAttention(MuiModule):
         else:
             o = hybrid_ops.latent_attention(q, cos_sin, w[:c.heads * c.dim], w[c.heads * c.dim:], state.c, state.r,
                                             cache_position, cache.row_start, c.heads, c.dim, c.vdim, c.scale, c.window, route)
+        o = cache.take(o)
         return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

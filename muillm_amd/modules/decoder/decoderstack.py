@@ -26,6 +26,7 @@ from ..linear import MuiLinear
 from ..multilinear import MuiMultiLinear
 from ..quantized.int8gateupdownmlp import MuiInt8GateUpDownMLP
 from ..quantized.int8linear import MuiInt8Linear
+from ..realrows import RealRows
 from .decoder import MuiDecoderLayer
 
 
@@ -499,6 +500,21 @@ class MuiPromptStack(MuiDecoderStack):
             if most is not None and t > most:
                 return False
         return True
+
+    def run_real(self, hidden_in: torch.Tensor, real: RealRows, position_ids: torch.Tensor, cache_position: torch.Tensor, seq_len: int,
+                 mask: torch.Tensor) -> torch.Tensor:
+        """hidden_in [1, real rows, hidden] of a padded batch of prompts -> output of the last layer, likewise. mask: the key mask that hides the padding."""
+        lib, x, stream = self.lib, hidden_in.contiguous(), muillm_ext._stream(hidden_in)
+        b, t, n = real.batch, real.tokens, real.n
+        ws = torch.empty(lib.mui_decoder_stack_prompt_rows_bytes(ctypes.byref(self.desc), b, t, n) + 256, dtype=torch.uint8, device=x.device)
+        linear_ws = muillm_ext._prompt_workspace(x, stream) if n > _lib.MUI_MAX_TOKENS else None
+        pos, out = position_ids.contiguous(), torch.empty_like(x)
+        muillm_ext.check(
+            lib.mui_decoder_stack_prompt_rows(stream, ctypes.byref(self.desc), b, t, n, real.rows.data_ptr(), real.slots.data_ptr(), x.data_ptr(),
+                                              out.data_ptr(), pos.data_ptr(), t if pos.shape[0] > 1 else 0, cache_position.data_ptr(), seq_len,
+                                              mask.data_ptr(), mask.stride(0), (ws.data_ptr() + 255) & ~255, _ptr(linear_ws),
+                                              0 if linear_ws is None else linear_ws.numel()), "mui_decoder_stack_prompt_rows")
+        return out
 
     def run(self, hidden_in: torch.Tensor, position_ids: torch.Tensor, cache_position: torch.Tensor, seq_len: Optional[int],
             mask: Optional[torch.Tensor]) -> torch.Tensor:

@@ -94,6 +94,7 @@ class MuiHybridCache(MuiCache):
         self.layers = [m.new_state(max_batch_size, self.max_cache_len, device, dtype) for m in mixers]
         self.front = None if front is None else front.new_state(max_batch_size, self.max_cache_len, device, dtype)
         self.row_start: Optional[torch.Tensor] = None
+        self.real = None  # while a padded batch's layers run on its real rows alone: those rows (RealRows)
         self._seen_tokens = 0
         # True while a captured decode step runs: positions are read from device memory only
         self.device_length_mode = False
@@ -111,6 +112,14 @@ class MuiHybridCache(MuiCache):
 
     def step_state(self) -> List[torch.Tensor]:
         return [t for s in self._states() for t in s.recurrent()]
+
+    def spread(self, x: torch.Tensor) -> torch.Tensor:
+        """What the layers pass on as [B, T, w], zeros where padding is left out."""
+        return x if self.real is None else self.real.spread(x)
+
+    def take(self, x: torch.Tensor) -> torch.Tensor:
+        """[B, T, w] as the layers pass it on: padding left out where it is."""
+        return x if self.real is None else self.real.take(x)
 
     def set_row_start(self, row_start: Optional[torch.Tensor]) -> None:
         """First real slot of every row; kept in one buffer so that a captured step stays valid."""

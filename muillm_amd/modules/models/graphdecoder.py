@@ -18,6 +18,7 @@ import torch
 from ... import muillm_ext
 from ..._lib import MUI_MAX_TOKENS
 from ..kvcache.cache_utils import MuiCache, _next_pow2
+from ..realrows import RealRows
 
 
 class MuiGraphDecoder:
@@ -213,7 +214,8 @@ class MuiGraphDecoder:
         lm = self.lm
         device = input_ids.device
         batch, prompt_len = input_ids.shape
-        padded = attention_mask is not None and not bool(torch.all(attention_mask == 1))
+        seen = None if attention_mask is None else attention_mask.to("cpu")  # (looked at here: one wait for the GPU, not one per question)
+        padded = seen is not None and not bool(torch.all(seen == 1))
         # a cache that already holds tokens continues after them (multi-turn): slots and rotary
         # positions are offset by what it has seen
         past = 0 if cache is None else cache.get_seq_length()
@@ -238,11 +240,13 @@ class MuiGraphDecoder:
         cache.device_length_mode = False
         if padded:
             am = attention_mask.to(device=device, dtype=torch.int64)
-            if bool((am[:, -1] == 0).any()):
+            real_tokens = seen.to(torch.int64) != 0
+            if not bool(real_tokens[:, -1].all()):
                 raise ValueError("padding must be on the left: the last prompt position of every row must be real")
             prompt_pos = (am.cumsum(-1) - 1).clamp_(min=0)
+            real = RealRows.of(lm, real_tokens, device)
             out = lm(input_ids=input_ids, attention_mask=am, position_ids=prompt_pos, past_key_values=cache,
-                     use_cache=True, all_ones_mask=False, num_logits_to_keep=1, float_logits=False)
+                     use_cache=True, all_ones_mask=False, num_logits_to_keep=1, float_logits=False, **({} if real is None else {"real": real}))
         else:
             out = lm(input_ids=input_ids, past_key_values=cache, use_cache=True, all_ones_mask=True,
                      num_logits_to_keep=1, float_logits=False)

@@ -38,6 +38,7 @@ from ...linear import MuiLinear
 from ...module import MuiModule, heard
 from ...multilinear import MuiMultiLinear
 from ...norm.rmsnorm import MuiRMSNorm
+from ...realrows import RealRows
 from ..generation import MuiGenerationMixin
 
 
@@ -96,6 +97,8 @@ _BUSY_PRODUCTS = 10 ** 11
 
 
 class MuiLlamaModel(MuiModule):
+    takes_real_rows = True
+
     def __init__(self, engine_config: MuiEngineConfig, config, embed_tokens: nn.Embedding, layers,
                  norm: MuiRMSNorm, rotary_emb: MuiRotaryEmbedding):
         super().__init__(engine_config=engine_config)
@@ -185,6 +188,27 @@ class MuiLlamaModel(MuiModule):
         st.remember()  # the next call need not examine the layers either
         return None
 
+    def _real_rows(self, input_ids, attention_mask, position_ids, cache_position, cache, real: RealRows) -> Optional[torch.Tensor]:
+        """The last layer's output for every row's last token [B, 1, hidden] of a padded batch, its padding left out; None: not a case for it, nothing has been done."""
+        embed = self.embed_tokens
+        if input_ids is None or not input_ids.is_cuda or tuple(attention_mask.shape) != tuple(input_ids.shape) or heard(self, embed, self.norm):
+            return None
+        if self.mdtype not in (torch.float16, torch.bfloat16):
+            return None
+        b, t = input_ids.shape
+        like = embed.weight.detach()[:1].expand(b * t, -1).view(b, t, -1)  # (what the layers would be given, as far as anyone looks)
+        stack = self._prompt_stack(cache, like, position_ids, cache_position, torch.empty((b, (t + 7) // 8 * 8), dtype=self.mdtype, device=like.device))
+        if not stack:
+            return None
+        mask = muillm_ext.key_padding_mask16(attention_mask, self.mdtype, t)
+        x = embed(input_ids.reshape(-1)[real.rows][None])
+        cache._seen_tokens += t
+        if cache.cpp_module is not None:
+            cache.cpp_module.seen_tokens = cache._seen_tokens
+        out = real.last_of(stack.run_real(x, real, position_ids, cache_position, cache._seen_tokens, mask))
+        cache.sync_back()
+        return out
+
     def _examine_layers(self, cache) -> Optional[MuiPromptStack]:
         return MuiPromptStack(self.layers, self.rotary_emb, cache) if MuiPromptStack.eligible(self.layers, self.rotary_emb, cache) else None
 
@@ -224,9 +248,11 @@ class MuiLlamaModel(MuiModule):
                 inputs_embeds: Optional[torch.Tensor] = None, use_cache: Optional[bool] = None,
                 output_attentions: Optional[bool] = None, output_hidden_states: Optional[bool] = None,
                 return_dict: Optional[bool] = None, cache_position: Optional[torch.LongTensor] = None,
-                all_ones_mask: Optional[bool] = None, skip_final_norm: bool = False):
+                all_ones_mask: Optional[bool] = None, skip_final_norm: bool = False, real: Optional[RealRows] = None):
         """skip_final_norm=True returns the un-normalised last hidden state: the causal-LM head
-        then applies the final RMSNorm inside its GEMV kernel (single-token decode)."""
+        then applies the final RMSNorm inside its GEMV kernel (single-token decode).
+        real: the tokens of a padded batch that are no padding, from a caller that reads the last position alone: where the single call takes the
+        prompt, padding is left out and last_hidden_state is [B, 1, hidden]."""
         output_attentions = bool(output_attentions)
         output_hidden_states = bool(output_hidden_states)
         use_cache = True if use_cache is None else use_cache
@@ -269,6 +295,10 @@ class MuiLlamaModel(MuiModule):
         if position_ids is None:
             position_ids = cache_position.unsqueeze(0)
 
+        if real is not None and use_cache and past_seen_tokens == 0 and not (windowed or output_hidden_states or output_attentions or skip_final_norm):
+            hidden_states = self._real_rows(input_ids, attention_mask, position_ids.contiguous(), cache_position, past_key_values, real)
+            if hidden_states is not None:
+                return MuiModelOutput(last_hidden_state=self.norm(hidden_states), past_key_values=past_key_values, hidden_states=None, attentions=None)
         if all_ones_mask is None:
             all_ones_mask = attention_mask is None
         causal_mask = None
@@ -419,6 +449,7 @@ class MuiLlamaForCausalLM(MuiGenerationMixin, MuiModule):
 
     # ---- what the decode loop asks of a causal LM ---------------------------------------------
     pads_in_cache = False  # left padding travels as an additive mask with every step
+    takes_real_rows = True
 
     def create_cache(self, batch_size: int, seq_len: int) -> MuiStaticCache:
         return create_static_cache(self.engine_config, self.config, batch_size, seq_len, self.model.mdevice, self.model.mdtype)
@@ -438,9 +469,9 @@ class MuiLlamaForCausalLM(MuiGenerationMixin, MuiModule):
                 output_attentions: Optional[bool] = None, output_hidden_states: Optional[bool] = None,
                 return_dict: Optional[bool] = None, cache_position: Optional[torch.LongTensor] = None,
                 all_ones_mask: Optional[bool] = None, num_logits_to_keep: int = 0, float_logits: bool = True,
-                logits_positions: Union[None, list, torch.Tensor] = None):
+                logits_positions: Union[None, list, torch.Tensor] = None, real: Optional[RealRows] = None):
         """logits_positions: the places among the tokens whose logits are wanted (default all;
-        num_logits_to_keep: the last ones)."""
+        num_logits_to_keep: the last ones). real: with num_logits_to_keep 1, the tokens that are no padding."""
         if labels is not None:
             raise NotImplementedError("inference only: labels/loss are not supported")
         shape = input_ids.shape if input_ids is not None else inputs_embeds.shape
@@ -452,7 +483,8 @@ class MuiLlamaForCausalLM(MuiGenerationMixin, MuiModule):
             input_ids=input_ids, attention_mask=attention_mask, position_ids=position_ids,
             past_key_values=past_key_values, inputs_embeds=inputs_embeds, use_cache=use_cache,
             output_attentions=output_attentions, output_hidden_states=output_hidden_states,
-            cache_position=cache_position, all_ones_mask=all_ones_mask, skip_final_norm=fuse_norm)
+            cache_position=cache_position, all_ones_mask=all_ones_mask, skip_final_norm=fuse_norm,
+            **({} if real is None or num_logits_to_keep != 1 or logits_positions is not None else {"real": real}))
         hidden_states = outputs.last_hidden_state
         if logits_positions is not None:
             hidden_states = hidden_states[:, logits_positions, :]

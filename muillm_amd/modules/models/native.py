@@ -11,8 +11,10 @@ from ...engineconfig import MuiEngineConfig
 from ..decoder.sandwichdecoder import run_layers
 from ..kvcache.hybridcache import MuiHybridCache
 from ..linear import MuiLinear
-from ..module import MuiModule
+from ..gateupdownmlp import MuiGateUpDownMLP
+from ..module import MuiModule, heard
 from ..norm.rmsnorm import MuiRMSNorm
+from ..realrows import RealRows, on_device
 from .generation import MuiGenerationMixin
 from .llama.model import MuiCausalLMOutput, MuiModelOutput
 
@@ -45,10 +47,13 @@ class MuiNativeModel(MuiModule):
 
     def forward(self, input_ids: Optional[torch.LongTensor] = None, attention_mask: Optional[torch.Tensor] = None,
                 past_key_values: Optional[MuiHybridCache] = None, inputs_embeds: Optional[torch.Tensor] = None,
-                output_hidden_states: Optional[bool] = None, cache_position: Optional[torch.LongTensor] = None) -> MuiModelOutput:
+                output_hidden_states: Optional[bool] = None, cache_position: Optional[torch.LongTensor] = None,
+                real: Optional[RealRows] = None) -> MuiModelOutput:
         """inputs_embeds are rows of the embedding table (their scale is applied here).
         attention_mask [B, T] of 0 / 1 marks left padding of the tokens an empty cache starts with.
-        hidden_states: the fp32 residual stream after every layer."""
+        hidden_states: the fp32 residual stream after every layer.
+        real: the tokens of a padded batch that are no padding, from a caller that reads the last position alone: where the layers take it padding is left out,
+        and last_hidden_state is [B, 1, hidden]."""
         if (input_ids is None) == (inputs_embeds is None):
             raise ValueError("specify either input_ids or inputs_embeds")
         src = input_ids if inputs_embeds is None else inputs_embeds
@@ -64,16 +69,29 @@ class MuiNativeModel(MuiModule):
         if not cache.device_length_mode:
             cache.grow_cache(past + t)
         if attention_mask is not None and past == 0:
-            cache.set_row_start(self._left_padding(attention_mask))
+            cache.set_row_start(self._left_padding(attention_mask) if real is None else on_device(self._left_padding(real.mask), attention_mask.device))
         if cache_position is None:
             cache_position = torch.arange(past, past + t, device=src.device)
         collect = [] if output_hidden_states else None
         x, h = self.start(input_ids, inputs_embeds, cache, cache_position)
-        h = run_layers(self.layers, x, h, self.norm, self.config.rms_norm_eps, cache, cache_position, collect,
-                       final_scale=self.logit_scale)
+        real = real if real is not None and past == 0 and collect is None and x.is_cuda and self._takes_real_rows() else None
+        if real is not None:
+            x, h, cache.real = real.take(x), real.take(h), real
+        try:
+            h = run_layers(self.layers, x, h, self.norm, self.config.rms_norm_eps, cache, cache_position, collect,
+                           final_scale=self.logit_scale)
+        finally:
+            cache.real = None
+        if real is not None:
+            h = real.last_of(h)
         cache.set_seen_tokens(past + t)
         return MuiModelOutput(last_hidden_state=h, past_key_values=cache,
                               hidden_states=None if collect is None else tuple(collect))
+
+    def _takes_real_rows(self) -> bool:
+        """Whether every layer is one that can be given the rows that are no padding alone, and nobody listens to what it is given."""
+        parts = [m for l in self.layers for m in (l.mixer, l.mlp) if m is not None]
+        return all("takes_real_rows" in type(m).__dict__ or type(m) is MuiGateUpDownMLP for m in parts) and not heard(*self.modules())
 
     @staticmethod
     def _left_padding(attention_mask: torch.Tensor) -> Optional[torch.Tensor]:
@@ -191,12 +209,15 @@ class MuiNativeForCausalLM(MuiGenerationMixin, MuiModule):
                 inputs_embeds: Optional[torch.Tensor] = None, use_cache: Optional[bool] = None,
                 output_hidden_states: Optional[bool] = None, cache_position: Optional[torch.LongTensor] = None,
                 all_ones_mask: Optional[bool] = None, num_logits_to_keep: int = 0,
-                logits_positions: Union[None, list, torch.Tensor] = None, float_logits: bool = True) -> MuiCausalLMOutput:
+                logits_positions: Union[None, list, torch.Tensor] = None, float_logits: bool = True,
+                real: Optional[RealRows] = None) -> MuiCausalLMOutput:
         """One step over the tokens given, from the state the cache holds. position_ids are accepted for the
         decode loop's sake: a token's position is its slot minus its row's first slot. logits_positions: the
-        places among the tokens whose logits are wanted (default all; num_logits_to_keep: the last ones)."""
+        places among the tokens whose logits are wanted (default all; num_logits_to_keep: the last ones). real: with num_logits_to_keep 1, the tokens that
+        are no padding."""
         out = self.model(input_ids=input_ids, attention_mask=attention_mask, past_key_values=past_key_values,
-                         inputs_embeds=inputs_embeds, output_hidden_states=output_hidden_states, cache_position=cache_position)
+                         inputs_embeds=inputs_embeds, output_hidden_states=output_hidden_states, cache_position=cache_position,
+                         **({} if real is None or num_logits_to_keep != 1 or logits_positions is not None else {"real": real}))
         h = out.last_hidden_state
         if logits_positions is not None:
             h = h[:, logits_positions, :]

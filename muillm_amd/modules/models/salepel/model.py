@@ -45,6 +45,8 @@ def _mixer_tensors(mixer) -> Iterator[Tuple[str, torch.Tensor]]:
 
 
 class MuiSalepelModel(MuiNativeModel):
+    takes_real_rows = True
+
     def __init__(self, engine_config: MuiEngineConfig, config: MuiSalepelConfig, device=None, dtype=None):
         super().__init__(engine_config, config)
         hid, eps = config.hidden_size, config.rms_norm_eps
@@ -67,6 +69,7 @@ class MuiSalepelModel(MuiNativeModel):
 
 
 class MuiSalepelForCausalLM(MuiNativeForCausalLM):
+    takes_real_rows = True
     model_class = MuiSalepelModel
     config_class = MuiSalepelConfig
 

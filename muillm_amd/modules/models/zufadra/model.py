@@ -46,6 +46,8 @@ def _mixer_tensors(mixer) -> Iterator[Tuple[str, torch.Tensor]]:
 
 
 class MuiZufadraModel(MuiNativeModel):
+    takes_real_rows = True
+
     def __init__(self, engine_config: MuiEngineConfig, config: MuiZufadraConfig, device=None, dtype=None):
         super().__init__(engine_config, config)
         hid, eps, bg = config.hidden_size, config.rms_norm_eps, config.bigram
@@ -81,6 +83,7 @@ class MuiZufadraModel(MuiNativeModel):
 
 
 class MuiZufadraForCausalLM(MuiNativeForCausalLM):
+    takes_real_rows = True
     model_class = MuiZufadraModel
     config_class = MuiZufadraConfig
 

@@ -27,6 +27,8 @@ class MuiMoEConfig:
 
 
 class MuiMoE(MuiModule):
+    takes_real_rows = True
+
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiMoEConfig, device=None, dtype=None):
         super().__init__(engine_config=engine_config)
         c = self.config = config

@@ -38,6 +38,8 @@ class MuiChannelDelta(MuiModule):
     """Everything that reads h is one projection q | k | v | a1 | g1 | b. The low-rank parts and b are padded with zero
     rows (and a2, g2 with zero columns) to multiples of eight, so that every part starts on a 16-byte boundary."""
 
+    takes_real_rows = True
+
     def takes_behind(self) -> bool:
         return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
@@ -76,5 +78,6 @@ class MuiChannelDelta(MuiModule):
 
     def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
         memory, ring = cache.layers[self.layer_idx].values
-        o = hybrid_ops.channel_delta(self.layer(), self.proj.linear(h), memory, ring, cache_position, cache.row_start)
+        o = hybrid_ops.channel_delta(self.layer(), cache.spread(self.proj.linear(h)), memory, ring, cache_position, cache.row_start)
+        o = cache.take(o)
         return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

@@ -22,6 +22,8 @@ class MuiMLstmConfig:
 
 
 class MuiMLstm(MuiModule):
+    takes_real_rows = True
+
     def takes_behind(self) -> bool:
         return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
@@ -47,10 +49,14 @@ class MuiMLstm(MuiModule):
 
     def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
         c = self.config
-        b, t = h.shape[0], h.shape[1]
-        q, k, v, gate = self.proj(h)
-        gates = hybrid_ops.linear_f32(h, self.gate_weight, self.gate_bias).view(b, t, 2 * c.heads)
+        if cache.real is None:
+            q, k, v, gate = self.proj(h)
+        else:
+            y = cache.spread(self.proj.linear(h))
+            q, k, v, gate = (y[..., lo:hi] for lo, hi in zip(self.proj.slice_starts, self.proj.slice_ends))
+        gates = cache.spread(hybrid_ops.linear_f32(h, self.gate_weight, self.gate_bias).view(h.shape[0], h.shape[1], 2 * c.heads))
         o = hybrid_ops.mlstm(q, k, v, gates, cache.layers[self.layer_idx].values, c.dim ** -0.5, c.gate_cap, cache_position,
                              cache.row_start, c.heads)
         o = hybrid_ops.mlstm_output(o, self.head_norm, gate, self.eps)
+        o = cache.take(o)
         return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

@@ -1202,6 +1202,20 @@ def greedy_workspace(rows: int, device) -> torch.Tensor:
     return torch.zeros(_lib.load().mui_greedy_workspace_bytes(int(rows)), dtype=torch.uint8, device=device)
 
 
+def take_rows(x: torch.Tensor, index: torch.Tensor) -> torch.Tensor:
+    """[len(index), w]: rows of x [n, w] by number, zeros for a number outside 0 .. n - 1 (-1: padding)."""
+    n, w = x.shape
+    row_bytes = w * x.element_size()
+    if x.is_cuda and index.device == x.device and index.dtype == torch.int64 and row_bytes and row_bytes % 16 == 0:
+        x, index = x.contiguous(), index.contiguous()
+        out = torch.empty((index.numel(), w), dtype=x.dtype, device=x.device)
+        if x.data_ptr() % 16 == 0:
+            check(_lib.load().mui_take_rows(_stream(x), x.data_ptr(), n, row_bytes, index.data_ptr(), out.data_ptr(), index.numel()), "mui_take_rows")
+            return out
+    live = (index >= 0) & (index < n)
+    return torch.where(live[:, None], x[index.clamp(0, max(n - 1, 0))], torch.zeros((), dtype=x.dtype, device=x.device))
+
+
 def fill_buffers(tensors: Sequence[torch.Tensor], values: Optional[Sequence[int]] = None) -> None:
     """Sets every tensor: int64 ones to values[i], any type to zero without values. Contiguous plain tensors of one GPU go in one
     launch; whatever else there is takes torch's own fill."""
