@@ -1180,90 +1180,96 @@ static int launch_prefill_xs(hipStream_t s, PrefillGemmParams p, int shares, voi
 
 // Gate/up whose 256 x 256 tiles (128 outputs each) end in a round that is at most half full: the
 // number of row tiles that make whole rounds of workgroups, for a launch of their own -- or 0
-static long gateup_bands(const PrefillGemmParams& p) {
+static long gateup_bands(const PrefillGemmParams& p, int tokens) {
   if (!g_prefill_bands) return 0;
   const long cus = device_cus();
-  const long tt = ceil_div(p.tokens, 256), row_tiles = ceil_div(p.n, 128);
+  const long tt = ceil_div(tokens, 256), row_tiles = ceil_div(p.n, 128);
   if (cus % tt != 0 || cus / tt < 2) return 0;
   const long per_round = cus / tt, whole_rows = row_tiles / per_round * per_round, rest = row_tiles - whole_rows;
   return (whole_rows > 0 && rest > 0 && 2 * rest <= per_round) ? whole_rows : 0;
 }
 
-template <typename T, int WF, int EPI>
-static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
-  // Big tiles re-read x and the weights least and keep the LDS traffic per matrix instruction
-  // low, but a grid much smaller than the chip leaves the work to too few CUs, and a grid of one
-  // and a bit rounds of workgroups costs two rounds. Each shape has a cost per round of
-  // workgroups (microseconds at K = 4096 on MI355X; only the ratios matter); the number of
-  // rounds the grid needs decides between them. Measured on the Llama-3-8B shapes: QKV at 1536
-  // tokens is 144 tiles of 256 x 256 (116 us) but 192 of 192 x 256 (92 us), at 2048 tokens 192
-  // (122 us) against 256 (99 us); o_proj and down at 2048 tokens are 128 tiles of 256 x 256 (112 / 363 us)
-  // and 256 of 128 x 256 (78 / 270 us); QKV at 512 is 192 tiles of 128 x 128 (68 us), 256 of
-  // 96 x 128 (62 us). Below three workgroups of 128 x 128 per four CUs: 64 x 128, then 32 x 64 (up
-  // to 256 tokens on the 4096-row matrices).
+// What it takes to multiply `tokens` tokens, in microseconds at K = 4096, and with which tile (see launch_prefill_t); 0 where no tile's cost was compared
+// Big tiles re-read x and the weights least and keep the LDS traffic per matrix instruction
+// low, but a grid much smaller than the chip leaves the work to too few CUs, and a grid of one
+// and a bit rounds of workgroups costs two rounds. Each shape has a cost per round of
+// workgroups (microseconds at K = 4096 on MI355X; only the ratios matter); the number of
+// rounds the grid needs decides between them. Measured on the Llama-3-8B shapes: QKV at 1536
+// tokens is 144 tiles of 256 x 256 (116 us) but 192 of 192 x 256 (92 us), at 2048 tokens 192
+// (122 us) against 256 (99 us); o_proj and down at 2048 tokens are 128 tiles of 256 x 256 (112 / 363 us)
+// and 256 of 128 x 256 (78 / 270 us); QKV at 512 is 192 tiles of 128 x 128 (68 us), 256 of
+// 96 x 128 (62 us). Below three workgroups of 128 x 128 per four CUs: 64 x 128, then 32 x 64 (up
+// to 256 tokens on the 4096-row matrices).
+static float prefill_plan(const PrefillGemmParams& p, int WF, int EPI, bool pipe, int tokens, int* chosen) {
   const long rows = (EPI == SK_GATEUP) ? 2L * p.n : p.n;
   const long cus = device_cus();
   const long want = 3L * cus / 4;
-  auto tiles = [&](int r, int tk) { return (long)ceil_div((int)rows, r) * ceil_div(p.tokens, tk); };
-  int which = g_prefill_tile;
-  if (which == 0) {
-    // few output tiles (short prompts on the 4096-row matrices): one workgroup per tile whose
-    // waves split every k-step between them -- four waves that each hold the whole 32 x 64 tile,
-    // or eight waves in two token halves of a 64 x 128 or 128 x 128 tile: the LDS traffic per
-    // matrix instruction of a larger tile, and enough waves per CU although the grid is a single
-    // round of workgroups (their 96-128 KB of LDS leave one per CU). 32 x 64 for up to 64 tokens
-    // on 8192 rows (o_proj at 128 tokens 21.7 vs 28.3 us, down 60 vs 91 us).
-    if (EPI == SK_LINEAR && tiles(32, 64) <= cus) which = 6;
-    // ... and 64 x 64 while that is still a single round: QKV at 128 tokens 33 -> 24.5 us, o_proj at
-    // 256 tokens 32 -> 23.5 us (k-steps of 128 instead of 256: 28.6 / 27.2 us)
-    else if (EPI == SK_LINEAR && tiles(64, 64) <= cus) which = 12;
-    else if (tiles(256, 256) >= 5 * cus / 8 || 2 * tiles(64, 128) > cus) {
-      // one workgroup per CU (eight waves): rounds x cost, a little more per round once the
-      // rounds follow each other (their weights compete for the L2)
-      auto whole = [&](long n_tiles, float one, float many) {
-        const long r = (n_tiles + cus - 1) / cus;
-        return (float)r * (r > 1 ? many : one);
-      };
-      // two workgroups per CU (four waves): up to `cus` tiles run one per CU, the next `cus` join them
-      auto pairs = [&](long n_tiles, float single, float twin) {
-        const long full = n_tiles / (2 * cus), rest = n_tiles % (2 * cus);
-        const float last = rest == 0 ? 0.f : rest <= cus ? single : single + (twin - single) * (float)(rest - cus) / (float)cus;
-        return (float)full * twin + last;
-      };
-      // (the three big tiles cost less per round where the software-pipelined loop serves them)
-      const bool pipe = kPipelined<T, WF> && !p.gamma && pipelined_loop_serves(p, WF);
-      const bool pipe8 = pipe && WF != WF_16BIT;  // (the conversion costs the loop a tenth)
-      float best = whole(tiles(256, 256), pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f);
-      which = 4;
-      // (gate/up in two launches, see below: whole rounds of 256 x 256 and one round of 128 x 256)
-      if constexpr (EPI == SK_GATEUP) {
-        if (pipe && gateup_bands(p) > 0) best = (float)((tiles(256, 256) + cus - 1) / cus - 1) * (pipe8 ? 109.f : 100.f) + (pipe8 ? 60.f : 53.f);
-      }
-      auto offer = [&](int id, float cost) {
-        if (cost < best * 0.97f) { best = cost; which = id; }  // bigger tiles win ties
-      };
-      if (pipe8 && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 81.f, 87.f));
-      else if (pipe && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 74.f, 80.f));
-      else if (pipe) offer(8, whole(tiles(192, 256), 92.f, 98.f));  // gate/up: twelve waves beside pipelined 256 x 256 and 128 x 256
-      else offer(8, whole(tiles(192, 256), 85.f, 92.f));
-      if (pipe8) offer(7, whole(tiles(128, 256), 60.f, 64.f));
-      else if (pipe) offer(7, whole(tiles(128, 256), 53.f, 58.f));  // (three LDS stages; 63 / 66 with two)
-      else offer(7, whole(tiles(128, 256), WF == WF_16BIT ? 67.f : 73.f, WF == WF_16BIT ? 70.f : 76.f));
-      offer(1, pairs(tiles(128, 128), 68.f, 92.f));
-      if (EPI == SK_LINEAR && WF == WF_16BIT) offer(10, pairs(tiles(96, 128), 60.f, 76.f));
-      // 128 x 128 on waves that split K: the fastest single tile (QKV at 512 tokens 43 vs 62 us,
-      // o_proj at 1024 44 vs 68 us, down at 1024 139 vs 219 us), one per CU
-      offer(9, whole(tiles(128, 128), 42.f, 40.f));
-      // the same with 64-token tiles: half the token bytes per workgroup for prompts of up to 64
-      // tokens (gate/up at 64 tokens 57 -> 50 us)
-      offer(11, whole(tiles(128, 64), 37.f, 36.5f));
-      // 64 x 128 likewise (o_proj at 512 tokens 32 us, down 99 us, QKV at 256 33 us; four waves
-      // that each held the whole tile took 40 / 118 / 41 us)
-      offer(5, whole(tiles(64, 128), 32.5f, 31.f));
-    } else {
-      which = (tiles(64, 128) >= want || EPI == SK_GATEUP) ? 2 : 3;
+  auto tiles = [&](int r, int tk) { return (long)ceil_div((int)rows, r) * ceil_div(tokens, tk); };
+  int which;
+  float best = 0.f;
+  // few output tiles (short prompts on the 4096-row matrices): one workgroup per tile whose
+  // waves split every k-step between them -- four waves that each hold the whole 32 x 64 tile,
+  // or eight waves in two token halves of a 64 x 128 or 128 x 128 tile: the LDS traffic per
+  // matrix instruction of a larger tile, and enough waves per CU although the grid is a single
+  // round of workgroups (their 96-128 KB of LDS leave one per CU). 32 x 64 for up to 64 tokens
+  // on 8192 rows (o_proj at 128 tokens 21.7 vs 28.3 us, down 60 vs 91 us).
+  if (EPI == SK_LINEAR && tiles(32, 64) <= cus) which = 6;
+  // ... and 64 x 64 while that is still a single round: QKV at 128 tokens 33 -> 24.5 us, o_proj at
+  // 256 tokens 32 -> 23.5 us (k-steps of 128 instead of 256: 28.6 / 27.2 us)
+  else if (EPI == SK_LINEAR && tiles(64, 64) <= cus) which = 12;
+  else if (tiles(256, 256) >= 5 * cus / 8 || 2 * tiles(64, 128) > cus) {
+    // one workgroup per CU (eight waves): rounds x cost, a little more per round once the
+    // rounds follow each other (their weights compete for the L2)
+    auto whole = [&](long n_tiles, float one, float many) {
+      const long r = (n_tiles + cus - 1) / cus;
+      return (float)r * (r > 1 ? many : one);
+    };
+    // two workgroups per CU (four waves): up to `cus` tiles run one per CU, the next `cus` join them
+    auto pairs = [&](long n_tiles, float single, float twin) {
+      const long full = n_tiles / (2 * cus), rest = n_tiles % (2 * cus);
+      const float last = rest == 0 ? 0.f : rest <= cus ? single : single + (twin - single) * (float)(rest - cus) / (float)cus;
+      return (float)full * twin + last;
+    };
+    // (the three big tiles cost less per round where the software-pipelined loop serves them)
+    const bool pipe8 = pipe && WF != WF_16BIT;  // (the conversion costs the loop a tenth)
+    best = whole(tiles(256, 256), pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f);
+    which = 4;
+    // (gate/up in two launches, see below: whole rounds of 256 x 256 and one round of 128 x 256)
+    if (EPI == SK_GATEUP) {
+      if (pipe && gateup_bands(p, tokens) > 0) best = (float)((tiles(256, 256) + cus - 1) / cus - 1) * (pipe8 ? 109.f : 100.f) + (pipe8 ? 60.f : 53.f);
     }
+    auto offer = [&](int id, float cost) {
+      if (cost < best * 0.97f) { best = cost; which = id; }  // bigger tiles win ties
+    };
+    if (pipe8 && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 81.f, 87.f));
+    else if (pipe && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 74.f, 80.f));
+    else if (pipe) offer(8, whole(tiles(192, 256), 92.f, 98.f));  // gate/up: twelve waves beside pipelined 256 x 256 and 128 x 256
+    else offer(8, whole(tiles(192, 256), 85.f, 92.f));
+    if (pipe8) offer(7, whole(tiles(128, 256), 60.f, 64.f));
+    else if (pipe) offer(7, whole(tiles(128, 256), 53.f, 58.f));  // (three LDS stages; 63 / 66 with two)
+    else offer(7, whole(tiles(128, 256), WF == WF_16BIT ? 67.f : 73.f, WF == WF_16BIT ? 70.f : 76.f));
+    offer(1, pairs(tiles(128, 128), 68.f, 92.f));
+    if (EPI == SK_LINEAR && WF == WF_16BIT) offer(10, pairs(tiles(96, 128), 60.f, 76.f));
+    // 128 x 128 on waves that split K: the fastest single tile (QKV at 512 tokens 43 vs 62 us,
+    // o_proj at 1024 44 vs 68 us, down at 1024 139 vs 219 us), one per CU
+    offer(9, whole(tiles(128, 128), 42.f, 40.f));
+    // the same with 64-token tiles: half the token bytes per workgroup for prompts of up to 64
+    // tokens (gate/up at 64 tokens 57 -> 50 us)
+    offer(11, whole(tiles(128, 64), 37.f, 36.5f));
+    // 64 x 128 likewise (o_proj at 512 tokens 32 us, down 99 us, QKV at 256 33 us; four waves
+    // that each held the whole tile took 40 / 118 / 41 us)
+    offer(5, whole(tiles(64, 128), 32.5f, 31.f));
+  } else {
+    which = (tiles(64, 128) >= want || EPI == SK_GATEUP) ? 2 : 3;
   }
+  *chosen = which;
+  return best;
+}
+
+template <typename T, int WF, int EPI>
+static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
+  int which = g_prefill_tile;
+  if (which == 0) prefill_plan(p, WF, EPI, kPipelined<T, WF> && !p.gamma && pipelined_loop_serves(p, WF), p.tokens, &which);
   // Where the software-pipelined eight-wave loop does not apply (fused norm, int8 weights, K not a
   // multiple of 64): sixteen waves per workgroup (four per SIMD, at most 128 registers each) on all
   // but the smallest shapes, with the compiler's own schedule 3-16 % ahead of eight waves with twice
@@ -1292,7 +1298,7 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
     // one, a round of the small tile two thirds of it).
     if (g_prefill_tile == 0 && which == 4 && !p.gamma && pipelined_loop_serves(p, WF)) {
       {
-        const long whole_rows = gateup_bands(p);
+        const long whole_rows = gateup_bands(p, p.tokens);
         if (whole_rows > 0) {
           PrefillGemmParams a = p, b = p;
           a.n = (int)(whole_rows * 128);
@@ -1379,6 +1385,23 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
   }
 }
 
+// Gate/up whose last token tiles hold few tokens: the number of tokens to leave to a launch of their own, for whole 256-token tiles in front of it -- or 0. 520
+// tokens of 14336 x 4096 are 336 tiles of 256 x 256 where 512 are 224, one round of workgroups; the weights of the few are read again instead, by the kernels
+// that stream them (16-bit ones find much of them in the last cache, int8 has 14 us of tiles' ramp whatever K is). Taken where it gains 7 % by the plan, whose
+// rounds of the big tiles are up to a tenth dear. us, one launch / two: 14336 x 4096 bf16, 520 / 640 / 1032 / 1152 / 1544 / 1664 tokens 167 / 140, 170 / 148,
+// 271 / 230, 275 / 243, 362 / 325, 369 / 341; 8192 x 2048, 520 / 1032 / 1152 / 2056 / 2176 52 / 49, 91 / 71, 91 / 79, 156 / 126, 157 / 134; int8 per channel
+// 14336 x 4096 (fp16), 520 / 640 / 1032 / 1544 197 / 149, 192 / 156, 299 / 250, 393 / 353; 8192 x 2048, 1032 / 2176 106 / 85, 172 / 150 (520 would be 56 / 61).
+static int gateup_rest(const PrefillGemmParams& p, int wf, bool pipelined) {
+  const int rest = p.tokens % 256;
+  if (!g_prefill_bands || !pipelined || p.tokens < 512 || rest == 0 || rest > 128) return 0;
+  int which = 0;
+  const float together = prefill_plan(p, wf, SK_GATEUP, true, p.tokens, &which), whole = prefill_plan(p, wf, SK_GATEUP, true, p.tokens - rest, &which);
+  if (together <= 0.f || whole <= 0.f) return 0;
+  const float per_weight = wf == WF_16BIT ? (rest <= 32 ? 28.f : rest <= 64 ? 36.f : 46.f) : rest <= 64 ? 25.f : 38.f;
+  const float few = (wf == WF_16BIT ? 12.f : 14.f * 4096.f / (float)p.k) + (float)p.n / 14336.f * per_weight;
+  return whole + few < 0.93f * together ? rest : 0;
+}
+
 constexpr int kWideDefaultMaxTokens = 0;  // 0: the built-in rule below
 static int g_wide_max_tokens = kWideDefaultMaxTokens;  // longest prompt taken by gemm_wide.hip
 
@@ -1421,6 +1444,19 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   if (wf == WF_U8_GROUP && (q.group_shift < 4 || (q.k & ((1 << q.group_shift) - 1)))) return MUI_ERR_UNSUPPORTED;
   if (q.k % (wf == WF_16BIT ? 8 : 16)) return MUI_ERR_UNSUPPORTED;
   if (q.x_pitch != 0 && q.x_pitch != q.k) return MUI_ERR_UNSUPPORTED;
+  if (epilogue == SK_GATEUP && g_prefill_tile == 0 && !q.gamma) {
+    const bool pipelined = (dtype == MUI_DTYPE_F16 || wf != WF_U8_GROUP) && pipelined_loop_serves(p, wf);
+    const int rest = gateup_rest(p, wf, pipelined);
+    if (rest) {
+      SkinnyParams a = q, b = q;
+      a.tokens = q.tokens - rest;
+      b.tokens = rest;
+      b.x = q.x + (long)a.tokens * q.k;
+      b.y = q.y + (long)a.tokens * q.n;
+      const int st = launch_prefill_gemm(s, dtype, wf, epilogue, a);
+      return st != MUI_OK ? st : launch_prefill_gemm(s, dtype, wf, epilogue, b);
+    }
+  }
 #define MUI_PF_CASE(TT, WFV, EPIV) \
   if (dtype == TT::kDtype && wf == WFV && epilogue == EPIV) return launch_prefill_t<TT, WFV, EPIV>(s, p);
   MUI_PF_CASE(F16, WF_16BIT, SK_LINEAR)
