@@ -74,8 +74,8 @@ int mui_tune_skinny(int min_tokens, int stream_b, int multi_max_tokens);
  * keep their sixteen / twelve waves. 400 + tile: the software-pipelined tiles are launched as one
  * workgroup per tile instead of a persistent round of workgroups. 800 + tile: an XCD's workgroups
  * walk one row tile after another instead of panels of four row tiles (1600 + tile: panels of
- * eight, 2400 + tile: of two). 3200 + tile: gate/up stays one launch whatever its last round of
- * tiles holds. 6400 / 12800 / 19200 + tile: the XCDs divide the tile grid 8 x 1 / 4 x 2 / 2 x 4 ways
+ * eight, 2400 + tile: of two). 3200 + tile: a product stays one launch whatever its last round of
+ * tiles or its last tokens hold. 6400 / 12800 / 19200 + tile: the XCDs divide the tile grid 8 x 1 / 4 x 2 / 2 x 4 ways
  * (rows x tokens) instead of the launcher's choice. 25600 + tile: the software-pipelined 128 x 256 tile
  * keeps two LDS stages instead of three. 51200 + tile: the software-pipelined 192 x 256 and 256 x 256 tiles
  * keep two stages of the weight tile instead of three. The offsets add up (e.g. 1204 = 800 + 400 + 4).

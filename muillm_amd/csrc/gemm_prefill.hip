@@ -168,7 +168,13 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   // one k-range of x for all row tiles)
   const int xs_share = XS ? (int)(vb % (unsigned)p.k_splits) : 0;
   const int xs_tile = XS ? (int)(vb / (unsigned)p.k_splits) : 0;
-  const int xcd = vb & 7, slot = vb >> 3;
+  const int xcd = vb & 7;
+  int slot = vb >> 3, piece = 0;
+  if (p.sub_rows) {
+    const int per_tile = p.sub_rows * p.sub_toks;
+    piece = slot % per_tile;
+    slot = p.first_slot + slot / per_tile;
+  }
   // The eight XCDs (each with an L2 of its own) divide the tile grid p.row_split ways by rows and
   // 8 / p.row_split ways by tokens, interleaved: what every XCD fetches is its share of the weights
   // and its share of x, and the split that fetches least depends on which of the two is bigger (the
@@ -191,6 +197,11 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
     tile_t = (w / rows_here) * ts + xt;
   }
   if (tile_n >= p.n_tiles || tile_t >= p.t_tiles) return;  // uniform for the workgroup, before any barrier
+  if (p.sub_rows) {
+    tile_n = tile_n * p.sub_rows + piece % p.sub_rows;
+    tile_t = tile_t * p.sub_toks + piece / p.sub_rows;
+    if (tile_n * OUT_TILE >= p.n || tile_t * TOKS >= p.tokens) return;
+  }
   const int o0 = tile_n * OUT_TILE;  // first output of the tile
   const int t0 = tile_t * TOKS;      // first token of the tile
 
@@ -1043,7 +1054,7 @@ static int g_prefill_pipe_small = 1;  // experiments: the pipelined loop on the 
 static int g_prefill_dma = 1;   // 0: operand tiles staged through registers everywhere
 static int g_prefill_row_group = 4;   // row tiles per panel of an XCD's tile walk (experiments: 1 = one row tile after another)
 static int g_prefill_row_split = 0;   // experiments: 8, 4 or 2 forces the XCDs' split of the grid (0: the launcher's choice)
-static int g_prefill_bands = 1;       // experiments: 0 keeps gate/up in one launch whatever its last round holds
+static int g_prefill_bands = 1;       // experiments: 0 keeps a product in one launch whatever its last round or its last tokens hold
 static int g_prefill_persistent = 1;  // experiments: 0 launches one workgroup per tile on the pipelined tiles too
 static int g_prefill_stages3_big = 1;  // experiments: 0 keeps the pipelined 192 x 256 and 256 x 256 tiles on two stages of both tiles
 static int g_prefill_stages3 = 1;     // experiments: 0 keeps the pipelined 128 x 256 tile on two LDS stages
@@ -1062,11 +1073,10 @@ static bool lds_direct_loads_serve(const PrefillGemmParams& p, int wf) {
 }
 static bool pipelined_loop_serves(const PrefillGemmParams& p, int wf) { return lds_direct_loads_serve(p, wf); }
 
-template <typename T, int WF, int EPI, int WR, int WT, int NWR, int NWT, int NWK, int KS, int NBUF, bool PIPE = false>
-static int launch_prefill_cfg(hipStream_t s, PrefillGemmParams p) {
-  constexpr int ROWS = 16 * WR * NWR, TOKS = 16 * WT * NWT;
-  p.n_tiles = ceil_div(p.n, EPI == SK_GATEUP ? ROWS / 2 : ROWS);
-  p.t_tiles = ceil_div(p.tokens, TOKS);
+// Tiles of `outputs` outputs x `toks` tokens and how the XCDs divide them; returns the slots of an XCD
+static long prefill_tiles(PrefillGemmParams& p, int wf, int epi, int outputs, int toks) {
+  p.n_tiles = ceil_div(p.n, outputs);
+  p.t_tiles = ceil_div(p.tokens, toks);
   // The XCDs' split of the grid: rows alone (8 x 1), or 4 x 2 / 2 x 4 rows x tokens where that cuts
   // the bytes the eight L2s fetch between them -- weights x token splits + x x row splits -- by a
   // fifth or more (down 4096 x 14336 at 4096 tokens: 0.70 instead of 1.06 GB; gate/up keeps 8 x 1).
@@ -1074,15 +1084,23 @@ static int launch_prefill_cfg(hipStream_t s, PrefillGemmParams p) {
   if (g_prefill_row_split) {
     p.row_split = g_prefill_row_split;
   } else {
-    const double wb = (double)(EPI == SK_GATEUP ? 2 : 1) * p.n * p.k * (WF == WF_16BIT ? 2 : 1), xb = (double)p.tokens * p.k * 2;
+    const double wb = (double)(epi == SK_GATEUP ? 2 : 1) * p.n * p.k * (wf == WF_16BIT ? 2 : 1), xb = (double)p.tokens * p.k * 2;
     double best = wb + 8 * xb;
     for (int rs = 4; rs >= 2; rs /= 2) {
       const double c = wb * (8 / rs) + xb * rs;
       if (c < 0.8 * best && p.t_tiles >= 8 / rs * 4 && p.n_tiles >= rs * 4) { best = c; p.row_split = rs; }
     }
   }
+  p.row_group = g_prefill_row_group;
   // every XCD gets the same number of slots: its share rounded up, the surplus exits
-  const long grid = (long)ceil_div(p.n_tiles, p.row_split) * ceil_div(p.t_tiles, 8 / p.row_split) * 8;
+  return (long)ceil_div(p.n_tiles, p.row_split) * ceil_div(p.t_tiles, 8 / p.row_split);
+}
+
+template <typename T, int WF, int EPI, int WR, int WT, int NWR, int NWT, int NWK, int KS, int NBUF, bool PIPE = false>
+static int launch_prefill_cfg(hipStream_t s, PrefillGemmParams p) {
+  constexpr int ROWS = 16 * WR * NWR, TOKS = 16 * WT * NWT;
+  const long all = p.sub_rows ? p.slots : prefill_tiles(p, WF, EPI, EPI == SK_GATEUP ? ROWS / 2 : ROWS, TOKS);
+  const long grid = (p.slots ? p.slots : all) * 8;
   if (grid > 0x7fffffffL) return MUI_ERR_UNSUPPORTED;
   constexpr size_t lds = PIPE && WF != WF_16BIT ? pipe8_lds_bytes<WF, ROWS, TOKS, KS, NBUF>()
                          : PIPE ? pipe_lds_bytes<ROWS, TOKS, KS, NBUF>() : prefill_lds_bytes<ROWS, TOKS, KS, NBUF>();
@@ -1108,7 +1126,6 @@ static int launch_prefill_cfg(hipStream_t s, PrefillGemmParams p) {
     return launch_status();
   };
   p.total_blocks = (int)grid;
-  p.row_group = g_prefill_row_group;
   if constexpr (!PIPE) {
     if (p.gamma) return launch(prefill_gemm_kernel<T, WF, true, EPI, WR, WT, NWR, NWT, NWK, KS, NBUF>);
   }
@@ -1178,15 +1195,12 @@ static int launch_prefill_xs(hipStream_t s, PrefillGemmParams p, int shares, voi
   return launch_status();
 }
 
-// Gate/up whose 256 x 256 tiles (128 outputs each) end in a round that is at most half full: the
-// number of row tiles that make whole rounds of workgroups, for a launch of their own -- or 0
-static long gateup_bands(const PrefillGemmParams& p, int tokens) {
-  if (!g_prefill_bands) return 0;
-  const long cus = device_cus();
-  const long tt = ceil_div(tokens, 256), row_tiles = ceil_div(p.n, 128);
-  if (cus % tt != 0 || cus / tt < 2) return 0;
-  const long per_round = cus / tt, whole_rows = row_tiles / per_round * per_round, rest = row_tiles - whole_rows;
-  return (whole_rows > 0 && rest > 0 && 2 * rest <= per_round) ? whole_rows : 0;
+// What a tile shape does with its last round of workgroups (see launch_prefill_t): by how many tiles a CU's XCD has left, of a round of `per`
+enum LastRound { kLastWhole, kLastHalves, kLastQuarters };
+static LastRound last_round(long slots, int per) {
+  const long rest = slots % per;
+  if (!g_prefill_bands || slots <= per || rest == 0 || 2 * rest > per) return kLastWhole;
+  return 4 * rest <= per ? kLastQuarters : kLastHalves;
 }
 
 // What it takes to multiply `tokens` tokens, in microseconds at K = 4096, and with which tile (see launch_prefill_t); 0 where no tile's cost was compared
@@ -1200,7 +1214,8 @@ static long gateup_bands(const PrefillGemmParams& p, int tokens) {
 // and 256 of 128 x 256 (78 / 270 us); QKV at 512 is 192 tiles of 128 x 128 (68 us), 256 of
 // 96 x 128 (62 us). Below three workgroups of 128 x 128 per four CUs: 64 x 128, then 32 x 64 (up
 // to 256 tokens on the 4096-row matrices).
-static float prefill_plan(const PrefillGemmParams& p, int WF, int EPI, bool pipe, int tokens, int* chosen) {
+static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int tokens, int* chosen) {
+  p.tokens = tokens;
   const long rows = (EPI == SK_GATEUP) ? 2L * p.n : p.n;
   const long cus = device_cus();
   const long want = 3L * cus / 4;
@@ -1232,12 +1247,19 @@ static float prefill_plan(const PrefillGemmParams& p, int WF, int EPI, bool pipe
     };
     // (the three big tiles cost less per round where the software-pipelined loop serves them)
     const bool pipe8 = pipe && WF != WF_16BIT;  // (the conversion costs the loop a tenth)
-    best = whole(tiles(256, 256), pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f);
+    // (and their last round goes to smaller tiles where it is at most half full. A launch of its own for it costs a linear more: its big tiles end on time of
+    // their own, 107 us at K = 4096 where the plan has 96, and the 192 x 256 tile is close behind: 6144 x 4096 at 3500 tokens 174 us with quarters, 159 on that)
+    const float second = (EPI == SK_GATEUP ? 8.f : 28.f) * 4096.f / (float)p.k;
+    auto rounds = [&](int r, int tk, float one, float many, float halves, float quarters) {
+      if (!pipe) return whole(tiles(r, tk), one, many);
+      const int per = (int)(cus / 8);
+      const long slots = prefill_tiles(p, WF, EPI, EPI == SK_GATEUP ? r / 2 : r, tk);
+      const LastRound last = last_round(slots, per);
+      const long n = last == kLastWhole ? (slots + per - 1) / per : slots / per;
+      return (float)n * (n > 1 ? many : one) + (last == kLastWhole ? 0.f : second + (last == kLastHalves ? halves : quarters));
+    };
+    best = rounds(256, 256, pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f, pipe8 ? 60.f : 53.f, 42.f);
     which = 4;
-    // (gate/up in two launches, see below: whole rounds of 256 x 256 and one round of 128 x 256)
-    if (EPI == SK_GATEUP) {
-      if (pipe && gateup_bands(p, tokens) > 0) best = (float)((tiles(256, 256) + cus - 1) / cus - 1) * (pipe8 ? 109.f : 100.f) + (pipe8 ? 60.f : 53.f);
-    }
     auto offer = [&](int id, float cost) {
       if (cost < best * 0.97f) { best = cost; which = id; }  // bigger tiles win ties
     };
@@ -1245,8 +1267,8 @@ static float prefill_plan(const PrefillGemmParams& p, int WF, int EPI, bool pipe
     else if (pipe && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 74.f, 80.f));
     else if (pipe) offer(8, whole(tiles(192, 256), 92.f, 98.f));  // gate/up: twelve waves beside pipelined 256 x 256 and 128 x 256
     else offer(8, whole(tiles(192, 256), 85.f, 92.f));
-    if (pipe8) offer(7, whole(tiles(128, 256), 60.f, 64.f));
-    else if (pipe) offer(7, whole(tiles(128, 256), 53.f, 58.f));  // (three LDS stages; 63 / 66 with two)
+    if (pipe8) offer(7, rounds(128, 256, 60.f, 64.f, 42.f, 32.5f));
+    else if (pipe) offer(7, rounds(128, 256, 53.f, 58.f, 42.f, 32.5f));  // (three LDS stages; 63 / 66 with two)
     else offer(7, whole(tiles(128, 256), WF == WF_16BIT ? 67.f : 73.f, WF == WF_16BIT ? 70.f : 76.f));
     offer(1, pairs(tiles(128, 128), 68.f, 92.f));
     if (EPI == SK_LINEAR && WF == WF_16BIT) offer(10, pairs(tiles(96, 128), 60.f, 76.f));
@@ -1291,43 +1313,40 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
     }
     return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 3, true>(s, q);
   };
-  if constexpr (EPI == SK_GATEUP) {
-    // Gate/up whose 256 x 256 tiles end in a round that is at most half full (2048 tokens: 896 tiles
-    // = 3.5 rounds of 256 CUs): the outputs of the whole rounds in one launch, the rest as one round
-    // of 128 x 256 tiles in a second one (a half-empty round of the big tile costs as much as a full
-    // one, a round of the small tile two thirds of it).
-    if (g_prefill_tile == 0 && which == 4 && !p.gamma && pipelined_loop_serves(p, WF)) {
-      {
-        const long whole_rows = gateup_bands(p, p.tokens);
-        if (whole_rows > 0) {
-          PrefillGemmParams a = p, b = p;
-          a.n = (int)(whole_rows * 128);
-          b.n = p.n - a.n;
-          b.w0 += (long)a.n * p.pitch;
-          b.w1 += (long)a.n * p.pitch;
-          b.y += a.n;
-          if (p.add_bias) {
-            b.add_bias += a.n;
-            b.mul_bias += a.n;
-          }
-          if (WF != WF_16BIT) {
-            b.s0 += (long)a.n * p.s_pitch;
-            b.s1 += (long)a.n * p.s_pitch;
-          }
-          int st = pipe_256(a);
-          if (st == MUI_OK) st = pipe_128(b);
-          if (st != MUI_ERR_UNSUPPORTED) return st;
-        }
-      }
-    }
-  }
+  auto ksplit_128 = [&](const PrefillGemmParams& q) { return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 2, 4, 128, 2>(s, q); };  // 128 x 128, 2 x 2 waves x 4 shares of K
+  auto ksplit_64 = [&](const PrefillGemmParams& q) {  // 64 x 128: 2 x 2 waves x 4 shares of K; int8: 2 token halves
+    if constexpr (WF == WF_16BIT) return launch_prefill_cfg<T, WF, EPI, 2, 4, 2, 2, 4, 128, 2>(s, q);
+    else return launch_prefill_cfg<T, WF, EPI, 4, 4, 1, 2, 4, 128, 2>(s, q);
+  };
+  // The big tiles run in rounds of one workgroup per CU, and a last round that holds a tile for every eighth CU takes as long as a full one. At most half
+  // full it is a launch of its own: of halves of the tiles, or, for a quarter of the CUs, of quarters, on the tiles that do those in one short round. us, one
+  // launch / two: gate/up 14336 x 4096 bf16, 768 / 1280 / 1792 / 3500 tokens 167 / 159, 268 / 245, 369 / 338, 660 / 633; 8192 x 2048, 1280 / 2304 / 4352 87 / 82,
+  // 152 / 137, 254 / 241; linear 4096 x 14336, 4352 / 5120 / 6144 512 / 464, 525 / 487, 592 / 544.
+  auto in_rounds = [&](auto& big, int rows, auto& halves, auto& quarters) {
+    PrefillGemmParams a = p;
+    const int per = device_cus() / 8;
+    const long slots = prefill_tiles(a, WF, EPI, EPI == SK_GATEUP ? rows / 2 : rows, 256);
+    const LastRound last = g_prefill_tile == 0 && slots < 0x7fffffffL ? last_round(slots, per) : kLastWhole;
+    if (last == kLastWhole || p.gamma || !pipelined_loop_serves(p, WF)) return big(p);
+    const int rest = (int)(slots % per);
+    PrefillGemmParams b = a;
+    a.slots = (int)slots - rest;
+    const int st = big(a);
+    if (st != MUI_OK) return st;
+    b.first_slot = a.slots;
+    // (256 x 256: halves are 128 x 256; 128 x 256: they are 128 x 128)
+    b.sub_rows = rows == 256 || last == kLastQuarters ? 2 : 1;
+    b.sub_toks = rows == 128 || last == kLastQuarters ? 2 : 1;
+    b.slots = rest * b.sub_rows * b.sub_toks;
+    return last == kLastHalves ? halves(b) : quarters(b);
+  };
   {
     // 256 x 256 on 4 x 2 waves of 64 x 128 with two operand register sets (the software-pipelined
     // loop): where its loads can go straight into LDS it is 5-8 % ahead of the sixteen waves below
     // (gate/up at 4096 tokens 775 -> 736 us, down 386 -> 356 us, QKV 224 -> 209 us, down at 2048
     // tokens 345 -> 315 us; bit-equal results: the same products in the same order)
     if (which == 4 && !p.gamma) {
-      const int st = pipe_256(p);
+      const int st = in_rounds(pipe_256, 256, pipe_128, ksplit_128);
       if (st != MUI_ERR_UNSUPPORTED) return st;
     }
   }
@@ -1336,7 +1355,7 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
     if (g_prefill_pipe_small && !p.gamma) {
       int st = MUI_ERR_UNSUPPORTED;
       // 128 x 256, 2 x 4 waves of 64 x 64, three LDS stages
-      if (which == 7) st = pipe_128(p);
+      if (which == 7) st = in_rounds(pipe_128, 128, ksplit_128, ksplit_64);
       if constexpr (EPI == SK_LINEAR) {
         // 192 x 256, 4 x 2 waves of 48 x 128
         if (which == 8) {
@@ -1356,16 +1375,15 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
   if (which == 8) return launch_prefill_cfg<T, WF, EPI, 4, 4, 3, 4, 1, 64, 2>(s, p);
   if constexpr (WF == WF_16BIT) {
     if (which == 7) return launch_prefill_cfg<T, WF, EPI, 2, 4, 4, 4, 1, 64, 2>(s, p);    // 128 x 256, 4 x 4 waves of 32 x 64
-    if (which == 5) return launch_prefill_cfg<T, WF, EPI, 2, 4, 2, 2, 4, 128, 2>(s, p);   // 64 x 128, 2 x 2 waves x 4 shares of K
     if constexpr (EPI == SK_LINEAR) {
       if (which == 10) return launch_prefill_cfg<T, WF, EPI, 3, 4, 2, 2, 1, 64, 2>(s, p);  // 96 x 128, 2 x 2 waves of 48 x 64
     }
   }
   if (which == 10) which = 1;  // int8 weights, gate/up
   if (which == 7) return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 2>(s, p);      // 128 x 256, 2 x 4 waves of 64 x 64
-  if (which == 9) return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 2, 4, 128, 2>(s, p);     // 128 x 128, 2 x 2 waves x 4 shares of K
+  if (which == 9) return ksplit_128(p);
   if (which == 11) return launch_prefill_cfg<T, WF, EPI, 2, 4, 4, 1, 4, 128, 2>(s, p);    // 128 x 64, 4 x 1 waves x 4 shares of K
-  if (which == 5) return launch_prefill_cfg<T, WF, EPI, 4, 4, 1, 2, 4, 128, 2>(s, p);     // 64 x 128, 2 token halves x 4 shares of K
+  if (which == 5) return ksplit_64(p);
   if constexpr (EPI == SK_LINEAR && WF == WF_16BIT) {
     // 32 x 64 on eight waves (2 row halves x 4 shares of K): QKV at 64 tokens 21.7 -> 20.7 us, o_proj 20.2 -> 19.1 us
     if (which == 6) return launch_prefill_cfg<T, WF, EPI, 1, 4, 2, 1, 4, 256, 2>(s, p);
@@ -1385,21 +1403,29 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
   }
 }
 
-// Gate/up whose last token tiles hold few tokens: the number of tokens to leave to a launch of their own, for whole 256-token tiles in front of it -- or 0. 520
-// tokens of 14336 x 4096 are 336 tiles of 256 x 256 where 512 are 224, one round of workgroups; the weights of the few are read again instead, by the kernels
-// that stream them (16-bit ones find much of them in the last cache, int8 has 14 us of tiles' ramp whatever K is). Taken where it gains 7 % by the plan, whose
-// rounds of the big tiles are up to a tenth dear. us, one launch / two: 14336 x 4096 bf16, 520 / 640 / 1032 / 1152 / 1544 / 1664 tokens 167 / 140, 170 / 148,
-// 271 / 230, 275 / 243, 362 / 325, 369 / 341; 8192 x 2048, 520 / 1032 / 1152 / 2056 / 2176 52 / 49, 91 / 71, 91 / 79, 156 / 126, 157 / 134; int8 per channel
-// 14336 x 4096 (fp16), 520 / 640 / 1032 / 1544 197 / 149, 192 / 156, 299 / 250, 393 / 353; 8192 x 2048, 1032 / 2176 106 / 85, 172 / 150 (520 would be 56 / 61).
-static int gateup_rest(const PrefillGemmParams& p, int wf, bool pipelined) {
+// Products whose last token tiles hold few tokens: the number of tokens to leave to a launch of their own, for whole 256-token tiles in front of it -- or 0. 520
+// tokens of a 14336 x 4096 gate/up are 336 tiles of 256 x 256 where 512 are 224, one round of workgroups; the weights of the few are read again instead, by the
+// kernels that stream them (16-bit ones find some of them in the last cache; int8 rows have 16 us of ramp whatever K is). Taken where the plan says that it gains, of
+// linears, whose big tiles cost less than planned where they leave CUs idle, 15 % and only from 2048 tokens on. us, one launch / two: gate/up 14336 x 4096 bf16, 520 / 640
+// / 1032 / 1152 / 1544 / 1664 tokens 165 / 146, 165 / 145, 262 / 224, 265 / 241, 361 / 314, 367 / 336; 8192 x 2048, 520 / 1032 / 1152 / 2056 49 / 47, 84 / 70, 86 / 75,
+// 147 / 124; int8 per channel 14336 x 4096 (fp16), 520 / 1032 / 1152 191 / 159, 293 / 239, 297 / 268; linears 4096 x 14336, 2056 / 4104 253 / 216, 478 / 365; 4096 x 4096
+// 84 / 73, 153 / 121; not taken: int8 gate/up 8192 x 2048 at 520 53 / 59, linear 2048 x 8192 at 2056 86 / 89, 4096 x 14336 at 520 117 / 124.
+static int rest_tokens(const PrefillGemmParams& p, int wf, int epi, bool pipelined) {
   const int rest = p.tokens % 256;
-  if (!g_prefill_bands || !pipelined || p.tokens < 512 || rest == 0 || rest > 128) return 0;
+  if (!g_prefill_bands || !pipelined || p.tokens < (epi == SK_GATEUP ? 512 : 2048) || rest == 0 || rest > 128) return 0;
   int which = 0;
-  const float together = prefill_plan(p, wf, SK_GATEUP, true, p.tokens, &which), whole = prefill_plan(p, wf, SK_GATEUP, true, p.tokens - rest, &which);
+  const float together = prefill_plan(p, wf, epi, true, p.tokens, &which), whole = prefill_plan(p, wf, epi, true, p.tokens - rest, &which);
   if (together <= 0.f || whole <= 0.f) return 0;
-  const float per_weight = wf == WF_16BIT ? (rest <= 32 ? 28.f : rest <= 64 ? 36.f : 46.f) : rest <= 64 ? 25.f : 38.f;
-  const float few = (wf == WF_16BIT ? 12.f : 14.f * 4096.f / (float)p.k) + (float)p.n / 14336.f * per_weight;
-  return whole + few < 0.93f * together ? rest : 0;
+  const float per_k = 4096.f / (float)p.k;
+  float few;
+  if (epi == SK_GATEUP) {
+    const float per_weight = wf == WF_16BIT ? (rest <= 32 ? 28.f : rest <= 64 ? 36.f : 46.f) : rest <= 64 ? 25.f : 38.f;
+    few = (wf == WF_16BIT ? 6.f + 6.f * per_k : 16.f * per_k) + (float)p.n / 14336.f * per_weight;
+  } else {
+    const float per_weight = wf == WF_16BIT ? (rest <= 16 ? 3.f : rest <= 32 ? 5.5f : rest <= 64 ? 8.f : 12.5f) : 14.f;
+    few = (wf == WF_16BIT ? 5.f : 8.f) * per_k + (float)p.n / 4096.f * per_weight;
+  }
+  return whole + few < (epi == SK_GATEUP ? 0.985f : 0.85f) * together ? rest : 0;
 }
 
 constexpr int kWideDefaultMaxTokens = 0;  // 0: the built-in rule below
@@ -1444,15 +1470,16 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   if (wf == WF_U8_GROUP && (q.group_shift < 4 || (q.k & ((1 << q.group_shift) - 1)))) return MUI_ERR_UNSUPPORTED;
   if (q.k % (wf == WF_16BIT ? 8 : 16)) return MUI_ERR_UNSUPPORTED;
   if (q.x_pitch != 0 && q.x_pitch != q.k) return MUI_ERR_UNSUPPORTED;
-  if (epilogue == SK_GATEUP && g_prefill_tile == 0 && !q.gamma) {
+  if (g_prefill_tile == 0 && !q.gamma) {
     const bool pipelined = (dtype == MUI_DTYPE_F16 || wf != WF_U8_GROUP) && pipelined_loop_serves(p, wf);
-    const int rest = gateup_rest(p, wf, pipelined);
+    const int rest = rest_tokens(p, wf, epilogue, pipelined);
     if (rest) {
       SkinnyParams a = q, b = q;
       a.tokens = q.tokens - rest;
       b.tokens = rest;
       b.x = q.x + (long)a.tokens * q.k;
       b.y = q.y + (long)a.tokens * q.n;
+      if (q.residual) b.residual = q.residual + (long)a.tokens * q.n;
       const int st = launch_prefill_gemm(s, dtype, wf, epilogue, a);
       return st != MUI_OK ? st : launch_prefill_gemm(s, dtype, wf, epilogue, b);
     }
@@ -1488,7 +1515,7 @@ extern "C" int mui_tune_prefill(int tile, int wide_max_tokens) {
   if (tile >= 25600) tile -= 25600;
   const int row_split = tile >= 19200 ? 2 : tile >= 12800 ? 4 : tile >= 6400 ? 8 : 0;
   if (tile >= 6400) tile -= tile >= 19200 ? 19200 : tile >= 12800 ? 12800 : 6400;
-  // 3200 + tile: gate/up stays one launch whatever its last round of tiles holds
+  // 3200 + tile: a product stays one launch whatever its last round of tiles or its last tokens hold
   const int bands = tile >= 3200 ? 0 : 1;
   if (tile >= 3200) tile -= 3200;
   // 800 + tile: an XCD walks one row tile after another; 1600 + tile / 2400 + tile: panels of 8 / 2 row tiles

@@ -57,7 +57,10 @@ struct PrefillGemmParams {
   int k_splits;
   int row_split;          // the XCDs divide the tile grid row_split ways by rows, 8 / row_split ways by tokens
   int row_group;          // row tiles per panel of an XCD's tile walk
-  int total_blocks;       // software-pipelined tiles: tiles of the launch (row tiles rounded up to 8, times token tiles)
+  int total_blocks;       // software-pipelined tiles: tiles of the launch (slots of an XCD, times 8)
+  int slots;              // tiles that each XCD takes (0: all of its share)
+  int first_slot;         // sub_rows > 0: the launch takes what another one's larger tiles left, from this slot on, every tile of it as
+  int sub_rows, sub_toks; // sub_rows x sub_toks smaller ones; n_tiles to row_group are the other launch's
   float* part;            // [tiles * k_splits] partial tiles in fp32
   unsigned* part_count;   // [tiles], zero between launches
 };
