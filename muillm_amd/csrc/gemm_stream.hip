@@ -17,7 +17,7 @@
 //
 // us at 32 tokens in bf16, tiled GEMM or 16-rows-per-workgroup kernel -> here: 6144 x 4096 20.7 -> 12.7, 4096 x 4096 15.0 -> 10.9,
 // gate/up 14336 x 4096 42.6 -> 37.4, 4096 x 14336 47 -> 24.2, 2048 x 8192 25.8 -> 11.7, 128256 x 4096 226 -> 167; at 101
-// tokens 24.3 -> 20.6, 19.6 -> 17.2, (gate/up stays on the tiled GEMM beyond 64 tokens), 49.3 -> 33.9, 33.2 -> 18.6.
+// tokens 24.3 -> 20.6, 19.6 -> 17.2, 49.3 -> 33.9, 33.2 -> 18.6, gate/up 8192 x 2048 (80 tokens) 22.9 -> 18.4.
 #include "skinny.cuh"
 
 namespace mui {
@@ -318,14 +318,16 @@ static int launch_stream_cfg(hipStream_t s, const StreamParams& p) {
 // token tiles of 16 per unit
 static int stream_token_tiles(int tokens) { return tokens <= 32 ? 2 : tokens <= 64 ? 4 : tokens <= 96 ? 6 : 8; }
 constexpr int stream_widest(int nt) { return 192 - 16 * nt < 128 ? 192 - 16 * nt : 128; }  // rows with three stages of 128 k-values
+template <int EPI>
+constexpr bool stream_built(int rows, int nt) { return rows <= stream_widest(nt) && (EPI == SK_LINEAR || nt <= 4 || rows == 48 || rows == 64); }
 
 template <typename T, int EPI, int ROWS>
 static int launch_stream_rows(hipStream_t s, const StreamParams& p) {
   switch (stream_token_tiles(p.tokens)) {
     case 2: return launch_stream_cfg<T, EPI, ROWS, 2>(s, p);
     case 4: return launch_stream_cfg<T, EPI, ROWS, 4>(s, p);
-    case 6: if constexpr (EPI == SK_LINEAR && ROWS <= stream_widest(6)) return launch_stream_cfg<T, EPI, ROWS, 6>(s, p); break;
-    default: if constexpr (EPI == SK_LINEAR && ROWS <= stream_widest(8)) return launch_stream_cfg<T, EPI, ROWS, 8>(s, p); break;
+    case 6: if constexpr (stream_built<EPI>(ROWS, 6)) return launch_stream_cfg<T, EPI, ROWS, 6>(s, p); break;
+    default: if constexpr (stream_built<EPI>(ROWS, 8)) return launch_stream_cfg<T, EPI, ROWS, 8>(s, p); break;
   }
   return MUI_ERR_UNSUPPORTED;
 }
@@ -362,8 +364,12 @@ static bool wide_is_faster(int tokens, int rows, int k) {
 // are slower beyond 32 tokens, but for rows that are whole multiples of 4 KB apart, which slows the tiles (us at 33 to 64 tokens, tiles / units: 14400 to 15600 outputs, K 512 12.5 to 14.1 / 12.6 to 14.2, 1024
 // 17.5 to 18.9 / 18.0 to 20.0, 2048 28.8 to 35 / 29 to 31, 4096 48 to 59 / 48 to 55, 5120 57 to 60 / 63 to 69, 8192 87 to 117 / 98 to 106; 30000 outputs, K 512 23 to 24 / 22 to 23, 4096
 // 93 to 114 / 96 to 105, 5120 111 to 125 / 124 to 144, 8192 183 to 222 / 182 to 189); elsewhere units take 0.63 to 1.02 of the tiles' time.
-static bool gateup_tiles_are_faster(int tokens, int rows, int k) {
+// Beyond 64 tokens units have 48 or 64 rows (what three stages leave room for): one round of those up to 16384 rows, us, tiles / units at 65 / 96 / 128 tokens: 8192 x 2048
+// 20.5 / 17.5, 22.4 / 19.4, 22.3 / 21.1, 8192 x 4096 33.7 / 28.7, 34.7 / 30.5, 36.7 / 34.3, 6144 x 4096 31.1 / 25.4, 32.1 / 26.7, 33.9 / 30.2, 4096 x 2048 29.4 / 14.9, 30.3 /
+// 15.6, 31.3 / 17.4. Two rounds read the tokens twice: 14336 x 4096 at 128 tokens 64 us, tiles 55.
+static bool gateup_tiles_are_faster(int tokens, int rows, int k, int units) {
   const int cus = device_cus();
+  if (tokens > 64) return units > cus;
   return tokens > 32 && k > 512 && k % 2048 && ceil_div(rows, 112 * cus) > ceil_div(rows, 128 * cus);
 }
 
@@ -383,7 +389,7 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int
   int width = 0;
   for (int c = 0; c < tried; ++c) {
     const int r = EPI == SK_GATEUP ? kGateup[c] : kLinear[c];
-    if (r > stream_widest(nt) || (g_stream_rows && r != g_stream_rows)) continue;
+    if (!stream_built<EPI>(r, nt) || (g_stream_rows && r != g_stream_rows)) continue;
     const int units = ceil_div(rows, r);
     for (int k = 1; k <= 8; ++k) {
       if (k > 1 && ((long)units * k > cus || (size_t)k * p.tokens * p.n * 4 > part_bytes || p.k / 256 < 2 * k)) break;
@@ -398,9 +404,9 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int
   if (!p.add && p.k_splits == 1) return MUI_ERR_UNSUPPORTED;
   if (splits) *splits = p.k_splits;
   if (!forced && EPI == SK_LINEAR && wide_is_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
-  if (forced && !width) return MUI_ERR_INVALID_ARG;
+  if (forced && !width) return EPI == SK_GATEUP && nt > 4 ? MUI_ERR_UNSUPPORTED : MUI_ERR_INVALID_ARG;
   if (!forced && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
-  if (!forced && EPI == SK_GATEUP && gateup_tiles_are_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
+  if (!forced && EPI == SK_GATEUP && gateup_tiles_are_faster(p.tokens, rows, p.k, p.n_units)) return MUI_ERR_UNSUPPORTED;
   switch (width) {
     case 16: return launch_stream_rows<T, EPI, 16>(s, p);
     case 32: return launch_stream_rows<T, EPI, 32>(s, p);
@@ -437,12 +443,10 @@ static StreamParams stream_params(const SkinnyParams& q, float* part, bool add) 
   return p;
 }
 
-// 17..128 tokens (gate/up ..64), 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve and for
+// 17..128 tokens, 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve and for
 // what another kernel does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
-  // gate/up beyond 64 tokens: the tiled GEMM. Units of six and eight token tiles are built for linears only; for gate/up they were measured at 128 tokens and
-  // 14336 x 4096 alone (64 us, tiles 55), between 65 and 127 not at all (tiles: 51 us at 65 tokens, 54 at 101)
-  if (!stream_serves(q, epilogue == SK_GATEUP ? 64 : 128)) return MUI_ERR_UNSUPPORTED;
+  if (!stream_serves(q, 128)) return MUI_ERR_UNSUPPORTED;
   const StreamParams p = stream_params(q, part, true);
   if (dtype == MUI_DTYPE_F16) return epilogue == SK_GATEUP ? launch_stream_t<F16, SK_GATEUP>(s, p, 0) : launch_stream_t<F16, SK_LINEAR>(s, p, part_bytes);
   if (dtype == MUI_DTYPE_BF16) return epilogue == SK_GATEUP ? launch_stream_t<BF16, SK_GATEUP>(s, p, 0) : launch_stream_t<BF16, SK_LINEAR>(s, p, part_bytes);

@@ -203,7 +203,7 @@ size_t prefill_workspace_bytes();  // what SkinnyParams::workspace must hold for
 size_t prefill_counter_bytes();    // of that, at its start: counters that stay zero
 // 17..128 tokens: 16 weight rows per workgroup, K split over its waves, token columns in up to 8 MFMA tiles (gemm_wide.hip)
 int launch_gemm_wide(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
-// 17..128 tokens (gate/up ..64), 16-bit weights, k % 256 == 0, n % 8 == 0, no fused norm: bands of weight rows streamed through LDS stages that
+// 17..128 tokens, 16-bit weights, k % 256 == 0, n % 8 == 0, no fused norm: bands of weight rows streamed through LDS stages that
 // the workgroup shares; part (part_bytes, may be none): fp32 partial outputs where shares of K are worth it (gemm_stream.hip). MUI_ERR_UNSUPPORTED
 // for everything else and for what the tiled GEMM does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);
