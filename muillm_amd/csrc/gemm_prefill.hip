@@ -1212,13 +1212,11 @@ static LastRound last_round(long slots, int per) {
 // tokens is 144 tiles of 256 x 256 (116 us) but 192 of 192 x 256 (92 us), at 2048 tokens 192
 // (122 us) against 256 (99 us); o_proj and down at 2048 tokens are 128 tiles of 256 x 256 (112 / 363 us)
 // and 256 of 128 x 256 (78 / 270 us); QKV at 512 is 192 tiles of 128 x 128 (68 us), 256 of
-// 96 x 128 (62 us). Below three workgroups of 128 x 128 per four CUs: 64 x 128, then 32 x 64 (up
-// to 256 tokens on the 4096-row matrices).
+// 96 x 128 (62 us). Where 64 x 128 tiles number half the CUs at most, tiles whose waves split K.
 static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int tokens, int* chosen) {
   p.tokens = tokens;
   const long rows = (EPI == SK_GATEUP) ? 2L * p.n : p.n;
   const long cus = device_cus();
-  const long want = 3L * cus / 4;
   auto tiles = [&](int r, int tk) { return (long)ceil_div((int)rows, r) * ceil_div(tokens, tk); };
   int which;
   float best = 0.f;
@@ -1282,7 +1280,9 @@ static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int t
     // that each held the whole tile took 40 / 118 / 41 us)
     offer(5, whole(tiles(64, 128), 32.5f, 31.f));
   } else {
-    which = (tiles(64, 128) >= want || EPI == SK_GATEUP) ? 2 : 3;
+    // gate/up of few rows: 64 x 128 whose waves split K, as above (int8, us at 17 / 64 / 128 tokens, waves that each hold the whole K / this: 2 x 4096 rows x 2048
+    // 29.2 / 21.8, 31.2 / 21.3, 32.1 / 21.9, x 4096 54.7 / 34.7, 55.7 / 35.1, 57.7 / 35.2, x 8192 104 / 63, 105 / 63, 109 / 64)
+    which = EPI == SK_GATEUP ? 5 : 3;
   }
   *chosen = which;
   return best;
