@@ -166,7 +166,7 @@ def test_a_class_of_its_own_is_not_asked():
     assert RealRows.of(lm, mask, DEV) is None
 
 
-@pytest.mark.parametrize("tokens,padding,hidden,worth", [(128, 100, 4096, False), (129, 15, 4096, True), (129, 14, 4096, False), (768, 200, 2048, True), (768, 50, 2048, False)])
+@pytest.mark.parametrize("tokens,padding,hidden,worth", [(128, 100, 4096, False), (129, 68, 4096, True), (129, 67, 4096, False), (768, 269, 2048, True), (768, 268, 2048, False)])
 def test_where_it_is_worth_it(monkeypatch, tokens, padding, hidden, worth):
     monkeypatch.undo()
     lm = _lm()
