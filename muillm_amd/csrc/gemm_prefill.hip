@@ -1405,11 +1405,11 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
 
 // Products whose last token tiles hold few tokens: the number of tokens to leave to a launch of their own, for whole 256-token tiles in front of it -- or 0. 520
 // tokens of a 14336 x 4096 gate/up are 336 tiles of 256 x 256 where 512 are 224, one round of workgroups; the weights of the few are read again instead, by the
-// kernels that stream them (16-bit ones find some of them in the last cache; int8 rows have 16 us of ramp whatever K is). Taken where the plan says that it gains, of
+// kernels that stream them (16-bit ones find some of them in the last cache; int8 beyond 64 tokens, on tiles, has 16 us of ramp whatever K is). Taken where the plan says that it gains, of
 // linears, whose big tiles cost less than planned where they leave CUs idle, 15 % and only from 2048 tokens on. us, one launch / two: gate/up 14336 x 4096 bf16, 520 / 640
 // / 1032 / 1152 / 1544 / 1664 tokens 165 / 146, 165 / 145, 262 / 224, 265 / 241, 361 / 314, 367 / 336; 8192 x 2048, 520 / 1032 / 1152 / 2056 49 / 47, 84 / 70, 86 / 75,
-// 147 / 124; int8 per channel 14336 x 4096 (fp16), 520 / 1032 / 1152 191 / 159, 293 / 239, 297 / 268; linears 4096 x 14336, 2056 / 4104 253 / 216, 478 / 365; 4096 x 4096
-// 84 / 73, 153 / 121; not taken: int8 gate/up 8192 x 2048 at 520 53 / 59, linear 2048 x 8192 at 2056 86 / 89, 4096 x 14336 at 520 117 / 124.
+// 147 / 124; int8 per channel 14336 x 4096 (fp16), 520 / 1032 / 1100 180 / 130, 286 / 225, 289 / 256; linears 4096 x 14336, 2056 / 4104 253 / 216, 478 / 365; 4096 x 4096
+// 84 / 73, 153 / 121; not taken: linear 2048 x 8192 at 2056 86 / 89, 4096 x 14336 at 520 117 / 124.
 static int rest_tokens(const PrefillGemmParams& p, int wf, int epi, bool pipelined) {
   const int rest = p.tokens % 256;
   if (!g_prefill_bands || !pipelined || p.tokens < (epi == SK_GATEUP ? 512 : 2048) || rest == 0 || rest > 128) return 0;
@@ -1419,11 +1419,11 @@ static int rest_tokens(const PrefillGemmParams& p, int wf, int epi, bool pipelin
   const float per_k = 4096.f / (float)p.k;
   float few;
   if (epi == SK_GATEUP) {
-    const float per_weight = wf == WF_16BIT ? (rest <= 32 ? 28.f : rest <= 64 ? 36.f : 46.f) : rest <= 64 ? 25.f : 38.f;
-    few = (wf == WF_16BIT ? 6.f + 6.f * per_k : 16.f * per_k) + (float)p.n / 14336.f * per_weight;
+    const float per_weight = wf == WF_16BIT ? (rest <= 32 ? 28.f : rest <= 64 ? 36.f : 46.f) : rest > 64 ? 38.f : wf == WF_I8_CHANNEL && rest <= 32 ? 22.f : 35.f;
+    few = (wf == WF_16BIT ? 6.f + 6.f * per_k : (rest <= 64 ? 6.f : 16.f) * per_k) + (float)p.n / 14336.f * per_weight;
   } else {
-    const float per_weight = wf == WF_16BIT ? (rest <= 16 ? 3.f : rest <= 32 ? 5.5f : rest <= 64 ? 8.f : 12.5f) : 14.f;
-    few = (wf == WF_16BIT ? 5.f : 8.f) * per_k + (float)p.n / 4096.f * per_weight;
+    const float per_weight = wf == WF_16BIT ? (rest <= 16 ? 3.f : rest <= 32 ? 5.5f : rest <= 64 ? 8.f : 12.5f) : rest <= 64 ? 8.f : 14.f;
+    few = (wf == WF_16BIT ? 5.f : rest <= 64 ? 6.f : 8.f) * per_k + (float)p.n / 4096.f * per_weight;
   }
   return whole + few < (epi == SK_GATEUP ? 0.985f : 0.85f) * together ? rest : 0;
 }
@@ -1435,8 +1435,8 @@ static int g_wide_max_tokens = kWideDefaultMaxTokens;  // longest prompt taken b
 // int8 codes; SkinnyParams as for the decode kernels (x, residual and y dense).
 int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const SkinnyParams& q) {
   if (q.tokens < 1 || q.n < 1 || q.k < 1) return MUI_ERR_INVALID_ARG;
-  // up to 128 tokens are bound by the weight stream. 16-bit weights: gemm_stream.hip, which takes rows of whole 256-value steps.
-  // What it declines and int8 codes: up to 40 tokens 16 rows per workgroup, K split over the waves, no LDS tiling
+  // up to 128 tokens (codes: 64) are bound by the weight stream: gemm_stream.hip, which takes rows of whole 256-value steps.
+  // What it declines: up to 40 tokens 16 rows per workgroup, K split over the waves, no LDS tiling
   // (gemm_wide.hip), while its grid is a single round of workgroups (o_proj at 33 tokens 16.0 vs 20.4 us for the smallest LDS
   // tile, 19.6 vs 20.6 at 48, 23.1 vs 21.2 at 64)
   PrefillGemmParams p = {};
@@ -1446,9 +1446,10 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   p.x = q.x; p.gamma = q.gamma; p.mul_bias = q.mul_bias; p.add_bias = q.add_bias; p.residual = q.residual;
   p.y = q.y; p.y_pitch = q.n; p.n = q.n; p.k = q.k; p.tokens = q.tokens; p.eps = q.eps;
   const bool scratch = q.workspace && ((uintptr_t)q.workspace & 255u) == 0 && q.workspace_bytes >= prefill_workspace_bytes();
-  if (wf == WF_16BIT && q.tokens <= 128 && g_prefill_tile == 0 && g_wide_max_tokens == kWideDefaultMaxTokens) {
-    const int st = launch_gemm_stream(s, dtype, epilogue, q, scratch ? (float*)((char*)q.workspace + kXsCounterBytes) : nullptr,
-                                      scratch ? q.workspace_bytes - kXsCounterBytes : 0);
+  if (q.tokens <= 128 && g_prefill_tile == 0 && g_wide_max_tokens == kWideDefaultMaxTokens) {
+    float* part = scratch ? (float*)((char*)q.workspace + kXsCounterBytes) : nullptr;
+    const size_t part_bytes = scratch ? q.workspace_bytes - kXsCounterBytes : 0;
+    const int st = wf == WF_16BIT ? launch_gemm_stream(s, dtype, epilogue, q, part, part_bytes) : launch_gemm_stream_int8(s, dtype, wf, epilogue, q, part, part_bytes);
     if (st != MUI_ERR_UNSUPPORTED) return st;
   }
   // a caller-provided workspace lets a long K be shared between workgroups when the tiles are few

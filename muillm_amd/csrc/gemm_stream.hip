@@ -1,4 +1,4 @@
-// Linear layers of 16-bit weights for 17..128 tokens (batched decoding beyond 16 rows, short prompts).
+// Linear layers for 17..128 tokens (batched decoding beyond 16 rows, short prompts); of int8 codes for 17..64.
 //
 // Bound by the weight stream, and by the tokens: a matrix is read once, but every workgroup reads all token rows again from L2.
 // A CU's vector cache returns data in the order of the requests, whichever wave made them, and holds a few tens of KB of them:
@@ -15,6 +15,9 @@
 // tiles; the shares' partial tiles meet in LDS at the end of a unit and are added in order. A workgroup takes the units blockIdx,
 // blockIdx + grid, ...; the stages run on across units, so the next unit is on its way while the last one is added up.
 //
+// int8 codes lie in the stages as they are, half the bytes; a lane reads sixteen of a row at a time (their k-values are two of a token's chunks) and converts them for two
+// matrix instructions. A scale per row is applied to the sums; the pairs of the group format, one per row and share, are part of the stage, and the weight is rounded to 16 bits.
+//
 // us at 32 tokens in bf16, tiled GEMM or 16-rows-per-workgroup kernel -> here: 6144 x 4096 20.7 -> 12.7, 4096 x 4096 15.0 -> 10.9,
 // gate/up 14336 x 4096 42.6 -> 37.4, 4096 x 14336 47 -> 24.2, 2048 x 8192 25.8 -> 11.7, 128256 x 4096 226 -> 167; at 101
 // tokens 24.3 -> 20.6, 19.6 -> 17.2, 49.3 -> 33.9, 33.2 -> 18.6, gate/up 8192 x 2048 (80 tokens) 22.9 -> 18.4.
@@ -27,6 +30,7 @@ constexpr int kStreamThreads = kStreamWaves * kWave;
 
 struct StreamParams {
   const uint8_t* w0; const uint8_t* w1; long pitch;  // bytes
+  const uint16_t* s0; const uint16_t* s1; long s_pitch; int group_shift;  // codes: as in SkinnyParams
   const uint16_t* x;
   const uint16_t* mul_bias; const uint16_t* add_bias; const uint16_t* residual;
   uint16_t* y;
@@ -38,26 +42,31 @@ struct StreamParams {
 };
 
 // Geometry for ROWS weight rows x NT token tiles of 16 per unit
-template <int ROWS, int NT>
+template <int ROWS, int NT, int WF>
 struct StreamShape {
-  static constexpr int KS = ROWS + 16 * NT <= 96 ? 256 : 128;     // k-values per step: at least three stages fit
+  static constexpr bool W8 = WF != WF_16BIT;  // codes
+  static constexpr int KS = W8 || ROWS + 16 * NT <= 96 ? 256 : 128;  // k-values per step: at least three stages fit
   static constexpr int KSH = KS / 64;                              // shares of a step
   static constexpr int RT = (ROWS + 15) / 16;
   static constexpr int GROUPS = kStreamWaves / KSH;
-  static constexpr int GT = NT == 2 ? 2 : NT == 6 ? 3 : GROUPS;    // groups of token tiles (six tiles: two waves only load)
+  // groups of token tiles (six tiles: two waves only load). Codes are converted by every group, so there is one where there are row tiles to deal out
+  static constexpr int GT = W8 && RT > 1 ? 1 : NT == 2 ? 2 : NT == 6 ? 3 : GROUPS;
   static constexpr int GR = GROUPS / GT;                           // groups of row tiles
   static constexpr int TW = NT / GT, RW = (RT + GR - 1) / GR;      // token and row tiles per wave
-  static constexpr int RPI = 512 / KS;                             // rows per load instruction (1 KB)
-  static constexpr int W_INSTR = ROWS / RPI, INSTR = (ROWS + 16 * NT) / RPI;
+  static constexpr int RPI = 512 / KS, WRPI = W8 ? 2 * RPI : RPI;  // token and weight rows per load instruction (1 KB)
+  static constexpr int W_INSTR = ROWS / WRPI, X_INSTR = 16 * NT / RPI, P_INSTR = WF == WF_U8_GROUP ? RT : 0, INSTR = W_INSTR + X_INSTR + P_INSTR;
+  static constexpr int ROW_BYTES = KS * 2, WROW_BYTES = W8 ? KS : KS * 2;
   static constexpr int Q = (INSTR + kStreamWaves - 1) / kStreamWaves;  // load instructions per wave and step (at most)
   static constexpr int FULL = INSTR - (Q - 1) * kStreamWaves;      // waves that have Q of them, the others Q - 1
-  static constexpr int STAGE = (ROWS + 16 * NT) * KS * 2;
-  static constexpr int MEET = RT * NT < 16 / KSH ? RT * NT : 16 / KSH;  // tiles that meet at a time (KSH KB each)
+  static constexpr int PAIRS = ROWS * WROW_BYTES + 16 * NT * ROW_BYTES;  // where a stage's (scale, min) pairs are: one per row and share
+  static constexpr int STAGE = PAIRS + P_INSTR * 256;
+  static constexpr int MOST_MEET = WF == WF_U8_GROUP && NT == 4 ? 3 : 16 / KSH;  // (three stages and what meets have to fit)
+  static constexpr int MEET = RT * NT < MOST_MEET ? RT * NT : MOST_MEET;  // tiles that meet at a time (KSH KB each)
   static constexpr int FIT = (160 * 1024 - MEET * KSH * 1024) / STAGE;
   static constexpr int S = FIT < 8 ? FIT : 8;
   static constexpr int LDS = S * STAGE + MEET * KSH * 1024;
   // row tiles read past the weights' rows (a half tile's other half, a last row group's spare tile) read token rows of the stage
-  static_assert(GR * RW * 16 <= ROWS + 16 * NT, "a wave's rows lie in its stage");
+  static_assert(GR * RW * 16 * WROW_BYTES <= STAGE, "a wave's rows lie in its stage");
   static_assert(S >= 3 && (S - 2) * Q <= 63 && ROWS % 8 == 0 && TW * GT == NT && GR >= 1, "shape");
 };
 
@@ -81,12 +90,13 @@ __device__ __forceinline__ void stream_wait_steps(int steps) {
   }
 }
 
-template <typename T, int EPI, int ROWS, int NT>
+template <typename T, int EPI, int ROWS, int NT, int WF>
 __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const StreamParams p) {
-  using G = StreamShape<ROWS, NT>;
-  constexpr int KS = G::KS, KSH = G::KSH, RT = G::RT, TW = G::TW, RW = G::RW, RPI = G::RPI, S = G::S, MEET = G::MEET;
-  constexpr int CPR = KS / 8;  // 16-byte chunks per row of a stage
-  constexpr int ROW_BYTES = KS * 2;
+  using G = StreamShape<ROWS, NT, WF>;
+  constexpr bool W8 = G::W8;
+  constexpr int KS = G::KS, KSH = G::KSH, RT = G::RT, TW = G::TW, RW = G::RW, RPI = G::RPI, WRPI = G::WRPI, S = G::S, MEET = G::MEET;
+  constexpr int CPR = KS / 8, WCPR = W8 ? KS / 16 : CPR;  // 16-byte chunks per row of a stage
+  constexpr int ROW_BYTES = G::ROW_BYTES, WROW_BYTES = G::WROW_BYTES;
   const int t = threadIdx.x, lane = t & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   f32x4* meet = (f32x4*)(st_smem + S * G::STAGE);
@@ -94,6 +104,7 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
   // this lane's place in a load instruction: row lr of RPI, chunk ls. Chunk c of row r lives in slot c ^ (r % 16) (16 rows
   // read at one chunk fall into 16 different bank groups); the row's upper bits come with the instruction.
   const int lr = lane / CPR, ls = (lane % CPR) ^ lr;
+  const int wlr = W8 ? lane / WCPR : lr, wls = W8 ? (lane % WCPR) ^ wlr : ls;
 
   const int all_steps = p.k / KS;
   const int share_k = p.k_splits > 1 ? (int)(blockIdx.x % (unsigned)p.k_splits) : 0;
@@ -110,42 +121,55 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
   int lu = first_unit, lc = 0, lslot = 0;
   auto load_next = [&]() {
     const int turned = lc + turn < unit_steps ? lc + turn : lc + turn - unit_steps;
-    const long kb = (long)(sb + turned) * ROW_BYTES;
+    const long kb = (long)(sb + turned) * ROW_BYTES, kbw = W8 ? kb / 2 : kb;
     const int row0 = lu * ROWS;
     unsigned char* stage = st_smem + lslot * G::STAGE;
 #pragma unroll
     for (int q = 0; q < G::Q; ++q) {
       const int i = q * kStreamWaves + wave;
       if (q == G::Q - 1 && G::FULL < kStreamWaves && wave >= G::FULL) continue;
-      const int r = i * RPI;  // rows r .. r + RPI of the stage
       if (i < G::W_INSTR) {
+        const int r = i * WRPI;  // weight rows r .. r + WRPI of the stage
         const uint8_t* base;
         if constexpr (EPI == SK_GATEUP) {  // a tile of 16 rows: eight gate rows, then the up rows of the same outputs
           int o = (row0 >> 1) + (r >> 4) * 8 + (r & 7);
-          o = o < p.n - RPI ? o : p.n - RPI;  // (past the matrix: rows that are there, never stored)
+          o = o < p.n - WRPI ? o : p.n - WRPI;  // (past the matrix: rows that are there, never stored)
           base = ((r & 8) ? p.w1 : p.w0) + (long)o * p.pitch;
         } else {
-          const int o = row0 + r < p.n - RPI ? row0 + r : p.n - RPI;
+          const int o = row0 + r < p.n - WRPI ? row0 + r : p.n - WRPI;
           base = p.w0 + (long)o * p.pitch;
         }
-        stream_load16<2>(base + kb, (unsigned)(lr * (unsigned)p.pitch) + (unsigned)((ls ^ (r & 15)) * 16), stage + r * ROW_BYTES);  // non-temporal
+        stream_load16<2>(base + kbw, (unsigned)(wlr * (unsigned)p.pitch) + (unsigned)((wls ^ (r & 15)) * 16), stage + r * WROW_BYTES);  // non-temporal
+      } else if (G::P_INSTR > 0 && i >= G::W_INSTR + G::X_INSTR) {
+        // pairs of a tile of 16 rows: lane 4 row + share
+        const int tile = i - G::W_INSTR - G::X_INSTR, tr = lane >> 2;
+        int o;
+        if constexpr (EPI == SK_GATEUP) o = (row0 >> 1) + tile * 8 + (tr & 7);
+        else o = row0 + tile * 16 + tr;
+        o = o < p.n ? o : p.n - 1;
+        const long at = (long)o * p.s_pitch + 2 * (((sb + turned) * KS + (lane & 3) * 64) >> p.group_shift);
+        const uint16_t* pair = (EPI == SK_GATEUP && (tr & 8) ? p.s1 : p.s0) + at;
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)pair,
+                                         (__attribute__((address_space(3))) void*)(stage + G::PAIRS + tile * 256), 4, 0, 0);
       } else {
-        const int tr = r - ROWS;  // tokens past the end read the last one
+        const int tr = (i - G::W_INSTR) * RPI;  // tokens past the end read the last one
         const int rb = tr < p.tokens ? tr : p.tokens - 1, most = p.tokens - 1 - rb;
         const int tk = lr < most ? lr : most;
         stream_load16<0>((const uint8_t*)p.x + (long)rb * p.k * 2 + kb, (unsigned)(tk * p.k * 2) + (unsigned)((ls ^ (tr & 15)) * 16),
-                         stage + r * ROW_BYTES);
+                         stage + ROWS * WROW_BYTES + tr * ROW_BYTES);
       }
     }
     lslot = lslot + 1 == S ? 0 : lslot + 1;
     if (++lc == unit_steps) { lc = 0; lu += (int)gridDim.x; }
   };
 
-  // operand reads: lane l takes row l % 16 of a tile, chunk 8 share + l / 16 (+ 4)
+  // operand reads: lane l takes row l % 16 of a tile, chunk 8 share + l / 16 (+ 4); int8: the 16 codes of chunk 4 share + l / 16 and the tokens' two chunks of the
+  // same k-values
   const int share = wave % KSH, group = wave / KSH;
   const int gt = group % G::GT, gr = group / G::GT;
-  const int rr = lane & 15, rc = share * 8 + (lane >> 4);
-  const int ro0 = rr * ROW_BYTES + ((rc ^ rr) * 16), ro1 = rr * ROW_BYTES + (((rc + 4) ^ rr) * 16);
+  const int rr = lane & 15, rc = share * 8 + (W8 ? 2 * (lane >> 4) : lane >> 4);
+  const int ro0 = rr * ROW_BYTES + ((rc ^ rr) * 16), ro1 = rr * ROW_BYTES + (((rc + (W8 ? 1 : 4)) ^ rr) * 16);
+  const int wo = rr * WROW_BYTES + (((share * 4 + (lane >> 4)) ^ rr) * 16);
   const bool multiplies = gr < G::GR;
 
   f32x4 acc[RW][TW];
@@ -165,8 +189,8 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
     asm volatile("" ::: "memory");
     if (S - 1 < left) load_next();
     if (multiplies) {
-      const unsigned char* ws = st_smem + slot * G::STAGE + gr * RW * 16 * ROW_BYTES;
-      const unsigned char* xs = st_smem + slot * G::STAGE + (ROWS + gt * TW * 16) * ROW_BYTES;
+      const unsigned char* ws = st_smem + slot * G::STAGE + gr * RW * 16 * WROW_BYTES;
+      const unsigned char* xs = st_smem + slot * G::STAGE + ROWS * WROW_BYTES + gt * TW * 16 * ROW_BYTES;
       u32x4 b[TW][2];
 #pragma unroll
       for (int j = 0; j < TW; ++j) {
@@ -175,7 +199,26 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
       }
 #pragma unroll
       for (int i = 0; i < RW; ++i) {
-        const u32x4 a0 = *(const u32x4*)(ws + i * 16 * ROW_BYTES + ro0), a1 = *(const u32x4*)(ws + i * 16 * ROW_BYTES + ro1);
+        u32x4 a0, a1;
+        if constexpr (W8) {
+          const u32x4 codes = *(const u32x4*)(ws + i * 16 * WROW_BYTES + wo);
+          if constexpr (WF == WF_U8_GROUP) {
+            const uint32_t pair = *(const uint32_t*)(st_smem + slot * G::STAGE + G::PAIRS + ((gr * RW + i) * 16 + rr) * 16 + share * 4);
+            if constexpr (T::kDtype == MUI_DTYPE_F16) {
+              a0 = convert_a_pair_f16(codes.x, codes.y, pair);
+              a1 = convert_a_pair_f16(codes.z, codes.w, pair);
+            } else {
+              a0 = convert_a_pair<T>(codes.x, codes.y, pair);
+              a1 = convert_a_pair<T>(codes.z, codes.w, pair);
+            }
+          } else {
+            a0 = convert_a<T, WF_I8_CHANNEL>(codes.x, codes.y, nullptr, 0, 0);
+            a1 = convert_a<T, WF_I8_CHANNEL>(codes.z, codes.w, nullptr, 0, 0);
+          }
+        } else {
+          a0 = *(const u32x4*)(ws + i * 16 * ROW_BYTES + ro0);
+          a1 = *(const u32x4*)(ws + i * 16 * ROW_BYTES + ro1);
+        }
 #pragma unroll
         for (int j = 0; j < TW; ++j) {
           acc[i][j] = mfma16x16x32<T>(a0, b[j][0], acc[i][j]);
@@ -227,6 +270,10 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               float gv = g[e], uv = h[e];
+              if constexpr (WF == WF_I8_CHANNEL) {
+                gv *= T::one(p.s0[(o + e) * p.s_pitch]);
+                uv *= T::one(p.s1[(o + e) * p.s_pitch]);
+              }
               if (p.add_bias) {
                 gv += T::one(p.add_bias[o + e]);
                 uv += T::one(p.mul_bias[o + e]);
@@ -244,6 +291,10 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
 #pragma unroll
           for (int w = 1; w < KSH; ++w) a += in[w * 64 + lane];
           if (tok < p.tokens && o < p.n && 16 * i + 4 * sub < ROWS) {
+            if constexpr (WF == WF_I8_CHANNEL) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) a[e] *= T::one(p.s0[(o + e) * p.s_pitch]);
+            }
             if (p.k_splits > 1) {
               *(f32x4*)(p.part + ((long)share_k * p.tokens + tok) * p.n + o) = a;
             } else {
@@ -303,12 +354,12 @@ __global__ void __launch_bounds__(256) gemm_stream_add_kernel(const StreamParams
   *(u32x2*)(p.y + at) = pk;
 }
 
-template <typename T, int EPI, int ROWS, int NT>
+template <typename T, int EPI, int ROWS, int NT, int WF>
 static int launch_stream_cfg(hipStream_t s, const StreamParams& p) {
-  using G = StreamShape<ROWS, NT>;
+  using G = StreamShape<ROWS, NT, WF>;
   static_assert(G::LDS <= 160 * 1024, "LDS of a workgroup");
   const int cus = device_cus(), wgs = p.n_units * p.k_splits;
-  const int st = launch_with_lds(gemm_stream_kernel<T, EPI, ROWS, NT>, dim3(wgs < cus ? wgs : cus), dim3(kStreamThreads), G::LDS, s, p);
+  const int st = launch_with_lds(gemm_stream_kernel<T, EPI, ROWS, NT, WF>, dim3(wgs < cus ? wgs : cus), dim3(kStreamThreads), G::LDS, s, p);
   if (st != MUI_OK || p.k_splits == 1 || !p.add) return st;
   const long threads = (long)p.tokens * p.n / 4;
   hipLaunchKernelGGL(gemm_stream_add_kernel<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p);
@@ -318,16 +369,19 @@ static int launch_stream_cfg(hipStream_t s, const StreamParams& p) {
 // token tiles of 16 per unit
 static int stream_token_tiles(int tokens) { return tokens <= 32 ? 2 : tokens <= 64 ? 4 : tokens <= 96 ? 6 : 8; }
 constexpr int stream_widest(int nt) { return 192 - 16 * nt < 128 ? 192 - 16 * nt : 128; }  // rows with three stages of 128 k-values
-template <int EPI>
-constexpr bool stream_built(int rows, int nt) { return rows <= stream_widest(nt) && (EPI == SK_LINEAR || nt <= 4 || rows == 48 || rows == 64); }
+template <int EPI, int WF>
+constexpr bool stream_built(int rows, int nt) {
+  if (WF != WF_16BIT) return nt == 2 ? rows <= 112 : nt == 4 && rows <= 64;  // (three stages of 256 k-values)
+  return rows <= stream_widest(nt) && (EPI == SK_LINEAR || nt <= 4 || rows == 48 || rows == 64);
+}
 
-template <typename T, int EPI, int ROWS>
+template <typename T, int EPI, int ROWS, int WF>
 static int launch_stream_rows(hipStream_t s, const StreamParams& p) {
   switch (stream_token_tiles(p.tokens)) {
-    case 2: return launch_stream_cfg<T, EPI, ROWS, 2>(s, p);
-    case 4: return launch_stream_cfg<T, EPI, ROWS, 4>(s, p);
-    case 6: if constexpr (stream_built<EPI>(ROWS, 6)) return launch_stream_cfg<T, EPI, ROWS, 6>(s, p); break;
-    default: if constexpr (stream_built<EPI>(ROWS, 8)) return launch_stream_cfg<T, EPI, ROWS, 8>(s, p); break;
+    case 2: if constexpr (stream_built<EPI, WF>(ROWS, 2)) return launch_stream_cfg<T, EPI, ROWS, 2, WF>(s, p); break;
+    case 4: if constexpr (stream_built<EPI, WF>(ROWS, 4)) return launch_stream_cfg<T, EPI, ROWS, 4, WF>(s, p); break;
+    case 6: if constexpr (stream_built<EPI, WF>(ROWS, 6)) return launch_stream_cfg<T, EPI, ROWS, 6, WF>(s, p); break;
+    default: if constexpr (stream_built<EPI, WF>(ROWS, 8)) return launch_stream_cfg<T, EPI, ROWS, 8, WF>(s, p); break;
   }
   return MUI_ERR_UNSUPPORTED;
 }
@@ -373,10 +427,24 @@ static bool gateup_tiles_are_faster(int tokens, int rows, int k, int units) {
   return tokens > 32 && k > 512 && k % 2048 && ceil_div(rows, 112 * cus) > ceil_div(rows, 128 * cus);
 }
 
+// Codes: what the other int8 kernels keep. Up to 32 tokens with a scale per row the 16-rows-per-workgroup kernel where it takes the matrix in one round and K is short for the
+// number of tokens (us, that / bands: 4096 x 4096 at 20 / 24 / 32 tokens 10.0 / 10.8, 10.7 / 10.9, 12.2 / 11.2; 2048 x 8192 16.4 / 17.4, 17.7 / 17.5, 20.3 / 17.9; 3072 x 2048
+// at 32 7.2 / 7.6; 4096 x 14336 at 17 / 24 26.1 / 26.9, 29.5 / 26.7); beyond 32 tokens several rounds (gate/up 14336 x 4096 at 64 tokens 41 / 44); groups in
+// bf16 bands of 112 rows (14336 x 4096 at 32 41.8 / 42.8: a pair for every 64 codes is as many cache lines as the codes). Everywhere else the bands: per row,
+// 6144 x 4096 at 17 / 32 / 64 tokens 21.5 / 12.0, 21.7 / 12.4, 21.9 / 15.4, 4096 x 14336 at 32 / 33 / 64 33.8 / 27.2, 54.0 / 31.8, 58.8 / 34.6, gate/up 14336 x 4096 at 32 40.3 / 27.2,
+// 8192 x 2048 21.3 / 11.8 and at 64 21.2 / 16.4; groups of 128, 6144 x 4096 at 32 22.5 / 13.5, 4096 x 14336 62.8 / 33.0, 2048 x 2048 13.6 / 8.4, gate/up 8192 x 2048 21.7 / 15.8.
+static bool codes_are_faster_elsewhere(bool groups, bool bf16, int epi, int tokens, int rows, int k, int width, int units) {
+  const int cus = device_cus();
+  if (tokens > 32) return units > cus;
+  if (groups) return bf16 && width == 112;
+  return epi == SK_LINEAR && ceil_div(rows, 16) <= cus && (long)(tokens - 16) * k < 49152;
+}
+
 static int g_stream_rows = 0, g_stream_shares = 0;  // mui_tune_stream
 
-template <typename T, int EPI>
+template <typename T, int EPI, int WF = WF_16BIT>
 static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int* splits = nullptr) {
+  constexpr bool W8 = WF != WF_16BIT;
   // Rows per unit and shares of K by the least time: what a CU takes in (27.5 KB of weights, 105 KB of token rows per microsecond, 82 in
   // steps of 128 k-values), a barrier per step, a fixed part per round of workgroups; for shares of K the second launch and the
   // partial outputs, written and read. Measured against every other pair at 17 to 128 tokens on matrices from 2048 x 2048 to 128256 x 4096 it
@@ -389,13 +457,13 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int
   int width = 0;
   for (int c = 0; c < tried; ++c) {
     const int r = EPI == SK_GATEUP ? kGateup[c] : kLinear[c];
-    if (!stream_built<EPI>(r, nt) || (g_stream_rows && r != g_stream_rows)) continue;
+    if (!stream_built<EPI, WF>(r, nt) || (g_stream_rows && r != g_stream_rows)) continue;
     const int units = ceil_div(rows, r);
     for (int k = 1; k <= 8; ++k) {
       if (k > 1 && ((long)units * k > cus || (size_t)k * p.tokens * p.n * 4 > part_bytes || p.k / 256 < 2 * k)) break;
       if (g_stream_shares && k != g_stream_shares) continue;
-      const float one = (float)p.k / k * 2.f * ((float)r / 27.5e3f + 16.f * nt / (nt > 4 ? 82e3f : 105e3f));
-      const float barriers = (float)p.k / k / (r + 16 * nt <= 96 ? 256 : 128) * 0.08f;
+      const float one = (float)p.k / k * 2.f * ((float)r / (W8 ? 55e3f : 27.5e3f) + 16.f * nt / (nt > 4 ? 82e3f : 105e3f));
+      const float barriers = (float)p.k / k / (W8 || r + 16 * nt <= 96 ? 256 : 128) * 0.08f;
       const float cost = ceil_div(units, cus) * (one + barriers + 1.f) + (k > 1 ? 2.5f + 0.3f * k + (float)k * p.tokens * p.n * 8.f / 4e6f : 0.f);
       if (width == 0 || cost < best) { best = cost; width = r; p.n_units = units; p.k_splits = k; }
     }
@@ -403,41 +471,44 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int
   const bool forced = g_stream_rows || g_stream_shares;
   if (!p.add && p.k_splits == 1) return MUI_ERR_UNSUPPORTED;
   if (splits) *splits = p.k_splits;
-  if (!forced && EPI == SK_LINEAR && wide_is_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
-  if (forced && !width) return EPI == SK_GATEUP && nt > 4 ? MUI_ERR_UNSUPPORTED : MUI_ERR_INVALID_ARG;
-  if (!forced && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
-  if (!forced && EPI == SK_GATEUP && gateup_tiles_are_faster(p.tokens, rows, p.k, p.n_units)) return MUI_ERR_UNSUPPORTED;
+  if (!forced && !W8 && EPI == SK_LINEAR && wide_is_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
+  if (!width && (W8 || (EPI == SK_GATEUP && nt > 4))) return MUI_ERR_UNSUPPORTED;
+  if (forced && !width) return MUI_ERR_INVALID_ARG;
+  if (!forced && !W8 && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
+  if (!forced && W8 && codes_are_faster_elsewhere(WF == WF_U8_GROUP, T::kDtype == MUI_DTYPE_BF16, EPI, p.tokens, rows, p.k, width, p.n_units)) return MUI_ERR_UNSUPPORTED;
+  if (!forced && !W8 && EPI == SK_GATEUP && gateup_tiles_are_faster(p.tokens, rows, p.k, p.n_units)) return MUI_ERR_UNSUPPORTED;
   switch (width) {
-    case 16: return launch_stream_rows<T, EPI, 16>(s, p);
-    case 32: return launch_stream_rows<T, EPI, 32>(s, p);
-    case 48: return launch_stream_rows<T, EPI, 48>(s, p);
-    case 64: return launch_stream_rows<T, EPI, 64>(s, p);
-    case 96: return launch_stream_rows<T, EPI, 96>(s, p);
+    case 16: return launch_stream_rows<T, EPI, 16, WF>(s, p);
+    case 32: return launch_stream_rows<T, EPI, 32, WF>(s, p);
+    case 48: return launch_stream_rows<T, EPI, 48, WF>(s, p);
+    case 64: return launch_stream_rows<T, EPI, 64, WF>(s, p);
+    case 96: return launch_stream_rows<T, EPI, 96, WF>(s, p);
   }
   if constexpr (EPI == SK_LINEAR) {
     switch (width) {
-      case 8: return launch_stream_rows<T, EPI, 8>(s, p);
-      case 24: return launch_stream_rows<T, EPI, 24>(s, p);
-      case 40: return launch_stream_rows<T, EPI, 40>(s, p);
-      case 56: return launch_stream_rows<T, EPI, 56>(s, p);
-      case 128: return launch_stream_rows<T, EPI, 128>(s, p);
+      case 8: return launch_stream_rows<T, EPI, 8, WF>(s, p);
+      case 24: return launch_stream_rows<T, EPI, 24, WF>(s, p);
+      case 40: return launch_stream_rows<T, EPI, 40, WF>(s, p);
+      case 56: return launch_stream_rows<T, EPI, 56, WF>(s, p);
+      case 128: return launch_stream_rows<T, EPI, 128, WF>(s, p);
     }
   } else if (width == 112) {
-    return launch_stream_rows<T, EPI, 112>(s, p);
+    return launch_stream_rows<T, EPI, 112, WF>(s, p);
   }
   return MUI_ERR_UNSUPPORTED;
 }
 
 // what the loads cannot serve
-static bool stream_serves(const SkinnyParams& q, int most) {
+static bool stream_serves(const SkinnyParams& q, int most, bool w8 = false) {
   if (q.tokens < 1 || q.tokens > most || q.gamma || (q.x_pitch != 0 && q.x_pitch != q.k)) return false;
-  if (q.k % 256 || q.n % 8 || q.n < 8 || q.pitch % 8 || q.pitch > (1L << 26)) return false;
+  if (q.k % 256 || q.n % 8 || q.n < 8 || q.pitch % (w8 ? 16 : 8) || q.pitch > (1L << 26)) return false;
   return !((((uintptr_t)q.w0 | (uintptr_t)q.w1 | (uintptr_t)q.x) & 15) || (((uintptr_t)q.y | (uintptr_t)q.residual) & 7));
 }
 
-static StreamParams stream_params(const SkinnyParams& q, float* part, bool add) {
+static StreamParams stream_params(const SkinnyParams& q, float* part, bool add, bool w8 = false) {
   StreamParams p = {};
-  p.w0 = (const uint8_t*)q.w0; p.w1 = (const uint8_t*)q.w1; p.pitch = q.pitch * 2;
+  p.w0 = (const uint8_t*)q.w0; p.w1 = (const uint8_t*)q.w1; p.pitch = q.pitch * (w8 ? 1 : 2);
+  p.s0 = q.s0; p.s1 = q.s1; p.s_pitch = q.s_pitch; p.group_shift = q.group_shift;
   p.x = q.x; p.mul_bias = q.mul_bias; p.add_bias = q.add_bias; p.residual = q.residual; p.y = q.y;
   p.n = q.n; p.k = q.k; p.tokens = q.tokens; p.part = part; p.k_splits = 1; p.add = add;
   return p;
@@ -451,6 +522,23 @@ int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParam
   if (dtype == MUI_DTYPE_F16) return epilogue == SK_GATEUP ? launch_stream_t<F16, SK_GATEUP>(s, p, 0) : launch_stream_t<F16, SK_LINEAR>(s, p, part_bytes);
   if (dtype == MUI_DTYPE_BF16) return epilogue == SK_GATEUP ? launch_stream_t<BF16, SK_GATEUP>(s, p, 0) : launch_stream_t<BF16, SK_LINEAR>(s, p, part_bytes);
   return MUI_ERR_UNSUPPORTED;
+}
+
+template <int WF>
+static int launch_stream_codes(hipStream_t s, int dtype, int epilogue, const StreamParams& p, size_t part_bytes) {
+  if (dtype == MUI_DTYPE_F16) return epilogue == SK_GATEUP ? launch_stream_t<F16, SK_GATEUP, WF>(s, p, 0) : launch_stream_t<F16, SK_LINEAR, WF>(s, p, part_bytes);
+  if (dtype == MUI_DTYPE_BF16) return epilogue == SK_GATEUP ? launch_stream_t<BF16, SK_GATEUP, WF>(s, p, 0) : launch_stream_t<BF16, SK_LINEAR, WF>(s, p, part_bytes);
+  return MUI_ERR_UNSUPPORTED;
+}
+
+// The same for int8 codes, 17 to 64 tokens; groups of 64 or more
+int launch_gemm_stream_int8(hipStream_t s, int dtype, int wf, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
+  if (!stream_serves(q, 64, true)) return MUI_ERR_UNSUPPORTED;
+  const StreamParams p = stream_params(q, part, true, true);
+  if (wf == WF_I8_CHANNEL) return launch_stream_codes<WF_I8_CHANNEL>(s, dtype, epilogue, p, part_bytes);
+  // (pairs are read in fours of bytes)
+  if (wf != WF_U8_GROUP || q.group_shift < 6 || q.k % (1 << q.group_shift) || q.s_pitch % 2 || (((uintptr_t)q.s0 | (uintptr_t)q.s1) & 3)) return MUI_ERR_UNSUPPORTED;
+  return launch_stream_codes<WF_U8_GROUP>(s, dtype, epilogue, p, part_bytes);
 }
 
 // The same for a caller whose next launch adds the partial outputs up itself: part [*splits][tokens][n] gets the products, nothing else is applied.

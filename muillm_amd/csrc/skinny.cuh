@@ -207,6 +207,7 @@ int launch_gemm_wide(hipStream_t s, int dtype, int weight_format, int epilogue, 
 // the workgroup shares; part (part_bytes, may be none): fp32 partial outputs where shares of K are worth it (gemm_stream.hip). MUI_ERR_UNSUPPORTED
 // for everything else and for what the tiled GEMM does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);
+int launch_gemm_stream_int8(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);  // codes, 17..64 tokens
 int launch_gemm_stream_parts(hipStream_t s, int dtype, const SkinnyParams& p, float* part, size_t part_bytes, int* splits);
 // launches gemm_skinny_kernel<dtype, weight format, epilogue>; returns a MUI_* status
 int launch_skinny(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
