@@ -163,8 +163,8 @@ int mui_silu_mul_interleaved(mui_stream_t stream, int dtype, const void* gate_up
  *   weights_i8 int8 [n_out, k_in] (row pitch w_pitch bytes), scales 16-bit [n_out],
  *   w[n, k] = q[n, k] * scales[n];   y = W xn + add_bias + residual   (xn as in mui_linear).
  * The reference passes the residual through add_bias (int8linear.py:53-57); here both exist.
- * Any tokens >= 1 (as mui_linear: beyond MUI_MAX_TOKENS the tiled GEMM converts the codes on their
- * way to LDS; the reference dequantises the whole matrix and calls the framework's GEMM,
+ * Any tokens >= 1 (as mui_linear: beyond MUI_MAX_TOKENS the kernels read codes and convert them on
+ * their way to the matrix instructions; the reference dequantises the whole matrix and calls the framework's GEMM,
  * muillm/modules/quantized/int8linear.py:279-293).
  * Requirements: k_in % 16 == 0, k_in <= 16384, 16-byte aligned rows. */
 int mui_int8_linear(mui_stream_t stream, int dtype, const void* weights_i8, long w_pitch,
@@ -187,8 +187,8 @@ int mui_int8_gateup_silu(mui_stream_t stream, int dtype, const void* gate_i8, co
  * (muillm/quantization/rtnquantizer.py:49-88): weights_u8 uint8 [n_out, k_in],
  * scales_min_vals 16-bit [n_out * G, 2] = (scale, min) per group of 2^group_size_shift
  * inputs, w = u8 * scale + min. Requirements as above plus group size >= 16. Any tokens >= 1:
- * beyond MUI_MAX_TOKENS the tiled GEMM turns every chunk of codes into u8 * scale + min, rounded
- * once to the 16-bit type -- the values mui_int8_group_dequantize writes -- on its way to LDS. */
+ * beyond MUI_MAX_TOKENS the kernels turn every chunk of codes into u8 * scale + min, rounded
+ * once to the 16-bit type -- the values mui_int8_group_dequantize writes -- before it is multiplied. */
 int mui_int8_group_linear(mui_stream_t stream, int dtype, const void* weights_u8, long w_pitch,
                           const void* scales_min_vals, int group_size_shift, const void* x,
                           const void* norm_weights, float epsilon, const void* add_bias,
