@@ -429,15 +429,16 @@ static bool gateup_tiles_are_faster(int tokens, int rows, int k, int units) {
 
 // Codes: what the other int8 kernels keep. Up to 32 tokens with a scale per row the 16-rows-per-workgroup kernel where it takes the matrix in one round and K is short for the
 // number of tokens (us, that / bands: 4096 x 4096 at 20 / 24 / 32 tokens 10.0 / 10.8, 10.7 / 10.9, 12.2 / 11.2; 2048 x 8192 16.4 / 17.4, 17.7 / 17.5, 20.3 / 17.9; 3072 x 2048
-// at 32 7.2 / 7.6; 4096 x 14336 at 17 / 24 26.1 / 26.9, 29.5 / 26.7); beyond 32 tokens several rounds (gate/up 14336 x 4096 at 64 tokens 41 / 44); groups in
+// at 32 7.2 / 7.6; 4096 x 14336 at 17 / 24 26.1 / 26.9, 29.5 / 26.7; 4096 x 256 and x 512
+// at 33 3.8 / 4.1, 4.8 / 4.8, 2048 x 1024 6.3 / 5.8); beyond 32 tokens several rounds (gate/up 14336 x 4096 at 64 tokens 41 / 44); groups in
 // bf16 bands of 112 rows (14336 x 4096 at 32 41.8 / 42.8: a pair for every 64 codes is as many cache lines as the codes). Everywhere else the bands: per row,
 // 6144 x 4096 at 17 / 32 / 64 tokens 21.5 / 12.0, 21.7 / 12.4, 21.9 / 15.4, 4096 x 14336 at 32 / 33 / 64 33.8 / 27.2, 54.0 / 31.8, 58.8 / 34.6, gate/up 14336 x 4096 at 32 40.3 / 27.2,
 // 8192 x 2048 21.3 / 11.8 and at 64 21.2 / 16.4; groups of 128, 6144 x 4096 at 32 22.5 / 13.5, 4096 x 14336 62.8 / 33.0, 2048 x 2048 13.6 / 8.4, gate/up 8192 x 2048 21.7 / 15.8.
 static bool codes_are_faster_elsewhere(bool groups, bool bf16, int epi, int tokens, int rows, int k, int width, int units) {
   const int cus = device_cus();
-  if (tokens > 32) return units > cus;
-  if (groups) return bf16 && width == 112;
-  return epi == SK_LINEAR && ceil_div(rows, 16) <= cus && (long)(tokens - 16) * k < 49152;
+  const bool wide = !groups && epi == SK_LINEAR && ceil_div(rows, 16) <= cus;
+  if (tokens > 32) return units > cus || (wide && tokens <= 40 && k <= 512);
+  return groups ? bf16 && width == 112 : wide && (long)(tokens - 16) * k < 49152;
 }
 
 static int g_stream_rows = 0, g_stream_shares = 0;  // mui_tune_stream
