@@ -39,7 +39,8 @@ struct F16 {
   static __device__ __forceinline__ uint16_t pack(float v) {
     return __builtin_bit_cast(uint16_t, (_Float16)v);
   }
-  // two values -> one packed word (a in the low half): one v_cvt_pk_f16_f32, same rounding
+  // two values -> one packed word (a in the low half): one v_cvt_pk_f16_f32. For values that are there in 32 bits; one that a product has just made is
+  // rounded to 32 bits first, where pack() lets the compiler round it to 16 straight away (v_fma_mixlo_f16)
   static __device__ __forceinline__ uint32_t pack2(float a, float b) {
     typedef float f32x2_t __attribute__((ext_vector_type(2)));
     const f32x2_t v = {a, b};
@@ -91,10 +92,17 @@ __device__ __forceinline__ void unpack8(const u32x4 w, float (&f)[8]) {
 template <typename T>
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
   u32x4 w;
-  w.x = T::pack2(f[0], f[1]);
-  w.y = T::pack2(f[2], f[3]);
-  w.z = T::pack2(f[4], f[5]);
-  w.w = T::pack2(f[6], f[7]);
+  if constexpr (T::kDtype == MUI_DTYPE_F16) {  // (one instruction per product with its only rounding, see pack2: a norm's eight values take 16 instead of 20)
+    w.x = (uint32_t)T::pack(f[0]) | ((uint32_t)T::pack(f[1]) << 16);
+    w.y = (uint32_t)T::pack(f[2]) | ((uint32_t)T::pack(f[3]) << 16);
+    w.z = (uint32_t)T::pack(f[4]) | ((uint32_t)T::pack(f[5]) << 16);
+    w.w = (uint32_t)T::pack(f[6]) | ((uint32_t)T::pack(f[7]) << 16);
+  } else {
+    w.x = T::pack2(f[0], f[1]);
+    w.y = T::pack2(f[2], f[3]);
+    w.z = T::pack2(f[4], f[5]);
+    w.w = T::pack2(f[6], f[7]);
+  }
   return w;
 }
 
