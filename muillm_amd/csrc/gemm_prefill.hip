@@ -1066,10 +1066,11 @@ constexpr bool kPipelined = WF != WF_U8_GROUP || T::kDtype == MUI_DTYPE_F16;
 
 // what the LDS-direct loads need: whole k-steps, 16-byte aligned rows, 32-bit byte offsets from
 // the operands' bases
-// (codes of the group format: a k-step of 64 lies in one group)
+// (codes of the group format: a k-step of 64 lies in one group, and a (scale, min) pair is one load of 4 bytes, which has to be aligned)
 static bool lds_direct_loads_serve(const PrefillGemmParams& p, int wf) {
   return g_prefill_dma && p.k % 64 == 0 && p.pitch % 16 == 0 && (long)p.n * p.pitch < (1L << 32) &&
-         (long)p.tokens * p.k * 2 < (1L << 32) && (wf != WF_U8_GROUP || p.group_shift >= 6);
+         (long)p.tokens * p.k * 2 < (1L << 32) &&
+         (wf != WF_U8_GROUP || (p.group_shift >= 6 && p.s_pitch % 2 == 0 && (((uintptr_t)p.s0 | (uintptr_t)p.s1) & 3) == 0));
 }
 static bool pipelined_loop_serves(const PrefillGemmParams& p, int wf) { return lds_direct_loads_serve(p, wf); }
 

@@ -380,8 +380,9 @@ class MuiPromptStack(MuiDecoderStack):
         self._bound(cache)
         # (the library's call converts codes, the modules dequantise long prompts' matrices)
         ks = (self.hidden, self.hq * self.d, layers[0].mlp.intermediate_size)
-        shifts = {x.int8_group_size_shift for x in self._layers if x.qkv_scales or x.o_scales or x.gate_scales or x.down_scales}
-        self._most_rows = min([muillm_ext.int8_dequantised_from(self.dtype, k, shift) - 1 for k in ks for shift in shifts], default=1 << 30)
+        codes = {(x.int8_group_size_shift, (x.qkv_scales or 0) | (x.o_scales or 0) | (x.gate_scales or 0) | (x.up_scales or 0) | (x.down_scales or 0))
+                 for x in self._layers if x.qkv_scales or x.o_scales or x.gate_scales or x.down_scales}
+        self._most_rows = min([muillm_ext.int8_dequantised_from(self.dtype, k, *of) - 1 for k in ks for of in codes], default=1 << 30)
 
     def _built_from(self, owners, cache_tensors) -> None:
         pass  # see remember()

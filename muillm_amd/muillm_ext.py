@@ -474,17 +474,17 @@ INT8_GROUP_CHUNK_MAX_TOKENS = MUI_MAX_TOKENS
 # 684 / 1378 / 2606; groups of 128 in fp16 at 1024 / 1536 / 2048 tokens 480 / 695 / 864 against 542 / 687 / 853.
 INT8_DEQUANT_MIN_TOKENS = 8192
 INT8_GROUP_DEQUANT_MIN_TOKENS = 1536
-# What the pipelined loop does not take (rows that are no multiple of 64 codes, groups of fewer, the group format in bf16) is converted on the way to LDS:
+# What the pipelined loop does not take (rows that are no multiple of 64 codes, groups of fewer, pairs off 4-byte addresses, the group format in bf16) is converted on the way to LDS:
 # at 4096 tokens QKV 227 against 182 us dequantised, gate/up 817 against 762; an 8B-shaped prefill 17.7 against 19.5 ms at 1024 tokens, 27.5 against 25.8 at 1536
 # (group format: level at 1024 tokens, 35.0 against 29.9 ms at 2048).
 INT8_STAGED_DEQUANT_MIN_TOKENS = 1280
 INT8_GROUP_STAGED_DEQUANT_MIN_TOKENS = 1024
 
 
-def int8_dequantised_from(dtype: torch.dtype, k: int, group_size_shift: int = 0) -> int:
-    """Tokens from which a matrix of rows of k codes is dequantised (group_size_shift 0: per-channel format)."""
+def int8_dequantised_from(dtype: torch.dtype, k: int, group_size_shift: int = 0, pairs_at: int = 0) -> int:
+    """Tokens from which a matrix of rows of k codes is dequantised (group_size_shift 0: per-channel format; else pairs_at is the (scale, min) pairs' address)."""
     if group_size_shift:
-        staged = k % 64 or group_size_shift < 6 or dtype != torch.float16
+        staged = k % 64 or group_size_shift < 6 or pairs_at % 4 or dtype != torch.float16
         return min(INT8_GROUP_DEQUANT_MIN_TOKENS, INT8_GROUP_STAGED_DEQUANT_MIN_TOKENS) if staged else INT8_GROUP_DEQUANT_MIN_TOKENS
     return min(INT8_DEQUANT_MIN_TOKENS, INT8_STAGED_DEQUANT_MIN_TOKENS) if k % 64 else INT8_DEQUANT_MIN_TOKENS
 
@@ -628,7 +628,7 @@ def muillm_int8_linear_forward(x, weights, scales_min_vals, group_size_shift, no
     _check_contiguous(scales_min_vals, "scales_min_vals")
     _check_activations(x, k, "muillm_int8_linear_forward", _MAX_CALL_TOKENS, weights,
                        scales_min_vals, norm_weights, add_bias, residual)
-    if _num_tokens(x) >= int8_dequantised_from(x.dtype, k, group_size_shift):
+    if _num_tokens(x) >= int8_dequantised_from(x.dtype, k, group_size_shift, scales_min_vals.data_ptr()):
         # a long prompt: the reference's route (dequantise the matrix, then a GEMM,
         # muillm/modules/quantized/int8linear.py:279-293) on this library's kernels; shorter ones go
         # to the GEMM that dequantises the codes on their way to LDS (one call below)
@@ -754,7 +754,7 @@ def muillm_int8_gateupsilu_forward(norm_weights, epsilon, gate_up_weights, gate_
         raise RuntimeError("gate_up_scales_min_vals must hold N * 2 * K / group (scale, min) pairs in the activation dtype")
     if norm_weights is not None and (norm_weights.dtype != x.dtype or norm_weights.numel() != k):
         raise RuntimeError("norm weights must be one value per input feature in the activation dtype")
-    if _num_tokens(x) >= int8_dequantised_from(x.dtype, k, group_size_shift):
+    if _num_tokens(x) >= int8_dequantised_from(x.dtype, k, group_size_shift, gate_up_scales_min_vals.data_ptr()):
         # a long prompt: dequantise gate and up once, then the tiled GEMM with the SiLU * mul epilogue
         gd, ud = muillm_int8_gateupsilu_dequantize_forward(gate_up_weights, gate_up_scales_min_vals, group_size_shift)
         return mui_gateup_silu(norm_weights, epsilon, gd, ud, x)

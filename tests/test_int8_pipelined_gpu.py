@@ -76,7 +76,32 @@ def test_groups(n, k, tokens, gateup, which, shift, tile):
     assert float((y.double() - ref).abs().max() / ref.abs().max()) <= REL[dtype]
 
 
+@pytest.mark.parametrize("tokens", [20, 40, 100, 300, 1100, 1600])
+@pytest.mark.parametrize("gateup", [False, True])
+@pytest.mark.parametrize("shift", [6, 7])
+def test_pairs_off_the_four_byte_grid(tokens, gateup, shift):
+    """(scale, min) pairs at an odd 2-byte address are taken by kernels that read them with ordinary loads, on every route by number of tokens."""
+    dtype, n, k, g = torch.float16, 520, 256, torch.Generator(device=DEV).manual_seed(tokens + shift)
+    rows = 2 * n if gateup else n
+    q, x = _codes(g, rows, k) + 128, torch.randn(tokens, k, device=DEV, generator=g).to(dtype)
+    room = torch.zeros(2 * rows * (k >> shift) + 1, dtype=dtype, device=DEV)
+    pairs = room[1:].view(-1, 2)
+    pairs[:, 0], pairs[:, 1] = torch.rand(len(pairs), device=DEV, generator=g) * 2e-3 + 1e-3, -torch.rand(len(pairs), device=DEV, generator=g) * 0.3
+    assert pairs.data_ptr() % 4 == 2
+    p = pairs.double().view(rows, k >> shift, 1, 2)
+    w, q = (q.double().view(rows, k >> shift, -1) * p[..., 0] + p[..., 1]).view(rows, k), q.to(torch.uint8)
+    if gateup:
+        a, b = x.double() @ w[0::2].T, x.double() @ w[1::2].T
+        ref = a * torch.sigmoid(a) * b
+        y = muillm_ext.muillm_int8_gateupsilu_forward(None, 0.0, q.view(n, 2, k), pairs.view(n, 2, k >> shift, 2), shift, x)
+    else:
+        ref = x.double() @ w.T
+        y = muillm_ext.muillm_int8_linear_forward(x, q, pairs, shift)
+    assert float((y.double() - ref).abs().max() / ref.abs().max()) <= REL[dtype]
+
+
 def test_where_matrices_are_dequantised():
     f, b, at = torch.float16, torch.bfloat16, muillm_ext.int8_dequantised_from
     assert at(f, 4096) == at(b, 14336) == 8192 and at(f, 4096 + 16) == at(b, 48) == 1280
     assert at(f, 4096, 7) == 1536 and at(f, 4096, 5) == at(b, 4096, 7) == 1024
+    assert at(f, 4096, 7, 1 << 20) == 1536 and at(f, 4096, 7, (1 << 20) + 2) == 1024
