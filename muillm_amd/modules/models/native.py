@@ -68,6 +68,8 @@ class MuiNativeModel(MuiModule):
             raise ValueError(f"batch {b} exceeds the cache's max_batch_size {cache.max_batch_size}")
         if not cache.device_length_mode:
             cache.grow_cache(past + t)
+        if real is not None and (real.batch, real.tokens) != (b, t):
+            real = None  # (a mask of another shape: what the layers say to it is not for a few of its rows to answer)
         if attention_mask is not None and past == 0:
             cache.set_row_start(self._left_padding(attention_mask) if real is None else on_device(self._left_padding(real.mask), attention_mask.device))
         if cache_position is None:

@@ -140,6 +140,20 @@ def _zufadra(cfg, w, dtype):
 
 
 @torch.no_grad()
+@pytest.mark.parametrize("util", [salepel_util, zufadra_util])
+def test_a_mask_of_another_shape_stays_refused(util):
+    """One row of a mask for two of tokens: the layers refuse it, and the real rows of its one row are not taken for the batch."""
+    cfg = util.default_config()
+    lm = util.build(cfg, util.random_weights(cfg, seed=4), torch.bfloat16)
+    ids = torch.randint(0, cfg["vocab"], (2, 9), device=DEV)
+    mask = torch.ones(1, 9, dtype=torch.int64, device=DEV)
+    mask[0, :4] = 0
+    for real in (None, RealRows.of(lm, mask.cpu() != 0, DEV)):
+        with pytest.raises(RuntimeError, match="row_start"):
+            lm(input_ids=ids, attention_mask=mask, past_key_values=lm.create_cache(2, 12), num_logits_to_keep=1, real=real)
+
+
+@torch.no_grad()
 def test_what_is_run_with_the_padding():
     lm = _lm()
     ids, mask = _batch((9, 4), 512)
