@@ -515,6 +515,7 @@ class MuiPromptStack(MuiDecoderStack):
                                               out.data_ptr(), pos.data_ptr(), t if pos.shape[0] > 1 else 0, cache_position.data_ptr(), seq_len,
                                               mask.data_ptr(), mask.stride(0), (ws.data_ptr() + 255) & ~255, _ptr(linear_ws),
                                               0 if linear_ws is None else linear_ws.numel()), "mui_decoder_stack_prompt_rows")
+        self.remember()
         return out
 
     def run(self, hidden_in: torch.Tensor, position_ids: torch.Tensor, cache_position: torch.Tensor, seq_len: Optional[int],

@@ -6,6 +6,8 @@ import torch
 from muillm_amd import _lib, muillm_ext
 from muillm_amd.modules.models.graphdecoder import MuiGraphDecoder
 from muillm_amd.modules import realrows
+from muillm_amd.modules.decoder.decoderstack import MuiPromptStack
+from muillm_amd.modules.models.llama import model as llama_model
 from muillm_amd.modules.realrows import RealRows
 from tests import salepel_util, zufadra_util
 from tests.test_prompt_stack_gpu import _lm
@@ -104,6 +106,22 @@ def test_llama(kind, lengths):
     for b, n in enumerate(lengths):
         alone = lm(input_ids=ids[b:b + 1, t - n:], num_logits_to_keep=1).logits[0, -1].float()
         assert _off(got[b], alone) <= LIMIT[dtype]
+
+
+@torch.no_grad()
+def test_layers_are_examined_once(monkeypatch):
+    """For several padded prompts in a row, of more rows than the decode kernels take or fewer, and caches of their own; again once a weight has been replaced."""
+    lm, built, examine = _lm(), [], MuiPromptStack.eligible
+    monkeypatch.setattr(MuiPromptStack, "eligible", staticmethod(lambda *a: built.append(1) or examine(*a)))
+    ids, mask = _batch((9, 4), 512)
+    for _ in range(3):
+        assert _prompt(lm, ids, mask, 1)[3] == 1 and len(built) == 1
+    monkeypatch.setattr(llama_model, "_BUSY_PRODUCTS", 0)  # (a long prompt, as far as the model knows: only a first one is left to the modules)
+    assert _prompt(lm, *_batch((30, 12, 7), 512), 1)[3] == 1 and len(built) == 1
+    down = lm.model.layers[1].mlp.down_proj
+    down.weight = torch.nn.Parameter(down.weight.detach().clone(), requires_grad=False)
+    down.finalize_init()
+    assert _prompt(lm, ids, mask, 1)[3] == 0 and len(built) == 2 and _prompt(lm, ids, mask, 1)[3] == 1 and len(built) == 2
 
 
 @torch.no_grad()
