@@ -38,7 +38,7 @@ from ...linear import MuiLinear
 from ...module import MuiModule, heard
 from ...multilinear import MuiMultiLinear
 from ...norm.rmsnorm import MuiRMSNorm
-from ...realrows import RealRows
+from ...realrows import RealRows, Worth
 from ..generation import MuiGenerationMixin
 
 
@@ -450,6 +450,7 @@ class MuiLlamaForCausalLM(MuiGenerationMixin, MuiModule):
     # ---- what the decode loop asks of a causal LM ---------------------------------------------
     pads_in_cache = False  # left padding travels as an additive mask with every step
     takes_real_rows = True
+    padding_worth = Worth(padding=1e10, tiles=2e10)
 
     def create_cache(self, batch_size: int, seq_len: int) -> MuiStaticCache:
         return create_static_cache(self.engine_config, self.config, batch_size, seq_len, self.model.mdevice, self.model.mdtype)

@@ -16,6 +16,7 @@ from ...decoder.sandwichdecoder import MuiSandwichDecoderLayer
 from ...embedding import MuiEmbedding
 from ...moe import MuiMoE
 from ...recurrent.mlstm import MuiMLstm
+from ...realrows import Worth
 from ..native import MuiNativeForCausalLM, MuiNativeModel
 from .config import MuiSalepelConfig
 
@@ -70,6 +71,7 @@ class MuiSalepelModel(MuiNativeModel):
 
 class MuiSalepelForCausalLM(MuiNativeForCausalLM):
     takes_real_rows = True
+    padding_worth = Worth(padding=8e9, passes=3800.0)
     model_class = MuiSalepelModel
     config_class = MuiSalepelConfig
 

@@ -17,6 +17,7 @@ from ...decoder.sandwichdecoder import MuiSandwichDecoderLayer
 from ...embedding import MuiBigramEmbedding, MuiEmbedding
 from ...gateupdownmlp import MuiGateUpDownMLP
 from ...recurrent.channeldelta import MuiChannelDelta
+from ...realrows import Worth
 from ..native import MuiNativeForCausalLM, MuiNativeModel
 from .config import MuiZufadraConfig
 
@@ -84,6 +85,7 @@ class MuiZufadraModel(MuiNativeModel):
 
 class MuiZufadraForCausalLM(MuiNativeForCausalLM):
     takes_real_rows = True
+    padding_worth = Worth(padding=2.7e10, tiles=3.7e10)
     model_class = MuiZufadraModel
     config_class = MuiZufadraConfig
 

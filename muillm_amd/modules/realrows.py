@@ -1,6 +1,6 @@
 """The tokens of a left-padded batch of prompts that are no padding. What works on one token at a time -- linears, norms, experts -- need not
 see the others: their rows are laid out one after the other, and only what looks at a token's neighbours (attention, recurrences) gets [batch, tokens] with zeros for the padding."""
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -8,12 +8,33 @@ from .. import muillm_ext
 from .module import heard
 
 
-# Leaving padding out costs a layer two launches and two passes over its projections (6 to 10 us), and up to a few hundred tokens linears take as long for fewer:
-# what is left out has to be beyond the 128 tokens whose linears are bound by their weights, and this many operations per layer (a layer has about 12 hidden^2
-# weights that a token meets; 30 us at 0.9 PFLOP/s). Eight layers of width 2048, 319 tokens of which 213 are real: 3743 us with the padding, 3777 without; 2048 wide,
-# eight prompts of up to 150 tokens (mLSTM, latent attention, experts) 12752 / 12309; 4096 wide (int8), 14 of up to 557 35357 / 29521.
-MOST_WEIGHT_BOUND = 128
-LEAST_OPERATIONS = 2.7e10
+# Leaving padding out costs a layer two launches and two passes over its projections (6 to 10 us), and where the modules are called one by one 33 us of host time. Linears of up to
+# 128 tokens are bound by their weights and beyond work on tiles of 256, so they take as long for fewer tokens unless tiles fall away; experts deal their tokens out and take less for
+# every one that is missing. In operations per layer (24 hidden^2 for a token; 0.9e9 a us): the padding's, those of the tiles that fall away, and, per token and value of its width, what the
+# passes cost where no tile pays for them. us, with it / without, prompts alone on eight layers (tokens -> real ones):
+#   Llama, one call: 2048 wide 319 -> 200 1656 / 1546, 640 -> 463 2014 / 1806, 900 -> 657 2193 / 2136, 928 -> 668 2089 / 2046, 4096 wide 192 -> 118 2379 / 1879, 320 -> 214 2979 / 2541;
+#     2050 -> 2020 7763 / 7316, 4100 -> 4066 13170 / 12880; no tile less: 2048 wide 256 -> 176 1473 / 1498, 450 -> 310 1653 / 1677, 4096 wide 256 -> 176 2461 / 2442, int8 2523 / 2582, 480 -> 342 3214 / 3174
+#   Zufadra: two tiles less 2048 wide 1200 -> 763 2938 / 2588, one 4096 wide 192 -> 118 2572 / 2206, 319 -> 200 3277 / 2913, 260 -> 173 3059 / 2658, 2048 wide 319 -> 200 1911 / 2039,
+#     900 -> 581 2336 / 2414, 1000 -> 570 2452 / 2466; none 4096 wide 256 -> 176 2668 / 2727, 400 -> 307 3211 / 3262
+#   Salepel: 2048 wide 256 -> 176 3335 / 3319, 319 -> 200 3636 / 3433, 450 -> 310 3685 / 3514, 1200 -> 763 4536 / 4132, 4096 wide 192 -> 118 6223 / 5994, 400 -> 307 7095 / 6614; few
+#     of many: 2048 wide 2056 -> 1926 5399 / 5766, 4096 wide 1026 -> 996 8524 / 8654, 4100 -> 4066 19464 / 20024
+class Worth(NamedTuple):
+    padding: float
+    tiles: float = 0.0
+    passes: float = 0.0
+
+
+MOST_WEIGHT_BOUND, TOKEN_TILE = 128, 256
+
+
+def _tiles(tokens: int) -> float:
+    return 0.5 if tokens <= MOST_WEIGHT_BOUND else -(-tokens // TOKEN_TILE)
+
+
+def worth_it(worth: Worth, hidden: int, tokens: int, padding: int) -> bool:
+    per_token = 24.0 * hidden ** 2
+    return (tokens > MOST_WEIGHT_BOUND and padding * per_token >= worth.padding + worth.passes * tokens * hidden
+            and (_tiles(tokens) - _tiles(tokens - padding)) * TOKEN_TILE * per_token >= worth.tiles)
 
 
 def on_device(x: torch.Tensor, device) -> torch.Tensor:
@@ -42,12 +63,13 @@ class RealRows:
 
     @staticmethod
     def of(lm, mask: torch.Tensor, device) -> Optional["RealRows"]:
-        """For a padded prompt of a causal LM whose forward takes `real`; None for any other, and where somebody listens to what it is given."""
+        """For a padded prompt of a causal LM whose forward takes `real`; None for any other, where it is not worth it (`padding_worth` of the model's class) and where
+        somebody listens to what it is given."""
         model = getattr(lm, "model", None)
         if torch.device(device).type != "cuda" or mask.dim() != 2 or not all("takes_real_rows" in type(m).__dict__ for m in (lm, model)) or heard(lm, model):
             return None
         padding = mask.numel() - int(mask.sum())
-        if not padding or mask.numel() <= MOST_WEIGHT_BOUND or padding * 24.0 * lm.config.hidden_size ** 2 < LEAST_OPERATIONS or not bool(mask[:, -1].all()):
+        if not padding or not worth_it(lm.padding_worth, lm.config.hidden_size, mask.numel(), padding) or not bool(mask[:, -1].all()):
             return None
         return RealRows(mask, device)
 

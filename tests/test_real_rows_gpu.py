@@ -9,6 +9,7 @@ from muillm_amd.modules import realrows
 from muillm_amd.modules.decoder.decoderstack import MuiPromptStack
 from muillm_amd.modules.models.llama import model as llama_model
 from muillm_amd.modules.realrows import RealRows
+from muillm_amd.modules.models.salepel.model import MuiSalepelForCausalLM
 from tests import salepel_util, zufadra_util
 from tests.test_prompt_stack_gpu import _lm
 
@@ -18,8 +19,7 @@ DEV = "cuda"
 
 @pytest.fixture(autouse=True)
 def _however_little(monkeypatch):
-    monkeypatch.setattr(realrows, "LEAST_OPERATIONS", 0)
-    monkeypatch.setattr(realrows, "MOST_WEIGHT_BOUND", 0)
+    monkeypatch.setattr(realrows, "worth_it", lambda *a: True)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16, torch.int64])
@@ -198,11 +198,17 @@ def test_a_class_of_its_own_is_not_asked():
     assert RealRows.of(lm, mask, DEV) is None
 
 
-@pytest.mark.parametrize("tokens,padding,hidden,worth", [(128, 100, 4096, False), (129, 68, 4096, True), (129, 67, 4096, False), (768, 269, 2048, True), (768, 268, 2048, False)])
+@pytest.mark.parametrize("tokens,padding,hidden,worth", [
+    (128, 100, 4096, False), (192, 64, 4096, True), (192, 63, 4096, False), (319, 120, 2048, True), (319, 100, 2048, True), (319, 99, 2048, False), (256, 100, 4096, False), (300, 44, 4096, True),
+    (300, 43, 4096, False), (192, 66, 2048, False), (4000, 300, 2048, True)])
 def test_where_it_is_worth_it(monkeypatch, tokens, padding, hidden, worth):
+    """Llama: padding of 1e10 operations a layer, with which a tile of 256 tokens falls away or the rest are no more than 128."""
     monkeypatch.undo()
     lm = _lm()
     lm.config.hidden_size = hidden
     mask = torch.ones(1, tokens, dtype=torch.bool)
     mask[0, :padding] = False
     assert (RealRows.of(lm, mask, DEV) is not None) == worth
+    # mixtures of experts: whatever tiles there are, but not a few of many tokens
+    least = 8e9 / (24 * hidden ** 2) + tokens * 3800 / (24 * hidden)
+    assert realrows.worth_it(MuiSalepelForCausalLM.padding_worth, hidden, tokens, padding) == (tokens > 128 and padding >= least)
