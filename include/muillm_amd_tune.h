@@ -61,7 +61,7 @@ int mui_tune_attention(int waves_per_workgroup, int min_tokens_per_split, int di
 int mui_tune_skinny(int min_tokens, int stream_b, int multi_max_tokens);
 
 /* Prompt GEMM (more than MUI_MAX_TOKENS tokens): tile = 0 built-in choice, 1 = 128 rows x 128
- * tokens, 2 = 64 x 128, 3 = 32 x 64 (linear only), 4 = 256 x 256, 5 = 64 x 128 whose waves split K
+ * tokens, 2 and 3 = 5 and 6, 4 = 256 x 256, 5 = 64 x 128 whose waves split K
  * four ways (2 x 2 wave tiles; int8: two token halves), 6 = 32 x 64 on four waves that split K,
  * 7 = 128 x 256, 8 = 192 x 256, 9 = 128 x 128 and 11 = 128 x 64 with waves that split K like 5,
  * 10 = 96 x 128 (linear only), 12 = 64 x 64 with waves that split K like 6 (linear only),

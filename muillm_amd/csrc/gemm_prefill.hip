@@ -20,8 +20,7 @@
 //   256 rows x 256 tokens x 64 k on eight waves (4 x 2; sixteen where a norm is fused or the loads
 //   cannot go straight into LDS), 128 x 256 x 64 on sixteen (4 x 4), 192 x 256 x 64 on
 //   twelve (3 x 4) while the grid covers most of the chip; 128 x 128 x 64 and 96 x 128 x 64 on four
-//   waves (2 x 2), two workgroups per CU; 64 x 128 x 128 and 32 x 64 x 256 with a single LDS stage
-//   for small matrices. For grids of a round or two of workgroups (short prompts, matrices of a few
+//   waves (2 x 2), two workgroups per CU. For grids of a round or two of workgroups (short prompts, matrices of a few
 //   thousand rows) shapes whose waves ALSO split K, each taking every fourth 32-value chunk of a
 //   k-step: 128 x 128 x 128, 128 x 64 x 128 and 64 x 128 x 128 on sixteen waves, 64 x 64 x 256 and
 //   32 x 64 x 256 on eight -- the LDS traffic per matrix instruction of a larger tile and four waves per SIMD
@@ -141,8 +140,7 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   static_assert(XCH >= 1 && WCH >= 1 && kPfThreads % CPR == 0, "tile shape");
   static_assert(XCHUNKS >= kPfThreads && WCHUNKS >= kPfThreads, "every thread stages at least one chunk of each operand");
   static_assert((XEXACT || XCHUNKS % 64 == 0) && (WEXACT || WCHUNKS % 64 == 0), "whole waves stage the last round of chunks");
-  // NBUF == 2: step s + 1 is written to the other LDS stage while step s is multiplied, one
-  // barrier per step instead of two
+  // step s + 1 is written to the other LDS stage while step s is multiplied, one barrier per step
   constexpr bool W8 = PIPE && WF != WF_16BIT;  // codes in the stages
   constexpr int WPITCH = W8 ? PITCH / 2 : PITCH;
   typedef uint16_t WStage[ROWS * WPITCH];
@@ -691,7 +689,8 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();  // the stages are free (and no load is still on its way into them)
-  } else if constexpr (NBUF == 2) {
+  } else {
+    static_assert(DMA || NBUF == 2, "register-staged tiles have two stages");
     load_step(sb, r0);
     // two LDS stages: step s + 1 moves from the registers to the other stage and step s + 2 is
     // requested from memory before step s is multiplied, so that the LDS writes and the loads
@@ -730,15 +729,6 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
         __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
       }
       __syncthreads();
-    }
-  } else {
-    load_step(sb, r0);
-    for (int s = 0; s < n_steps; ++s) {
-      __syncthreads();  // the previous step's operands have been read
-      store_step(s, 0, r0);
-      __syncthreads();
-      load_step(s + 1, r0);  // in flight during this step's multiplications
-      multiply(0);
     }
   }
 
@@ -1044,7 +1034,7 @@ __global__ void __launch_bounds__(64 * NWR * NWT * NWK)
   }
 }
 
-static int g_prefill_tile = 0;  // experiments: 0 = built-in choice, 1 = 128 x 128, 2 = 64 x 128, 3 = 32 x 64, 4 = 256 x 256,
+static int g_prefill_tile = 0;  // experiments: 0 = built-in choice, 1 = 128 x 128, 4 = 256 x 256,
                                 // 5 = 64 x 128 on eight waves that split K four ways, 6 = 32 x 64 on four waves that split K,
                                 // 7 = 128 x 256, 8 = 192 x 256, 9 = 128 x 128 on eight waves that split K four ways,
                                 // 10 = 96 x 128 (linear only), 11 = 128 x 64 on sixteen waves that split K four ways,
@@ -1131,7 +1121,7 @@ static int launch_prefill_cfg(hipStream_t s, PrefillGemmParams p) {
     if (p.gamma) return launch(prefill_gemm_kernel<T, WF, true, EPI, WR, WT, NWR, NWT, NWK, KS, NBUF>);
   }
   constexpr int kWaves8 = 8 * NWR * NWT * NWK;
-  if constexpr ((WF == WF_16BIT || (PIPE && kPipelined<T, WF>)) && (NBUF == 2 || (PIPE && NBUF == 3)) && NWK == 1 && KS == 64 && ROWS % kWaves8 == 0 &&
+  if constexpr ((WF == WF_16BIT || (PIPE && kPipelined<T, WF>)) && NWK == 1 && KS == 64 && ROWS % kWaves8 == 0 &&
                 TOKS % kWaves8 == 0 && (PIPE || ROWS * TOKS >= 256 * 256)) {
     // LDS-direct operand loads: always with the software-pipelined loop; with the sixteen-wave loop
     // on the 256 x 256 tile only, where a k-step (2048 matrix-pipe cycles per SIMD) covers an L2
@@ -1196,7 +1186,7 @@ static int launch_prefill_xs(hipStream_t s, PrefillGemmParams p, int shares, voi
   return launch_status();
 }
 
-// What a tile shape does with its last round of workgroups (see launch_prefill_t): by how many tiles a CU's XCD has left, of a round of `per`
+// What becomes of the last round of 256 x 256 tiles (see launch_prefill_t): by how many tiles a CU's XCD has left, of a round of `per`
 enum LastRound { kLastWhole, kLastHalves, kLastQuarters };
 static LastRound last_round(long slots, int per) {
   const long rest = slots % per;
@@ -1249,15 +1239,15 @@ static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int t
     // (and their last round goes to smaller tiles where it is at most half full. A launch of its own for it costs a linear more: its big tiles end on time of
     // their own, 107 us at K = 4096 where the plan has 96, and the 192 x 256 tile is close behind: 6144 x 4096 at 3500 tokens 174 us with quarters, 159 on that)
     const float second = (EPI == SK_GATEUP ? 8.f : 28.f) * 4096.f / (float)p.k;
-    auto rounds = [&](int r, int tk, float one, float many, float halves, float quarters) {
+    auto rounds = [&](int r, int tk, float one, float many, bool split) {
       if (!pipe) return whole(tiles(r, tk), one, many);
       const int per = (int)(cus / 8);
       const long slots = prefill_tiles(p, WF, EPI, EPI == SK_GATEUP ? r / 2 : r, tk);
-      const LastRound last = last_round(slots, per);
+      const LastRound last = split ? last_round(slots, per) : kLastWhole;
       const long n = last == kLastWhole ? (slots + per - 1) / per : slots / per;
-      return (float)n * (n > 1 ? many : one) + (last == kLastWhole ? 0.f : second + (last == kLastHalves ? halves : quarters));
+      return (float)n * (n > 1 ? many : one) + (last == kLastWhole ? 0.f : second + (last == kLastQuarters ? 42.f : pipe8 ? 60.f : 53.f));
     };
-    best = rounds(256, 256, pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f, pipe8 ? 60.f : 53.f, 42.f);
+    best = rounds(256, 256, pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f, true);
     which = 4;
     auto offer = [&](int id, float cost) {
       if (cost < best * 0.97f) { best = cost; which = id; }  // bigger tiles win ties
@@ -1266,8 +1256,8 @@ static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int t
     else if (pipe && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 74.f, 80.f));
     else if (pipe) offer(8, whole(tiles(192, 256), 92.f, 98.f));  // gate/up: twelve waves beside pipelined 256 x 256 and 128 x 256
     else offer(8, whole(tiles(192, 256), 85.f, 92.f));
-    if (pipe8) offer(7, rounds(128, 256, 60.f, 64.f, 42.f, 32.5f));
-    else if (pipe) offer(7, rounds(128, 256, 53.f, 58.f, 42.f, 32.5f));  // (three LDS stages; 63 / 66 with two)
+    if (pipe8) offer(7, rounds(128, 256, 60.f, 64.f, false));
+    else if (pipe) offer(7, rounds(128, 256, 53.f, 58.f, false));  // (three LDS stages; 63 / 66 with two)
     else offer(7, whole(tiles(128, 256), WF == WF_16BIT ? 67.f : 73.f, WF == WF_16BIT ? 70.f : 76.f));
     offer(1, pairs(tiles(128, 128), 68.f, 92.f));
     if (EPI == SK_LINEAR && WF == WF_16BIT) offer(10, pairs(tiles(96, 128), 60.f, 76.f));
@@ -1281,9 +1271,9 @@ static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int t
     // that each held the whole tile took 40 / 118 / 41 us)
     offer(5, whole(tiles(64, 128), 32.5f, 31.f));
   } else {
-    // gate/up of few rows: 64 x 128 whose waves split K, as above (int8, us at 17 / 64 / 128 tokens, waves that each hold the whole K / this: 2 x 4096 rows x 2048
+    // gate/up of few rows (linears of as few have been served above): 64 x 128 whose waves split K, as above (int8, us at 17 / 64 / 128 tokens, waves that each hold the whole K / this: 2 x 4096 rows x 2048
     // 29.2 / 21.8, 31.2 / 21.3, 32.1 / 21.9, x 4096 54.7 / 34.7, 55.7 / 35.1, 57.7 / 35.2, x 8192 104 / 63, 105 / 63, 109 / 64)
-    which = EPI == SK_GATEUP ? 5 : 3;
+    which = 5;
   }
   *chosen = which;
   return best;
@@ -1319,27 +1309,27 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
     if constexpr (WF == WF_16BIT) return launch_prefill_cfg<T, WF, EPI, 2, 4, 2, 2, 4, 128, 2>(s, q);
     else return launch_prefill_cfg<T, WF, EPI, 4, 4, 1, 2, 4, 128, 2>(s, q);
   };
-  // The big tiles run in rounds of one workgroup per CU, and a last round that holds a tile for every eighth CU takes as long as a full one. At most half
-  // full it is a launch of its own: of halves of the tiles, or, for a quarter of the CUs, of quarters, on the tiles that do those in one short round. us, one
+  // The 256 x 256 tiles run in rounds of one workgroup per CU, and a last round that holds a tile for every eighth CU takes as long as a full one. At most half
+  // full it is a launch of its own: of halves of the tiles (128 x 256), or, for a quarter of the CUs, of quarters, on the tile that does those in one short round. us, one
   // launch / two: gate/up 14336 x 4096 bf16, 768 / 1280 / 1792 / 3500 tokens 167 / 159, 268 / 245, 369 / 338, 660 / 633; 8192 x 2048, 1280 / 2304 / 4352 87 / 82,
-  // 152 / 137, 254 / 241; linear 4096 x 14336, 4352 / 5120 / 6144 512 / 464, 525 / 487, 592 / 544.
-  auto in_rounds = [&](auto& big, int rows, auto& halves, auto& quarters) {
+  // 152 / 137, 254 / 241; linear 4096 x 14336, 4352 / 5120 / 6144 512 / 464, 525 / 487, 592 / 544. Of 500 products of K from 1024 to 14336 it makes nine in ten faster, halves by 7 % at
+  // the median and quarters by 12. Of 128 x 256 tiles it does not (gate/up 1024 x 11008 at 4625 tokens 218 / 227).
+  auto in_rounds = [&]() {
     PrefillGemmParams a = p;
     const int per = device_cus() / 8;
-    const long slots = prefill_tiles(a, WF, EPI, EPI == SK_GATEUP ? rows / 2 : rows, 256);
+    const long slots = prefill_tiles(a, WF, EPI, EPI == SK_GATEUP ? 128 : 256, 256);
     const LastRound last = g_prefill_tile == 0 && slots < 0x7fffffffL ? last_round(slots, per) : kLastWhole;
-    if (last == kLastWhole || p.gamma || !pipelined_loop_serves(p, WF)) return big(p);
+    if (last == kLastWhole || p.gamma || !pipelined_loop_serves(p, WF)) return pipe_256(p);
     const int rest = (int)(slots % per);
     PrefillGemmParams b = a;
     a.slots = (int)slots - rest;
-    const int st = big(a);
+    const int st = pipe_256(a);
     if (st != MUI_OK) return st;
     b.first_slot = a.slots;
-    // (256 x 256: halves are 128 x 256; 128 x 256: they are 128 x 128)
-    b.sub_rows = rows == 256 || last == kLastQuarters ? 2 : 1;
-    b.sub_toks = rows == 128 || last == kLastQuarters ? 2 : 1;
+    b.sub_rows = 2;
+    b.sub_toks = last == kLastQuarters ? 2 : 1;
     b.slots = rest * b.sub_rows * b.sub_toks;
-    return last == kLastHalves ? halves(b) : quarters(b);
+    return last == kLastHalves ? pipe_128(b) : ksplit_128(b);
   };
   {
     // 256 x 256 on 4 x 2 waves of 64 x 128 with two operand register sets (the software-pipelined
@@ -1347,7 +1337,7 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
     // (gate/up at 4096 tokens 775 -> 736 us, down 386 -> 356 us, QKV 224 -> 209 us, down at 2048
     // tokens 345 -> 315 us; bit-equal results: the same products in the same order)
     if (which == 4 && !p.gamma) {
-      const int st = in_rounds(pipe_256, 256, pipe_128, ksplit_128);
+      const int st = in_rounds();
       if (st != MUI_ERR_UNSUPPORTED) return st;
     }
   }
@@ -1356,7 +1346,7 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
     if (g_prefill_pipe_small && !p.gamma) {
       int st = MUI_ERR_UNSUPPORTED;
       // 128 x 256, 2 x 4 waves of 64 x 64, three LDS stages
-      if (which == 7) st = in_rounds(pipe_128, 128, ksplit_128, ksplit_64);
+      if (which == 7) st = pipe_128(p);
       if constexpr (EPI == SK_LINEAR) {
         // 192 x 256, 4 x 2 waves of 48 x 128
         if (which == 8) {
@@ -1384,7 +1374,7 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
   if (which == 7) return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 4, 1, 64, 2>(s, p);      // 128 x 256, 2 x 4 waves of 64 x 64
   if (which == 9) return ksplit_128(p);
   if (which == 11) return launch_prefill_cfg<T, WF, EPI, 2, 4, 4, 1, 4, 128, 2>(s, p);    // 128 x 64, 4 x 1 waves x 4 shares of K
-  if (which == 5) return ksplit_64(p);
+  if (which == 5 || (which == 12 && EPI == SK_GATEUP)) return ksplit_64(p);
   if constexpr (EPI == SK_LINEAR && WF == WF_16BIT) {
     // 32 x 64 on eight waves (2 row halves x 4 shares of K): QKV at 64 tokens 21.7 -> 20.7 us, o_proj 20.2 -> 19.1 us
     if (which == 6) return launch_prefill_cfg<T, WF, EPI, 1, 4, 2, 1, 4, 256, 2>(s, p);
@@ -1393,15 +1383,8 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
   if constexpr (EPI == SK_LINEAR) {
     if (which == 12) return launch_prefill_cfg<T, WF, EPI, 4, 4, 1, 1, 4, 256, 2>(s, p);  // int8: four waves that each hold the 64 x 64 tile
   }
-  if (which == 12) which = 5;
   if (which == 6) return launch_prefill_cfg<T, WF, EPI, 2, 4, 1, 1, 4, 256, 2>(s, p);   // 32 x 64, four waves that each hold the tile split K
-  if (which == 1) return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 2, 1, 64, 2>(s, p);
-  if constexpr (EPI == SK_GATEUP) {
-    return launch_prefill_cfg<T, WF, EPI, 2, 4, 2, 2, 1, 128, 1>(s, p);
-  } else {
-    if (which == 2) return launch_prefill_cfg<T, WF, EPI, 2, 4, 2, 2, 1, 128, 1>(s, p);
-    return launch_prefill_cfg<T, WF, EPI, 1, 2, 2, 2, 1, 256, 1>(s, p);
-  }
+  return launch_prefill_cfg<T, WF, EPI, 4, 4, 2, 2, 1, 64, 2>(s, p);
 }
 
 // Products whose last token tiles hold few tokens: the number of tokens to leave to a launch of their own, for whole 256-token tiles in front of it -- or 0. 520
@@ -1529,6 +1512,7 @@ extern "C" int mui_tune_prefill(int tile, int wide_max_tokens) {
   if (tile >= 200) tile -= 200;
   const int dma = tile >= 100 ? 0 : 1;
   if (tile >= 100) tile -= 100;
+  if (tile == 2 || tile == 3) tile += 3;  // (64 x 128, 32 x 64: by waves that split K)
   if (tile < 0 || tile > 13 || wide_max_tokens > 128) return MUI_ERR_INVALID_ARG;
   mui::g_prefill_stages3_big = stages3_big;
   mui::g_prefill_stages3 = stages3;
