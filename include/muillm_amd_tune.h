@@ -83,6 +83,13 @@ int mui_tune_skinny(int min_tokens, int stream_b, int multi_max_tokens);
  * instead of the LDS-tiled one (0 restores the built-in choice; at most 128; negative: never) */
 int mui_tune_prefill(int tile, int wide_max_tokens);
 
+/* Measurement aid: what the built-in rules do with a prompt product on tiles whose operands are dense and aligned to 16 bytes (needs no GPU). weight_format
+ * 0 = 16-bit, 1 = int8 with a scale per row, 2 = int8 in groups of 1 << group_size_shift; scratch: whether a workspace is given.
+ * *rest_tokens: how many of the last tokens are a launch of their own; *tile: the tile of the others, as numbered above;
+ * *last_round: 0 = one launch of it, 1 / 2 = its last round as a launch of halves / quarters. */
+int mui_probe_prefill_plan(int dtype, int weight_format, int gateup, int n, int k, int tokens, int group_size_shift, int scratch, int* rest_tokens,
+                           int* tile, int* last_round);
+
 /* The kernel that streams 16-bit weights for 17..128 tokens: weight rows per unit (8, 16, 24, 32, 40, 48, 56, 64, 96 or 128; gate and up
  * rows together 16, 32, 48, 64, 96 or 112) and shares of K (1..8; more than one needs a workspace). 0 restores the built-in
  * choice. A pair that does not exist for a call (too wide for its tokens, more units than CUs, less than 512 k-values a

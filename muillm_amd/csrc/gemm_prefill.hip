@@ -1063,6 +1063,9 @@ static bool lds_direct_loads_serve(const PrefillGemmParams& p, int wf) {
          (wf != WF_U8_GROUP || (p.group_shift >= 6 && p.s_pitch % 2 == 0 && (((uintptr_t)p.s0 | (uintptr_t)p.s1) & 3) == 0));
 }
 static bool pipelined_loop_serves(const PrefillGemmParams& p, int wf) { return lds_direct_loads_serve(p, wf); }
+static bool pipelined(const PrefillGemmParams& p, int dtype, int wf) {
+  return (wf != WF_U8_GROUP || dtype == MUI_DTYPE_F16) && !p.gamma && pipelined_loop_serves(p, wf);
+}
 
 // Tiles of `outputs` outputs x `toks` tokens and how the XCDs divide them; returns the slots of an XCD
 static long prefill_tiles(PrefillGemmParams& p, int wf, int epi, int outputs, int toks) {
@@ -1194,7 +1197,14 @@ static LastRound last_round(long slots, int per) {
   return 4 * rest <= per ? kLastQuarters : kLastHalves;
 }
 
-// What it takes to multiply `tokens` tokens, in microseconds at K = 4096, and with which tile (see launch_prefill_t); 0 where no tile's cost was compared
+struct PrefillPlan {
+  float cost;      // microseconds at K = 4096; 0 where no tile's cost was compared
+  int tile;        // see launch_prefill_t
+  LastRound last;
+  float settled;   // cost, with less for a last round of big tiles that leaves CUs idle: the others' clock rises, half of what is idle is made up for
+};
+
+// How `tokens` tokens are multiplied, and what it takes.
 // Big tiles re-read x and the weights least and keep the LDS traffic per matrix instruction
 // low, but a grid much smaller than the chip leaves the work to too few CUs, and a grid of one
 // and a bit rounds of workgroups costs two rounds. Each shape has a cost per round of
@@ -1204,13 +1214,14 @@ static LastRound last_round(long slots, int per) {
 // (122 us) against 256 (99 us); o_proj and down at 2048 tokens are 128 tiles of 256 x 256 (112 / 363 us)
 // and 256 of 128 x 256 (78 / 270 us); QKV at 512 is 192 tiles of 128 x 128 (68 us), 256 of
 // 96 x 128 (62 us). Where 64 x 128 tiles number half the CUs at most, tiles whose waves split K.
-static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int tokens, int* chosen) {
+static PrefillPlan prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int tokens) {
   p.tokens = tokens;
   const long rows = (EPI == SK_GATEUP) ? 2L * p.n : p.n;
   const long cus = device_cus();
   auto tiles = [&](int r, int tk) { return (long)ceil_div((int)rows, r) * ceil_div(tokens, tk); };
   int which;
   float best = 0.f;
+  LastRound big_last = kLastWhole;
   // few output tiles (short prompts on the 4096-row matrices): one workgroup per tile whose
   // waves split every k-step between them -- four waves that each hold the whole 32 x 64 tile,
   // or eight waves in two token halves of a 64 x 128 or 128 x 128 tile: the LDS traffic per
@@ -1245,6 +1256,7 @@ static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int t
       const long slots = prefill_tiles(p, WF, EPI, EPI == SK_GATEUP ? r / 2 : r, tk);
       const LastRound last = split ? last_round(slots, per) : kLastWhole;
       const long n = last == kLastWhole ? (slots + per - 1) / per : slots / per;
+      if (split) big_last = last;
       return (float)n * (n > 1 ? many : one) + (last == kLastWhole ? 0.f : second + (last == kLastQuarters ? 42.f : pipe8 ? 60.f : 53.f));
     };
     best = rounds(256, 256, pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f, true);
@@ -1275,14 +1287,19 @@ static float prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe, int t
     // 29.2 / 21.8, 31.2 / 21.3, 32.1 / 21.9, x 4096 54.7 / 34.7, 55.7 / 35.1, 57.7 / 35.2, x 8192 104 / 63, 105 / 63, 109 / 64)
     which = 5;
   }
-  *chosen = which;
-  return best;
+  const LastRound last = which == 4 ? big_last : kLastWhole;
+  float settled = best;
+  if (best > 0.f && last == kLastWhole && (which == 4 || which == 7 || which == 8)) {
+    const long n = tiles(which == 4 ? 256 : which == 7 ? 128 : 192, 256), full = (n + cus - 1) / cus;
+    settled -= 0.5f * best / (float)full * (float)(full * cus - n) / (float)cus;
+  }
+  return {best, which, last, settled};
 }
 
 template <typename T, int WF, int EPI>
 static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
   int which = g_prefill_tile;
-  if (which == 0) prefill_plan(p, WF, EPI, kPipelined<T, WF> && !p.gamma && pipelined_loop_serves(p, WF), p.tokens, &which);
+  if (which == 0) which = prefill_plan(p, WF, EPI, kPipelined<T, WF> && !p.gamma && pipelined_loop_serves(p, WF), p.tokens).tile;
   // Where the software-pipelined eight-wave loop does not apply (fused norm, int8 weights, K not a
   // multiple of 64): sixteen waves per workgroup (four per SIMD, at most 128 registers each) on all
   // but the smallest shapes, with the compiler's own schedule 3-16 % ahead of eight waves with twice
@@ -1389,31 +1406,43 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
 
 // Products whose last token tiles hold few tokens: the number of tokens to leave to a launch of their own, for whole 256-token tiles in front of it -- or 0. 520
 // tokens of a 14336 x 4096 gate/up are 336 tiles of 256 x 256 where 512 are 224, one round of workgroups; the weights of the few are read again instead, by the
-// kernels that stream them (16-bit ones find some of them in the last cache; int8 beyond 64 tokens, on tiles, has 16 us of ramp whatever K is). Taken where the plan says that it gains, of
-// linears, whose big tiles cost less than planned where they leave CUs idle, 15 % and only from 2048 tokens on. us, one launch / two: gate/up 14336 x 4096 bf16, 520 / 640
-// / 1032 / 1152 / 1544 / 1664 tokens 165 / 146, 165 / 145, 262 / 224, 265 / 241, 361 / 314, 367 / 336; 8192 x 2048, 520 / 1032 / 1152 / 2056 49 / 47, 84 / 70, 86 / 75,
-// 147 / 124; int8 per channel 14336 x 4096 (fp16), 520 / 1032 / 1100 180 / 130, 286 / 225, 289 / 256; linears 4096 x 14336, 2056 / 4104 253 / 216, 478 / 365; 4096 x 4096
-// 84 / 73, 153 / 121; not taken: linear 2048 x 8192 at 2056 86 / 89, 4096 x 14336 at 520 117 / 124.
-static int rest_tokens(const PrefillGemmParams& p, int wf, int epi, bool pipelined) {
+// kernels that stream them or, what those decline, by tiles: 16 to 42 us a round at K = 4096 and 5 of ramp, next to the streaming kernel's own estimate and its ramp (groups of codes take
+// 1.6 times that estimate). The two launches take what each takes alone, within 5 %, so they are taken where the sum is less; of linears, whose big tiles the plan knows less well,
+// 15 % less and only from 2048 tokens on. us, one launch / two: gate/up 14336 x 4096 bf16, 520 / 640
+// / 1032 / 1152 / 1544 / 1664 tokens 165 / 146, 165 / 145, 262 / 224, 265 / 241, 361 / 314, 367 / 336; 14336 x 2880 (tiles) 520 / 1032 120 / 110, 196 / 171; 8192 x 2048, 1032 / 1152 / 2056
+// 84 / 70, 86 / 75, 147 / 124; int8 per channel 14336 x 4096 (fp16), 520 / 1032 / 1100 180 / 130, 286 / 225, 289 / 256; linears 4096 x 14336, 4104 478 / 365; 4096 x 4096
+// 153 / 121; not taken: gate/up 8192 x 8256 at 520 166 / 180, 2048 x 8256 int8 at 529 69 / 123, 2560 x 11008 int8 at 2305 238 / 452, linear 2048 x 8192 at 2056 86 / 89, 4096 x 14400 at 2088 223 / 247. Of
+// 600 products of 512 to 8191 tokens that end up to 128 beyond a whole tile it takes 88, none of them slower by more than 2 %; the sum of logarithms is 1.1 % less than without, 2.1 at best.
+static int rest_tokens(const PrefillGemmParams& p, const SkinnyParams& q, int dtype, int wf, int epi, bool pipelined, size_t part_bytes) {
   const int rest = p.tokens % 256;
   if (!g_prefill_bands || !pipelined || p.tokens < (epi == SK_GATEUP ? 512 : 2048) || rest == 0 || rest > 128) return 0;
-  int which = 0;
-  const float together = prefill_plan(p, wf, epi, true, p.tokens, &which), whole = prefill_plan(p, wf, epi, true, p.tokens - rest, &which);
+  const float together = prefill_plan(p, wf, epi, true, p.tokens).settled, whole = prefill_plan(p, wf, epi, true, p.tokens - rest).settled;
   if (together <= 0.f || whole <= 0.f) return 0;
-  const float per_k = 4096.f / (float)p.k;
-  float few;
-  if (epi == SK_GATEUP) {
-    const float per_weight = wf == WF_16BIT ? (rest <= 32 ? 28.f : rest <= 64 ? 36.f : 46.f) : rest > 64 ? 38.f : wf == WF_I8_CHANNEL && rest <= 32 ? 22.f : 35.f;
-    few = (wf == WF_16BIT ? 6.f + 6.f * per_k : (rest <= 64 ? 6.f : 16.f) * per_k) + (float)p.n / 14336.f * per_weight;
+  const float per_k = (float)p.k / 4096.f;
+  SkinnyParams few = q;
+  few.tokens = rest;
+  float us = gemm_stream_time(dtype, wf, epi, few, part_bytes);
+  if (us >= 0.f) {
+    us = wf == WF_16BIT ? us + 3.5f : wf == WF_I8_CHANNEL ? us + 4.5f : 1.6f * us + 4.f;
   } else {
-    const float per_weight = wf == WF_16BIT ? (rest <= 16 ? 3.f : rest <= 32 ? 5.5f : rest <= 64 ? 8.f : 12.5f) : rest <= 64 ? 8.f : 14.f;
-    few = (wf == WF_16BIT ? 5.f : rest <= 64 ? 6.f : 8.f) * per_k + (float)p.n / 4096.f * per_weight;
+    const PrefillPlan tiles = prefill_plan(p, wf, epi, true, rest);
+    us = 5.f + per_k * (tiles.cost > 0.f ? tiles.cost : tiles.tile == 6 ? 16.f : tiles.tile == 12 ? 22.f : 32.5f);
   }
-  return whole + few < (epi == SK_GATEUP ? 0.985f : 0.85f) * together ? rest : 0;
+  return whole * per_k + us < (epi == SK_GATEUP ? 0.97f : 0.85f) * together * per_k ? rest : 0;
 }
 
 constexpr int kWideDefaultMaxTokens = 0;  // 0: the built-in rule below
 static int g_wide_max_tokens = kWideDefaultMaxTokens;  // longest prompt taken by gemm_wide.hip
+
+static PrefillGemmParams prefill_params(const SkinnyParams& q, int wf) {
+  PrefillGemmParams p = {};
+  const long esz = (wf == WF_16BIT) ? 2 : 1;
+  p.w0 = (const uint8_t*)q.w0; p.w1 = (const uint8_t*)q.w1; p.pitch = q.pitch * esz;
+  p.s0 = q.s0; p.s1 = q.s1; p.s_pitch = q.s_pitch; p.group_shift = q.group_shift;
+  p.x = q.x; p.gamma = q.gamma; p.mul_bias = q.mul_bias; p.add_bias = q.add_bias; p.residual = q.residual;
+  p.y = q.y; p.y_pitch = q.n; p.n = q.n; p.k = q.k; p.tokens = q.tokens; p.eps = q.eps;
+  return p;
+}
 
 // Any number of tokens >= 1 (meant for more than MUI_MAX_TOKENS), 16-bit weights or per-channel
 // int8 codes; SkinnyParams as for the decode kernels (x, residual and y dense).
@@ -1423,12 +1452,7 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   // What it declines: up to 40 tokens 16 rows per workgroup, K split over the waves, no LDS tiling
   // (gemm_wide.hip), while its grid is a single round of workgroups (o_proj at 33 tokens 16.0 vs 20.4 us for the smallest LDS
   // tile, 19.6 vs 20.6 at 48, 23.1 vs 21.2 at 64)
-  PrefillGemmParams p = {};
-  const long esz = (wf == WF_16BIT) ? 2 : 1;
-  p.w0 = (const uint8_t*)q.w0; p.w1 = (const uint8_t*)q.w1; p.pitch = q.pitch * esz;
-  p.s0 = q.s0; p.s1 = q.s1; p.s_pitch = q.s_pitch; p.group_shift = q.group_shift;
-  p.x = q.x; p.gamma = q.gamma; p.mul_bias = q.mul_bias; p.add_bias = q.add_bias; p.residual = q.residual;
-  p.y = q.y; p.y_pitch = q.n; p.n = q.n; p.k = q.k; p.tokens = q.tokens; p.eps = q.eps;
+  const PrefillGemmParams p = prefill_params(q, wf);
   const bool scratch = q.workspace && ((uintptr_t)q.workspace & 255u) == 0 && q.workspace_bytes >= prefill_workspace_bytes();
   if (q.tokens <= 128 && g_prefill_tile == 0 && g_wide_max_tokens == kWideDefaultMaxTokens) {
     float* part = scratch ? (float*)((char*)q.workspace + kXsCounterBytes) : nullptr;
@@ -1456,8 +1480,7 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   if (q.k % (wf == WF_16BIT ? 8 : 16)) return MUI_ERR_UNSUPPORTED;
   if (q.x_pitch != 0 && q.x_pitch != q.k) return MUI_ERR_UNSUPPORTED;
   if (g_prefill_tile == 0 && !q.gamma) {
-    const bool pipelined = (dtype == MUI_DTYPE_F16 || wf != WF_U8_GROUP) && pipelined_loop_serves(p, wf);
-    const int rest = rest_tokens(p, wf, epilogue, pipelined);
+    const int rest = rest_tokens(p, q, dtype, wf, epilogue, pipelined(p, dtype, wf), scratch ? q.workspace_bytes - kXsCounterBytes : 0);
     if (rest) {
       SkinnyParams a = q, b = q;
       a.tokens = q.tokens - rest;
@@ -1488,6 +1511,25 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
 }
 
 }  // namespace mui
+
+extern "C" int mui_probe_prefill_plan(int dtype, int weight_format, int gateup, int n, int k, int tokens, int group_size_shift, int scratch, int* rest_tokens,
+                                      int* tile, int* last_round) {
+  using namespace mui;
+  MUI_CHECK_ARG((dtype == MUI_DTYPE_F16 || dtype == MUI_DTYPE_BF16) && weight_format >= 0 && weight_format <= 2 && n >= 1 && k >= 1 && tokens >= 1 && rest_tokens &&
+                tile && last_round);
+  const int wf = weight_format == 0 ? WF_16BIT : weight_format == 1 ? WF_I8_CHANNEL : WF_U8_GROUP, epi = gateup ? SK_GATEUP : SK_LINEAR;
+  SkinnyParams q = {};
+  q.pitch = k; q.n = n; q.k = k; q.tokens = tokens; q.group_shift = group_size_shift;
+  q.s_pitch = wf == WF_U8_GROUP ? 2L * (k >> group_size_shift) : 1;
+  PrefillGemmParams p = prefill_params(q, wf);
+  const bool pipe = pipelined(p, dtype, wf);
+  *rest_tokens = mui::rest_tokens(p, q, dtype, wf, epi, pipe, scratch && wf == WF_16BIT ? prefill_workspace_bytes() - kXsCounterBytes : 0);
+  p.tokens -= *rest_tokens;
+  const PrefillPlan plan = prefill_plan(p, wf, epi, pipe, p.tokens);
+  *tile = plan.tile;
+  *last_round = plan.last;
+  return MUI_OK;
+}
 
 extern "C" int mui_tune_prefill(int tile, int wide_max_tokens) {
   MUI_TUNE_GUARD();

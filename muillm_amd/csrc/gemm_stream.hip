@@ -443,8 +443,13 @@ static bool codes_are_faster_elsewhere(bool groups, bool bf16, int epi, int toke
 
 static int g_stream_rows = 0, g_stream_shares = 0;  // mui_tune_stream
 
-template <typename T, int EPI, int WF = WF_16BIT>
-static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int* splits = nullptr) {
+// (forced units that do not exist are an error, but where the kernel has none for the call at all)
+template <int EPI, int WF>
+static bool stream_forced_must_exist(int tokens) { return WF == WF_16BIT && (EPI == SK_LINEAR || stream_token_tiles(tokens) <= 4); }
+
+// The time of the units that it chooses in us, or a negative number where another kernel is faster or, with forced units, none exist (*width 0 then)
+template <typename T, int EPI, int WF>
+static float plan_stream(StreamParams& p, size_t part_bytes, int* chosen) {
   constexpr bool W8 = WF != WF_16BIT;
   // Rows per unit and shares of K by the least time: what a CU takes in (27.5 KB of weights, 105 KB of token rows per microsecond, 82 in
   // steps of 128 k-values), a barrier per step, a fixed part per round of workgroups; for shares of K the second launch and the
@@ -469,15 +474,27 @@ static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int
       if (width == 0 || cost < best) { best = cost; width = r; p.n_units = units; p.k_splits = k; }
     }
   }
+  *chosen = width;
   const bool forced = g_stream_rows || g_stream_shares;
-  if (!p.add && p.k_splits == 1) return MUI_ERR_UNSUPPORTED;
+  if ((!p.add && p.k_splits == 1) || !width) return -1.f;
+  if (forced) return best;
+  if constexpr (W8) {
+    if (codes_are_faster_elsewhere(WF == WF_U8_GROUP, T::kDtype == MUI_DTYPE_BF16, EPI, p.tokens, rows, p.k, width, p.n_units)) return -1.f;
+  } else if constexpr (EPI == SK_GATEUP) {
+    if (gateup_tiles_are_faster(p.tokens, rows, p.k, p.n_units)) return -1.f;
+  } else {
+    if (wide_is_faster(p.tokens, rows, p.k)) return -1.f;
+    if (p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return -1.f;
+  }
+  return best;
+}
+
+template <typename T, int EPI, int WF = WF_16BIT>
+static int launch_stream_t(hipStream_t s, StreamParams p, size_t part_bytes, int* splits = nullptr) {
+  int width = 0;
+  const float us = plan_stream<T, EPI, WF>(p, part_bytes, &width);
   if (splits) *splits = p.k_splits;
-  if (!forced && !W8 && EPI == SK_LINEAR && wide_is_faster(p.tokens, rows, p.k)) return MUI_ERR_UNSUPPORTED;
-  if (!width && (W8 || (EPI == SK_GATEUP && nt > 4))) return MUI_ERR_UNSUPPORTED;
-  if (forced && !width) return MUI_ERR_INVALID_ARG;
-  if (!forced && !W8 && EPI == SK_LINEAR && p.k_splits == 1 && tiles_are_faster(p.tokens, rows, p.k, width, ceil_div(p.n_units, cus))) return MUI_ERR_UNSUPPORTED;
-  if (!forced && W8 && codes_are_faster_elsewhere(WF == WF_U8_GROUP, T::kDtype == MUI_DTYPE_BF16, EPI, p.tokens, rows, p.k, width, p.n_units)) return MUI_ERR_UNSUPPORTED;
-  if (!forced && !W8 && EPI == SK_GATEUP && gateup_tiles_are_faster(p.tokens, rows, p.k, p.n_units)) return MUI_ERR_UNSUPPORTED;
+  if (us < 0.f) return (g_stream_rows || g_stream_shares) && p.add && !width && stream_forced_must_exist<EPI, WF>(p.tokens) ? MUI_ERR_INVALID_ARG : MUI_ERR_UNSUPPORTED;
   switch (width) {
     case 16: return launch_stream_rows<T, EPI, 16, WF>(s, p);
     case 32: return launch_stream_rows<T, EPI, 32, WF>(s, p);
@@ -515,6 +532,31 @@ static StreamParams stream_params(const SkinnyParams& q, float* part, bool add, 
   return p;
 }
 
+// (pairs are read in fours of bytes)
+static bool stream_serves_codes(const SkinnyParams& q, int wf) {
+  if (!stream_serves(q, 64, true)) return false;
+  if (wf == WF_I8_CHANNEL) return true;
+  return wf == WF_U8_GROUP && q.group_shift >= 6 && q.k % (1 << q.group_shift) == 0 && q.s_pitch % 2 == 0 && (((uintptr_t)q.s0 | (uintptr_t)q.s1) & 3) == 0;
+}
+
+template <typename T, int WF>
+static float stream_time_t(int epilogue, StreamParams p, size_t part_bytes) {
+  int width = 0;
+  return epilogue == SK_GATEUP ? plan_stream<T, SK_GATEUP, WF>(p, 0, &width) : plan_stream<T, SK_LINEAR, WF>(p, part_bytes, &width);
+}
+
+// What the launches below take in us, by the plan that chooses their units, or a negative number for what they decline
+float gemm_stream_time(int dtype, int wf, int epilogue, const SkinnyParams& q, size_t part_bytes) {
+  if (!(wf == WF_16BIT ? stream_serves(q, 128) : stream_serves_codes(q, wf))) return -1.f;
+  const StreamParams p = stream_params(q, nullptr, true, wf != WF_16BIT);
+  auto of = [&](auto t) {
+    using T = decltype(t);
+    return wf == WF_16BIT ? stream_time_t<T, WF_16BIT>(epilogue, p, part_bytes)
+           : wf == WF_I8_CHANNEL ? stream_time_t<T, WF_I8_CHANNEL>(epilogue, p, 0) : stream_time_t<T, WF_U8_GROUP>(epilogue, p, 0);
+  };
+  return dtype == MUI_DTYPE_F16 ? of(F16{}) : dtype == MUI_DTYPE_BF16 ? of(BF16{}) : -1.f;
+}
+
 // 17..128 tokens, 16-bit weights, no fused norm, x / residual / y dense; MUI_ERR_UNSUPPORTED for what the loads cannot serve and for
 // what another kernel does faster
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
@@ -534,11 +576,9 @@ static int launch_stream_codes(hipStream_t s, int dtype, int epilogue, const Str
 
 // The same for int8 codes, 17 to 64 tokens; groups of 64 or more
 int launch_gemm_stream_int8(hipStream_t s, int dtype, int wf, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
-  if (!stream_serves(q, 64, true)) return MUI_ERR_UNSUPPORTED;
+  if (!stream_serves_codes(q, wf)) return MUI_ERR_UNSUPPORTED;
   const StreamParams p = stream_params(q, part, true, true);
   if (wf == WF_I8_CHANNEL) return launch_stream_codes<WF_I8_CHANNEL>(s, dtype, epilogue, p, part_bytes);
-  // (pairs are read in fours of bytes)
-  if (wf != WF_U8_GROUP || q.group_shift < 6 || q.k % (1 << q.group_shift) || q.s_pitch % 2 || (((uintptr_t)q.s0 | (uintptr_t)q.s1) & 3)) return MUI_ERR_UNSUPPORTED;
   return launch_stream_codes<WF_U8_GROUP>(s, dtype, epilogue, p, part_bytes);
 }
 

@@ -206,6 +206,7 @@ int launch_gemm_wide(hipStream_t s, int dtype, int weight_format, int epilogue, 
 // 17..128 tokens, 16-bit weights, k % 256 == 0, n % 8 == 0, no fused norm: bands of weight rows streamed through LDS stages that
 // the workgroup shares; part (part_bytes, may be none): fp32 partial outputs where shares of K are worth it (gemm_stream.hip). MUI_ERR_UNSUPPORTED
 // for everything else and for what the tiled GEMM does faster
+float gemm_stream_time(int dtype, int weight_format, int epilogue, const SkinnyParams& p, size_t part_bytes);  // of the next two, in us; negative: they decline
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);
 int launch_gemm_stream_int8(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);  // codes, 17..64 tokens
 int launch_gemm_stream_parts(hipStream_t s, int dtype, const SkinnyParams& p, float* part, size_t part_bytes, int* splits);
