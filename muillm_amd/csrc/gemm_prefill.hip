@@ -1247,6 +1247,9 @@ static PrefillPlan prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe,
   // 256 tokens 32 -> 23.5 us (k-steps of 128 instead of 256: 28.6 / 27.2 us)
   else if (EPI == SK_LINEAR && tiles(64, 64) <= cus) which = 12;
   else if (tiles(256, 256) >= 5 * cus / 8 || 2 * tiles(64, 128) > cus) {
+    // Rounds are counted from what the fullest XCD has: 36 row tiles of 7 token tiles are 252 workgroups, but four XCDs have 35 for their 32 CUs. (Counted from all of the grid for some
+    // tiles, as it was, gate/up 2304 x 4096 at 1764 tokens took 121 us for 106, linear 5120 x 14336 at 2198 439 for 295; of 920 products 44 were more than 10 % above their best tile, now 19.)
+    auto grid = [&](int r, int tk) { return 8 * prefill_tiles(p, WF, EPI, EPI == SK_GATEUP ? r / 2 : r, tk); };
     // one workgroup per CU (eight waves): rounds x cost, a little more per round once the
     // rounds follow each other (their weights compete for the L2)
     auto whole = [&](long n_tiles, float one, float many) {
@@ -1264,38 +1267,35 @@ static PrefillPlan prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe,
     // (and their last round goes to smaller tiles where it is at most half full. A launch of its own for it costs a linear more: its big tiles end on time of
     // their own, 107 us at K = 4096 where the plan has 96, and the 192 x 256 tile is close behind: 6144 x 4096 at 3500 tokens 174 us with quarters, 159 on that)
     const float second = (EPI == SK_GATEUP ? 8.f : 28.f) * 4096.f / (float)p.k;
-    auto rounds = [&](int r, int tk, float one, float many, bool split) {
-      if (!pipe) return whole(tiles(r, tk), one, many);
-      const int per = (int)(cus / 8);
-      const long slots = prefill_tiles(p, WF, EPI, EPI == SK_GATEUP ? r / 2 : r, tk);
-      const LastRound last = split ? last_round(slots, per) : kLastWhole;
-      const long n = last == kLastWhole ? (slots + per - 1) / per : slots / per;
-      if (split) big_last = last;
-      return (float)n * (n > 1 ? many : one) + (last == kLastWhole ? 0.f : second + (last == kLastQuarters ? 42.f : pipe8 ? 60.f : 53.f));
-    };
-    best = rounds(256, 256, pipe8 ? 104.f : pipe ? 96.f : 100.f, pipe8 ? 109.f : pipe ? 100.f : 111.f, true);
+    const float one = pipe8 ? 104.f : pipe ? 96.f : 100.f, many = pipe8 ? 109.f : pipe ? 100.f : 111.f;
+    best = whole(grid(256, 256), one, many);
     which = 4;
+    if (pipe) {
+      const long per = cus / 8, slots = grid(256, 256) / 8, n = slots / per;
+      big_last = last_round(slots, (int)per);
+      if (big_last != kLastWhole) best = (float)n * (n > 1 ? many : one) + second + (big_last == kLastQuarters ? 42.f : pipe8 ? 60.f : 53.f);
+    }
     auto offer = [&](int id, float cost) {
       if (cost < best * 0.97f) { best = cost; which = id; }  // bigger tiles win ties
     };
-    if (pipe8 && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 81.f, 87.f));
-    else if (pipe && EPI == SK_LINEAR) offer(8, whole(tiles(192, 256), 74.f, 80.f));
-    else if (pipe) offer(8, whole(tiles(192, 256), 92.f, 98.f));  // gate/up: twelve waves beside pipelined 256 x 256 and 128 x 256
-    else offer(8, whole(tiles(192, 256), 85.f, 92.f));
-    if (pipe8) offer(7, rounds(128, 256, 60.f, 64.f, false));
-    else if (pipe) offer(7, rounds(128, 256, 53.f, 58.f, false));  // (three LDS stages; 63 / 66 with two)
-    else offer(7, whole(tiles(128, 256), WF == WF_16BIT ? 67.f : 73.f, WF == WF_16BIT ? 70.f : 76.f));
-    offer(1, pairs(tiles(128, 128), 68.f, 92.f));
-    if (EPI == SK_LINEAR && WF == WF_16BIT) offer(10, pairs(tiles(96, 128), 60.f, 76.f));
+    if (pipe8 && EPI == SK_LINEAR) offer(8, whole(grid(192, 256), 81.f, 87.f));
+    else if (pipe && EPI == SK_LINEAR) offer(8, whole(grid(192, 256), 74.f, 80.f));
+    else if (pipe) offer(8, whole(grid(192, 256), 92.f, 98.f));  // gate/up: twelve waves beside pipelined 256 x 256 and 128 x 256
+    else offer(8, whole(grid(192, 256), 85.f, 92.f));
+    if (pipe8) offer(7, whole(grid(128, 256), 60.f, 64.f));
+    else if (pipe) offer(7, whole(grid(128, 256), 53.f, 58.f));  // (three LDS stages; 63 / 66 with two)
+    else offer(7, whole(grid(128, 256), WF == WF_16BIT ? 67.f : 73.f, WF == WF_16BIT ? 70.f : 76.f));
+    offer(1, pairs(grid(128, 128), 68.f, 92.f));
+    if (EPI == SK_LINEAR && WF == WF_16BIT) offer(10, pairs(grid(96, 128), 60.f, 76.f));
     // 128 x 128 on waves that split K: the fastest single tile (QKV at 512 tokens 43 vs 62 us,
     // o_proj at 1024 44 vs 68 us, down at 1024 139 vs 219 us), one per CU
-    offer(9, whole(tiles(128, 128), 42.f, 40.f));
+    offer(9, whole(grid(128, 128), 42.f, 40.f));
     // the same with 64-token tiles: half the token bytes per workgroup for prompts of up to 64
     // tokens (gate/up at 64 tokens 57 -> 50 us)
-    offer(11, whole(tiles(128, 64), 37.f, 36.5f));
+    offer(11, whole(grid(128, 64), 37.f, 36.5f));
     // 64 x 128 likewise (o_proj at 512 tokens 32 us, down 99 us, QKV at 256 33 us; four waves
     // that each held the whole tile took 40 / 118 / 41 us)
-    offer(5, whole(tiles(64, 128), 32.5f, 31.f));
+    offer(5, whole(grid(64, 128), 32.5f, 31.f));
   } else {
     // gate/up of few rows (linears of as few have been served above): 64 x 128 whose waves split K, as above (int8, us at 17 / 64 / 128 tokens, waves that each hold the whole K / this: 2 x 4096 rows x 2048
     // 29.2 / 21.8, 31.2 / 21.3, 32.1 / 21.9, x 4096 54.7 / 34.7, 55.7 / 35.1, 57.7 / 35.2, x 8192 104 / 63, 105 / 63, 109 / 64)

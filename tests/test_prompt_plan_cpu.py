@@ -24,3 +24,11 @@ def test_never():
     for weights, form, n, k, tokens in [("bf16", "gateup", 14336, 4096, 512), ("bf16", "gateup", 14336, 4096, 512 + 129), ("bf16", "gateup", 14336, 4096, 511),
                                         ("bf16", "linear", 4096, 4096, 2047), ("bf16", "gateup", 14336, 4096 + 8, 520), ("int8", "gateup", 14336, 4096 + 16, 520)]:
         assert prompt_plan(weights, form, n, k, tokens)[0] == 0
+
+
+@pytest.mark.parametrize("weights,form,n,k,tokens,tile", [
+    ("bf16", "gateup", 1024, 1024, 5392, 4), ("bf16", "gateup", 2304, 11008, 388, 9), ("int8_group", "linear", 2304, 14336, 772, 9), ("int8", "linear", 4104, 14336, 2593, 4),
+    ("fp16", "linear", 3584, 14336, 1032, 7), ("fp16", "linear", 5120, 14336, 2198, 4), ("int8", "linear", 5120, 1024, 3199, 8)])
+def test_rounds_are_counted_by_the_fullest_xcd(weights, form, n, k, tokens, tile):
+    """Row tiles that do not come out even over the eight XCDs: products that took 1.4 to 1.6 times as long on another tile."""
+    assert prompt_plan(weights, form, n, k, tokens)[1] == tile
