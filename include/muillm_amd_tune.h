@@ -90,8 +90,8 @@ int mui_tune_prefill(int tile, int wide_max_tokens);
 int mui_probe_prefill_plan(int dtype, int weight_format, int gateup, int n, int k, int tokens, int group_size_shift, int scratch, int* rest_tokens,
                            int* tile, int* last_round);
 
-/* The kernel that streams 16-bit weights for 17..128 tokens: weight rows per unit (8, 16, 24, 32, 40, 48, 56, 64, 96 or 128; gate and up
- * rows together 16, 32, 48, 64, 96 or 112) and shares of K (1..8; more than one needs a workspace). 0 restores the built-in
+/* The kernel that streams 16-bit weights for 17..128 tokens and codes for 17..64: weight rows per unit (8, 16, 24, 32, 40, 48, 56, 64, 96 or 128; gate and up
+ * rows together 16, 32, 48, 64, 96 or 112) and shares of K (1..8; more than one needs a workspace, and codes have none). 0 restores the built-in
  * choice. A pair that does not exist for a call (too wide for its tokens, more units than CUs, less than 512 k-values a
  * share) makes the call return MUI_ERR_INVALID_ARG. */
 int mui_tune_stream(int rows_per_unit, int shares);

@@ -1471,7 +1471,7 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   if (q.tokens <= 128 && g_prefill_tile == 0 && g_wide_max_tokens == kWideDefaultMaxTokens) {
     float* part = scratch ? (float*)((char*)q.workspace + kXsCounterBytes) : nullptr;
     const size_t part_bytes = scratch ? q.workspace_bytes - kXsCounterBytes : 0;
-    const int st = wf == WF_16BIT ? launch_gemm_stream(s, dtype, epilogue, q, part, part_bytes) : launch_gemm_stream_int8(s, dtype, wf, epilogue, q, part, part_bytes);
+    const int st = wf == WF_16BIT ? launch_gemm_stream(s, dtype, epilogue, q, part, part_bytes) : launch_gemm_stream_int8(s, dtype, wf, epilogue, q);
     if (st != MUI_ERR_UNSUPPORTED) return st;
   }
   // a caller-provided workspace lets a long K be shared between workgroups when the tiles are few

@@ -38,7 +38,7 @@ struct StreamParams {
   bool add;        // a launch behind this one adds the partial outputs up (else the caller's does)
   int n, k, tokens;
   int n_units;     // bands of ROWS weight rows (gate/up: gate and up rows together)
-  int k_splits;    // more than one: every workgroup has one unit, a share of K of one band
+  int k_splits;    // more than one (16-bit weights): every workgroup has one unit, a share of K of one band
 };
 
 // Geometry for ROWS weight rows x NT token tiles of 16 per unit
@@ -107,11 +107,12 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
   const int wlr = W8 ? lane / WCPR : lr, wls = W8 ? (lane % WCPR) ^ wlr : ls;
 
   const int all_steps = p.k / KS;
-  const int share_k = p.k_splits > 1 ? (int)(blockIdx.x % (unsigned)p.k_splits) : 0;
-  const int first_unit = p.k_splits > 1 ? (int)(blockIdx.x / (unsigned)p.k_splits) : (int)blockIdx.x;
-  const int sb = (int)((long)all_steps * share_k / p.k_splits);
-  const int unit_steps = (int)((long)all_steps * (share_k + 1) / p.k_splits) - sb;
-  const int units = p.k_splits > 1 ? 1 : (p.n_units - first_unit + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int k_splits = W8 ? 1 : p.k_splits;
+  const int share_k = k_splits > 1 ? (int)(blockIdx.x % (unsigned)k_splits) : 0;
+  const int first_unit = k_splits > 1 ? (int)(blockIdx.x / (unsigned)k_splits) : (int)blockIdx.x;
+  const int sb = (int)((long)all_steps * share_k / k_splits);
+  const int unit_steps = (int)((long)all_steps * (share_k + 1) / k_splits) - sb;
+  const int units = k_splits > 1 ? 1 : (p.n_units - first_unit + (int)gridDim.x - 1) / (int)gridDim.x;
   const int steps = unit_steps * units;
   // workgroups start at different steps: their rows are whole multiples of the memory channels' interleave apart, so
   // workgroups that walked K in step would all ask the same channels (reads of a matrix 6.0 -> 6.9 TB/s)
@@ -295,7 +296,7 @@ __global__ void __launch_bounds__(kStreamThreads, 2) gemm_stream_kernel(const St
 #pragma unroll
               for (int e = 0; e < 4; ++e) a[e] *= T::one(p.s0[(o + e) * p.s_pitch]);
             }
-            if (p.k_splits > 1) {
+            if (k_splits > 1) {
               *(f32x4*)(p.part + ((long)share_k * p.tokens + tok) * p.n + o) = a;
             } else {
               float res[4] = {0.f, 0.f, 0.f, 0.f};
@@ -360,7 +361,7 @@ static int launch_stream_cfg(hipStream_t s, const StreamParams& p) {
   static_assert(G::LDS <= 160 * 1024, "LDS of a workgroup");
   const int cus = device_cus(), wgs = p.n_units * p.k_splits;
   const int st = launch_with_lds(gemm_stream_kernel<T, EPI, ROWS, NT, WF>, dim3(wgs < cus ? wgs : cus), dim3(kStreamThreads), G::LDS, s, p);
-  if (st != MUI_OK || p.k_splits == 1 || !p.add) return st;
+  if (WF != WF_16BIT || st != MUI_OK || p.k_splits == 1 || !p.add) return st;
   const long threads = (long)p.tokens * p.n / 4;
   hipLaunchKernelGGL(gemm_stream_add_kernel<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p);
   return launch_status();
@@ -466,7 +467,7 @@ static float plan_stream(StreamParams& p, size_t part_bytes, int* chosen) {
     if (!stream_built<EPI, WF>(r, nt) || (g_stream_rows && r != g_stream_rows)) continue;
     const int units = ceil_div(rows, r);
     for (int k = 1; k <= 8; ++k) {
-      if (k > 1 && ((long)units * k > cus || (size_t)k * p.tokens * p.n * 4 > part_bytes || p.k / 256 < 2 * k)) break;
+      if (k > 1 && (W8 || (long)units * k > cus || (size_t)k * p.tokens * p.n * 4 > part_bytes || p.k / 256 < 2 * k)) break;
       if (g_stream_shares && k != g_stream_shares) continue;
       const float one = (float)p.k / k * 2.f * ((float)r / (W8 ? 55e3f : 27.5e3f) + 16.f * nt / (nt > 4 ? 82e3f : 105e3f));
       const float barriers = (float)p.k / k / (W8 || r + 16 * nt <= 96 ? 256 : 128) * 0.08f;
@@ -568,18 +569,18 @@ int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParam
 }
 
 template <int WF>
-static int launch_stream_codes(hipStream_t s, int dtype, int epilogue, const StreamParams& p, size_t part_bytes) {
-  if (dtype == MUI_DTYPE_F16) return epilogue == SK_GATEUP ? launch_stream_t<F16, SK_GATEUP, WF>(s, p, 0) : launch_stream_t<F16, SK_LINEAR, WF>(s, p, part_bytes);
-  if (dtype == MUI_DTYPE_BF16) return epilogue == SK_GATEUP ? launch_stream_t<BF16, SK_GATEUP, WF>(s, p, 0) : launch_stream_t<BF16, SK_LINEAR, WF>(s, p, part_bytes);
+static int launch_stream_codes(hipStream_t s, int dtype, int epilogue, const StreamParams& p) {
+  if (dtype == MUI_DTYPE_F16) return epilogue == SK_GATEUP ? launch_stream_t<F16, SK_GATEUP, WF>(s, p, 0) : launch_stream_t<F16, SK_LINEAR, WF>(s, p, 0);
+  if (dtype == MUI_DTYPE_BF16) return epilogue == SK_GATEUP ? launch_stream_t<BF16, SK_GATEUP, WF>(s, p, 0) : launch_stream_t<BF16, SK_LINEAR, WF>(s, p, 0);
   return MUI_ERR_UNSUPPORTED;
 }
 
-// The same for int8 codes, 17 to 64 tokens; groups of 64 or more
-int launch_gemm_stream_int8(hipStream_t s, int dtype, int wf, int epilogue, const SkinnyParams& q, float* part, size_t part_bytes) {
+// The same for int8 codes, 17 to 64 tokens; groups of 64 or more. (Their entry points take no scratch, so K is never divided between workgroups.)
+int launch_gemm_stream_int8(hipStream_t s, int dtype, int wf, int epilogue, const SkinnyParams& q) {
   if (!stream_serves_codes(q, wf)) return MUI_ERR_UNSUPPORTED;
-  const StreamParams p = stream_params(q, part, true, true);
-  if (wf == WF_I8_CHANNEL) return launch_stream_codes<WF_I8_CHANNEL>(s, dtype, epilogue, p, part_bytes);
-  return launch_stream_codes<WF_U8_GROUP>(s, dtype, epilogue, p, part_bytes);
+  const StreamParams p = stream_params(q, nullptr, true, true);
+  if (wf == WF_I8_CHANNEL) return launch_stream_codes<WF_I8_CHANNEL>(s, dtype, epilogue, p);
+  return launch_stream_codes<WF_U8_GROUP>(s, dtype, epilogue, p);
 }
 
 // The same for a caller whose next launch adds the partial outputs up itself: part [*splits][tokens][n] gets the products, nothing else is applied.

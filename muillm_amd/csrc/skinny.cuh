@@ -208,7 +208,7 @@ int launch_gemm_wide(hipStream_t s, int dtype, int weight_format, int epilogue, 
 // for everything else and for what the tiled GEMM does faster
 float gemm_stream_time(int dtype, int weight_format, int epilogue, const SkinnyParams& p, size_t part_bytes);  // of the next two, in us; negative: they decline
 int launch_gemm_stream(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);
-int launch_gemm_stream_int8(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p, float* part, size_t part_bytes);  // codes, 17..64 tokens
+int launch_gemm_stream_int8(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);  // codes, 17..64 tokens
 int launch_gemm_stream_parts(hipStream_t s, int dtype, const SkinnyParams& p, float* part, size_t part_bytes, int* splits);
 // launches gemm_skinny_kernel<dtype, weight format, epilogue>; returns a MUI_* status
 int launch_skinny(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
