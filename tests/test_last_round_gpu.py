@@ -1,50 +1,27 @@
-"""Products whose big tiles leave a last round of workgroups at most half full (it is a launch of its own, of smaller tiles): sizes on both sides of a quarter and
-of half a round, with outputs and tokens that do not come out even, against float64 products and against one launch."""
+"""Products whose 256 x 256 tiles leave a last round of workgroups at most half full, which is a launch of its own of halves (1) or quarters (2) of the tiles: with outputs
+and tokens that do not come out even, with bias and residual, and where the XCDs divide rows and tokens (4096 x 5120), against products in 32 bits, and the same in one launch."""
 import pytest
 import torch
 
-from muillm_amd import _lib, muillm_ext
+from muillm_amd import _lib
+
+from tests.prompt_util import prompt_plan, prompt_product
 
 pytestmark = pytest.mark.gpu
-DEV = "cuda"
-REL = {torch.bfloat16: 2 ** -7, torch.float16: 2 ** -10}  # as a share of the largest output: four times one rounding to 16 bits
-K = 128
-# (outputs, tokens); 256 CUs: a quarter of a round is 8 tiles of an XCD, half of it 16
-GATEUP = [(14336, 2048), (14336, 1280), (14336, 3500), (14300, 3585), (8192, 1100), (8200, 1281), (4090, 2500)]
-LINEAR = [(4096, 4352), (4096, 2304), (4100, 2305), (8192, 2300), (12290, 1700), (28672, 777), (6144, 2600), (4096, 8191)]
+REL = {"bf16": 2 ** -7, "fp16": 2 ** -10, "int8": 2 ** -10, "int8_group": 2 ** -10}  # as a share of the largest output: four times one rounding to 16 bits
+CASES = [(w, "gateup", *s) for w in ("bf16", "fp16", "int8") for s in
+         [(8192, 1024, 2500, 1), (14336, 1024, 3500, 2), (12290, 1024, 2500, 2), (4100, 512, 6144, 1), (14300, 512, 2500, 1)]] + \
+        [("int8_group", "gateup", *s) for s in [(12290, 2048, 1281, 1), (8192, 1024, 1281, 1), (11008, 1024, 700, 2)]] + \
+        [(w, "linear", *s) for w in ("bf16", "fp16", "int8") for s in
+         [(14330, 2048, 3500, 2), (14336, 2048, 3585, 1), (4096, 5120, 4352, 2), (4100, 8192, 4352, 1)]] + \
+        [("int8_group", "linear", *s) for s in [(12288, 4096, 1281, 2), (12290, 8192, 1281, 1)]]
 
 
-@pytest.mark.parametrize("weights", ["bf16", "fp16", "int8", "int8_group"])
-@pytest.mark.parametrize("form,n,tokens", [("gateup", *s) for s in GATEUP] + [("linear", *s) for s in LINEAR])
-def test_last_round(weights, form, n, tokens):
-    dtype, g = torch.bfloat16 if weights == "bf16" else torch.float16, torch.Generator(device=DEV).manual_seed(n + tokens)
-    gateup, rows = form == "gateup", 2 * n if form == "gateup" else n
-    x = torch.randn(tokens, K, device=DEV, generator=g).to(dtype)
-    bias, res = torch.randn(n, device=DEV, generator=g).to(dtype), torch.randn(tokens, n, device=DEV, generator=g).to(dtype)
-    if "int8" in weights:
-        q = torch.randint(-128, 128, (rows, K), device=DEV, generator=g, dtype=torch.int32)
-        s = (torch.rand(rows, device=DEV, generator=g) * 2e-3 + 1e-3).to(dtype)
-        w = q.float() * s.float()[:, None]
-    else:
-        w = (torch.randn(rows, K, device=DEV, generator=g) * 0.1).to(dtype)
-    if weights == "int8":
-        c = q.to(torch.int8)
-        pair, sp = c.view(n, 2, K) if gateup else None, s.view(n, 2) if gateup else None
-        call = (lambda: muillm_ext.mui_int8_channel_gateupsilu_forward(None, 0.0, pair[:, 0], pair[:, 1], sp[:, 0], sp[:, 1], x)) if gateup else \
-            (lambda: muillm_ext.mui_int8_channel_linear_forward(x, c, s, add_bias=bias, residual=res))
-    elif weights == "int8_group":  # one group of 128 per row: (scale, smallest value)
-        c, low = (q + 128).to(torch.uint8), (s.float() * -128).to(dtype)
-        pairs = torch.stack([s, low], 1)
-        w = (q + 128).float() * s.float()[:, None] + low.float()[:, None]
-        call = (lambda: muillm_ext.muillm_int8_gateupsilu_forward(None, 0.0, c.view(n, 2, K), pairs.view(n, 2, 1, 2), 7, x)) if gateup else \
-            (lambda: muillm_ext.muillm_int8_linear_forward(x, c, pairs.contiguous(), 7, add_bias=bias, residual=res))
-    else:
-        pair = w.view(n, 2, K) if gateup else None
-        call = (lambda: muillm_ext.mui_gateup_silu(None, 0.0, pair[:, 0], pair[:, 1], x)) if gateup else \
-            (lambda: muillm_ext.muillm_linear_forward(None, x, w, add_bias=bias, residual=res))
-    ref = x.double() @ w.double().T
-    ref = ref[:, 0::2] * torch.sigmoid(ref[:, 0::2]) * ref[:, 1::2] if gateup else ref + bias.double() + res.double()
-    lib = _lib.load()
+@pytest.mark.parametrize("weights,form,n,k,tokens,last", CASES)
+def test_last_round(weights, form, n, k, tokens, last):
+    assert prompt_plan(weights, form, n, k, tokens) == (0, 4, last)
+    call, ref = prompt_product(weights, form, n, k, tokens)
+    lib, most = _lib.load(), float(ref.abs().max())
     y = call()
     assert lib.mui_tune_prefill(3200, 0) == 0
     try:
@@ -52,4 +29,4 @@ def test_last_round(weights, form, n, tokens):
     finally:
         lib.mui_tune_prefill(0, 0)
     for out in (y, one):
-        assert float((out.double() - ref).abs().max() / ref.abs().max()) <= REL[dtype]
+        assert float((out.float() - ref).abs().max()) <= REL[weights] * most

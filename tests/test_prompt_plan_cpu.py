@@ -1,7 +1,7 @@
 """Where the last few tokens of a prompt are a launch of their own: products that were measured both ways and differ by 5 % or more (256 CUs)."""
 import pytest
 
-from .prompt_util import prompt_plan
+from tests.prompt_util import prompt_plan
 
 # us in one launch / two
 TWO = [("bf16", "gateup", 14336, 4096, 520, 165, 146), ("bf16", "gateup", 14336, 2880, 520, 120, 110), ("bf16", "gateup", 14336, 4160, 1032, 271, 237),
