@@ -1421,12 +1421,12 @@ static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
 // Products whose last token tiles hold few tokens: the number of tokens to leave to a launch of their own, for whole 256-token tiles in front of it -- or 0. 520
 // tokens of a 14336 x 4096 gate/up are 336 tiles of 256 x 256 where 512 are 224, one round of workgroups; the weights of the few are read again instead, by the
 // kernels that stream them or, what those decline, by tiles: 16 to 42 us a round at K = 4096 and 5 of ramp, next to the streaming kernel's own estimate and its ramp (groups of codes take
-// 1.6 times that estimate). The two launches take what each takes alone, within 5 %, so they are taken where the sum is less; of linears, whose big tiles the plan knows less well,
-// 15 % less and only from 2048 tokens on. us, one launch / two: gate/up 14336 x 4096 bf16, 520 / 640
+// 1.6 times that estimate). The two launches take what each takes alone, within 5 %, so they are taken where the sum is less by 3 %; of linears only
+// from 2048 tokens on. us, one launch / two: gate/up 14336 x 4096 bf16, 520 / 640
 // / 1032 / 1152 / 1544 / 1664 tokens 165 / 146, 165 / 145, 262 / 224, 265 / 241, 361 / 314, 367 / 336; 14336 x 2880 (tiles) 520 / 1032 120 / 110, 196 / 171; 8192 x 2048, 1032 / 1152 / 2056
-// 84 / 70, 86 / 75, 147 / 124; int8 per channel 14336 x 4096 (fp16), 520 / 1032 / 1100 180 / 130, 286 / 225, 289 / 256; linears 4096 x 14336, 4104 478 / 365; 4096 x 4096
+// 84 / 70, 86 / 75, 147 / 124; int8 per channel 14336 x 4096 (fp16), 520 / 1032 / 1100 180 / 130, 286 / 225, 289 / 256; linears 4096 x 14336, 2056 / 4104 237 / 219, 478 / 365; 4096 x 4096
 // 153 / 121; not taken: gate/up 8192 x 8256 at 520 166 / 180, 2048 x 8256 int8 at 529 69 / 123, 2560 x 11008 int8 at 2305 238 / 452, linear 2048 x 8192 at 2056 86 / 89, 4096 x 14400 at 2088 223 / 247. Of
-// 600 products of 512 to 8191 tokens that end up to 128 beyond a whole tile it takes 88, none of them slower by more than 2 %; the sum of logarithms is 1.1 % less than without, 2.1 at best.
+// 600 products of 512 to 8191 tokens that end up to 128 beyond a whole tile it takes 98, none of them slower by more than 2 %; the sum of logarithms is 1.1 % less than without, 2.1 at best.
 static int rest_tokens(const PrefillGemmParams& p, const SkinnyParams& q, int dtype, int wf, int epi, bool pipelined, size_t part_bytes) {
   const int rest = p.tokens % 256;
   if (!g_prefill_bands || !pipelined || p.tokens < (epi == SK_GATEUP ? 512 : 2048) || rest == 0 || rest > 128) return 0;
@@ -1442,7 +1442,7 @@ static int rest_tokens(const PrefillGemmParams& p, const SkinnyParams& q, int dt
     const PrefillPlan tiles = prefill_plan(p, wf, epi, true, rest);
     us = 5.f + per_k * (tiles.cost > 0.f ? tiles.cost : tiles.tile == 6 ? 16.f : tiles.tile == 12 ? 22.f : 32.5f);
   }
-  return whole * per_k + us < (epi == SK_GATEUP ? 0.97f : 0.85f) * together * per_k ? rest : 0;
+  return whole * per_k + us < 0.97f * together * per_k ? rest : 0;
 }
 
 constexpr int kWideDefaultMaxTokens = 0;  // 0: the built-in rule below
