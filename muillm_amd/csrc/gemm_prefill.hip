@@ -1314,8 +1314,8 @@ template <typename T, int WF, int EPI>
 static int launch_prefill_t(hipStream_t s, const PrefillGemmParams& p) {
   int which = g_prefill_tile;
   if (which == 0) which = prefill_plan(p, WF, EPI, kPipelined<T, WF> && !p.gamma && pipelined_loop_serves(p, WF), p.tokens).tile;
-  // Where the software-pipelined eight-wave loop does not apply (fused norm, int8 weights, K not a
-  // multiple of 64): sixteen waves per workgroup (four per SIMD, at most 128 registers each) on all
+  // Where the software-pipelined eight-wave loop does not apply (fused norm, K not a multiple of 64, codes in groups
+  // in bf16 or of fewer than 64): sixteen waves per workgroup (four per SIMD, at most 128 registers each) on all
   // but the smallest shapes, with the compiler's own schedule 3-16 % ahead of eight waves with twice
   // the wave tile, although a wave then reads 8
   // instead of 6 KB of operands per 16 matrix instructions -- more waves to fill the gaps between

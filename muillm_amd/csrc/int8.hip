@@ -375,7 +375,7 @@ extern "C" int mui_int8_linear(mui_stream_t stream, int dtype, const void* weigh
   if (st != MUI_OK) return st;
   MUI_CHECK_ARG(scales && y);
   hipStream_t s = (hipStream_t)stream;
-  if (tokens > MUI_MAX_TOKENS) {  // a prompt: the tiled matrix-core GEMM, codes converted on the way to LDS
+  if (tokens > MUI_MAX_TOKENS) {  // a prompt: the kernels for more tokens, which convert the codes themselves
     SkinnyParams sp = {};
     sp.w0 = weights_i8; sp.pitch = w_pitch; sp.s0 = (const uint16_t*)scales; sp.s_pitch = 1;
     sp.x = (const uint16_t*)x; sp.gamma = (const uint16_t*)norm_weights;
@@ -468,7 +468,7 @@ extern "C" int mui_int8_group_linear(mui_stream_t stream, int dtype, const void*
   if (group_size_shift < 4 || group_size_shift > 30) return MUI_ERR_UNSUPPORTED;
   if (k_in & ((1 << group_size_shift) - 1)) return MUI_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
-  if (tokens > MUI_MAX_TOKENS) {  // a prompt: the tiled matrix-core GEMM, codes dequantised on the way to LDS
+  if (tokens > MUI_MAX_TOKENS) {  // a prompt: the kernels for more tokens, which dequantise the codes themselves
     SkinnyParams sp = {};
     sp.w0 = weights_u8; sp.pitch = w_pitch; sp.s0 = (const uint16_t*)scales_min_vals;
     sp.s_pitch = 2L * (k_in >> group_size_shift); sp.group_shift = group_size_shift;

@@ -631,7 +631,7 @@ def muillm_int8_linear_forward(x, weights, scales_min_vals, group_size_shift, no
     if _num_tokens(x) >= int8_dequantised_from(x.dtype, k, group_size_shift, scales_min_vals.data_ptr()):
         # a long prompt: the reference's route (dequantise the matrix, then a GEMM,
         # muillm/modules/quantized/int8linear.py:279-293) on this library's kernels; shorter ones go
-        # to the GEMM that dequantises the codes on their way to LDS (one call below)
+        # to the kernels that dequantise the codes themselves (one call below)
         w = muillm_int8_dequantize_forward(weights, scales_min_vals, group_size_shift)
         return muillm_linear_forward(None, x, w, norm_weights, epsilon, None, add_bias, residual)
     if scales_min_vals.dtype != x.dtype or scales_min_vals.numel() != 2 * n * (k >> group_size_shift):
