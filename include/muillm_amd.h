@@ -101,9 +101,9 @@ int mui_linear(mui_stream_t stream, int dtype, const void* weights, long w_pitch
  * inside its calls, csrc/linear/linear.cu:178-189). With more than MUI_MAX_TOKENS tokens on a matrix of
  * few rows and a long K (the down projection up to about 256 tokens) one workgroup per output tile
  * would leave most of the chip idle or narrow its tiles: given a workspace, K is shared between workgroups, whose
- * fp32 partial outputs go through it. Up to 128 tokens and a K that is a multiple of 256 a second launch adds
- * them (4096 x 14336 at 64 tokens 29 instead of 38 us); otherwise the last workgroup of a tile to arrive does, which it learns from the counters
- * at the workspace's start (at 256 tokens 62 instead of 68 us). workspace: mui_linear_workspace_bytes() bytes of device memory, 256-byte aligned,
+ * fp32 partial outputs go through it. Up to 128 tokens and a K that is a multiple of 256, beyond and a multiple of 64 a second launch adds
+ * them (4096 x 14336 at 64 tokens 29 instead of 38 us, at 768 tokens 88 instead of 127); otherwise the last workgroup of a tile to arrive does, which it learns from the counters
+ * at the workspace's start (4096 x 14344 at 64 tokens 51 instead of 62 us). workspace: mui_linear_workspace_bytes() bytes of device memory, 256-byte aligned,
  * zero-filled ONCE by the caller before its first use (the kernels leave its counters at zero);
  * calls that may overlap on the device (different streams) need a workspace each. workspace may
  * be NULL (workspace_bytes 0): then, or when norm_weights is given, or for shapes that do not
@@ -116,8 +116,8 @@ int mui_linear_ws(mui_stream_t stream, int dtype, const void* weights, long w_pi
                   void* y, int n_out, int k_in, int tokens, void* workspace, size_t workspace_bytes);
 
 /* A linear with a residual and the norm that follows it, in one call: y = W x (+ add_bias) + residual, h = next_gain * y * rsqrt(mean(y^2) + epsilon)
- * over each row of y -- mui_linear_ws and mui_rmsnorm, whose contracts hold here. Where K is divided between workgroups (17 to 128 tokens, a
- * workspace given, at most 8192 outputs) the launch that adds the partial outputs up takes the norm as well. */
+ * over each row of y -- mui_linear_ws and mui_rmsnorm, whose contracts hold here. Where K is divided between workgroups and a launch adds up (a
+ * workspace given, at most 8192 outputs) that launch takes the norm as well. */
 int mui_linear_norm(mui_stream_t stream, int dtype, const void* weights, long w_pitch, const void* x, const void* add_bias,
                     const void* residual, const void* next_gain, float epsilon, void* y, void* h, int n_out, int k_in, int tokens,
                     void* workspace, size_t workspace_bytes);
@@ -589,7 +589,7 @@ int mui_moe_residual_norm(mui_stream_t stream, int dtype, const float* residual_
                           float next_scale, float epsilon, float* residual_out, void* h, int rows, int k);
 
 /* y = W x (+ add_bias) and mui_residual_norm of it (y_scale 1), in one call; 16-bit types. workspace as for mui_linear_ws. Where K is divided
- * between workgroups (17 to 128 tokens, a workspace given, at most 8192 outputs, h given) the launch that adds the partial outputs up joins them, too. */
+ * between workgroups and a launch adds up (a workspace given, at most 8192 outputs, h given) that launch joins them, too. */
 int mui_linear_residual_norm(mui_stream_t stream, int dtype, const void* weights, long w_pitch, const void* x, const void* add_bias,
                              const float* residual_in, const void* post_gain, float branch_scale, const void* next_gain, float next_scale,
                              float epsilon, void* y, float* residual_out, void* h, int n_out, int k_in, int tokens, void* workspace,

@@ -157,6 +157,8 @@ _SIGNATURES = {
     "mui_tune_skinny": (c_int, [c_int, c_int, c_int]),
     "mui_tune_prefill": (c_int, [c_int, c_int]),
     "mui_probe_prefill_plan": (c_int, [c_int] * 8 + [ctypes.POINTER(c_int)] * 3),
+    "mui_tune_prompt_shares": (c_int, [c_int, c_int]),
+    "mui_probe_prompt_shares": (c_int, [c_int] * 6 + [ctypes.POINTER(c_int)] * 2),
     "mui_tune_stream": (c_int, [c_int, c_int]),
     "mui_tune_prefill_attention": (c_int, [c_int]),
     "mui_tune_warm": (c_int, [c_int, c_int, c_int]),

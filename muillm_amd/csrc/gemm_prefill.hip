@@ -26,8 +26,8 @@
 //   32 x 64 x 256 on eight -- the LDS traffic per matrix instruction of a larger tile and four waves per SIMD
 //   although there is one workgroup per CU; their partial tiles are exchanged through LDS in three
 //   rounds at the end. (int8 weights keep eight / four waves where more would leave threads
-//   without a chunk to stage.) With a caller-provided workspace a long K is shared between
-//   workgroups as well (XS below).
+//   without a chunk to stage.) With a caller-provided workspace K is shared between
+//   workgroups as well where that is faster: big tiles on the pipelined loop (parts_plan), or, of a K that it does not take, 128 x 128 (XS below).
 //   Under the gate/up epilogue half of a wave's rows are gate rows and the other half the up
 //   rows of the same outputs, so SiLU * mul happens in registers.
 //   Token tiles of one row tile are placed on the same XCD (workgroup id modulo 8) so that the
@@ -81,7 +81,8 @@ __device__ __forceinline__ f32x4 xs_load(const float* src) {
                __uint_as_float((uint32_t)(b >> 32))};
 }
 
-// XS: K is also split over p.k_splits workgroups per tile (short prompts on matrices of few row
+// XS with PIPE: K is also split over p.k_splits workgroups per tile, which leave fp32 partial outputs to a launch behind (parts_plan).
+// XS without: K is also split over p.k_splits workgroups per tile (short prompts on matrices of few row
 // tiles, where one workgroup per tile would leave most CUs idle and a long K to each): every
 // workgroup delivers its partial tile in fp32 and counts itself in; whoever arrives last adds the
 // partials up in index order (the same sum whichever workgroup that is) and runs the epilogue.
@@ -114,7 +115,7 @@ template <typename T, int WF, bool NORM, int EPI, int WR, int WT, int NWR, int N
 // one tile: the work of workgroup id `vb` of a grid of one workgroup per tile
 __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, const unsigned vb) {
   constexpr int kPfThreads = 64 * NWR * NWT * NWK;
-  static_assert(!XS || (!NORM && EPI == SK_LINEAR && NBUF == 2), "workgroups that split K: plain linear, two stages");
+  static_assert(!XS || (!NORM && EPI == SK_LINEAR && (PIPE || NBUF == 2)), "workgroups that split K: plain linear, two stages or the pipelined loop");
   static_assert((KS / 32) % NWK == 0 && WT % NWK == 0, "k-split of the waves");
   constexpr int ROWS = 16 * WR * NWR, TOKS = 16 * WT * NWT;
   // The big tiles run in grids of several rounds in which the token tiles of a row tile share its
@@ -164,8 +165,8 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   // 8 XCDs, so ids that share id % 8 share an L2; give each XCD whole row tiles
   // (XS: the share of K is the fastest index -- with 8 shares it is the XCD, whose L2 then holds
   // one k-range of x for all row tiles)
-  const int xs_share = XS ? (int)(vb % (unsigned)p.k_splits) : 0;
-  const int xs_tile = XS ? (int)(vb / (unsigned)p.k_splits) : 0;
+  int xs_share = XS ? (int)(vb % (unsigned)p.k_splits) : 0;
+  int xs_tile = XS ? (int)(vb / (unsigned)p.k_splits) : 0;
   const int xcd = vb & 7;
   int slot = vb >> 3, piece = 0;
   if (p.sub_rows) {
@@ -180,7 +181,15 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   // token tiles, rows fastest: the 32 workgroups that it runs at a time then share few row tiles AND
   // few token tiles (4 x 8 instead of 1 x 32 at 8192 tokens), a third of the fetches again.
   int tile_n, tile_t;
-  if constexpr (XS) {
+  if constexpr (XS && PIPE) {
+    // an XCD has consecutive tiles of one share, the token tiles of a row tile side by side: they read the same weights and the same values of x at the same time
+    const unsigned tiles = (unsigned)(p.n_tiles * p.t_tiles), id = (vb & 7) * (unsigned)(p.total_blocks >> 3) + (vb >> 3);
+    xs_share = (int)(id / tiles);
+    xs_tile = (int)(id - (unsigned)xs_share * tiles);
+    if (xs_share >= p.k_splits) return;
+    tile_n = xs_tile / p.t_tiles;
+    tile_t = xs_tile % p.t_tiles;
+  } else if constexpr (XS) {
     tile_n = xs_tile / p.t_tiles;
     tile_t = xs_tile % p.t_tiles;
   } else {
@@ -261,7 +270,7 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
   unsigned dma_wo[WQ], dma_xo[XQ];
   auto w_block = [&](int q, int w) { return !W8 || q * kNWaves + w < WBLOCKS ? q * kNWaves + w : w; };
   if constexpr (DMA) {
-    static_assert(!DMA || ((WF == WF_16BIT || W8) && !NORM && NBUF >= 2 && !XS && CPR >= 8 && CPR <= 64), "what the DMA path covers");
+    static_assert(!DMA || ((WF == WF_16BIT || W8) && !NORM && NBUF >= 2 && (!XS || PIPE) && CPR >= 8 && CPR <= 64), "what the DMA path covers");
     static_assert(!DMA || (WQ >= 1 && XQ >= 1 && (W8 || WQ * DRW * kNWaves == ROWS) && XQ * DRI * kNWaves == TOKS), "whole 1 KB blocks per wave");
     static_assert(!DMA || EPI != SK_GATEUP || (8 * WR) % DRW == 0, "gate and up rows change at multiples of a block's rows");
     const int sr = lane / CPR, sc = lane % CPR;
@@ -774,8 +783,23 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
     }
   }
 
+  // ---- workgroups that split K, pipelined loop: the share's sums, a launch behind this one adds them up
+  if constexpr (XS && PIPE) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // (the last loads into LDS, which nobody reads)
+    float* part = p.part + (long)xs_share * p.tokens * p.n;
+    const int tok_0 = t0 + wt * 16 * WT + (lane & 15), o_0 = o0 + wr * 16 * WR + (lane >> 4) * 4;
+#pragma unroll
+    for (int j = 0; j < WT; ++j) {
+      const int tok = tok_0 + 16 * j;
+      if (tok >= p.tokens) continue;
+#pragma unroll
+      for (int i = 0; i < WR; ++i)
+        if (o_0 + 16 * i < p.n) *(f32x4*)(part + (long)tok * p.n + o_0 + 16 * i) = acc[i][j];  // (n is a multiple of 4)
+    }
+    return;
+  }
   // ---- workgroups that split K: deliver, count, and the last one adds up
-  if constexpr (XS) {
+  if constexpr (XS && !PIPE) {
     constexpr int SLOT = (kPfThreads / 64) * WR * JW * 64 * 4;  // floats per partial tile
     float* mine = p.part + ((long)xs_tile * p.k_splits + xs_share) * SLOT;
 #pragma unroll
@@ -1158,13 +1182,15 @@ constexpr int kXsMaxWorkgroups = 512;                          // partial tiles
 constexpr size_t kXsSlotBytes = 128 * 128 * sizeof(float);     // one 128 x 128 partial tile
 constexpr size_t kXsCounterBytes = kXsMaxTiles * sizeof(unsigned);
 size_t prefill_counter_bytes() { return kXsCounterBytes; }
-size_t prefill_workspace_bytes() { return kXsCounterBytes + kXsMaxWorkgroups * kXsSlotBytes; }
+size_t prefill_workspace_bytes() { return kXsCounterBytes + kXsMaxWorkgroups * kXsSlotBytes; }  // the least that is used
+// Shares of K of the pipelined tiles gain 17.8 % of the time of the products that parts_plan was fitted to with 64 MB of scratch, 16.2 with 34, 18.0 with 160
+size_t prefill_workspace_best() { return kXsCounterBytes + ((size_t)64 << 20); }
 
 // shares of K per 128 x 128 tile worth taking, or 0: the grid of whole tiles leaves at least three
 // quarters of the CUs idle and every share keeps at least twelve k-steps of 128 -- the exchange
 // (write-through of the partial tile, the counter, the last workgroup's reads) costs 10-15 us, so
 // it pays on long rows only. gemm_stream.hip has the 17 to 128 tokens of rows whose K is a multiple of 256; what comes here
-// is longer, or a K like 14344. Measured on MI355X: 4096 x 14336 at 192 and 256 tokens 68 -> 61 us, 4096 x 14344 at 64 tokens
+// is longer, or a K like 14344, and what parts_plan has (K a multiple of 64, more than 128 tokens) does not come here. Measured on MI355X: 4096 x 14344 at 64 tokens
 // 62 -> 51 us, at 128 61 -> 55 us (8 shares, 4 beyond 128 tokens); 1000 x 6152 is below the line's gain (29 -> 31 us at 64 tokens).
 static int xs_shares(const PrefillGemmParams& p) {
   const long tiles = (long)ceil_div(p.n, 128) * ceil_div(p.tokens, 128);
@@ -1308,6 +1334,75 @@ static PrefillPlan prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe,
     settled -= 0.5f * best / (float)full * (float)(full * cus - n) / (float)cus;
   }
   return {best, which, last, settled};
+}
+
+// K in shares for linears of more than 128 tokens whose big tiles leave CUs idle: the tiles of the pipelined loop, every one `shares` times over a part of K, the
+// sums in fp32 through the caller's workspace ([shares][tokens][n]), and a launch that adds them up in order (gemm_stream.hip, or with the norm behind in linear_join.hip).
+// A product of few tiles is otherwise left to small tiles, which read two to four times the operand bytes per product, and to a part of the chip. us in bf16 with a
+// residual, cold weights, one launch / shares: 4096 x 14336 at 200 / 333 / 535 / 768 / 1280 / 2048 tokens 61 / 49, 93 / 62, 117 / 84, 127 / 88, 173 / 128, 200 / 188;
+// 2048 x 8192 at 333 / 768 / 1280 44 / 32, 56 / 40, 70 / 51; 4096 x 4096 at 333 / 768 32 / 29, 43 / 40; 6144 x 4096 at 200 / 333 / 768 33 / 27, 42 / 38, 55 / 55 (not taken).
+// (Partial tiles that the last workgroup of a tile to arrive adds up, with tiles of 256 x 256, had cost what they saved: that workgroup reads a megabyte by itself.)
+struct PartsPlan { int tile, shares; float us; };
+constexpr int kMostParts = 8;
+static int g_parts_tile = 0, g_parts_shares = 0;  // mui_tune_prompt_shares; tile -1: never
+
+// Rounds of workgroups by the fullest XCD; a round is its k-steps (a little shorter where CUs are idle: the clock rises) and 3.7 us, the second launch 7.5 and its bytes,
+// written and read, at 3.6 TB/s. Fitted to 2500 products of 18 matrices, 129 to 2500 tokens: within 3 % at the median and 8 % nine times in ten; the pair chosen by
+// it is within 1.4 % of the best nine times in ten.
+static PartsPlan parts_plan(const PrefillGemmParams& p, bool codes, size_t part_bytes) {
+  constexpr struct { int id, rows; float step; } kTiles[] = {{7, 128, 0.78f}, {8, 192, 1.10f}, {4, 256, 1.37f}};
+  PartsPlan best = {0, 0, 0.f};
+  const long cus = device_cus();
+  const int steps = p.k / 64;
+  for (const auto& t : kTiles) {
+    if (g_parts_tile > 0 && t.id != g_parts_tile) continue;
+    const long tiles = (long)ceil_div(p.n, t.rows) * ceil_div(p.tokens, 256);
+    for (int c = 2; c <= kMostParts; ++c) {
+      const size_t bytes = (size_t)c * p.tokens * p.n * 4;
+      if (bytes > part_bytes || steps < 6 * c) break;
+      if (g_parts_tile > 0 && c != g_parts_shares) continue;
+      const long rounds = (8 * ((tiles * c + 7) / 8) + cus - 1) / cus;
+      if (rounds > 3) break;
+      const float busy = (float)(tiles * c) / (float)(rounds * cus);
+      const float step = t.step * (codes ? 1.09f : 1.f) * (0.78f + 0.22f * busy);
+      const float us = (float)rounds * (3.7f + (float)ceil_div(steps, c) * step) + 7.5f + 0.28e-6f * (float)bytes;
+      if (best.shares == 0 || us < best.us) best = {t.id, c, us};
+    }
+  }
+  return best;
+}
+
+// Against the plan without shares, whose costs are rounds of tiles at K = 4096 and leave out what a launch takes besides. Of the products above shares are
+// taken for two thirds, 17 % of the time of all of them on average; of 2500 twenty lost more than 2 %, 9 % at worst.
+static bool parts_are_faster(const PrefillGemmParams& p, int wf, const PartsPlan& parts) {
+  if (parts.shares == 0) return false;
+  if (g_parts_tile > 0) return true;
+  const PrefillPlan whole = prefill_plan(p, wf, SK_LINEAR, true, p.tokens);
+  const float per_k = (float)p.k / 4096.f;
+  const float us = whole.tile == 6    ? 5.7f + 12.2f * per_k
+                   : whole.tile == 12 ? 4.7f + 19.6f * per_k
+                   : whole.tile == 4 || whole.tile == 7 || whole.tile == 8 ? 14.f + 0.9f * whole.cost * per_k
+                                                                         : 6.5f + 0.82f * whole.cost * per_k;
+  return parts.us < 0.95f * us;
+}
+
+template <typename T, int WF, int WR, int WT, int NWR, int NWT>
+static int launch_parts_cfg(hipStream_t s, PrefillGemmParams p) {
+  constexpr int ROWS = 16 * WR * NWR, TOKS = 16 * WT * NWT, KS = 64, NBUF = 3;
+  p.n_tiles = ceil_div(p.n, ROWS);
+  p.t_tiles = ceil_div(p.tokens, TOKS);
+  const long grid = ((long)p.n_tiles * p.t_tiles * p.k_splits + 7) / 8 * 8, round = device_cus() / 8 * 8;
+  if (round < 8) return MUI_ERR_UNSUPPORTED;
+  p.total_blocks = (int)grid;  // (three rounds at most)
+  constexpr size_t lds = WF != WF_16BIT ? pipe8_lds_bytes<WF, ROWS, TOKS, KS, NBUF>() : pipe_lds_bytes<ROWS, TOKS, KS, NBUF>();
+  return launch_with_lds(prefill_gemm_kernel<T, WF, false, SK_LINEAR, WR, WT, NWR, NWT, 1, KS, NBUF, true, true, true>,
+                         dim3((unsigned)(grid > round ? round : grid)), dim3(64 * NWR * NWT), lds, s, p);
+}
+template <typename T, int WF>
+static int launch_parts_t(hipStream_t s, const PrefillGemmParams& p, int tile) {
+  if (tile == 7) return launch_parts_cfg<T, WF, 4, 4, 2, 4>(s, p);  // the tiles of launch_prefill_t
+  if (tile == 8) return launch_parts_cfg<T, WF, 3, 8, 4, 2>(s, p);
+  return launch_parts_cfg<T, WF, 4, 8, 4, 2>(s, p);
 }
 
 template <typename T, int WF, int EPI>
@@ -1458,6 +1553,28 @@ static PrefillGemmParams prefill_params(const SkinnyParams& q, int wf) {
   return p;
 }
 
+static PartsPlan parts_taken(const PrefillGemmParams& p, int dtype, int wf, size_t part_bytes) {
+  PartsPlan plan = {0, 1, 0.f};
+  if (wf != WF_16BIT || g_parts_tile < 0 || p.tokens <= 128 || p.n % 4 || !pipelined(p, dtype, wf)) return plan;
+  const PartsPlan best = parts_plan(p, wf != WF_16BIT, part_bytes);
+  return parts_are_faster(p, wf, best) ? best : plan;
+}
+
+// part [*shares][tokens][n] gets the products of the shares of K, a launch of the caller's adds them up. MUI_ERR_UNSUPPORTED for what is not taken or faster otherwise
+int launch_prefill_parts(hipStream_t s, int dtype, int wf, const SkinnyParams& q, float* part, size_t part_bytes, int* shares) {
+  PrefillGemmParams p = prefill_params(q, wf);
+  if (g_prefill_tile || g_wide_max_tokens != kWideDefaultMaxTokens) return MUI_ERR_UNSUPPORTED;  // (experiments)
+  if (!part || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;
+  if (((uintptr_t)p.y | (uintptr_t)p.residual) & 7) return MUI_ERR_UNSUPPORTED;  // (four outputs at a time)
+  const PartsPlan plan = parts_taken(p, dtype, wf, part_bytes);
+  if (plan.shares < 2) return MUI_ERR_UNSUPPORTED;
+  p.part = part;
+  p.k_splits = *shares = plan.shares;
+  if (dtype == MUI_DTYPE_F16) return launch_parts_t<F16, WF_16BIT>(s, p, plan.tile);
+  if (dtype == MUI_DTYPE_BF16) return launch_parts_t<BF16, WF_16BIT>(s, p, plan.tile);
+  return MUI_ERR_UNSUPPORTED;
+}
+
 // Any number of tokens >= 1 (meant for more than MUI_MAX_TOKENS), 16-bit weights or per-channel
 // int8 codes; SkinnyParams as for the decode kernels (x, residual and y dense).
 int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const SkinnyParams& q) {
@@ -1478,6 +1595,11 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   // (in front of the 16-rows-per-workgroup kernel only for K beyond 8192: 4096 x 14344 at 33 tokens 49 vs 57 us, at 17 tokens 49 vs 40)
   const bool wide_default = q.tokens <= 40 && epilogue == SK_LINEAR && ceil_div(q.n, 16) <= device_cus();
   const bool wide = g_wide_max_tokens == kWideDefaultMaxTokens ? wide_default : q.tokens <= g_wide_max_tokens;
+  if (epilogue == SK_LINEAR && scratch) {
+    int shares = 1;
+    const int st = launch_prefill_parts(s, dtype, wf, q, (float*)((char*)q.workspace + kXsCounterBytes), q.workspace_bytes - kXsCounterBytes, &shares);
+    if (st != MUI_ERR_UNSUPPORTED) return st != MUI_OK ? st : launch_parts_add(s, dtype, q, (float*)((char*)q.workspace + kXsCounterBytes), shares);
+  }
   if (q.workspace && g_prefill_tile == 0 && g_wide_max_tokens == kWideDefaultMaxTokens && wf == WF_16BIT &&
       epilogue == SK_LINEAR && !q.gamma && q.k % 8 == 0 && (q.x_pitch == 0 || q.x_pitch == q.k) &&
       ((uintptr_t)q.workspace & 255u) == 0 && q.workspace_bytes >= prefill_workspace_bytes() &&
@@ -1524,6 +1646,13 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   return MUI_ERR_INVALID_ARG;
 }
 
+static SkinnyParams probe_params(int wf, int n, int k, int tokens, int group_shift) {  // dense, aligned operands
+  SkinnyParams q = {};
+  q.pitch = k; q.n = n; q.k = k; q.tokens = tokens; q.group_shift = group_shift;
+  q.s_pitch = wf == WF_U8_GROUP ? 2L * (k >> group_shift) : 1;
+  return q;
+}
+
 }  // namespace mui
 
 extern "C" int mui_probe_prefill_plan(int dtype, int weight_format, int gateup, int n, int k, int tokens, int group_size_shift, int scratch, int* rest_tokens,
@@ -1532,16 +1661,33 @@ extern "C" int mui_probe_prefill_plan(int dtype, int weight_format, int gateup, 
   MUI_CHECK_ARG((dtype == MUI_DTYPE_F16 || dtype == MUI_DTYPE_BF16) && weight_format >= 0 && weight_format <= 2 && n >= 1 && k >= 1 && tokens >= 1 && rest_tokens &&
                 tile && last_round);
   const int wf = weight_format == 0 ? WF_16BIT : weight_format == 1 ? WF_I8_CHANNEL : WF_U8_GROUP, epi = gateup ? SK_GATEUP : SK_LINEAR;
-  SkinnyParams q = {};
-  q.pitch = k; q.n = n; q.k = k; q.tokens = tokens; q.group_shift = group_size_shift;
-  q.s_pitch = wf == WF_U8_GROUP ? 2L * (k >> group_size_shift) : 1;
+  const SkinnyParams q = probe_params(wf, n, k, tokens, group_size_shift);
   PrefillGemmParams p = prefill_params(q, wf);
   const bool pipe = pipelined(p, dtype, wf);
-  *rest_tokens = mui::rest_tokens(p, q, dtype, wf, epi, pipe, scratch && wf == WF_16BIT ? prefill_workspace_bytes() - kXsCounterBytes : 0);
+  *rest_tokens = mui::rest_tokens(p, q, dtype, wf, epi, pipe, scratch && wf == WF_16BIT ? prefill_workspace_best() - kXsCounterBytes : 0);
   p.tokens -= *rest_tokens;
   const PrefillPlan plan = prefill_plan(p, wf, epi, pipe, p.tokens);
   *tile = plan.tile;
   *last_round = plan.last;
+  return MUI_OK;
+}
+
+extern "C" int mui_probe_prompt_shares(int dtype, int weight_format, int n, int k, int tokens, int group_size_shift, int* tile, int* shares) {
+  using namespace mui;
+  MUI_CHECK_ARG((dtype == MUI_DTYPE_F16 || dtype == MUI_DTYPE_BF16) && weight_format >= 0 && weight_format <= 2 && n >= 1 && k >= 1 && tokens >= 1 && tile && shares);
+  const int wf = weight_format == 0 ? WF_16BIT : weight_format == 1 ? WF_I8_CHANNEL : WF_U8_GROUP;
+  const PartsPlan plan = parts_taken(prefill_params(probe_params(wf, n, k, tokens, group_size_shift), wf), dtype, wf, prefill_workspace_best() - kXsCounterBytes);
+  *tile = plan.tile;
+  *shares = plan.shares;
+  return MUI_OK;
+}
+
+extern "C" int mui_tune_prompt_shares(int tile, int shares) {
+  MUI_TUNE_GUARD();
+  if (tile && tile != -1 && tile != 4 && tile != 7 && tile != 8) return MUI_ERR_INVALID_ARG;
+  if (tile > 0 ? shares < 2 || shares > mui::kMostParts : shares != 0) return MUI_ERR_INVALID_ARG;
+  mui::g_parts_tile = tile;
+  mui::g_parts_shares = shares;
   return MUI_OK;
 }
 

@@ -355,6 +355,8 @@ __global__ void __launch_bounds__(256) gemm_stream_add_kernel(const StreamParams
   *(u32x2*)(p.y + at) = pk;
 }
 
+static unsigned add_blocks(int tokens, int n) { return (unsigned)(((long)tokens * n / 4 + 255) / 256); }
+
 template <typename T, int EPI, int ROWS, int NT, int WF>
 static int launch_stream_cfg(hipStream_t s, const StreamParams& p) {
   using G = StreamShape<ROWS, NT, WF>;
@@ -362,8 +364,7 @@ static int launch_stream_cfg(hipStream_t s, const StreamParams& p) {
   const int cus = device_cus(), wgs = p.n_units * p.k_splits;
   const int st = launch_with_lds(gemm_stream_kernel<T, EPI, ROWS, NT, WF>, dim3(wgs < cus ? wgs : cus), dim3(kStreamThreads), G::LDS, s, p);
   if (WF != WF_16BIT || st != MUI_OK || p.k_splits == 1 || !p.add) return st;
-  const long threads = (long)p.tokens * p.n / 4;
-  hipLaunchKernelGGL(gemm_stream_add_kernel<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p);
+  hipLaunchKernelGGL(gemm_stream_add_kernel<T>, dim3(add_blocks(p.tokens, p.n)), dim3(256), 0, s, p);
   return launch_status();
 }
 
@@ -591,6 +592,16 @@ int launch_gemm_stream_parts(hipStream_t s, int dtype, const SkinnyParams& q, fl
   if (dtype == MUI_DTYPE_F16) return launch_stream_t<F16, SK_LINEAR>(s, p, part_bytes, splits);
   if (dtype == MUI_DTYPE_BF16) return launch_stream_t<BF16, SK_LINEAR>(s, p, part_bytes, splits);
   return MUI_ERR_UNSUPPORTED;
+}
+
+// The launch that adds up what launch_prefill_parts has left
+int launch_parts_add(hipStream_t s, int dtype, const SkinnyParams& q, float* part, int shares) {
+  StreamParams p = stream_params(q, part, true);
+  p.k_splits = shares;
+  if (dtype == MUI_DTYPE_F16) hipLaunchKernelGGL(gemm_stream_add_kernel<F16>, dim3(add_blocks(p.tokens, p.n)), dim3(256), 0, s, p);
+  else if (dtype == MUI_DTYPE_BF16) hipLaunchKernelGGL(gemm_stream_add_kernel<BF16>, dim3(add_blocks(p.tokens, p.n)), dim3(256), 0, s, p);
+  else return MUI_ERR_UNSUPPORTED;
+  return launch_status();
 }
 
 }  // namespace mui

@@ -308,7 +308,7 @@ extern "C" int mui_tune_gemv(int rows_linear, int wgs_per_cu) {
   return MUI_OK;
 }
 
-extern "C" size_t mui_linear_workspace_bytes(void) { return prefill_workspace_bytes(); }
+extern "C" size_t mui_linear_workspace_bytes(void) { return prefill_workspace_best(); }
 
 // rows per row group of the single-token kernels (gemv_multi.hip launch_mt_t, int8_multi.hip
 // launch_i8m_t at one token) times the row pitch

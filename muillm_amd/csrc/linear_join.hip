@@ -196,7 +196,8 @@ static int linear_join(hipStream_t s, int dtype, const void* weights, long w_pit
   q.w0 = weights; q.pitch = w_pitch; q.x = (const uint16_t*)x; q.y = p.y; q.n = p.n; q.k = k; q.tokens = p.tokens;
   float* part = (float*)((char*)workspace + prefill_counter_bytes());
   // (K is divided only where it is without the norm, too: whether the boundary was taken along, a hook was listening or all layers came in one call does not show in the bits)
-  const int st = launch_gemm_stream_parts(s, dtype, q, part, workspace_bytes - prefill_counter_bytes(), &p.splits);
+  const size_t part_bytes = workspace_bytes - prefill_counter_bytes();
+  const int st = p.tokens <= 128 ? launch_gemm_stream_parts(s, dtype, q, part, part_bytes, &p.splits) : launch_prefill_parts(s, dtype, WF_16BIT, q, part, part_bytes, &p.splits);
   if (st != MUI_OK) return st;
   p.part = part;
   if (dtype == MUI_DTYPE_F16) return f32 ? launch_join<F16, true>(s, p) : launch_join<F16, false>(s, p);

@@ -200,6 +200,10 @@ __device__ __forceinline__ u32x4 convert_a_pair_f16(uint32_t w0, uint32_t w1, ui
 // tiled matrix-core GEMM for prompts (gemm_prefill.hip): any token count, 16-bit weights or int8 codes of either format
 int launch_prefill_gemm(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
 size_t prefill_workspace_bytes();  // what SkinnyParams::workspace must hold for the prompt GEMM to use it
+size_t prefill_workspace_best();   // beyond, more of it is no use
+// more than 128 tokens, n % 4 == 0: fp32 partial outputs [*shares][tokens][n] of shares of K, where they are worth it, and what adds them up behind
+int launch_prefill_parts(hipStream_t s, int dtype, int weight_format, const SkinnyParams& p, float* part, size_t part_bytes, int* shares);
+int launch_parts_add(hipStream_t s, int dtype, const SkinnyParams& p, float* part, int shares);
 size_t prefill_counter_bytes();    // of that, at its start: counters that stay zero
 // 17..128 tokens: 16 weight rows per workgroup, K split over its waves, token columns in up to 8 MFMA tiles (gemm_wide.hip)
 int launch_gemm_wide(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);

@@ -169,7 +169,7 @@ class ResidualBehind:
     the linear, which fills it in where it can, and asks with the very tensor that the sublayer has returned whether it was. A tensor that somebody has put
     in its place, or has written to since, finds nothing here and is joined the ordinary way: the stream is not updated in place. (A write that raises no version cannot be
     seen: where a hook listens nothing is taken along to begin with.)"""
-    MAX_TOKENS = 128  # beyond, K is not divided and nothing is saved
+    MAX_TOKENS = 128  # beyond, a launch of its own is a small part of the boundary
 
     def __init__(self, stream: torch.Tensor, post_gain: torch.Tensor, branch_scale: float, next_gain: Optional[torch.Tensor], next_scale: float,
                  eps: float):

@@ -46,3 +46,10 @@ def prompt_product(weights: str, form: str, n: int, k: int, tokens: int):
             (lambda: muillm_ext.muillm_linear_forward(None, x, v, add_bias=bias, residual=res))
     ref = x.float() @ w.T
     return call, ref[:, 0::2] * torch.sigmoid(ref[:, 0::2]) * ref[:, 1::2] if gateup else ref + bias.float() + res.float()
+
+
+def prompt_shares(weights: str, n: int, k: int, tokens: int, shift: int = 7):
+    """(tile, shares) of a linear whose K is shared between workgroups; one share: it is not."""
+    (dtype, fmt), out = WEIGHTS[weights], [ctypes.c_int() for _ in range(2)]
+    _lib.check(_lib.load().mui_probe_prompt_shares(dtype, fmt, n, k, tokens, shift if fmt == 2 else 0, *[ctypes.byref(x) for x in out]), "mui_probe_prompt_shares")
+    return tuple(x.value for x in out)

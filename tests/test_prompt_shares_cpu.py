@@ -1,0 +1,17 @@
+"""Where linears of more than 128 tokens share K between workgroups: products that were measured both ways (256 CUs)."""
+import pytest
+
+from tests.prompt_util import prompt_shares
+
+
+@pytest.mark.parametrize("weights,n,k,tokens,whole,shared", [
+    ("bf16", 4096, 14336, 200, 61, 49), ("fp16", 4096, 14336, 333, 93, 62), ("bf16", 4096, 14336, 768, 127, 88), ("bf16", 4096, 14336, 1280, 173, 128),
+    ("bf16", 2048, 8192, 768, 56, 40), ("bf16", 6144, 4096, 333, 42, 38), ("bf16", 6144, 4096, 2048, 84, 116),
+    ("bf16", 4096, 4096, 2048, 63, 75), ("bf16", 2048, 2048, 1280, 25, 27), ("bf16", 4096, 14336, 4096, 348, 400)])
+def test_k_is_shared_where_it_is_faster(weights, n, k, tokens, whole, shared):
+    assert (prompt_shares(weights, n, k, tokens)[1] > 1) == (shared < whole)
+
+
+def test_never():
+    for weights, n, k, tokens in [("bf16", 4096, 14336, 128), ("bf16", 4098, 14336, 333), ("bf16", 4096, 14336 + 8, 333), ("bf16", 4096, 640, 333), ("bf16", 1 << 20, 14336, 333)]:
+        assert prompt_shares(weights, n, k, tokens)[1] == 1
