@@ -172,6 +172,11 @@ int mui_int8_linear(mui_stream_t stream, int dtype, const void* weights_i8, long
                     const void* add_bias, const void* residual, void* y, int n_out, int k_in,
                     int tokens);
 
+/* The same with a scratch buffer for prompts, as mui_linear_ws has (its contract holds here): from 65 tokens on, and a K that is a multiple of 64, K is shared between
+ * workgroups where that is faster. */
+int mui_int8_linear_ws(mui_stream_t stream, int dtype, const void* weights_i8, long w_pitch, const void* scales, const void* x, const void* norm_weights, float epsilon,
+                       const void* add_bias, const void* residual, void* y, int n_out, int k_in, int tokens, void* workspace, size_t workspace_bytes);
+
 /* muillm_int8_gateupsilu_forward (csrc/module.cpp:248; csrc/int8_gateup_kernels.cu:871-940),
  * per-channel format. gate/up are int8 [n_inter, k_in] sharing the row pitch gu_pitch (bytes):
  * two dense matrices, or the two halves of a row-interleaved [n_inter, 2, k_in] buffer
@@ -193,6 +198,11 @@ int mui_int8_group_linear(mui_stream_t stream, int dtype, const void* weights_u8
                           const void* scales_min_vals, int group_size_shift, const void* x,
                           const void* norm_weights, float epsilon, const void* add_bias,
                           const void* residual, void* y, int n_out, int k_in, int tokens);
+
+/* The same with a scratch buffer for prompts, as mui_int8_linear_ws (fp16 and groups of 64 or more). */
+int mui_int8_group_linear_ws(mui_stream_t stream, int dtype, const void* weights_u8, long w_pitch, const void* scales_min_vals, int group_size_shift, const void* x,
+                             const void* norm_weights, float epsilon, const void* add_bias, const void* residual, void* y, int n_out, int k_in, int tokens,
+                             void* workspace, size_t workspace_bytes);
 
 /* muillm_int8_gateupsilu_forward on the reference's RTN format. gate/up rows share gu_pitch
  * (bytes); the (scale, min) pairs of row n start at gate_smv + n * smv_pitch and

@@ -61,8 +61,10 @@ _SIGNATURES = {
     "mui_gateup_silu_bias": (c_int, [_P, c_int, _P, _P, c_long, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int]),
     "mui_silu_mul_interleaved": (c_int, [_P, c_int, _P, _P, c_long, c_int]),
     "mui_int8_linear": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int]),
+    "mui_int8_linear_ws": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int, _P, ctypes.c_size_t]),
     "mui_int8_gateup_silu": (c_int, [_P, c_int, _P, _P, c_long, _P, _P, c_long, _P, _P, c_float, _P, c_int, c_int, c_int]),
     "mui_int8_group_linear": (c_int, [_P, c_int, _P, c_long, _P, c_int, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int]),
+    "mui_int8_group_linear_ws": (c_int, [_P, c_int, _P, c_long, _P, c_int, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int, _P, ctypes.c_size_t]),
     "mui_int8_group_gateup_silu": (c_int, [_P, c_int, _P, _P, c_long, _P, _P, c_long, c_int, _P, _P, c_float, _P, c_int, c_int, c_int]),
     "mui_int8_repack_gateup": (c_int, [_P, _P, _P, c_int, _P, _P, c_int, c_int]),
     "mui_int8_dequantize": (c_int, [_P, c_int, _P, c_long, _P, c_long, _P, c_long, c_int, c_int]),

@@ -10,7 +10,7 @@
 // projection takes 16-bit weights or int8 codes, the latter with per-channel scales or in the
 // reference's group-wise (scale, min) format (muillm/modules/quantized/int8linear.py:279-293,
 // int8gateupdownmlp.py, muillm/quantization/rtnquantizer.py:49-88).
-#include "common.cuh"
+#include "skinny.cuh"
 
 using namespace mui;
 
@@ -192,8 +192,18 @@ static int prompt_layers(mui_stream_t stream, const mui_decoder_stack_t* m, int 
                     int k, const void* next) -> int {
     int st;
     if (scales) {
-      st = shift ? mui_int8_group_linear(stream, m->dtype, weight, pitch, scales, shift, x, gain, m->norm_eps, nullptr, residual, y, n, k, rows)
-                 : mui_int8_linear(stream, m->dtype, weight, pitch, scales, x, gain, m->norm_eps, nullptr, residual, y, n, k, rows);
+      if (next && residual) {
+        SkinnyParams q = {};
+        q.w0 = weight; q.pitch = pitch; q.s0 = (const uint16_t*)scales; q.s_pitch = shift ? 2L * (k >> shift) : 1; q.group_shift = shift;
+        q.x = (const uint16_t*)x; q.residual = (const uint16_t*)residual; q.y = (uint16_t*)y; q.n = n; q.k = k; q.tokens = rows;
+        q.workspace = linear_workspace; q.workspace_bytes = linear_workspace_bytes;
+        st = gain ? MUI_ERR_UNSUPPORTED : launch_codes_norm((hipStream_t)stream, m->dtype, shift ? WF_U8_GROUP : WF_I8_CHANNEL, q, next, m->norm_eps, w.normed);
+        if (st != MUI_ERR_UNSUPPORTED) return st;
+      }
+      st = shift ? mui_int8_group_linear_ws(stream, m->dtype, weight, pitch, scales, shift, x, gain, m->norm_eps, nullptr, residual, y, n, k, rows, linear_workspace,
+                                            linear_workspace_bytes)
+                 : mui_int8_linear_ws(stream, m->dtype, weight, pitch, scales, x, gain, m->norm_eps, nullptr, residual, y, n, k, rows, linear_workspace,
+                                      linear_workspace_bytes);
     } else if (next) {
       return mui_linear_norm(stream, m->dtype, weight, pitch, x, nullptr, residual, next, m->norm_eps, y, w.normed, n, k, rows, linear_workspace,
                              linear_workspace_bytes);

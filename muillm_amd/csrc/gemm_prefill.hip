@@ -788,6 +788,17 @@ __device__ __forceinline__ void prefill_gemm_tile(const PrefillGemmParams& p, co
     __builtin_amdgcn_s_waitcnt(0x0F70);  // (the last loads into LDS, which nobody reads)
     float* part = p.part + (long)xs_share * p.tokens * p.n;
     const int tok_0 = t0 + wt * 16 * WT + (lane & 15), o_0 = o0 + wr * 16 * WR + (lane >> 4) * 4;
+    if constexpr (WF == WF_I8_CHANNEL) {
+#pragma unroll
+      for (int i = 0; i < WR; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int o = o_0 + 16 * i + e;
+          const float c = T::one(p.s0[(long)(o < p.n ? o : p.n - 1) * p.s_pitch]);
+#pragma unroll
+          for (int j = 0; j < WT; ++j) acc[i][j][e] *= c;
+        }
+    }
 #pragma unroll
     for (int j = 0; j < WT; ++j) {
       const int tok = tok_0 + 16 * j;
@@ -1341,6 +1352,7 @@ static PrefillPlan prefill_plan(PrefillGemmParams p, int WF, int EPI, bool pipe,
 // A product of few tiles is otherwise left to small tiles, which read two to four times the operand bytes per product, and to a part of the chip. us in bf16 with a
 // residual, cold weights, one launch / shares: 4096 x 14336 at 200 / 333 / 535 / 768 / 1280 / 2048 tokens 61 / 49, 93 / 62, 117 / 84, 127 / 88, 173 / 128, 200 / 188;
 // 2048 x 8192 at 333 / 768 / 1280 44 / 32, 56 / 40, 70 / 51; 4096 x 4096 at 333 / 768 32 / 29, 43 / 40; 6144 x 4096 at 200 / 333 / 768 33 / 27, 42 / 38, 55 / 55 (not taken).
+// int8 codes per row in fp16, 4096 x 14336 at 100 / 333 / 800 tokens 59 / 39, 105 / 67, 135 / 110; of groups of 128 68 / 44, 116 / 73, 156 / 122.
 // (Partial tiles that the last workgroup of a tile to arrive adds up, with tiles of 256 x 256, had cost what they saved: that workgroup reads a megabyte by itself.)
 struct PartsPlan { int tile, shares; float us; };
 constexpr int kMostParts = 8;
@@ -1349,7 +1361,7 @@ static int g_parts_tile = 0, g_parts_shares = 0;  // mui_tune_prompt_shares; til
 // Rounds of workgroups by the fullest XCD; a round is its k-steps (a little shorter where CUs are idle: the clock rises) and 3.7 us, the second launch 7.5 and its bytes,
 // written and read, at 3.6 TB/s. Fitted to 2500 products of 18 matrices, 129 to 2500 tokens: within 3 % at the median and 8 % nine times in ten; the pair chosen by
 // it is within 1.4 % of the best nine times in ten.
-static PartsPlan parts_plan(const PrefillGemmParams& p, bool codes, size_t part_bytes) {
+static PartsPlan parts_plan(const PrefillGemmParams& p, int wf, size_t part_bytes) {
   constexpr struct { int id, rows; float step; } kTiles[] = {{7, 128, 0.78f}, {8, 192, 1.10f}, {4, 256, 1.37f}};
   PartsPlan best = {0, 0, 0.f};
   const long cus = device_cus();
@@ -1364,7 +1376,7 @@ static PartsPlan parts_plan(const PrefillGemmParams& p, bool codes, size_t part_
       const long rounds = (8 * ((tiles * c + 7) / 8) + cus - 1) / cus;
       if (rounds > 3) break;
       const float busy = (float)(tiles * c) / (float)(rounds * cus);
-      const float step = t.step * (codes ? 1.09f : 1.f) * (0.78f + 0.22f * busy);
+      const float step = t.step * (wf == WF_U8_GROUP ? 1.19f : wf == WF_I8_CHANNEL ? 1.08f : 1.f) * (0.78f + 0.22f * busy);
       const float us = (float)rounds * (3.7f + (float)ceil_div(steps, c) * step) + 7.5f + 0.28e-6f * (float)bytes;
       if (best.shares == 0 || us < best.us) best = {t.id, c, us};
     }
@@ -1373,16 +1385,18 @@ static PartsPlan parts_plan(const PrefillGemmParams& p, bool codes, size_t part_
 }
 
 // Against the plan without shares, whose costs are rounds of tiles at K = 4096 and leave out what a launch takes besides. Of the products above shares are
-// taken for two thirds, 17 % of the time of all of them on average; of 2500 twenty lost more than 2 %, 9 % at worst.
+// taken for two thirds, 17 % of the time of all of them on average; of 2500 twenty lost more than 2 %, 9 % at worst. Codes (5700 products of 13 matrices, 65 to 1600
+// tokens): taken for half, 17 to 20 %, six lost more than 2 %, 6 % at worst.
 static bool parts_are_faster(const PrefillGemmParams& p, int wf, const PartsPlan& parts) {
   if (parts.shares == 0) return false;
   if (g_parts_tile > 0) return true;
   const PrefillPlan whole = prefill_plan(p, wf, SK_LINEAR, true, p.tokens);
-  const float per_k = (float)p.k / 4096.f;
-  const float us = whole.tile == 6    ? 5.7f + 12.2f * per_k
-                   : whole.tile == 12 ? 4.7f + 19.6f * per_k
+  const bool codes = wf != WF_16BIT;
+  const float per_k = (float)p.k / 4096.f * (wf == WF_U8_GROUP ? 1.15f : 1.f);
+  const float us = whole.tile == 6    ? (codes ? 5.3f + 14.8f * per_k : 5.7f + 12.2f * per_k)
+                   : whole.tile == 12 ? (codes ? 8.f + 20.5f * per_k : 4.7f + 19.6f * per_k)
                    : whole.tile == 4 || whole.tile == 7 || whole.tile == 8 ? 14.f + 0.9f * whole.cost * per_k
-                                                                         : 6.5f + 0.82f * whole.cost * per_k;
+                                                                         : (codes ? 9.f : 6.5f) + 0.82f * whole.cost * per_k;
   return parts.us < 0.95f * us;
 }
 
@@ -1555,8 +1569,8 @@ static PrefillGemmParams prefill_params(const SkinnyParams& q, int wf) {
 
 static PartsPlan parts_taken(const PrefillGemmParams& p, int dtype, int wf, size_t part_bytes) {
   PartsPlan plan = {0, 1, 0.f};
-  if (wf != WF_16BIT || g_parts_tile < 0 || p.tokens <= 128 || p.n % 4 || !pipelined(p, dtype, wf)) return plan;
-  const PartsPlan best = parts_plan(p, wf != WF_16BIT, part_bytes);
+  if (g_parts_tile < 0 || p.tokens <= (wf == WF_16BIT ? 128 : 64) || p.n % 4 || !pipelined(p, dtype, wf)) return plan;
+  const PartsPlan best = parts_plan(p, wf, part_bytes);
   return parts_are_faster(p, wf, best) ? best : plan;
 }
 
@@ -1570,8 +1584,14 @@ int launch_prefill_parts(hipStream_t s, int dtype, int wf, const SkinnyParams& q
   if (plan.shares < 2) return MUI_ERR_UNSUPPORTED;
   p.part = part;
   p.k_splits = *shares = plan.shares;
-  if (dtype == MUI_DTYPE_F16) return launch_parts_t<F16, WF_16BIT>(s, p, plan.tile);
-  if (dtype == MUI_DTYPE_BF16) return launch_parts_t<BF16, WF_16BIT>(s, p, plan.tile);
+#define MUI_PARTS_CASE(TT, WFV) \
+  if (dtype == TT::kDtype && wf == WFV) return launch_parts_t<TT, WFV>(s, p, plan.tile);
+  MUI_PARTS_CASE(F16, WF_16BIT)
+  MUI_PARTS_CASE(BF16, WF_16BIT)
+  MUI_PARTS_CASE(F16, WF_I8_CHANNEL)
+  MUI_PARTS_CASE(BF16, WF_I8_CHANNEL)
+  MUI_PARTS_CASE(F16, WF_U8_GROUP)
+#undef MUI_PARTS_CASE
   return MUI_ERR_UNSUPPORTED;
 }
 

@@ -367,13 +367,13 @@ extern "C" int mui_tune_int8(int rows, int wgs_per_cu) {
   return MUI_OK;
 }
 
-extern "C" int mui_int8_linear(mui_stream_t stream, int dtype, const void* weights_i8, long w_pitch,
+extern "C" int mui_int8_linear_ws(mui_stream_t stream, int dtype, const void* weights_i8, long w_pitch,
                                const void* scales, const void* x, const void* norm_weights,
                                float epsilon, const void* add_bias, const void* residual, void* y,
-                               int n_out, int k_in, int tokens) {
+                               int n_out, int k_in, int tokens, void* workspace, size_t workspace_bytes) {
   int st = check_int8_common(dtype, weights_i8, w_pitch, x, norm_weights, n_out, k_in, tokens, true);
   if (st != MUI_OK) return st;
-  MUI_CHECK_ARG(scales && y);
+  MUI_CHECK_ARG(scales && y && (workspace || workspace_bytes == 0));
   hipStream_t s = (hipStream_t)stream;
   if (tokens > MUI_MAX_TOKENS) {  // a prompt: the kernels for more tokens, which convert the codes themselves
     SkinnyParams sp = {};
@@ -381,6 +381,7 @@ extern "C" int mui_int8_linear(mui_stream_t stream, int dtype, const void* weigh
     sp.x = (const uint16_t*)x; sp.gamma = (const uint16_t*)norm_weights;
     sp.add_bias = (const uint16_t*)add_bias; sp.residual = (const uint16_t*)residual;
     sp.y = (uint16_t*)y; sp.n = n_out; sp.k = k_in; sp.tokens = tokens; sp.eps = epsilon;
+    sp.workspace = workspace; sp.workspace_bytes = workspace_bytes;
     return launch_prefill_gemm(s, dtype, WF_I8_CHANNEL, SK_LINEAR, sp);
   }
   if (tokens >= 2 || (g_int8_dot2 && dtype == MUI_DTYPE_F16)) {
@@ -409,6 +410,13 @@ extern "C" int mui_int8_linear(mui_stream_t stream, int dtype, const void* weigh
     if (st != MUI_OK) return st;
   }
   return MUI_OK;
+}
+
+extern "C" int mui_int8_linear(mui_stream_t stream, int dtype, const void* weights_i8, long w_pitch,
+                               const void* scales, const void* x, const void* norm_weights,
+                               float epsilon, const void* add_bias, const void* residual, void* y,
+                               int n_out, int k_in, int tokens) {
+  return mui_int8_linear_ws(stream, dtype, weights_i8, w_pitch, scales, x, norm_weights, epsilon, add_bias, residual, y, n_out, k_in, tokens, nullptr, 0);
 }
 
 extern "C" int mui_int8_gateup_silu(mui_stream_t stream, int dtype, const void* gate_i8,
@@ -457,14 +465,14 @@ extern "C" int mui_int8_gateup_silu(mui_stream_t stream, int dtype, const void* 
   return MUI_OK;
 }
 
-extern "C" int mui_int8_group_linear(mui_stream_t stream, int dtype, const void* weights_u8,
+extern "C" int mui_int8_group_linear_ws(mui_stream_t stream, int dtype, const void* weights_u8,
                                      long w_pitch, const void* scales_min_vals, int group_size_shift,
                                      const void* x, const void* norm_weights, float epsilon,
                                      const void* add_bias, const void* residual, void* y, int n_out,
-                                     int k_in, int tokens) {
+                                     int k_in, int tokens, void* workspace, size_t workspace_bytes) {
   int st = check_int8_common(dtype, weights_u8, w_pitch, x, norm_weights, n_out, k_in, tokens, true);
   if (st != MUI_OK) return st;
-  MUI_CHECK_ARG(scales_min_vals && y);
+  MUI_CHECK_ARG(scales_min_vals && y && (workspace || workspace_bytes == 0));
   if (group_size_shift < 4 || group_size_shift > 30) return MUI_ERR_UNSUPPORTED;
   if (k_in & ((1 << group_size_shift) - 1)) return MUI_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
@@ -475,6 +483,7 @@ extern "C" int mui_int8_group_linear(mui_stream_t stream, int dtype, const void*
     sp.x = (const uint16_t*)x; sp.gamma = (const uint16_t*)norm_weights;
     sp.add_bias = (const uint16_t*)add_bias; sp.residual = (const uint16_t*)residual;
     sp.y = (uint16_t*)y; sp.n = n_out; sp.k = k_in; sp.tokens = tokens; sp.eps = epsilon;
+    sp.workspace = workspace; sp.workspace_bytes = workspace_bytes;
     return launch_prefill_gemm(s, dtype, WF_U8_GROUP, SK_LINEAR, sp);
   }
   if (tokens >= 2 || (g_int8_dot2 && dtype == MUI_DTYPE_F16)) {
@@ -505,6 +514,14 @@ extern "C" int mui_int8_group_linear(mui_stream_t stream, int dtype, const void*
     if (st != MUI_OK) return st;
   }
   return MUI_OK;
+}
+
+extern "C" int mui_int8_group_linear(mui_stream_t stream, int dtype, const void* weights_u8,
+                                     long w_pitch, const void* scales_min_vals, int group_size_shift,
+                                     const void* x, const void* norm_weights, float epsilon,
+                                     const void* add_bias, const void* residual, void* y, int n_out,
+                                     int k_in, int tokens) {
+  return mui_int8_group_linear_ws(stream, dtype, weights_u8, w_pitch, scales_min_vals, group_size_shift, x, norm_weights, epsilon, add_bias, residual, y, n_out, k_in, tokens, nullptr, 0);
 }
 
 extern "C" int mui_int8_group_gateup_silu(mui_stream_t stream, int dtype, const void* gate_u8,

@@ -185,23 +185,39 @@ static int launch_join(hipStream_t s, const JoinRow& p) {
 }
 constexpr int kJoinMost = 8192;  // outputs
 
-// MUI_ERR_UNSUPPORTED: not a case for it, nothing has been launched
-static int linear_join(hipStream_t s, int dtype, const void* weights, long w_pitch, const void* x, int k, JoinRow p, bool f32, void* workspace,
-                       size_t workspace_bytes) {
+// q: the product, without what its end applies. MUI_ERR_UNSUPPORTED: not a case for it, nothing has been launched
+static int linear_join(hipStream_t s, int dtype, int wf, SkinnyParams q, JoinRow p, bool f32, void* workspace, size_t workspace_bytes) {
   if (p.tokens <= MUI_MAX_TOKENS || p.n > kJoinMost || !p.h || !workspace || ((uintptr_t)workspace & 255u) || workspace_bytes < prefill_workspace_bytes()) return MUI_ERR_UNSUPPORTED;
-  const void* ptrs[] = {p.add_bias, p.r32, p.r16, p.post_gain, p.next_gain, p.y, p.r_out, p.h};
-  for (const void* q : ptrs)
-    if (!aligned16(q)) return MUI_ERR_UNSUPPORTED;
-  SkinnyParams q = {};
-  q.w0 = weights; q.pitch = w_pitch; q.x = (const uint16_t*)x; q.y = p.y; q.n = p.n; q.k = k; q.tokens = p.tokens;
+  const void* ptrs[] = {q.w0, q.x, p.add_bias, p.r32, p.r16, p.post_gain, p.next_gain, p.y, p.r_out, p.h};
+  for (const void* at : ptrs)
+    if (!aligned16(at)) return MUI_ERR_UNSUPPORTED;
+  q.y = p.y; q.n = p.n; q.tokens = p.tokens;
   float* part = (float*)((char*)workspace + prefill_counter_bytes());
   // (K is divided only where it is without the norm, too: whether the boundary was taken along, a hook was listening or all layers came in one call does not show in the bits)
   const size_t part_bytes = workspace_bytes - prefill_counter_bytes();
-  const int st = p.tokens <= 128 ? launch_gemm_stream_parts(s, dtype, q, part, part_bytes, &p.splits) : launch_prefill_parts(s, dtype, WF_16BIT, q, part, part_bytes, &p.splits);
+  const int st = wf == WF_16BIT && p.tokens <= 128 ? launch_gemm_stream_parts(s, dtype, q, part, part_bytes, &p.splits)
+                                                   : launch_prefill_parts(s, dtype, wf, q, part, part_bytes, &p.splits);
   if (st != MUI_OK) return st;
   p.part = part;
   if (dtype == MUI_DTYPE_F16) return f32 ? launch_join<F16, true>(s, p) : launch_join<F16, false>(s, p);
   return f32 ? launch_join<BF16, true>(s, p) : launch_join<BF16, false>(s, p);
+}
+
+static SkinnyParams product(const void* weights, long w_pitch, const void* x, int k) {
+  SkinnyParams q = {};
+  q.w0 = weights; q.pitch = w_pitch; q.x = (const uint16_t*)x; q.k = k;
+  return q;
+}
+
+// int8 codes with the residual and the norm behind, where K is shared between workgroups; MUI_ERR_UNSUPPORTED: it is not, nothing has been launched
+int launch_codes_norm(hipStream_t s, int dtype, int wf, const SkinnyParams& q, const void* next_gain, float eps, void* h) {
+  if (q.gamma || q.mul_bias) return MUI_ERR_UNSUPPORTED;
+  JoinRow p = {};
+  p.n = q.n; p.tokens = q.tokens; p.add_bias = q.add_bias; p.r16 = q.residual; p.next_gain = (const uint16_t*)next_gain;
+  p.next_scale = 1.f; p.eps = eps; p.y = q.y; p.h = (uint16_t*)h;
+  SkinnyParams a = q;
+  a.add_bias = a.residual = nullptr;
+  return linear_join(s, dtype, wf, a, p, false, q.workspace, q.workspace_bytes);
 }
 
 static bool linear_args(int dtype, const void* weights, long w_pitch, const void* x, const void* y, int n, int k, int tokens) {
@@ -218,12 +234,12 @@ extern "C" int mui_linear_residual_norm(mui_stream_t stream, int dtype, const vo
                                         void* workspace, size_t workspace_bytes) {
   MUI_CHECK_ARG(linear_args(dtype, weights, w_pitch, x, y, n_out, k_in, tokens));
   MUI_CHECK_ARG(residual_out && (h || !next_gain) && (workspace || workspace_bytes == 0));
-  if (aligned16(weights) && aligned16(x)) {
+  {
     JoinRow p = {};
     p.n = n_out; p.tokens = tokens; p.add_bias = (const uint16_t*)add_bias; p.r32 = residual_in; p.post_gain = (const uint16_t*)post_gain;
     p.next_gain = (const uint16_t*)next_gain; p.branch_scale = branch_scale; p.next_scale = next_scale; p.eps = epsilon;
     p.y = (uint16_t*)y; p.r_out = residual_out; p.h = (uint16_t*)h;
-    const int st = linear_join((hipStream_t)stream, dtype, weights, w_pitch, x, k_in, p, true, workspace, workspace_bytes);
+    const int st = linear_join((hipStream_t)stream, dtype, WF_16BIT, product(weights, w_pitch, x, k_in), p, true, workspace, workspace_bytes);
     if (st != MUI_ERR_UNSUPPORTED) return st;
   }
   const int st = mui_linear_ws(stream, dtype, weights, w_pitch, x, nullptr, 0.f, nullptr, add_bias, nullptr, y, n_out, k_in, tokens, workspace, workspace_bytes);
@@ -236,11 +252,11 @@ extern "C" int mui_linear_norm(mui_stream_t stream, int dtype, const void* weigh
                                size_t workspace_bytes) {
   MUI_CHECK_ARG(linear_args(dtype, weights, w_pitch, x, y, n_out, k_in, tokens));
   MUI_CHECK_ARG(residual && next_gain && h && (workspace || workspace_bytes == 0));
-  if (aligned16(weights) && aligned16(x)) {
+  {
     JoinRow p = {};
     p.n = n_out; p.tokens = tokens; p.add_bias = (const uint16_t*)add_bias; p.r16 = (const uint16_t*)residual; p.next_gain = (const uint16_t*)next_gain;
     p.next_scale = 1.f; p.eps = epsilon; p.y = (uint16_t*)y; p.h = (uint16_t*)h;
-    const int st = linear_join((hipStream_t)stream, dtype, weights, w_pitch, x, k_in, p, false, workspace, workspace_bytes);
+    const int st = linear_join((hipStream_t)stream, dtype, WF_16BIT, product(weights, w_pitch, x, k_in), p, false, workspace, workspace_bytes);
     if (st != MUI_ERR_UNSUPPORTED) return st;
   }
   const int st = mui_linear_ws(stream, dtype, weights, w_pitch, x, nullptr, 0.f, nullptr, add_bias, residual, y, n_out, k_in, tokens, workspace, workspace_bytes);

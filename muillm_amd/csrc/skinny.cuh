@@ -203,6 +203,7 @@ size_t prefill_workspace_bytes();  // what SkinnyParams::workspace must hold for
 size_t prefill_workspace_best();   // beyond, more of it is no use
 // more than 128 tokens, n % 4 == 0: fp32 partial outputs [*shares][tokens][n] of shares of K, where they are worth it, and what adds them up behind
 int launch_prefill_parts(hipStream_t s, int dtype, int weight_format, const SkinnyParams& p, float* part, size_t part_bytes, int* shares);
+int launch_codes_norm(hipStream_t s, int dtype, int weight_format, const SkinnyParams& p, const void* next_gain, float eps, void* h);  // (linear_join.hip)
 int launch_parts_add(hipStream_t s, int dtype, const SkinnyParams& p, float* part, int shares);
 size_t prefill_counter_bytes();    // of that, at its start: counters that stay zero
 // 17..128 tokens: 16 weight rows per workgroup, K split over its waves, token columns in up to 8 MFMA tiles (gemm_wide.hip)

@@ -163,6 +163,12 @@ def _prompt_workspace(x: torch.Tensor, stream: int) -> Optional[torch.Tensor]:
     return ws
 
 
+def _codes_workspace(x: torch.Tensor, tokens: int):
+    """(address, bytes) of the scratch of int8 linears, which share K from 65 tokens on."""
+    ws = _prompt_workspace(x, _stream(x)) if tokens > 64 else None
+    return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
+
+
 class ResidualBehind:
     """The boundary between two sublayers with an fp32 residual stream (hybrid_ops.residual_norm) that follows a linear and is taken along by its
     library call: the stream and the next sublayer's input. An object lives for one boundary of one forward pass: whoever makes it hands it to
@@ -542,15 +548,16 @@ def mui_int8_channel_linear_forward(x, weights_i8, scales, norm_weights=None, ep
         residual = residual.contiguous()
     y = torch.empty(list(x.shape[:-1]) + [n], dtype=x.dtype, device=x.device)
     esz = x.element_size()
+    ws_args = _codes_workspace(x, tokens)
     for off, cnt in _token_chunks(tokens):
         check(
-            _lib.load().mui_int8_linear(_stream(x), _dtype_code(x), weights_i8.data_ptr(),
-                                        _byte_pitch(weights_i8, "weights"), scales.data_ptr(),
-                                        x.data_ptr() + off * k * esz, _ptr(norm_weights), float(epsilon),
-                                        _ptr(add_bias),
-                                        None if residual is None else residual.data_ptr() + off * n * esz,
-                                        y.data_ptr() + off * n * esz, n, k, cnt),
-            "mui_int8_linear",
+            _lib.load().mui_int8_linear_ws(_stream(x), _dtype_code(x), weights_i8.data_ptr(),
+                                           _byte_pitch(weights_i8, "weights"), scales.data_ptr(),
+                                           x.data_ptr() + off * k * esz, _ptr(norm_weights), float(epsilon),
+                                           _ptr(add_bias),
+                                           None if residual is None else residual.data_ptr() + off * n * esz,
+                                           y.data_ptr() + off * n * esz, n, k, cnt, *ws_args),
+            "mui_int8_linear_ws",
         )
     return y
 
@@ -647,15 +654,16 @@ def muillm_int8_linear_forward(x, weights, scales_min_vals, group_size_shift, no
         residual = residual.contiguous()
     y = torch.empty(list(x.shape[:-1]) + [n], dtype=x.dtype, device=x.device)
     esz = x.element_size()
+    ws_args = _codes_workspace(x, tokens)
     for off, cnt in _token_chunks(tokens, group_format=True):
         check(
-            _lib.load().mui_int8_group_linear(_stream(x), _dtype_code(x), weights.data_ptr(),
-                                              _byte_pitch(weights, "weights"), scales_min_vals.data_ptr(),
-                                              int(group_size_shift), x.data_ptr() + off * k * esz,
-                                              _ptr(norm_weights), float(epsilon), _ptr(add_bias),
-                                              None if residual is None else residual.data_ptr() + off * n * esz,
-                                              y.data_ptr() + off * n * esz, n, k, cnt),
-            "mui_int8_group_linear",
+            _lib.load().mui_int8_group_linear_ws(_stream(x), _dtype_code(x), weights.data_ptr(),
+                                                 _byte_pitch(weights, "weights"), scales_min_vals.data_ptr(),
+                                                 int(group_size_shift), x.data_ptr() + off * k * esz,
+                                                 _ptr(norm_weights), float(epsilon), _ptr(add_bias),
+                                                 None if residual is None else residual.data_ptr() + off * n * esz,
+                                                 y.data_ptr() + off * n * esz, n, k, cnt, *ws_args),
+            "mui_int8_group_linear_ws",
         )
     return y
 

@@ -68,3 +68,64 @@ def test_by_the_rule_and_with_the_norm_behind(n, k, tokens, dtype):
     _lib.check(lib.mui_residual_norm(s, code, stream.data_ptr(), y2.data_ptr(), 1.0, post.data_ptr(), 0.5, after.data_ptr(), 2.0, EPS, out2.data_ptr(), h2.data_ptr(), tokens, n), "norm")
     _call("mui_linear_residual_norm", x, w, k, None, (stream.data_ptr(), post.data_ptr(), 0.5, after.data_ptr(), 2.0, EPS, y.data_ptr(), out.data_ptr(), h.data_ptr()), y, ws)
     assert torch.equal(y, y2) and torch.equal(out, out2) and torch.equal(h, h2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shift", [0, 6, 7])
+@pytest.mark.parametrize("tile,shares", [(7, 7), (8, 3), (4, 5)])
+@pytest.mark.parametrize("n,k,tokens", [(4, 3072, 65), (260, 3200, 257), (4104, 2816, 300)])
+def test_codes(n, k, tokens, tile, shares, shift, dtype, tune):
+    """int8 with a scale per row (shift 0) and in groups: forced shares, and the same without scratch. Groups in bf16 are left whole."""
+    lib, s, g = _lib.load(), torch.cuda.current_stream().cuda_stream, _gen(n + k + tokens + shift)
+    q = torch.randint(-128, 128, (n, k), device=DEV, generator=g, dtype=torch.int16)
+    x, res, bias = _rand((tokens, k), dtype, g), _rand((tokens, n), dtype, g), _rand((n,), dtype, g)
+    if shift:
+        groups = k >> shift
+        scale = (torch.rand(n, groups, device=DEV, generator=g) * 2e-3 + 1e-3).to(dtype)
+        pairs = torch.stack([scale, (scale.float() * -128).to(dtype)], 2).contiguous()
+        codes = (q + 128).to(torch.uint8)
+        w = (codes.float().view(n, groups, -1) * pairs[..., :1].float() + pairs[..., 1:].float()).to(dtype).double().view(n, k)  # (what is multiplied is rounded)
+    else:
+        pairs, codes = (torch.rand(n, device=DEV, generator=g) * 2e-3 + 1e-3).to(dtype), q.to(torch.int8)
+        w = codes.double() * pairs.double()[:, None]
+    ref = x.double() @ w.T + bias.double() + res.double()
+    ws = torch.zeros(lib.mui_linear_workspace_bytes(), dtype=torch.uint8, device=DEV)
+    tune(tile, shares)
+    for scratch in (ws, None):
+        y = torch.full((tokens, n), float("nan"), dtype=dtype, device=DEV)
+        end = (x.data_ptr(), None, 0.0, bias.data_ptr(), res.data_ptr(), y.data_ptr(), n, k, tokens, _ptr(scratch), 0 if scratch is None else scratch.numel())
+        if shift:
+            _lib.check(lib.mui_int8_group_linear_ws(s, CODE[dtype], codes.data_ptr(), k, pairs.data_ptr(), shift, *end), "groups")
+        else:
+            _lib.check(lib.mui_int8_linear_ws(s, CODE[dtype], codes.data_ptr(), k, pairs.data_ptr(), *end), "rows")
+        _close(y, ref, 2 * HALF_ULP[dtype])
+    assert bool(ws[4096:].any()) == (not shift or dtype == torch.float16)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("group", [0, 128])
+def test_int8_prompts_in_one_call_and_layer_by_layer(group, monkeypatch):
+    """The norms behind shared linears, taken along in the single call, give the bits of the layers' own calls."""
+    from muillm_amd.engine import init_engine
+    from muillm_amd.engineconfig import MuiEngineConfig
+    from muillm_amd.modules.models.llama.model import MuiDecoderConfig, MuiLlamaForCausalLM
+    from muillm_amd.quantization.quantizationmethod import Int8WeightOnlyQuantizationMethod
+
+    torch.manual_seed(3)
+    config = MuiDecoderConfig(hidden_size=2048, intermediate_size=8192, num_hidden_layers=2, num_attention_heads=16, num_key_value_heads=4, vocab_size=512)
+    lm = MuiLlamaForCausalLM.from_config(MuiEngineConfig(), config, dtype=torch.float16, device=DEV, finalize=False)
+    lm = init_engine(lm, device=DEV, engine_config=MuiEngineConfig(Int8WeightOnlyQuantizationMethod(group_size=group, modules=["qkv_proj", "o_proj", "mlp"])))
+    assert prompt_shares("int8_group" if group else "int8", 2048, 8192, 150)[1] > 1
+    ids = torch.randint(0, 512, (1, 150), generator=torch.Generator().manual_seed(4)).to(DEV)
+
+    def logits():
+        cache = lm.create_cache(1, 160)
+        return lm(input_ids=ids, past_key_values=cache, use_cache=True, all_ones_mask=True).logits
+
+    one = logits()
+    handle = lm.model.norm.register_forward_pre_hook(lambda *a: None)
+    hooks = [layer.self_attn.o_proj.register_forward_hook(lambda *a: None) for layer in lm.model.layers]
+    apart = logits()
+    for h in [handle] + hooks:
+        h.remove()
+    assert bool(torch.isfinite(one).all()) and torch.equal(one, apart)
