@@ -119,6 +119,7 @@ _SIGNATURES = {
     "mui_moe_route": (c_int, [_P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, _P, _P, _P, _P]),
     "mui_moe_gateup": (c_int, [_P, c_int, _P, _P, c_long, _P, c_float, _P, _P, _P, c_int, _P, c_int, c_int, c_int,
                                c_int, c_int]),
+    "mui_moe_route_gateup": (c_int, [_P, c_int, _P, _P, c_int, _P, _P, c_long, _P, c_float, c_int, _P, _P, _P, _P, _P] + [c_int] * 5),
     "mui_moe_down": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int]),
     "mui_latent_prepare": (c_int, [_P, c_int, _P, c_long, _P, _P, c_float, _P, _P, _P, _P, _P, _P, c_long, _P, c_long,
                                    c_int, c_int, c_int, c_int, c_int, c_int]),

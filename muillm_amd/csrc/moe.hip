@@ -35,6 +35,18 @@ __device__ __forceinline__ float moe_act(float g, float u, float limit) {
   return g / (1.0f + __expf(-1.702f * g)) * (u + 1.0f);
 }
 
+template <typename T>
+__device__ __forceinline__ float moe_dot2(uint32_t a, uint32_t b, float c);
+template <>
+__device__ __forceinline__ float moe_dot2<F16>(uint32_t a, uint32_t b, float c) {
+  return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), c, false);
+}
+typedef __bf16 bf16x2_moe __attribute__((ext_vector_type(2)));
+template <>
+__device__ __forceinline__ float moe_dot2<BF16>(uint32_t a, uint32_t b, float c) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_moe, a), __builtin_bit_cast(bf16x2_moe, b), c, false);
+}
+
 // ---------------------------------------------------------------------------------------
 // fp32 outputs of a small matrix: y[t, n] = W[n, :] . x[t, :] + bias[n], one workgroup per row
 // ---------------------------------------------------------------------------------------
@@ -916,6 +928,141 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(const MoeGemmParams p) {
   }
 }
 
+// One token: routing, gate and up in one launch. Every workgroup chooses the experts by itself: a thread per output counts those that are ahead of its own (top rounds of
+// a maximum over a wave took 3 us longer), about a microsecond behind the logits, where a launch for it is five. Then the chosen experts' rows are one long list for the
+// single-token GEMV structure of gemv_multi.hip: gate and up rows of two outputs at a time, thread t has chunks t, t + 256 of every row, the next rows are requested before
+// the sums meet. A matrix instruction has no use for fifteen of its sixteen columns here, and weights go from memory to registers to the ALU without LDS between. Workgroup
+// 0 writes down what was chosen, and the tiles of one pair that the down product reads. us of routing, gate and up in bf16 as captured, two launches / this: 64 experts of 1792 x 4096, 8 / 7 / 6 of them
+// 46.8 / 39.3, 44.6 / 35.5, 36.9 / 30.9 (their bytes take 33.1, 28.9, 24.8); of 1408 x 2048, 6 / 5 21.6 / 16.1, 18.8 / 14.3 (9.7, 8.1).
+constexpr int kMoeOneOutputs = 256, kMoeOneTop = 8;
+template <typename T, int CH, bool STREAM>
+__global__ void __launch_bounds__(256) moe_one_gateup_kernel(const float* logits, const uint16_t* corr, const uint16_t* x, int n_out, int k, const uint16_t* w0,
+                                                             const uint16_t* w1, int n_experts, int top, long expert_stride, int n, float limit, uint16_t* act,
+                                                             int32_t* expert, float* weight, int32_t* pairs, MoeTile* tiles, int max_tiles) {
+  constexpr int R = 4, OUT = R / 2;
+  __shared__ float red[2][16][R];  // [buffer][16-lane row of the workgroup][row]
+  __shared__ float meet[2][4];
+  __shared__ __align__(16) float value[kMoeOneOutputs];
+  __shared__ int list[kMoeOneTop][2];  // of the chosen with matrices: which it is, its place in the choice
+  __shared__ int real_s;
+  const int t = threadIdx.x, lane = t & (kWave - 1), kc = k >> 3;
+  const bool there = t < n_out;
+  float lg = logits[there ? t : 0], add = T::one(*(corr ? corr + (there ? t : 0) : x));
+  int coff[CH];
+  u32x4 xq[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int c = t + 256 * j;
+    coff[j] = c < kc ? c << 3 : 0;
+    xq[j] = ld16(x + coff[j]);
+  }
+  lg = there ? lg : -INFINITY;
+  const float wave_mx = wave_max(lg);
+  if (lane == 0) meet[0][t >> 6] = wave_mx;
+  if (t == 0) real_s = 0;
+  if (t < 2 * kMoeOneTop) list[t >> 1][t & 1] = 0;
+  __syncthreads();
+  const float ex = expf(lg - fmaxf(fmaxf(meet[0][0], meet[0][1]), fmaxf(meet[0][2], meet[0][3])));
+  const float wave_ex = wave_sum(ex);
+  if (lane == 0) meet[1][t >> 6] = wave_ex;
+  __syncthreads();
+  const float share = ex / ((meet[1][0] + meet[1][1]) + (meet[1][2] + meet[1][3]));
+  float choice = share + (corr ? add : 0.f);
+  choice = there & (choice == choice) ? choice : -INFINITY;
+  value[t] = choice;
+  __syncthreads();
+  if (there) {
+    // how many outputs are ahead of this one, and how many of them have matrices (those past the last one are behind all)
+    int ahead = 0, ahead_real = 0;
+#pragma unroll 2
+    for (int i = 0; i < n_out; i += 8) {
+      const f32x4 v0 = *(const f32x4*)&value[i], v1 = *(const f32x4*)&value[(i + 4) & (kMoeOneOutputs - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float v = u < 4 ? v0[u & 3] : v1[u & 3];
+        const int before = (int)(v > choice) | ((int)(v == choice) & (int)(i + u < t));
+        ahead += before;
+        ahead_real += i + u < n_experts ? before : 0;
+      }
+    }
+    if (ahead < top) {
+      if (t < n_experts) {
+        list[ahead_real][0] = t;
+        list[ahead_real][1] = ahead;
+        atomicAdd(&real_s, 1);
+      }
+      if (blockIdx.x == 0) {
+        expert[ahead] = t;
+        weight[ahead] = share;
+      }
+    }
+  }
+  __syncthreads();
+  const int real = __builtin_amdgcn_readfirstlane(real_s);
+#pragma unroll
+  for (int j = 0; j < CH; ++j)
+    if (t + 256 * j >= kc) xq[j] = u32x4{0u, 0u, 0u, 0u};
+  if (blockIdx.x == 0) {
+    if (t == 0) tiles[0] = MoeTile{0, 0, real, 0};
+    if (t < max_tiles) {
+      tiles[1 + t] = t < real ? MoeTile{list[t][0], t, 1, 0} : MoeTile{0, 0, 0, 0};
+      if (t < real) pairs[t] = list[t][1];
+    }
+  }
+  const int groups = real * (n / OUT);  // (n is even)
+  struct Place { int slot, row, expert, place; } now = {0, (int)blockIdx.x * OUT, 0, 0}, next;
+  auto settle = [&](Place& p) {  // the row's expert
+    while (p.row >= n && p.slot + 1 < kMoeOneTop) {
+      p.row -= n;
+      ++p.slot;
+    }
+    p.expert = __builtin_amdgcn_readfirstlane(list[p.slot][0]);
+    p.place = __builtin_amdgcn_readfirstlane(list[p.slot][1]);
+  };
+  u32x4 w[R][CH];
+  auto request = [&](const Place& p) {
+    const long base = (long)p.expert * expert_stride + (long)p.row * k;
+    const uint16_t *gate = w0 + base, *up = w1 + base;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int j = 0; j < CH; ++j) w[r][j] = ld16_sel<STREAM>(((r & 1) ? up : gate) + (long)(r >> 1) * k + coff[j]);
+  };
+  int buf = 0;
+  if ((int)blockIdx.x >= groups) return;  // uniform for the workgroup
+  settle(now);
+  request(now);
+  for (int g = blockIdx.x; g < groups; g += gridDim.x) {
+    next = now;
+    next.row += (int)gridDim.x * OUT;
+    settle(next);
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      float a = 0.f;
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        a = moe_dot2<T>(w[r][j].x, xq[j].x, a);
+        a = moe_dot2<T>(w[r][j].y, xq[j].y, a);
+        a = moe_dot2<T>(w[r][j].z, xq[j].z, a);
+        a = moe_dot2<T>(w[r][j].w, xq[j].w, a);
+      }
+      acc[r] = a;
+    }
+    if (g + (int)gridDim.x < groups) request(next);
+    row16_reduce_scatter<R>(acc, lane);
+    if ((lane & (16 / R - 1)) == 0) red[buf][t >> 4][(lane & 15) / (16 / R)] = acc[0];
+    __syncthreads();
+    if (t < 16 * OUT) {  // sixteen lanes per output
+      const int part = t & 15, o = t >> 4;
+      const float v0 = row16_sum(red[buf][part][2 * o]), v1 = row16_sum(red[buf][part][2 * o + 1]);
+      if (part == 0) act[(long)now.place * n + now.row + o] = T::pack(moe_act(v0, v1, limit));
+    }
+    buf ^= 1;
+    now = next;
+  }
+}
+
 // one wave per output of a pair: fp32 storage, and sizes that are no multiple of 8
 template <typename T, int EPI>
 __global__ void __launch_bounds__(256) moe_rows_kernel(const typename T::storage* w0, const typename T::storage* w1,
@@ -1141,6 +1288,51 @@ extern "C" int mui_moe_gateup(mui_stream_t stream, int dtype, const void* gate, 
   p.limit = limit; p.max_tiles = mui_moe_max_tiles(tokens, top, n_experts, tile_pairs);
   p.once = read_once(n_experts, n_inter, k_in, gate, up);
   MUI_BY_DTYPE((launch_moe_product<TT, MOE_GATEUP>((hipStream_t)stream, p, expert, n_experts, tokens * top, tile_pairs)));
+}
+
+namespace mui {
+// One token and sizes that moe_one_gateup_kernel covers, else MUI_ERR_UNSUPPORTED (nothing launched)
+template <typename T>
+static int launch_moe_one(hipStream_t s, const MoeGemmParams& p, const float* logits, const void* corr, int n_out, int n_experts, int32_t* expert, float* weight,
+                          int32_t* pairs, MoeTile* tiles) {
+  if constexpr (T::kDtype == MUI_DTYPE_F32) {
+    return MUI_ERR_UNSUPPORTED;
+  } else {
+    if (p.tokens != 1 || n_out > kMoeOneOutputs || p.top > kMoeOneTop || p.n % 2 || p.k % 8 || p.k > 2 * 256 * 8 || p.expert_stride % 8) return MUI_ERR_UNSUPPORTED;
+    if (!aligned16(p.w0) || !aligned16(p.w1) || !aligned16(p.x) || (long)p.top * p.n >= (1L << 30)) return MUI_ERR_UNSUPPORTED;
+    const dim3 grid(balanced_grid(p.top * (p.n / 2), 3)), block(256);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, 0, s, logits, (const uint16_t*)corr, p.x, n_out, p.k, p.w0, p.w1, n_experts, p.top, p.expert_stride, p.n, p.limit,
+                         (uint16_t*)p.y, expert, weight, pairs, tiles, p.max_tiles);
+      return launch_status();
+    };
+    if (p.k <= 256 * 8) return p.once ? launch(moe_one_gateup_kernel<T, 1, true>) : launch(moe_one_gateup_kernel<T, 1, false>);
+    return p.once ? launch(moe_one_gateup_kernel<T, 2, true>) : launch(moe_one_gateup_kernel<T, 2, false>);
+  }
+}
+
+}  // namespace mui
+
+extern "C" int mui_moe_route_gateup(mui_stream_t stream, int dtype, const float* logits, const void* correction, int n_identity, const void* gate, const void* up,
+                                    long expert_stride, const void* x, float limit, int tile_pairs, int32_t* expert, float* weight, int32_t* pairs, void* tiles,
+                                    void* act, int n_experts, int n_inter, int k_in, int top, int tokens) {
+  if (tile_pairs == 16 && tokens == 1) {
+    MUI_CHECK_ARG(logits && gate && up && x && act && expert && weight && pairs && tiles && n_experts > 0 && n_identity >= 0 && n_inter > 0 && k_in > 0);
+    MUI_CHECK_ARG(top > 0 && top <= n_experts + n_identity);
+    MoeGemmParams p = {};
+    p.w0 = (const uint16_t*)gate; p.w1 = (const uint16_t*)up; p.expert_stride = expert_stride; p.x = (const uint16_t*)x; p.y = act;
+    p.n = n_inter; p.k = k_in; p.top = top; p.tokens = 1; p.limit = limit;
+    p.max_tiles = mui_moe_max_tiles(1, top, n_experts, 16);
+    p.once = read_once(n_experts, n_inter, k_in, gate, up);
+    auto one = [&](auto t) {
+      return launch_moe_one<decltype(t)>((hipStream_t)stream, p, logits, correction, n_experts + n_identity, n_experts, expert, weight, pairs, (MoeTile*)tiles);
+    };
+    const int st = dtype == MUI_DTYPE_F16 ? one(F16{}) : dtype == MUI_DTYPE_BF16 ? one(BF16{}) : MUI_ERR_UNSUPPORTED;
+    if (st != MUI_ERR_UNSUPPORTED) return st;
+  }
+  const int st = mui_moe_route(stream, dtype, logits, correction, n_experts, n_identity, top, tokens, tile_pairs, expert, weight, pairs, tiles);
+  if (st != MUI_OK) return st;
+  return mui_moe_gateup(stream, dtype, gate, up, expert_stride, x, limit, expert, pairs, tiles, tile_pairs, act, n_experts, n_inter, k_in, top, tokens);
 }
 
 extern "C" int mui_moe_down(mui_stream_t stream, int dtype, const void* down, long expert_stride, const void* act,

@@ -128,6 +128,17 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
 # --------------------------------------------------------------------------------------
 # mixture of experts
 # --------------------------------------------------------------------------------------
+def _routing(tokens: int, top: int, n_experts: int, tile_pairs: int, dev):
+    expert = torch.empty((tokens, top), dtype=torch.int32, device=dev)
+    weight = torch.empty((tokens, top), dtype=torch.float32, device=dev)
+    pairs = tiles = None
+    if tile_pairs:
+        pairs = torch.empty(tokens * top, dtype=torch.int32, device=dev)
+        n_tiles = _lib.load().mui_moe_max_tiles(tokens, top, n_experts, tile_pairs)
+        tiles = torch.empty((n_tiles + 1, 4), dtype=torch.int32, device=dev)
+    return expert, weight, pairs, tiles
+
+
 def moe_route(logits: torch.Tensor, correction: Optional[torch.Tensor], n_experts: int, top: int, tile_pairs: int):
     """(expert int32 [T, top], weight fp32 [T, top], pairs, tiles): see mui_moe_route. logits fp32
     [T, outputs]; outputs beyond n_experts are identity experts."""
@@ -136,13 +147,7 @@ def moe_route(logits: torch.Tensor, correction: Optional[torch.Tensor], n_expert
     dtype = logits.dtype if correction is None else correction.dtype
     _operand(correction, "correction", logits, (n_out,), dtype)
     lib, dev = _lib.load(), logits.device
-    expert = torch.empty((tokens, top), dtype=torch.int32, device=dev)
-    weight = torch.empty((tokens, top), dtype=torch.float32, device=dev)
-    pairs = tiles = None
-    if tile_pairs:
-        pairs = torch.empty(tokens * top, dtype=torch.int32, device=dev)
-        n_tiles = lib.mui_moe_max_tiles(tokens, top, n_experts, tile_pairs)
-        tiles = torch.empty((n_tiles + 1, 4), dtype=torch.int32, device=dev)
+    expert, weight, pairs, tiles = _routing(tokens, top, n_experts, tile_pairs, dev)
     check(lib.mui_moe_route(_stream(logits), dtype_code(dtype), logits.data_ptr(), _ptr(correction), n_experts,
                             n_out - n_experts, top, tokens, tile_pairs, expert.data_ptr(), weight.data_ptr(),
                             _ptr(pairs), _ptr(tiles)), "mui_moe_route")
@@ -155,19 +160,49 @@ def moe_experts(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, down: tor
     gate, up [E, ff, width], down [E, width, ff]."""
     n_experts, ff, width = gate.shape
     tokens, top = expert.shape
+    _expert_operands(x, gate, up, down, tokens)
+    lib, code, st = _lib.load(), dtype_code(x.dtype), _stream(x)
+    act = torch.empty((tokens * top, ff), dtype=x.dtype, device=x.device)
+    check(lib.mui_moe_gateup(st, code, gate.data_ptr(), up.data_ptr(), ff * width, x.data_ptr(), float(limit),
+                             expert.data_ptr(), _ptr(pairs), _ptr(tiles), tile_pairs, act.data_ptr(), n_experts, ff,
+                             width, top, tokens), "mui_moe_gateup")
+    return _moe_down(act, down, expert, pairs, tiles, tile_pairs)
+
+
+def _expert_operands(x, gate, up, down, tokens):
+    n_experts, ff, width = gate.shape
     _operand(x, "x", x, (tokens, width))
     _operand(gate, "gate", x)
     _operand(up, "up", x, (n_experts, ff, width))
     _operand(down, "down", x, (n_experts, width, ff))
-    lib, code, st = _lib.load(), dtype_code(x.dtype), _stream(x)
-    act = torch.empty((tokens * top, ff), dtype=x.dtype, device=x.device)
-    out = torch.empty((tokens * top, width), dtype=x.dtype, device=x.device)
-    check(lib.mui_moe_gateup(st, code, gate.data_ptr(), up.data_ptr(), ff * width, x.data_ptr(), float(limit),
-                             expert.data_ptr(), _ptr(pairs), _ptr(tiles), tile_pairs, act.data_ptr(), n_experts, ff,
-                             width, top, tokens), "mui_moe_gateup")
+
+
+def _moe_down(act, down, expert, pairs, tiles, tile_pairs):
+    (n_experts, width, ff), (tokens, top) = down.shape, expert.shape
+    lib, code, st = _lib.load(), dtype_code(act.dtype), _stream(act)
+    out = torch.empty((tokens * top, width), dtype=act.dtype, device=act.device)
     check(lib.mui_moe_down(st, code, down.data_ptr(), width * ff, act.data_ptr(), expert.data_ptr(), _ptr(pairs),
                            _ptr(tiles), tile_pairs, out.data_ptr(), n_experts, width, ff, top, tokens), "mui_moe_down")
     return out
+
+
+def moe(x: torch.Tensor, logits: torch.Tensor, correction: Optional[torch.Tensor], gate: torch.Tensor, up: torch.Tensor, down: torch.Tensor, limit: float, top: int) -> MoEOutput:
+    """moe_route and moe_experts; a single token's routing goes with its gate and up product."""
+    n_experts, ff, width = gate.shape
+    tokens, n_out = logits.shape
+    tile = moe_tile_pairs(x.dtype, tokens, top, n_experts, width, ff)
+    if tokens != 1 or not tile or (correction is not None and correction.dtype != x.dtype):
+        expert, weight, pairs, tiles = moe_route(logits, correction, n_experts, top, tile)
+        return MoEOutput(moe_experts(x, gate, up, down, limit, expert, pairs, tiles, tile), x, expert, weight, n_experts)
+    _expert_operands(x, gate, up, down, tokens)
+    _operand(logits, "logits", x, None, torch.float32)
+    _operand(correction, "correction", x, (n_out,))
+    expert, weight, pairs, tiles = _routing(tokens, top, n_experts, tile, x.device)
+    act = torch.empty((tokens * top, ff), dtype=x.dtype, device=x.device)
+    check(_lib.load().mui_moe_route_gateup(_stream(x), dtype_code(x.dtype), logits.data_ptr(), _ptr(correction), n_out - n_experts, gate.data_ptr(), up.data_ptr(),
+                                           ff * width, x.data_ptr(), float(limit), tile, expert.data_ptr(), weight.data_ptr(), pairs.data_ptr(), tiles.data_ptr(),
+                                           act.data_ptr(), n_experts, ff, width, top, tokens), "mui_moe_route_gateup")
+    return MoEOutput(_moe_down(act, down, expert, pairs, tiles, tile), x, expert, weight, n_experts)
 
 
 def moe_tile_pairs(dtype: torch.dtype, tokens: int, top: int, n_experts: int, width: int, ff: int) -> int:

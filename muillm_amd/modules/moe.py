@@ -47,8 +47,4 @@ class MuiMoE(MuiModule):
     def forward(self, h: torch.Tensor) -> hybrid_ops.MoEOutput:
         c = self.config
         x = h.reshape(-1, h.shape[-1])
-        tile = hybrid_ops.moe_tile_pairs(x.dtype, x.shape[0], c.top, c.experts, x.shape[1], c.ff)
-        logits = hybrid_ops.linear_f32(x, self.router)
-        expert, weight, pairs, tiles = hybrid_ops.moe_route(logits, self.correction, c.experts, c.top, tile)
-        out = hybrid_ops.moe_experts(x, self.gate_proj, self.up_proj, self.down_proj, c.limit, expert, pairs, tiles, tile)
-        return hybrid_ops.MoEOutput(out, x, expert, weight, c.experts)
+        return hybrid_ops.moe(x, hybrid_ops.linear_f32(x, self.router), self.correction, self.gate_proj, self.up_proj, self.down_proj, c.limit, c.top)

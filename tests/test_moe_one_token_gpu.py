@@ -1,0 +1,87 @@
+"""A single token's routing with its gate and up product in one launch, against the same in 64 bits: row ends, experts that are not there, sizes that the launch
+declines, ties. Gate: the roundings to 16 bits of the activation and of the result, in proportion."""
+import pytest
+import torch
+
+from muillm_amd import _lib
+from muillm_amd import hybrid_ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+ULP = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}
+
+
+def _make(experts, identity, top, width, ff, dtype, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed + width + ff + experts)
+    rand = lambda *s, std=1.0: torch.empty(s, device=DEV).normal_(0.0, std, generator=g).to(dtype)  # noqa: E731
+    return (rand(1, width), torch.empty(1, experts + identity, device=DEV).normal_(generator=g), rand(experts + identity, std=0.05),
+            rand(experts, ff, width, std=width ** -0.5), rand(experts, ff, width, std=width ** -0.5), rand(experts, width, ff, std=ff ** -0.5))
+
+
+def _reference(x, logits, corr, gate, up, down, limit, top):
+    share = torch.softmax(logits.double(), -1)[0]
+    chosen = torch.sort(share + corr.double(), descending=True, stable=True).indices[:top]
+    y = torch.zeros(x.shape[1], dtype=torch.float64, device=DEV)
+    for e in chosen.tolist():
+        if e >= gate.shape[0]:
+            y += share[e] * x[0].double()
+            continue
+        a, u = (gate[e].double() @ x[0].double()).clamp(max=limit), (up[e].double() @ x[0].double()).clamp(-limit, limit)
+        y += share[e] * (down[e].double() @ (a * torch.sigmoid(1.702 * a) * (u + 1)))
+    return chosen, share[chosen], y
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("experts,identity,top,width,ff", [
+    (64, 8, 8, 4096, 1792), (64, 8, 6, 2048, 1408), (3, 1, 4, 8, 2), (2, 6, 5, 264, 64), (200, 56, 8, 2056, 30), (16, 0, 1, 4088, 512), (5, 0, 5, 512, 2000),
+    (70, 200, 3, 256, 64), (16, 2, 9, 256, 64), (8, 1, 2, 4104, 64), (8, 0, 2, 256, 65), (8, 0, 2, 256, 72)])
+def test_against_64_bits(experts, identity, top, width, ff, dtype):
+    """The last ones but one are sizes that go the general way: 270 outputs, nine chosen, a long row, an odd number of activations."""
+    x, logits, corr, gate, up, down = _make(experts, identity, top, width, ff, dtype)
+    out = ops.moe(x, logits, corr, gate, up, down, 7.0, top)
+    chosen, share, want = _reference(x, logits, corr, gate, up, down, 7.0, top)
+    assert out.expert[0].tolist() == chosen.tolist()
+    assert float((out.weight[0].double() - share).abs().max() / share.max()) < 1e-5
+    got = out.dense()[0].double()
+    assert float((got - want).norm() / want.norm()) < ULP[dtype]
+
+
+@pytest.mark.parametrize("width,ff,once", [(2048, 1408, True), (512, 64, False)])
+def test_same_as_apart(width, ff, once):
+    """The general way gives the same choice, and the same values but for the order of sums; the down product takes the tiles as they are left."""
+    x, logits, corr, gate, up, down = _make(64, 8, 8, width, ff, torch.bfloat16)
+    assert (64 * ff * width * 4 > 32 << 20) == once
+    tile = ops.moe_tile_pairs(x.dtype, 1, 8, 64, width, ff)
+    expert, weight, pairs, tiles = ops.moe_route(logits, corr, 64, 8, tile)
+    apart = ops.MoEOutput(ops.moe_experts(x, gate, up, down, 7.0, expert, pairs, tiles, tile), x, expert, weight, 64).dense()
+    out = ops.moe(x, logits, corr, gate, up, down, 7.0, 8)
+    assert torch.equal(out.expert, expert)
+    assert float(((out.weight - weight) / weight).abs().max()) <= 72 * 2.0 ** -24  # (a sum of 72 in another order)
+    assert float((out.dense() - apart).norm() / apart.norm()) < 2 * ULP[torch.bfloat16]
+
+
+def test_ties_nothing_real_and_nan():
+    x, logits, corr, gate, up, down = _make(6, 4, 4, 64, 16, torch.bfloat16)
+    logits.fill_(1.0)
+    assert ops.moe(x, logits, None, gate, up, down, 7.0, 4).expert[0].tolist() == [0, 1, 2, 3]  # the lowest of equals
+    logits[0, :6] = -50.0
+    out = ops.moe(x, logits, None, gate, up, down, 7.0, 4)  # identity experts only
+    assert out.expert[0].tolist() == [6, 7, 8, 9]
+    assert float((out.dense() - x.float()).abs().max()) < 1e-5
+    logits.fill_(float("nan"))
+    out = ops.moe(x, logits, None, gate, up, down, 7.0, 4)
+    assert int(out.expert.max()) < 10 and int(out.expert.min()) >= 0
+    assert bool(torch.isnan(out.weight).any()) or float(out.weight.abs().max()) == 0.0
+    torch.cuda.synchronize()
+
+
+def test_refused():
+    lib = _lib.load()
+    x, logits, corr, gate, up, down = _make(4, 0, 2, 64, 16, torch.bfloat16)
+    args = [torch.empty(64, dtype=torch.int32, device=DEV).data_ptr() for _ in range(4)]
+    act = torch.empty(2, 16, dtype=torch.bfloat16, device=DEV)
+    for top, n_identity in ((5, 0), (0, 0), (2, -1)):
+        assert lib.mui_moe_route_gateup(None, 1, logits.data_ptr(), None, n_identity, gate.data_ptr(), up.data_ptr(), 16 * 64, x.data_ptr(), 7.0, 16, *args, act.data_ptr(),
+                                        4, 16, 64, top, 1) == -1
+    with pytest.raises(RuntimeError):
+        ops.moe(x, logits, corr, gate, up[:2], down, 7.0, 2)
