@@ -69,9 +69,10 @@ struct DeltaRow {  // one batch row
   const S* ring;
   long p0, start;  // slot of token 0, first slot of the row
   int ring0;       // ring row of token 0
-  __device__ __forceinline__ DeltaRow(const DeltaParams& p, int b)
-      : proj((const S*)p.proj + (long)b * p.t * p.pitch), ring((const S*)p.ring + (long)b * p.ring_rows * p.channels),
-        p0(p.cache_position[0]), start(p.row_start ? p.row_start[b] : 0), ring0((int)((uint32_t)p0 % (uint32_t)p.ring_rows)) {}
+  __device__ __forceinline__ DeltaRow(const DeltaParams& p, int b) : DeltaRow(p, b, p.cache_position[0], p.row_start ? p.row_start[b] : 0) {}
+  __device__ __forceinline__ DeltaRow(const DeltaParams& p, int b, long first_slot, long row_start)
+      : proj((const S*)p.proj + (long)b * p.t * p.pitch), ring((const S*)p.ring + (long)b * p.ring_rows * p.channels), p0(first_slot), start(row_start),
+        ring0((int)((uint32_t)p0 % (uint32_t)p.ring_rows)) {}
   // ring row of token tok, -ring_rows <= tok < 0
   __device__ __forceinline__ int ring_row(const DeltaParams& p, int tok) const { return ring0 + tok + (ring0 + tok < 0 ? p.ring_rows : 0); }
   __device__ __forceinline__ bool live(int tok) const { return p0 + tok >= start; }
@@ -88,22 +89,28 @@ struct DeltaRow {  // one batch row
     for (int j = p.taps - 1; j >= 0; --j) a = fmaf(T::one(w[p.taps - 1 - j]), raw(p, tok - j, col, c), a);
     return silu(a);
   }
-  // the same for up to four taps, all operands requested at once (taps that are not there, or inputs in front of the
-  // sequence, read something valid and count as zero)
-  __device__ __forceinline__ float conv4(const DeltaParams& p, int tok, int col, int c) const {
+  // the same for up to four taps: all operands requested at once (taps that are not there, or inputs in front of the
+  // sequence, read something valid and count as zero), ..
+  struct Taps { S x[4], f[4]; };
+  // channel c + lane, column col + lane (col, c: the same for all lanes)
+  __device__ __forceinline__ Taps taps4(const DeltaParams& p, int tok, int col, int c, unsigned lane) const {
     const S* w = (const S*)p.conv + (long)c * p.taps;
-    float x[4], a = 0.f;
-    S f[4];
+    Taps in;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const S* src = tok >= j ? proj + (long)(tok - j) * p.pitch + col : ring + (long)ring_row(p, tok - j) * p.channels + c;
-      x[j] = T::one(*src);
-      f[j] = w[j < p.taps ? p.taps - 1 - j : 0];
+      in.x[j] = src[lane];
+      in.f[j] = w[lane * (unsigned)p.taps + (unsigned)(j < p.taps ? p.taps - 1 - j : 0)];
     }
+    return in;
+  }
+  // .. and used
+  __device__ __forceinline__ float conv4(const DeltaParams& p, int tok, const Taps& in) const {
+    float a = 0.f;
 #pragma unroll
     for (int j = 3; j >= 0; --j) {
       const bool on = j < p.taps && p0 + tok - j >= (start > 0 ? start : 0);
-      a = on ? fmaf(T::one(f[j]), x[j], a) : a;
+      a = on ? fmaf(T::one(in.f[j]), T::one(in.x[j]), a) : a;
     }
     return silu(a);
   }
@@ -217,12 +224,14 @@ struct LowRankHeld {
 };
 
 // NR > 0: NR rows of S per thread in registers, for the sizes that delta_step_held names. 0: every size, S stays in memory.
-// TWO, for more workgroups than CUs: at most 128 registers, so that a CU runs two workgroups and one's chain of barriers lies under the other's. The low-rank matrices
-// are then read where they are used (batch rows share them in L2), and addresses are formed again instead of kept. us in bf16, one per CU / two, heads of
-// 128 x 128: 320 workgroups (16 heads, 20 rows) 24.4 / 18.9, 512 27.0 / 21.7, 288 (32 heads, 9 rows) 23.9 / 18.1, 544 36.0 / 32.5, 1024 51.2 / 39.5; heads of 64 x 64, 512 17.8 / 13.0. Calls of several tokens
-// read the low-rank matrices for each of them and are faster all the same: 320 workgroups of 128 x 128, 2 / 4 / 16 tokens 36.7 / 28.1, 61.3 / 45.2, 211 / 151; 64 x 64, 272, 16 tokens 163 / 97.
-template <typename T, int NR, bool TWO = false>
-__global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 1, 8))) delta_step_kernel(const DeltaParams p, int cgp) {
+// TWO, for more workgroups than CUs: at most 128 registers, so that a CU runs two workgroups and one's chain of barriers lies under the other's. Where there is no room for
+// them (of one token with four rows of S they are no gain) the low-rank matrices are read where they are used (batch rows share them in L2), and addresses are formed again instead of kept. Calls of several tokens
+// read the low-rank matrices for each of them and are faster all the same, us in bf16, one per CU / two: 320 workgroups of 128 x 128, 2 / 4 / 16 tokens 36.7 / 28.1, 61.3 / 45.2, 211 / 151; 64 x 64, 272, 16 tokens 163 / 97.
+// ONE: calls of one token. It is bound by a chain of loads and barriers and by what a CU takes in (S and the low-rank matrices of a workgroup are 128 KB, 2.6 us), which
+// lie one under the other only if the inputs are asked for before S. us as captured, S first / inputs first, heads of 128 x 128: 16 / 32 workgroups 13.1 / 10.7, 14.0 / 11.6, 256 19.4 / 16.9,
+// 288 24.6 / 19.8, 320 (16 heads, 20 rows) 24.8 / 19.7, 512 28.6 / 22.8, 1024 49.5 / 37.7; 64 x 64, 32 10.9 / 9.5, 320 14.0 / 11.7; 96 x 80, 640 33.5 / 24.2.
+template <typename T, int NR, bool TWO = false, bool ONE = false>
+__global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(TWO ? 4 : 1, 8))) delta_step_kernel(const int64_t* cache_position, const int64_t* row_start, const DeltaParams p, int cgp) {
   typedef typename T::storage S;
   __shared__ float red[8][4];
   int t = threadIdx.x;
@@ -236,11 +245,10 @@ __global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_
   float* gs = ks + dkp;         // dkp: first the decays' biases, then the decays
   float* vs = gs + dkp;         // cols; later u
   float* og = vs + cols;        // dv: gain, then gain times output gate
-  float* gz = og + p.dv;        // dv: output gate before its sigmoid
-  float* av = gz + p.dv;        // ra
+  float* av = og + p.dv;        // ra
   float* gv = av + p.ra;        // rg
-  float* part = gv + p.rg + ((4 - ((3 * dkp + 2 * p.dv + p.ra + p.rg) & 3)) & 3);  // [2][parts][cols]
-  const DeltaRow<T> row(p, b);
+  float* part = gv + p.rg + ((4 - ((3 * dkp + p.dv + p.ra + p.rg) & 3)) & 3);  // [2][parts][cols]
+  const DeltaRow<T> row(p, b, cache_position[0], row_start ? row_start[b] : 0);
   const int cg = t & (cgp - 1), rg = t / cgp, RG = kStepThreads / cgp, c0 = cg * 4;
   float* st = p.s + ((long)b * p.heads + h) * p.dk * p.dv;
   const float neg_a = -expf(T::one(((const S*)p.a_log)[h]));
@@ -270,23 +278,55 @@ __global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_
     }
   };
   const S *a2 = (const S*)p.a2 + (long)h * p.dk * p.ra, *g2 = (const S*)p.g2 + (long)h * p.dv * p.rg;
+  // A token's inputs, a channel of q, k and v per thread. Those of a call's only token are requested in front of the state and the low-rank matrices: a CU answers in the order of
+  // the requests, and the chain of sums up to the decays then runs while those, 128 KB, arrive.
+  struct Inputs { typename DeltaRow<T>::Taps q, k, v; S bias, gain, a, g, b; } in;
+  auto request = [&](int tok) {
+    Inputs r;
+    const S* pr = row.proj + (long)tok * p.pitch;
+    const unsigned from_end = kStepThreads - 1 - t;  // (v, the gate and the gain from the other end)
+    const unsigned d = t < p.dk ? t : p.dk - 1, e = (int)from_end < p.dv ? from_end : p.dv - 1;
+    const int cq = kvh * p.dk, cv = h * p.dv;
+    r.q = row.taps4(p, tok, p.q_off + cq, cq, d);
+    r.k = row.taps4(p, tok, p.k_off + cq, nq + cq, d);
+    r.v = row.taps4(p, tok, p.v_off + cv, 2 * nq + cv, e);
+    r.bias = ((const S*)p.dt_bias + h * p.dk)[d];
+    r.gain = ((const S*)p.gain)[e];
+    r.a = (pr + p.a_off)[t < p.ra ? (unsigned)t : 0u];
+    r.g = (pr + p.g_off)[(int)from_end < p.rg ? from_end : 0u];
+    r.b = pr[p.b_off + h];
+    return r;
+  };
   LowRankHeld<T> held_a, held_g;
-  if constexpr (NR > 0 && !TWO) {
+  if constexpr (ONE) {
+    in = request(0);
+    asm volatile("" ::: "memory");
+  }
+  constexpr bool HOLD = NR > 0 && (!TWO || (ONE && NR == 8));  // the low-rank matrices in registers
+  if constexpr (HOLD) {
     held_a.load(t, a2, p.dk, p.ra);
     held_g.load(t, g2, p.dv, p.rg);
   }
   if constexpr (NR > 0) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) sreg[i] = load_s(rg + RG * i);
+    if constexpr (ONE) asm volatile("" ::: "memory");
   }
-  auto conv = [&](int tok, int col, int c) {
-    if constexpr (NR > 0) return row.conv4(p, tok, col, c);
-    else return row.conv(p, tok, col, c);
-  };
+  if constexpr (ONE) {  // the inputs into the ring, as keep_inputs does it
+    if (p.taps > 1) {
+      const int e = kStepThreads - 1 - t;
+      S* ring = (S*)p.ring + ((long)b * p.ring_rows + row.ring0) * p.channels;
+      if (h % share == 0 && t < p.dk) {
+        ring[kvh * p.dk + t] = in.q.x[0];
+        ring[nq + kvh * p.dk + t] = in.k.x[0];
+      }
+      if (e < p.dv) ring[2 * nq + h * p.dv + e] = in.v.x[0];
+    }
+  }
   for (int i = p.dk + t; i < dkp; i += kStepThreads) qs[i] = ks[i] = gs[i] = 0.f;
   for (int i = p.dv + t; i < cols; i += kStepThreads) vs[i] = 0.f;
-  for (int tok = 0; tok < p.t; ++tok) {
-    asm volatile("" : "+v"(t));  // (one token is the rule: addresses kept from token to token would only cost registers)
+  for (int tok = 0; tok < (ONE ? 1 : p.t); ++tok) {
+    if constexpr (!ONE) asm volatile("" : "+v"(t));  // (addresses kept from token to token would only cost registers)
     int r0 = rg;
     if constexpr (TWO) asm volatile("" : "+v"(r0));
     S* yrow = (S*)p.y + (((long)b * p.t + tok) * p.heads + h) * p.dv;
@@ -296,25 +336,40 @@ __global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_
     }
     const S* pr = row.proj + (long)tok * p.pitch;
     // inputs of the recurrence
-    float qq = 0.f, kk = 0.f, qk = 0.f;
-    for (int d = t; d < p.dk; d += kStepThreads) {
-      const int c = kvh * p.dk + d;
-      const float x = conv(tok, p.q_off + c, c), y = conv(tok, p.k_off + c, nq + c);
+    float qq = 0.f, kk = 0.f, qk = 0.f, beta;
+    auto channel = [&](int d, float x, float y, S bias) {
       qs[d] = x;
       ks[d] = y;
-      gs[d] = T::one(((const S*)p.dt_bias)[h * p.dk + d]);
+      gs[d] = T::one(bias);
       qq = fmaf(x, x, qq);
       kk = fmaf(y, y, kk);
       qk = fmaf(x, y, qk);
+    };
+    if constexpr (NR > 0) {  // (no more than a channel per thread: launch_delta_step)
+      if constexpr (!ONE) in = request(tok);
+      if (t < p.dk) channel(t, row.conv4(p, tok, in.q), row.conv4(p, tok, in.k), in.bias);
+      const int e = kStepThreads - 1 - t;
+      if (e < p.dv) {
+        vs[e] = row.conv4(p, tok, in.v);
+        og[e] = T::one(in.gain);
+      }
+      if (t < p.ra) av[t] = T::one(in.a);
+      if (e < p.rg) gv[e] = T::one(in.g);
+      beta = sigm(T::one(in.b));
+    } else {
+      for (int d = t; d < p.dk; d += kStepThreads) {
+        const int c = kvh * p.dk + d;
+        channel(d, row.conv(p, tok, p.q_off + c, c), row.conv(p, tok, p.k_off + c, nq + c), ((const S*)p.dt_bias)[h * p.dk + d]);
+      }
+      for (int e = kStepThreads - 1 - t; e < p.dv; e += kStepThreads) {  // (from the other end: dk threads are busy above)
+        const int c = h * p.dv + e;
+        vs[e] = row.conv(p, tok, p.v_off + c, 2 * nq + c);
+        og[e] = T::one(((const S*)p.gain)[e]);
+      }
+      for (int i = t; i < p.ra; i += kStepThreads) av[i] = T::one(pr[p.a_off + i]);
+      for (int i = kStepThreads - 1 - t; i < p.rg; i += kStepThreads) gv[i] = T::one(pr[p.g_off + i]);
+      beta = sigm(T::one(pr[p.b_off + h]));
     }
-    for (int e = kStepThreads - 1 - t; e < p.dv; e += kStepThreads) {  // (from the other end: dk threads are busy above)
-      const int c = h * p.dv + e;
-      vs[e] = conv(tok, p.v_off + c, 2 * nq + c);
-      og[e] = T::one(((const S*)p.gain)[e]);
-    }
-    for (int i = t; i < p.ra; i += kStepThreads) av[i] = T::one(pr[p.a_off + i]);
-    for (int i = kStepThreads - 1 - t; i < p.rg; i += kStepThreads) gv[i] = T::one(pr[p.g_off + i]);
-    const float beta = sigm(T::one(pr[p.b_off + h]));
     qq = wave_sum(qq);
     kk = wave_sum(kk);
     qk = wave_sum(qk);
@@ -324,9 +379,9 @@ __global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_
       red[wave][2] = qk;
     }
     __syncthreads();
-    auto decay = [&](int d, float z) { gs[d] += z; };
-    auto open = [&](int e, float z) { gz[e] = z; };
-    if constexpr (NR > 0 && !TWO) {
+    auto decay = [&](int d, float z) { gs[d] = decay_of(neg_a, gs[d] + z); };
+    auto open = [&](int e, float z) { og[e] *= sigm(z); };
+    if constexpr (HOLD) {
       held_a.run(t, av, p.ra, decay);
       held_g.run(t, gv, p.rg, open);
     } else {
@@ -341,9 +396,6 @@ __global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_
       qk += red[w][2];
     }
     const float rq = p.q_scale / sqrtf(qq + kUnitEps), rk = 1.f / sqrtf(kk + kUnitEps);
-    __syncthreads();
-    for (int d = t; d < p.dk; d += kStepThreads) gs[d] = decay_of(neg_a, gs[d]);
-    for (int e = kStepThreads - 1 - t; e < p.dv; e += kStepThreads) og[e] *= sigm(gz[e]);
     __syncthreads();
     // decayed S against k and q
     f32x4 pk = {0.f, 0.f, 0.f, 0.f}, pq = pk;
@@ -431,7 +483,7 @@ __global__ void __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_
 #pragma unroll
     for (int i = 0; i < NR; ++i) store_s(r0 + RG * i, sreg[i]);
   }
-  keep_inputs<T>(p, b, h, t, kStepThreads);
+  if constexpr (!ONE) keep_inputs<T>(p, b, h, t, kStepThreads);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1161,7 +1213,8 @@ static int delta_dkp(int dk) { return dk <= 64 ? 64 : (dk <= 128 ? 128 : 256); }
 // sizes whose operands the step kernel may keep in registers
 static bool delta_step_held(const DeltaParams& p) {
   auto fits = [](int rows, int r) { return r % 8 == 0 && ceil_div(rows, 64) * ceil_div(r, 64) <= kLowRankHeld; };
-  return p.vec && p.dv % 4 == 0 && p.taps <= 4 && fits(p.dk, p.ra) && fits(p.dv, p.rg);
+  // (a channel and a low-rank input per thread at most)
+  return p.vec && p.dv % 4 == 0 && p.taps <= 4 && p.dk <= kStepThreads && p.dv <= kStepThreads && p.ra <= kStepThreads && p.rg <= kStepThreads && fits(p.dk, p.ra) && fits(p.dv, p.rg);
 }
 
 template <typename T>
@@ -1173,18 +1226,24 @@ static int launch_delta_step(hipStream_t s, const DeltaParams& p) {
   const dim3 grid(p.heads, p.batch), block(kStepThreads);
   auto launch = [&](auto kernel, int nr) {
     const size_t dkp = nr > 0 ? (size_t)nr * (kStepThreads / cgp) : p.dk;
-    const size_t lds = (3 * dkp + 4 * cgp + 2 * p.dv + p.ra + p.rg + 4 + (size_t)2 * parts * 4 * cgp) * 4;
+    const size_t lds = (3 * dkp + 4 * cgp + p.dv + p.ra + p.rg + 4 + (size_t)2 * parts * 4 * cgp) * 4;
     if (lds > 160 * 1024) return (int)MUI_ERR_UNSUPPORTED;
     if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return (int)MUI_ERR_LAUNCH;
-    hipLaunchKernelGGL(kernel, grid, block, lds, s, p, cgp);
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, p.cache_position, p.row_start, p, cgp);
     return launch_status();
   };
   if constexpr (T::kDtype != MUI_DTYPE_F32) {
     if (delta_step_held(p)) {
-      const bool two = (long)p.heads * p.batch > device_cus();  // (up to there a workgroup has its CU to itself: 256 of 128 x 128 14.6 us)
-      if (rows <= 4) return two ? launch(delta_step_kernel<T, 4, true>, 4) : launch(delta_step_kernel<T, 4>, 4);
-      if (rows <= 8) return two ? launch(delta_step_kernel<T, 8, true>, 8) : launch(delta_step_kernel<T, 8>, 8);
+      const bool two = (long)p.heads * p.batch > device_cus();  // (up to there a workgroup has its CU to itself)
+      auto held = [&](auto nr) {
+        constexpr int NR = decltype(nr)::value;
+        if (p.t > 1) return two ? launch(delta_step_kernel<T, NR, true>, NR) : launch(delta_step_kernel<T, NR>, NR);
+        if constexpr (NR == 8) return launch(delta_step_kernel<T, NR, true, true>, NR);  // (128 registers either way)
+        else return two ? launch(delta_step_kernel<T, NR, true, true>, NR) : launch(delta_step_kernel<T, NR, false, true>, NR);
+      };
+      if (rows <= 4) return held(std::integral_constant<int, 4>());
+      if (rows <= 8) return held(std::integral_constant<int, 8>());
       if (rows <= 16) return launch(delta_step_kernel<T, 16>, 16);
     }
   }
