@@ -600,7 +600,7 @@ __global__ void __launch_bounds__(64 * NWR * NWT, NWR * NWT == 4 ? 2 : 1) moe_ti
   const MoeTile tile = p.tiles[1 + ti];
   const int o0 = (in_sup / SUP) * OUT;
 
-  const int t = threadIdx.x, lane = t & (kWave - 1), wave = t >> 6;
+  const int t = threadIdx.x, lane = t & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wr = wave / NWT, wt = wave % NWT;
   if (t < PAIRS) prow[t] = p.pairs[tile.first + (t < tile.count ? t : 0)];
   __syncthreads();
@@ -632,13 +632,27 @@ __global__ void __launch_bounds__(64 * NWR * NWT, NWR * NWT == 4 ? 2 : 1) moe_ti
     xsrc[q] = p.x + (long)(EPI == MOE_GATEUP ? pr / p.top : pr) * p.k + chunk;
   }
   const int steps = (p.k + kMgK - 1) / kMgK;
+  // Tiles start at different k-steps, those of an expert's rows at the same: rows are whole multiples of the memory channels' interleave apart, and tiles that walk K in step ask
+  // the same channels. Pairs that are not there are not loaded. Weights that no other tile reads, in this call and the next, are requested non-temporally, of gate and up where the tile
+  // is a few pairs. us in bf16, 64 experts, before / now, 1408 x 2048, 6 per token, 130 / 400 / 732 /
+  // 1100 tokens gate and up 152 / 114, 165 / 127, 169 / 141, 177 / 150, down 68 / 60, 74 / 65, 82 / 72, 90 / 81; 1792 x 4096, 8 per token, 120 / 300 / 600 346 / 297, 344 / 312, 358 / 352 and 164 / 150,
+  // 175 / 168, 197 / 190; 16 of 1024 x 2048, 4 per token, 200 tokens 37 / 35, 20 / 18. (From 400 tokens of 1408 x 2048 on, 141 us at 732, gate and up are slower non-temporally, 144. A third stage of weights, or
+  // weights of two steps requested together, changes nothing.)
+  const int turn = DMA ? (int)((unsigned)(in_sup / SUP + 8 * tile.expert) % (unsigned)steps) : 0;
+  const bool alone = p.once && (ti == 0 || p.tiles[ti].expert != tile.expert) && (ti + 1 >= n_tiles || p.tiles[ti + 2].expert != tile.expert) &&
+                     (EPI == MOE_DOWN || tile.count <= 32);
   auto dma = [&](int s, int buf) {
+    s = s + turn < steps ? s + turn : s + turn - steps;
+    if (alone) {
 #pragma unroll
-    for (int q = 0; q < WQ; ++q)
-      load_lds16(wsrc[q] + s * kMgK, &w_lds[buf][(q * NW + wave) * 8 * kMgK]);
+      for (int q = 0; q < WQ; ++q) load_lds16_stream(wsrc[q] + s * kMgK, &w_lds[buf][(q * NW + wave) * 8 * kMgK]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < WQ; ++q) load_lds16(wsrc[q] + s * kMgK, &w_lds[buf][(q * NW + wave) * 8 * kMgK]);
+    }
 #pragma unroll
     for (int q = 0; q < XQ; ++q)
-      load_lds16(xsrc[q] + s * kMgK, &x_lds[buf][(q * NW + wave) * 8 * kMgK]);
+      if ((q * NW + wave) * 8 < tile.count) load_lds16(xsrc[q] + s * kMgK, &x_lds[buf][(q * NW + wave) * 8 * kMgK]);
   };
   u32x4 rw[WQ], rx[XQ];
   auto fetch = [&](int s) {
@@ -679,17 +693,19 @@ __global__ void __launch_bounds__(64 * NWR * NWT, NWR * NWT == 4 ? 2 : 1) moe_ti
       if constexpr (DMA) dma(s + 1, buf ^ 1);
       else fetch(s + 1);
     }
+    if (wt * 64 < tile.count) {  // (a wave whose pairs are not there only loads)
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      u32x4 a[4], b[4];
+      for (int kk = 0; kk < 2; ++kk) {
+        u32x4 a[4], b[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = *(const u32x4*)&x_lds[buf][b_base + j * 16 * kMgK + (((kk * 4 + lg) ^ lsw) * 8)];
+        for (int j = 0; j < 4; ++j) b[j] = *(const u32x4*)&x_lds[buf][b_base + j * 16 * kMgK + (((kk * 4 + lg) ^ lsw) * 8)];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = *(const u32x4*)&w_lds[buf][a_base + i * 16 * kMgK + (((kk * 4 + lg) ^ lsw) * 8)];
+        for (int i = 0; i < 4; ++i) a[i] = *(const u32x4*)&w_lds[buf][a_base + i * 16 * kMgK + (((kk * 4 + lg) ^ lsw) * 8)];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mfma16x16x32<T>(a[i], b[j], acc[i][j]);
+          for (int j = 0; j < 4; ++j) acc[i][j] = mfma16x16x32<T>(a[i], b[j], acc[i][j]);
+      }
     }
     if constexpr (!DMA) {
       if (more) put(buf ^ 1);
