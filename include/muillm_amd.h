@@ -598,6 +598,18 @@ int mui_moe_residual_norm(mui_stream_t stream, int dtype, const float* residual_
                           int top, const void* post_gain, float branch_scale, const void* next_gain,
                           float next_scale, float epsilon, float* residual_out, void* h, int rows, int k);
 
+/* mui_residual_norm (y_scale 1) and the product that reads its h, in one call; 16-bit types: mui_linear_ws (no norm of its own), mui_gateup_silu_bias, mui_linear_f32, whose
+ * contracts hold. h is always written. Of a single token (k_in <= 4096, or 8192 and at most 256 outputs for mui_joined_linear_f32; residual_out another buffer than residual_in) one launch;
+ * the bits are those of the two calls. */
+int mui_joined_linear(mui_stream_t stream, int dtype, const float* residual_in, const void* y, const void* post_gain, float branch_scale, const void* next_gain,
+                      float next_scale, float epsilon, float* residual_out, void* h, const void* weights, long w_pitch, const void* add_bias, void* out, int n_out, int k_in,
+                      int tokens, void* workspace, size_t workspace_bytes);
+int mui_joined_gateup_silu(mui_stream_t stream, int dtype, const float* residual_in, const void* y, const void* post_gain, float branch_scale, const void* next_gain,
+                           float next_scale, float epsilon, float* residual_out, void* h, const void* gate, const void* up, long gu_pitch, const void* gate_bias,
+                           const void* up_bias, void* out, int n_inter, int k_in, int tokens);
+int mui_joined_linear_f32(mui_stream_t stream, int dtype, const float* residual_in, const void* y, const void* post_gain, float branch_scale, const void* next_gain,
+                          float next_scale, float epsilon, float* residual_out, void* h, const void* weights, const void* bias, float* out, int n_out, int k_in, int tokens);
+
 /* y = W x (+ add_bias) and mui_residual_norm of it (y_scale 1), in one call; 16-bit types. workspace as for mui_linear_ws. Where K is divided
  * between workgroups and a launch adds up (a workspace given, at most 8192 outputs, h given) that launch joins them, too. */
 int mui_linear_residual_norm(mui_stream_t stream, int dtype, const void* weights, long w_pitch, const void* x, const void* add_bias,

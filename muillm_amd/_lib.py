@@ -109,6 +109,9 @@ _SIGNATURES = {
     "mui_decoder_stack_prompt_rows": (c_int, [_P, _P, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_long, _P, c_int, _P, c_long, _P, _P, ctypes.c_size_t]),
     "mui_decoder_stack_step": (c_int, [_P, _P, c_int, _P, _P, _P, c_long, _P, c_int, _P, c_long, c_int, _P]),
     "mui_residual_norm": (c_int, [_P, c_int, _P, _P, c_float, _P, c_float, _P, c_float, c_float, _P, _P, c_int, c_int]),
+    "mui_joined_linear": (c_int, [_P, c_int, _P, _P, _P, c_float, _P, c_float, c_float, _P, _P] + [_P, c_long, _P, _P, c_int, c_int, c_int, _P, ctypes.c_size_t]),
+    "mui_joined_gateup_silu": (c_int, [_P, c_int, _P, _P, _P, c_float, _P, c_float, c_float, _P, _P] + [_P, _P, c_long, _P, _P, _P, c_int, c_int, c_int]),
+    "mui_joined_linear_f32": (c_int, [_P, c_int, _P, _P, _P, c_float, _P, c_float, c_float, _P, _P] + [_P, _P, _P, c_int, c_int, c_int]),
     "mui_linear_residual_norm": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_float, _P, c_float, c_float, _P, _P, _P, c_int, c_int,
                                          c_int, _P, ctypes.c_size_t]),
     "mui_moe_residual_norm": (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int, c_int, _P, c_float, _P, c_float, c_float, _P, _P,

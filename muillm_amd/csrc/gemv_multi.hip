@@ -8,6 +8,8 @@
 //
 // The reference has no kernel for this case (csrc/modules/linear_module.cpp:57-79 falls back to
 // RMSNorm + torch matmul + add; muillm/modules/gateupdownmlp.py:343-359).
+#include <type_traits>
+
 #include "skinny.cuh"
 
 namespace mui {
@@ -27,15 +29,22 @@ __device__ __forceinline__ float dot2_mt<BF16>(uint32_t a, uint32_t b, float c) 
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_mt, a), __builtin_bit_cast(bf16x2_mt, b), c, false);
 }
 
+// JOIN (one token, no norm of the linear's own): what is multiplied is the boundary in front, which every workgroup computes for itself while its first weights are
+// on their way: stream + branch_scale * post_gain * rms(x), and of that next_scale * next_gain * rms(..), x being the sublayer's output; the values and the order of
+// sums are residual_norm.hip's, bit for bit. Workgroup 0 writes the stream and the product's input down. What it saves is the launch of one workgroup in front,
+// 3 to 4 us of which half is its start: us of both in bf16 as captured, apart / here: gate and up 14336 x 4096 40.9 / 37.9, 8192 x 2048 15.3 / 13.3;
+// linears 12576 x 4096 21.4 / 19.8, 6272 x 2048 8.6 / 7.1, 2112 x 4096 (both norms) 8.1 / 6.7; a router of 72 x 4096 (moe.hip) 5.3 / 3.1.
 // TWO (one token, work lists of several row groups per workgroup -- the lm_head): two register
 // sets; the weights of group i + 2 are requested as soon as group i has been multiplied, so a
 // workgroup always has a whole group in flight while it reduces, synchronises and stores.
-template <typename T, int R, int CH, bool NORM, int EPI, int TOK, bool TWO = false>
+struct NoJoin {};
+template <typename T, int R, int CH, bool NORM, int EPI, int TOK, bool TWO = false, bool JOIN = false>
 __global__ void __launch_bounds__(kMtThreads) gemv_multi_kernel(
     // scalars, hottest first (preloaded into SGPRs at wave launch)
     const uint16_t* w0, const uint16_t* w1, long pitch, const uint16_t* x, const uint16_t* gamma,
     uint16_t* y, int n, int k, int tokens, int x_pitch, float eps, const uint16_t* residual,
-    const uint16_t* mul_bias, const uint16_t* add_bias) {
+    const uint16_t* mul_bias, const uint16_t* add_bias, const std::conditional_t<JOIN, BoundaryInFront, NoJoin> front) {
+  static_assert(!JOIN || (TOK == 1 && !NORM), "a boundary in front: one token, no other norm");
   constexpr int OUT = (EPI == SK_GATEUP) ? R / 2 : R;
   static_assert(EPI != SK_GATEUP || (R % 2 == 0), "gate/up needs row pairs");
   static_assert(16 * OUT * TOK <= kMtThreads, "sixteen epilogue lanes per output");
@@ -124,6 +133,8 @@ __global__ void __launch_bounds__(kMtThreads) gemv_multi_kernel(
 #pragma unroll
     for (int j = 0; j < CH; ++j) gq[j] = ld16(gamma + coff[j]);
   }
+  FrontOperands<T, JOIN ? CH : 1> ahead;
+  if constexpr (JOIN) ahead.request(front, x, coff);
   issue_w(sets[0], rg);
   issue_res(sets[0], rg);
   // group i of this workgroup is blockIdx.x + i * gridDim.x
@@ -135,10 +146,15 @@ __global__ void __launch_bounds__(kMtThreads) gemv_multi_kernel(
     issue_res(sets[1], group_of(n_my > 1 ? 1 : 0));
   }
 
+  if constexpr (JOIN) {
+    __shared__ float red_join[2][kMtWaves];
+    ahead.finish(front, xq[0], cvalid, coff, k, eps, red_join, blockIdx.x == 0);
+  }
   float ss[TOK];
 #pragma unroll
   for (int tk = 0; tk < TOK; ++tk) {
     ss[tk] = 0.f;
+    if constexpr (JOIN) continue;
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const bool live = cvalid[j] && tk < tokens;
@@ -323,7 +339,7 @@ static int launch_mt_rc(hipStream_t s, const SkinnyParams& p, int grid) {
 #define MUI_MT_LAUNCH(NORMV, TWOV)                                                                              \
   hipLaunchKernelGGL((gemv_multi_kernel<T, R, CH, NORMV, EPI, TOK, TWOV>), dim3(grid), dim3(kMtThreads), 0, s,  \
                      (const uint16_t*)p.w0, (const uint16_t*)p.w1, p.pitch, p.x, p.gamma, p.y, p.n, p.k,        \
-                     p.tokens, (int)(p.x_pitch > 0 ? p.x_pitch : (long)p.k), p.eps, p.residual, p.mul_bias, p.add_bias)
+                     p.tokens, (int)(p.x_pitch > 0 ? p.x_pitch : (long)p.k), p.eps, p.residual, p.mul_bias, p.add_bias, NoJoin{})
   if constexpr (TOK == 1 && CH <= 2 && EPI == SK_LINEAR) {
     constexpr int OUT = R;
     if (g_mt_two_min_passes > 0 && ceil_div(p.n, OUT) >= (long)g_mt_two_min_passes * grid) {
@@ -369,6 +385,34 @@ static int launch_mt_t(hipStream_t s, const SkinnyParams& p) {
   if (ch <= 7) return launch_mt_rc<T, R, 7, EPI, TOK>(s, p, grid);
   return MUI_ERR_UNSUPPORTED;
   }
+}
+
+template <typename T, int EPI, int CH>
+static int launch_mt_join(hipStream_t s, const SkinnyParams& p, const BoundaryInFront& front) {
+  constexpr int R = 4, OUT = (EPI == SK_GATEUP) ? 2 : 4;
+  const int tuned = gemv_tuned_wgs_per_cu(), groups = ceil_div(p.n, OUT), grid = balanced_grid(groups, tuned > 0 ? tuned : 3);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kMtThreads), 0, s, (const uint16_t*)p.w0, (const uint16_t*)p.w1, p.pitch, p.x, (const uint16_t*)nullptr, p.y, p.n, p.k, 1,
+                       p.k, p.eps, (const uint16_t*)nullptr, p.mul_bias, p.add_bias, front);
+    return launch_status();
+  };
+  if constexpr (EPI == SK_LINEAR) {
+    if (g_mt_two_min_passes > 0 && groups >= (long)g_mt_two_min_passes * grid) return launch(gemv_multi_kernel<T, R, CH, false, EPI, 1, true, true>);
+  }
+  return launch(gemv_multi_kernel<T, R, CH, false, EPI, 1, false, true>);
+}
+
+// One token: p.x is the sublayer's output; the kernels that the product takes without a boundary in front. MUI_ERR_UNSUPPORTED: not a case for it (nothing launched)
+int launch_gemv_join(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p, const BoundaryInFront& front) {
+  if (p.tokens != 1 || p.k > 2 * 8 * kMtThreads || p.residual || p.gamma) return MUI_ERR_UNSUPPORTED;
+  const bool one = p.k <= 8 * kMtThreads;
+  if (epilogue == SK_LINEAR) {
+    if (dtype == MUI_DTYPE_F16) return one ? launch_mt_join<F16, SK_LINEAR, 1>(s, p, front) : launch_mt_join<F16, SK_LINEAR, 2>(s, p, front);
+    if (dtype == MUI_DTYPE_BF16) return one ? launch_mt_join<BF16, SK_LINEAR, 1>(s, p, front) : launch_mt_join<BF16, SK_LINEAR, 2>(s, p, front);
+  } else if (epilogue == SK_GATEUP && dtype == MUI_DTYPE_BF16) {  // (a single token's gate and up in fp16 are another kernel's)
+    return one ? launch_mt_join<BF16, SK_GATEUP, 1>(s, p, front) : launch_mt_join<BF16, SK_GATEUP, 2>(s, p, front);
+  }
+  return MUI_ERR_UNSUPPORTED;
 }
 
 // longest row one launch covers: 7 chunks of 8 values per thread

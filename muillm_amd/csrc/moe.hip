@@ -98,6 +98,60 @@ __global__ void __launch_bounds__(256) linear_f32_rows_kernel(const typename T::
   }
 }
 
+// One token, with the boundary in front (gemv_join.hip): every row's workgroup computes that for itself; x is the sublayer's output
+template <typename T, int CH>
+__global__ void __launch_bounds__(256) linear_f32_join_kernel(const uint16_t* x, const uint16_t* w, const uint16_t* bias, float* y, int k, float eps, const BoundaryInFront front) {
+  __shared__ float red[4], red_join[2][4];
+  const int t = threadIdx.x, row = blockIdx.x;
+  int at[CH];
+  bool valid[CH];
+  u32x4 xq[CH], wq[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const int c = (t + 256 * j) * 8;
+    valid[j] = c < k;
+    at[j] = valid[j] ? c : 0;
+    xq[j] = ld16(x + at[j]);
+  }
+  FrontOperands<T, CH> ahead;
+  ahead.request(front, x, at);
+#pragma unroll
+  for (int j = 0; j < CH; ++j) wq[j] = ld16(w + (long)row * k + at[j]);
+  ahead.finish(front, xq, valid, at, k, eps, red_join, row == 0);
+  float acc = 0.f;
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    float wf[8], xf[8];
+    unpack8<T>(wq[j], wf);
+    unpack8<T>(xq[j], xf);
+    if (valid[j])
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc = fmaf(wf[i], xf[i], acc);
+  }
+  acc = wave_sum(acc);
+  if ((t & 63) == 0) red[t >> 6] = acc;
+  __syncthreads();
+  if (t == 0) y[row] = ((red[0] + red[1]) + (red[2] + red[3])) + (bias ? T::one(bias[row]) : 0.f);
+}
+
+template <typename T>
+static int launch_linear_f32_join_t(hipStream_t s, const void* w, const void* x, const void* bias, float* y, int n, int k, float eps, const BoundaryInFront& front) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y, k, eps, front);
+    return launch_status();
+  };
+  // every row repeats the boundary, 24 KB from L2 at 4096: for as many as fill the chip once
+  if (n > device_cus() || k > 4 * 256 * 8) return MUI_ERR_UNSUPPORTED;
+  if (k <= 256 * 8) return launch(linear_f32_join_kernel<T, 1>);
+  if (k <= 2 * 256 * 8) return launch(linear_f32_join_kernel<T, 2>);
+  return launch(linear_f32_join_kernel<T, 4>);
+}
+int launch_linear_f32_join(hipStream_t s, int dtype, const void* w, const void* x, const void* bias, float* y, int n, int k, float eps, const BoundaryInFront& front) {
+  if (dtype == MUI_DTYPE_F16) return launch_linear_f32_join_t<F16>(s, w, x, bias, y, n, k, eps, front);
+  if (dtype == MUI_DTYPE_BF16) return launch_linear_f32_join_t<BF16>(s, w, x, bias, y, n, k, eps, front);
+  return MUI_ERR_UNSUPPORTED;
+}
+
 // ---------------------------------------------------------------------------------------
 // routing
 // ---------------------------------------------------------------------------------------

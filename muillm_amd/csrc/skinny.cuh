@@ -221,6 +221,91 @@ int launch_skinny(hipStream_t s, int dtype, int weight_format, int epilogue, con
 void skinny_set_bstat(int on);
 void skinny_set_lt(int on);  // 0: operands loaded straight from HBM in MFMA order (older kernels)
 
+// The boundary between two sublayers (residual_norm.hip) in front of a product of one token
+struct BoundaryInFront {
+  const float* stream;
+  const uint16_t *post_gain, *next_gain;  // or null
+  float branch_scale, next_scale;
+  float* stream_out;  // not stream: other workgroups still read that
+  uint16_t* h;        // the product's input
+};
+// What a workgroup of 256 threads reads of it, thread t having values 8 (t + 256 j) .. + 7; values and order of sums are residual_norm.hip's
+template <typename T, int CH>
+struct FrontOperands {
+  f32x4 stream[CH][2];
+  u32x4 post[CH], next[CH];
+  // y: the sublayer's output (read where a gain is not there)
+  __device__ __forceinline__ void request(const BoundaryInFront& f, const uint16_t* y, const int (&at)[CH]) {
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      stream[j][0] = *(const f32x4*)(f.stream + at[j]);
+      stream[j][1] = *(const f32x4*)(f.stream + at[j] + 4);
+      post[j] = ld16((f.post_gain ? f.post_gain : y) + at[j]);
+      next[j] = ld16((f.next_gain ? f.next_gain : y) + at[j]);
+    }
+  }
+  // x: the sublayer's output on the way in, the next one's input on the way out (zeros past the end)
+  __device__ __forceinline__ void finish(const BoundaryInFront& f, u32x4 (&x)[CH], const bool (&valid)[CH], const int (&at)[CH], int k, float eps, float (&red)[2][4], bool writes) {
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    auto block_sum = [&](float v, float (&meet)[4]) {
+      v = wave_sum(v);
+      if (lane == 0) meet[wave] = v;
+      __syncthreads();
+      return (meet[0] + meet[1]) + (meet[2] + meet[3]);
+    };
+    float xs[CH][8], ys[CH][8], g[8], sq = 0.f;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      unpack8<T>(x[j], ys[j]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) xs[j][i] = stream[j][i >> 2][i & 3];
+    }
+    if (f.post_gain) {
+#pragma unroll
+      for (int j = 0; j < CH; ++j)
+        if (valid[j])
+#pragma unroll
+          for (int i = 0; i < 8; ++i) sq = fmaf(ys[j][i], ys[j][i], sq);
+      const float rs = rsqrtf(block_sum(sq, red[0]) / (float)k + eps);
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        unpack8<T>(post[j], g);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xs[j][i] = fmaf(g[i] * f.branch_scale, ys[j][i] * rs, xs[j][i]);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < CH; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xs[j][i] += ys[j][i];
+    }
+    float rs = f.next_scale;
+    if (f.next_gain) {
+      sq = 0.f;
+#pragma unroll
+      for (int j = 0; j < CH; ++j)
+        if (valid[j])
+#pragma unroll
+          for (int i = 0; i < 8; ++i) sq = fmaf(xs[j][i], xs[j][i], sq);
+      rs = rsqrtf(block_sum(sq, red[1]) / (float)k + eps) * f.next_scale;
+    }
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      unpack8<T>(next[j], g);
+      float o[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = (f.next_gain ? g[i] : 1.f) * (xs[j][i] * rs);
+      const u32x4 b = pack8<T>(o), zero = {0u, 0u, 0u, 0u};
+      if (writes && valid[j]) {
+        *(f32x4*)(f.stream_out + at[j]) = f32x4{xs[j][0], xs[j][1], xs[j][2], xs[j][3]};
+        *(f32x4*)(f.stream_out + at[j] + 4) = f32x4{xs[j][4], xs[j][5], xs[j][6], xs[j][7]};
+        *(u32x4*)(f.h + at[j]) = b;
+      }
+      x[j] = valid[j] ? b : zero;
+    }
+  }
+};
+int launch_gemv_join(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p, const BoundaryInFront& front);
 // 1..8 tokens, 16-bit weights: the single-token GEMV structure with the token operands packed
 // in registers (gemv_multi.hip); returns MUI_ERR_UNSUPPORTED for shapes it does not cover
 int launch_gemv_multi(hipStream_t s, int dtype, int epilogue, const SkinnyParams& p);

@@ -13,6 +13,7 @@ import torch
 
 from . import _lib
 from ._lib import MUI_DTYPE_BF16, MUI_DTYPE_F16, MUI_DTYPE_F32, check
+from .muillm_ext import ResidualFront
 
 _CODES = {torch.float16: MUI_DTYPE_F16, torch.bfloat16: MUI_DTYPE_BF16, torch.float32: MUI_DTYPE_F32}
 
@@ -110,8 +111,8 @@ def residual_norm(residual: Optional[torch.Tensor], y, post_gain: Optional[torch
     return out, h
 
 
-def linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """fp32 [tokens, n] = x W^T + bias for x [..., k]: outputs that stay in 32 bits (router logits, gates)."""
+def linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, front: Optional[ResidualFront] = None) -> torch.Tensor:
+    """fp32 [tokens, n] = x W^T + bias for x [..., k]: outputs that stay in 32 bits (router logits, gates). front: as muillm_linear_forward's."""
     n, k = weight.shape
     if x.shape[-1] != k:
         raise RuntimeError(f"input has {x.shape[-1]} features but the weights expect {k}")
@@ -120,6 +121,10 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     _operand(bias, "bias", x, (n,))
     tokens = x.numel() // k
     y = torch.empty((tokens, n), dtype=torch.float32, device=x.device)
+    if front is not None:
+        front.along(lambda args: check(_lib.load().mui_joined_linear_f32(_stream(x), dtype_code(x.dtype), *args, weight.data_ptr(), _ptr(bias), y.data_ptr(), n, k, tokens),
+                                       "mui_joined_linear_f32"))
+        return y
     check(_lib.load().mui_linear_f32(_stream(x), dtype_code(x.dtype), weight.data_ptr(), x.data_ptr(), _ptr(bias),
                                      y.data_ptr(), n, k, tokens), "mui_linear_f32")
     return y

@@ -47,6 +47,9 @@ class MuiHybridAttention(MuiModule):
     def takes_behind(self) -> bool:
         return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
+    def takes_front(self) -> bool:
+        return type(self.proj) is MuiMultiLinear and self.proj.linear.takes_front() and not heard(self, self.proj)
+
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiHybridAttentionConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):
         super().__init__(engine_config=engine_config)
@@ -68,10 +71,10 @@ class MuiHybridAttention(MuiModule):
     def new_state(self, batch: int, capacity: int, device, dtype) -> MuiKeyValueState:
         return MuiKeyValueState(batch, capacity, self.config.kv_heads, self.config.dim, self.config.vdim, device, dtype)
 
-    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None, front=None) -> torch.Tensor:
         """h [B, T, hidden] -> [B, T, hidden]; the tokens' rows go to slots cache_position."""
         c, state = self.config, cache.layers[self.layer_idx]
-        proj = cache.spread(self.proj.linear(h))
+        proj = cache.spread(self.proj.linear(h) if front is None else self.proj.linear(h, front=front))
         o = hybrid_ops.hybrid_step(proj, c.heads, c.kv_heads, c.dim, c.vdim, self.q_norm, self.k_norm, self.eps, self.inv_freq, cache_position,
                                    cache.row_start, state.k, state.v, c.gated, c.scale, c.softcap, c.window, c.keep_first)
         if o is None:

@@ -12,7 +12,7 @@ import torch.nn as nn
 
 from ... import hybrid_ops
 from ...engineconfig import MuiEngineConfig
-from ...muillm_ext import ResidualBehind
+from ...muillm_ext import ResidualBehind, ResidualFront
 from ..module import MuiModule
 from ..norm.rmsnorm import MuiRMSNorm
 
@@ -20,7 +20,7 @@ from ..norm.rmsnorm import MuiRMSNorm
 class MuiSandwichDecoderLayer(MuiModule):
     """mixer: a module with forward(h, cache, cache_position) and new_state(...); mlp: a module with
     forward(h), or None for a layer without feed-forward. Where the class of either has a takes_behind() that is true, its forward takes a
-    `behind` for its last linear. branch_scale: m."""
+    `behind` for its last linear, and where it has a takes_front() that is, a `front` for its first. branch_scale: m."""
 
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, mixer: MuiModule, mlp: Optional[MuiModule], eps: float,
                  device=None, dtype=None, pre_norms: bool = True, branch_scale: float = 1.0):
@@ -44,26 +44,41 @@ def run_layers(layers: List[MuiSandwichDecoderLayer], x: torch.Tensor, h: torch.
         return hybrid_ops.residual_norm(x, y, post.weight, None if following is None else following.weight, eps,
                                         branch_scale=m, next_scale=scale, emit=True)
 
-    # where it saves a launch the sublayer's last linear takes the join along
-    along = ResidualBehind.worth_it(h.numel() // h.shape[-1])
+    # where it saves a launch the sublayer's last linear takes the join along, or the next sublayer's first product
+    rows = h.numel() // h.shape[-1]
+    along = ResidualBehind.worth_it(rows)
+    ahead = rows == 1 and collect is None
 
-    def sublayer(module, args, x, post: MuiRMSNorm, m: float, following: Optional[MuiRMSNorm], scale: float = 1.0):
-        if not (along and "takes_behind" in type(module).__dict__ and module.takes_behind()):
-            return join(x, module(*args), post, m, following, scale)
-        behind = ResidualBehind(x, post.weight, m, None if following is None else following.weight, scale, eps)
-        y = module(*args, behind=behind)
-        return behind.take(y) or join(x, y, post, m, following, scale)
+    def boundary(module, args, x, post: MuiRMSNorm, m: float, following: Optional[MuiRMSNorm], scale: float = 1.0, **kw):
+        """(x, h) behind a sublayer, or what the next one takes in front of itself."""
+        if along and "takes_behind" in type(module).__dict__ and module.takes_behind():
+            behind = ResidualBehind(x, post.weight, m, None if following is None else following.weight, scale, eps)
+            y = module(*args, behind=behind)
+            return behind.take(y) or join(x, y, post, m, following, scale)
+        y = module(*args, **kw)
+        if "front" in kw:
+            x = kw["front"].joined()[0]
+        front = ResidualFront.of(x, y, post.weight, m, None if following is None else following.weight, scale, eps) if ahead else None
+        return front or join(x, y, post, m, following, scale)
 
+    def sublayer(module, rest, state, *behind):
+        if isinstance(state, ResidualFront):
+            if "takes_front" in type(module).__dict__ and module.takes_front():
+                return boundary(module, (state.y.reshape(shape),) + rest, None, *behind, front=state)
+            state = state.joined()
+        x, h = state
+        return boundary(module, (h.reshape(shape),) + rest, x, *behind)
+
+    state = x, h
     for i, layer in enumerate(layers):
         last, m = i + 1 == len(layers), layer.branch_scale
         following = (final_norm, final_scale) if last else (layers[i + 1].pre_mixer_norm,)
-        mixer = (layer.mixer, (h, cache, cache_position))
+        at = (cache, cache_position)
         if layer.mlp is None:
-            x, h = sublayer(*mixer, x, layer.post_mixer_norm, m, *following)
+            state = sublayer(layer.mixer, at, state, layer.post_mixer_norm, m, *following)
         else:
-            x, h = sublayer(*mixer, x, layer.post_mixer_norm, m, layer.pre_mlp_norm)
-            x, h = sublayer(layer.mlp, (h,), x, layer.post_mlp_norm, m, *following)
-        h = h.reshape(shape)
+            state = sublayer(layer.mixer, at, state, layer.post_mixer_norm, m, layer.pre_mlp_norm)
+            state = sublayer(layer.mlp, (), state, layer.post_mlp_norm, m, *following)
         if collect is not None:
-            collect.append(x.clone())
-    return h
+            collect.append(state[0].clone())
+    return (state.joined() if isinstance(state, ResidualFront) else state)[1].reshape(shape)

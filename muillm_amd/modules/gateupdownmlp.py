@@ -36,9 +36,9 @@ class _MuiGateUpSiLUMethod(Enum):
 class _MuiGateUpSiLU(torch.autograd.Function):
     @staticmethod
     def forward(ctx, engine, inputs, norm_weights, variance_epsilon, gate_weights, up_weights,
-                down_weights, residual, biases, behind=None):
+                down_weights, residual, biases, behind=None, front=None):
         return muillm_ext.muillm_gateupsilu_forward(
-            engine, norm_weights, variance_epsilon, gate_weights, up_weights, down_weights, residual, inputs, biases, behind)
+            engine, norm_weights, variance_epsilon, gate_weights, up_weights, down_weights, residual, inputs, biases, behind, front)
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -48,9 +48,9 @@ class _MuiGateUpSiLU(torch.autograd.Function):
 class _MuiGateUpSiLUSplit(torch.autograd.Function):
     @staticmethod
     def forward(ctx, engine, inputs, norm_weights, variance_epsilon, gate_weights, up_weights,
-                down_weights, residual, biases, behind=None):
+                down_weights, residual, biases, behind=None, front=None):
         return muillm_ext.muillm_gateupsilu_split_forward(
-            engine, norm_weights, variance_epsilon, gate_weights, up_weights, down_weights, residual, inputs, biases, behind)
+            engine, norm_weights, variance_epsilon, gate_weights, up_weights, down_weights, residual, inputs, biases, behind, front)
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -207,26 +207,30 @@ class MuiGateUpDownMLP(MuiModule):
         return (self.dispatchable and muillm_ext.kernel_dispatchable(input)
                 and isinstance(self.gate_proj, MuiLinear) and isinstance(self.up_proj, MuiLinear))
 
-    def _forward_fused(self, input: Tensor, residual: Optional[Tensor] = None, behind=None) -> Tensor:
+    def _forward_fused(self, input: Tensor, residual: Optional[Tensor] = None, behind=None, front=None) -> Tensor:
         if self._kernel_ok(input):
             return _MuiGateUpSiLU.apply(self.cpp_engine, input, self.norm_weights, self.variance_epsilon,
-                                        self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind)
-        return self._forward_unfused(input=input, residual=residual)
+                                        self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind, front)
+        return self._forward_unfused(input=input if front is None else front.joined()[1], residual=residual)
 
-    def _forward_split(self, input: Tensor, residual: Optional[Tensor] = None, behind=None) -> Tensor:
+    def _forward_split(self, input: Tensor, residual: Optional[Tensor] = None, behind=None, front=None) -> Tensor:
         if self._kernel_ok(input):
             return _MuiGateUpSiLUSplit.apply(self.cpp_engine, input, self.norm_weights, self.variance_epsilon,
-                                             self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind)
-        return self._forward_unfused(input=input, residual=residual)
+                                             self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind, front)
+        return self._forward_unfused(input=input if front is None else front.joined()[1], residual=residual)
 
     def takes_behind(self) -> bool:
         return type(self.down_proj) is MuiLinear and self.method != _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED and not heard(self)
 
-    def forward(self, input: Tensor, residual: Optional[Tensor] = None, behind: Optional[muillm_ext.ResidualBehind] = None) -> Tensor:
+    def takes_front(self) -> bool:
+        return not self.normalize and self.method != _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED and not heard(self)
+
+    def forward(self, input: Tensor, residual: Optional[Tensor] = None, behind: Optional[muillm_ext.ResidualBehind] = None,
+                front: Optional[muillm_ext.ResidualFront] = None) -> Tensor:
         if self.method == _MuiGateUpSiLUMethod.GATEUPSILU_FUSED:
-            return self._forward_fused(input=input, residual=residual, behind=behind)
+            return self._forward_fused(input=input, residual=residual, behind=behind, front=front)
         elif self.method == _MuiGateUpSiLUMethod.GATEUPSILU_UNFUSED:
-            return self._forward_unfused(input=input, residual=residual)
+            return self._forward_unfused(input=input if front is None else front.joined()[1], residual=residual)
         elif self.method == _MuiGateUpSiLUMethod.GATEUPSILU_SPLIT:
-            return self._forward_split(input=input, residual=residual, behind=behind)
+            return self._forward_split(input=input, residual=residual, behind=behind, front=front)
         raise ValueError("Unsupported Gate/Up Silu method")

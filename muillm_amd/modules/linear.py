@@ -19,7 +19,7 @@ from .._hf import LlamaRMSNorm, MistralRMSNorm
 from ..engineconfig import MuiEngineConfig
 from ..replacement.replacementcontext import MuiReplacementContext
 from ._fusion import AbsorbedNorm, fill_parameter, is_kernel_dtype, rmsnorm_reference
-from .module import MuiModule
+from .module import MuiModule, heard
 from .norm.rmsnorm import MuiRMSNorm, _MuiRMSNorm
 
 
@@ -27,8 +27,8 @@ class _MuiLinear(torch.autograd.Function):
     """The library call as an autograd node without a backward (inference only)."""
 
     @staticmethod
-    def forward(ctx, module, x, residual, behind=None):
-        return muillm_ext.muillm_linear_module_forward(module, x, residual=residual, behind=behind)
+    def forward(ctx, module, x, residual, behind=None, front=None):
+        return muillm_ext.muillm_linear_module_forward(module, x, residual=residual, behind=behind, front=front)
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -128,9 +128,15 @@ class MuiLinear(MuiModule, nn.Linear):
         self.dispatchable = is_kernel_dtype(self.weight)
 
     # ---- forward -----------------------------------------------------------------------------
-    def forward(self, input: Tensor, residual: Optional[Tensor] = None, behind: Optional[muillm_ext.ResidualBehind] = None) -> Tensor:
+    def takes_front(self) -> bool:
+        return type(self) is MuiLinear and self.cpp_module is not None and not self.normalize and not heard(self)
+
+    def forward(self, input: Tensor, residual: Optional[Tensor] = None, behind: Optional[muillm_ext.ResidualBehind] = None,
+                front: Optional[muillm_ext.ResidualFront] = None) -> Tensor:
         if self.cpp_module is not None:
-            return _MuiLinear.apply(self.cpp_module, input, residual, behind)
+            return _MuiLinear.apply(self.cpp_module, input, residual, behind, front)
+        if front is not None:
+            input = front.joined()[1]
         # before finalize_init: plain torch, with the library's norm kernel where it applies
         x = input
         if self.normalize:

@@ -10,7 +10,7 @@ import torch.nn as nn
 
 from .. import hybrid_ops
 from ..engineconfig import MuiEngineConfig
-from .module import MuiModule
+from .module import MuiModule, heard
 
 
 @dataclass
@@ -44,7 +44,13 @@ class MuiMoE(MuiModule):
         self.up_proj = weight(c.experts, c.ff, hidden)
         self.down_proj = weight(c.experts, hidden, c.ff)
 
-    def forward(self, h: torch.Tensor) -> hybrid_ops.MoEOutput:
+    def takes_front(self) -> bool:
+        return not heard(self)
+
+    def forward(self, h: torch.Tensor, front=None) -> hybrid_ops.MoEOutput:
         c = self.config
         x = h.reshape(-1, h.shape[-1])
-        return hybrid_ops.moe(x, hybrid_ops.linear_f32(x, self.router), self.correction, self.gate_proj, self.up_proj, self.down_proj, c.limit, c.top)
+        logits = hybrid_ops.linear_f32(x, self.router, front=front)
+        if front is not None:
+            x = front.joined()[1].reshape(x.shape)
+        return hybrid_ops.moe(x, logits, self.correction, self.gate_proj, self.up_proj, self.down_proj, c.limit, c.top)

@@ -43,6 +43,9 @@ class MuiChannelDelta(MuiModule):
     def takes_behind(self) -> bool:
         return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
+    def takes_front(self) -> bool:
+        return type(self.proj) is MuiMultiLinear and self.proj.linear.takes_front() and not heard(self, self.proj)
+
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiChannelDeltaConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):
         super().__init__(engine_config=engine_config)
@@ -76,8 +79,8 @@ class MuiChannelDelta(MuiModule):
         return MuiRecurrentState(torch.zeros((batch, c.heads, c.dim, c.vdim), dtype=torch.float32, device=device),
                                  torch.zeros((batch, layer.ring_rows, layer.channels), dtype=dtype, device=device))
 
-    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, cache: MuiHybridCache, cache_position: torch.Tensor, behind=None, front=None) -> torch.Tensor:
         memory, ring = cache.layers[self.layer_idx].values
-        o = hybrid_ops.channel_delta(self.layer(), cache.spread(self.proj.linear(h)), memory, ring, cache_position, cache.row_start)
+        o = hybrid_ops.channel_delta(self.layer(), cache.spread(self.proj.linear(h) if front is None else self.proj.linear(h, front=front)), memory, ring, cache_position, cache.row_start)
         o = cache.take(o)
         return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

@@ -208,6 +208,44 @@ class ResidualBehind:
         return self.result if self.of is not None and y is self.of and y._version == self._version else None
 
 
+class ResidualFront:
+    """The boundary in front of a sublayer (hybrid_ops.residual_norm) that is left to the first product of that sublayer, for single tokens: every workgroup of the product computes it
+    while its first weights are on their way. The sublayer is handed `y`, the output of the one before it, in the place of its input, and this object; whoever needs the input itself
+    asks with joined(). An object lives for one boundary of one forward pass."""
+
+    def __init__(self, stream: torch.Tensor, y: torch.Tensor, post_gain: Optional[torch.Tensor], branch_scale: float, next_gain: Optional[torch.Tensor], next_scale: float,
+                 eps: float):
+        self.stream, self.y, self.post_gain, self.next_gain = stream, y, post_gain, next_gain
+        self.branch_scale, self.next_scale, self.eps = float(branch_scale), float(next_scale), float(eps)
+        self.result = None  # (the stream behind it, the sublayer's input)
+
+    @classmethod
+    def of(cls, stream, y, post_gain, branch_scale, next_gain, next_scale, eps) -> Optional["ResidualFront"]:
+        """None where a library call in front of a product could not take it along."""
+        if torch.is_grad_enabled() or not torch.is_tensor(y) or not y.is_cuda or y.dtype not in (torch.float16, torch.bfloat16):
+            return None
+        if y.numel() != y.shape[-1] or not y.is_contiguous() or stream.dtype != torch.float32 or stream.device != y.device or stream.numel() != y.numel() or not stream.is_contiguous():
+            return None
+        for gain in (post_gain, next_gain):
+            if gain is not None and (gain.dtype != y.dtype or gain.device != y.device or gain.numel() != y.shape[-1] or not gain.is_contiguous()):
+                return None
+        return cls(stream, y, post_gain, branch_scale, next_gain, next_scale, eps)
+
+    def joined(self) -> Tuple[torch.Tensor, torch.Tensor]:
+        if self.result is None:
+            from . import hybrid_ops
+
+            stream, h = hybrid_ops.residual_norm(self.stream, self.y, self.post_gain, self.next_gain, self.eps, branch_scale=self.branch_scale, next_scale=self.next_scale, emit=True)
+            self.result = stream, h.reshape(self.y.shape)
+        return self.result
+
+    def along(self, call) -> None:
+        """call(arguments of the boundary between the type and the product's own)"""
+        stream, h = torch.empty_like(self.stream), torch.empty_like(self.y)
+        call((self.stream.data_ptr(), self.y.data_ptr(), _ptr(self.post_gain), self.branch_scale, _ptr(self.next_gain), self.next_scale, self.eps, stream.data_ptr(), h.data_ptr()))
+        self.result = stream, h
+
+
 def _token_calls(tokens: int, chunk_max: int):
     """(first token, count) of the library calls that cover `tokens` rows: chunks of MUI_MAX_TOKENS
     for the decode kernels up to chunk_max tokens, one call (the tiled GEMM) beyond."""
@@ -302,9 +340,13 @@ def muillm_linear_forward(
     add_bias: Optional[torch.Tensor] = None,
     residual: Optional[torch.Tensor] = None,
     behind: Optional[ResidualBehind] = None,
+    front: Optional[ResidualFront] = None,
 ) -> torch.Tensor:
     """y = (W . rmsnorm?(x)) * mul_bias + add_bias + residual, output shape x.shape[:-1] + [N]. behind: filled in where the call can
-    take it along."""
+    take it along. front: x is the output of the sublayer before the boundary, what is multiplied is what the boundary makes of it."""
+    if front is not None and (norm_weights is not None or mul_bias is not None or residual is not None or weights.dtype != x.dtype or weights.dim() != 2 or weights.shape[1] != x.shape[-1]
+                              or weights.device != x.device or not kernel_dispatchable(x)):
+        x, front = front.joined()[1], None
     if weights.dim() != 2:
         raise RuntimeError("weights must be 2-D [out_features, in_features]")
     n, k = weights.shape
@@ -338,6 +380,10 @@ def muillm_linear_forward(
             raise RuntimeError("residual must match the output's shape and dtype")
         residual = residual.contiguous()
     y = torch.empty(out_shape, dtype=x.dtype, device=x.device)
+    if front is not None:
+        front.along(lambda args: check(_lib.load().mui_joined_linear(_stream(x), _dtype_code(x), *args, weights.data_ptr(), pitch, _ptr(add_bias), y.data_ptr(), n, k, tokens,
+                                                                     None, 0), "mui_joined_linear"))
+        return y
     lib, stream, code, esz = _lib.load(), _stream(x), _dtype_code(x), x.element_size()
     ws = _prompt_workspace(x, stream) if tokens > FUSED_CHUNK_MAX_TOKENS else None
     ws_args = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
@@ -382,19 +428,21 @@ def muillm_linear_module_deinit(module: MuiLinearModuleHandle) -> None:
     module.weights = module.norm_weights = module.mul_bias = module.add_bias = None
 
 
-def muillm_linear_module_forward(module: MuiLinearModuleHandle, inputs: torch.Tensor, residual=None, behind=None):
+def muillm_linear_module_forward(module: MuiLinearModuleHandle, inputs: torch.Tensor, residual=None, behind=None, front=None):
     return muillm_linear_forward(
         module.engine, inputs, module.weights, module.norm_weights, module.epsilon,
-        module.mul_bias, module.add_bias, residual, behind,
+        module.mul_bias, module.add_bias, residual, behind, front,
     )
 
 
 # --------------------------------------------------------------------------------------
 # Gate/Up/Down MLP  (csrc/module.cpp:182,215; csrc/ffn/gateup.cu:88-391)
 # --------------------------------------------------------------------------------------
-def mui_gateup_silu(norm_weights, epsilon, gate_weights, up_weights, x, gate_bias=None, up_bias=None) -> torch.Tensor:
+def mui_gateup_silu(norm_weights, epsilon, gate_weights, up_weights, x, gate_bias=None, up_bias=None, front: Optional[ResidualFront] = None) -> torch.Tensor:
     """h = silu(G xn + gate_bias) * (U xn + up_bias) for any number of tokens; gate/up may be views into one
-    interleaved [N, 2, K] buffer (common row pitch)."""
+    interleaved [N, 2, K] buffer (common row pitch). front: as muillm_linear_forward's."""
+    if front is not None and norm_weights is not None:
+        x, front = front.joined()[1], None
     n, k = gate_weights.shape
     if up_weights.shape != gate_weights.shape:
         raise RuntimeError("gate and up weights must have the same shape")
@@ -416,6 +464,10 @@ def mui_gateup_silu(norm_weights, epsilon, gate_weights, up_weights, x, gate_bia
     tokens = _num_tokens(x)
     h = torch.empty(list(x.shape[:-1]) + [n], dtype=x.dtype, device=x.device)
     lib, stream, code, esz = _lib.load(), _stream(x), _dtype_code(x), x.element_size()
+    if front is not None:
+        front.along(lambda args: check(lib.mui_joined_gateup_silu(stream, code, *args, gate_weights.data_ptr(), up_weights.data_ptr(), pitch, _ptr(gate_bias), _ptr(up_bias),
+                                                                  h.data_ptr(), n, k, tokens), "mui_joined_gateup_silu"))
+        return h
     for off, cnt in _token_calls(tokens, FUSED_CHUNK_MAX_TOKENS):
         check(
             lib.mui_gateup_silu_bias(
@@ -440,23 +492,23 @@ def mui_silu_mul_interleaved(gate_up: torch.Tensor) -> torch.Tensor:
 
 
 def muillm_gateupsilu_forward(engine, norm_weights, epsilon, gate_weights, up_weights, down_weights,
-                              residual, x, biases=None, behind: Optional[ResidualBehind] = None) -> torch.Tensor:
+                              residual, x, biases=None, behind: Optional[ResidualBehind] = None, front: Optional[ResidualFront] = None) -> torch.Tensor:
     """out = Wd (silu(Wg xn) * (Wu xn)) + residual, argument order of csrc/module.cpp:182. biases: (gate, up, down)
-    vectors added to the three products, or None; behind: as muillm_linear_forward's."""
+    vectors added to the three products, or None; behind, front: as muillm_linear_forward's."""
     if not (kernel_dispatchable(x) and gate_weights.dtype == x.dtype):
         raise RuntimeError("muillm_gateupsilu_forward needs fp16 / bf16 CUDA tensors with k % 8 == 0")
     gate_bias, up_bias, down_bias = biases or (None, None, None)
-    h = mui_gateup_silu(norm_weights, epsilon, gate_weights, up_weights, x, gate_bias, up_bias)
+    h = mui_gateup_silu(norm_weights, epsilon, gate_weights, up_weights, x, gate_bias, up_bias, front)
     return muillm_linear_forward(engine, h, down_weights, add_bias=down_bias, residual=residual, behind=behind)
 
 
 def muillm_gateupsilu_split_forward(engine, norm_weights, epsilon, gate_weights, up_weights,
-                                    down_weights, residual, x, biases=None, behind=None) -> torch.Tensor:
+                                    down_weights, residual, x, biases=None, behind=None, front=None) -> torch.Tensor:
     """The reference's split-K variant (csrc/module.cpp:215) exists to create more blocks on
     MI300; the gfx950 kernel already sizes its grid to the CU count, so both names run the
     same path."""
     return muillm_gateupsilu_forward(engine, norm_weights, epsilon, gate_weights, up_weights,
-                                     down_weights, residual, x, biases, behind)
+                                     down_weights, residual, x, biases, behind, front)
 
 
 # --------------------------------------------------------------------------------------
