@@ -668,6 +668,15 @@ int mui_latent_prepare(mui_stream_t stream, int dtype, const void* down, long do
                        long r_batch_stride, int batch, int t, int q_rank, int kv_rank, int rot_dim,
                        int max_cache_len);
 
+/* mui_latent_prepare's rows and mui_latent_attention of ONE new token per batch row in one launch, 16-bit types: q as for mui_latent_attention, projected from the normed query
+ * latent; kv [batch, kv_pitch]: the down projection's latent row and key part of the new token (its row is normed with kv_gain, its key part rotated, both go to slot
+ * cache_position[0]), or NULL where the caches hold them already. Values as by the separate calls but for roundings in between, which stay in fp32. mui_latent_step_serves: 1 where
+ * the visible keys -- window, or the capacity -- and the heads of all rows are few enough and the sizes covered, else 0 (the call returns MUI_ERR_UNSUPPORTED). */
+int mui_latent_step_serves(int dtype, int batch, int heads, int dim, int rot_dim, int vdim, int kv_rank, int window, int max_cache_len);
+int mui_latent_step(mui_stream_t stream, int dtype, const void* q, const void* w_uk, const void* w_uv, const void* kv, long kv_pitch, const void* kv_gain, float epsilon,
+                    const double* inv_freq, void* c_cache, long c_batch_stride, void* r_cache, long r_batch_stride, const int64_t* cache_position, const int64_t* row_start,
+                    float scale, int window, void* out, int batch, int heads, int dim, int rot_dim, int vdim, int kv_rank, int max_cache_len);
+
 /* Which kernels serve a call: PLAIN (one workgroup per query and head: fp32, odd sizes), DECODE (attention
  * over the latent rows themselves), PREFILL (mui_latent_prefill_attention). `tokens`: per batch row. */
 #define MUI_LATENT_PLAIN 0

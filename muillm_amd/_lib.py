@@ -126,6 +126,8 @@ _SIGNATURES = {
     "mui_moe_down": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int]),
     "mui_latent_prepare": (c_int, [_P, c_int, _P, c_long, _P, _P, c_float, _P, _P, _P, _P, _P, _P, c_long, _P, c_long,
                                    c_int, c_int, c_int, c_int, c_int, c_int]),
+    "mui_latent_step_serves": (c_int, [c_int] * 9),
+    "mui_latent_step": (c_int, [_P, c_int, _P, _P, _P, _P, c_long, _P, c_float, _P, _P, c_long, _P, c_long, _P, _P, c_float, c_int, _P] + [c_int] * 7),
     "mui_latent_attention_route": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "mui_latent_decode_scratch_bytes": (ctypes.c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "mui_latent_attention": (c_int, [_P, c_int, c_int, _P, _P, _P, _P, _P, c_long, _P, c_long, _P, _P, c_float, c_int,

@@ -284,6 +284,43 @@ def latent_attention(q: torch.Tensor, cos_sin: torch.Tensor, w_uk: torch.Tensor,
     return out
 
 
+def latent_step_serves(like: torch.Tensor, batch: int, heads: int, dim: int, rot: int, vdim: int, w_uk: torch.Tensor, w_uv: torch.Tensor, c_cache: torch.Tensor,
+                       r_cache: torch.Tensor, window: int) -> bool:
+    """Whether latent_step takes one new token per row."""
+    if like.dtype not in (torch.float16, torch.bfloat16) or not like.is_cuda or c_cache.stride(0) % 8 or r_cache.stride(0) % 8:
+        return False
+    if any(x.data_ptr() % 16 or not x.is_contiguous() for x in (w_uk, w_uv, c_cache, r_cache)):
+        return False
+    return bool(_lib.load().mui_latent_step_serves(dtype_code(like.dtype), batch, heads, dim, rot, vdim, c_cache.shape[-1], int(window), c_cache.shape[1]))
+
+
+def latent_step(q: torch.Tensor, kv: Optional[torch.Tensor], kv_gain: Optional[torch.Tensor], eps: float, inv_freq: torch.Tensor, w_uk: torch.Tensor, w_uv: torch.Tensor,
+                c_cache: torch.Tensor, r_cache: torch.Tensor, cache_position: torch.Tensor, row_start: Optional[torch.Tensor], heads: int, dim: int, vdim: int, scale: float,
+                window: int) -> torch.Tensor:
+    """Attention of one new token per row, [B, 1, heads * vdim], where latent_step_serves. kv [B, 1, kv_rank + rot], a slice of the down projection's output: the new token's row and key
+    part go to the caches as by latent_prepare; None: they are there."""
+    kv_rank, rot, cap = c_cache.shape[-1], r_cache.shape[-1], c_cache.shape[1]
+    b = q.shape[0]
+    _operand(q, "q", q, (b, 1, heads * (dim + rot)))
+    _operand(w_uk, "w_uk", q, (heads * dim, kv_rank))
+    _operand(w_uv, "w_uv", q, (heads * vdim, kv_rank))
+    _operand(c_cache, "c_cache", q)
+    _operand(r_cache, "r_cache", q, (c_cache.shape[0], cap, rot))
+    _operand(inv_freq, "inv_freq", q, (rot // 2,), torch.float64)
+    _positions(cache_position, row_start, q, b, 1)
+    if b > c_cache.shape[0]:
+        raise RuntimeError("more batch rows than the cache has")
+    if kv is not None:
+        _operand(kv_gain, "kv_gain", q, (kv_rank,))
+        if kv.dtype != q.dtype or kv.device != q.device or kv.shape != (b, 1, kv_rank + rot) or kv.stride(2) != 1:
+            raise RuntimeError("kv must be the latent rows and key parts of a projection's output")
+    out = torch.empty((b, 1, heads * vdim), dtype=q.dtype, device=q.device)
+    check(_lib.load().mui_latent_step(_stream(q), dtype_code(q.dtype), q.data_ptr(), w_uk.data_ptr(), w_uv.data_ptr(), _ptr(kv), 0 if kv is None else kv.stride(0), _ptr(kv_gain),
+                                      float(eps), inv_freq.data_ptr(), c_cache.data_ptr(), c_cache.stride(0), r_cache.data_ptr(), r_cache.stride(0), cache_position.data_ptr(),
+                                      _ptr(row_start), float(scale), int(window), out.data_ptr(), b, heads, dim, rot, vdim, kv_rank, cap), "mui_latent_step")
+    return out
+
+
 def latent_prefill_attention(q: torch.Tensor, cos_sin: torch.Tensor, kv: Union[torch.Tensor, List[torch.Tensor]], kv_first: int,
                              r_cache: torch.Tensor, row_start: Optional[torch.Tensor], q_first: int, heads: int, dim: int,
                              vdim: int, scale: float, window: int) -> torch.Tensor:

@@ -1,6 +1,6 @@
 """MuiLatentAttention: attention whose keys and values are linear maps of one cached latent row per token
 plus a rotated key part shared by all heads, with queries through a latent of their own and a sliding
-window. Kernels: csrc/latent_attention.hip.
+window. Kernels: csrc/latent_attention.hip, csrc/latent_step.hip.
 
 A layer may read another layer's cached rows (kv_source) instead of keeping its own: it then has no key /
 value down projection, only its own up projections, queries and window."""
@@ -10,10 +10,10 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
-from ... import _lib, hybrid_ops
+from ... import _lib, hybrid_ops, muillm_ext
 from ...engineconfig import MuiEngineConfig
 from ..kvcache.hybridcache import MuiHybridCache, MuiLatentState
-from ..linear import MuiLinear
+from ..linear import MuiLinear, _MuiLinear
 from ..module import MuiModule, heard
 from ..multilinear import MuiMultiLinear
 
@@ -71,12 +71,25 @@ class MuiLatentAttention(MuiModule):
         down = cache.spread(self.down.linear(h))
         b, t = down.shape[0], down.shape[1]
         state: MuiLatentState = cache.layers[self.layer_idx if self.own_rows else c.kv_source]
+        w = self.up_kv.weight
+        w_uk, w_uv = w[:c.heads * c.dim], w[c.heads * c.dim:]
+        step = t == 1 and hybrid_ops.latent_step_serves(down, b, c.heads, c.dim, c.rot_dim, c.vdim, w_uk, w_uv, state.c, state.r, c.window)
+        if step and b == 1 and c.q_rank % 8 == 0 and down.data_ptr() % 16 == 0 and self.up_q.takes_front():
+            # the query's norm goes with its projection, the token's rows with the attention
+            up = self.up_q.cpp_module
+            normed = muillm_ext.MuiLinearModuleHandle(up.engine, up.weights, self.q_norm, self.eps, up.mul_bias, up.add_bias)
+            q = _MuiLinear.apply(normed, down[..., :c.q_rank], None)
+            kv = down[..., c.q_rank:] if self.own_rows else None
+            o = hybrid_ops.latent_step(q, kv, self.kv_norm, self.eps, self.inv_freq, w_uk, w_uv, state.c, state.r, cache_position, cache.row_start, c.heads, c.dim, c.vdim,
+                                       c.scale, c.window)
+            return self._project(cache.take(o), behind)
         q_latent, cos_sin = hybrid_ops.latent_prepare(down, self.q_norm, self.kv_norm, self.eps, self.inv_freq,
                                                       cache_position, cache.row_start, state.c, state.r)
         q = self.up_q(q_latent)
         route = hybrid_ops.latent_route(h.dtype, t, c.heads, c.dim, c.rot_dim, c.vdim, c.kv_rank)
-        w = self.up_kv.weight
-        if route == _lib.MUI_LATENT_PREFILL:
+        if step:
+            o = hybrid_ops.latent_step(q, None, None, self.eps, self.inv_freq, w_uk, w_uv, state.c, state.r, cache_position, cache.row_start, c.heads, c.dim, c.vdim, c.scale, c.window)
+        elif route == _lib.MUI_LATENT_PREFILL:
             # keys and values of everything the tokens can see, once per call
             q_first = cache.get_seq_length()
             kv_first = max(0, q_first - c.window + 1) if c.window else 0
@@ -84,7 +97,9 @@ class MuiLatentAttention(MuiModule):
             o = hybrid_ops.latent_prefill_attention(q, cos_sin, kv, kv_first, state.r, cache.row_start, q_first, c.heads, c.dim,
                                                     c.vdim, c.scale, c.window)
         else:
-            o = hybrid_ops.latent_attention(q, cos_sin, w[:c.heads * c.dim], w[c.heads * c.dim:], state.c, state.r,
+            o = hybrid_ops.latent_attention(q, cos_sin, w_uk, w_uv, state.c, state.r,
                                             cache_position, cache.row_start, c.heads, c.dim, c.vdim, c.scale, c.window, route)
-        o = cache.take(o)
+        return self._project(cache.take(o), behind)
+
+    def _project(self, o: torch.Tensor, behind) -> torch.Tensor:
         return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)
