@@ -1618,7 +1618,7 @@ static int launch_attn(hipStream_t s, int dtype, const AttnParams& p, int batch)
 using namespace mui;
 
 static int g_attn_min_tokens = 0;  // 0: built-in choice; else fewest tokens worth a split
-// prompt attention: 0 = built-in choice (the KV-group kernel from 512 query tokens), n > 0 = from n
+// prompt attention: 0 = built-in choice (kv_group_is_faster), n > 0 = the KV-group kernel from n
 // tokens, negative = never
 static int g_prefill_group_tokens = 0;
 static int g_prefill_attn_direct = 1;  // 0: K / V rows staged through registers
@@ -1952,6 +1952,25 @@ extern "C" int mui_rope_kv_write(mui_stream_t stream, int dtype, const void* q, 
   return launch_status();
 }
 
+static bool kv_group_built(int group) { return group == 1 || group == 2 || group == 4 || group == 8; }
+
+// Which kernel takes a prompt. With 1, 2, 4 or 8 query heads per KV head, K/V rows can cross LDS once per 32 query positions of the whole KV group
+// (attn_prefill_group_kernel). attn_prefill_mfma_kernel splits the keys of 16 query positions of one head over four waves: shorter chains, more workgroups, of which two fit a CU.
+// us, split / group, 32 query heads on 8 without a mask unless said:
+//   more than 256 tokens    272 tokens 15.8 / 11.6
+//   rounds of workgroups    the split kernel's rounds follow each other at 7 us and more each: 4 rows of 101 / 200 / 256 tokens 16.7 / 8.2, 30.4 / 10.3, 39.6 / 12.0, 32 rows of 24 / 100
+//                           28.2 / 6.4, 115 / 22.5, 14 rows of 40 21.2 / 6.6, 4 of 150 behind 2000 cached 112.8 / 53.1; 16 heads on 4: 4 rows of 150 behind 40 / 2000 (640 workgroups)
+//                           17.0 / 9.6, 57.5 / 51.5. Eight heads per KV head are 8 waves with a longer chain: 640 workgroups 16.9 / 13.1 behind 40, 26.3 / 27.1 behind 500; 832 17.8 / 13.4
+//   part of a round         (up to two workgroups per CU) 4 rows of 101 9.4 / 7.9, under a mask 9.5 / 9.2; longer keys and one workgroup per CU are the split kernel's: 1 row of 256
+//                           10.5 / 10.9 and 10.8 / 13.3, 1 of 101 7.3 / 7.4 and 7.2 / 8.7, 4 of 24 behind 200 8.9 / 9.7
+//   one block of keys       nothing is worth splitting: 1 row of 24 6.8 / 5.5, 4 of 48 8.9 / 6.2; 8 heads per KV head 6.7 / 7.3
+static bool kv_group_is_faster(int group, int batch, int heads, int tokens, int seq_len) {
+  if (!kv_group_built(group)) return false;
+  const long workgroups = (long)batch * heads * ceil_div(tokens, 16), cus = device_cus();
+  if (tokens > 256 || workgroups > (group == 8 ? 3 : 2) * cus) return true;
+  return group <= 4 && (seq_len <= 48 || (seq_len <= 128 && workgroups > cus));
+}
+
 static int prefill_attention_impl(mui_stream_t stream, int dtype, const void* q_rotated, const void* k_cache,
                                   const void* v_cache, long cache_batch_stride, long cache_head_stride,
                                   long cache_token_stride, int seq_len, int q_start, const void* key_mask,
@@ -1981,14 +2000,9 @@ static int prefill_attention_impl(mui_stream_t stream, int dtype, const void* q_
   p.key_mask = (const uint16_t*)key_mask; p.mask_bs = mask_batch_stride;
   const bool masked = key_mask != nullptr;
   hipStream_t s = (hipStream_t)stream;
-  // Long prompts with 1, 2, 4 or 8 query heads per KV head: K/V rows cross LDS once per 32 query
-  // positions of the whole KV group. Short prompts keep the kernel that splits the key range of
-  // 16 query positions over four waves (more workgroups, shorter chains) up to 256 tokens, while
-  // its grid (32 heads x 16 tiles) is a single round of workgroups: both take 7-12 us there; at 272
-  // tokens it is 15.8 us against 11.6 us.
   const int group = n_q_heads / n_kv_heads;
-  const bool grouped = (group == 1 || group == 2 || group == 4 || group == 8) &&
-                       (g_prefill_group_tokens > 0 ? tokens >= g_prefill_group_tokens : g_prefill_group_tokens == 0 && tokens > 256);
+  const bool grouped = g_prefill_group_tokens > 0 ? kv_group_built(group) && tokens >= g_prefill_group_tokens
+                                                  : g_prefill_group_tokens == 0 && kv_group_is_faster(group, batch, n_q_heads, tokens, seq_len);
   if (grouped) {
     if (ceil_div(tokens, 16) > 65535) return MUI_ERR_UNSUPPORTED;  // position tiles are the grid's y
     // K / V rows straight into LDS where every cache row is 16-byte aligned

@@ -452,6 +452,29 @@ def test_prefill_attention_long_prompts(b, hq, hkv, t, past, dtype, choice):
         _lib.check(lib.mui_tune_prefill_attention(0), "tune")
 
 
+@pytest.mark.parametrize("b,hq,hkv,t,past", [
+    (1, 8, 2, 2, 0), (1, 8, 2, 48, 0), (1, 8, 2, 17, 31), (1, 8, 2, 49, 0),  # one block of keys, one more
+    (8, 32, 8, 17, 0), (9, 32, 8, 17, 47), (4, 32, 8, 100, 28), (4, 32, 8, 100, 29),  # one workgroup per CU and beyond, 128 keys and 129
+    (17, 32, 8, 16, 100), (16, 32, 8, 16, 100), (17, 16, 16, 24, 65),  # two per CU and beyond
+    (24, 32, 4, 16, 3), (25, 32, 4, 16, 3),  # eight heads per KV head: three
+    (11, 24, 8, 33, 0),  # three: always per head
+])
+@pytest.mark.parametrize("hidden", [False, True])
+def test_prefill_attention_of_several_rows(b, hq, hkv, t, past, hidden):
+    """Both sides of the lines between the prompt kernels; hidden: a row's first keys, a different number in each row."""
+    g, s, dtype = _gen(31), past + t, torch.float16
+    q, kc, vc = (_mk((b, h, n, D), g, dtype=dtype) for h, n in ((hq, t), (hkv, s), (hkv, s)))
+    keep = (torch.arange(s)[None, :] >= torch.arange(b)[:, None] % (s - 1) * int(hidden)).long()
+    mask = muillm_ext.key_padding_mask16(keep.to(DEV), dtype) if hidden else None
+    out = muillm_ext.mui_prefill_attention(q.to(DEV), kc.to(DEV), vc.to(DEV), key_mask=mask).cpu()
+    mask4 = _causal_mask(t, s, past).expand(b, 1, t, s).clone().masked_fill(keep[:, None, None, :] == 0, float("-inf"))
+    sees = torch.isfinite(mask4).any(dim=-1)[:, 0]
+    mask4[~sees[:, None].expand(b, 1, t)] = 0.0
+    ref = oracle.decode_attention(q, kc, vc, mask4).reshape(b, t, hq * D)
+    assert _attn_err(out[sees], ref[sees]) <= ATOL
+    assert (out[~sees] == 0).all()
+
+
 @pytest.mark.parametrize("choice", ["kv-group", "kv-group-register-staged", "per-head"])
 @pytest.mark.parametrize("b,hq,hkv,t,past,padding", [
     (3, 32, 8, 200, 0, "left"),      # the reference's padded batches (tokenizer padding on the left)
