@@ -89,26 +89,6 @@ __device__ __forceinline__ float dot2_acc<BF16>(uint32_t a, uint32_t b, float c)
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Maximum / sum over the four 16-lane rows of a wave (lanes i, i + 16, i + 32, i + 48), the same
-// value in all four: gfx950's row-swap instructions exchange rows between two registers in the
-// vector ALU, without the LDS round trip of ds_bpermute that a shuffle by 16 or 32 lanes costs.
-// (permlane16_swap: rows 1, 3 of the first operand <-> rows 0, 2 of the second; permlane32_swap:
-// upper half of the first <-> lower half of the second.) The additions pair the rows as the two
-// shuffles did -- (r0 + r1) + (r2 + r3) --, so the results are bit-identical.
-__device__ __forceinline__ float rows_max(float v) {
-  const unsigned u = __float_as_uint(v);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  const unsigned w = __float_as_uint(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
-  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float rows_sum(float v) {
-  const unsigned u = __float_as_uint(v);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  const unsigned w = __float_as_uint(__uint_as_float(a[0]) + __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
 // The two registers of one swap: OFF = 16 -> a = rows (0, 0, 2, 2), b = rows (1, 1, 3, 3) of v;
 // OFF = 32 -> a = rows (0, 1, 0, 1), b = rows (2, 3, 2, 3). Every row sees its own value in one of
 // them and its partner's (lane ^ OFF) in the other, in the same order in all rows.

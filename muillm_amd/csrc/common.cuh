@@ -196,6 +196,27 @@ __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Maximum / sum over the four 16-lane rows of a wave (lanes i, i + 16, i + 32, i + 48), the same
+// value in all four: gfx950's row-swap instructions exchange rows between two registers in the
+// vector ALU, without the LDS round trip of ds_bpermute that a shuffle by 16 or 32 lanes costs.
+// (permlane16_swap: rows 1, 3 of the first operand <-> rows 0, 2 of the second; permlane32_swap:
+// upper half of the first <-> lower half of the second.) The additions pair the rows as the two
+// shuffles did -- (r0 + r1) + (r2 + r3) --, so the results are bit-identical.
+__device__ __forceinline__ float rows_max(float v) {
+  const unsigned u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned w = __float_as_uint(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float rows_sum(float v) {
+  const unsigned u = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned w = __float_as_uint(__uint_as_float(a[0]) + __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 // A 4 x 16 block of 16-bit elements read transposed from LDS: within a group of 16 lanes, lane i
 // receives element i % 4 of the 8-byte rows addressed by lanes i / 4, i / 4 + 4, i / 4 + 8 and
 // i / 4 + 12 -- four rows of column i when lane i points at row i / 4, columns 4 (i % 4) .. + 3.

@@ -35,4 +35,29 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// The order of a prompt attention's matrix instructions and operand reads, for 64 keys and two tiles of 16 queries: left alone the compiler waits
+// for an LDS read in front of half of the products. Scores: the operands of two chunks of 32 dimensions requested ahead, then four reads per eight products.
+template <int DKC>
+__device__ __forceinline__ void pin_scores() {
+  __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+  for (int c = 2; c < DKC; ++c) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+  __builtin_amdgcn_sched_barrier(0x6);  // only scalar and vector ALU work may move across
+}
+// Values: four tiles requested ahead, then two reads per two products.
+template <int DVT>
+__device__ __forceinline__ void pin_values() {
+  __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);
+#pragma unroll
+  for (int j = 4; j < 2 * DVT; ++j) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 2, 1);
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, 8, 1);
+}
+
 }  // namespace mui

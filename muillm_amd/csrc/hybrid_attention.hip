@@ -725,18 +725,22 @@ __global__ void __launch_bounds__(128) hybrid_combine_kernel(const HybridAttnPar
 
 // ---------------------------------------------------------------------------------------
 // prefill: grid (batch * heads / head_waves, tiles of queries, longest first); NW waves, wave w serves query head
-// w % head_waves and the block of 32 queries w / head_waves. LDS holds two stages of 64 keys and one of their
-// values: while block s is multiplied with the queries, its values and the keys of block s + 1 are on their way.
+// w % head_waves and the block of 32 queries w / head_waves. LDS holds two stages of 64 keys and their
+// values, one of them on its way while the other is multiplied: one barrier per block, with the matrix instructions in a pinned order and a raised
+// priority while they run. Bound by the softmax's instructions (three transcendental ones per score under a cap) and what two waves per SIMD cannot hide
+// of the chain behind them: 4000 tokens, 32 heads on 8 of 128 under a cap 298 -> 266 us (0.49 PFLOP/s) against one stage of values, two barriers and
+// the compiler's order; the same order with two stages 272. Two bodies, with and without hidden keys, do not fit the registers (spills: 298). A maximum that
+// lags by up to 2^8 would save rescaling (252) and costs up to a fifth in precision: the largest probability is no longer exactly 1.
 // ---------------------------------------------------------------------------------------
 template <int DKC, int DVT>
-constexpr size_t hybrid_prefill_lds() { return (size_t)64 * (2 * DKC * 32 + DVT * 16) * 2; }
+constexpr size_t hybrid_prefill_lds() { return (size_t)64 * 2 * (DKC * 32 + DVT * 16) * 2; }
 
 template <typename T, int DKC, int DVT, int NW, bool CAP>
 __global__ void __launch_bounds__(64 * NW, DKC > 4 ? 1 : 2) hybrid_prefill_kernel(const HybridAttnParams p) {
   static_assert(DKC % 2 == 0 && DVT % 4 == 0 && (NW == 2 || NW == 4), "tiles of 64 columns");
-  constexpr int KG = DKC / 2, VG = DVT / 4, RB = 8 / NW, RSTEP = 8 * NW, KSTAGE = KG * 64 * 64;
+  constexpr int KG = DKC / 2, VG = DVT / 4, RB = 8 / NW, RSTEP = 8 * NW, KSTAGE = KG * 64 * 64, VSTAGE = VG * 64 * 64;
   uint16_t* smem = (uint16_t*)ha_smem;
-  uint16_t* vl = smem + 2 * KSTAGE;
+  uint16_t* values = smem + 2 * KSTAGE;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4, i16 = lane & 15;
   const int hw = p.head_waves, hgs = p.heads / hw, b = blockIdx.x / hgs;
   const int h = (blockIdx.x - b * hgs) * hw + wave % hw, kvh = h / (p.heads / p.kv_heads);
@@ -769,16 +773,21 @@ __global__ void __launch_bounds__(64 * NW, DKC > 4 ? 1 : 2) hybrid_prefill_kerne
         load_lds16(src + (cg * 64 + lc < p.dim ? cg * 64 + lc : 0), &dst[(cg * 64 + wave * 8 + RSTEP * u) * 64]);
     }
   };
-  auto load_v = [&](int s0) {
+  auto load_v = [&](int s0, uint16_t* dst) {
 #pragma unroll
     for (int u = 0; u < RB; ++u) {
       const int n = s0 + lrow + RSTEP * u;
       const uint16_t* src = vc + kr.slot(n < n_keys ? n : n_keys - 1) * vp;
 #pragma unroll
       for (int cg = 0; cg < VG; ++cg)
-        load_lds16(src + (cg * 64 + lc < p.vdim ? cg * 64 + lc : 0), &vl[(cg * 64 + wave * 8 + RSTEP * u) * 64]);
+        load_lds16(src + (cg * 64 + lc < p.vdim ? cg * 64 + lc : 0), &dst[(cg * 64 + wave * 8 + RSTEP * u) * 64]);
     }
   };
+  auto load_block = [&](int s0, int stage) {
+    load_k(s0, smem + stage * KSTAGE);
+    load_v(s0, values + stage * VSTAGE);
+  };
+  if (n_keys > 0) load_block(0, 0);
   u32x4 q[2][DKC];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
@@ -791,106 +800,103 @@ __global__ void __launch_bounds__(64 * NW, DKC > 4 ? 1 : 2) hybrid_prefill_kerne
       q[qt][c] = e < p.dim ? v : u32x4{0u, 0u, 0u, 0u};
     }
   }
-  if (n_keys > 0) load_k(0, smem);
   // this wave's queries, counted like the window's keys
   const int wq0 = (int)(q_first + wq - kr.first) - kr.shift, wq1 = wq0 + 31;
-  for (int s0 = 0, buf = 0; s0 < n_keys; s0 += 64, buf ^= 1) {
-    const uint16_t* kl = smem + buf * KSTAGE;
-    const bool more = s0 + 64 < n_keys;
-    // (blocks that none of the wave's queries sees are skipped)
-    const bool mine = s0 <= wq1 && (p.window <= 0 || s0 + 63 > wq0 - p.window || s0 < p.keep);
-    wait_loads<0>();  // this wave's rows of the keys have landed
-    __syncthreads();  // ... and everybody's; everybody is done with the values and the other keys
-    load_v(s0);
-    if (more) load_k(s0 + 64, smem + (buf ^ 1) * KSTAGE);
-    u32x4 pb[2][2];
-    if (mine) {
-      f32x4 s4[2][4];
+  // full: every query of the wave sees every key of the block
+  auto attend = [&](const uint16_t* kl, const uint16_t* vl, int s0, const bool full) {
+    f32x4 s4[2][4];
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) s4[qt][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+    for (int c = 0; c < DKC; ++c)
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt) {
+        const u32x4 a = *(const u32x4*)&kl[tile_at<64>(kt * 16 + i16, c * 32 + 8 * g)];
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt) s4[qt][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < DKC; ++c) {
-          const u32x4 a = *(const u32x4*)&kl[tile_at<64>(kt * 16 + i16, c * 32 + 8 * g)];
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) s4[qt][kt] = mfma16x16x32<T>(a, q[qt][c], s4[qt][kt]);
-        }
+        for (int qt = 0; qt < 2; ++qt) s4[qt][kt] = mfma16x16x32<T>(a, q[qt][c], s4[qt][kt]);
       }
-      const bool full = s0 + 63 <= wq0 && (p.window <= 0 || s0 > wq1 - p.window || s0 + 63 < p.keep);
+    pin_scores<DKC>();
+    __builtin_amdgcn_s_setprio(0);
+    u32x4 pb[2][2];
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        float mx = -INFINITY;
-        if (full) {
-#pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              s4[qt][kt][r] = score_log2<CAP>(s4[qt][kt][r], c1, c2);
-              mx = fmaxf(mx, s4[qt][kt][r]);
-            }
-        } else {
-          // keys counted from the block's start: the last one seen, the last one in front of the window, the
-          // first one that is not kept
-          const int last = wq0 + qt * 16 + i16 - s0, before = p.window > 0 ? last - p.window : -1, kept = p.keep - s0;
-#pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int s = kt * 16 + 4 * g + r;
-              const float v = score_log2<CAP>(s4[qt][kt][r], c1, c2);
-              s4[qt][kt][r] = s <= last && (s > before || s < kept) ? v : -INFINITY;
-              mx = fmaxf(mx, s4[qt][kt][r]);
-            }
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        if (__any(mx > m[qt])) {
-          const float mn = fmaxf(m[qt], mx), keep = __builtin_amdgcn_exp2f(m[qt] - mn);
-          m[qt] = mn;
-          l[qt] *= keep;
-#pragma unroll
-          for (int j = 0; j < DVT; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[qt][j][r] *= keep;
-        }
-        float e[4][4], sum = 0.f;
+    for (int qt = 0; qt < 2; ++qt) {
+      float mx = -INFINITY;
+      if (full) {
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            e[kt][r] = __builtin_amdgcn_exp2f(s4[qt][kt][r] - m[qt]);
-            sum += e[kt][r];
+            s4[qt][kt][r] = score_log2<CAP>(s4[qt][kt][r], c1, c2);
+            mx = fmaxf(mx, s4[qt][kt][r]);
           }
-        l[qt] += sum;  // this lane's keys only; the lane groups are added up at the end
+      } else {
+        // keys counted from the block's start: the last one seen, the last one in front of the window, the
+        // first one that is not kept
+        const int last = wq0 + qt * 16 + i16 - s0, before = p.window > 0 ? last - p.window : -1, kept = p.keep - s0;
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-          pb[qt][kk] = u32x4{T::pack2(e[2 * kk][0], e[2 * kk][1]), T::pack2(e[2 * kk][2], e[2 * kk][3]),
-                             T::pack2(e[2 * kk + 1][0], e[2 * kk + 1][1]), T::pack2(e[2 * kk + 1][2], e[2 * kk + 1][3])};
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int s = kt * 16 + 4 * g + r;
+            const float v = score_log2<CAP>(s4[qt][kt][r], c1, c2);
+            s4[qt][kt][r] = s <= last && (s > before || s < kept) ? v : -INFINITY;
+            mx = fmaxf(mx, s4[qt][kt][r]);
+          }
       }
-    }
-    // the values were requested before the next keys
-    if (more) wait_loads<RB * KG>();
-    else wait_loads<0>();
-    __syncthreads();
-    if (mine) {
+      mx = rows_max(mx);
+      if (__any(mx > m[qt])) {
+        const float mn = fmaxf(m[qt], mx), keep = __builtin_amdgcn_exp2f(m[qt] - mn);
+        m[qt] = mn;
+        l[qt] *= keep;
+#pragma unroll
+        for (int j = 0; j < DVT; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[qt][j][r] *= keep;
+      }
+      float e[4][4], sum = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          e[kt][r] = __builtin_amdgcn_exp2f(s4[qt][kt][r] - m[qt]);
+          sum += e[kt][r];
+        }
+      l[qt] += sum;  // this lane's keys only; the lane groups are added up at the end
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-        for (int j = 0; j < DVT; ++j) {
-          const int row = 32 * kk + 4 * g + (i16 >> 2), col = 16 * j + 4 * (i16 & 3);
-          const u32x2 a0 = lds_read_tr16(&vl[tile_at<64>(row, col)]), a1 = lds_read_tr16(&vl[tile_at<64>(row + 16, col)]);
-          const u32x4 va = {a0.x, a0.y, a1.x, a1.y};
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) acc[qt][j] = mfma16x16x32<T>(va, pb[qt][kk], acc[qt][j]);
-        }
+        pb[qt][kk] = u32x4{T::pack2(e[2 * kk][0], e[2 * kk][1]), T::pack2(e[2 * kk][2], e[2 * kk][3]),
+                           T::pack2(e[2 * kk + 1][0], e[2 * kk + 1][1]), T::pack2(e[2 * kk + 1][2], e[2 * kk + 1][3])};
     }
+    __builtin_amdgcn_sched_barrier(0x6);
+    __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < DVT; ++j) {
+        const int row = 32 * kk + 4 * g + (i16 >> 2), col = 16 * j + 4 * (i16 & 3);
+        const u32x2 a0 = lds_read_tr16(&vl[tile_at<64>(row, col)]), a1 = lds_read_tr16(&vl[tile_at<64>(row + 16, col)]);
+        const u32x4 va = {a0.x, a0.y, a1.x, a1.y};
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) acc[qt][j] = mfma16x16x32<T>(va, pb[qt][kk], acc[qt][j]);
+      }
+    pin_values<DVT>();
+    __builtin_amdgcn_s_setprio(0);
+  };
+  for (int s0 = 0, buf = 0; s0 < n_keys; s0 += 64, buf ^= 1) {
+    wait_loads<0>();  // this wave's rows of the block have landed
+    __syncthreads();  // ... and everybody's; everybody is done with the block before
+    if (s0 + 64 < n_keys) load_block(s0 + 64, buf ^ 1);
+    const uint16_t *kl = smem + buf * KSTAGE, *vl = values + buf * VSTAGE;
+    // (blocks that none of the wave's queries sees are skipped)
+    if (s0 > wq1 || (p.window > 0 && s0 + 63 <= wq0 - p.window && s0 >= p.keep)) continue;
+    attend(kl, vl, s0, s0 + 63 <= wq0 && (p.window <= 0 || s0 > wq1 - p.window || s0 + 63 < p.keep));
   }
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
-    float s = l[qt];
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
+    const float s = rows_sum(l[qt]);
     const float inv = s > 0.f ? 1.f / s : 0.f;
     const int tq = wq + qt * 16 + i16;
     if (tq >= p.t) continue;

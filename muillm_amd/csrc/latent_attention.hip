@@ -577,22 +577,24 @@ __global__ void __launch_bounds__(256) latent_output_kernel(const LatentParams p
 // ---------------------------------------------------------------------------------------
 // prefill: grid (heads, tiles of 32 NW queries, longest first, batch rows); NW waves of 32 queries, two or more
 // workgroups per CU. Rows of a batch share a launch: a row of 150 tokens and 16 heads is 48 workgroups, and eight launches of
-// those took 24 us each where one takes 29 us (the keys and values of all rows come from one product likewise). LDS holds two stages of 64 keys and one of their values: while block s is multiplied with
-// the queries, its values and the keys of block s + 1 are on their way (LDS-direct loads, no registers).
+// those took 24 us each where one takes 29 us (the keys and values of all rows come from one product likewise). LDS holds two stages of 64 keys and their
+// values (80 KB for keys of 192: two workgroups fill a CU's), one of them on its way while the other is multiplied (LDS-direct loads, no registers); one
+// barrier per block and a pinned order as in hybrid_attention.hip. 2000 tokens, 32 heads of 128 + 64: 119 -> 108 us; one softmax block for both query tiles
+// spills (129), short tiles as companions of long ones on a CU change nothing (108).
 // ---------------------------------------------------------------------------------------
 template <int DKC, int DVT, int NW>
-constexpr size_t latent_prefill_lds() {  // K stage, then (the queries, before the loop | second K stage, V)
-  constexpr size_t k = (size_t)64 * DKC * 32 * 2, v = (size_t)64 * DVT * 16 * 2, q = (size_t)32 * NW * DKC * 32 * 2;
-  return k + (q > k + v ? q : k + v);
+constexpr size_t latent_prefill_lds() {  // two stages of keys and values; the queries, before the loop, behind the first keys
+  constexpr size_t k = (size_t)64 * DKC * 32 * 2, all = 2 * (k + (size_t)64 * DVT * 16 * 2);
+  static_assert(k + (size_t)32 * NW * DKC * 32 * 2 <= all, "the queries fit behind the first keys");
+  return all;
 }
 template <typename T, int DKC, int DVT, int NW>
 __global__ void __launch_bounds__(64 * NW, DKC > 6 ? 1 : 2) latent_prefill_kernel(const LatentParams p) {
   static_assert(DKC % 2 == 0 && DVT % 4 == 0 && (NW == 2 || NW == 4), "tiles of 64 columns");
   constexpr int QT = 32 * NW, KG = DKC / 2, VG = DVT / 4;  // queries per workgroup, blocks of 64 columns
   constexpr int RB = 8 / NW, RSTEP = 8 * NW;               // blocks of eight rows per wave, rows between them
-  constexpr int KSTAGE = KG * 64 * 64;
+  constexpr int KSTAGE = KG * 64 * 64, STAGE = KSTAGE + VG * 64 * 64;  // keys, then values
   uint16_t* smem = (uint16_t*)la_smem;
-  uint16_t* vl = smem + 2 * KSTAGE;
   uint16_t* ql = smem + KSTAGE;  // [KG][QT][64], until the loop starts
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), g = lane >> 4, i16 = lane & 15;
   const int h = blockIdx.x, qt0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * QT;
@@ -643,20 +645,20 @@ __global__ void __launch_bounds__(64 * NW, DKC > 6 ? 1 : 2) latent_prefill_kerne
       }
     }
   };
-  auto load_v = [&](int s0) {
+  auto load_v = [&](int s0, uint16_t* dst) {
     if (vec) {
 #pragma unroll
       for (int u = 0; u < RB; ++u) {
         const long row = s0 + lrow + RSTEP * u < n_keys ? s0 + lrow + RSTEP * u : n_keys - 1;
 #pragma unroll
         for (int cg = 0; cg < VG; ++cg)
-          load_lds16(vbase + row * kvp + (cg * 64 + lc < p.vdim ? cg * 64 + lc : 0), &vl[(cg * 64 + wave * 8 + RSTEP * u) * 64]);
+          load_lds16(vbase + row * kvp + (cg * 64 + lc < p.vdim ? cg * 64 + lc : 0), &dst[(cg * 64 + wave * 8 + RSTEP * u) * 64]);
       }
     } else {
       for (int c = t; c < 64 * DVT * 16; c += 64 * NW) {
         const int r = c / (DVT * 16), e = c - r * DVT * 16;
         const long row = s0 + r < n_keys ? s0 + r : n_keys - 1;
-        vl[tile_at<64>(r, e)] = e < p.vdim ? vbase[row * kvp + e] : (uint16_t)0;
+        dst[tile_at<64>(r, e)] = e < p.vdim ? vbase[row * kvp + e] : (uint16_t)0;
       }
     }
   };
@@ -676,105 +678,107 @@ __global__ void __launch_bounds__(64 * NW, DKC > 6 ? 1 : 2) latent_prefill_kerne
   for (int qt = 0; qt < 2; ++qt)
 #pragma unroll
     for (int c = 0; c < DKC; ++c) q[qt][c] = *(const u32x4*)&ql[tile_at<QT>(wave * 32 + qt * 16 + i16, c * 32 + 8 * g)];
+  __syncthreads();  // the first values go where the queries were
+  if (n_keys > 0) load_v(0, smem + KSTAGE);
   // this wave's queries, as positions counted from lo
   const int wq0 = (int)((long)p.q_first + qt0 + wave * 32 - lo), wq1 = wq0 + 31;
-  for (int s0 = 0, buf = 0; s0 < n_keys; s0 += 64, buf ^= 1) {
-    const uint16_t* kl = smem + buf * KSTAGE;
-    const bool more = s0 + 64 < n_keys;
-    // (blocks that none of the wave's queries sees are skipped)
-    const bool mine = s0 <= wq1 && (p.window <= 0 || s0 + 63 > wq0 - p.window);
-    wait_loads<0>();  // this wave's rows of the keys have landed
-    __syncthreads();                     // ... and everybody's; everybody is done with the values and the other keys
-    load_v(s0);
-    if (more) load_k(s0 + 64, smem + (buf ^ 1) * KSTAGE);
-    u32x4 pb[2][2];
-    if (mine) {
-      f32x4 s4[2][4];
+  // full: every query of the wave sees every key of the block
+  auto attend = [&](const uint16_t* kl, const uint16_t* vl, int s0, const bool full) {
+    f32x4 s4[2][4];
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) s4[qt][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+    for (int c = 0; c < DKC; ++c)
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt) {
+        const u32x4 a = *(const u32x4*)&kl[tile_at<64>(kt * 16 + i16, c * 32 + 8 * g)];
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt) s4[qt][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < DKC; ++c) {
-          const u32x4 a = *(const u32x4*)&kl[tile_at<64>(kt * 16 + i16, c * 32 + 8 * g)];
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) s4[qt][kt] = mfma16x16x32<T>(a, q[qt][c], s4[qt][kt]);
-        }
+        for (int qt = 0; qt < 2; ++qt) s4[qt][kt] = mfma16x16x32<T>(a, q[qt][c], s4[qt][kt]);
       }
-      const bool full = s0 + 63 <= wq0 && (p.window <= 0 || s0 >= wq1 - p.window + 1);
+    pin_scores<DKC>();
+    __builtin_amdgcn_s_setprio(0);
+    u32x4 pb[2][2];
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        float mx = -INFINITY;
-        if (full) {
-#pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              s4[qt][kt][r] *= sc;
-              mx = fmaxf(mx, s4[qt][kt][r]);
-            }
-        } else {
-          // keys counted from the block's start: the last one seen, and the last one in front of the window
-          const int last = wq0 + qt * 16 + i16 - s0, before = p.window > 0 ? last - p.window : -1;
-#pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int s = kt * 16 + 4 * g + r;
-              const float v = s4[qt][kt][r] * sc;
-              s4[qt][kt][r] = s <= last && s > before ? v : -INFINITY;
-              mx = fmaxf(mx, s4[qt][kt][r]);
-            }
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        if (__any(mx > m[qt])) {
-          const float mn = fmaxf(m[qt], mx), keep = __builtin_amdgcn_exp2f(m[qt] - mn);
-          m[qt] = mn;
-          l[qt] *= keep;
-#pragma unroll
-          for (int j = 0; j < DVT; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[qt][j][r] *= keep;
-        }
-        float e[4][4], sum = 0.f;
+    for (int qt = 0; qt < 2; ++qt) {
+      float mx = -INFINITY;
+      if (full) {
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            e[kt][r] = __builtin_amdgcn_exp2f(s4[qt][kt][r] - m[qt]);
-            sum += e[kt][r];
+            s4[qt][kt][r] = s4[qt][kt][r] * sc;
+            mx = fmaxf(mx, s4[qt][kt][r]);
           }
-        l[qt] += sum;  // this lane's keys only; the lane groups are added up at the end
+      } else {
+        // keys counted from the block's start: the last one seen, and the last one in front of the window
+        const int last = wq0 + qt * 16 + i16 - s0, before = p.window > 0 ? last - p.window : -1;
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-          pb[qt][kk] = u32x4{T::pack2(e[2 * kk][0], e[2 * kk][1]), T::pack2(e[2 * kk][2], e[2 * kk][3]),
-                             T::pack2(e[2 * kk + 1][0], e[2 * kk + 1][1]), T::pack2(e[2 * kk + 1][2], e[2 * kk + 1][3])};
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int s = kt * 16 + 4 * g + r;
+            const float v = s4[qt][kt][r] * sc;
+            s4[qt][kt][r] = s <= last && s > before ? v : -INFINITY;
+            mx = fmaxf(mx, s4[qt][kt][r]);
+          }
       }
-    }
-    // the values were requested before the next keys
-    if (more) wait_loads<RB * KG>();
-    else wait_loads<0>();
-    __syncthreads();
-    if (mine) {
+      mx = rows_max(mx);
+      if (__any(mx > m[qt])) {
+        const float mn = fmaxf(m[qt], mx), keep = __builtin_amdgcn_exp2f(m[qt] - mn);
+        m[qt] = mn;
+        l[qt] *= keep;
+#pragma unroll
+        for (int j = 0; j < DVT; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[qt][j][r] *= keep;
+      }
+      float e[4][4], sum = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          e[kt][r] = __builtin_amdgcn_exp2f(s4[qt][kt][r] - m[qt]);
+          sum += e[kt][r];
+        }
+      l[qt] += sum;  // this lane's keys only; the lane groups are added up at the end
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-        for (int j = 0; j < DVT; ++j) {
-          const int row = 32 * kk + 4 * g + (i16 >> 2), col = 16 * j + 4 * (i16 & 3);
-          const u32x2 a0 = lds_read_tr16(&vl[tile_at<64>(row, col)]);
-          const u32x2 a1 = lds_read_tr16(&vl[tile_at<64>(row + 16, col)]);
-          const u32x4 va = {a0.x, a0.y, a1.x, a1.y};
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) acc[qt][j] = mfma16x16x32<T>(va, pb[qt][kk], acc[qt][j]);
-        }
+        pb[qt][kk] = u32x4{T::pack2(e[2 * kk][0], e[2 * kk][1]), T::pack2(e[2 * kk][2], e[2 * kk][3]),
+                           T::pack2(e[2 * kk + 1][0], e[2 * kk + 1][1]), T::pack2(e[2 * kk + 1][2], e[2 * kk + 1][3])};
     }
+    __builtin_amdgcn_sched_barrier(0x6);
+    __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < DVT; ++j) {
+        const int row = 32 * kk + 4 * g + (i16 >> 2), col = 16 * j + 4 * (i16 & 3);
+        const u32x2 a0 = lds_read_tr16(&vl[tile_at<64>(row, col)]), a1 = lds_read_tr16(&vl[tile_at<64>(row + 16, col)]);
+        const u32x4 va = {a0.x, a0.y, a1.x, a1.y};
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) acc[qt][j] = mfma16x16x32<T>(va, pb[qt][kk], acc[qt][j]);
+      }
+    pin_values<DVT>();
+    __builtin_amdgcn_s_setprio(0);
+  };
+  for (int s0 = 0, buf = 0; s0 < n_keys; s0 += 64, buf ^= 1) {
+    wait_loads<0>();  // this wave's rows of the block have landed
+    __syncthreads();  // ... and everybody's; everybody is done with the block before
+    if (s0 + 64 < n_keys) {
+      load_k(s0 + 64, smem + (buf ^ 1) * STAGE);
+      load_v(s0 + 64, smem + (buf ^ 1) * STAGE + KSTAGE);
+    }
+    const uint16_t *kl = smem + buf * STAGE, *vl = kl + KSTAGE;
+    // (blocks that none of the wave's queries sees are skipped)
+    if (s0 > wq1 || (p.window > 0 && s0 + 63 <= wq0 - p.window)) continue;
+    attend(kl, vl, s0, s0 + 63 <= wq0 && (p.window <= 0 || s0 >= wq1 - p.window + 1));
   }
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
-    float s = l[qt];
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
+    const float s = rows_sum(l[qt]);
     const float inv = s > 0.f ? 1.f / s : 0.f;
     const int tq = qt0 + wave * 32 + qt * 16 + i16;
     if (tq >= p.t) continue;
