@@ -124,6 +124,7 @@ _SIGNATURES = {
                                c_int, c_int]),
     "mui_moe_route_gateup": (c_int, [_P, c_int, _P, _P, c_int, _P, _P, c_long, _P, c_float, c_int, _P, _P, _P, _P, _P] + [c_int] * 5),
     "mui_moe_down": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int]),
+    "mui_moe_one_down": (c_int, [_P, c_int, _P, c_long, _P, _P, _P, _P, c_int, _P, c_int, c_int, c_int, c_int]),
     "mui_latent_prepare": (c_int, [_P, c_int, _P, c_long, _P, _P, c_float, _P, _P, _P, _P, _P, _P, c_long, _P, c_long,
                                    c_int, c_int, c_int, c_int, c_int, c_int]),
     "mui_latent_step_serves": (c_int, [c_int] * 9),

@@ -1133,6 +1133,74 @@ __global__ void __launch_bounds__(256) moe_one_gateup_kernel(const float* logits
   }
 }
 
+// One token's down product, built like gate and up above: R rows of one chosen expert at a time, thread t has chunks t, t + 256 of every row, the next rows are on their
+// way before the sums meet. The chosen are read by lane; a pair's activations are requested with its rows. Bound by the rows' bytes and a cold chain of two loads. us in
+// bf16 as captured, 16-pair tiles / this (at 7.1 TB/s): 64 experts of 1792 x 4096, 8 / 7 / 5 with matrices 19.7 / 19.0 (16.5), 18.6 / 17.4 (14.5), 14.3 / 12.6 (10.3); of
+// 1408 x 2048 10.8 / 9.8 (6.5), 10.3 / 8.6 (5.7), 9.1 / 6.7 (4.1); 32 of 4096 x 1024, 8 / 2 15.0 / 12.8 (9.5), 8.4 / 4.8 (2.4); 16 of 768 x 2048, 8 / 5 7.9 / 7.6, 7.0 / 5.3; 8 of
+// 1024 x 512, 8 4.2 / 3.4. Rows of 512 keep a quarter of the threads: 64 of 512 x 4096, 8 9.0 / 11.7, so shorter rows than 768 stay with the tiles.
+template <typename T, int CH, int R, bool STREAM>
+__global__ void __launch_bounds__(256) moe_one_down_kernel(const int32_t* expert, const uint16_t* act, int top, int n_experts, int n, int k, const uint16_t* w0,
+                                                           long expert_stride, uint16_t* y) {
+  __shared__ float red[2][16][R];  // [buffer][16-lane row of the workgroup][row]
+  const int t = threadIdx.x, lane = t & (kWave - 1), kc = k >> 3;
+  const int mine = lane < top ? expert[lane] : n_experts;
+  int coff[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) coff[j] = t + 256 * j < kc ? (t + 256 * j) << 3 : 0;
+  uint64_t real = __ballot(mine < n_experts);  // places of the chosen with matrices, those behind `row`'s taken out
+  const int groups = __popcll(real) * (n / R);
+  if ((int)blockIdx.x >= groups) return;  // uniform for the workgroup
+  int row = (int)blockIdx.x * R, place = 0;
+  u32x4 w[R][CH], xq[CH], xn[CH];
+  auto request = [&]() {
+    while (row >= n) {
+      row -= n;
+      real &= real - 1;
+    }
+    place = __ffsll((unsigned long long)real) - 1;
+    const uint16_t* base = w0 + (long)__builtin_amdgcn_readlane(mine, place) * expert_stride + (long)row * k;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) xn[j] = ld16(act + (long)place * k + coff[j]);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int j = 0; j < CH; ++j) w[r][j] = ld16_sel<STREAM>(base + (long)r * k + coff[j]);
+  };
+  request();
+  int buf = 0;
+  for (int g = blockIdx.x; g < groups; g += gridDim.x) {
+    const int out_place = place, out_row = row;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) xq[j] = t + 256 * j < kc ? xn[j] : u32x4{0u, 0u, 0u, 0u};
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      float a = 0.f;
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        a = moe_dot2<T>(w[r][j].x, xq[j].x, a);
+        a = moe_dot2<T>(w[r][j].y, xq[j].y, a);
+        a = moe_dot2<T>(w[r][j].z, xq[j].z, a);
+        a = moe_dot2<T>(w[r][j].w, xq[j].w, a);
+      }
+      acc[r] = a;
+    }
+    if (g + (int)gridDim.x < groups) {
+      row += (int)gridDim.x * R;
+      request();
+    }
+    row16_reduce_scatter<R>(acc, lane);
+    if ((lane & (16 / R - 1)) == 0) red[buf][t >> 4][(lane & 15) / (16 / R)] = acc[0];
+    __syncthreads();
+    if (t < 16 * R) {  // sixteen lanes per output
+      const int part = t & 15, o = t >> 4;
+      const float v = row16_sum(red[buf][part][o]);
+      if (part == 0) y[(long)out_place * n + out_row + o] = T::pack(v);
+    }
+    buf ^= 1;
+  }
+}
+
 // one wave per output of a pair: fp32 storage, and sizes that are no multiple of 8
 template <typename T, int EPI>
 __global__ void __launch_bounds__(256) moe_rows_kernel(const typename T::storage* w0, const typename T::storage* w1,
@@ -1259,7 +1327,9 @@ static int launch_route(hipStream_t s, const float* logits, const void* corr, in
                         int tokens, int tile_pairs, int max_tiles, int32_t* expert, float* weight, int32_t* pairs,
                         MoeTile* tiles) {
   typedef typename T::storage S;
-  const bool one = tokens <= 64 && tile_pairs;
+  // One launch of one workgroup, whose waves route a token each, or another workgroup per four tokens in front: us, one launch / two, 64 experts, 8 chosen: 8 tokens 6.7 / 7.6,
+  // 16 8.0 / 7.6, 20 9.7 / 7.6, 32 12.6 / 7.6, 64 22.0 / 7.6; 6 chosen 6.0 / 6.9, 7.2 / 6.9, 8.3 / 6.9, 10.9 / 6.9, 18.7 / 6.9
+  const bool one = tokens <= 8 && tile_pairs;
   if (!one)
     hipLaunchKernelGGL((moe_route_kernel<T>), dim3(ceil_div(tokens, 4)), dim3(256), 0, s, logits, (const S*)corr, n_out,
                        top, tokens, expert, weight);
@@ -1416,4 +1486,33 @@ extern "C" int mui_moe_down(mui_stream_t stream, int dtype, const void* down, lo
   p.max_tiles = mui_moe_max_tiles(tokens, top, n_experts, tile_pairs);
   p.once = read_once(n_experts, n_out, k_in, down, down);
   MUI_BY_DTYPE((launch_moe_product<TT, MOE_DOWN>((hipStream_t)stream, p, expert, n_experts, tokens * top, tile_pairs)));
+}
+
+namespace mui {
+// Sizes that moe_one_down_kernel covers, else MUI_ERR_UNSUPPORTED (nothing launched)
+template <typename T>
+static int launch_moe_one_down(hipStream_t s, const MoeGemmParams& p, const int32_t* expert, int n_experts) {
+  if (p.tokens != 1 || p.top > kWave || p.n % 8 || p.k % 8 || p.k < 768 || p.k > 2 * 256 * 8 || p.expert_stride % 8) return MUI_ERR_UNSUPPORTED;
+  if (!aligned16(p.w0) || !aligned16(p.x) || (long)p.top * p.n >= (1L << 30)) return MUI_ERR_UNSUPPORTED;
+  auto launch = [&](auto kernel, int rows) {
+    hipLaunchKernelGGL(kernel, dim3(balanced_grid(p.top * (p.n / rows), 3)), dim3(256), 0, s, expert, p.x, p.top, n_experts, p.n, p.k, p.w0, p.expert_stride, (uint16_t*)p.y);
+    return launch_status();
+  };
+  if (p.k <= 256 * 8) return p.once ? launch(moe_one_down_kernel<T, 1, 8, true>, 8) : launch(moe_one_down_kernel<T, 1, 8, false>, 8);
+  return p.once ? launch(moe_one_down_kernel<T, 2, 4, true>, 4) : launch(moe_one_down_kernel<T, 2, 4, false>, 4);
+}
+}  // namespace mui
+
+extern "C" int mui_moe_one_down(mui_stream_t stream, int dtype, const void* down, long expert_stride, const void* act, const int32_t* expert, const int32_t* pairs,
+                                const void* tiles, int tile_pairs, void* out, int n_experts, int n_out, int k_in, int top) {
+  if (tile_pairs == 16) {
+    MUI_CHECK_ARG(down && act && expert && out && pairs && tiles && n_experts > 0 && n_out > 0 && k_in > 0 && top > 0);
+    MoeGemmParams p = {};
+    p.w0 = (const uint16_t*)down; p.expert_stride = expert_stride; p.x = (const uint16_t*)act; p.y = out; p.n = n_out; p.k = k_in; p.top = top; p.tokens = 1;
+    p.once = read_once(n_experts, n_out, k_in, down, down);
+    const int st = dtype == MUI_DTYPE_F16 ? launch_moe_one_down<F16>((hipStream_t)stream, p, expert, n_experts)
+                   : dtype == MUI_DTYPE_BF16 ? launch_moe_one_down<BF16>((hipStream_t)stream, p, expert, n_experts) : MUI_ERR_UNSUPPORTED;
+    if (st != MUI_ERR_UNSUPPORTED) return st;
+  }
+  return mui_moe_down(stream, dtype, down, expert_stride, act, expert, pairs, tiles, tile_pairs, out, n_experts, n_out, k_in, top, 1);
 }

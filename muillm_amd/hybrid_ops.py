@@ -182,17 +182,21 @@ def _expert_operands(x, gate, up, down, tokens):
     _operand(down, "down", x, (n_experts, width, ff))
 
 
-def _moe_down(act, down, expert, pairs, tiles, tile_pairs):
+def _moe_down(act, down, expert, pairs, tiles, tile_pairs, one=False):
     (n_experts, width, ff), (tokens, top) = down.shape, expert.shape
     lib, code, st = _lib.load(), dtype_code(act.dtype), _stream(act)
     out = torch.empty((tokens * top, width), dtype=act.dtype, device=act.device)
+    if one:  # (other sums than in mui_moe_down, whose rows do not depend on how many there are)
+        check(lib.mui_moe_one_down(st, code, down.data_ptr(), width * ff, act.data_ptr(), expert.data_ptr(), pairs.data_ptr(), tiles.data_ptr(), tile_pairs,
+                                   out.data_ptr(), n_experts, width, ff, top), "mui_moe_one_down")
+        return out
     check(lib.mui_moe_down(st, code, down.data_ptr(), width * ff, act.data_ptr(), expert.data_ptr(), _ptr(pairs),
                            _ptr(tiles), tile_pairs, out.data_ptr(), n_experts, width, ff, top, tokens), "mui_moe_down")
     return out
 
 
 def moe(x: torch.Tensor, logits: torch.Tensor, correction: Optional[torch.Tensor], gate: torch.Tensor, up: torch.Tensor, down: torch.Tensor, limit: float, top: int) -> MoEOutput:
-    """moe_route and moe_experts; a single token's routing goes with its gate and up product."""
+    """moe_route and moe_experts; a single token's routing goes with its gate and up product, and its products have kernels of their own."""
     n_experts, ff, width = gate.shape
     tokens, n_out = logits.shape
     tile = moe_tile_pairs(x.dtype, tokens, top, n_experts, width, ff)
@@ -207,7 +211,7 @@ def moe(x: torch.Tensor, logits: torch.Tensor, correction: Optional[torch.Tensor
     check(_lib.load().mui_moe_route_gateup(_stream(x), dtype_code(x.dtype), logits.data_ptr(), _ptr(correction), n_out - n_experts, gate.data_ptr(), up.data_ptr(),
                                            ff * width, x.data_ptr(), float(limit), tile, expert.data_ptr(), weight.data_ptr(), pairs.data_ptr(), tiles.data_ptr(),
                                            act.data_ptr(), n_experts, ff, width, top, tokens), "mui_moe_route_gateup")
-    return MoEOutput(_moe_down(act, down, expert, pairs, tiles, tile), x, expert, weight, n_experts)
+    return MoEOutput(_moe_down(act, down, expert, pairs, tiles, tile, one=True), x, expert, weight, n_experts)
 
 
 def moe_tile_pairs(dtype: torch.dtype, tokens: int, top: int, n_experts: int, width: int, ff: int) -> int:

@@ -85,3 +85,33 @@ def test_refused():
                                         4, 16, 64, top, 1) == -1
     with pytest.raises(RuntimeError):
         ops.moe(x, logits, corr, gate, up[:2], down, 7.0, 2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("experts,chosen,ff,width", [
+    (16, [3, 20, 0, 15], 768, 8), (16, [20, 20, 5], 768, 4104), (9, [8, 7, 6, 5, 4, 3, 2, 1, 0, 9], 2048, 264), (6, [5], 2056, 512), (4, [0, 9, 3], 4096, 1000),
+    (4, [0, 3], 760, 64), (4, [3, 9, 1], 4104, 64), (4, [2, 1], 1024, 12), (4, [9, 9], 1024, 64)])
+def test_down_against_64_bits(experts, chosen, ff, width, dtype):
+    """Rows of one and two chunks per thread, whole and part filled; the first and the last expert; identity experts in front, between and alone, whose rows stay as they
+    are; from (760 ..) on sizes that go the general way, and nothing chosen that has a matrix. Gate: the rounding of the result to 16 bits."""
+    g = torch.Generator(device=DEV).manual_seed(ff + width)
+    act = torch.empty(len(chosen), ff, device=DEV).normal_(generator=g).to(dtype)
+    down = torch.empty(experts, width, ff, device=DEV).normal_(0.0, ff ** -0.5, generator=g).to(dtype)
+    expert = torch.tensor([chosen], dtype=torch.int32, device=DEV)
+    real = [(i, e) for i, e in enumerate(chosen) if e < experts]
+    pairs = torch.tensor([i for i, _ in real] + [0], dtype=torch.int32, device=DEV)
+    most = _lib.load().mui_moe_max_tiles(1, len(chosen), experts, 16)
+    tiles = torch.zeros(most + 1, 4, dtype=torch.int32)
+    tiles[0, 2] = len(real)
+    for j, (_, e) in enumerate(real):
+        tiles[1 + j] = torch.tensor([e, j, 1, 0])
+    tiles, out = tiles.to(DEV), torch.full((len(chosen), width), 7.0, dtype=dtype, device=DEV)
+    st = torch.cuda.current_stream().cuda_stream
+    _lib.check(_lib.load().mui_moe_one_down(st, ops.dtype_code(dtype), down.data_ptr(), width * ff, act.data_ptr(), expert.data_ptr(), pairs.data_ptr(), tiles.data_ptr(), 16,
+                                            out.data_ptr(), experts, width, ff, len(chosen)), "mui_moe_one_down")
+    for i, e in enumerate(chosen):
+        if e >= experts:
+            assert bool((out[i] == 7.0).all())
+            continue
+        want = down[e].double() @ act[i].double()
+        assert float((out[i].double() - want).norm() / want.norm()) < ULP[dtype] / 2
