@@ -240,10 +240,12 @@ extern "C" int mui_greedy_advance_ws(mui_stream_t stream, int dtype, const void*
   p.embed_table = (const uint16_t*)embed_table; p.embed_stride = embed_row_stride;
   p.embed_out = (uint16_t*)embed_out; p.embed_dim = embed_dim;
   hipStream_t s = (hipStream_t)stream;
-  // one workgroup per 1024 chunks of 16 bytes (one load per thread), 32 at most; rows that cannot be
-  // read in 16-byte chunks, rows of a single part and calls without a workspace take one workgroup
+  // One workgroup per 4096 chunks of 16 bytes (what its threads request together), 32 at most; rows that cannot be read in 16-byte chunks, rows of a single part and calls
+  // without a workspace take one workgroup. More parts scan no faster and their atomics, neighbours in memory and ordered device-wide, queue: us, parts of 1024 / 4096
+  // chunks, 128256 entries, 1 / 4 / 8 / 20 / 32 / 64 rows 7.4 / 7.1, 8.4 / 7.4, 9.4 / 7.6, 12.6 / 8.2, 15.4 / 8.9, 29.9 / 11.0; 32768 entries, 1 / 20 / 64 rows 7.6 / 5.4, 8.4 / 6.1,
+  // 10.9 / 6.1. Fewer are slower up to 32 rows (two: 8.2, 8.6, 8.8, 9.1, 9.2, 10.4).
   const bool vec = ((row_stride & 7) == 0) && ((((uintptr_t)logits) & 15u) == 0);
-  int parts = vec ? ((vocab >> 3) + kArgmaxThreads - 1) / kArgmaxThreads : 1;
+  int parts = vec ? ((vocab >> 3) + 4 * kArgmaxThreads - 1) / (4 * kArgmaxThreads) : 1;
   parts = parts > 32 ? 32 : parts;
   if (parts > 1 && workspace && (((uintptr_t)workspace) & 7u) == 0 && workspace_bytes >= mui_greedy_workspace_bytes(rows)) {
     unsigned long long* best_word = (unsigned long long*)workspace;

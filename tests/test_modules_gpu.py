@@ -576,6 +576,25 @@ def test_greedy_advance_on_several_workgroups(dtype):
     assert torch.equal(out2[:, 0].cpu(), lg.float().argmax(-1).cpu())
 
 
+@pytest.mark.parametrize("vocab", [32768, 32776, 65544, 128256, 8 * 4096 * 32, 8 * 4096 * 32 + 8, 8 * 4096 * 33])
+def test_greedy_advance_parts(vocab):
+    """Rows of one workgroup and of two, whole and part filled, of 32 and beyond: the winner in a part's first and last chunk and behind the last, ties to the lowest."""
+    from muillm_amd import muillm_ext
+    g, parts = torch.Generator().manual_seed(vocab), min(32, -(-vocab // 32768))
+    per = -(-(vocab // 8) // parts) * 8
+    at = [0, per - 1, per % vocab, vocab - 1, (parts - 1) * per]
+    logits = torch.randn(len(at) + 1, vocab, generator=g).half()
+    for row, i in enumerate(at):
+        logits[row, i] = 20.0
+    logits[-1, [0, per - 1, vocab - 1]] = 20.0
+    n = len(logits)
+    ids, step, toks = (torch.zeros(*shape, dtype=torch.int64, device=DEV) for shape in ((n, 1), (n,), (n, 3)))
+    ws = muillm_ext.greedy_workspace(n, DEV)
+    for _ in range(3):
+        muillm_ext.mui_greedy_advance(logits.to(DEV), ids, step, toks, workspace=ws)
+    assert toks.cpu().tolist() == [[i] * 3 for i in at + [0]] and int(ws.sum()) == 0
+
+
 def test_greedy_advance_leaves_the_embedding_row():
     """With an embedding table the launch that chooses the token also copies that token's row to
     embed_out (finished rows: the pad token's), in the single-workgroup form and in the workspace form."""
