@@ -117,7 +117,7 @@ int mui_linear_ws(mui_stream_t stream, int dtype, const void* weights, long w_pi
 
 /* A linear with a residual and the norm that follows it, in one call: y = W x (+ add_bias) + residual, h = next_gain * y * rsqrt(mean(y^2) + epsilon)
  * over each row of y -- mui_linear_ws and mui_rmsnorm, whose contracts hold here. Where K is divided between workgroups and a launch adds up (a
- * workspace given, at most 8192 outputs) that launch takes the norm as well. */
+ * workspace given, at most 8192 outputs and a multiple of 8) that launch takes the norm as well. */
 int mui_linear_norm(mui_stream_t stream, int dtype, const void* weights, long w_pitch, const void* x, const void* add_bias,
                     const void* residual, const void* next_gain, float epsilon, void* y, void* h, int n_out, int k_in, int tokens,
                     void* workspace, size_t workspace_bytes);
@@ -611,7 +611,7 @@ int mui_joined_linear_f32(mui_stream_t stream, int dtype, const float* residual_
                           float next_scale, float epsilon, float* residual_out, void* h, const void* weights, const void* bias, float* out, int n_out, int k_in, int tokens);
 
 /* y = W x (+ add_bias) and mui_residual_norm of it (y_scale 1), in one call; 16-bit types. workspace as for mui_linear_ws. Where K is divided
- * between workgroups and a launch adds up (a workspace given, at most 8192 outputs, h given) that launch joins them, too. */
+ * between workgroups and a launch adds up (a workspace given, at most 8192 outputs and a multiple of 8, h given) that launch joins them, too. */
 int mui_linear_residual_norm(mui_stream_t stream, int dtype, const void* weights, long w_pitch, const void* x, const void* add_bias,
                              const float* residual_in, const void* post_gain, float branch_scale, const void* next_gain, float next_scale,
                              float epsilon, void* y, float* residual_out, void* h, int n_out, int k_in, int tokens, void* workspace,

@@ -187,7 +187,8 @@ constexpr int kJoinMost = 8192;  // outputs
 
 // q: the product, without what its end applies. MUI_ERR_UNSUPPORTED: not a case for it, nothing has been launched
 static int linear_join(hipStream_t s, int dtype, int wf, SkinnyParams q, JoinRow p, bool f32, void* workspace, size_t workspace_bytes) {
-  if (p.tokens <= MUI_MAX_TOKENS || p.n > kJoinMost || !p.h || !workspace || ((uintptr_t)workspace & 255u) || workspace_bytes < prefill_workspace_bytes()) return MUI_ERR_UNSUPPORTED;
+  // (rows are read and written eight values at a time; what leaves the shares of K asks for four only)
+  if (p.tokens <= MUI_MAX_TOKENS || p.n > kJoinMost || p.n % 8 || !p.h || !workspace || ((uintptr_t)workspace & 255u) || workspace_bytes < prefill_workspace_bytes()) return MUI_ERR_UNSUPPORTED;
   const void* ptrs[] = {q.w0, q.x, p.add_bias, p.r32, p.r16, p.post_gain, p.next_gain, p.y, p.r_out, p.h};
   for (const void* at : ptrs)
     if (!aligned16(at)) return MUI_ERR_UNSUPPORTED;

@@ -71,6 +71,38 @@ def test_by_the_rule_and_with_the_norm_behind(n, k, tokens, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k,tokens", [(4100, 14336, 333), (2052, 8192, 768), (1004, 6144, 1300)])
+def test_rows_of_whole_fours_with_the_norm_behind(n, k, tokens, dtype):
+    """K is shared for rows that are no multiple of eight, but the launch that takes the norm along moves eight values at a time: these are two calls, and nothing behind the
+    outputs is written."""
+    lib, s, code, guard = _lib.load(), torch.cuda.current_stream().cuda_stream, CODE[dtype], 64
+    assert prompt_shares("fp16" if dtype == torch.float16 else "bf16", n, k, tokens)[1] > 1
+    g = _gen(n + k + tokens)
+    w, x, res = _rand((n, k), dtype, g, k ** -0.5), _rand((tokens, k), dtype, g), _rand((tokens, n), dtype, g)
+    post, after = 1 + _rand((n,), dtype, g, 0.2), 1 + _rand((n,), dtype, g, 0.2)
+    stream = torch.empty(tokens, n, device=DEV).normal_(generator=g)
+    ws = torch.zeros(lib.mui_linear_workspace_bytes(), dtype=torch.uint8, device=DEV)
+
+    def guarded(kind):
+        buffer = torch.full((tokens * n + guard,), 7.0, dtype=kind, device=DEV)
+        return buffer[:tokens * n].view(tokens, n), buffer[tokens * n:]
+
+    (y, y_end), (h, h_end), (out, out_end) = guarded(dtype), guarded(dtype), guarded(torch.float32)
+    y2, h2, out2 = _linear(x, w, None, None, res, ws), torch.empty_like(res), torch.empty_like(stream)
+    _lib.check(lib.mui_rmsnorm(s, code, after.data_ptr(), y2.data_ptr(), EPS, h2.data_ptr(), tokens, n), "norm")
+    _call("mui_linear_norm", x, w, k, None, (res.data_ptr(), after.data_ptr(), EPS, y.data_ptr(), h.data_ptr()), y, ws)
+    assert torch.equal(y, y2) and torch.equal(h, h2)
+    plain = x.double() @ w.double().T
+    _close(h, _rms(plain + res.double(), after.double()), 2 * HALF_ULP[dtype])
+    y2 = _linear(x, w, None, None, None, ws)
+    _lib.check(lib.mui_residual_norm(s, code, stream.data_ptr(), y2.data_ptr(), 1.0, post.data_ptr(), 0.5, after.data_ptr(), 2.0, EPS, out2.data_ptr(), h2.data_ptr(), tokens, n), "norm")
+    _call("mui_linear_residual_norm", x, w, k, None, (stream.data_ptr(), post.data_ptr(), 0.5, after.data_ptr(), 2.0, EPS, y.data_ptr(), out.data_ptr(), h.data_ptr()), y, ws)
+    assert torch.equal(y, y2) and torch.equal(out, out2) and torch.equal(h, h2)
+    for end in (y_end, h_end, out_end):
+        assert bool((end == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("shift", [0, 6, 7])
 @pytest.mark.parametrize("tile,shares", [(7, 7), (8, 3), (4, 5)])
 @pytest.mark.parametrize("n,k,tokens", [(4, 3072, 65), (260, 3200, 257), (4104, 2816, 300)])
