@@ -194,7 +194,7 @@ static int prompt_layers(mui_stream_t stream, const mui_decoder_stack_t* m, int 
     if (scales) {
       if (next && residual) {
         SkinnyParams q = {};
-        q.w0 = weight; q.pitch = pitch; q.s0 = (const uint16_t*)scales; q.s_pitch = shift ? 2L * (k >> shift) : 1; q.group_shift = shift;
+        q.w0 = weight; q.pitch = pitch; q.s0 = (const uint16_t*)scales; q.group_shift = shift;
         q.x = (const uint16_t*)x; q.residual = (const uint16_t*)residual; q.y = (uint16_t*)y; q.n = n; q.k = k; q.tokens = rows;
         q.workspace = linear_workspace; q.workspace_bytes = linear_workspace_bytes;
         st = gain ? MUI_ERR_UNSUPPORTED : launch_codes_norm((hipStream_t)stream, m->dtype, shift ? WF_U8_GROUP : WF_I8_CHANNEL, q, next, m->norm_eps, w.normed);

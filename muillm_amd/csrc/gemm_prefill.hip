@@ -1105,11 +1105,11 @@ constexpr bool kPipelined = WF != WF_U8_GROUP || T::kDtype == MUI_DTYPE_F16;
 
 // what the LDS-direct loads need: whole k-steps, 16-byte aligned rows, 32-bit byte offsets from
 // the operands' bases
-// (codes of the group format: a k-step of 64 lies in one group, and a (scale, min) pair is one load of 4 bytes, which has to be aligned)
+// (codes of the group format: whole groups, a k-step of 64 lies in one, and a (scale, min) pair is one load of 4 bytes, which has to be aligned)
 static bool lds_direct_loads_serve(const PrefillGemmParams& p, int wf) {
   return g_prefill_dma && p.k % 64 == 0 && p.pitch % 16 == 0 && (long)p.n * p.pitch < (1L << 32) &&
          (long)p.tokens * p.k * 2 < (1L << 32) &&
-         (wf != WF_U8_GROUP || (p.group_shift >= 6 && p.s_pitch % 2 == 0 && (((uintptr_t)p.s0 | (uintptr_t)p.s1) & 3) == 0));
+         (wf != WF_U8_GROUP || (p.group_shift >= 6 && p.group_shift <= 30 && p.k % (1 << p.group_shift) == 0 && p.s_pitch % 2 == 0 && (((uintptr_t)p.s0 | (uintptr_t)p.s1) & 3) == 0));
 }
 static bool pipelined_loop_serves(const PrefillGemmParams& p, int wf) { return lds_direct_loads_serve(p, wf); }
 static bool pipelined(const PrefillGemmParams& p, int dtype, int wf) {
@@ -1695,6 +1695,7 @@ extern "C" int mui_probe_prefill_plan(int dtype, int weight_format, int gateup, 
 extern "C" int mui_probe_prompt_shares(int dtype, int weight_format, int n, int k, int tokens, int group_size_shift, int* tile, int* shares) {
   using namespace mui;
   MUI_CHECK_ARG((dtype == MUI_DTYPE_F16 || dtype == MUI_DTYPE_BF16) && weight_format >= 0 && weight_format <= 2 && n >= 1 && k >= 1 && tokens >= 1 && tile && shares);
+  MUI_CHECK_ARG(weight_format != 2 || (group_size_shift >= 0 && group_size_shift <= 30));
   const int wf = weight_format == 0 ? WF_16BIT : weight_format == 1 ? WF_I8_CHANNEL : WF_U8_GROUP;
   const PartsPlan plan = parts_taken(prefill_params(probe_params(wf, n, k, tokens, group_size_shift), wf), dtype, wf, prefill_workspace_best() - kXsCounterBytes);
   *tile = plan.tile;

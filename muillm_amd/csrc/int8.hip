@@ -348,6 +348,17 @@ static int check_int8_common(int dtype, const void* w, long pitch, const void* x
   return MUI_OK;
 }
 
+static int check_int8_groups(int shift, int k) {
+  return shift < 4 || shift > 30 || (k & ((1 << shift) - 1)) ? MUI_ERR_UNSUPPORTED : MUI_OK;
+}
+
+int check_int8_linear(int dtype, const void* codes, long pitch, const void* scales, int group_shift, const void* x, int n, int k, int tokens) {
+  const int st = check_int8_common(dtype, codes, pitch, x, nullptr, n, k, tokens, true);
+  if (st != MUI_OK) return st;
+  if (!scales) return MUI_ERR_INVALID_ARG;
+  return group_shift ? check_int8_groups(group_shift, k) : MUI_OK;
+}
+
 }  // namespace mui
 
 using namespace mui;
@@ -473,8 +484,7 @@ extern "C" int mui_int8_group_linear_ws(mui_stream_t stream, int dtype, const vo
   int st = check_int8_common(dtype, weights_u8, w_pitch, x, norm_weights, n_out, k_in, tokens, true);
   if (st != MUI_OK) return st;
   MUI_CHECK_ARG(scales_min_vals && y && (workspace || workspace_bytes == 0));
-  if (group_size_shift < 4 || group_size_shift > 30) return MUI_ERR_UNSUPPORTED;
-  if (k_in & ((1 << group_size_shift) - 1)) return MUI_ERR_UNSUPPORTED;
+  if ((st = check_int8_groups(group_size_shift, k_in)) != MUI_OK) return st;
   hipStream_t s = (hipStream_t)stream;
   if (tokens > MUI_MAX_TOKENS) {  // a prompt: the kernels for more tokens, which dequantise the codes themselves
     SkinnyParams sp = {};
@@ -533,8 +543,7 @@ extern "C" int mui_int8_group_gateup_silu(mui_stream_t stream, int dtype, const 
   if (st != MUI_OK) return st;
   MUI_CHECK_ARG(up_u8 && gate_smv && up_smv && h);
   if (!aligned16(up_u8)) return MUI_ERR_ALIGNMENT;
-  if (group_size_shift < 4 || group_size_shift > 30) return MUI_ERR_UNSUPPORTED;
-  if (k_in & ((1 << group_size_shift) - 1)) return MUI_ERR_UNSUPPORTED;
+  if ((st = check_int8_groups(group_size_shift, k_in)) != MUI_OK) return st;
   if (smv_pitch < 2L * (k_in >> group_size_shift) || (smv_pitch & 1)) return MUI_ERR_INVALID_ARG;
   hipStream_t s = (hipStream_t)stream;
   if (tokens > MUI_MAX_TOKENS) {

@@ -210,14 +210,17 @@ static SkinnyParams product(const void* weights, long w_pitch, const void* x, in
   return q;
 }
 
-// int8 codes with the residual and the norm behind, where K is shared between workgroups; MUI_ERR_UNSUPPORTED: it is not, nothing has been launched
+// int8 codes (dense pairs) with the residual and the norm behind, where K is shared between workgroups; MUI_ERR_UNSUPPORTED: it is not, nothing has been launched
 int launch_codes_norm(hipStream_t s, int dtype, int wf, const SkinnyParams& q, const void* next_gain, float eps, void* h) {
   if (q.gamma || q.mul_bias) return MUI_ERR_UNSUPPORTED;
+  const int st = check_int8_linear(dtype, q.w0, q.pitch, q.s0, wf == WF_U8_GROUP ? q.group_shift : 0, q.x, q.n, q.k, q.tokens);
+  if (st != MUI_OK) return st;
   JoinRow p = {};
   p.n = q.n; p.tokens = q.tokens; p.add_bias = q.add_bias; p.r16 = q.residual; p.next_gain = (const uint16_t*)next_gain;
   p.next_scale = 1.f; p.eps = eps; p.y = q.y; p.h = (uint16_t*)h;
   SkinnyParams a = q;
   a.add_bias = a.residual = nullptr;
+  a.s_pitch = wf == WF_U8_GROUP ? 2L * (q.k >> q.group_shift) : 1;
   return linear_join(s, dtype, wf, a, p, false, q.workspace, q.workspace_bytes);
 }
 

@@ -1,6 +1,7 @@
 """Where linears of more than 128 tokens share K between workgroups: products that were measured both ways (256 CUs)."""
 import pytest
 
+from muillm_amd import _lib
 from tests.prompt_util import prompt_shares
 
 
@@ -15,3 +16,12 @@ def test_k_is_shared_where_it_is_faster(weights, n, k, tokens, whole, shared):
 def test_never():
     for weights, n, k, tokens in [("bf16", 4096, 14336, 128), ("bf16", 4098, 14336, 333), ("bf16", 4096, 14336 + 8, 333), ("bf16", 4096, 640, 333), ("bf16", 1 << 20, 14336, 333)]:
         assert prompt_shares(weights, n, k, tokens)[1] == 1
+
+
+def test_groups_that_do_not_divide_k():
+    """The last group's part would have no (scale, smallest value) pair."""
+    assert prompt_shares("int8_group", 2048, 8320, 333, shift=7)[1] > 1  # 65 groups
+    assert prompt_shares("int8_group", 2048, 8320, 333, shift=8)[1] == 1  # 32 and a half
+    for shift in (-1, 31):
+        with pytest.raises(_lib.MuiLibraryError):
+            prompt_shares("int8_group", 2048, 8320, 333, shift=shift)

@@ -1,9 +1,12 @@
 """Prompts, and steps of more rows than the decode kernels take, through one library call against the same layers called one by one: plain and int8 weights, several
 turns, padding, captured steps; and what has to stay with the single layers. The two run the same products and sums: the same bits."""
 
+import ctypes
+
 import pytest
 import torch
 
+from muillm_amd import _lib, muillm_ext
 from muillm_amd.engine import init_engine
 from muillm_amd.engineconfig import MuiEngineConfig
 from muillm_amd.modules.decoder.decoderstack import MuiPromptStack
@@ -260,3 +263,32 @@ def test_first_long_prompt_runs_on_the_modules(monkeypatch):
         first, second = _run(lm, True, [ids], 256, 1), _run(lm, True, [ids], 256, 1)
         assert first[2] == calls_first and second[2] == 1
         assert torch.equal(first[0], second[0]) and torch.equal(first[1], second[1])
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("group,layer,field,value,status", [
+    (128, 0, "int8_group_size_shift", 8, -2),  # o has a K of three groups and a half (all other products have whole ones)
+    (128, 0, "int8_group_size_shift", 40, -2),
+    (128, 0, "o_weight", None, -1), (0, 0, "o_weight", None, -1), (0, 0, "down_weight", None, -1),
+    (0, 0, "o_pitch", 880, -1), (0, 0, "down_pitch", 1008, -1), (0, 0, "o_pitch", 904, -2)])
+def test_int8_operands_are_refused_where_k_is_shared_too(group, layer, field, value, status):
+    """As by mui_int8_linear and mui_int8_group_linear: nothing is read through a descriptor that those refuse."""
+    lm = _lm(torch.float16, group, hidden_size=1024, intermediate_size=1024, num_attention_heads=8, num_key_value_heads=1)
+    cache, lib, t = lm.create_cache(1, 128), _lib.load(), 80
+    stack = MuiPromptStack(lm.model.layers, lm.model.rotary_emb, cache)
+    stack.desc.n_q_heads = 7  # (the first 896 columns of o)
+    x = torch.randn(1, t, 1024, device=DEV).half()
+    pos, out = torch.arange(t, device=DEV), torch.empty_like(x)
+    ws, scratch = torch.empty(lib.mui_decoder_stack_prompt_bytes(ctypes.byref(stack.desc), 1, t, 1), dtype=torch.uint8, device=DEV), muillm_ext.new_linear_workspace(DEV)
+
+    def run():
+        return lib.mui_decoder_stack_prompt(torch.cuda.current_stream().cuda_stream, ctypes.byref(stack.desc), 1, t, x.data_ptr(), out.data_ptr(), pos.data_ptr(), 0,
+                                            pos.data_ptr(), t, None, 0, 1, ws.data_ptr(), scratch.data_ptr(), scratch.numel())
+
+    try:
+        _lib.check(lib.mui_tune_prompt_shares(7, 2), "mui_tune_prompt_shares")
+        assert run() == 0 and bool(scratch[4096:].any())  # K is shared
+        setattr(stack.desc.layers[layer], field, value)
+        assert run() == status
+    finally:
+        _lib.check(lib.mui_tune_prompt_shares(0, 0), "mui_tune_prompt_shares")
