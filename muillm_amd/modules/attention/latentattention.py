@@ -74,7 +74,7 @@ class MuiLatentAttention(MuiModule):
         w = self.up_kv.weight
         w_uk, w_uv = w[:c.heads * c.dim], w[c.heads * c.dim:]
         step = t == 1 and hybrid_ops.latent_step_serves(down, b, c.heads, c.dim, c.rot_dim, c.vdim, w_uk, w_uv, state.c, state.r, c.window)
-        if step and b == 1 and c.q_rank % 8 == 0 and down.data_ptr() % 16 == 0 and self.up_q.takes_front():
+        if step and b == 1 and self._norm_goes_with_query(down):
             # the query's norm goes with its projection, the token's rows with the attention
             up = self.up_q.cpp_module
             normed = muillm_ext.MuiLinearModuleHandle(up.engine, up.weights, self.q_norm, self.eps, up.mul_bias, up.add_bias)
@@ -100,6 +100,11 @@ class MuiLatentAttention(MuiModule):
             o = hybrid_ops.latent_attention(q, cos_sin, w_uk, w_uv, state.c, state.r,
                                             cache_position, cache.row_start, c.heads, c.dim, c.vdim, c.scale, c.window, route)
         return self._project(cache.take(o), behind)
+
+    def _norm_goes_with_query(self, down: torch.Tensor) -> bool:
+        """Whether the projection's own norm stands in for latent_prepare's. In fp16 it does not: it multiplies latent and gain in 16 bits in front of the scale, where a product beyond
+        65504 or below 6e-5 does not fit, and latent_prepare does so in 32 bits behind it."""
+        return down.dtype == torch.bfloat16 and self.config.q_rank % 8 == 0 and down.data_ptr() % 16 == 0 and self.up_q.takes_front()
 
     def _project(self, o: torch.Tensor, behind) -> torch.Tensor:
         return self.out_proj(o) if behind is None else self.out_proj(o, behind=behind)

@@ -97,3 +97,27 @@ def test_decoder(listened):
     outs += [lm(input_ids=torch.tensor([[t]], device=DEV), past_key_values=cache).logits[0] for t in tokens[40:]]
     assert_rows(row_error(torch.cat(outs), oracle.forward(cfg, w, tokens)[0]), torch.bfloat16)
     assert heard == (([40] * 3 + [1] * 3 * 110) if listened else [])
+
+
+def _logits(lm, tokens, first):
+    cache = lm.create_cache(1, 200)
+    outs = [lm(input_ids=torch.tensor([tokens[:first]], device=DEV), past_key_values=cache).logits[0]]
+    return torch.cat(outs + [lm(input_ids=torch.tensor([[t]], device=DEV), past_key_values=cache).logits[0] for t in tokens[first:]])
+
+
+def _assert_fp16(err):
+    """fp16 rounds eight times finer than bf16, for which the gate is 0.08; every single token for itself."""
+    assert float(err[20:].max()) <= 0.08 / 8, err
+
+
+@pytest.mark.parametrize("latents,gains", [(1.0, 1.0), (2.0 ** 11, 2.0 ** 7), (2.0 ** -10, 2.0 ** -10)])
+def test_latents_and_gains_whose_product_is_out_of_fp16s_range(latents, gains):
+    """The normed query latent is gain times latent times the norm's scale: the first two alone need not fit."""
+    cfg = config([(latent(rot=16), None), (latent(rot=16, window=21, kv_from=0), None)])
+    w = random_weights(cfg, seed=6, close_calls=False)
+    for i in range(2):
+        w[f"l{i}.mix.dq"] *= latents
+        w[f"l{i}.mix.dq.norm"] *= gains
+        w[f"l{i}.mix.uq"] /= gains
+    tokens = torch.randint(0, cfg["vocab"], (30,), generator=torch.Generator().manual_seed(6)).tolist()
+    _assert_fp16(row_error(_logits(build(cfg, w, torch.float16), tokens, 20), oracle.forward(cfg, w, tokens)[0]))
