@@ -121,3 +121,22 @@ def test_latents_and_gains_whose_product_is_out_of_fp16s_range(latents, gains):
         w[f"l{i}.mix.uq"] /= gains
     tokens = torch.randint(0, cfg["vocab"], (30,), generator=torch.Generator().manual_seed(6)).tolist()
     _assert_fp16(row_error(_logits(build(cfg, w, torch.float16), tokens, 20), oracle.forward(cfg, w, tokens)[0]))
+
+
+@pytest.mark.parametrize("name", ["q_norm", "kv_norm"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gains_in_the_middle_of_a_buffer(dtype, name):
+    """Where a parameter lies (views into one flat buffer) is no matter to the single token."""
+    cfg = config([(latent(rot=16), None)])
+    w = random_weights(cfg, seed=7, close_calls=False)
+    tokens = torch.randint(0, cfg["vocab"], (30,), generator=torch.Generator().manual_seed(7)).tolist()
+    lm = build(cfg, w, dtype)
+    for m in lm.modules():
+        if isinstance(m, MuiLatentAttention):
+            gain = getattr(m, name)
+            flat = torch.zeros(gain.numel() + 8, dtype=dtype, device=DEV)
+            flat[1:1 + gain.numel()] = gain
+            setattr(m, name, torch.nn.Parameter(flat[1:1 + gain.numel()], requires_grad=False))
+            assert getattr(m, name).data_ptr() % 16
+    err = row_error(_logits(lm, tokens, 20), oracle.forward(cfg, w, tokens)[0])
+    _assert_fp16(err) if dtype == torch.float16 else assert_rows(err, dtype)
