@@ -599,8 +599,8 @@ int mui_moe_residual_norm(mui_stream_t stream, int dtype, const float* residual_
                           float next_scale, float epsilon, float* residual_out, void* h, int rows, int k);
 
 /* mui_residual_norm (y_scale 1) and the product that reads its h, in one call; 16-bit types: mui_linear_ws (no norm of its own), mui_gateup_silu_bias, mui_linear_f32, whose
- * contracts hold. h is always written. Of a single token (k_in <= 4096, or 8192 and at most 256 outputs for mui_joined_linear_f32; residual_out another buffer than residual_in) one launch;
- * the bits are those of the two calls. */
+ * contracts hold. h is always written. Of a single token (k_in <= 4096, or 8192 and at most 256 outputs for mui_joined_linear_f32; residual_out, h and out clear of residual_in, y, the gains
+ * and each other) one launch; the bits are those of the two calls, which everything else runs as. */
 int mui_joined_linear(mui_stream_t stream, int dtype, const float* residual_in, const void* y, const void* post_gain, float branch_scale, const void* next_gain,
                       float next_scale, float epsilon, float* residual_out, void* h, const void* weights, long w_pitch, const void* add_bias, void* out, int n_out, int k_in,
                       int tokens, void* workspace, size_t workspace_bytes);

@@ -7,11 +7,24 @@ namespace mui {
 
 int launch_linear_f32_join(hipStream_t s, int dtype, const void* w, const void* x, const void* bias, float* y, int n, int k, float eps, const BoundaryInFront& front);
 
-// operands and sizes that the kernels' loads cannot take
-static bool joins(int dtype, int tokens, int k, const BoundaryInFront& f, const void* y) {
+struct Bytes { const void* at; size_t n; };
+static bool apart(Bytes a, Bytes b) {
+  const uintptr_t x = (uintptr_t)a.at, y = (uintptr_t)b.at;
+  return !a.at || !b.at || x + a.n <= y || y + b.n <= x;
+}
+
+// Operands and sizes that the kernels' loads cannot take. Every workgroup reads the boundary's inputs while others are writing: no output may lie on one of them, nor on another output,
+// where the two calls, one after the other, allow it.
+static bool joins(int dtype, int tokens, int k, const BoundaryInFront& f, const void* y, Bytes out) {
   const void* ptrs[] = {y, f.stream, f.post_gain, f.next_gain, f.stream_out, f.h};
-  bool ok = tokens == 1 && k % 8 == 0 && f.stream && f.stream != f.stream_out && f.h != y && (dtype == MUI_DTYPE_F16 || dtype == MUI_DTYPE_BF16);
+  bool ok = tokens == 1 && k % 8 == 0 && f.stream && (dtype == MUI_DTYPE_F16 || dtype == MUI_DTYPE_BF16);
   for (const void* p : ptrs) ok = ok && aligned16(p);
+  const size_t row = (size_t)k * 2;
+  const Bytes in[] = {{f.stream, 2 * row}, {y, row}, {f.post_gain, row}, {f.next_gain, row}}, outs[] = {{f.stream_out, 2 * row}, {f.h, row}, out};
+  for (int i = 0; i < 3; ++i) {
+    for (const Bytes& b : in) ok = ok && apart(outs[i], b);
+    for (int j = 0; j < i; ++j) ok = ok && apart(outs[i], outs[j]);
+  }
   return ok;
 }
 
@@ -28,7 +41,7 @@ extern "C" int mui_joined_linear(mui_stream_t stream, int dtype, const float* re
                                  int n_out, int k_in, int tokens, void* workspace, size_t workspace_bytes) {
   MUI_CHECK_ARG(y && residual_out && h && weights && out && n_out > 0 && k_in > 0 && tokens > 0 && w_pitch >= k_in && (workspace || workspace_bytes == 0));
   const BoundaryInFront front = boundary(residual_in, post_gain, branch_scale, next_gain, next_scale, residual_out, h);
-  if (joins(dtype, tokens, k_in, front, y) && aligned16(weights) && w_pitch % 8 == 0) {
+  if (joins(dtype, tokens, k_in, front, y, {out, (size_t)n_out * 2}) && aligned16(weights) && w_pitch % 8 == 0) {
     SkinnyParams p = {};
     p.w0 = weights; p.pitch = w_pitch; p.x = (const uint16_t*)y; p.add_bias = (const uint16_t*)add_bias; p.y = (uint16_t*)out; p.n = n_out; p.k = k_in; p.tokens = 1;
     p.eps = epsilon;
@@ -45,7 +58,7 @@ extern "C" int mui_joined_gateup_silu(mui_stream_t stream, int dtype, const floa
                                       long gu_pitch, const void* gate_bias, const void* up_bias, void* out, int n_inter, int k_in, int tokens) {
   MUI_CHECK_ARG(y && residual_out && h && gate && up && out && n_inter > 0 && k_in > 0 && tokens > 0 && gu_pitch >= k_in && (gate_bias == nullptr) == (up_bias == nullptr));
   const BoundaryInFront front = boundary(residual_in, post_gain, branch_scale, next_gain, next_scale, residual_out, h);
-  if (joins(dtype, tokens, k_in, front, y) && aligned16(gate) && aligned16(up) && gu_pitch % 8 == 0) {
+  if (joins(dtype, tokens, k_in, front, y, {out, (size_t)n_inter * 2}) && aligned16(gate) && aligned16(up) && gu_pitch % 8 == 0) {
     SkinnyParams p = {};
     p.w0 = gate; p.w1 = up; p.pitch = gu_pitch; p.x = (const uint16_t*)y; p.add_bias = (const uint16_t*)gate_bias; p.mul_bias = (const uint16_t*)up_bias;
     p.y = (uint16_t*)out; p.n = n_inter; p.k = k_in; p.tokens = 1; p.eps = epsilon;
@@ -62,7 +75,7 @@ extern "C" int mui_joined_linear_f32(mui_stream_t stream, int dtype, const float
                                      float* out, int n_out, int k_in, int tokens) {
   MUI_CHECK_ARG(y && residual_out && h && weights && out && n_out > 0 && k_in > 0 && tokens > 0);
   const BoundaryInFront front = boundary(residual_in, post_gain, branch_scale, next_gain, next_scale, residual_out, h);
-  if (joins(dtype, tokens, k_in, front, y) && aligned16(weights)) {
+  if (joins(dtype, tokens, k_in, front, y, {out, (size_t)n_out * 4}) && aligned16(weights)) {
     const int st = launch_linear_f32_join((hipStream_t)stream, dtype, weights, y, bias, out, n_out, k_in, epsilon, front);
     if (st != MUI_ERR_UNSUPPORTED) return st;
   }

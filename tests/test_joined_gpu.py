@@ -65,6 +65,46 @@ def test_stream_in_place_and_refused_arguments():
     assert call(stream, apart, None) == -1
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("where", ["y", "behind y", "stream", "gain", "h on the stream", "h on y"])
+def test_outputs_on_inputs(where, dtype):
+    """Where an output lies on what the boundary reads, the two calls follow each other: every workgroup would still be reading."""
+    lib, s, code, g, k = _lib.load(), torch.cuda.current_stream().cuda_stream, CODE[dtype], _gen(2), 4096
+    y, w, post = _rand((1, k), dtype, g), _rand((k, k), dtype, g, k ** -0.5), 1 + _rand((k,), dtype, g, 0.2)
+    stream = torch.empty(1, k, device=DEV).normal_(generator=g)
+
+    def run(name):
+        pool = torch.zeros(8 * k, dtype=torch.int32, device=DEV)  # [stream | y, gain | stream behind | h, out], 4 k bytes each
+        at = lambda part, n=0: pool.data_ptr() + 4 * k * part + 2 * n  # noqa: E731
+        pool[:k].view(torch.float32).copy_(stream[0])
+        pool[k:2 * k].view(dtype).copy_(torch.cat([y[0], post]))
+        x_out, h, out = at(2), at(3), at(3, k)
+        out = {"y": at(1), "behind y": at(1, k - 8), "stream": at(0, k), "gain": at(1, k)}.get(where, out)
+        h = {"h on the stream": at(0, k), "h on y": at(1)}.get(where, h)
+        if name:
+            args = (s, code, at(0), at(1), at(1, k), 0.5, at(1, k), 2.0, EPS, x_out, h)
+            if name == "mui_joined_linear":
+                _lib.check(lib.mui_joined_linear(*args, w.data_ptr(), k, None, out, k, k, 1, None, 0), name)
+            elif name == "mui_joined_gateup_silu":
+                _lib.check(lib.mui_joined_gateup_silu(*args, w.data_ptr(), w[k // 2:].data_ptr(), k, None, None, out, k // 2, k, 1), name)
+            else:
+                _lib.check(lib.mui_joined_linear_f32(*args, w.data_ptr(), None, out, 256, k, 1), name)
+            return pool
+        return pool, (at(0), at(1), at(1, k), x_out, h, out)
+
+    for name in ("mui_joined_linear", "mui_joined_gateup_silu", "mui_joined_linear_f32"):
+        got = run(name)
+        want, (x_in, y_at, gain, x_out, h, out) = run(None)
+        _lib.check(lib.mui_residual_norm(s, code, x_in, y_at, 1.0, gain, 0.5, gain, 2.0, EPS, x_out, h, 1, k), "norm")
+        if name == "mui_joined_linear":
+            _lib.check(lib.mui_linear(s, code, w.data_ptr(), k, h, None, 0.0, None, None, None, out, k, k, 1), name)
+        elif name == "mui_joined_gateup_silu":
+            _lib.check(lib.mui_gateup_silu_bias(s, code, w.data_ptr(), w[k // 2:].data_ptr(), k, h, None, 0.0, None, None, out, k // 2, k, 1), name)
+        else:
+            _lib.check(lib.mui_linear_f32(s, code, w.data_ptr(), h, None, out, 256, k, 1), name)
+        assert torch.equal(got, want), name
+
+
 @torch.no_grad()
 @pytest.mark.parametrize("util", [zufadra_util, salepel_util])
 def test_hybrid_layers_use_it_and_hooks_are_heard(util, monkeypatch):
