@@ -1605,6 +1605,7 @@ int launch_prefill_gemm(hipStream_t s, int dtype, int wf, int epilogue, const Sk
   // tile, 19.6 vs 20.6 at 48, 23.1 vs 21.2 at 64)
   const PrefillGemmParams p = prefill_params(q, wf);
   const bool scratch = q.workspace && ((uintptr_t)q.workspace & 255u) == 0 && q.workspace_bytes >= prefill_workspace_bytes();
+  const auto turn = scratch_turn(scratch ? q.workspace : nullptr);
   if (q.tokens <= 128 && g_prefill_tile == 0 && g_wide_max_tokens == kWideDefaultMaxTokens) {
     float* part = scratch ? (float*)((char*)q.workspace + kXsCounterBytes) : nullptr;
     const size_t part_bytes = scratch ? q.workspace_bytes - kXsCounterBytes : 0;

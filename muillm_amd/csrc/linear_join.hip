@@ -193,6 +193,7 @@ static int linear_join(hipStream_t s, int dtype, int wf, SkinnyParams q, JoinRow
   for (const void* at : ptrs)
     if (!aligned16(at)) return MUI_ERR_UNSUPPORTED;
   q.y = p.y; q.n = p.n; q.tokens = p.tokens;
+  const auto turn = scratch_turn(workspace);
   float* part = (float*)((char*)workspace + prefill_counter_bytes());
   // (K is divided only where it is without the norm, too: whether the boundary was taken along, a hook was listening or all layers came in one call does not show in the bits)
   const size_t part_bytes = workspace_bytes - prefill_counter_bytes();

@@ -1,6 +1,8 @@
 // Interface between the single-token GEMV entry points and the small-batch MFMA kernel.
 #pragma once
 
+#include <mutex>
+
 #include "common.cuh"
 
 namespace mui {
@@ -197,6 +199,13 @@ __device__ __forceinline__ u32x4 convert_a_pair_f16(uint32_t w0, uint32_t w1, ui
   return u32x4{o[0], o[1], o[2], o[3]};
 }
 
+// A linear that shares K writes its scratch in one launch and reads it in the next. Threads may issue linears on one stream, and with it on one scratch: whoever holds this has both
+// launches in the stream before another thread's calls. (20 ns; none: without scratch)
+inline std::unique_lock<std::recursive_mutex> scratch_turn(const void* scratch) {
+  static std::recursive_mutex turns[16];
+  if (!scratch) return {};
+  return std::unique_lock<std::recursive_mutex>(turns[((uintptr_t)scratch >> 20) % 16]);
+}
 // tiled matrix-core GEMM for prompts (gemm_prefill.hip): any token count, 16-bit weights or int8 codes of either format
 int launch_prefill_gemm(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
 size_t prefill_workspace_bytes();  // what SkinnyParams::workspace must hold for the prompt GEMM to use it

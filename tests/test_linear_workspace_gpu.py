@@ -84,3 +84,40 @@ def test_tile_exchange_at_a_k_that_steps_do_not_divide(tokens, n, k, dtype):
     assert int(ws[4096:].count_nonzero()) > 0, "K was not shared"
     assert_parity(outs[0], ref, 1e-2, f"tile exchange {tokens}x{n}x{k}")
     assert all(torch.equal(outs[0], y) for y in outs[1:])
+
+
+@torch.no_grad()
+def test_threads_on_one_stream():
+    """Threads share the stream that they start on, and its scratch: what a linear's first launch leaves there is its own until its second has read it."""
+    import threading
+
+    from muillm_amd import muillm_ext
+
+    def product(seed, kind, n, k, tokens):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        x, res = torch.randn(tokens, k, device=DEV, generator=g).half(), torch.randn(tokens, n, device=DEV, generator=g).half()
+        if kind == "16":
+            w = (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).half()
+            return lambda: muillm_ext.muillm_linear_forward(None, x, w, residual=res)
+        codes, scales = torch.randint(-128, 128, (n, k), device=DEV, generator=g, dtype=torch.int16).to(torch.int8), torch.full((n,), 1e-3, device=DEV).half()
+        return lambda: muillm_ext.mui_int8_channel_linear_forward(x, codes, scales, residual=res)
+
+    # two launches beyond 128 tokens and up to them, of codes, and one whose last workgroups add up
+    calls = [product(1, "16", 2048, 8192, 333), product(2, "16", 4096, 14336, 48), product(3, "8", 2048, 8192, 100), product(4, "16", 1024, 8200, 200), product(5, "8", 4096, 8192, 333)]
+    wants, wrong, start = [call() for call in calls], [], threading.Barrier(len(calls))
+    torch.cuda.synchronize()
+
+    def work(i):
+        start.wait()
+        for _ in range(40):
+            outs = [calls[i]() for _ in range(5)]
+            if not all(torch.equal(o, wants[i]) for o in outs):
+                wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(calls))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not wrong
