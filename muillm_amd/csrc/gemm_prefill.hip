@@ -1194,7 +1194,7 @@ constexpr size_t kXsSlotBytes = 128 * 128 * sizeof(float);     // one 128 x 128 
 constexpr size_t kXsCounterBytes = kXsMaxTiles * sizeof(unsigned);
 size_t prefill_counter_bytes() { return kXsCounterBytes; }
 size_t prefill_workspace_bytes() { return kXsCounterBytes + kXsMaxWorkgroups * kXsSlotBytes; }  // the least that is used
-// Shares of K of the pipelined tiles gain 17.8 % of the time of the products that parts_plan was fitted to with 64 MB of scratch, 16.2 with 34, 18.0 with 160
+// What is used of a larger one; shares of K of the pipelined tiles gain little by more
 size_t prefill_workspace_best() { return kXsCounterBytes + ((size_t)64 << 20); }
 
 // shares of K per 128 x 128 tile worth taking, or 0: the grid of whole tiles leaves at least three
@@ -1580,7 +1580,8 @@ int launch_prefill_parts(hipStream_t s, int dtype, int wf, const SkinnyParams& q
   if (g_prefill_tile || g_wide_max_tokens != kWideDefaultMaxTokens) return MUI_ERR_UNSUPPORTED;  // (experiments)
   if (!part || (q.x_pitch != 0 && q.x_pitch != q.k)) return MUI_ERR_UNSUPPORTED;
   if (((uintptr_t)p.y | (uintptr_t)p.residual) & 7) return MUI_ERR_UNSUPPORTED;  // (four outputs at a time)
-  const PartsPlan plan = parts_taken(p, dtype, wf, part_bytes);
+  const size_t most = prefill_workspace_best() - kXsCounterBytes;  // (a caller with more of it gets the same sums)
+  const PartsPlan plan = parts_taken(p, dtype, wf, part_bytes < most ? part_bytes : most);
   if (plan.shares < 2) return MUI_ERR_UNSUPPORTED;
   p.part = part;
   p.k_splits = *shares = plan.shares;

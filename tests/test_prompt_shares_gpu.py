@@ -70,6 +70,15 @@ def test_by_the_rule_and_with_the_norm_behind(n, k, tokens, dtype):
     assert torch.equal(y, y2) and torch.equal(out, out2) and torch.equal(h, h2)
 
 
+@pytest.mark.parametrize("n,k,tokens", [(6144, 8192, 1281), (6144, 8192, 1500), (4096, 14336, 1345)])
+def test_more_scratch_than_asked_for(n, k, tokens):
+    """... changes neither whether K is shared nor the sums: shares that only a larger one would hold are not taken."""
+    g, dtype = _gen(n + k + tokens), torch.float16
+    w, x, res = _rand((n, k), dtype, g, k ** -0.5), _rand((tokens, k), dtype, g), _rand((tokens, n), dtype, g)
+    size = _lib.load().mui_linear_workspace_bytes()
+    assert torch.equal(*(_linear(x, w, None, None, res, torch.zeros(b, dtype=torch.uint8, device=DEV)) for b in (size, 4 * size)))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("n,k,tokens", [(4100, 14336, 333), (2052, 8192, 768), (1004, 6144, 1300)])
 def test_rows_of_whole_fours_with_the_norm_behind(n, k, tokens, dtype):
