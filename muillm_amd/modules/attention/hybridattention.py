@@ -48,7 +48,7 @@ class MuiHybridAttention(MuiModule):
         return type(self.out_proj) is MuiLinear and not heard(self, self.out_proj)
 
     def takes_front(self) -> bool:
-        return type(self.proj) is MuiMultiLinear and self.proj.linear.takes_front() and not heard(self, self.proj)
+        return type(self.proj) is MuiMultiLinear and type(self.proj.linear) is MuiLinear and self.proj.linear.takes_front() and not heard(self, self.proj)
 
     def __init__(self, engine_config: MuiEngineConfig, hidden: int, config: MuiHybridAttentionConfig, layer_idx: int, eps: float,
                  device=None, dtype=None):

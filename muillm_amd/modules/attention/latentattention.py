@@ -104,7 +104,7 @@ class MuiLatentAttention(MuiModule):
     def _norm_goes_with_query(self, down: torch.Tensor) -> bool:
         """Whether the projection's own norm stands in for latent_prepare's. In fp16 it does not: it multiplies latent and gain in 16 bits in front of the scale, where a product beyond
         65504 or below 6e-5 does not fit, and latent_prepare does so in 32 bits behind it. Nor are gains and rows taken that cannot be read 16 bytes at a time."""
-        return (down.dtype == torch.bfloat16 and self.config.q_rank % 8 == 0 and self.up_q.takes_front()
+        return (down.dtype == torch.bfloat16 and self.config.q_rank % 8 == 0 and type(self.up_q) is MuiLinear and self.up_q.takes_front()
                 and all(x is None or x.data_ptr() % 16 == 0 for x in (down, self.q_norm, self.kv_norm)))
 
     def _project(self, o: torch.Tensor, behind) -> torch.Tensor:

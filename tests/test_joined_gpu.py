@@ -133,3 +133,41 @@ def test_hybrid_layers_use_it_and_hooks_are_heard(util, monkeypatch):
     assert torch.equal(got, steps()) and not torch.equal(got, fused)
     for handle in handles:
         handle.remove()
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("util", [zufadra_util, salepel_util])
+def test_projections_that_stand_in_for_the_models_own(util):
+    """A projection may be wrapped or replaced by a module that knows of no boundary in front (nor of a norm of the queries' latent): it is called as before."""
+    class Around(torch.nn.Module):
+        def __init__(self, linear):
+            super().__init__()
+            self.inner, self.weight = linear, linear.weight
+
+        def forward(self, x):
+            return self.inner(x)
+
+    cfg = util.default_config() if util is zufadra_util else util.config([(util.latent(rot=16), util.moe()), (util.mlstm(), None), (util.latent(rot=16, window=5, kv_from=0), None)])
+    lm = util.build(cfg, util.random_weights(cfg, seed=1), torch.bfloat16, DEV)
+    ids = torch.randint(0, cfg["vocab"], (1, 9), generator=torch.Generator().manual_seed(2)).to(DEV)
+
+    def steps():
+        cache = lm.create_cache(1, 16)
+        return torch.cat([lm(input_ids=ids[:, i:i + 1], past_key_values=cache, use_cache=True).logits.float() for i in range(ids.shape[1])], 1)
+
+    heard = lambda m: m.register_forward_hook(lambda *a: None)  # noqa: E731
+    handles = []
+    for layer in lm.model.layers:
+        mixer = layer.mixer
+        handles += [heard(mixer.proj.linear)] if hasattr(mixer, "proj") else []
+        handles += [heard(mixer.up_q)] if hasattr(mixer, "up_q") else []
+    want = steps()  # with a hook that listens each of them is called by itself
+    for handle in handles:
+        handle.remove()
+    for layer in lm.model.layers:
+        mixer = layer.mixer
+        if hasattr(mixer, "proj"):
+            mixer.proj.linear = Around(mixer.proj.linear)
+        if hasattr(mixer, "up_q"):
+            mixer.up_q = Around(mixer.up_q)
+    assert torch.equal(steps(), want)
