@@ -1359,8 +1359,8 @@ constexpr int kMostParts = 8;
 static int g_parts_tile = 0, g_parts_shares = 0;  // mui_tune_prompt_shares; tile -1: never
 
 // Rounds of workgroups by the fullest XCD; a round is its k-steps (a little shorter where CUs are idle: the clock rises) and 3.7 us, the second launch 7.5 and its bytes,
-// written and read, at 3.6 TB/s. Fitted to 2500 products of 18 matrices, 129 to 2500 tokens: within 3 % at the median and 8 % nine times in ten; the pair chosen by
-// it is within 1.4 % of the best nine times in ten.
+// written and read, at 3.6 TB/s. Against 15000 timed pairs of 1080 products, 18 matrices at 129 to 2500 tokens: within 4 % at the median and 9 % nine times in ten; the pair
+// chosen by it is within 2.2 % of the best nine times in ten. Codes (19000 pairs of 1170 products, 13 matrices in both formats, 65 to 1600 tokens): 3 %, 9 %, 1.9 %.
 static PartsPlan parts_plan(const PrefillGemmParams& p, int wf, size_t part_bytes) {
   constexpr struct { int id, rows; float step; } kTiles[] = {{7, 128, 0.78f}, {8, 192, 1.10f}, {4, 256, 1.37f}};
   PartsPlan best = {0, 0, 0.f};
@@ -1384,9 +1384,8 @@ static PartsPlan parts_plan(const PrefillGemmParams& p, int wf, size_t part_byte
   return best;
 }
 
-// Against the plan without shares, whose costs are rounds of tiles at K = 4096 and leave out what a launch takes besides. Of the products above shares are
-// taken for two thirds, 17 % of the time of all of them on average; of 2500 twenty lost more than 2 %, 9 % at worst. Codes (5700 products of 13 matrices, 65 to 1600
-// tokens): taken for half, 17 to 20 %, six lost more than 2 %, 6 % at worst.
+// Against the plan without shares, whose costs are rounds of tiles at K = 4096 and leave out what a launch takes besides. Of the products above shares are taken for half, 13 % of
+// the time of all of them; ten of 1080 lost more than 2 %, 6 % at worst (12288 x 4096 at 280 tokens). Codes: for four of five, 22 %; one of 1170 lost more than 2 %, 3 %.
 static bool parts_are_faster(const PrefillGemmParams& p, int wf, const PartsPlan& parts) {
   if (parts.shares == 0) return false;
   if (g_parts_tile > 0) return true;
@@ -1397,7 +1396,12 @@ static bool parts_are_faster(const PrefillGemmParams& p, int wf, const PartsPlan
                    : whole.tile == 12 ? (codes ? 8.f + 20.5f * per_k : 4.7f + 19.6f * per_k)
                    : whole.tile == 4 || whole.tile == 7 || whole.tile == 8 ? 14.f + 0.9f * whole.cost * per_k
                                                                          : (codes ? 9.f : 6.5f) + 0.82f * whole.cost * per_k;
-  return parts.us < 0.95f * us;
+  // Shares of eight k-steps and fewer have hardly left the loop's start behind when their sums, 6 MB and more, all come at once: parts_plan is 2 to 4 us too low for them. us as
+  // captured, whole / shared, 2112 x 4096 at 241 tokens 23.4 / 25.0, 1024 x 4096 at 539 24.1 / 24.6, codes per row 2048 x 3072 at 322 24.1 / 26.2, of groups 1024 x 4096 at 344
+  // 23.2 / 24.9; with fewer bytes (512 x 4096 at 149 17.7 / 15.4) or longer shares it is not.
+  const bool short_shares = p.k / 64 <= 8 * parts.shares && (long)parts.shares * p.tokens * p.n * 4 >= 6000000;
+  const float start = short_shares ? (codes ? 1.f : 2.5f) : 0.f;
+  return parts.us < 0.95f * us - start;
 }
 
 template <typename T, int WF, int WR, int WT, int NWR, int NWT>
