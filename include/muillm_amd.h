@@ -173,7 +173,7 @@ int mui_int8_linear(mui_stream_t stream, int dtype, const void* weights_i8, long
                     int tokens);
 
 /* The same with a scratch buffer for prompts, as mui_linear_ws has (its contract holds here): from 65 tokens on, and a K that is a multiple of 64, K is shared between
- * workgroups where that is faster. */
+ * workgroups where that is faster. Calls without it, and mui_int8_linear, leave K whole: other sums of the same products. */
 int mui_int8_linear_ws(mui_stream_t stream, int dtype, const void* weights_i8, long w_pitch, const void* scales, const void* x, const void* norm_weights, float epsilon,
                        const void* add_bias, const void* residual, void* y, int n_out, int k_in, int tokens, void* workspace, size_t workspace_bytes);
 
@@ -423,7 +423,7 @@ int mui_greedy_advance(mui_stream_t stream, int dtype, const void* logits, long 
                        const int64_t* eos_ids, int n_eos, long pad_token);
 
 /* mui_greedy_advance with the scan of a long row dealt out to several workgroups (one workgroup per
- * 1024 chunks of 16 bytes, at most 32): a single workgroup pulls a 128k-entry row through one CU's
+ * 4096 chunks of 16 bytes, at most 32): a single workgroup pulls a 128k-entry row through one CU's
  * load path. No counterpart in the reference (its argmax is torch's). `workspace` is
  * mui_greedy_workspace_bytes(rows) bytes of 8-byte aligned device memory, zero-filled once by the
  * caller before the first call; every call leaves it zero-filled again, so one buffer serves all the

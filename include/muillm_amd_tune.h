@@ -90,7 +90,7 @@ int mui_tune_prefill(int tile, int wide_max_tokens);
 int mui_probe_prefill_plan(int dtype, int weight_format, int gateup, int n, int k, int tokens, int group_size_shift, int scratch, int* rest_tokens,
                            int* tile, int* last_round);
 
-/* Shares of K of the pipelined tiles for more than 128 tokens (a workspace given): tile 4, 7 or 8 as numbered above with 2 to 8 shares wherever that exists (six k-steps
+/* Shares of K of the pipelined tiles for more than 128 tokens, of codes more than 64 (a workspace given): tile 4, 7 or 8 as numbered above with 2 to 8 shares wherever that exists (six k-steps
  * of 64 a share, partial outputs that the workspace holds, three rounds of workgroups at most), -1 with 0 shares: never, 0 with 0: the built-in choice. */
 int mui_tune_prompt_shares(int tile, int shares);
 /* What the built-in rule does with a linear of dense, aligned operands and a workspace of mui_linear_workspace_bytes() (needs no GPU; formats as above):
@@ -98,7 +98,7 @@ int mui_tune_prompt_shares(int tile, int shares);
 int mui_probe_prompt_shares(int dtype, int weight_format, int n, int k, int tokens, int group_size_shift, int* tile, int* shares);
 
 /* The kernel that streams 16-bit weights for 17..128 tokens and codes for 17..64: weight rows per unit (8, 16, 24, 32, 40, 48, 56, 64, 96 or 128; gate and up
- * rows together 16, 32, 48, 64, 96 or 112) and shares of K (1..8; more than one needs a workspace, and codes have none). 0 restores the built-in
+ * rows together 16, 32, 48, 64, 96 or 112) and shares of K (1..8; more than one needs a workspace and 16-bit weights). 0 restores the built-in
  * choice. A pair that does not exist for a call (too wide for its tokens, more units than CUs, less than 512 k-values a
  * share) makes the call return MUI_ERR_INVALID_ARG. */
 int mui_tune_stream(int rows_per_unit, int shares);

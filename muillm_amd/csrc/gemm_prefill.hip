@@ -1201,7 +1201,7 @@ size_t prefill_workspace_best() { return kXsCounterBytes + ((size_t)64 << 20); }
 // quarters of the CUs idle and every share keeps at least twelve k-steps of 128 -- the exchange
 // (write-through of the partial tile, the counter, the last workgroup's reads) costs 10-15 us, so
 // it pays on long rows only. gemm_stream.hip has the 17 to 128 tokens of rows whose K is a multiple of 256; what comes here
-// is longer, or a K like 14344, and what parts_plan has (K a multiple of 64, more than 128 tokens) does not come here. Measured on MI355X: 4096 x 14344 at 64 tokens
+// is longer, or a K like 14344, and what parts_plan has taken (K a multiple of 64, more than 128 tokens) does not come here. Measured on MI355X: 4096 x 14344 at 64 tokens
 // 62 -> 51 us, at 128 61 -> 55 us (8 shares, 4 beyond 128 tokens); 1000 x 6152 is below the line's gain (29 -> 31 us at 64 tokens).
 static int xs_shares(const PrefillGemmParams& p) {
   const long tiles = (long)ceil_div(p.n, 128) * ceil_div(p.tokens, 128);

@@ -576,7 +576,7 @@ static int launch_stream_codes(hipStream_t s, int dtype, int epilogue, const Str
   return MUI_ERR_UNSUPPORTED;
 }
 
-// The same for int8 codes, 17 to 64 tokens; groups of 64 or more. (Their entry points take no scratch, so K is never divided between workgroups.)
+// The same for int8 codes, 17 to 64 tokens; groups of 64 or more. (K is never divided here: from 65 tokens on launch_prefill_parts does so.)
 int launch_gemm_stream_int8(hipStream_t s, int dtype, int wf, int epilogue, const SkinnyParams& q) {
   if (!stream_serves_codes(q, wf)) return MUI_ERR_UNSUPPORTED;
   const StreamParams p = stream_params(q, nullptr, true, true);

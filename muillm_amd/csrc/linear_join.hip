@@ -3,8 +3,8 @@
 //                           h = next_scale * next_gain * r * rsqrt(mean(r^2) + eps)          (mui_residual_norm behind mui_linear)
 //   16-bit residual stream  y = W x + bias + r;  h = next_gain * y * rsqrt(mean(y^2) + eps)  (mui_rmsnorm behind mui_linear)
 //
-// With 17 to 128 tokens the linear divides its K between workgroups wherever that is worth a launch that adds the fp32 partial
-// outputs up (gemm_stream.hip). That launch and the norm's are one here: one workgroup per token adds the token's row up and has it in registers for
+// The linear divides its K between workgroups wherever that is worth a launch that adds the fp32 partial outputs up: with 17 to 128 tokens in gemm_stream.hip,
+// with more of them, and codes from 65 on, in gemm_prefill.hip. That launch and the norm's are one here: one workgroup per token adds the token's row up and has it in registers for
 // the norms. Neither is bound by its bytes (a few hundred KB per row at most); each is a launch, a chain of cold loads and one or two sums over the
 // workgroup, so one of them is what is saved. Everything else runs as the two calls it stands for, and K is divided as without the norm: the bits are those of the two
 // calls. (Dividing it also where only the adding launch spoke against it gave 14.8 -> 12.5 us for 4096 x 4096 at 32 tokens, and other sums than a model whose boundaries are not

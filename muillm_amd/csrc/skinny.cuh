@@ -210,7 +210,7 @@ inline std::unique_lock<std::recursive_mutex> scratch_turn(const void* scratch) 
 int launch_prefill_gemm(hipStream_t s, int dtype, int weight_format, int epilogue, const SkinnyParams& p);
 size_t prefill_workspace_bytes();  // what SkinnyParams::workspace must hold for the prompt GEMM to use it
 size_t prefill_workspace_best();   // beyond, more of it is no use
-// more than 128 tokens, n % 4 == 0: fp32 partial outputs [*shares][tokens][n] of shares of K, where they are worth it, and what adds them up behind
+// more than 128 tokens (codes: 64), n % 4 == 0: fp32 partial outputs [*shares][tokens][n] of shares of K, where they are worth it, and what adds them up behind
 int launch_prefill_parts(hipStream_t s, int dtype, int weight_format, const SkinnyParams& p, float* part, size_t part_bytes, int* shares);
 // what mui_int8_linear_ws (group_shift 0) and mui_int8_group_linear_ws ask of their operands (int8.hip)
 int check_int8_linear(int dtype, const void* codes, long pitch, const void* scales, int group_shift, const void* x, int n, int k, int tokens);
