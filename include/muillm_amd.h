@@ -644,7 +644,8 @@ int mui_moe_gateup(mui_stream_t stream, int dtype, const void* gate, const void*
                    int top, int tokens);
 
 /* mui_moe_route and mui_moe_gateup, whose contracts hold, in one call: of a single token (16-bit types, tile_pairs 16, at most 256 outputs, 8 of them chosen, k_in <= 4096 and a
- * multiple of 8, n_inter even, aligned matrices) one launch. Such a token's pairs and tiles are in the order of the choice, not sorted by expert. */
+ * multiple of 8, n_inter even, aligned matrices) one launch where that is faster (long rows, few outputs). The pairs and tiles of that launch are in the order of the choice, not
+ * sorted by expert. */
 int mui_moe_route_gateup(mui_stream_t stream, int dtype, const float* logits, const void* correction, int n_identity, const void* gate, const void* up,
                          long expert_stride, const void* x, float limit, int tile_pairs, int32_t* expert, float* weight, int32_t* pairs, void* tiles, void* act,
                          int n_experts, int n_inter, int k_in, int top, int tokens);

@@ -1431,6 +1431,15 @@ extern "C" int mui_moe_gateup(mui_stream_t stream, int dtype, const void* gate, 
 }
 
 namespace mui {
+// Microseconds: what counting who is ahead takes, outputs after outputs in every workgroup, the more of them on a CU the longer, and what rounds of rows too short for 256 threads lose
+// against the tiles' (long ones gain), against the launch in front. Of 1530 sizes (8 to 256 outputs, 1 to 8 chosen, 256 to 4096 activations of rows of 256 to 4096, cold weights) it is taken
+// for 783, 25 % faster, six of them 2 to 8 % slower; taken wherever the kernel could, 554 were slower: us, two launches / one, 128 outputs, 4 of 1024 x 256 9.1 / 11.1; 248, 2 of 1024 x 512
+// 9.4 / 14.7; 64, 8 of 4096 x 512 18.5 / 26.4.
+static bool one_launch_is_faster(int n_out, int top, int n, int k, int grid) {
+  const int per_cu = ceil_div(grid, device_cus()), rounds = ceil_div(top * (n / 2), grid);
+  return (float)n_out * (0.022f + 0.008f * (float)per_cu) + (k < 768 ? 0.5f : k < 1536 ? 0.2f : -0.2f) * (float)rounds < 5.f;
+}
+
 // One token and sizes that moe_one_gateup_kernel covers, else MUI_ERR_UNSUPPORTED (nothing launched)
 template <typename T>
 static int launch_moe_one(hipStream_t s, const MoeGemmParams& p, const float* logits, const void* corr, int n_out, int n_experts, int32_t* expert, float* weight,
@@ -1441,6 +1450,7 @@ static int launch_moe_one(hipStream_t s, const MoeGemmParams& p, const float* lo
     if (p.tokens != 1 || n_out > kMoeOneOutputs || p.top > kMoeOneTop || p.n % 2 || p.k % 8 || p.k > 2 * 256 * 8 || p.expert_stride % 8) return MUI_ERR_UNSUPPORTED;
     if (!aligned16(p.w0) || !aligned16(p.w1) || !aligned16(p.x) || (long)p.top * p.n >= (1L << 30)) return MUI_ERR_UNSUPPORTED;
     const dim3 grid(balanced_grid(p.top * (p.n / 2), 3)), block(256);
+    if (!one_launch_is_faster(n_out, p.top, p.n, p.k, (int)grid.x)) return MUI_ERR_UNSUPPORTED;
     auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, block, 0, s, logits, (const uint16_t*)corr, p.x, n_out, p.k, p.w0, p.w1, n_experts, p.top, p.expert_stride, p.n, p.limit,
                          (uint16_t*)p.y, expert, weight, pairs, tiles, p.max_tiles);

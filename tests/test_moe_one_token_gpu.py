@@ -46,6 +46,22 @@ def test_against_64_bits(experts, identity, top, width, ff, dtype):
     assert float((got - want).norm() / want.norm()) < ULP[dtype]
 
 
+@pytest.mark.parametrize("outputs,top,width,ff,one", [
+    (72, 8, 4096, 1792, True), (72, 6, 2048, 1408, True), (128, 8, 2048, 1024, True), (64, 2, 512, 512, True), (8, 2, 256, 4096, True),
+    (128, 4, 256, 1024, False), (256, 2, 512, 1024, False), (64, 8, 512, 4096, False), (192, 2, 1024, 1024, False)])
+def test_one_launch_where_it_is_faster(outputs, top, width, ff, one):
+    """Its tiles are in the order of the choice, those of the general way sorted by expert (which follows where rows are short, outputs many)."""
+    lib, bf16 = _lib.load(), torch.bfloat16
+    logits = torch.arange(outputs, 0, -1, device=DEV).mul(-1.0)[None].contiguous()  # the last one is chosen first
+    w, x, act = torch.zeros(outputs, ff, width, dtype=bf16, device=DEV), torch.zeros(1, width, dtype=bf16, device=DEV), torch.empty(top, ff, dtype=bf16, device=DEV)
+    expert, weight, pairs, tiles = ops._routing(1, top, outputs, 16, x.device)
+    _lib.check(lib.mui_moe_route_gateup(torch.cuda.current_stream().cuda_stream, ops.dtype_code(bf16), logits.data_ptr(), None, 0, w.data_ptr(), w.data_ptr(), ff * width, x.data_ptr(), 7.0,
+                                        16, expert.data_ptr(), weight.data_ptr(), pairs.data_ptr(), tiles.data_ptr(), act.data_ptr(), outputs, ff, width, top, 1), "mui_moe_route_gateup")
+    chosen = list(range(outputs - 1, outputs - 1 - top, -1))
+    assert expert[0].tolist() == chosen
+    assert tiles[1:1 + top, 0].tolist() == (chosen if one else chosen[::-1])
+
+
 @pytest.mark.parametrize("width,ff,once", [(2048, 1408, True), (512, 64, False)])
 def test_same_as_apart(width, ff, once):
     """The general way gives the same choice, and the same values but for the order of sums; the down product takes the tiles as they are left."""
