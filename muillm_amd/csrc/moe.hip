@@ -1328,8 +1328,9 @@ static int launch_route(hipStream_t s, const float* logits, const void* corr, in
                         MoeTile* tiles) {
   typedef typename T::storage S;
   // One launch of one workgroup, whose waves route a token each, or another workgroup per four tokens in front: us, one launch / two, 64 experts, 8 chosen: 8 tokens 6.7 / 7.6,
-  // 16 8.0 / 7.6, 20 9.7 / 7.6, 32 12.6 / 7.6, 64 22.0 / 7.6; 6 chosen 6.0 / 6.9, 7.2 / 6.9, 8.3 / 6.9, 10.9 / 6.9, 18.7 / 6.9
-  const bool one = tokens <= 8 && tile_pairs;
+  // 12 7.1 / 7.2, 16 8.0 / 7.6, 20 9.7 / 7.6, 32 12.6 / 7.6, 64 22.0 / 7.6; 6 chosen 6.0 / 6.9, 6.3 / 6.7, 7.2 / 6.9, 8.3 / 6.9, 10.9 / 6.9, 18.7 / 6.9; 4 chosen 12 5.8 / 6.1,
+  // 16 6.1 / 6.2, 20 6.8 / 6.1; 1 chosen 12 4.7 / 5.3, 16 5.1 / 5.3, 24 5.5 / 5.4
+  const bool one = tokens <= (top <= 4 ? 16 : 12) && tile_pairs;
   if (!one)
     hipLaunchKernelGGL((moe_route_kernel<T>), dim3(ceil_div(tokens, 4)), dim3(256), 0, s, logits, (const S*)corr, n_out,
                        top, tokens, expert, weight);

@@ -88,7 +88,7 @@ def test_linear_f32(dtype, tokens, n, k):
 # mixture of experts
 # --------------------------------------------------------------------------------------
 @pytest.mark.parametrize("tokens,experts,identity,top", [(1, 5, 2, 3), (7, 1, 0, 1), (40, 70, 60, 9), (100, 6, 3, 9), (300, 12, 1, 2),
-                                                         (9, 200, 0, 1)])
+                                                         (9, 200, 0, 1), (12, 20, 0, 6), (13, 20, 0, 6), (16, 20, 4, 4), (17, 20, 4, 4)])
 @pytest.mark.parametrize("tile", [0, 16, 128, 256])
 def test_route(tokens, experts, identity, top, tile):
     g = torch.Generator().manual_seed(tokens)
