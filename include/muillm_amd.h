@@ -423,7 +423,7 @@ int mui_greedy_advance(mui_stream_t stream, int dtype, const void* logits, long 
                        const int64_t* eos_ids, int n_eos, long pad_token);
 
 /* mui_greedy_advance with the scan of a long row dealt out to several workgroups (one workgroup per
- * 4096 chunks of 16 bytes, at most 32): a single workgroup pulls a 128k-entry row through one CU's
+ * 4096 chunks of 16 bytes, of few rows per 1024, at most 32): a single workgroup pulls a 128k-entry row through one CU's
  * load path. No counterpart in the reference (its argmax is torch's). `workspace` is
  * mui_greedy_workspace_bytes(rows) bytes of 8-byte aligned device memory, zero-filled once by the
  * caller before the first call; every call leaves it zero-filled again, so one buffer serves all the

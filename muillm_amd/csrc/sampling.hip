@@ -243,9 +243,12 @@ extern "C" int mui_greedy_advance_ws(mui_stream_t stream, int dtype, const void*
   // One workgroup per 4096 chunks of 16 bytes (what its threads request together), 32 at most; rows that cannot be read in 16-byte chunks, rows of a single part and calls
   // without a workspace take one workgroup. More parts scan no faster and their atomics, neighbours in memory and ordered device-wide, queue: us, parts of 1024 / 4096
   // chunks, 128256 entries, 1 / 4 / 8 / 20 / 32 / 64 rows 7.4 / 7.1, 8.4 / 7.4, 9.4 / 7.6, 12.6 / 8.2, 15.4 / 8.9, 29.9 / 11.0; 32768 entries, 1 / 20 / 64 rows 7.6 / 5.4, 8.4 / 6.1,
-  // 10.9 / 6.1. Fewer are slower up to 32 rows (two: 8.2, 8.6, 8.8, 9.1, 9.2, 10.4).
+  // 10.9 / 6.1. Fewer are slower up to 32 rows (two: 8.2, 8.6, 8.8, 9.1, 9.2, 10.4). Where the parts of 1024 of all rows are 32 at most their atomics don't queue and the scans
+  // are shorter: behind a launch that has just written the rows (its time included), 1 row of 128256 7.8 / 8.5, 2 rows 7.9 / 8.6, 4 rows of 65536 9.3 / 9.8, 1 of 256000 9.1 / 9.8.
   const bool vec = ((row_stride & 7) == 0) && ((((uintptr_t)logits) & 15u) == 0);
   int parts = vec ? ((vocab >> 3) + 4 * kArgmaxThreads - 1) / (4 * kArgmaxThreads) : 1;
+  const long short_parts = ((vocab >> 3) + kArgmaxThreads - 1) / kArgmaxThreads;
+  if (parts > 1 && rows * short_parts <= 32) parts = (int)short_parts;
   parts = parts > 32 ? 32 : parts;
   if (parts > 1 && workspace && (((uintptr_t)workspace) & 7u) == 0 && workspace_bytes >= mui_greedy_workspace_bytes(rows)) {
     unsigned long long* best_word = (unsigned long long*)workspace;

@@ -595,6 +595,24 @@ def test_greedy_advance_parts(vocab):
     assert toks.cpu().tolist() == [[i] * 3 for i in at + [0]] and int(ws.sum()) == 0
 
 
+@pytest.mark.parametrize("vocab,rows", [(32776, 1), (32776, 6), (65536, 4), (65536, 5), (128256, 2), (128256, 3), (8 * 1024 * 31 + 8, 1), (8 * 1024 * 32 + 8, 1)])
+def test_greedy_advance_parts_of_few_rows(vocab, rows):
+    """Parts of 1024 chunks, 32 of them at most over all rows, and more than that: the winner in a part's first and last chunk and behind the last, ties to the lowest."""
+    from muillm_amd import muillm_ext
+    g, parts = torch.Generator().manual_seed(vocab), -(-(vocab // 8) // 1024)
+    per = -(-(vocab // 8) // parts) * 8
+    ws = muillm_ext.greedy_workspace(rows, DEV)
+    for at in ([0], [per - 1], [per], [vocab - 1], [(parts - 1) * per], [per - 1, per, vocab - 1]):
+        logits = torch.randn(rows, vocab, generator=g).half()
+        logits[-1, at] = 20.0
+        want = logits.float().argmax(-1)
+        want[-1] = at[0]
+        ids, step, toks = (torch.zeros(*shape, dtype=torch.int64, device=DEV) for shape in ((rows, 1), (rows,), (rows, 2)))
+        for _ in range(2):
+            muillm_ext.mui_greedy_advance(logits.to(DEV), ids, step, toks, workspace=ws)
+        assert toks.cpu().tolist() == [[i] * 2 for i in want.tolist()] and int(ws.sum()) == 0
+
+
 def test_greedy_advance_leaves_the_embedding_row():
     """With an embedding table the launch that chooses the token also copies that token's row to
     embed_out (finished rows: the pad token's), in the single-workgroup form and in the workspace form."""
