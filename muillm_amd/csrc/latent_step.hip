@@ -12,6 +12,7 @@
 //              61 keys                      256 keys
 //   1 row      16 heads 19.6 / 12.5         16 heads 20.0 / 17.9, 32 heads 21.4 / 18.0
 //   8 rows     32 heads 25.9 / 12.5         32 heads 26.3 / 18.0 (16 heads, 156 keys: 23.2 / 15.9)
+// (attention alone; with what is around it, and at other ranks, MuiLatentAttention has the line.)
 // A sum per key over the wave and an exponential in every lane made 256 keys 19.5: the eight keys of a batch are reduced together, a key per two lanes.
 #include "hybrid.cuh"
 

@@ -73,7 +73,7 @@ class MuiLatentAttention(MuiModule):
         state: MuiLatentState = cache.layers[self.layer_idx if self.own_rows else c.kv_source]
         w = self.up_kv.weight
         w_uk, w_uv = w[:c.heads * c.dim], w[c.heads * c.dim:]
-        step = t == 1 and hybrid_ops.latent_step_serves(down, b, c.heads, c.dim, c.rot_dim, c.vdim, w_uk, w_uv, state.c, state.r, c.window)
+        step = t == 1 and self._one_launch_is_faster(b, state.c.shape[1], down.dtype) and hybrid_ops.latent_step_serves(down, b, c.heads, c.dim, c.rot_dim, c.vdim, w_uk, w_uv, state.c, state.r, c.window)
         if step and b == 1 and self._norm_goes_with_query(down):
             # the query's norm goes with its projection, the token's rows with the attention
             up = self.up_q.cpp_module
@@ -100,6 +100,16 @@ class MuiLatentAttention(MuiModule):
             o = hybrid_ops.latent_attention(q, cos_sin, w_uk, w_uv, state.c, state.r,
                                             cache_position, cache.row_start, c.heads, c.dim, c.vdim, c.scale, c.window, route)
         return self._project(cache.take(o), behind)
+
+    def _one_launch_is_faster(self, batch: int, capacity: int, dtype: torch.dtype) -> bool:
+        """Whether single tokens over caches of so many visible rows take latent_step, whose workgroups have all keys of a head one after the other (28 ns each); the launches apart take as
+        long for few as for many, and longer where the matrices are (rank). A single fp16 row gains least: in bf16 its preparation goes along, several take longer apart. us from the down
+        projection's output to the attention's, apart / one launch, caches full, 1 row of 16 heads of 128 in bf16: rank 64, 128 / 192 / 256 keys 15.7 / 14.8, 15.6 / 16.3, 16.1 / 18.5; 256,
+        192 / 256 keys 17.1 / 16.6, 17.1 / 18.7; 512, 256 keys 19.7 / 20.0; in fp16 rank 64, 64 / 128 / 192 keys 15.9 / 13.9, 16.5 / 16.2, 16.5 / 17.7; 512, 192 / 256 keys 20.4 / 19.4,
+        20.4 / 21.0; 16 rows of 4 heads without the projection: rank 128, 128 / 256 keys 15.6 / 14.0, 15.6 / 17.2; 512, 256 keys 18.9 / 17.3."""
+        c = self.config
+        span = min(c.window, capacity) if c.window > 0 else capacity
+        return span <= (168 if batch > 1 or dtype == torch.bfloat16 else 104) + 3 * c.kv_rank // 16
 
     def _norm_goes_with_query(self, down: torch.Tensor) -> bool:
         """Whether the projection's own norm stands in for latent_prepare's. In fp16 it does not: it multiplies latent and gain in 16 bits in front of the scale, where a product beyond

@@ -99,6 +99,21 @@ def test_decoder(listened):
     assert heard == (([40] * 3 + [1] * 3 * 110) if listened else [])
 
 
+@pytest.mark.parametrize("window,used", [(160, True), (200, False)])
+def test_decoder_beyond_the_keys_of_one_launch(window, used, monkeypatch):
+    cfg = config([(latent(rot=16, window=window), None), (latent(rot=16, window=window, kv_from=0), None)])
+    w = random_weights(cfg, seed=5, close_calls=False)
+    tokens = torch.randint(0, cfg["vocab"], (230,), generator=torch.Generator().manual_seed(5)).tolist()
+    calls, step = [], ops.latent_step
+    monkeypatch.setattr(ops, "latent_step", lambda *a, **kw: calls.append(1) or step(*a, **kw))
+    lm = build(cfg, w, torch.bfloat16)
+    cache = lm.create_cache(1, 240)
+    outs = [lm(input_ids=torch.tensor([tokens[:210]], device=DEV), past_key_values=cache).logits[0]]
+    outs += [lm(input_ids=torch.tensor([[t]], device=DEV), past_key_values=cache).logits[0] for t in tokens[210:]]
+    assert_rows(row_error(torch.cat(outs), oracle.forward(cfg, w, tokens)[0]), torch.bfloat16)
+    assert len(calls) == (2 * 20 if used else 0)
+
+
 def _logits(lm, tokens, first):
     cache = lm.create_cache(1, 200)
     outs = [lm(input_ids=torch.tensor([tokens[:first]], device=DEV), past_key_values=cache).logits[0]]
