@@ -655,8 +655,8 @@ int mui_moe_down(mui_stream_t stream, int dtype, const void* down, long expert_s
                  const int32_t* expert, const int32_t* pairs, const void* tiles, int tile_pairs, void* out,
                  int n_experts, int n_out, int k_in, int top, int tokens);
 
-/* mui_moe_down of a single token (16-bit types, tile_pairs 16, k_in from 768 to 4096 and a multiple of 8, n_out a multiple of 8, at most 64 chosen, aligned matrices: by a kernel of
- * its own, with other sums; everything else by mui_moe_down). */
+/* mui_moe_down of a single token (16-bit types, tile_pairs 16, k_in from 768 to 4096 and a multiple of 8, n_out a multiple of 8, at most 64 chosen, less than 32768 rows of them
+ * unless k_in is 1280 and more, aligned matrices: by a kernel of its own, with other sums; everything else by mui_moe_down). */
 int mui_moe_one_down(mui_stream_t stream, int dtype, const void* down, long expert_stride, const void* act, const int32_t* expert, const int32_t* pairs,
                      const void* tiles, int tile_pairs, void* out, int n_experts, int n_out, int k_in, int top);
 

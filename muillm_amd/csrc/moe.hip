@@ -1137,7 +1137,8 @@ __global__ void __launch_bounds__(256) moe_one_gateup_kernel(const float* logits
 // way before the sums meet. The chosen are read by lane; a pair's activations are requested with its rows. Bound by the rows' bytes and a cold chain of two loads. us in
 // bf16 as captured, 16-pair tiles / this (at 7.1 TB/s): 64 experts of 1792 x 4096, 8 / 7 / 5 with matrices 19.7 / 19.0 (16.5), 18.6 / 17.4 (14.5), 14.3 / 12.6 (10.3); of
 // 1408 x 2048 10.8 / 9.8 (6.5), 10.3 / 8.6 (5.7), 9.1 / 6.7 (4.1); 32 of 4096 x 1024, 8 / 2 15.0 / 12.8 (9.5), 8.4 / 4.8 (2.4); 16 of 768 x 2048, 8 / 5 7.9 / 7.6, 7.0 / 5.3; 8 of
-// 1024 x 512, 8 4.2 / 3.4. Rows of 512 keep a quarter of the threads: 64 of 512 x 4096, 8 9.0 / 11.7, so shorter rows than 768 stay with the tiles.
+// 1024 x 512, 8 4.2 / 3.4. Rows of 512 keep a quarter of the threads: 64 of 512 x 4096, 8 9.0 / 11.7, so shorter rows than 768 stay with the tiles, and those below 1280 where there
+// are 32768 of them and more: 64 of 768 x 4096, 4 / 8 / 32 8.1 / 7.9, 11.1 / 13.1, 32.5 / 38.6; of 1024 x 4096, 4 / 16 8.9 / 8.3, 22.4 / 23.8 (of 1408 x 4096, 8 16.6 / 16.3).
 template <typename T, int CH, int R, bool STREAM>
 __global__ void __launch_bounds__(256) moe_one_down_kernel(const int32_t* expert, const uint16_t* act, int top, int n_experts, int n, int k, const uint16_t* w0,
                                                            long expert_stride, uint16_t* y) {
@@ -1504,6 +1505,7 @@ namespace mui {
 template <typename T>
 static int launch_moe_one_down(hipStream_t s, const MoeGemmParams& p, const int32_t* expert, int n_experts) {
   if (p.tokens != 1 || p.top > kWave || p.n % 8 || p.k % 8 || p.k < 768 || p.k > 2 * 256 * 8 || p.expert_stride % 8) return MUI_ERR_UNSUPPORTED;
+  if (p.k < 1280 && (long)p.top * p.n >= 32768) return MUI_ERR_UNSUPPORTED;
   if (!aligned16(p.w0) || !aligned16(p.x) || (long)p.top * p.n >= (1L << 30)) return MUI_ERR_UNSUPPORTED;
   auto launch = [&](auto kernel, int rows) {
     hipLaunchKernelGGL(kernel, dim3(balanced_grid(p.top * (p.n / rows), 3)), dim3(256), 0, s, expert, p.x, p.top, n_experts, p.n, p.k, p.w0, p.expert_stride, (uint16_t*)p.y);

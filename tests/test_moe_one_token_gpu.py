@@ -131,3 +131,18 @@ def test_down_against_64_bits(experts, chosen, ff, width, dtype):
             continue
         want = down[e].double() @ act[i].double()
         assert float((out[i].double() - want).norm() / want.norm()) < ULP[dtype] / 2
+
+
+@pytest.mark.parametrize("experts,top,width,ff,general", [(32, 8, 4096, 768, True), (32, 32, 1024, 1272, True), (8, 4, 8192, 1024, True), (32, 8, 4088, 768, False), (8, 8, 4096, 1280, False)])
+def test_down_of_many_short_rows(experts, top, width, ff, general):
+    """Short rows, 32768 of them and more, go the general way, whose sums are others."""
+    g, st = torch.Generator(device=DEV).manual_seed(ff + width), torch.cuda.current_stream().cuda_stream
+    act, down = (torch.empty(s, device=DEV).normal_(generator=g).bfloat16() for s in ((top, ff), (experts, width, ff)))
+    logits = torch.empty(1, experts, device=DEV).normal_(generator=g)
+    expert, _, pairs, tiles = ops.moe_route(logits, None, experts, top, 16)
+    one, apart = (torch.empty(top, width, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    args = (st, ops.dtype_code(act.dtype), down.data_ptr(), width * ff, act.data_ptr(), expert.data_ptr(), pairs.data_ptr(), tiles.data_ptr(), 16)
+    _lib.check(_lib.load().mui_moe_one_down(*args, one.data_ptr(), experts, width, ff, top), "mui_moe_one_down")
+    _lib.check(_lib.load().mui_moe_down(*args, apart.data_ptr(), experts, width, ff, top, 1), "mui_moe_down")
+    assert torch.equal(one, apart) == general
+    assert float((one.double() - apart.double()).norm() / apart.double().norm()) < ULP[torch.bfloat16]
