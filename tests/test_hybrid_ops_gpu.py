@@ -88,7 +88,7 @@ def test_linear_f32(dtype, tokens, n, k):
 # mixture of experts
 # --------------------------------------------------------------------------------------
 @pytest.mark.parametrize("tokens,experts,identity,top", [(1, 5, 2, 3), (7, 1, 0, 1), (40, 70, 60, 9), (100, 6, 3, 9), (300, 12, 1, 2),
-                                                         (9, 200, 0, 1), (12, 20, 0, 6), (13, 20, 0, 6), (16, 20, 4, 4), (17, 20, 4, 4)])
+                                                         (9, 200, 0, 1)])
 @pytest.mark.parametrize("tile", [0, 16, 128, 256])
 def test_route(tokens, experts, identity, top, tile):
     g = torch.Generator().manual_seed(tokens)
@@ -111,6 +111,12 @@ def test_route(tokens, experts, identity, top, tile):
         seen += part.tolist()
     assert sorted(seen) == real.nonzero().flatten().tolist()
     assert bool((tiles[1 + n_tiles:, 2] == 0).all())
+
+
+@pytest.mark.parametrize("tokens,experts,identity,top", [(12, 20, 0, 6), (13, 20, 0, 6), (16, 20, 4, 4), (17, 20, 4, 4)])
+@pytest.mark.parametrize("tile", [16, 128])
+def test_route_by_one_workgroup_and_by_more(tokens, experts, identity, top, tile):
+    test_route(tokens, experts, identity, top, tile)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
