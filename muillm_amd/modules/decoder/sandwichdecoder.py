@@ -40,45 +40,48 @@ def run_layers(layers: List[MuiSandwichDecoderLayer], x: torch.Tensor, h: torch.
     final_scale times the final norm's output. collect: a list that receives the residual stream after every layer."""
     shape = h.shape
 
-    def join(x, y, post: MuiRMSNorm, m: float, following: Optional[MuiRMSNorm], scale: float = 1.0):
+    # (the functions in here carry no annotations: those are evaluated on every call)
+    def join(x, y, post, m, following, scale=1.0):
         return hybrid_ops.residual_norm(x, y, post.weight, None if following is None else following.weight, eps,
                                         branch_scale=m, next_scale=scale, emit=True)
 
-    # where it saves a launch the sublayer's last linear takes the join along, or the next sublayer's first product
+    # where it saves a launch the sublayer's last linear takes the join along, or, of a single row, the next sublayer's first product
     rows = h.numel() // h.shape[-1]
     along = ResidualBehind.worth_it(rows)
     ahead = rows == 1 and collect is None
 
-    def boundary(module, args, x, post: MuiRMSNorm, m: float, following: Optional[MuiRMSNorm], scale: float = 1.0, **kw):
-        """(x, h) behind a sublayer, or what the next one takes in front of itself."""
-        if along and "takes_behind" in type(module).__dict__ and module.takes_behind():
-            behind = ResidualBehind(x, post.weight, m, None if following is None else following.weight, scale, eps)
-            y = module(*args, behind=behind)
-            return behind.take(y) or join(x, y, post, m, following, scale)
-        y = module(*args, **kw)
-        if "front" in kw:
-            x = kw["front"].joined()[0]
-        front = ResidualFront.of(x, y, post.weight, m, None if following is None else following.weight, scale, eps) if ahead else None
-        return front or join(x, y, post, m, following, scale)
+    def sublayer(module, args, x, post, m, following, scale=1.0):
+        if not (along and "takes_behind" in type(module).__dict__ and module.takes_behind()):
+            return join(x, module(*args), post, m, following, scale)
+        behind = ResidualBehind(x, post.weight, m, None if following is None else following.weight, scale, eps)
+        y = module(*args, behind=behind)
+        return behind.take(y) or join(x, y, post, m, following, scale)
 
-    def sublayer(module, rest, state, *behind):
-        if isinstance(state, ResidualFront):
-            if "takes_front" in type(module).__dict__ and module.takes_front():
-                return boundary(module, (state.y.reshape(shape),) + rest, None, *behind, front=state)
-            state = state.joined()
-        x, h = state
-        return boundary(module, (h.reshape(shape),) + rest, x, *behind)
+    def single(module, args, state, post, m, following, scale=1.0):
+        """(x, h) behind a sublayer of one row, or what the next one takes in front of itself."""
+        front = isinstance(state, ResidualFront)
+        if front and "takes_front" in type(module).__dict__ and module.takes_front():
+            y = module(state.y.reshape(shape), *args, front=state)
+            x = state.joined()[0]
+        else:
+            x, h = state.joined() if front else state
+            y = module(h.reshape(shape), *args)
+        return ResidualFront.of(x, y, post.weight, m, None if following is None else following.weight, scale, eps) or join(x, y, post, m, following, scale)
 
     state = x, h
     for i, layer in enumerate(layers):
         last, m = i + 1 == len(layers), layer.branch_scale
         following = (final_norm, final_scale) if last else (layers[i + 1].pre_mixer_norm,)
-        at = (cache, cache_position)
-        if layer.mlp is None:
-            state = sublayer(layer.mixer, at, state, layer.post_mixer_norm, m, *following)
-        else:
-            state = sublayer(layer.mixer, at, state, layer.post_mixer_norm, m, layer.pre_mlp_norm)
-            state = sublayer(layer.mlp, (), state, layer.post_mlp_norm, m, *following)
+        behind_mixer = following if layer.mlp is None else (layer.pre_mlp_norm,)
+        if ahead:
+            state = single(layer.mixer, (cache, cache_position), state, layer.post_mixer_norm, m, *behind_mixer)
+            if layer.mlp is not None:
+                state = single(layer.mlp, (), state, layer.post_mlp_norm, m, *following)
+            continue
+        x, h = sublayer(layer.mixer, (h, cache, cache_position), x, layer.post_mixer_norm, m, *behind_mixer)
+        if layer.mlp is not None:
+            x, h = sublayer(layer.mlp, (h,), x, layer.post_mlp_norm, m, *following)
+        h = h.reshape(shape)
         if collect is not None:
-            collect.append(state[0].clone())
-    return (state.joined() if isinstance(state, ResidualFront) else state)[1].reshape(shape)
+            collect.append(x.clone())
+    return (state.joined() if isinstance(state, ResidualFront) else state)[1].reshape(shape) if ahead else h

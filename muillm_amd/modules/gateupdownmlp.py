@@ -210,13 +210,13 @@ class MuiGateUpDownMLP(MuiModule):
     def _forward_fused(self, input: Tensor, residual: Optional[Tensor] = None, behind=None, front=None) -> Tensor:
         if self._kernel_ok(input):
             return _MuiGateUpSiLU.apply(self.cpp_engine, input, self.norm_weights, self.variance_epsilon,
-                                        self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind, front)
+                                        self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind, *(() if front is None else (front,)))
         return self._forward_unfused(input=input if front is None else front.joined()[1], residual=residual)
 
     def _forward_split(self, input: Tensor, residual: Optional[Tensor] = None, behind=None, front=None) -> Tensor:
         if self._kernel_ok(input):
             return _MuiGateUpSiLUSplit.apply(self.cpp_engine, input, self.norm_weights, self.variance_epsilon,
-                                             self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind, front)
+                                             self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, residual, self._biases(), behind, *(() if front is None else (front,)))
         return self._forward_unfused(input=input if front is None else front.joined()[1], residual=residual)
 
     def takes_behind(self) -> bool:

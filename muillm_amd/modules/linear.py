@@ -134,6 +134,8 @@ class MuiLinear(MuiModule, nn.Linear):
     def forward(self, input: Tensor, residual: Optional[Tensor] = None, behind: Optional[muillm_ext.ResidualBehind] = None,
                 front: Optional[muillm_ext.ResidualFront] = None) -> Tensor:
         if self.cpp_module is not None:
+            if front is None:  # (an argument more is half a microsecond of every call)
+                return _MuiLinear.apply(self.cpp_module, input, residual, behind)
             return _MuiLinear.apply(self.cpp_module, input, residual, behind, front)
         if front is not None:
             input = front.joined()[1]
